@@ -92,6 +92,11 @@ struct PrefillArgs {
     float scale;
     uint32_t nblocks;  // images per kv head
     uint32_t *tiles_taken;  // tiles handed out past every workgroup's first (zero at the start: the prepare kernel's doing)
+    // Split keys (attention_prefill_kernel<true>): a tile's keys are taken in parts of `part_blocks` blocks, each of which
+    // leaves its unnormalised O and (m, l) in the workspace for prefill_merge_kernel.
+    uint32_t part_blocks;
+    float *part_o;   // [part][tile][kv head][8 waves][16][64 lanes][4]: the accumulators as they are
+    float *part_ml;  // [part][tile][kv head][4 row groups][32 rows][m, l]
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, uint32_t bytes) {
@@ -323,8 +328,15 @@ constexpr int LDS_BYTES = 8 * MERGE_WAVE_BYTES > 8 * PART_BYTES ? 8 * MERGE_WAVE
 __device__ __forceinline__ uint32_t k_slot(uint32_t b) { return (b & 3) * PART_BYTES; }
 __device__ __forceinline__ uint32_t v_slot(uint32_t b) { return (4 + (b & 3)) * PART_BYTES; }
 
-// One tile of TQ tokens x 8 heads of kv head `kv` against the keys it sees.
-__device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char *tiles, uint32_t tile, uint32_t kv, bool ask, uint32_t *next_tile) {
+// Blocks of keys that tile `tile` sees.
+__device__ __host__ __forceinline__ uint32_t tile_blocks(uint32_t pos, uint32_t tokens, uint32_t tile) {
+    const uint32_t end = tile * TQ + TQ < tokens ? tile * TQ + TQ : tokens;
+    return (pos + end + BK - 1) / BK;
+}
+
+// One tile of TQ tokens x 8 heads of kv head `kv` against the keys it sees, or (SPLIT) against part `part` of them.
+template <bool SPLIT>
+__device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char *tiles, uint32_t tile, uint32_t kv, uint32_t part_index, bool ask, uint32_t *next_tile) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hf = lane >> 5;
@@ -336,21 +348,25 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     const uint32_t tok = tok0 + (col >> 3);
     const uint32_t head = kv * 8 + (col & 7);
 
-    // Keys this workgroup walks: up to what its last token sees; what this wave needs.
-    const uint32_t wg_keys = a.pos + min(tile * TQ + TQ, a.tokens);
-    const uint32_t nblocks = (wg_keys + BK - 1) / BK;
-    const uint32_t wave_first_len = a.pos + tok0 + 1;            // keys the wave's first token sees
-    const uint32_t wave_keys = a.pos + min(tok0 + 4, a.tokens);  // keys its last token sees
+    // Keys this workgroup walks: up to what its last token sees; what this wave needs.  A part's keys count from its
+    // first block on: key0 is that block's first key, and a row of the tile may see none of the part (the tile's tokens
+    // cross a block's end where the last part begins).
+    const uint32_t block0 = SPLIT ? part_index * a.part_blocks : 0, key_base = block0 * BK;
+    const uint32_t all_blocks = tile_blocks(a.pos, a.tokens, tile) - block0;
+    const uint32_t nblocks = SPLIT ? min(all_blocks, a.part_blocks) : all_blocks;
+    auto from_base = [&](uint32_t keys) { return SPLIT ? (keys > key_base ? keys - key_base : 0) : keys; };
+    const uint32_t wave_first_len = from_base(a.pos + tok0 + 1);            // keys the wave's first token sees
+    const uint32_t wave_keys = from_base(a.pos + min(tok0 + 4, a.tokens));  // keys its last token sees
     const uint32_t wave_blocks = tok0 < a.tokens ? min((wave_keys + BK - 1) / BK, nblocks) : 0;
     const uint32_t full_blocks = min(wave_first_len / BK, wave_blocks);  // blocks that need no mask
 
     const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(tiles));
     const uint32_t lane16 = lane * 16;
-    const unsigned char *images = a.images + size_t(kv) * a.nblocks * IMG_BYTES;
+    const unsigned char *images = a.images + (size_t(kv) * a.nblocks + block0) * IMG_BYTES;
     // Half `half` (8 KB) of part `v` (0 = K, 1 = V^T) of block b.  Blocks past the cache's end
     // are read from the last image instead; nobody looks at their slots.
     auto piece = [&](uint32_t b, int v, int half) {
-        const uint32_t bb = min(b, a.nblocks - 1);
+        const uint32_t bb = min(b, a.nblocks - block0 - 1);
         Copy cp;
         cp.src = reinterpret_cast<uint64_t>(images) + uint64_t(bb) * IMG_BYTES + v * PART_BYTES + half * 8192;
         cp.dst = lds0 + (v ? v_slot(b) : k_slot(b)) + half * 8192;
@@ -407,7 +423,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     auto mask_max = [&](floatx16 &s, uint32_t key0, bool masked) {
         float bm = NO_SCORE;
         if (masked) {
-            const uint32_t len = a.pos + tok + 1;              // keys this row sees
+            const uint32_t len = from_base(a.pos + tok + 1);   // keys this row sees
             const uint32_t vis = len > key0 ? len - key0 : 0;  // of which in this block
 #pragma unroll
             for (int r = 0; r < 16; r++) {
@@ -525,7 +541,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     // The gate values of this wave's half of the dims, asked for before the merge below so that they travel while
     // it runs (scattered 16-byte pieces, one round trip for the lot; a token past the end: the last token's, unused).
     float4 g[16];
-    {
+    if constexpr (!SPLIT) {
         const size_t grow = size_t(min(tok, a.tokens - 1)) * a.heads + head;
         const float *gate = a.q_and_gate + grow * 2 * DIM + DIM + 128 * parity;
 #pragma unroll
@@ -561,6 +577,31 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     const float mine = __builtin_amdgcn_exp2f(m_ref - m_new), theirs = __builtin_amdgcn_exp2f(m_other - m_new);
     l_sum = l_sum * mine + l_other * theirs;
 
+    if constexpr (SPLIT) {
+        // The part's O, m and l as they are, a contiguous kilobyte per store of a wave.  (Rows past the chunk's end leave
+        // what their masked lanes hold; nothing reads it.)
+        const float l = l_sum + __shfl_xor(l_sum, 32);
+        const uint32_t ntiles = (a.tokens + TQ - 1) / TQ;
+        const size_t item = (size_t(part_index) * ntiles + tile) * a.kv_heads + kv;
+        float *po = a.part_o + ((item * WAVES + group * 2 + parity) * 16 * 64 + lane) * 4;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int mt = i >> 2, q4 = i & 3;
+            float4 w;
+            w.x = fin[mt][4 * q4] * mine + theirs_in[(16 * mt + 4 * q4) * 64] * theirs;
+            w.y = fin[mt][4 * q4 + 1] * mine + theirs_in[(16 * mt + 4 * q4 + 1) * 64] * theirs;
+            w.z = fin[mt][4 * q4 + 2] * mine + theirs_in[(16 * mt + 4 * q4 + 2) * 64] * theirs;
+            w.w = fin[mt][4 * q4 + 3] * mine + theirs_in[(16 * mt + 4 * q4 + 3) * 64] * theirs;
+            *reinterpret_cast<float4 *>(po + i * 64 * 4) = w;
+        }
+        if (parity == 0 && hf == 0) {
+            float2 ml = {m_new, l};
+            *reinterpret_cast<float2 *>(a.part_ml + ((item * 4 + group) * 32 + col) * 2) = ml;
+        }
+        if (tid == 0) *next_tile = got;
+        return;
+    }
+
     // ---- out = O / l * sigmoid(gate) ---------------------------------------------------
     // The lane's row sum is split over the two lane halves (each saw half the keys).
     const float l = l_sum + __shfl_xor(l_sum, 32);
@@ -588,6 +629,23 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     if (tid == 0) *next_tile = got;
 }
 
+// The first tile that has a part `part` of part_blocks blocks (tiles see more keys the later they are), and how many
+// (tile, part) pairs there are.
+__device__ __host__ __forceinline__ uint32_t prefill_first_tile(uint32_t pos, uint32_t tokens, uint32_t part_blocks, uint32_t part) {
+    const uint32_t ntiles = (tokens + TQ - 1) / TQ;
+    const uint32_t keys = part * part_blocks * BK;  // a tile has the part if it sees more keys than these
+    if (pos + tokens <= keys) return ntiles;
+    if (pos + TQ > keys) return 0;
+    const uint32_t t = (keys - pos) / TQ;  // tokens up to keys - pos see no key of it
+    return t < ntiles ? t : ntiles - 1;
+}
+__device__ __host__ __forceinline__ uint32_t prefill_items(uint32_t pos, uint32_t tokens, uint32_t part_blocks) {
+    const uint32_t ntiles = (tokens + TQ - 1) / TQ;
+    uint32_t n = 0;
+    for (uint32_t p = 0, first; (first = prefill_first_tile(pos, tokens, part_blocks, p)) < ntiles; p++) n += ntiles - first;
+    return n;
+}
+
 // A workgroup takes tiles until there are none left: with more tiles than workgroups (one per CU: the LDS ring
 // fills a CU), the next tile starts without a new workgroup having to be dispatched.  Tiles are numbered from the
 // one with the most keys down, the kv heads side by side.  Workgroup w starts with tile w; the others are handed
@@ -595,16 +653,83 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
 // before the tile's epilogue so that the answer is there when it ends): a workgroup that took a long tile, or runs
 // on a slower CU, asks later and gets a shorter one, so that all of them end together (tiles dealt beforehand, the
 // longest with the shortest, ended 40 us apart: the workgroups' rates differ by a tenth).
+// SPLIT: an item is a part of a tile's keys, parts side by side in tiles and kv heads (workgroups that run together walk
+// the same keys); the tiles that have a part p are the ones from prefill_first_tile(p) on.
+template <bool SPLIT>
 __global__ __launch_bounds__(THREADS, 2) void attention_prefill_kernel(PrefillArgs a) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char tiles[];
     __shared__ uint32_t next_tile;
-    const uint32_t ntiles = (a.tokens + TQ - 1) / TQ, total = ntiles * a.kv_heads, G = gridDim.x;
+    const uint32_t ntiles = (a.tokens + TQ - 1) / TQ, G = gridDim.x;
+    uint32_t total = ntiles * a.kv_heads;
+    if constexpr (SPLIT) total = prefill_items(a.pos, a.tokens, a.part_blocks) * a.kv_heads;
     for (uint32_t idx = blockIdx.x; idx < total;) {
         // (the tiles from G on are handed out by one question each: the tiles before the last G ask one, when they end,
         // and the last G none: nothing is left by then, and the kernel's last epilogues do not wait for an answer)
-        prefill_tile(a, tiles, ntiles - 1 - idx / a.kv_heads, idx % a.kv_heads, idx + G < total, &next_tile);
+        uint32_t at = idx / a.kv_heads, part = 0;
+        if constexpr (SPLIT) {
+            for (uint32_t n; at >= (n = ntiles - prefill_first_tile(a.pos, a.tokens, a.part_blocks, part)); part++) at -= n;
+        }
+        prefill_tile<SPLIT>(a, tiles, ntiles - 1 - at, idx % a.kv_heads, part, idx + G < total, &next_tile);
         lds_barrier();  // the next tile is known; this tile's merge has been read: the next tile's keys may land on it (its stores go on meanwhile)
         idx = next_tile;
+    }
+}
+
+// Joins the parts of every tile: out = sum_p 2^(m_p - m) O_p / sum_p 2^(m_p - m) l_p * sigmoid(gate).  A workgroup takes
+// one token of one kv head: 8 rows x 256 dims, two float4 per thread.  The parts lie in accumulator order, where the 8
+// rows' pieces of four dims are one line of 128 bytes: 8 neighbouring lanes take a line of a part and 16 bytes each of
+// 8 rows of `out`, of which a wave writes 128 bytes (a lane per piece of ONE row made every lane of a load its own
+// line: 22 us for 50 MB of parts).
+constexpr int MERGE_THREADS = 256, MERGE_BATCH = 8;
+__global__ __launch_bounds__(MERGE_THREADS) void prefill_merge_kernel(PrefillArgs a) {
+    const uint32_t tok = blockIdx.x, kv = blockIdx.y, tile = tok / TQ, group = (tok % TQ) / 4;
+    const uint32_t ntiles = (a.tokens + TQ - 1) / TQ;
+    const uint32_t parts = (tile_blocks(a.pos, a.tokens, tile) + a.part_blocks - 1) / a.part_blocks;
+    const size_t item_stride = size_t(ntiles) * a.kv_heads, item0 = size_t(tile) * a.kv_heads + kv;
+    const uint32_t h = threadIdx.x & 7;
+#pragma unroll
+    for (int half = 0; half < 2; half++) {
+        const uint32_t piece = 32 * half + (threadIdx.x >> 3);       // dims 4 piece .. + 3 of the row
+        const uint32_t i = (piece >> 1) & 15, parity = piece >> 5;   // mt % 4 and q4; which half of the dims
+        const uint32_t col = (tok % 4) * 8 + h, lane = (piece & 1) * 32 + col;
+        const size_t row = size_t(tok) * a.heads + kv * SAETTA_GQA_GROUP + h;
+        const float4 g = *reinterpret_cast<const float4 *>(a.q_and_gate + row * 2 * DIM + DIM + 4 * piece);
+        const float *ml = a.part_ml + ((item0 * 4 + group) * 32 + col) * 2;
+        const float *po = a.part_o + (((item0 * WAVES + group * 2 + parity) * 16 + i) * 64 + lane) * 4;
+        // MERGE_BATCH parts at a time, all of their loads requested before the first is used (past the last part: the last
+        // part again, with no weight)
+        float m = 4.0f * NO_SCORE, l = 0.0f;
+        float4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (uint32_t p0 = 0; p0 < parts; p0 += MERGE_BATCH) {
+            float2 x[MERGE_BATCH];
+            float4 y[MERGE_BATCH];
+#pragma unroll
+            for (int j = 0; j < MERGE_BATCH; j++) {
+                const uint32_t p = min(p0 + j, parts - 1);
+                x[j] = *reinterpret_cast<const float2 *>(ml + p * item_stride * (4 * 32 * 2));
+                y[j] = *reinterpret_cast<const float4 *>(po + p * item_stride * (WAVES * 16 * 64 * 4));
+            }
+            float m_new = m;
+#pragma unroll
+            for (int j = 0; j < MERGE_BATCH; j++) m_new = fmaxf(m_new, x[j].x);
+            const float old = __builtin_amdgcn_exp2f(m - m_new);
+            m = m_new;
+            l *= old;
+            o.x *= old, o.y *= old, o.z *= old, o.w *= old;
+#pragma unroll
+            for (int j = 0; j < MERGE_BATCH; j++) {
+                const float now = p0 + j < parts ? __builtin_amdgcn_exp2f(x[j].x - m_new) : 0.0f;
+                l += x[j].y * now;
+                o.x += y[j].x * now, o.y += y[j].y * now, o.z += y[j].z * now, o.w += y[j].w * now;
+            }
+        }
+        const float inv = 1.0f / l;
+        float4 w;
+        w.x = o.x * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.x));
+        w.y = o.y * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.y));
+        w.z = o.z * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.z));
+        w.w = o.w * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.w));
+        *reinterpret_cast<float4 *>(a.out + row * DIM + 4 * piece) = w;
     }
 }
 
@@ -624,7 +749,71 @@ size_t images_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) {
     const size_t blocks = (size_t(pos) + tokens + BK - 1) / BK;
     return blocks * kv_heads * IMG_BYTES;
 }
-size_t workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) { return images_bytes(pos, tokens, kv_heads) + 256; }
+size_t plain_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) { return images_bytes(pos, tokens, kv_heads) + 256; }
+
+// Compute units of the current device.
+uint32_t cu_count() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
+        (void)hipGetLastError();
+        cus = 256;
+    }
+    return uint32_t(cus);
+}
+
+constexpr size_t PART_O_BYTES = size_t(TQ) * SAETTA_GQA_GROUP * DIM * 4, PART_ML_BYTES = size_t(TQ) * SAETTA_GQA_GROUP * 8;
+size_t parts_bytes(uint32_t tokens, uint32_t kv_heads, uint32_t nparts) {
+    return size_t((tokens + TQ - 1) / TQ) * kv_heads * nparts * (PART_O_BYTES + PART_ML_BYTES);
+}
+uint32_t parts_of(uint32_t pos, uint32_t tokens, uint32_t part_blocks) {
+    return (uint32_t((uint64_t(pos) + tokens + BK - 1) / BK) + part_blocks - 1) / part_blocks;
+}
+
+// Blocks of keys per part of a tile's keys, or 0: the keys are not split.  A tile is one workgroup's work, and 16 tokens
+// of 2 kv heads are all a CU gets of it: chunks under 2048 tokens leave CUs idle, and between 2048 and 4096 a second round
+// of tiles fills a part of them.  The rule takes the smallest of what the rounds of workgroups would take, in us, out of
+// 1 to 32 parts, from figures measured on the MI355X: a workgroup's block of 32 keys takes 0.6 us while the chip has
+// power to spare (up to ~170 workgroups) and the chip as a whole 284 blocks a us beyond that; the ends of an item (its
+// first loads, the store of its part) 12 us, with the gate 14.5; the merge a launch and 128 KB read back per item.
+// Measured, unsplit -> split by this rule, the whole call (8-bit cache): 100 tokens at 10000: 211 -> 47 us, at 100000
+// (4-bit): 1886 -> 225; 500 at 40000: 770 -> 330; 2100 at 9000: 497 -> 405.  A full chunk (4096 tokens: two whole rounds)
+// is never split.
+uint32_t choose_part_blocks(uint32_t pos, uint32_t tokens, uint32_t kv_heads, uint32_t cus) {
+    constexpr float BLOCK_US = 0.6f, CHIP_BLOCKS_PER_US = 284.0f / 256.0f, PART_US = 12.0f, TILE_US = 14.5f, MERGE_US = 4.0f, MERGE_ITEM_US = 0.03f;
+    const uint32_t ntiles = (tokens + TQ - 1) / TQ;
+    const uint32_t longest = tile_blocks(pos, tokens, ntiles - 1), shortest = tile_blocks(pos, tokens, 0);
+    const float per_us = CHIP_BLOCKS_PER_US * float(cus);
+    // n items in order of length, from `high` down to `low` blocks, handed out one by one
+    auto rounds_us = [&](uint32_t n, float high, float low, float ends_us) {
+        float us = 0.0f, at = 0.0f;
+        for (uint32_t left = n; left > 0;) {
+            const uint32_t now = left < cus ? left : cus;
+            const float mid = high - (high - low) * (at + 0.5f * float(now)) / float(n);  // mean length of the round's items
+            const float alone = mid * BLOCK_US, shared = mid * float(now) / per_us;
+            us += (alone > shared ? alone : shared) + ends_us;
+            at += float(now), left -= now;
+        }
+        const float one = high * BLOCK_US + ends_us;
+        return us > one ? us : one;
+    };
+    float best = 0.95f * rounds_us(ntiles * kv_heads, float(longest), float(shortest), TILE_US);
+    uint32_t part_blocks = 0;
+    for (uint32_t parts = 2; parts <= 32; parts++) {
+        const uint32_t pb = ((longest + parts - 1) / parts + 1) / 2 * 2;  // (a step of the kernel is two blocks)
+        if (pb < 4 || pb >= longest) continue;
+        const uint32_t items = prefill_items(pos, tokens, pb) * kv_heads;
+        const float mid = 0.5f * float(longest + shortest) * float(ntiles * kv_heads) / float(items);
+        const float us = rounds_us(items, mid, mid, PART_US) + MERGE_US + MERGE_ITEM_US * float(items);
+        if (us < best) best = us, part_blocks = pb;
+    }
+    return part_blocks;
+}
+size_t workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) {
+    size_t n = plain_workspace_bytes(pos, tokens, kv_heads);
+    if (tokens == 0 || kv_heads == 0) return n;
+    if (const uint32_t pb = choose_part_blocks(pos, tokens, kv_heads, cu_count())) n += parts_bytes(tokens, kv_heads, parts_of(pos, tokens, pb));
+    return n;
+}
 
 // The checks both prefill paths share.
 int check_prefill(int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
@@ -707,21 +896,31 @@ int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kda
     const uint64_t rows = uint64_t(p.pos) + p.tokens;
     if (int rc = ensure_device()) return rc;
     if (p.tokens == 0) return SAETTA_OK;
-    const size_t need = workspace_bytes(p.pos, p.tokens, p.kv_heads);
+    const uint32_t cus = cu_count();
+    uint32_t part_blocks = choose_part_blocks(p.pos, p.tokens, p.kv_heads, cus);
+    const size_t plain = plain_workspace_bytes(p.pos, p.tokens, p.kv_heads);
+    const uint32_t nparts = part_blocks ? parts_of(p.pos, p.tokens, part_blocks) : 0;
+    size_t need = plain + parts_bytes(p.tokens, p.kv_heads, nparts);
+    // A workspace that holds the images and no parts (one made for a longer chunk, say): the keys are not split.
+    if (workspace && workspace_size < need) part_blocks = 0, need = plain;
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
     if (int rc = acquire_workspace(stream, workspace, workspace_size, need, owned_lock, what, "saetta_prefill_workspace_bytes")) return rc;
-    uint32_t *tiles_taken = reinterpret_cast<uint32_t *>(static_cast<unsigned char *>(workspace) + images_bytes(p.pos, p.tokens, p.kv_heads));
+    unsigned char *ws = static_cast<unsigned char *>(workspace);
+    uint32_t *tiles_taken = reinterpret_cast<uint32_t *>(ws + images_bytes(p.pos, p.tokens, p.kv_heads));
     const uint32_t nblocks = launch_prepare(stream, bits, kdata, vdata, ks, kz, vs, vz, workspace, p.kv_heads, rows, tiles_taken);
+    float *part_o = reinterpret_cast<float *>(ws + plain);
+    float *part_ml = reinterpret_cast<float *>(ws + plain + size_t(nparts) * ((p.tokens + TQ - 1) / TQ) * p.kv_heads * PART_O_BYTES);
     PrefillArgs a{q, static_cast<const unsigned char *>(workspace), q_and_gate, out, p.heads, p.kv_heads, p.pos,
-                  p.tokens, p.scale, nblocks, tiles_taken};
+                  p.tokens, p.scale, nblocks, tiles_taken, part_blocks, part_o, part_ml};
     // one workgroup per CU at most: a workgroup's LDS ring fills a CU, and further tiles are taken in the kernel
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
-        (void)hipGetLastError();
-        cus = 256;
+    if (part_blocks) {
+        const uint32_t total = prefill_items(p.pos, p.tokens, part_blocks) * p.kv_heads;
+        attention_prefill_kernel<true><<<dim3(total < cus ? total : cus), THREADS, LDS_BYTES, stream>>>(a);
+        prefill_merge_kernel<<<dim3(p.tokens, p.kv_heads), MERGE_THREADS, 0, stream>>>(a);
+    } else {
+        const uint32_t total = (p.tokens + TQ - 1) / TQ * p.kv_heads;
+        attention_prefill_kernel<false><<<dim3(total < cus ? total : cus), THREADS, LDS_BYTES, stream>>>(a);
     }
-    const uint32_t total = (p.tokens + TQ - 1) / TQ * p.kv_heads;
-    attention_prefill_kernel<<<dim3(total < uint32_t(cus) ? total : uint32_t(cus)), THREADS, LDS_BYTES, stream>>>(a);
     return launch_status(what);
 }
 
@@ -1152,10 +1351,13 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
 }  // namespace
 
 int setup_prefill() {
-    if (int rc = load_kernel(reinterpret_cast<const void *>(attention_prefill_kernel))) return rc;
+    if (int rc = load_kernel(reinterpret_cast<const void *>(attention_prefill_kernel<false>))) return rc;
+    if (int rc = load_kernel(reinterpret_cast<const void *>(prefill_merge_kernel))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_scores_kernel))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_pv_kernel))) return rc;
-    return int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_prefill_kernel),
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_prefill_kernel<true>),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES))) return rc;
+    return int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_prefill_kernel<false>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
 }
 }  // namespace saetta

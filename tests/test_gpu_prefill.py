@@ -237,3 +237,32 @@ def test_chunk_from_a_position_that_splits_a_row_group(kind, pos):
     want = oracle.prefill(q16.astype(np.float32), kf, vf, pos, tokens, q_and_gate=qg, threads=8)
     assert oracle.rel_rms(got, want) < REL_RMS
     assert np.abs(got - want).max() < MAX_ABS
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("pos,tokens", [(250, 16), (1018, 20), (2040, 33), (5000, 7), (9985, 50)])
+def test_keys_in_parts(kind, pos, tokens):
+    # Few tokens behind a long prefix: a tile's keys go to several workgroups and a second kernel joins the parts.
+    # (250, 16) is next to the smallest split, (1018, 20) and (2040, 33) have tiles whose tokens cross a key block where
+    # parts end (rows that see nothing of the last part), (9985, 50) the most parts and a ragged last tile.
+    rng = np.random.default_rng(pos)
+    n = pos + tokens
+    k = rng.standard_normal((n, VALUES)).astype(np.float32)
+    v = rng.standard_normal((n, VALUES)).astype(np.float32)
+    q16 = rng.standard_normal((tokens, H, D)).astype(np.float16)
+    qg = rng.standard_normal((tokens, H, 2 * D)).astype(np.float32)
+    kc, vc, kf, vf = make_cache(kind, k, v, n + 5, chunk_from=pos)
+    want = oracle.prefill(q16.astype(np.float32), kf, vf, pos, tokens, q_and_gate=qg, threads=8)
+    p = saetta.FlashParams(H, KV, pos, tokens, 1.0 / math.sqrt(D))
+    images = saetta.ffi.lib().saetta_prefill_workspace_bytes(0, -(-n // 32) * 32, KV)  # of one tile-aligned chunk: no parts
+    for nbytes in (saetta.attention_prefill.workspace_bytes(p), images):  # and a workspace that holds no parts
+        ws = torch.full((nbytes,), 0xff, dtype=torch.uint8, device="cuda")
+        out = torch.full((tokens, H, D), float("nan"), device="cuda")
+        if kind is saetta.KvBits.Half:
+            saetta.attention_prefill.encode(saetta.attention_prefill.DEFAULT, dev(q16), kc, vc, dev(qg), out, p, workspace=ws)
+        else:
+            saetta.attention_prefill.encode_quant(dev(q16), kc, vc, dev(qg), out, p, workspace=ws)
+        got = host(out)
+        assert np.isfinite(got).all()
+        assert oracle.rel_rms(got, want) < REL_RMS
+        assert np.abs(got - want).max() < MAX_ABS
