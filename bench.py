@@ -50,8 +50,7 @@ MFMA_F16_PEAK_TFLOPS = 2500.0
 # the runs are summarised in profiles/*_hbm_traffic.txt).  Counters cannot be read inside this
 # script, so the figures are carried here for the workloads they were measured on.
 MEASURED_TRAFFIC = {"decode8_32k": 38.2e6, "prefill": 421.5e6, "decode4_150k": 88.9e6, "verify4": 45.0e6,
-                    "deltanet_prefill": 664.1e6,  # (the three kernels of the chunk together)
-                    "prefill_gemm": 2.18e9}       # (the 2 launches of a call together)
+                    "deltanet_prefill": 664.1e6}  # (the three kernels of the chunk together)
 
 
 def median(xs):
@@ -381,8 +380,8 @@ def bench_reader_floor(s, torch, args, ctx=32768, layers=32):
 
 
 def bench_prefill(s, torch, args, tokens=4096, pos=4096, bits=8, gemm=False):
-    """gemm: the same chunk by AttGemm (src/attention_gemm.rs), block by block of 1024 keys with the block's
-    probabilities written out and read back, instead of the flash kernel."""
+    """gemm: the same chunk through AttGemm (src/attention_gemm.rs), the reference's other route to the same result; its
+    whole call takes the same kernels here."""
     import numpy as np
     import oracle  # CPU-baseline leg only
 
@@ -436,7 +435,7 @@ def bench_prefill(s, torch, args, tokens=4096, pos=4096, bits=8, gemm=False):
     achieved = flops / (kern_us * 1e-6) / 1e12
     roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": MFMA_F16_PEAK_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(achieved / MFMA_F16_PEAK_TFLOPS, 4),
-                "traffic": MEASURED_TRAFFIC.get("prefill") if (tokens, pos, bits, gemm) == (4096, 4096, 8, False) else None,
+                "traffic": MEASURED_TRAFFIC.get("prefill") if (tokens, pos, bits) == (4096, 4096, 8) else None,
                 "kernel": "attention_prefill_kernel", "avg_us": round(kern_us, 2)}
     if not gemm and not args.no_reader_floor:
         # what the kernel's own MFMA streams reach with no softmax, prologue or epilogue around them
@@ -444,22 +443,6 @@ def bench_prefill(s, torch, args, tokens=4096, pos=4096, bits=8, gemm=False):
         stream_only = floor["the prefill kernel's streams (LDS fragment reads, copies, barrier), no softmax"]["TFLOP/s"]
         roofline["mfma_streams_alone"] = floor
         roofline["frac_of_streams_alone"] = round(achieved / stream_only, 4)
-    if gemm:
-        # What bounds this route is the scratch it writes and reads back.  Algorithmic bytes per query row: 2 B out
-        # and 2 B in per key its 16-token tile sees (in whole tiles of 32 keys), and a maximum and a sum (8 B)
-        # out and in per tile of 32 keys; per span of eight blocks of 1024 keys it touches, its q twice (one read
-        # per part of the span's tiles: two at this chunk length) and 1 KB of output sums in and 1 KB out.
-        nbytes = 0
-        for t0 in range(0, tokens, 16):
-            last_key = pos + min(t0 + 16, tokens) - 1
-            rows = (min(t0 + 16, tokens) - t0) * H
-            nbytes += rows * ((last_key // 32 + 1) * (32 * 4 + 16) + (last_key // 8192 + 1) * 3072)
-        gbs = nbytes / (kern_us * 1e-6) / 1e9
-        roofline = {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                    "frac": round(gbs / HBM_PEAK_GBS, 4),
-                    "traffic": MEASURED_TRAFFIC.get("prefill_gemm") if (tokens, pos, bits) == (4096, 4096, 8) else None,
-                    "kernel": "attention_gemm_scores_kernel + attention_gemm_pv_kernel", "avg_us": round(kern_us, 2),
-                    "bytes": nbytes, "mfma_TFLOPs": round(achieved, 2), "mfma_frac": round(achieved / MFMA_F16_PEAK_TFLOPS, 4)}
     # CPU baseline on a bounded sample: the last `sample` tokens of the chunk (the longest rows).
     sample = max(16, 512 * 8192 // (pos + tokens))  # 512 tokens at the headline shape: about 7 s on one core
     groups = (pos + tokens) * 8
@@ -486,11 +469,10 @@ def bench_prefill(s, torch, args, tokens=4096, pos=4096, bits=8, gemm=False):
         "dtype": "f16 MFMA, f32 softmax state",
         "config": {"workload": f"causal prefill chunk of {tokens} tokens at position {pos}, {bits}-bit KV cache "
                                "read in place, chunk K/V quantized on append inside the step"
-                               + (", attention as matrix products over blocks of 1024 keys (AttGemm)" if gemm else ""),
+                               + (", through AttGemm" if gemm else ""),
                    "heads": H, "kv_heads": KV, "head_dim": D, "flops": flops,
                    "timing": "value: wall time of steps (2 x kv_quantize of the chunk + prepare + attention); "
-                             "roofline: median of event-timed prepare + attention calls"
-                             + (f" ({2 * -(-(pos + tokens) // 8192)} launches: scores and pv per span of eight blocks of 1024 keys)" if gemm else ""),
+                             "roofline: median of event-timed prepare + attention calls",
                    "inputs": "q (through bf16), K, V, gate ~ N(0,1) from torch's device generator (Philox, seed 99)"},
         "roofline": roofline,
         "cpu_baseline": {"value": round(cpu_flops / cpu_s / 1e12, 6), "unit": "TFLOP/s", "cores": 1, "kind": "port",

@@ -404,8 +404,11 @@ int saetta_deltanet_rows_fused(saetta_stream_t stream, const float *x, const flo
 
 /* ---- prefill attention (src/attention_prefill.rs, src/prefill.rs) ---------- */
 
-/* Bytes of workspace a prefill chunk at (pos, tokens) needs: the f16 key and
- * value tile images of the pos + tokens rows the chunk can see.  The reference
+/* Bytes of workspace a prefill chunk at (pos, tokens) wants: the f16 key and
+ * value tile images of the pos + tokens rows the chunk can see and, for a chunk with too few
+ * tokens to fill the GPU, room for partial results of parts of the keys (up to 32 parts of
+ * 1 KB + 8 B per query row).  A call given the images' part only (one sized for
+ * another chunk of as many rows) runs too, without the split.  The reference
  * has no counterpart (its kernels dequantize in place); the closest is the
  * half scratch of Prefill::new (src/prefill.rs:1674-1686). */
 size_t saetta_prefill_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads);
@@ -414,8 +417,8 @@ size_t saetta_prefill_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv
  * over a half cache that already holds the chunk's rows.  q f16
  * [tokens][heads][256]; keys, values f16 [capacity][kv_heads][256] from
  * position 0, capacity >= pos + tokens; q_and_gate f32 [tokens][heads][512];
- * out f32 [tokens][heads][256].  workspace: device memory of at least
- * saetta_prefill_workspace_bytes(pos, tokens, kv_heads) bytes, 16-byte
+ * out f32 [tokens][heads][256].  workspace: device memory of
+ * saetta_prefill_workspace_bytes(pos, tokens, kv_heads) bytes (at least the images), 16-byte
  * aligned, overwritten by the call; NULL makes the library use one of its own
  * per device and stream, which it grows with hipMalloc when needed (so not
  * under stream capture) and keeps until the process ends.  Kernel replaced:
@@ -439,25 +442,25 @@ int saetta_attn_prefill_quant(saetta_stream_t stream, int bits, const uint16_t *
 /* attention_gemm::KEYS (src/attention_gemm.rs:28): keys per block. */
 #define SAETTA_AG_KEYS 1024
 
-/* Bytes of workspace AttGemm needs for a chunk at (pos, tokens) run in slices
+/* Bytes of workspace AttGemm needs for a chunk at (pos, tokens) whose passes run in slices
  * of up to slice_tokens tokens (0: one slice): the key and value tile images
  * of saetta_prefill_workspace_bytes, then what AttGemm::new allocates for one
  * slice (src/attention_gemm.rs:118-142): the probabilities of eight blocks of
- * keys (a pair of launches takes eight blocks, so that q and the output sums
- * go through memory once per eight), the tile maxima and sums, the output sums
+ * keys, the tile maxima and sums, the output sums
  * and the per-row softmax state; about 19 KB per query row of a slice. */
 size_t saetta_attn_gemm_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t slice_tokens,
                                         uint32_t kv_heads);
 
 /* AttGemm::encode (src/attention_gemm.rs:144-188, encode_slice :190-364), the
- * default (fused) variant: the same chunk and the same buffers as
- * saetta_attn_prefill / saetta_attn_prefill_quant, computed block by block of
- * SAETTA_AG_KEYS keys with the block's probabilities written out and read
- * back.  bits 16: keys.data and values.data are the half caches and the scales
+ * default (fused) variant: the same chunk, the same buffers and the same result as
+ * saetta_attn_prefill / saetta_attn_prefill_quant.  stages (AttGemm::stages,
+ * src/attention_gemm.rs:112-114): 0 gives the outputs, by the kernels of saetta_attn_prefill,
+ * which are the faster way to them at every size; 1, 2 and 3 run the passes of the blocked
+ * form and write no outputs, to time them: block by block of SAETTA_AG_KEYS keys, the block's
+ * probabilities written out (1 or 2: only this) and read back into the second product (3).
+ * bits 16: keys.data and values.data are the half caches and the scales
  * and biases are not read (the reference's quant = None); bits 8 or 4: the
- * quantized rows, seen through half.  stages (AttGemm::stages,
- * src/attention_gemm.rs:112-114): 0 runs everything; 1 or 2 only the scores
- * pass of each block; 3 scores and pv and no outputs.  workspace as for
+ * quantized rows, seen through half.  workspace as for
  * saetta_attn_prefill, of saetta_attn_gemm_workspace_bytes bytes.  Kernels
  * replaced: prefill_ag_scores_t{,_q8,_q4}, prefill_ag_pv_t{,_q8,_q4},
  * prefill_ag_final (kernels/attention_gemm.metal). */

@@ -11,8 +11,8 @@
 // cache is seen "through half": every value is f16(f32(s)*code + f32(z)),
 // exactly what round_trip_as_half (src/kv_quant.rs:119-125) gives the CPU path.
 //
-// Two kernels (and, further down, the reference's other route to the same output, AttGemm of
-// src/attention_gemm.rs: two more kernels on the same images, block by block of 1024 keys).
+// Two kernels, and a third where a tile's keys are taken in parts (further down: the passes of the reference's other
+// route to the same output, AttGemm of src/attention_gemm.rs, on the same images, block by block of 1024 keys).
 //
 // prefill_prepare_kernel<16|8|4> turns the keys and values the chunk can see into
 // f16 tile images in a workspace, one image per (kv head, block of 32 keys): the K tile
@@ -808,13 +808,6 @@ uint32_t choose_part_blocks(uint32_t pos, uint32_t tokens, uint32_t kv_heads, ui
     }
     return part_blocks;
 }
-size_t workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) {
-    size_t n = plain_workspace_bytes(pos, tokens, kv_heads);
-    if (tokens == 0 || kv_heads == 0) return n;
-    if (const uint32_t pb = choose_part_blocks(pos, tokens, kv_heads, cu_count())) n += parts_bytes(tokens, kv_heads, parts_of(pos, tokens, pb));
-    return n;
-}
-
 // The checks both prefill paths share.
 int check_prefill(int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
                   const uint16_t *kz, const uint16_t *vs, const uint16_t *vz, const float *q_and_gate, const float *out,
@@ -888,40 +881,66 @@ uint32_t launch_prepare(hipStream_t stream, int bits, const void *kdata, const v
     return nblocks;
 }
 
+// What a chunk needs of a workspace, and how its keys are split.
+struct FlashPlan {
+    uint32_t cus, part_blocks, nparts;
+    size_t plain, parts;  // bytes: the images and the tile count; the parts behind them
+    size_t bytes() const { return plain + parts; }
+};
+FlashPlan flash_plan(const saetta_flash_params &p) {
+    FlashPlan f{};
+    f.cus = cu_count();
+    f.plain = plain_workspace_bytes(p.pos, p.tokens, p.kv_heads);
+    if (p.tokens && p.kv_heads) f.part_blocks = choose_part_blocks(p.pos, p.tokens, p.kv_heads, f.cus);
+    if (f.part_blocks) {
+        f.nparts = parts_of(p.pos, p.tokens, f.part_blocks);
+        f.parts = parts_bytes(p.tokens, p.kv_heads, f.nparts);
+    }
+    return f;
+}
+
+size_t workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) {
+    return flash_plan(saetta_flash_params{0, kv_heads, pos, tokens, 0.0f}).bytes();
+}
+
+// The launches of a chunk in a workspace of at least plan.plain bytes, plan.bytes() with `split`.
+int launch_flash(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
+                 const uint16_t *kz, const uint16_t *vs, const uint16_t *vz, const float *q_and_gate, float *out,
+                 const saetta_flash_params &p, void *workspace, bool split, const FlashPlan &plan, const char *what) {
+    const uint64_t rows = uint64_t(p.pos) + p.tokens;
+    unsigned char *ws = static_cast<unsigned char *>(workspace);
+    uint32_t *tiles_taken = reinterpret_cast<uint32_t *>(ws + images_bytes(p.pos, p.tokens, p.kv_heads));
+    const uint32_t nblocks = launch_prepare(stream, bits, kdata, vdata, ks, kz, vs, vz, workspace, p.kv_heads, rows, tiles_taken);
+    const uint32_t ntiles = (p.tokens + TQ - 1) / TQ;
+    PrefillArgs a{q, ws, q_and_gate, out, p.heads, p.kv_heads, p.pos, p.tokens, p.scale, nblocks, tiles_taken, 0, nullptr, nullptr};
+    // one workgroup per CU at most: a workgroup's LDS ring fills a CU, and further tiles are taken in the kernel
+    if (split && plan.part_blocks) {
+        a.part_blocks = plan.part_blocks;
+        a.part_o = reinterpret_cast<float *>(ws + plan.plain);
+        a.part_ml = reinterpret_cast<float *>(ws + plan.plain + size_t(plan.nparts) * ntiles * p.kv_heads * PART_O_BYTES);
+        const uint32_t total = prefill_items(p.pos, p.tokens, plan.part_blocks) * p.kv_heads;
+        attention_prefill_kernel<true><<<dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream>>>(a);
+        prefill_merge_kernel<<<dim3(p.tokens, p.kv_heads), MERGE_THREADS, 0, stream>>>(a);
+    } else {
+        const uint32_t total = ntiles * p.kv_heads;
+        attention_prefill_kernel<false><<<dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream>>>(a);
+    }
+    return launch_status(what);
+}
+
 int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata,
                 const uint16_t *ks, const uint16_t *kz, const uint16_t *vs, const uint16_t *vz,
                 const float *q_and_gate, float *out, saetta_flash_params p, void *workspace, size_t workspace_size,
                 const char *what) {
     if (int rc = check_prefill(bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, what)) return rc;
-    const uint64_t rows = uint64_t(p.pos) + p.tokens;
     if (int rc = ensure_device()) return rc;
     if (p.tokens == 0) return SAETTA_OK;
-    const uint32_t cus = cu_count();
-    uint32_t part_blocks = choose_part_blocks(p.pos, p.tokens, p.kv_heads, cus);
-    const size_t plain = plain_workspace_bytes(p.pos, p.tokens, p.kv_heads);
-    const uint32_t nparts = part_blocks ? parts_of(p.pos, p.tokens, part_blocks) : 0;
-    size_t need = plain + parts_bytes(p.tokens, p.kv_heads, nparts);
-    // A workspace that holds the images and no parts (one made for a longer chunk, say): the keys are not split.
-    if (workspace && workspace_size < need) part_blocks = 0, need = plain;
+    const FlashPlan plan = flash_plan(p);
+    size_t need = plan.bytes();
+    if (workspace && workspace_size < need) need = plan.plain;  // (room for the images only: the keys are not split)
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
     if (int rc = acquire_workspace(stream, workspace, workspace_size, need, owned_lock, what, "saetta_prefill_workspace_bytes")) return rc;
-    unsigned char *ws = static_cast<unsigned char *>(workspace);
-    uint32_t *tiles_taken = reinterpret_cast<uint32_t *>(ws + images_bytes(p.pos, p.tokens, p.kv_heads));
-    const uint32_t nblocks = launch_prepare(stream, bits, kdata, vdata, ks, kz, vs, vz, workspace, p.kv_heads, rows, tiles_taken);
-    float *part_o = reinterpret_cast<float *>(ws + plain);
-    float *part_ml = reinterpret_cast<float *>(ws + plain + size_t(nparts) * ((p.tokens + TQ - 1) / TQ) * p.kv_heads * PART_O_BYTES);
-    PrefillArgs a{q, static_cast<const unsigned char *>(workspace), q_and_gate, out, p.heads, p.kv_heads, p.pos,
-                  p.tokens, p.scale, nblocks, tiles_taken, part_blocks, part_o, part_ml};
-    // one workgroup per CU at most: a workgroup's LDS ring fills a CU, and further tiles are taken in the kernel
-    if (part_blocks) {
-        const uint32_t total = prefill_items(p.pos, p.tokens, part_blocks) * p.kv_heads;
-        attention_prefill_kernel<true><<<dim3(total < cus ? total : cus), THREADS, LDS_BYTES, stream>>>(a);
-        prefill_merge_kernel<<<dim3(p.tokens, p.kv_heads), MERGE_THREADS, 0, stream>>>(a);
-    } else {
-        const uint32_t total = (p.tokens + TQ - 1) / TQ * p.kv_heads;
-        attention_prefill_kernel<false><<<dim3(total < cus ? total : cus), THREADS, LDS_BYTES, stream>>>(a);
-    }
-    return launch_status(what);
+    return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, need >= plan.bytes(), plan, what);
 }
 
 // ---- the same chunk as matrix products over blocks of 1024 keys ---------------------------------
@@ -932,6 +951,11 @@ int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kda
 // each tile of keys, with the tile's maximum and sum beside them, and a second launch folds the block
 // into the running (m, l, O) of every row: O = alpha O + sum over tiles of e^(t - m) (P_tile V_tile).
 // The scratch is for one slice of the chunk's tokens; the slices run one after the other.
+//
+// A whole call (stages 0) does NOT take these passes: what they compute is what attention_prefill_kernel computes, and it
+// needs no trip of the probabilities through memory (2048 tokens at 118784, half cache: 5.98 ms by the passes, scores 2.7
+// + pv 3.2, against 3.6 ms; 64 to 4096 tokens at 0 to 130000: 1.6 to 4 times).  The passes run where a caller asks
+// for them by number (stages 1 to 3), to see what the scores and the second product take by themselves.
 //
 // Here the pair of launches takes a span of AG_SPAN blocks (the scratch holds that many blocks'
 // probabilities: q and the output sums then go through memory once per span, and there are as many times
@@ -944,8 +968,7 @@ int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kda
 //            stored as the P^T operands of the second product (the accumulator's registers 8 sp .. 8 sp + 7
 //            are the operand of k-step sp: 1 KB per wave and k-step, read back as it was written);
 //   pv       m' = max(m, max_t t), O^T = alpha O^T + sum_t V^T_t (f_t P^T_t) with f_t = 2^(t - m') rounded
-//            to f16 (the row sum takes the same rounded f_t); the span that holds a tile's last visible
-//            key writes out = O / l * sigmoid(gate) instead of O.
+//            to f16 (the row sum takes the same rounded f_t).  O, m and l stay in the scratch.
 constexpr int AG_KEYS = SAETTA_AG_KEYS;
 constexpr int AG_TILES = AG_KEYS / BK;
 constexpr int AG_SPAN = 8;                // blocks that one pair of launches takes
@@ -960,8 +983,6 @@ constexpr int AG_P_TILE_BYTES = BK * 32 * 2;  // the P^T operands of one row gro
 struct GemmArgs {
     const uint16_t *q;
     const unsigned char *images;
-    const float *q_and_gate;
-    float *out;
     unsigned char *p;    // f16 [kv head][token tile][tile of keys][row group of the token tile][2 k-steps][64 lanes][8]
     float *tmax, *tsum;  // [kv head][token tile][tile of keys][row group of the token tile][32 rows], log2 domain
     float *o;            // [kv head][row group][8 dim tiles][4][64 lanes][4]: the accumulators as they are
@@ -972,7 +993,6 @@ struct GemmArgs {
     uint32_t row_groups; // per kv head in the scratch
     uint32_t g0;         // the first key of the span of blocks the launch takes
     uint32_t split;      // scores: workgroups that share a span's tiles for one token tile (a power of two)
-    uint32_t write_out;  // 0: the outputs are never written (timing the passes apart)
 };
 
 // Key of the last token of a token tile of `span` tokens at tok0, and how many of the tiles of the launch's span
@@ -1142,9 +1162,7 @@ __global__ __launch_bounds__(AG_THREADS, 2) void attention_gemm_pv_kernel(GemmAr
     const uint32_t tok0 = blockIdx.y * AG_TOKENS, kv = blockIdx.z;
     const uint32_t need = ag_tiles(a, tok0);
     if (need == 0) return;  // nothing of this span (the outputs were written at an earlier one)
-    const bool last_block = ag_last_key(a, tok0) < a.g0 + AG_SPAN * AG_KEYS;
     const uint32_t rg = blockIdx.y * AG_WAVES + wave;
-    const uint32_t tok = tok0 + 4 * wave + (col >> 3), head = kv * SAETTA_GQA_GROUP + (col & 7);
     const size_t rows = size_t(kv) * a.row_groups + rg;
     const size_t state = rows * 32 + col;
     const bool first_block = a.g0 == 0;
@@ -1237,30 +1255,6 @@ __global__ __launch_bounds__(AG_THREADS, 2) void attention_gemm_pv_kernel(GemmAr
     if (t < need) tile(pre[0], t);
     const float l_new = alpha * l_old + lsum;
 
-    if (last_block && a.write_out) {
-        if (tok < a.tokens) {
-            const float inv = 1.0f / l_new;
-            const size_t row = size_t(tok) * a.heads + head;
-#pragma unroll
-            for (int dh = 0; dh < 2; dh++) {  // (half of the dims at a time: 16 gate loads in flight)
-                const float *gate = a.q_and_gate + row * 2 * DIM + DIM + 128 * dh + 4 * hf;
-                float *out = a.out + row * DIM + 128 * dh + 4 * hf;
-                floatx4 g[16];
-#pragma unroll
-                for (int i = 0; i < 16; i++) g[i] = *reinterpret_cast<const floatx4 *>(gate + 32 * (i >> 2) + 8 * (i & 3));
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int mt = 4 * dh + (i >> 2), q4 = i & 3;
-                    floatx4 w;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) w[e] = acc[mt][4 * q4 + e] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i][e]));
-                    *reinterpret_cast<floatx4 *>(out + 32 * (i >> 2) + 8 * q4) = w;
-                }
-                asm volatile("" ::: "memory");
-            }
-        }
-        return;
-    }
     if (hf == 0) a.m[state] = m_new, a.l[state] = l_new;
 #pragma unroll
     for (int mt = 0; mt < 8; mt++)
@@ -1290,8 +1284,11 @@ uint32_t gemm_slice(uint32_t tokens, uint32_t slice_tokens) {
     return slice_tokens == 0 || slice_tokens > tokens ? tokens : slice_tokens;
 }
 
+// The images and the passes' scratch, or the images and the parts of the flash kernel's keys: what is more.
 size_t gemm_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t slice_tokens, uint32_t kv_heads) {
-    return align_up(workspace_bytes(pos, tokens, kv_heads), 256) + gemm_scratch_bytes(gemm_slice(tokens, slice_tokens), kv_heads);
+    const size_t passes = align_up(plain_workspace_bytes(pos, tokens, kv_heads), 256) + gemm_scratch_bytes(gemm_slice(tokens, slice_tokens), kv_heads);
+    const size_t flash = workspace_bytes(pos, tokens, kv_heads);
+    return passes > flash ? passes : flash;
 }
 
 int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
@@ -1307,10 +1304,12 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
     const size_t need = gemm_workspace_bytes(p.pos, p.tokens, slice, p.kv_heads);
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
     if (int rc = acquire_workspace(stream, workspace, workspace_size, need, owned_lock, what, "saetta_attn_gemm_workspace_bytes")) return rc;
+    // All of the call: the flash kernel's result is the same and it is there in 0.5 to 0.6 of the time (see above).
+    if (stages == 0) return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, true, flash_plan(p), what);
     const uint32_t nblocks = launch_prepare(stream, bits, kdata, vdata, ks, kz, vs, vz, workspace, p.kv_heads, rows);
 
     const size_t groups = gemm_row_groups(slice) * p.kv_heads;
-    unsigned char *at = static_cast<unsigned char *>(workspace) + align_up(workspace_bytes(p.pos, p.tokens, p.kv_heads), 256);
+    unsigned char *at = static_cast<unsigned char *>(workspace) + align_up(plain_workspace_bytes(p.pos, p.tokens, p.kv_heads), 256);
     GemmArgs a{};
     a.images = static_cast<const unsigned char *>(workspace);
     a.p = at, at += groups * AG_SPAN_TILES * AG_P_TILE_BYTES;
@@ -1323,14 +1322,13 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
     a.c = p.scale * 1.4426950408889634f;
     a.nblocks = nblocks;
     a.row_groups = uint32_t(gemm_row_groups(slice));
-    a.write_out = stages == 0;
     const size_t width = size_t(p.heads) * DIM;
     // A slice of tokens is a chunk of its own at pos + t0: its rows of q, q_and_gate and out, the whole
     // cache (src/attention_gemm.rs:162-188).
     for (uint32_t t0 = 0; t0 < p.tokens; t0 += slice) {
         a.tokens = p.tokens - t0 < slice ? p.tokens - t0 : slice;
         a.pos = p.pos + t0;
-        a.q = q + t0 * width, a.q_and_gate = q_and_gate + t0 * width * 2, a.out = out + t0 * width;
+        a.q = q + t0 * width;
         const uint32_t tiles = (a.tokens + AG_TOKENS - 1) / AG_TOKENS;
         const uint64_t end = uint64_t(a.pos) + a.tokens;
         // scores: as many workgroups per token tile as make AG_WGS in all (2 for chunks of 4096 tokens, 4 for 2048)

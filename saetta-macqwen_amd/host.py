@@ -866,8 +866,8 @@ class attention_gemm:
         tokens of a chunk, and `encode`.  Only the reference's default variant exists here (`fused` and
         `texp` both true: the scores pass writes the probabilities relative to each tile's maximum and the
         tiles' sums, the pv pass scales a tile once); SAETTA_AG_FUSED=0 or SAETTA_AG_TEXP=0 raise.
-        `stages` as in the reference's bench: 0 all passes, 1 or 2 scores only, 3 scores and pv and no
-        outputs."""
+        `stages`: 0 gives the outputs (by the flash kernel, which is the faster way to them); as in the
+        reference's bench 1 or 2 run the scores pass only, 3 scores and pv, both without outputs."""
 
         def __init__(self, chunk, kv_heads, device="cuda"):
             import os
@@ -913,7 +913,8 @@ class attention_gemm:
     def bench(contexts, chunk, layers, device="cuda"):
         """bench (src/attention_gemm.rs:366-470): for each context the chunk of `chunk` tokens at its end and
         at its middle through attention_prefill.encode_rows2 and through AttGemm, best of 3 after a warm-up;
-        the gemm passes of the last chunk one by one as differences of runs that stop early; the largest and
+        the gemm passes of the last chunk one by one as differences of runs that stop early (a whole call does not
+        take them, so what it has over them, final_ms, is 0 where it is the faster); the largest and
         the rms relative difference of the two outputs.  One dict per context."""
         heads, kv, dim = 16, 2, DIM
         gemm = attention_gemm.AttGemm(chunk, kv, device)
@@ -969,7 +970,7 @@ class attention_gemm:
             row["stages"] = {"scores_ms": prefix[1], "scores_TFLOP/s": flops(last) / 2 / prefix[1] / 1e9,
                              "softmax_ms": prefix[2] - prefix[1], "pv_ms": prefix[3] - prefix[2],
                              "pv_TFLOP/s": flops(last) / 2 / max(prefix[3] - prefix[2], 1e-9) / 1e9,
-                             "final_ms": whole - prefix[3]}
+                             "final_ms": max(0.0, whole - prefix[3])}
             # both outputs are now of the last chunk
             best_ms(False, last)
             diff = (want - got).double()

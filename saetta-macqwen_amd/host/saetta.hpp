@@ -748,8 +748,8 @@ inline size_t slices() {
 struct AttGemm {
     size_t slice, rows_pad, chunk, kv_heads;
     bool fused = true, texp = true;
-    // For a bench: only the first `stages` passes of each block (1, 2: scores; 3: scores and pv, no
-    // outputs); 0 runs all (src/attention_gemm.rs:112-114).
+    // 0 gives the outputs.  For a bench: only the first `stages` passes of each block, without outputs (1, 2:
+    // scores; 3: scores and pv; src/attention_gemm.rs:112-114).
     mutable uint32_t stages = 0;
 
     AttGemm(const gpu::Gpu &, size_t chunk_, size_t kv_heads_) : chunk(chunk_), kv_heads(kv_heads_) {
