@@ -182,6 +182,27 @@ const char *saetta_last_error(void);
  * at threadgroup barriers only. */
 uint32_t saetta_device_status(int clear);
 
+/* ---- plans (src/plan.rs) ------------------------------------------------------ */
+
+/* Plan::set_params (src/plan.rs:144-146): writes `value` to the record in device memory, in stream
+ * order.  The value travels with the launch, so the caller keeps nothing until it has run. */
+int saetta_token_params_set(saetta_stream_t stream, saetta_token_params *d_tp, saetta_token_params value);
+
+/* A list of launches recorded once and run for every token (src/plan.rs:63-146,157-168).  Between
+ * saetta_plan_begin and saetta_plan_end every entry point that this thread calls checks its
+ * arguments and records the launches it would have made, with their arguments, instead of making
+ * them (the stream it is given is not used).  saetta_plan_run makes them on a stream, one after the
+ * other, with one call and no further checks: 2 us of host time per launch.  Buffers named in the
+ * plan must outlive it.  A plan runs on the device it was recorded on (that device current), from
+ * any thread, also on several at once; under stream capture it becomes part of the graph.  begin
+ * fails while the thread is recording, end returns NULL when it is not. */
+typedef struct saetta_plan saetta_plan;
+int saetta_plan_begin(void);
+saetta_plan *saetta_plan_end(void);
+uint32_t saetta_plan_launches(const saetta_plan *plan);
+int saetta_plan_run(saetta_stream_t stream, const saetta_plan *plan);
+void saetta_plan_free(saetta_plan *plan);
+
 /* ---- kv_quant (src/kv_quant.rs) -------------------------------------------- */
 
 /* QuantRows::record / record_at (src/kv_quant.rs:192-221) when d_tp != NULL:

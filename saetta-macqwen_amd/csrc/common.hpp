@@ -7,6 +7,11 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <cstring>
+#include <tuple>
+#include <type_traits>
+#include <utility>
+#include <vector>
 
 #include "../../include/saetta_hip.h"
 
@@ -47,6 +52,46 @@ inline int load_kernel(const void *kernel) {
 }
 
 inline hipStream_t as_stream(saetta_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
+
+// ---- launches, made or recorded ------------------------------------------------
+// A kernel launch with its arguments, as a plan keeps it.
+struct LaunchRecord {
+    const void *kernel;
+    dim3 grid, block;
+    uint32_t lds;
+    uint32_t first_arg, args;  // of LaunchList::offsets
+};
+// Launches in order; the arguments lie in `bytes`, each at its offset, 16-byte aligned.
+struct LaunchList {
+    std::vector<LaunchRecord> launches;
+    std::vector<uint32_t> offsets;
+    std::vector<unsigned char> bytes;
+    int device = 0;
+};
+// The list this thread records into, or nullptr: launches are made.
+LaunchList *&recording();
+
+template <class T>
+void record_arg(LaunchList &list, const T &value) {
+    static_assert(std::is_trivially_copyable<T>::value, "kernel arguments are plain values");
+    const size_t at = (list.bytes.size() + 15) / 16 * 16;
+    list.bytes.resize(at + sizeof(T));
+    memcpy(list.bytes.data() + at, &value, sizeof(T));
+    list.offsets.push_back(uint32_t(at));
+}
+
+// kernel<<<grid, block, lds, stream>>>(args...), or the same launch at the end of the list that this thread records.
+// Every launch of the library goes through here.
+template <class... P, class... A>
+void launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, A &&...args) {
+    static_assert(sizeof...(P) == sizeof...(A), "one argument per kernel parameter");
+    if (LaunchList *list = recording()) {
+        list->launches.push_back({reinterpret_cast<const void *>(kernel), grid, block, uint32_t(lds), uint32_t(list->offsets.size()), uint32_t(sizeof...(P))});
+        (record_arg<std::remove_cv_t<P>>(*list, static_cast<P>(args)), ...);
+        return;
+    }
+    kernel<<<grid, block, lds, stream>>>(std::forward<A>(args)...);
+}
 
 inline bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 

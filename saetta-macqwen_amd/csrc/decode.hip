@@ -2538,15 +2538,15 @@ void launch_partial(hipStream_t stream, const PartialArgs &a, bool one_per_cu, b
     int lds_bytes;
     if constexpr (BITS != 16) {
         if (keys_first) {
-            auto launch = [&](auto rows_c) {
+            auto launch_rows = [&](auto rows_c) {
                 constexpr int MR = decltype(rows_c)::value;
                 using W = KeysFirst<BITS, MR>;
-                attention_partial_kernel_s<BITS, MR><<<dim3(a.nsplits, a.kv_heads), (W::LOADERS + W::WAVES) * 64, W::LDS_BYTES, stream>>>(a);
+                launch(attention_partial_kernel_s<BITS, MR>, dim3(a.nsplits, a.kv_heads), (W::LOADERS + W::WAVES) * 64, W::LDS_BYTES, stream, a);
             };
-            if (a.rows == 1) launch(std::integral_constant<int, 1>());
-            else if (a.rows == 2) launch(std::integral_constant<int, 2>());
-            else if (a.rows == 3) launch(std::integral_constant<int, 3>());
-            else launch(std::integral_constant<int, 4>());
+            if (a.rows == 1) launch_rows(std::integral_constant<int, 1>());
+            else if (a.rows == 2) launch_rows(std::integral_constant<int, 2>());
+            else if (a.rows == 3) launch_rows(std::integral_constant<int, 3>());
+            else launch_rows(std::integral_constant<int, 4>());
             return;
         }
     }
@@ -2566,7 +2566,7 @@ void launch_partial(hipStream_t stream, const PartialArgs &a, bool one_per_cu, b
         lds_bytes = Shape<BITS, TILES, PACKED, itb_rows<TILES>()>::LDS_BYTES;
     }
     // (the dynamic LDS limit of every variant was raised in setup_decode)
-    kernel<<<dim3(a.nsplits, a.kv_heads), THREADS, lds_bytes, stream>>>(a);
+    launch(kernel, dim3(a.nsplits, a.kv_heads), THREADS, lds_bytes, stream, a);
 }
 
 template <int BITS>
@@ -2633,7 +2633,7 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
     }
     if (stages & SAETTA_STAGE_REDUCE) {
         ReduceArgs r{part_o, part_ml, q_and_gate, out, heads, capacity, nsplits, rows, d_tp, decode_len ? 1u : 0u};
-        attention_reduce_kernel<<<dim3(heads, rows, DIM / REDUCE_DIMS), 256, 0, stream>>>(r);
+        launch(attention_reduce_kernel, dim3(heads, rows, DIM / REDUCE_DIMS), 256, 0, stream, r);
     }
     return launch_status(what);
 }

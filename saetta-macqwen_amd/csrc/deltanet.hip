@@ -712,12 +712,12 @@ void launch_small_rows(const SmallRowsArgs &args, hipStream_t stream) {
     const saetta_rows_fused_params &p = args.p;
     const dim3 grid((p.v_dim + 15) / 16, p.v_heads);
     if (p.snapshots) {
-        deltanet_rows_small_kernel<true><<<grid, SMALL_THREADS, 0, stream>>>(args);
+        launch(deltanet_rows_small_kernel<true>, grid, SMALL_THREADS, 0, stream, args);
     } else {
-        deltanet_rows_small_kernel<false><<<grid, SMALL_THREADS, 0, stream>>>(args);
+        launch(deltanet_rows_small_kernel<false>, grid, SMALL_THREADS, 0, stream, args);
     }
     const uint32_t pair_blocks = (p.rows * p.v_heads + 3) / 4, chan_blocks = (args.channels + TAIL_CHANNELS - 1) / TAIL_CHANNELS;
-    deltanet_rows_small_tail_kernel<<<pair_blocks > chan_blocks ? pair_blocks : chan_blocks, 256, 0, stream>>>(args);
+    launch(deltanet_rows_small_tail_kernel, pair_blocks > chan_blocks ? pair_blocks : chan_blocks, 256, 0, stream, args);
 }
 
 }  // namespace
@@ -738,7 +738,7 @@ extern "C" int saetta_deltanet_conv(saetta_stream_t stream, const float *x, cons
                    p.kernel_size);
     if (int rc = ensure_device()) return rc;
     if (p.channels == 0) return SAETTA_OK;
-    deltanet_conv_kernel<<<(p.channels + 255) / 256, 256, 0, as_stream(stream)>>>(x, w, state, out, p);
+    launch(deltanet_conv_kernel, (p.channels + 255) / 256, 256, 0, as_stream(stream), x, w, state, out, p);
     return launch_status("deltanet_conv");
 }
 
@@ -764,7 +764,7 @@ extern "C" int saetta_deltanet_step(saetta_stream_t stream, const float *q, cons
         return saetta_deltanet_rows(stream, q, a, b, a_log, dt_bias, state, z, norm_w, y, nullptr, rp);
     }
     StepArgs args{q, k, v, a, b, a_log, dt_bias, state, z, norm_w, y, p};
-    deltanet_step_kernel<<<p.v_heads, STEP_THREADS, 0, as_stream(stream)>>>(args);
+    launch(deltanet_step_kernel, p.v_heads, STEP_THREADS, 0, as_stream(stream), args);
     return launch_status("deltanet_step");
 }
 
@@ -782,15 +782,15 @@ extern "C" int saetta_deltanet_conv_rows(saetta_stream_t stream, const float *x,
     const bool by_four = p.tokens >= CONV_TILE && p.channels % 4 == 0 && aligned(x, 16) && aligned(w, 16) && aligned(state, 16) && aligned(out, 16) &&
                          (!p.snapshots || aligned(snaps, 16));
     if (p.kernel_size == 4 && by_four) {
-        deltanet_conv_rows4_kernel<<<dim3((p.channels / 4 + 255) / 256, grid.y), 256, 0, as_stream(stream)>>>(x, w, state, out, snaps, p);
+        launch(deltanet_conv_rows4_kernel, dim3((p.channels / 4 + 255) / 256, grid.y), 256, 0, as_stream(stream), x, w, state, out, snaps, p);
     } else if (p.kernel_size == 4) {
-        deltanet_conv_rows_kernel<4><<<grid, 256, 0, as_stream(stream)>>>(x, w, state, out, snaps, p);
+        launch(deltanet_conv_rows_kernel<4>, grid, 256, 0, as_stream(stream), x, w, state, out, snaps, p);
     } else if (p.kernel_size == 2) {
-        deltanet_conv_rows_kernel<2><<<grid, 256, 0, as_stream(stream)>>>(x, w, state, out, snaps, p);
+        launch(deltanet_conv_rows_kernel<2>, grid, 256, 0, as_stream(stream), x, w, state, out, snaps, p);
     } else {
-        deltanet_conv_rows_kernel<0><<<grid, 256, 0, as_stream(stream)>>>(x, w, state, out, snaps, p);
+        launch(deltanet_conv_rows_kernel<0>, grid, 256, 0, as_stream(stream), x, w, state, out, snaps, p);
     }
-    deltanet_conv_state_kernel<<<grid.x, 256, 0, as_stream(stream)>>>(x, state, p);
+    launch(deltanet_conv_state_kernel, grid.x, 256, 0, as_stream(stream), x, state, p);
     return launch_status("deltanet_conv_rows");
 }
 
@@ -833,21 +833,21 @@ extern "C" int saetta_deltanet_rows_ws(saetta_stream_t stream, const float *mixe
         constexpr int LANES = ROWS_LANES_PER_ROW, ROWS_PER_WG = 256 / LANES;
         const dim3 grid((p.v_dim + ROWS_PER_WG - 1) / ROWS_PER_WG, p.v_heads);
         if (p.snapshots) {
-            deltanet_rows_kernel<true, LANES><<<grid, 256, 0, as_stream(stream)>>>(args);
+            launch(deltanet_rows_kernel<true, LANES>, grid, 256, 0, as_stream(stream), args);
         } else {
-            deltanet_rows_kernel<false, LANES><<<grid, 256, 0, as_stream(stream)>>>(args);
+            launch(deltanet_rows_kernel<false, LANES>, grid, 256, 0, as_stream(stream), args);
         }
     }
     const uint32_t pairs = p.tokens * p.v_heads;
     const bool wide = blocks && aligned(y, 16) && aligned(z, 16) && aligned(norm_w, 16);
     if (wide && p.v_dim == 128) {
-        deltanet_gated_norm_wide_kernel<32><<<(pairs * 32 + 255) / 256, 256, 0, as_stream(stream)>>>(y, z, norm_w, pairs, p.eps);
+        launch(deltanet_gated_norm_wide_kernel<32>, (pairs * 32 + 255) / 256, 256, 0, as_stream(stream), y, z, norm_w, pairs, p.eps);
     } else if (wide && p.v_dim == 64) {
-        deltanet_gated_norm_wide_kernel<16><<<(pairs * 16 + 255) / 256, 256, 0, as_stream(stream)>>>(y, z, norm_w, pairs, p.eps);
+        launch(deltanet_gated_norm_wide_kernel<16>, (pairs * 16 + 255) / 256, 256, 0, as_stream(stream), y, z, norm_w, pairs, p.eps);
     } else if (wide && p.v_dim == 256) {
-        deltanet_gated_norm_wide_kernel<64><<<(pairs * 64 + 255) / 256, 256, 0, as_stream(stream)>>>(y, z, norm_w, pairs, p.eps);
+        launch(deltanet_gated_norm_wide_kernel<64>, (pairs * 64 + 255) / 256, 256, 0, as_stream(stream), y, z, norm_w, pairs, p.eps);
     } else {
-        deltanet_gated_norm_rows_kernel<<<(pairs + 3) / 4, 256, 0, as_stream(stream)>>>(y, z, norm_w, pairs, p.v_dim, p.eps);
+        launch(deltanet_gated_norm_rows_kernel, (pairs + 3) / 4, 256, 0, as_stream(stream), y, z, norm_w, pairs, p.v_dim, p.eps);
     }
     return launch_status("deltanet_rows");
 }

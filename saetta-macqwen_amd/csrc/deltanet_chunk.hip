@@ -750,11 +750,11 @@ int run_deltanet_chunk(hipStream_t stream, const float *mixed, const float *a, c
     const uint32_t nblocks = (p.tokens + C - 1) / C;
     ChunkArgs args{mixed, a, b, a_log, dt_bias, state, o, static_cast<unsigned char *>(workspace), p.k_heads, p.v_heads, p.v_dim, p.tokens, channels, p.eps};
     if (p.v_heads == 2 * p.k_heads) {
-        deltanet_chunk_prepare_kernel<2><<<dim3(nblocks, p.k_heads), 256, PrepLds<2>::BYTES, stream>>>(args);
+        launch(deltanet_chunk_prepare_kernel<2>, dim3(nblocks, p.k_heads), 256, PrepLds<2>::BYTES, stream, args);
     } else {
-        deltanet_chunk_prepare_kernel<1><<<dim3(nblocks, p.v_heads), 256, PrepLds<1>::BYTES, stream>>>(args);
+        launch(deltanet_chunk_prepare_kernel<1>, dim3(nblocks, p.v_heads), 256, PrepLds<1>::BYTES, stream, args);
     }
-    deltanet_chunk_chain_kernel<<<dim3(p.v_dim / DV * p.v_heads), 512, ChainLds::BYTES, stream>>>(args);
+    launch(deltanet_chunk_chain_kernel, dim3(p.v_dim / DV * p.v_heads), 512, ChainLds::BYTES, stream, args);
     return SAETTA_OK;
 }
 

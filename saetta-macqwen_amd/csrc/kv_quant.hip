@@ -159,10 +159,10 @@ extern "C" int saetta_kv_quantize(saetta_stream_t stream, int bits, const float 
     const uint32_t lanes = bits == 8 ? 16 : 8;
     const uint32_t blocks = (p.groups * lanes + 255) / 256;
     if (bits == 8) {
-        kv_quantize_kernel<8><<<blocks, 256, 0, as_stream(stream)>>>(x, rows.data, rows.scales,
+        launch(kv_quantize_kernel<8>, blocks, 256, 0, as_stream(stream), x, rows.data, rows.scales,
                                                                      rows.biases, p, d_tp, pos);
     } else {
-        kv_quantize_kernel<4><<<blocks, 256, 0, as_stream(stream)>>>(x, rows.data, rows.scales,
+        launch(kv_quantize_kernel<4>, blocks, 256, 0, as_stream(stream), x, rows.data, rows.scales,
                                                                      rows.biases, p, d_tp, pos);
     }
     return launch_status("kv_quantize");
@@ -179,10 +179,10 @@ extern "C" int saetta_kv_dequantize(saetta_stream_t stream, int bits, saetta_qua
     const uint32_t lanes = bits == 8 ? 16 : 8;
     const uint32_t blocks = (p.groups * lanes + 255) / 256;
     if (bits == 8) {
-        kv_dequantize_kernel<8><<<blocks, 256, 0, as_stream(stream)>>>(rows.data, rows.scales,
+        launch(kv_dequantize_kernel<8>, blocks, 256, 0, as_stream(stream), rows.data, rows.scales,
                                                                        rows.biases, out_f16, p);
     } else {
-        kv_dequantize_kernel<4><<<blocks, 256, 0, as_stream(stream)>>>(rows.data, rows.scales,
+        launch(kv_dequantize_kernel<4>, blocks, 256, 0, as_stream(stream), rows.data, rows.scales,
                                                                        rows.biases, out_f16, p);
     }
     return launch_status("kv_dequantize");
@@ -198,9 +198,9 @@ extern "C" int saetta_kv_dequantize_f32(saetta_stream_t stream, int bits, saetta
     const uint32_t lanes = bits == 8 ? 16 : 8;
     const uint32_t blocks = (p.groups * lanes + 255) / 256;
     if (bits == 8) {
-        kv_dequantize_f32_kernel<8><<<blocks, 256, 0, as_stream(stream)>>>(rows.data, rows.scales, rows.biases, out, p);
+        launch(kv_dequantize_f32_kernel<8>, blocks, 256, 0, as_stream(stream), rows.data, rows.scales, rows.biases, out, p);
     } else {
-        kv_dequantize_f32_kernel<4><<<blocks, 256, 0, as_stream(stream)>>>(rows.data, rows.scales, rows.biases, out, p);
+        launch(kv_dequantize_f32_kernel<4>, blocks, 256, 0, as_stream(stream), rows.data, rows.scales, rows.biases, out, p);
     }
     return launch_status("kv_dequantize_f32");
 }
@@ -212,6 +212,6 @@ extern "C" int saetta_to_half(saetta_stream_t stream, const float *x, uint16_t *
     if (int rc = ensure_device()) return rc;
     if (n == 0) return SAETTA_OK;
     const size_t blocks = (n + 1023) / 1024;
-    to_half_kernel<<<dim3(uint32_t(blocks)), 256, 0, as_stream(stream)>>>(x, out_f16, n);
+    launch(to_half_kernel, dim3(uint32_t(blocks)), 256, 0, as_stream(stream), x, out_f16, n);
     return launch_status("to_half");
 }

@@ -641,8 +641,10 @@ __device__ __host__ __forceinline__ uint32_t prefill_first_tile(uint32_t pos, ui
 }
 __device__ __host__ __forceinline__ uint32_t prefill_items(uint32_t pos, uint32_t tokens, uint32_t part_blocks) {
     const uint32_t ntiles = (tokens + TQ - 1) / TQ;
-    uint32_t n = 0;
-    for (uint32_t p = 0, first; (first = prefill_first_tile(pos, tokens, part_blocks, p)) < ntiles; p++) n += ntiles - first;
+    // the parts that begin at a key the first tile sees are every tile's
+    const uint32_t whole = (pos + (tokens < TQ ? tokens : TQ) - 1) / (part_blocks * BK) + 1;
+    uint32_t n = whole * ntiles;
+    for (uint32_t p = whole, first; (first = prefill_first_tile(pos, tokens, part_blocks, p)) < ntiles; p++) n += ntiles - first;
     return n;
 }
 
@@ -838,7 +840,8 @@ int acquire_workspace(hipStream_t stream, void *&workspace, size_t workspace_siz
         return SAETTA_OK;
     }
     // No workspace given: use (and grow) the library's own for this stream.  This may allocate, which a
-    // stream under capture cannot do.
+    // stream under capture cannot do; and a plan outlives the buffer, which a later call may grow.
+    SAETTA_REQUIRE(!recording(), SAETTA_E_SCRATCH, "%s: a recorded call needs a workspace of the caller's (%zu bytes, %s)", what, need, sizer);
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) (void)hipGetLastError();
     SAETTA_REQUIRE(capturing == hipStreamCaptureStatusNone, SAETTA_E_SCRATCH,
@@ -872,11 +875,11 @@ uint32_t launch_prepare(hipStream_t stream, int bits, const void *kdata, const v
                    uint32_t(rows), tiles_taken};
     const dim3 pgrid(nblocks, kv_heads);
     if (bits == 8) {
-        prefill_prepare_kernel<8><<<pgrid, PREP_THREADS, 0, stream>>>(pa);
+        launch(prefill_prepare_kernel<8>, pgrid, PREP_THREADS, 0, stream, pa);
     } else if (bits == 4) {
-        prefill_prepare_kernel<4><<<pgrid, PREP_THREADS, 0, stream>>>(pa);
+        launch(prefill_prepare_kernel<4>, pgrid, PREP_THREADS, 0, stream, pa);
     } else {
-        prefill_prepare_kernel<16><<<pgrid, PREP_THREADS, 0, stream>>>(pa);
+        launch(prefill_prepare_kernel<16>, pgrid, PREP_THREADS, 0, stream, pa);
     }
     return nblocks;
 }
@@ -919,11 +922,11 @@ int launch_flash(hipStream_t stream, int bits, const uint16_t *q, const void *kd
         a.part_o = reinterpret_cast<float *>(ws + plan.plain);
         a.part_ml = reinterpret_cast<float *>(ws + plan.plain + size_t(plan.nparts) * ntiles * p.kv_heads * PART_O_BYTES);
         const uint32_t total = prefill_items(p.pos, p.tokens, plan.part_blocks) * p.kv_heads;
-        attention_prefill_kernel<true><<<dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream>>>(a);
-        prefill_merge_kernel<<<dim3(p.tokens, p.kv_heads), MERGE_THREADS, 0, stream>>>(a);
+        launch(attention_prefill_kernel<true>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
+        launch(prefill_merge_kernel, dim3(p.tokens, p.kv_heads), MERGE_THREADS, 0, stream, a);
     } else {
         const uint32_t total = ntiles * p.kv_heads;
-        attention_prefill_kernel<false><<<dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream>>>(a);
+        launch(attention_prefill_kernel<false>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
     }
     return launch_status(what);
 }
@@ -1338,9 +1341,9 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
         // a span of AG_SPAN blocks of AG_KEYS keys at a time: its scores, then its pv
         for (uint64_t g0 = 0; g0 < end; g0 += uint64_t(AG_SPAN) * AG_KEYS) {
             a.g0 = uint32_t(g0);
-            attention_gemm_scores_kernel<<<dim3(a.split, wide, p.kv_heads), AG_THREADS, 0, stream>>>(a);
+            launch(attention_gemm_scores_kernel, dim3(a.split, wide, p.kv_heads), AG_THREADS, 0, stream, a);
             if (stages == 1 || stages == 2) continue;
-            attention_gemm_pv_kernel<<<dim3(1, tiles, p.kv_heads), AG_THREADS, 0, stream>>>(a);
+            launch(attention_gemm_pv_kernel, dim3(1, tiles, p.kv_heads), AG_THREADS, 0, stream, a);
         }
     }
     return launch_status(what);

@@ -130,11 +130,11 @@ extern "C" int saetta_attn_prep_store(saetta_stream_t stream, int bits, const fl
     PrepArgs a{q_and_gate, k, v, q_norm, k_norm, q_out, keys_half, values_half, keys, values, k_back, p, d_tp, capacity};
     const dim3 grid(p.heads + 2 * p.kv_heads, rows);
     if (bits == 8) {
-        attention_prep_store_kernel<8><<<grid, 256, 0, as_stream(stream)>>>(a);
+        launch(attention_prep_store_kernel<8>, grid, 256, 0, as_stream(stream), a);
     } else if (bits == 4) {
-        attention_prep_store_kernel<4><<<grid, 256, 0, as_stream(stream)>>>(a);
+        launch(attention_prep_store_kernel<4>, grid, 256, 0, as_stream(stream), a);
     } else {
-        attention_prep_store_kernel<16><<<grid, 256, 0, as_stream(stream)>>>(a);
+        launch(attention_prep_store_kernel<16>, grid, 256, 0, as_stream(stream), a);
     }
     return launch_status("attn_prep_store");
 }

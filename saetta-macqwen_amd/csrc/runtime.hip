@@ -36,6 +36,8 @@ struct DeviceSetup {
 DeviceSetup g_devices[MAX_DEVICES];
 }  // namespace
 
+int setup_runtime();
+
 int ensure_device() {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -73,7 +75,7 @@ int ensure_device() {
             d.status_host = static_cast<volatile uint32_t *>(host);
             d.status_dev = static_cast<uint32_t *>(devp);
         }
-        int (*const setups[])() = {setup_kv_quant, setup_prep, setup_deltanet, setup_decode, setup_prefill};
+        int (*const setups[])() = {setup_runtime, setup_kv_quant, setup_prep, setup_deltanet, setup_decode, setup_prefill};
         for (auto setup : setups) {
             if (int rc = setup()) {
                 d.status = SAETTA_E_DEVICE;
@@ -121,7 +123,76 @@ int launch_status(const char *what) {
     return SAETTA_OK;
 }
 
+LaunchList *&recording() {
+    static thread_local LaunchList *list = nullptr;
+    return list;
+}
+
+namespace {
+__global__ __launch_bounds__(64) void token_params_kernel(saetta_token_params *dst, saetta_token_params value) {
+    if (threadIdx.x == 0) *dst = value;
+}
+}  // namespace
+
+int setup_runtime() { return load_kernel(reinterpret_cast<const void *>(token_params_kernel)); }
+
 }  // namespace saetta
+
+// A plan: what the calls between begin and end would have launched.
+struct saetta_plan {
+    saetta::LaunchList list;
+};
+
+extern "C" int saetta_plan_begin(void) {
+    using namespace saetta;
+    SAETTA_REQUIRE(!recording(), SAETTA_E_SHAPE, "plan_begin: this thread is recording a plan already");
+    if (int rc = ensure_device()) return rc;
+    LaunchList *list = new LaunchList;
+    if (hipGetDevice(&list->device) != hipSuccess) (void)hipGetLastError();
+    recording() = list;
+    return SAETTA_OK;
+}
+
+extern "C" saetta_plan *saetta_plan_end(void) {
+    using namespace saetta;
+    LaunchList *list = recording();
+    recording() = nullptr;
+    if (!list) {
+        fail(SAETTA_E_SHAPE, "plan_end: this thread is recording no plan");
+        return nullptr;
+    }
+    saetta_plan *plan = new saetta_plan{std::move(*list)};
+    delete list;
+    return plan;
+}
+
+extern "C" uint32_t saetta_plan_launches(const saetta_plan *plan) { return plan ? uint32_t(plan->list.launches.size()) : 0; }
+
+extern "C" int saetta_plan_run(saetta_stream_t stream, const saetta_plan *plan) {
+    using namespace saetta;
+    SAETTA_REQUIRE(plan, SAETTA_E_NULL, "plan_run: null plan");
+    const LaunchList &list = plan->list;
+    int dev = 0;
+    SAETTA_REQUIRE(hipGetDevice(&dev) == hipSuccess && dev == list.device, SAETTA_E_DEVICE,
+                   "plan_run: the plan was recorded on device %d, the current one is %d", list.device, dev);
+    for (const LaunchRecord &r : list.launches) {
+        void *args[16];
+        for (uint32_t i = 0; i < r.args; i++) args[i] = const_cast<unsigned char *>(list.bytes.data()) + list.offsets[r.first_arg + i];
+        const hipError_t e = hipLaunchKernel(r.kernel, r.grid, r.block, args, r.lds, as_stream(stream));
+        if (e != hipSuccess) return fail(int(e), "plan_run: %s", hipGetErrorString(e));
+    }
+    return launch_status("plan_run");
+}
+
+extern "C" void saetta_plan_free(saetta_plan *plan) { delete plan; }
+
+extern "C" int saetta_token_params_set(saetta_stream_t stream, saetta_token_params *d_tp, saetta_token_params value) {
+    using namespace saetta;
+    SAETTA_REQUIRE(d_tp && aligned(d_tp, 4), SAETTA_E_NULL, "token_params_set: null or misaligned record");
+    if (int rc = ensure_device()) return rc;
+    launch(token_params_kernel, dim3(1), dim3(64), 0, as_stream(stream), d_tp, value);
+    return launch_status("token_params_set");
+}
 
 extern "C" int saetta_init(void) { return saetta::ensure_device(); }
 

@@ -7,7 +7,8 @@ LIB_PATH = os.environ.get("SAETTA_HIP_LIB") or os.path.join(_HERE, "lib", "libsa
 
 # Every symbol include/saetta_hip.h declares; tests check the library exports each.
 SYMBOLS = [
-    "saetta_init", "saetta_last_error", "saetta_device_status", "saetta_kv_quantize", "saetta_kv_dequantize", "saetta_kv_dequantize_f32", "saetta_to_half", "saetta_attn_prep_store", "saetta_deltanet_conv", "saetta_deltanet_step", "saetta_deltanet_conv_rows", "saetta_deltanet_rows", "saetta_deltanet_rows_ws", "saetta_deltanet_rows_workspace_bytes", "saetta_deltanet_token", "saetta_deltanet_rows_fused",
+    "saetta_init", "saetta_last_error", "saetta_device_status", "saetta_token_params_set", "saetta_plan_begin",
+    "saetta_plan_end", "saetta_plan_launches", "saetta_plan_run", "saetta_plan_free", "saetta_kv_quantize", "saetta_kv_dequantize", "saetta_kv_dequantize_f32", "saetta_to_half", "saetta_attn_prep_store", "saetta_deltanet_conv", "saetta_deltanet_step", "saetta_deltanet_conv_rows", "saetta_deltanet_rows", "saetta_deltanet_rows_ws", "saetta_deltanet_rows_workspace_bytes", "saetta_deltanet_token", "saetta_deltanet_rows_fused",
     "saetta_part_o_bytes", "saetta_part_ml_bytes", "saetta_attn_decode", "saetta_attn_decode_quant",
     "saetta_attn_rows", "saetta_attn_rows_quant", "saetta_static_scratch_bytes", "saetta_attn_decode_quant_static", "saetta_prefill_workspace_bytes", "saetta_attn_prefill", "saetta_attn_prefill_quant",
     "saetta_attn_gemm_workspace_bytes", "saetta_attn_gemm",
@@ -62,6 +63,13 @@ def lib():
         l.saetta_init.restype, l.saetta_init.argtypes = i32, []
         l.saetta_last_error.restype, l.saetta_last_error.argtypes = ctypes.c_char_p, []
         l.saetta_device_status.restype, l.saetta_device_status.argtypes = u32, [i32]
+        l.saetta_token_params_set.restype = i32
+        l.saetta_token_params_set.argtypes = [vp, vp, TokenParamsC]
+        l.saetta_plan_begin.restype, l.saetta_plan_begin.argtypes = i32, []
+        l.saetta_plan_end.restype, l.saetta_plan_end.argtypes = vp, []
+        l.saetta_plan_launches.restype, l.saetta_plan_launches.argtypes = u32, [vp]
+        l.saetta_plan_run.restype, l.saetta_plan_run.argtypes = i32, [vp, vp]
+        l.saetta_plan_free.restype, l.saetta_plan_free.argtypes = None, [vp]
         l.saetta_kv_quantize.restype = i32
         l.saetta_kv_quantize.argtypes = [vp, i32, vp, QuantRowsC, KvQuantParamsC, vp, u32]
         l.saetta_kv_dequantize.restype = i32

@@ -15,6 +15,7 @@ view with an offset); a Metal encoder is a HIP stream.  Shape violations raise
 import ctypes
 import enum
 import math
+import threading
 import time
 
 import torch
@@ -61,8 +62,10 @@ class TokenParams:
 def _stream(stream=None):
     if isinstance(stream, ctypes.c_void_p):  # what a plan op is handed
         return stream
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is None:
+        # the handle of torch's current stream, without the Stream object of torch.cuda.current_stream()
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    return ctypes.c_void_p(stream.cuda_stream)
 
 
 def _ptr(t):
@@ -81,6 +84,50 @@ def _need(t, dtype, what):
     return t
 
 
+class _Call:
+    """A plan op that is one call of the library: its function and arguments, bound once, and the tensors
+    whose memory they point at."""
+
+    def __init__(self, name, what, args, keep=()):
+        self.name, self.what, self.args, self.keep = name, what, args, keep
+
+    def __call__(self, s):
+        ffi.check(getattr(ffi.lib(), self.name)(s, *self.args), self.what)
+
+
+class _Launches:
+    """A run of _Calls as the library's own plan (saetta_plan_*): recorded at the first run, then one call
+    makes all the launches."""
+
+    def __init__(self, calls):
+        self.calls, self.plan, self.lock = calls, None, threading.Lock()
+
+    def _record(self, l, s):
+        with self.lock:
+            if self.plan is not None:
+                return
+            ffi.check(l.saetta_plan_begin(), "plan_begin")
+            try:
+                for call in self.calls:
+                    call(s)
+            except BaseException:
+                l.saetta_plan_free(l.saetta_plan_end())
+                raise
+            self.free, self.plan = l.saetta_plan_free, ctypes.c_void_p(l.saetta_plan_end())
+
+    def __call__(self, s):
+        l = ffi.lib()
+        if self.plan is None:
+            self._record(l, s)
+        rc = l.saetta_plan_run(s, self.plan)
+        if rc:
+            ffi.check(rc, "plan_run")
+
+    def __del__(self):
+        if self.plan is not None:
+            self.free(self.plan)
+
+
 class Plan:
     """A list of launches recorded once and run for every token (src/plan.rs:63-146).
 
@@ -96,10 +143,10 @@ class Plan:
         self.ops.append((kernel, launch))
 
     def set_params(self, tp):
-        """Plan::set_params (src/plan.rs:144-146): a small async copy on the current stream."""
-        host = torch.tensor([tp.token, tp.position, tp.kv_len, tp.pad], dtype=torch.int32).pin_memory()
-        self.params.copy_(host, non_blocking=True)
-        self._keep = host
+        """Plan::set_params (src/plan.rs:144-146): one small launch on the current stream that carries the
+        values (a copy from pinned memory took 10 us of the host and 7 us of the stream, this 3 and 1.6)."""
+        ffi.check(ffi.lib().saetta_token_params_set(_stream(), _ptr(self.params), ffi.TokenParamsC(
+            tp.token, tp.position, tp.kv_len, tp.pad)), "token_params_set")
 
     def __len__(self):
         return len(self.ops)
@@ -148,6 +195,16 @@ class Built:
     def __init__(self, ops, graph=False):
         self.ops = ops
         self.graph = None
+        # what a run without a graph does: the library's own calls in runs of one native plan each, any other
+        # callable as it is
+        self._parts = []
+        for _, launch in ops:
+            if not isinstance(launch, _Call):
+                self._parts.append(launch)
+            elif self._parts and isinstance(self._parts[-1], _Launches):
+                self._parts[-1].calls.append(launch)
+            else:
+                self._parts.append(_Launches([launch]))
         if graph and ops:
             # The library's one-time set-up (code objects, LDS limits) must not happen under capture;
             # the launches themselves are not run here: a plan may hold ops that advance a state.
@@ -171,8 +228,8 @@ class Built:
             self.graph.replay()
             return
         s = _stream(stream)
-        for _, launch in self.ops:
-            launch(s)
+        for part in self._parts:
+            part(s)
 
     def run_timed(self, stream=None):
         """Built::run_timed (src/plan.rs:249-251): runs, waits, and returns (wall seconds, the
@@ -211,18 +268,18 @@ class QuantRows:
     def c(self):
         return ffi.QuantRowsC(self.data.data_ptr(), self.scales.data_ptr(), self.biases.data_ptr())
 
+    def tensors(self):
+        return self.data, self.scales, self.biases
+
     def record(self, plan, x):
         self.record_at(plan, x, plan.params)
 
     def record_at(self, plan, x, params, parallel=False):
         _need(x, torch.float32, "QuantRows.record x")
         p = ffi.KvQuantParamsC(self.per_token, self.per_token)
-        rows, bits = self.c(), self.bits.value
-
-        def launch(s):
-            ffi.check(ffi.lib().saetta_kv_quantize(s, bits, _ptr(x), rows, p, _ptr(params), 0), "kv_quantize")
-
-        plan.op(f"kv_quantize_{bits}", launch)
+        bits = self.bits.value
+        plan.op(f"kv_quantize_{bits}", _Call("saetta_kv_quantize", "kv_quantize", (
+            bits, _ptr(x), self.c(), p, _ptr(params), 0), (x, params, *self.tensors())))
 
     def encode(self, x, pos, tokens, stream=None):
         _need(x, torch.float32, "QuantRows.encode x")
@@ -330,34 +387,20 @@ class DecodeAttention:
     def record(self, plan, q, keys, values, q_and_gate, out):
         _need(q, torch.float32, "q"), _need(keys, torch.float16, "keys"), _need(values, torch.float16, "values")
         _need(q_and_gate, torch.float32, "q_and_gate"), _need(out, torch.float32, "out")
-        p, tp, po, pml, flags = self._params(), plan.params, self.part_o, self.part_ml, self._flags()
-
-        def launch(stage):
-            def f(s):
-                ffi.check(ffi.lib().saetta_attn_decode(s, _ptr(q), _ptr(keys), _ptr(values), _ptr(po), _ptr(pml),
-                                                       _ptr(q_and_gate), _ptr(out), p, _ptr(tp), stage | flags),
-                          "attn_decode")
-            return f
-
-        plan.op(self.kernel, launch(ffi.STAGE_PARTIAL))
-        plan.op("attention_reduce", launch(ffi.STAGE_REDUCE))
+        flags, keep = self._flags(), (q, keys, values, self.part_o, self.part_ml, q_and_gate, out, plan.params)
+        args = (*[_ptr(t) for t in keep[:-1]], self._params(), _ptr(plan.params))
+        for kernel, stage in ((self.kernel, ffi.STAGE_PARTIAL), ("attention_reduce", ffi.STAGE_REDUCE)):
+            plan.op(kernel, _Call("saetta_attn_decode", "attn_decode", (*args, stage | flags), keep))
 
     def record_quant(self, plan, q, keys, values, q_and_gate, out):
         if keys.bits is KvBits.Half:
             raise ValueError("a half cache goes through record")
         _need(q, torch.float32, "q"), _need(q_and_gate, torch.float32, "q_and_gate"), _need(out, torch.float32, "out")
-        p, tp, po, pml, bits = self._params(), plan.params, self.part_o, self.part_ml, keys.bits.value
-        kc, vc, flags = keys.c(), values.c(), self._flags()
-
-        def launch(stage):
-            def f(s):
-                ffi.check(ffi.lib().saetta_attn_decode_quant(s, bits, _ptr(q), kc, vc, _ptr(po), _ptr(pml),
-                                                             _ptr(q_and_gate), _ptr(out), p, _ptr(tp), stage | flags),
-                          "attn_decode_quant")
-            return f
-
-        plan.op(f"{self.kernel}_q{bits}", launch(ffi.STAGE_PARTIAL))
-        plan.op("attention_reduce", launch(ffi.STAGE_REDUCE))
+        bits, flags = keys.bits.value, self._flags()
+        keep = (q, self.part_o, self.part_ml, q_and_gate, out, plan.params, *keys.tensors(), *values.tensors())
+        args = (bits, _ptr(q), keys.c(), values.c(), *[_ptr(t) for t in keep[1:5]], self._params(), _ptr(plan.params))
+        for kernel, stage in ((f"{self.kernel}_q{bits}", ffi.STAGE_PARTIAL), ("attention_reduce", ffi.STAGE_REDUCE)):
+            plan.op(kernel, _Call("saetta_attn_decode_quant", "attn_decode_quant", (*args, stage | flags), keep))
 
 
 class PrepParams:
@@ -388,15 +431,11 @@ def record_store(plan, q_and_gate, k, v, q_norm, k_norm, q, keys, values, p, cap
     else:
         _need(keys, torch.float16, "keys"), _need(values, torch.float16, "values")
         bits, kh, vh, kq, vq = 16, _ptr(keys), _ptr(values), none, none
-    pc, tp = p.c(), plan.params
     kb = None if k_back is None else _ptr(k_back)
-
-    def launch(s):
-        ffi.check(ffi.lib().saetta_attn_prep_store(s, bits, _ptr(q_and_gate), _ptr(k), _ptr(v), _ptr(q_norm),
-                                                   _ptr(k_norm), _ptr(q), kh, vh, kq, vq, kb, pc, rows, capacity,
-                                                   _ptr(tp)), "attn_prep_store")
-
-    plan.op("attention_prep_store", launch)
+    ts = (q_and_gate, k, v, q_norm, k_norm, q)
+    keep = (*ts, k_back, plan.params, *(keys.tensors() + values.tensors() if quant else (keys, values)))
+    plan.op("attention_prep_store", _Call("saetta_attn_prep_store", "attn_prep_store", (
+        bits, *[_ptr(t) for t in ts], kh, vh, kq, vq, kb, p.c(), rows, capacity, _ptr(plan.params)), keep))
 
 
 def deltanet_conv(plan, x, w, state, out, channels, kernel_size):
@@ -407,8 +446,8 @@ def deltanet_conv(plan, x, w, state, out, channels, kernel_size):
     if x.numel() < channels or w.numel() < channels * kernel_size or state.numel() < (kernel_size - 1) * channels:
         raise ValueError("deltanet_conv: buffers too small")
     p = ffi.ConvParamsC(channels, kernel_size)
-    plan.op("deltanet_conv", lambda s: ffi.check(
-        ffi.lib().saetta_deltanet_conv(s, _ptr(x), _ptr(w), _ptr(state), _ptr(out), p), "deltanet_conv"))
+    ts = (x, w, state, out)
+    plan.op("deltanet_conv", _Call("saetta_deltanet_conv", "deltanet_conv", (*[_ptr(t) for t in ts], p), ts))
 
 
 def deltanet_step(plan, q, k, v, a, b, a_log, dt_bias, state, z, norm_w, y, k_heads, v_heads, v_dim, eps):
@@ -420,8 +459,7 @@ def deltanet_step(plan, q, k, v, a, b, a_log, dt_bias, state, z, norm_w, y, k_he
     if state.numel() < v_heads * v_dim * 128 or q.numel() < k_heads * 128 or v.numel() < v_heads * v_dim:
         raise ValueError("deltanet_step: buffers too small")
     p = ffi.StepParamsC(k_heads, v_heads, v_dim, eps)
-    plan.op("deltanet_step", lambda s: ffi.check(
-        ffi.lib().saetta_deltanet_step(s, *[_ptr(t) for t in ts], p), "deltanet_step"))
+    plan.op("deltanet_step", _Call("saetta_deltanet_step", "deltanet_step", (*[_ptr(t) for t in ts], p), ts))
 
 
 def deltanet_token(plan, x, w, conv_state, a, b, a_log, dt_bias, state, z, norm_w, y, k_heads, v_heads, v_dim,
@@ -437,8 +475,7 @@ def deltanet_token(plan, x, w, conv_state, a, b, a_log, dt_bias, state, z, norm_
             or state.numel() < v_heads * v_dim * 128 or y.numel() < v_heads * v_dim or z.numel() < v_heads * v_dim):
         raise ValueError("deltanet_token: buffers too small")
     cp, sp = ffi.ConvParamsC(channels, kernel_size), ffi.StepParamsC(k_heads, v_heads, v_dim, eps)
-    plan.op("deltanet_token", lambda s: ffi.check(
-        ffi.lib().saetta_deltanet_token(s, *[_ptr(t) for t in ts], cp, sp), "deltanet_token"))
+    plan.op("deltanet_token", _Call("saetta_deltanet_token", "deltanet_token", (*[_ptr(t) for t in ts], cp, sp), ts))
 
 
 def deltanet_conv_rows(plan, x, w, state, out, channels, kernel_size, tokens, snaps=None):
@@ -455,9 +492,9 @@ def deltanet_conv_rows(plan, x, w, state, out, channels, kernel_size, tokens, sn
             or state.numel() < (kernel_size - 1) * channels):
         raise ValueError("deltanet_conv_rows: buffers too small")
     p = ffi.ConvRowsParamsC(channels, kernel_size, tokens, int(snaps is not None))
-    plan.op("deltanet_conv_rows", lambda s: ffi.check(
-        ffi.lib().saetta_deltanet_conv_rows(s, _ptr(x), _ptr(w), _ptr(state), _ptr(out),
-                                            _ptr(snaps) if snaps is not None else None, p), "deltanet_conv_rows"))
+    ts = (x, w, state, out)
+    plan.op("deltanet_conv_rows", _Call("saetta_deltanet_conv_rows", "deltanet_conv_rows", (
+        *[_ptr(t) for t in ts], _ptr(snaps) if snaps is not None else None, p), (*ts, snaps)))
 
 
 def deltanet_rows(plan, mixed, a, b, a_log, dt_bias, state, z, norm_w, y, k_heads, v_heads, v_dim, tokens, eps,
@@ -483,10 +520,9 @@ def deltanet_rows(plan, mixed, a, b, a_log, dt_bias, state, z, norm_w, y, k_head
     # recorded op owns (the reference's prefill works in buffers of its own, src/prefill.rs:1433-1578)
     need = ffi.lib().saetta_deltanet_rows_workspace_bytes(p)
     ws = torch.empty(need, dtype=torch.uint8, device=mixed.device) if need else None
-    plan.op("deltanet_rows", lambda s: ffi.check(
-        ffi.lib().saetta_deltanet_rows_ws(s, *[_ptr(t) for t in ts], _ptr(snaps) if snaps is not None else None, p,
-                                          _ptr(ws) if ws is not None else None, need),
-        "deltanet_rows"))
+    plan.op("deltanet_rows", _Call("saetta_deltanet_rows_ws", "deltanet_rows", (
+        *[_ptr(t) for t in ts], _ptr(snaps) if snaps is not None else None, p, _ptr(ws) if ws is not None else None, need),
+        (*ts, snaps, ws)))
 
 
 def deltanet_rows_fused(plan, x, w, conv_state, a, b, a_log, dt_bias, state, z, norm_w, y, k_heads, v_heads, v_dim,
@@ -514,11 +550,9 @@ def deltanet_rows_fused(plan, x, w, conv_state, a, b, a_log, dt_bias, state, z, 
         if conv_snaps.numel() < rows * (kernel_size - 1) * channels or state_snaps.numel() < rows * v_heads * v_dim * 128:
             raise ValueError("deltanet_rows_fused: snapshots too small")
     p = ffi.RowsFusedParamsC(k_heads, v_heads, v_dim, kernel_size, eps, rows, int(conv_snaps is not None))
-    plan.op("deltanet_rows_fused", lambda s: ffi.check(
-        ffi.lib().saetta_deltanet_rows_fused(s, *[_ptr(t) for t in ts],
-                                             _ptr(conv_snaps) if conv_snaps is not None else None,
-                                             _ptr(state_snaps) if state_snaps is not None else None, p),
-        "deltanet_rows_fused"))
+    plan.op("deltanet_rows_fused", _Call("saetta_deltanet_rows_fused", "deltanet_rows_fused", (
+        *[_ptr(t) for t in ts], _ptr(conv_snaps) if conv_snaps is not None else None,
+        _ptr(state_snaps) if state_snaps is not None else None, p), (*ts, conv_snaps, state_snaps)))
 
 
 KV_ALIGN = 128  # src/gpu_layers.rs:199: the decode chunk, and a multiple of the prefill key block
@@ -682,16 +716,11 @@ class AttentionRows:
             raise ValueError("AttentionRows.record: too many rows")
         _need(q, torch.float32, "q"), _need(keys, torch.float16, "keys"), _need(values, torch.float16, "values")
         _need(q_and_gate, torch.float32, "q_and_gate"), _need(out, torch.float32, "out")
-        p, tp, po, pml = self._params(m), params[0], self.part_o, self.part_ml
-
-        def launch(stage):
-            def f(s):
-                ffi.check(ffi.lib().saetta_attn_rows(s, _ptr(q), _ptr(keys), _ptr(values), _ptr(po), _ptr(pml),
-                                                     _ptr(q_and_gate), _ptr(out), p, _ptr(tp), stage), "attn_rows")
-            return f
-
-        plan.op("attention_partial_rows_chunks", launch(ffi.STAGE_PARTIAL))
-        plan.op("attention_reduce_rows_chunks", launch(ffi.STAGE_REDUCE))
+        keep = (q, keys, values, self.part_o, self.part_ml, q_and_gate, out, params[0])
+        args = (*[_ptr(t) for t in keep[:-1]], self._params(m), _ptr(params[0]))
+        for kernel, stage in (("attention_partial_rows_chunks", ffi.STAGE_PARTIAL),
+                              ("attention_reduce_rows_chunks", ffi.STAGE_REDUCE)):
+            plan.op(kernel, _Call("saetta_attn_rows", "attn_rows", (*args, stage), keep))
 
     def record_quant(self, plan, m, q, keys, values, q_and_gate, out, params):
         if m > self.rows or len(params) < m:
@@ -699,18 +728,12 @@ class AttentionRows:
         if keys.bits is KvBits.Half:
             raise ValueError("a half cache goes through record")
         _need(q, torch.float32, "q"), _need(q_and_gate, torch.float32, "q_and_gate"), _need(out, torch.float32, "out")
-        p, tp, po, pml, bits = self._params(m), params[0], self.part_o, self.part_ml, keys.bits.value
-        kc, vc = keys.c(), values.c()
-
-        def launch(stage):
-            def f(s):
-                ffi.check(ffi.lib().saetta_attn_rows_quant(s, bits, _ptr(q), kc, vc, _ptr(po), _ptr(pml),
-                                                           _ptr(q_and_gate), _ptr(out), p, _ptr(tp), stage),
-                          "attn_rows_quant")
-            return f
-
-        plan.op(f"attention_partial_rows_q{bits}", launch(ffi.STAGE_PARTIAL))
-        plan.op("attention_reduce_rows", launch(ffi.STAGE_REDUCE))
+        bits = keys.bits.value
+        keep = (q, self.part_o, self.part_ml, q_and_gate, out, params[0], *keys.tensors(), *values.tensors())
+        args = (bits, _ptr(q), keys.c(), values.c(), *[_ptr(t) for t in keep[1:5]], self._params(m), _ptr(params[0]))
+        for kernel, stage in ((f"attention_partial_rows_q{bits}", ffi.STAGE_PARTIAL),
+                              ("attention_reduce_rows", ffi.STAGE_REDUCE)):
+            plan.op(kernel, _Call("saetta_attn_rows_quant", "attn_rows_quant", (*args, stage), keep))
 
 
 def _workspace(t):
@@ -720,13 +743,13 @@ def _workspace(t):
     return _ptr(t), t.numel()
 
 
-def _workspace_or_own(t, nbytes, like, stream):
-    """The caller's workspace, or a tensor of this call's own from torch's allocator (which hands a
+def _workspace_or_own(t, p, like, stream):
+    """The caller's workspace for the chunk of FlashParams p, or a tensor of this call's own from torch's allocator (which hands a
     block out again only behind the work queued on its stream): the library's own workspace, which a
     NULL pointer would select, is one per device and stream that stays for the life of the process."""
     if t is not None:
         return t
-    t = torch.empty(nbytes, dtype=torch.uint8, device=like.device)
+    t = torch.empty(attention_prefill.workspace_bytes(p), dtype=torch.uint8, device=like.device)
     if isinstance(stream, torch.cuda.Stream):
         t.record_stream(stream)
     return t
@@ -766,7 +789,7 @@ class attention_prefill:
             raise ValueError(f"{kernel} needs 8 q heads per kv head")
         _need(q, torch.float16, "q"), _need(keys, torch.float16, "keys"), _need(values, torch.float16, "values")
         _need(q_and_gate, torch.float32, "q_and_gate"), _need(out, torch.float32, "out")
-        workspace = _workspace_or_own(workspace, attention_prefill.workspace_bytes(p), q, stream)
+        workspace = _workspace_or_own(workspace, p, q, stream)
         ffi.check(ffi.lib().saetta_attn_prefill(_stream(stream), _ptr(q), _ptr(keys), _ptr(values),
                                                 _ptr(q_and_gate), _ptr(out), p.c(), *_workspace(workspace)),
                   "attn_prefill")
@@ -837,7 +860,7 @@ class attention_prefill:
         if p.heads != p.kv_heads * 8:
             raise ValueError("prefill attention needs 8 q heads per kv head")
         _need(q, torch.float16, "q"), _need(q_and_gate, torch.float32, "q_and_gate"), _need(out, torch.float32, "out")
-        workspace = _workspace_or_own(workspace, attention_prefill.workspace_bytes(p), q, stream)
+        workspace = _workspace_or_own(workspace, p, q, stream)
         ffi.check(ffi.lib().saetta_attn_prefill_quant(_stream(stream), keys.bits.value, _ptr(q), keys.c(), values.c(),
                                                       _ptr(q_and_gate), _ptr(out), p.c(), *_workspace(workspace)),
                   "attn_prefill_quant")
