@@ -362,6 +362,17 @@ int saetta_deltanet_token(saetta_stream_t stream, const float *x, const float *w
                           float *state, const float *z, const float *norm_w, float *y,
                           saetta_conv_params cp, saetta_step_params sp);
 
+/* The same call with counters of the caller's in device memory, which make it ONE launch where
+ * the value dim is 128 and the conv has 4 taps (7.1 -> 4.4 us for the model's layer in a graph):
+ * saetta_deltanet_fused_sync_bytes(k_heads) bytes, 4-byte aligned, zero before the first call.
+ * Every call leaves them at zero, so a layer's calls share them as they share its conv state;
+ * calls that may overlap bring different ones.  sync NULL: saetta_deltanet_token. */
+size_t saetta_deltanet_fused_sync_bytes(uint32_t k_heads);
+int saetta_deltanet_token_sync(saetta_stream_t stream, const float *x, const float *w, float *conv_state,
+                               const float *a, const float *b, const float *a_log, const float *dt_bias,
+                               float *state, const float *z, const float *norm_w, float *y,
+                               saetta_conv_params cp, saetta_step_params sp, uint32_t *sync);
+
 /* ---- Gated DeltaNet, several tokens in order: verify rows and prefill chunks -- */
 
 /* conv over `tokens` tokens: kernels conv_rows2 + conv_state
@@ -422,6 +433,13 @@ int saetta_deltanet_rows_fused(saetta_stream_t stream, const float *x, const flo
                                const float *a, const float *b, const float *a_log, const float *dt_bias,
                                float *state, const float *z, const float *norm_w, float *y,
                                float *conv_snaps, float *state_snaps, saetta_rows_fused_params p);
+
+/* The same call with the counters of saetta_deltanet_token_sync: one launch. */
+int saetta_deltanet_rows_fused_sync(saetta_stream_t stream, const float *x, const float *w, float *conv_state,
+                                    const float *a, const float *b, const float *a_log, const float *dt_bias,
+                                    float *state, const float *z, const float *norm_w, float *y,
+                                    float *conv_snaps, float *state_snaps, saetta_rows_fused_params p,
+                                    uint32_t *sync);
 
 /* ---- prefill attention (src/attention_prefill.rs, src/prefill.rs) ---------- */
 

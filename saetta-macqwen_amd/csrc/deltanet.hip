@@ -708,8 +708,177 @@ __global__ __launch_bounds__(256) void deltanet_rows_small_tail_kernel(SmallRows
     }
 }
 
-void launch_small_rows(const SmallRowsArgs &args, hipStream_t stream) {
+// ---- the same in one launch: a workgroup per value head ------------------------------------------
+//
+// Everything after the conv belongs to one value head, so with the head's whole state in one workgroup (64 KB in the
+// registers of 1024 threads) the gated norm needs no second launch.  32 workgroups pull the 2.1 MB of the model's states
+// through 32 CUs: reading and writing them back takes 3.5 us with the launch, against 2.5 us with 256 workgroups, and a
+// second launch in a graph 1.6 us before it does anything.
+// What is left over is the conv state, which is moved in place: the q and k channels of a key head are read by the
+// workgroups of all of its value heads, and may be written only when the last of them has read.  Each of the four waves
+// that hold these channels adds one to a counter of its own when its loads have come back (it has the inputs in registers,
+// and nobody waits); the wave that finds the others there before it is the last and writes the channels and the zero back.
+// The counters (4 per key head, zero before the first call, left at zero) come with the call: see
+// saetta_deltanet_fused_sync_bytes.
+// The snapshots are stored past the caches: as plain stores their lines, 2 MB of dirty data in the L2s per token, are
+// written back when the kernel ends (4 rows 10.7 instead of 8.8 us).  More workgroups to a head, each writing a part of
+// the snapshots, are no faster (9.2 us).
+// Measured per layer (30 layers in a graph, with the two-launch form before it): one token 7.1 -> 4.4 us, 4 rows with
+// snapshots 11.3 -> 8.9; 8 rows 14.2 -> 12.8. (A workgroup stores 64 KB a row, at 1 us each.)
+typedef float nt4 __attribute__((ext_vector_type(4)));
+constexpr int HEAD_THREADS = 1024, HEAD_V_DIM = 128, HEAD_TAPS = 4;
+constexpr int HEAD_QK_WAVES = 2 * K_DIM / 64;  // waves that hold a key head's q and k channels
+
+// M tokens (1..8), 128 value dims, 4 taps.
+template <int M>
+__global__ __launch_bounds__(HEAD_THREADS) void deltanet_head_kernel(SmallRowsArgs a, uint32_t *sync) {
+    constexpr int PAST = HEAD_TAPS - 1;
+    __shared__ __attribute__((aligned(16))) float in_lds[M][2 * K_DIM + HEAD_V_DIM];  // conv outputs: q, k, v
+    __shared__ float gb_lds[M][2];                                                    // decay, beta
+    __shared__ float o_lds[M][HEAD_V_DIM];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, part = lane & 15;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t h = blockIdx.x, v_heads = a.p.v_heads, per_key = v_heads / a.p.k_heads, kh = h / per_key;
+    const uint32_t key_size = a.p.k_heads * K_DIM, channels = a.channels;
+    const size_t value_size = size_t(v_heads) * HEAD_V_DIM;
+    constexpr uint32_t CONV_WAVES = (2 * K_DIM + HEAD_V_DIM) / 64;
+    const bool conv = wave < CONV_WAVES;  // thread = channel: q (waves 0, 1), k (2, 3), v (4, 5)
+    const uint32_t c = tid < K_DIM       ? kh * K_DIM + tid
+                       : tid < 2 * K_DIM ? key_size + kh * K_DIM + (tid - K_DIM)
+                                         : 2 * key_size + h * HEAD_V_DIM + (tid - 2 * K_DIM);
+
+    // Everything is requested before anything is used, the conv's inputs first: loads return in order.
+    float seq[PAST + M];  // stored inputs, oldest first, then the new ones
+    float4 taps;
+    if (conv) {
+        taps = *reinterpret_cast<const float4 *>(a.w + size_t(c) * HEAD_TAPS);
+#pragma unroll
+        for (int k = 0; k < PAST; k++) seq[k] = a.conv_state[size_t(k) * channels + c];
+#pragma unroll
+        for (int t = 0; t < M; t++) seq[PAST + t] = a.x[size_t(t) * channels + c];
+    }
+    float gate_a = 0.0f, gate_b = 0.0f, gate_log = 0.0f, gate_bias = 0.0f;
+    const bool gates = wave == CONV_WAVES && lane < M;
+    if (gates) {
+        gate_a = a.a[size_t(lane) * v_heads + h], gate_b = a.b[size_t(lane) * v_heads + h];
+        gate_log = a.a_log[h], gate_bias = a.dt_bias[h];
+    }
+    // 16 lanes a row of the state, dims 4 part .. + 3 and 64 + 4 part .. + 3; rows 8 wave + lane / 16 and four further
+    const uint32_t row = 8 * wave + (lane >> 4);
+    float *sp = a.state + (size_t(h) * HEAD_V_DIM + row) * K_DIM + part * 4;
+    float4 st[2][2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) st[r][i] = *reinterpret_cast<const float4 *>(sp + r * 4 * K_DIM + i * 64);
+    }
+    const uint32_t out_t = tid / HEAD_V_DIM, out_d = tid % HEAD_V_DIM;  // the output this thread finishes (out_t < M)
+    float z = 0.0f, norm = 0.0f;
+    if (out_t < M) {
+        z = a.z[size_t(out_t) * value_size + size_t(h) * HEAD_V_DIM + out_d];
+        norm = a.norm_w[out_d];
+    }
+
+    if (conv) {
+#pragma unroll
+        for (int t = 0; t < M; t++) {
+            // (the sum as the single-token conv adds it: oldest first)
+            float acc = taps.x * seq[t];
+            acc += taps.y * seq[t + 1];
+            acc += taps.z * seq[t + 2];
+            in_lds[t][tid] = silu_f(acc + taps.w * seq[t + 3]);
+        }
+    }
+    if (gates) fast_gates(gate_a + gate_bias, __expf(gate_log), gate_b, gb_lds[lane][0], gb_lds[lane][1]);
+    __syncthreads();
+
+    // This wave's conv inputs are in registers (its outputs above were made of them).
+    uint32_t before = 0;
+    if (wave < HEAD_QK_WAVES && lane == 0) before = atomicAdd(sync + kh * HEAD_QK_WAVES + wave, 1u);
+
+#pragma unroll
+    for (int t = 0; t < M; t++) {
+        float4 q[2], k[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            q[i] = *reinterpret_cast<const float4 *>(&in_lds[t][64 * i + part * 4]);
+            k[i] = *reinterpret_cast<const float4 *>(&in_lds[t][K_DIM + 64 * i + part * 4]);
+        }
+        const float g = gb_lds[t][0], beta = gb_lds[t][1];
+        // One round of 16-lane sums per token: |q|^2, |k|^2, q.k, and S.k and S.q of both rows, S before the decay and
+        // the update: (g S + d k^T) q = g S q + d (k.q).
+        const float qq = group_reduce<16>(dot4(q[0], q[0]) + dot4(q[1], q[1]), SumOp());
+        const float kk = group_reduce<16>(dot4(k[0], k[0]) + dot4(k[1], k[1]), SumOp());
+        const float kq = group_reduce<16>(dot4(k[0], q[0]) + dot4(k[1], q[1]), SumOp());
+        const float qi = (1.0f / sqrtf(float(K_DIM))) * __builtin_amdgcn_rsqf(qq + a.p.eps), ki = __builtin_amdgcn_rsqf(kk + a.p.eps);
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const float sk = group_reduce<16>(dot4(st[r][0], k[0]) + dot4(st[r][1], k[1]), SumOp());
+            const float sq = group_reduce<16>(dot4(st[r][0], q[0]) + dot4(st[r][1], q[1]), SumOp());
+            const float delta = (in_lds[t][2 * K_DIM + row + 4 * r] - g * ki * sk) * beta * ki;
+            const float o = qi * (g * sq + delta * kq);
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                st[r][i].x = g * st[r][i].x + delta * k[i].x, st[r][i].y = g * st[r][i].y + delta * k[i].y;
+                st[r][i].z = g * st[r][i].z + delta * k[i].z, st[r][i].w = g * st[r][i].w + delta * k[i].w;
+            }
+            if (part == 0) o_lds[t][row + 4 * r] = o;
+        }
+        if (a.p.snapshots) {
+            float *snap = a.state_snaps + size_t(t) * value_size * K_DIM + (size_t(h) * HEAD_V_DIM + row) * K_DIM + part * 4;
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+#pragma unroll
+                for (int i = 0; i < 2; i++) __builtin_nontemporal_store(__builtin_bit_cast(nt4, st[r][i]), reinterpret_cast<nt4 *>(snap + r * 4 * K_DIM + i * 64));
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) *reinterpret_cast<float4 *>(sp + r * 4 * K_DIM + i * 64) = st[r][i];
+    }
+    __syncthreads();
+    if (out_t < M) {
+        // the head's outputs of the token, two per lane of either of its waves
+        const float o0 = o_lds[out_t][lane], o1 = o_lds[out_t][lane + 64];
+        const float total = group_reduce<64>(o0 * o0 + o1 * o1, SumOp());
+        const float inv = 1.0f / sqrtf(total / float(HEAD_V_DIM) + a.p.eps);
+        a.y[size_t(out_t) * value_size + size_t(h) * HEAD_V_DIM + out_d] = (out_d < 64 ? o0 : o1) * (inv * norm) * silu_f(z);
+    }
+    if (conv) {
+        // after token t the conv state is the inputs t + 1 .. t + PAST of the sequence
+        const bool own = wave >= HEAD_QK_WAVES;
+        if (a.p.snapshots && (own || h == kh * per_key)) {
+#pragma unroll
+            for (int t = 0; t < M; t++) {
+#pragma unroll
+                for (int j = 0; j < PAST; j++) __builtin_nontemporal_store(seq[t + 1 + j], a.conv_snaps + (size_t(t) * PAST + j) * channels + c);
+            }
+        }
+        if (own || uint32_t(__builtin_amdgcn_readfirstlane(before)) == per_key - 1) {
+#pragma unroll
+            for (int j = 0; j < PAST; j++) a.conv_state[size_t(j) * channels + c] = seq[M + j];
+            if (!own && lane == 0) __hip_atomic_store(sync + kh * HEAD_QK_WAVES + wave, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+
+template <int M>
+void launch_head_rows(const SmallRowsArgs &args, uint32_t *sync, hipStream_t stream) {
+    if (args.p.rows == uint32_t(M)) {
+        launch(deltanet_head_kernel<M>, dim3(args.p.v_heads), HEAD_THREADS, 0, stream, args, sync);
+    } else if constexpr (M < SMALL_ROWS_MAX) {
+        launch_head_rows<M + 1>(args, sync, stream);
+    }
+}
+
+void launch_small_rows(const SmallRowsArgs &args, uint32_t *sync, hipStream_t stream) {
     const saetta_rows_fused_params &p = args.p;
+    if (sync && p.v_dim == HEAD_V_DIM && p.kernel_size == HEAD_TAPS && aligned(args.w, 16)) {
+        launch_head_rows<1>(args, sync, stream);
+        return;
+    }
     const dim3 grid((p.v_dim + 15) / 16, p.v_heads);
     if (p.snapshots) {
         launch(deltanet_rows_small_kernel<true>, grid, SMALL_THREADS, 0, stream, args);
@@ -852,10 +1021,19 @@ extern "C" int saetta_deltanet_rows_ws(saetta_stream_t stream, const float *mixe
     return launch_status("deltanet_rows");
 }
 
+extern "C" size_t saetta_deltanet_fused_sync_bytes(uint32_t k_heads) { return size_t(k_heads) * HEAD_QK_WAVES * sizeof(uint32_t); }
+
 extern "C" int saetta_deltanet_token(saetta_stream_t stream, const float *x, const float *w, float *conv_state,
                                      const float *a, const float *b, const float *a_log, const float *dt_bias,
                                      float *state, const float *z, const float *norm_w, float *y,
                                      saetta_conv_params cp, saetta_step_params sp) {
+    return saetta_deltanet_token_sync(stream, x, w, conv_state, a, b, a_log, dt_bias, state, z, norm_w, y, cp, sp, nullptr);
+}
+
+extern "C" int saetta_deltanet_token_sync(saetta_stream_t stream, const float *x, const float *w, float *conv_state,
+                                          const float *a, const float *b, const float *a_log, const float *dt_bias,
+                                          float *state, const float *z, const float *norm_w, float *y,
+                                          saetta_conv_params cp, saetta_step_params sp, uint32_t *sync) {
     SAETTA_REQUIRE(x && w && conv_state && a && b && a_log && dt_bias && state && z && norm_w && y, SAETTA_E_NULL,
                    "deltanet_token: null buffer");
     SAETTA_REQUIRE(cp.kernel_size >= 2 && cp.kernel_size <= 16, SAETTA_E_SHAPE, "deltanet_token: kernel size %u (2..16)",
@@ -866,11 +1044,11 @@ extern "C" int saetta_deltanet_token(saetta_stream_t stream, const float *x, con
                    sp.v_dim);
     SAETTA_REQUIRE(cp.channels == 2 * sp.k_heads * K_DIM + sp.v_heads * sp.v_dim, SAETTA_E_SHAPE,
                    "deltanet_token: %u channels, the heads make %u", cp.channels, 2 * sp.k_heads * K_DIM + sp.v_heads * sp.v_dim);
-    SAETTA_REQUIRE(aligned(state, 16), SAETTA_E_ALIGN, "deltanet_token: the state must be 16-byte aligned");
+    SAETTA_REQUIRE(aligned(state, 16) && aligned(sync, 4), SAETTA_E_ALIGN, "deltanet_token: the state must be 16-byte aligned");
     if (int rc = ensure_device()) return rc;
     const saetta_rows_fused_params p{sp.k_heads, sp.v_heads, sp.v_dim, cp.kernel_size, sp.eps, 1, 0};
     SmallRowsArgs args{x, w, conv_state, a, b, a_log, dt_bias, state, z, norm_w, y, nullptr, nullptr, p, cp.channels};
-    launch_small_rows(args, as_stream(stream));
+    launch_small_rows(args, sync, as_stream(stream));
     return launch_status("deltanet_token");
 }
 
@@ -878,6 +1056,15 @@ extern "C" int saetta_deltanet_rows_fused(saetta_stream_t stream, const float *x
                                           const float *a, const float *b, const float *a_log, const float *dt_bias,
                                           float *state, const float *z, const float *norm_w, float *y,
                                           float *conv_snaps, float *state_snaps, saetta_rows_fused_params p) {
+    return saetta_deltanet_rows_fused_sync(stream, x, w, conv_state, a, b, a_log, dt_bias, state, z, norm_w, y, conv_snaps,
+                                           state_snaps, p, nullptr);
+}
+
+extern "C" int saetta_deltanet_rows_fused_sync(saetta_stream_t stream, const float *x, const float *w, float *conv_state,
+                                               const float *a, const float *b, const float *a_log, const float *dt_bias,
+                                               float *state, const float *z, const float *norm_w, float *y,
+                                               float *conv_snaps, float *state_snaps, saetta_rows_fused_params p,
+                                               uint32_t *sync) {
     SAETTA_REQUIRE(x && w && conv_state && a && b && a_log && dt_bias && state && z && norm_w && y, SAETTA_E_NULL,
                    "deltanet_rows_fused: null buffer");
     SAETTA_REQUIRE(!p.snapshots || (conv_snaps && state_snaps), SAETTA_E_NULL,
@@ -889,12 +1076,12 @@ extern "C" int saetta_deltanet_rows_fused(saetta_stream_t stream, const float *x
                    "deltanet_rows_fused: %u value heads over %u key heads", p.v_heads, p.k_heads);
     SAETTA_REQUIRE(p.v_dim >= 1 && p.v_dim <= 256, SAETTA_E_SHAPE,
                    "deltanet_rows_fused: value dim %u (1..256); the key dim is 128", p.v_dim);
-    SAETTA_REQUIRE(aligned(state, 16) && (!p.snapshots || aligned(state_snaps, 16)), SAETTA_E_ALIGN,
+    SAETTA_REQUIRE(aligned(state, 16) && (!p.snapshots || aligned(state_snaps, 16)) && aligned(sync, 4), SAETTA_E_ALIGN,
                    "deltanet_rows_fused: the state and its snapshots must be 16-byte aligned");
     if (int rc = ensure_device()) return rc;
     if (p.rows == 0) return SAETTA_OK;
     const uint32_t channels = 2 * p.k_heads * K_DIM + p.v_heads * p.v_dim;
     SmallRowsArgs args{x, w, conv_state, a, b, a_log, dt_bias, state, z, norm_w, y, conv_snaps, state_snaps, p, channels};
-    launch_small_rows(args, as_stream(stream));
+    launch_small_rows(args, sync, as_stream(stream));
     return launch_status("deltanet_rows_fused");
 }

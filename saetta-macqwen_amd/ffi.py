@@ -8,7 +8,8 @@ LIB_PATH = os.environ.get("SAETTA_HIP_LIB") or os.path.join(_HERE, "lib", "libsa
 # Every symbol include/saetta_hip.h declares; tests check the library exports each.
 SYMBOLS = [
     "saetta_init", "saetta_last_error", "saetta_device_status", "saetta_token_params_set", "saetta_plan_begin",
-    "saetta_plan_end", "saetta_plan_launches", "saetta_plan_run", "saetta_plan_free", "saetta_kv_quantize", "saetta_kv_dequantize", "saetta_kv_dequantize_f32", "saetta_to_half", "saetta_attn_prep_store", "saetta_deltanet_conv", "saetta_deltanet_step", "saetta_deltanet_conv_rows", "saetta_deltanet_rows", "saetta_deltanet_rows_ws", "saetta_deltanet_rows_workspace_bytes", "saetta_deltanet_token", "saetta_deltanet_rows_fused",
+    "saetta_plan_end", "saetta_plan_launches", "saetta_plan_run", "saetta_plan_free", "saetta_kv_quantize", "saetta_kv_dequantize", "saetta_kv_dequantize_f32", "saetta_to_half", "saetta_attn_prep_store", "saetta_deltanet_conv", "saetta_deltanet_step", "saetta_deltanet_conv_rows", "saetta_deltanet_rows", "saetta_deltanet_rows_ws", "saetta_deltanet_rows_workspace_bytes", "saetta_deltanet_token", "saetta_deltanet_rows_fused", "saetta_deltanet_fused_sync_bytes",
+    "saetta_deltanet_token_sync", "saetta_deltanet_rows_fused_sync",
     "saetta_part_o_bytes", "saetta_part_ml_bytes", "saetta_attn_decode", "saetta_attn_decode_quant",
     "saetta_attn_rows", "saetta_attn_rows_quant", "saetta_static_scratch_bytes", "saetta_attn_decode_quant_static", "saetta_prefill_workspace_bytes", "saetta_attn_prefill", "saetta_attn_prefill_quant",
     "saetta_attn_gemm_workspace_bytes", "saetta_attn_gemm",
@@ -83,6 +84,11 @@ def lib():
         l.saetta_deltanet_step.argtypes = [vp] * 12 + [StepParamsC]
         l.saetta_deltanet_token.restype = i32
         l.saetta_deltanet_token.argtypes = [vp] * 12 + [ConvParamsC, StepParamsC]
+        l.saetta_deltanet_fused_sync_bytes.restype, l.saetta_deltanet_fused_sync_bytes.argtypes = sz, [u32]
+        l.saetta_deltanet_token_sync.restype = i32
+        l.saetta_deltanet_token_sync.argtypes = [vp] * 12 + [ConvParamsC, StepParamsC, vp]
+        l.saetta_deltanet_rows_fused_sync.restype = i32
+        l.saetta_deltanet_rows_fused_sync.argtypes = [vp] * 14 + [RowsFusedParamsC, vp]
         l.saetta_deltanet_rows_fused.restype = i32
         l.saetta_deltanet_rows_fused.argtypes = [vp] * 14 + [RowsFusedParamsC]
         l.saetta_deltanet_conv_rows.restype = i32

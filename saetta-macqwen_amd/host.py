@@ -138,9 +138,17 @@ class Plan:
         self.device = torch.device(device)
         self.params = torch.zeros(4, dtype=torch.int32, device=self.device)
         self.ops = []  # (kernel name, callable(stream))
+        self._counters = None
 
     def op(self, kernel, launch):
         self.ops.append((kernel, launch))
+
+    def counters(self, n):
+        """n zeros (int32) of this plan's own, for an op whose workgroups count one another."""
+        if self._counters is None or self._counters.numel() < n:
+            self._counters = torch.zeros(max(n, 4096), dtype=torch.int32, device=self.device)
+        taken, self._counters = self._counters[:n], self._counters[n:]
+        return taken
 
     def set_params(self, tp):
         """Plan::set_params (src/plan.rs:144-146): one small launch on the current stream that carries the
@@ -475,7 +483,9 @@ def deltanet_token(plan, x, w, conv_state, a, b, a_log, dt_bias, state, z, norm_
             or state.numel() < v_heads * v_dim * 128 or y.numel() < v_heads * v_dim or z.numel() < v_heads * v_dim):
         raise ValueError("deltanet_token: buffers too small")
     cp, sp = ffi.ConvParamsC(channels, kernel_size), ffi.StepParamsC(k_heads, v_heads, v_dim, eps)
-    plan.op("deltanet_token", _Call("saetta_deltanet_token", "deltanet_token", (*[_ptr(t) for t in ts], cp, sp), ts))
+    sync = plan.counters(ffi.lib().saetta_deltanet_fused_sync_bytes(k_heads) // 4)
+    plan.op("deltanet_token", _Call("saetta_deltanet_token_sync", "deltanet_token", (
+        *[_ptr(t) for t in ts], cp, sp, _ptr(sync)), (*ts, sync)))
 
 
 def deltanet_conv_rows(plan, x, w, state, out, channels, kernel_size, tokens, snaps=None):
@@ -550,9 +560,10 @@ def deltanet_rows_fused(plan, x, w, conv_state, a, b, a_log, dt_bias, state, z, 
         if conv_snaps.numel() < rows * (kernel_size - 1) * channels or state_snaps.numel() < rows * v_heads * v_dim * 128:
             raise ValueError("deltanet_rows_fused: snapshots too small")
     p = ffi.RowsFusedParamsC(k_heads, v_heads, v_dim, kernel_size, eps, rows, int(conv_snaps is not None))
-    plan.op("deltanet_rows_fused", _Call("saetta_deltanet_rows_fused", "deltanet_rows_fused", (
+    sync = plan.counters(ffi.lib().saetta_deltanet_fused_sync_bytes(k_heads) // 4)
+    plan.op("deltanet_rows_fused", _Call("saetta_deltanet_rows_fused_sync", "deltanet_rows_fused", (
         *[_ptr(t) for t in ts], _ptr(conv_snaps) if conv_snaps is not None else None,
-        _ptr(state_snaps) if state_snaps is not None else None, p), (*ts, conv_snaps, state_snaps)))
+        _ptr(state_snaps) if state_snaps is not None else None, p, _ptr(sync)), (*ts, conv_snaps, state_snaps, sync)))
 
 
 KV_ALIGN = 128  # src/gpu_layers.rs:199: the decode chunk, and a multiple of the prefill key block

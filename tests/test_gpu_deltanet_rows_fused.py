@@ -109,3 +109,22 @@ def test_rejections():
     saetta.deltanet_rows_fused(plan, z, z, z, z, z, z, z, z, z, z, z, 1, 2, 8, 17, 2, EPS)
     with pytest.raises(saetta.ffi.SaettaError, match="kernel size"):
         plan.build().run()
+
+
+@pytest.mark.parametrize("k_heads,v_heads,rows", [(1, 1, 1), (1, 3, 8), (2, 4, 1), (3, 3, 2), (2, 8, 5)])
+def test_heads_that_share_conv_channels(k_heads, v_heads, rows):
+    # 128 value dims and 4 taps: one workgroup per value head, the q and k channels of a key head written back by
+    # the last of its heads' workgroups, which count one another; the counts are zero again after every call.
+    layer = Layer(k_heads, v_heads, 128, 4, seed=100 * k_heads + v_heads)
+    check(layer, [rows, rows, 1], snapshots=True)
+    conv, state = layer.zero_state()
+    x, z, a, b = (dev(np.ascontiguousarray(t)) for t in layer.inputs(rows))
+    y = torch.empty(rows, layer.val, device="cuda")
+    plan = saetta.Plan()
+    saetta.deltanet_rows_fused(plan, x, dev(layer.conv_w), conv, a, b, dev(layer.a_log), dev(layer.dt_bias), state, z,
+                               dev(layer.norm), y, k_heads, v_heads, 128, 4, rows, EPS)
+    sync = plan.ops[0][1].keep[-1]
+    assert sync.numel() == 4 * k_heads
+    for _ in range(3):
+        plan.build().run()
+        assert not host(sync).any()
