@@ -42,6 +42,7 @@
 #include "common.hpp"
 #include "lanes.hpp"
 
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -735,6 +736,306 @@ __global__ __launch_bounds__(MERGE_THREADS) void prefill_merge_kernel(PrefillArg
     }
 }
 
+// ---- short chunks over short contexts: one launch ------------------------------------------------
+//
+// A chunk of 166 tokens is 22 workgroups of the kernel above, which then walk their 166 keys in three steps behind a
+// prologue and an epilogue of 7 us, and the prepare kernel is 3.8 us more before them: 22 us in all for 2 us of work.
+// Here a workgroup takes ONE row group (4 tokens x 8 heads = 32 rows) of a kv head, eight times as many workgroups, and
+// its 8 waves take alternate blocks of 32 keys, so that 256 keys are one step; each wave keeps its own (m, l, O) and they
+// are joined at the end, each wave finishing 32 of the 256 dims.  Nothing of a block is shared between waves, so the
+// cache is read where it lies, once per row group: the keys go from memory to MFMA operands in registers, the values to a
+// tile of the wave's own in LDS, row by row as in memory, and come back transposed (ds_read_b64_tr_b16).  Codes are
+// dequantized on the way, with the arithmetic of the prepare kernel.
+// The price is that every row group pulls (and dequantizes) the keys for itself: from some hundred keys on the tiles of 16
+// tokens and their images win; the line is in flash_plan.
+// Measured, the whole call, halves (tiles before): 16 tokens at 16 18.3 -> 7.5 us, 166 from 0 21.7 -> 10.8, 500 from 0
+// 31.2 -> 19.2.  A block of keys per wave takes 5 us with eight waves at it: 256 KB through the CU's 64 bytes a cycle are
+// 1.8 of them, the values' way through LDS and the query operands 1.4.
+constexpr int SMALL_WAVES = 8, SMALL_THREADS = 64 * SMALL_WAVES;
+
+struct SmallArgs {
+    const uint16_t *q;  // f16 [tokens][heads][256]
+    const unsigned char *kdata, *vdata;
+    const uint16_t *kscales, *kbiases, *vscales, *vbiases;
+    const float *q_and_gate;
+    float *out;
+    uint32_t heads, kv_heads, pos, tokens;
+    float scale;
+};
+
+template <int BITS>
+struct SmallLds {
+    // the values of a wave's block: f16 rows as in memory.  Codes: rows of 576 bytes, halves (copied in by 16-byte pieces in
+    // whole kilobytes): rows of 512 rotated by 64 bytes per row; either way the four rows of a transposing read, 32 bytes
+    // each, and those of its neighbours fall on different banks.
+    static constexpr int VROW = BITS == 16 ? 512 : 576;
+    static constexpr int VTILE = BK * VROW;
+    static constexpr int Q_OFF = 0, V_OFF = 16 * 1024;
+    // the merge, over both: four waves' O at a time, [wave][8 dim tiles][4][64 lanes][16 bytes], and [wave][row][m, l]
+    static constexpr int ML_OFF = 4 * 32 * 1024;
+    static constexpr int MERGE_BYTES = ML_OFF + SMALL_WAVES * 32 * 8;
+    static constexpr int TILES_BYTES = V_OFF + SMALL_WAVES * VTILE;
+    static constexpr int BYTES = TILES_BYTES > MERGE_BYTES ? TILES_BYTES : MERGE_BYTES;
+    static_assert(BYTES <= 160 * 1024, "LDS of a CU");
+};
+
+// Which dims MFMA k-step st holds in lane half hf (8 of them): what a 16-byte piece of a row gives, whatever a value's size.
+template <int BITS>
+__device__ __forceinline__ constexpr int small_dim(int st, int hf) {
+    constexpr int STEPS = 16 / BITS;  // k-steps per piece
+    return (st / STEPS * 2 + hf) * 8 * STEPS + st % STEPS * 8;
+}
+
+template <int BITS>
+__global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallArgs a) {
+    using L = SmallLds<BITS>;
+    constexpr int RB = row_bytes<BITS>(), PIECES = RB / 16, STEPS = 16 / BITS, VALUES = 128 / BITS;  // pieces of a row; values of one
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 31, hf = lane >> 5;
+    const uint32_t kv = blockIdx.y, kvh = a.kv_heads;
+    const uint32_t tok0 = (gridDim.x - 1 - blockIdx.x) * 4;  // (the row groups that see the most keys first)
+    const uint32_t tok = tok0 + (col >> 3), head = kv * SAETTA_GQA_GROUP + (col & 7);
+    const float c = a.scale * 1.4426950408889634f;
+    const uint32_t keys = a.pos + min(tok0 + 4, a.tokens);  // what the last of its tokens sees
+    const uint32_t nblocks = (keys + BK - 1) / BK;
+    const uint32_t active = min(nblocks, uint32_t(SMALL_WAVES));  // waves that have a block
+    const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(lds));
+    const uint32_t vtile = lds0 + L::V_OFF + wave * L::VTILE;
+
+    // ---- what a block needs of memory ----
+    u32x4 kreg[PIECES / 2];           // lane (key col, half hf): the pieces 2i + hf of its row
+    u32x2 kss = {0, 0}, kzs = {0, 0};  // scales and biases of the key's four groups
+    constexpr int V_LOADS = BK * PIECES / 64, V_KEYS = 64 / PIECES;  // loads that bring the values; keys of one
+    u32x4 vreg[BITS == 16 ? 1 : V_LOADS];
+    uint32_t vss[BITS == 16 ? 1 : V_LOADS], vzs[BITS == 16 ? 1 : V_LOADS];
+    const uint32_t vp = lane % PIECES, vk = lane / PIECES;  // codes: the lane's piece and key of a load
+    auto row_of = [&](uint32_t key) { return size_t(min(key, keys - 1)) * kvh + kv; };  // (past the end: the last row, masked)
+    auto fetch_keys = [&](uint32_t b) {
+        const size_t row = row_of(b * BK + col);
+        const u32x4 *src = reinterpret_cast<const u32x4 *>(a.kdata + row * RB) + hf;
+#pragma unroll
+        for (int i = 0; i < PIECES / 2; i++) kreg[i] = src[2 * i];
+        if constexpr (BITS != 16) {
+            kss = *reinterpret_cast<const u32x2 *>(a.kscales + row * 4);
+            kzs = *reinterpret_cast<const u32x2 *>(a.kbiases + row * 4);
+        }
+    };
+    auto fetch_values = [&](uint32_t b) {
+        if constexpr (BITS == 16) {
+            // straight to the tile: place p of row k holds piece p - 4 (k % 4)
+#pragma unroll
+            for (int u = 0; u < V_LOADS; u++) {
+                const uint32_t k = 2 * u + (lane >> 5);
+                const uint64_t src = reinterpret_cast<uint64_t>(a.vdata) + row_of(b * BK + k) * RB + ((lane - 4 * (k & 3)) & 31) * 16;
+                asm volatile("s_mov_b32 m0, %0\n"
+                             "s_nop 0\n"
+                             "global_load_lds_dwordx4 %1, off\n"
+                             :
+                             : "s"(vtile + u * 1024), "v"(src)
+                             : "memory", "m0");
+            }
+            // (loads into registers and into LDS do not come back in one order, and the compiler counts only the former:
+            // all that is out is waited for here, in front of anything it may do with the keys)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        } else {
+#pragma unroll
+            for (int u = 0; u < V_LOADS; u++) {
+                const size_t row = row_of(b * BK + u * V_KEYS + vk);
+                vreg[u] = *reinterpret_cast<const u32x4 *>(a.vdata + row * RB + vp * 16);
+                vss[u] = a.vscales[row * 4 + vp * 4 / PIECES], vzs[u] = a.vbiases[row * 4 + vp * 4 / PIECES];
+            }
+        }
+    };
+    // The 8 values of sub-step `sub` of a piece, as halves.
+    auto eight = [&](const u32x4 &piece, int sub, float s, float z) {
+        if constexpr (BITS == 16) {
+            return __builtin_bit_cast(half8, piece);
+        } else {
+            uint32_t o[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                constexpr int PER = 32 / BITS;
+                const int at = 8 * sub + 2 * i;
+                o[i] = pack_half2(dequant(s, z, code_of<BITS>(piece[at / PER], at % PER)), dequant(s, z, code_of<BITS>(piece[at / PER], at % PER + 1)));
+            }
+            return __builtin_bit_cast(half8, u32x4{o[0], o[1], o[2], o[3]});
+        }
+    };
+
+    if (uint32_t(wave) < active) fetch_keys(wave);
+    // Q^T operands: through LDS, where all waves read them
+    {
+        half8 qv[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int st = 2 * wave + i;
+            qv[i] = *reinterpret_cast<const half8 *>(a.q + (size_t(min(tok, a.tokens - 1)) * a.heads + head) * DIM + small_dim<BITS>(st, hf));
+        }
+        if (uint32_t(wave) < active) fetch_values(wave);
+#pragma unroll
+        for (int i = 0; i < 2; i++) *reinterpret_cast<half8 *>(lds + L::Q_OFF + (2 * wave + i) * 1024 + lane * 16) = qv[i];
+    }
+    lds_barrier();
+
+    floatx16 acc[8];
+#pragma unroll
+    for (int mt = 0; mt < 8; mt++) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[mt][r] = 0.0f;
+    }
+    float m = 0.25f * NO_SCORE * c, l = 0.0f;  // (above a masked score, as in the kernel above)
+    for (uint32_t b = wave; b < nblocks; b += SMALL_WAVES) {
+        // ---- S^T = K Q^T ----
+        floatx16 s;
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[r] = 0.0f;
+#pragma unroll
+        for (int st = 0; st < 16; st++) {
+            const int i = st / STEPS;
+            float ks = 0.0f, kz = 0.0f;
+            if constexpr (BITS != 16) {
+                const int g = i * 2 * VALUES / SAETTA_QUANT_GROUP;
+                ks = h2f(kss[g >> 1] >> (16 * (g & 1))), kz = h2f(kzs[g >> 1] >> (16 * (g & 1)));
+            }
+            const half8 q = *reinterpret_cast<const half8 *>(lds + L::Q_OFF + st * 1024 + lane * 16);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(eight(kreg[i], st % STEPS, ks, kz), q, s, 0, 0, 0);
+        }
+        if (b + SMALL_WAVES < nblocks) fetch_keys(b + SMALL_WAVES);
+        // ---- softmax: register r is key 4 hf + r % 4 + 8 (r / 4) of the block, the lane's row col ----
+        const uint32_t key0 = b * BK;
+        if (key0 + BK > a.pos + tok0 + 1) {
+            const uint32_t len = a.pos + tok + 1, vis = len > key0 ? len - key0 : 0;
+#pragma unroll
+            for (int r = 0; r < 16; r++) s[r] = uint32_t(4 * hf + (r & 3) + 8 * (r >> 2)) < vis ? s[r] : NO_SCORE;
+        }
+        float bm = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; r++) bm = fmaxf(bm, s[r]);
+        bm = fmaxf(max_across_halves(bm) * c, NO_SCORE);
+        if (__any(bm > m + TAU)) {
+            const float m_new = bm > m + TAU ? bm : m, alpha = __builtin_amdgcn_exp2f(m - m_new);
+            m = m_new, l *= alpha;
+#pragma unroll
+            for (int mt = 0; mt < 8; mt++) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[mt][r] *= alpha;
+            }
+        }
+        half8 p[2];
+        float sum = 0.0f;
+#pragma unroll
+        for (int sp = 0; sp < 2; sp++) {
+            uint32_t w[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float x = __builtin_amdgcn_exp2f(fmaf(s[8 * sp + 2 * i], c, -m)), y = __builtin_amdgcn_exp2f(fmaf(s[8 * sp + 2 * i + 1], c, -m));
+                sum += x + y;
+                w[i] = pack_half2(x, y);
+            }
+            p[sp] = __builtin_bit_cast(half8, u32x4{w[0], w[1], w[2], w[3]});
+        }
+        l += sum;
+        // ---- the values to the wave's tile (halves: they are there) ----
+        if constexpr (BITS != 16) {
+#pragma unroll
+            for (int u = 0; u < V_LOADS; u++) {
+                const float vs = h2f(vss[u]), vz = h2f(vzs[u]);
+                half8 *dst = reinterpret_cast<half8 *>(lds + L::V_OFF + wave * L::VTILE + (u * V_KEYS + vk) * L::VROW + vp * VALUES * 2);
+#pragma unroll
+                for (int sub = 0; sub < STEPS; sub++) dst[sub] = eight(vreg[u], sub, vs, vz);
+            }
+            if (b + SMALL_WAVES < nblocks) fetch_values(b + SMALL_WAVES);
+        }
+        // ---- O^T += V^T P^T: k-step sp, lane half hf: keys 16 sp + 4 hf .. + 3 and 8 further; a wave's LDS accesses run in order ----
+        const uint32_t e = (lane >> 2) & 3, dim = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+        const uint32_t vrow = vtile + (4 * hf + e) * L::VROW;
+#pragma unroll
+        for (int mt = 0; mt < 8; mt++) {
+            const uint32_t d = BITS == 16 ? ((32 * mt + dim) * 2 + 64 * e) & 511 : (32 * mt + dim) * 2;
+            u32x2 r[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(r[i]) : "v"(vrow + d + 8 * i * L::VROW) : "memory");
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3])::"memory");
+#pragma unroll
+            for (int sp = 0; sp < 2; sp++) {
+                const half8 v = __builtin_bit_cast(half8, u32x4{r[2 * sp].x, r[2 * sp].y, r[2 * sp + 1].x, r[2 * sp + 1].y});
+                acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, p[sp], acc[mt], 0, 0, 0);
+            }
+        }
+        if constexpr (BITS == 16) {
+            if (b + SMALL_WAVES < nblocks) fetch_values(b + SMALL_WAVES);
+        }
+    }
+
+    // ---- the waves' parts joined: wave w finishes dims 32 w .. 32 w + 31 ----
+    const size_t row = size_t(min(tok, a.tokens - 1)) * a.heads + head;
+    float4 g[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) g[i] = *reinterpret_cast<const float4 *>(a.q_and_gate + row * 2 * DIM + DIM + 32 * wave + 8 * i + 4 * hf);
+    lds_barrier();  // every wave is through with its tile and the query operands
+    float2 *ml = reinterpret_cast<float2 *>(lds + L::ML_OFF);
+    const float l_row = l + __shfl_xor(l, 32);
+    if (hf == 0) ml[wave * 32 + col] = float2{m, l_row};
+    auto tile_of = [&](int w, int mt) { return reinterpret_cast<float4 *>(lds + (w & 3) * 32768 + mt * 4096) + lane; };
+    floatx16 fin;
+#pragma unroll
+    for (int r = 0; r < 16; r++) fin[r] = 0.0f;
+    auto hand_out = [&]() {  // this wave's O, all dims
+#pragma unroll
+        for (int mt = 0; mt < 8; mt++) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) tile_of(wave, mt)[i * 64] = float4{acc[mt][4 * i], acc[mt][4 * i + 1], acc[mt][4 * i + 2], acc[mt][4 * i + 3]};
+        }
+    };
+    float weight[SMALL_WAVES], l_all = 0.0f;
+    auto take_in = [&](int first) {  // the dims this wave finishes, from waves first .. first + 3
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            if (uint32_t(first + w) < active) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float4 x = tile_of(w, wave)[i * 64];
+                    fin[4 * i] += x.x * weight[first + w], fin[4 * i + 1] += x.y * weight[first + w];
+                    fin[4 * i + 2] += x.z * weight[first + w], fin[4 * i + 3] += x.w * weight[first + w];
+                }
+            }
+        }
+    };
+    if (wave < 4 && uint32_t(wave) < active) hand_out();
+    lds_barrier();
+    {
+        float2 x[SMALL_WAVES];
+        float top = 4.0f * NO_SCORE;
+#pragma unroll
+        for (int w = 0; w < SMALL_WAVES; w++) x[w] = ml[w * 32 + col];  // (a wave without a block: l = 0)
+#pragma unroll
+        for (int w = 0; w < SMALL_WAVES; w++) top = fmaxf(top, x[w].x);
+#pragma unroll
+        for (int w = 0; w < SMALL_WAVES; w++) weight[w] = __builtin_amdgcn_exp2f(x[w].x - top), l_all += x[w].y * weight[w];
+    }
+    take_in(0);
+    if (active > 4) {
+        lds_barrier();
+        if (wave >= 4 && uint32_t(wave) < active) hand_out();
+        lds_barrier();
+        take_in(4);
+    }
+    if (tok < a.tokens) {
+        const float inv = 1.0f / l_all;
+        float *out = a.out + row * DIM + 32 * wave + 4 * hf;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float4 w;
+            w.x = fin[4 * i] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].x));
+            w.y = fin[4 * i + 1] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].y));
+            w.z = fin[4 * i + 2] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].z));
+            w.w = fin[4 * i + 3] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].w));
+            *reinterpret_cast<float4 *>(out + 8 * i) = w;
+        }
+    }
+}
+
 // Workspaces the library owns when the caller passes none: one per (device, stream), grown on demand,
 // so that calls on different streams never share one (work on one stream runs in order).  They are
 // kept until the process ends: a caller with many short-lived streams passes its own.
@@ -753,13 +1054,20 @@ size_t images_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) {
 }
 size_t plain_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) { return images_bytes(pos, tokens, kv_heads) + 256; }
 
-// Compute units of the current device.
+// Compute units of the current device (asked for once per device).
 uint32_t cu_count() {
+    static std::atomic<int> known[OWNED_DEVICES];
     int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= OWNED_DEVICES) {
         (void)hipGetLastError();
-        cus = 256;
+        return 256;
     }
+    if ((cus = known[dev].load(std::memory_order_relaxed)) > 0) return uint32_t(cus);
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
+        (void)hipGetLastError();
+        return 256;
+    }
+    known[dev].store(cus, std::memory_order_relaxed);
     return uint32_t(cus);
 }
 
@@ -771,25 +1079,41 @@ uint32_t parts_of(uint32_t pos, uint32_t tokens, uint32_t part_blocks) {
     return (uint32_t((uint64_t(pos) + tokens + BK - 1) / BK) + part_blocks - 1) / part_blocks;
 }
 
-// Blocks of keys per part of a tile's keys, or 0: the keys are not split.  A tile is one workgroup's work, and 16 tokens
-// of 2 kv heads are all a CU gets of it: chunks under 2048 tokens leave CUs idle, and between 2048 and 4096 a second round
-// of tiles fills a part of them.  The rule takes the smallest of what the rounds of workgroups would take, in us, out of
-// 1 to 32 parts, from figures measured on the MI355X: a workgroup's block of 32 keys takes 0.6 us while the chip has
-// power to spare (up to ~170 workgroups) and the chip as a whole 284 blocks a us beyond that; the ends of an item (its
-// first loads, the store of its part) 12 us, with the gate 14.5; the merge a launch and 128 KB read back per item.
+// How a chunk's launches are laid out: the row groups' own launch (small), or tiles, with their keys in parts of
+// `part_blocks` blocks where that is not 0.
+struct FlashPlan {
+    bool small;
+    uint32_t cus, part_blocks, nparts;
+    size_t plain, parts;  // bytes of workspace: the images and the tile count; the parts behind them
+    size_t bytes() const { return plain + parts; }
+};
+
+// A tile is one workgroup's work, and 16 tokens of 2 kv heads are all a CU gets of it: chunks under 2048 tokens leave CUs
+// idle, and between 2048 and 4096 a second round of tiles fills a part of them.  The rule takes the smallest of what the
+// rounds of workgroups would take, in us, unsplit and with the keys in 2 to 32 parts, from figures measured on the MI355X:
+// a workgroup's block of 32 keys takes 0.6 us while the chip has power to spare (up to ~170 workgroups) and the chip as a
+// whole 284 blocks a us beyond that; the ends of an item (its first loads, the store of its part) 12 us, with the gate
+// 14.5; the merge a launch and 128 KB read back per item.  The small kernel's workgroups take as long for a block, with a
+// quarter of the rows, but their ends take 7 us (8.5 with codes) and there are no images to prepare (4 us and more).
 // Measured, unsplit -> split by this rule, the whole call (8-bit cache): 100 tokens at 10000: 211 -> 47 us, at 100000
 // (4-bit): 1886 -> 225; 500 at 40000: 770 -> 330; 2100 at 9000: 497 -> 405.  A full chunk (4096 tokens: two whole rounds)
-// is never split.
-uint32_t choose_part_blocks(uint32_t pos, uint32_t tokens, uint32_t kv_heads, uint32_t cus) {
+// is never split.  Tiles -> the small kernel: 16 tokens at 16 18.6 -> 8.6, 300 from 0 24.6 -> 16.7, 500 at 500 36.8 -> 30.4;
+// past its line 100 at 1000 would take 29.4 for 27.5, 700 at 700 (halves) 51.5 for 41.9.
+FlashPlan flash_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, int bits) {
     constexpr float BLOCK_US = 0.6f, CHIP_BLOCKS_PER_US = 284.0f / 256.0f, PART_US = 12.0f, TILE_US = 14.5f, MERGE_US = 4.0f, MERGE_ITEM_US = 0.03f;
+    constexpr float SMALL_US = 7.0f, SMALL_CODES_US = 1.5f, PREPARE_US = 4.0f;
+    FlashPlan f{};
+    f.cus = cu_count();
+    f.plain = plain_workspace_bytes(pos, tokens, kv_heads);
+    if (tokens == 0 || kv_heads == 0) return f;
     const uint32_t ntiles = (tokens + TQ - 1) / TQ;
     const uint32_t longest = tile_blocks(pos, tokens, ntiles - 1), shortest = tile_blocks(pos, tokens, 0);
-    const float per_us = CHIP_BLOCKS_PER_US * float(cus);
+    const float per_us = CHIP_BLOCKS_PER_US * float(f.cus);
     // n items in order of length, from `high` down to `low` blocks, handed out one by one
     auto rounds_us = [&](uint32_t n, float high, float low, float ends_us) {
         float us = 0.0f, at = 0.0f;
         for (uint32_t left = n; left > 0;) {
-            const uint32_t now = left < cus ? left : cus;
+            const uint32_t now = left < f.cus ? left : f.cus;
             const float mid = high - (high - low) * (at + 0.5f * float(now)) / float(n);  // mean length of the round's items
             const float alone = mid * BLOCK_US, shared = mid * float(now) / per_us;
             us += (alone > shared ? alone : shared) + ends_us;
@@ -798,18 +1122,29 @@ uint32_t choose_part_blocks(uint32_t pos, uint32_t tokens, uint32_t kv_heads, ui
         const float one = high * BLOCK_US + ends_us;
         return us > one ? us : one;
     };
-    float best = 0.95f * rounds_us(ntiles * kv_heads, float(longest), float(shortest), TILE_US);
-    uint32_t part_blocks = 0;
+    const float unsplit = rounds_us(ntiles * kv_heads, float(longest), float(shortest), TILE_US);
+    float best = 0.95f * unsplit;
     for (uint32_t parts = 2; parts <= 32; parts++) {
         const uint32_t pb = ((longest + parts - 1) / parts + 1) / 2 * 2;  // (a step of the kernel is two blocks)
         if (pb < 4 || pb >= longest) continue;
         const uint32_t items = prefill_items(pos, tokens, pb) * kv_heads;
         const float mid = 0.5f * float(longest + shortest) * float(ntiles * kv_heads) / float(items);
         const float us = rounds_us(items, mid, mid, PART_US) + MERGE_US + MERGE_ITEM_US * float(items);
-        if (us < best) best = us, part_blocks = pb;
+        if (us < best) best = us, f.part_blocks = pb;
     }
-    return part_blocks;
+    if (f.part_blocks) {
+        f.nparts = parts_of(pos, tokens, f.part_blocks);
+        f.parts = parts_bytes(tokens, kv_heads, f.nparts);
+    } else {
+        best = unsplit;
+    }
+    const uint32_t groups = (tokens + 3) / 4 * kv_heads;
+    f.small = rounds_us(groups, float(longest), float(shortest), SMALL_US + (bits == 16 ? 0.0f : SMALL_CODES_US)) < best + PREPARE_US;
+    return f;
 }
+
+size_t workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) { return flash_plan(pos, tokens, kv_heads, 16).bytes(); }
+
 // The checks both prefill paths share.
 int check_prefill(int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
                   const uint16_t *kz, const uint16_t *vs, const uint16_t *vz, const float *q_and_gate, const float *out,
@@ -884,26 +1219,19 @@ uint32_t launch_prepare(hipStream_t stream, int bits, const void *kdata, const v
     return nblocks;
 }
 
-// What a chunk needs of a workspace, and how its keys are split.
-struct FlashPlan {
-    uint32_t cus, part_blocks, nparts;
-    size_t plain, parts;  // bytes: the images and the tile count; the parts behind them
-    size_t bytes() const { return plain + parts; }
-};
-FlashPlan flash_plan(const saetta_flash_params &p) {
-    FlashPlan f{};
-    f.cus = cu_count();
-    f.plain = plain_workspace_bytes(p.pos, p.tokens, p.kv_heads);
-    if (p.tokens && p.kv_heads) f.part_blocks = choose_part_blocks(p.pos, p.tokens, p.kv_heads, f.cus);
-    if (f.part_blocks) {
-        f.nparts = parts_of(p.pos, p.tokens, f.part_blocks);
-        f.parts = parts_bytes(p.tokens, p.kv_heads, f.nparts);
+int launch_small(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
+                 const uint16_t *kz, const uint16_t *vs, const uint16_t *vz, const float *q_and_gate, float *out,
+                 const saetta_flash_params &p, const char *what) {
+    SmallArgs a{q, static_cast<const unsigned char *>(kdata), static_cast<const unsigned char *>(vdata), ks, kz, vs, vz, q_and_gate, out, p.heads, p.kv_heads, p.pos, p.tokens, p.scale};
+    const dim3 grid((p.tokens + 3) / 4, p.kv_heads);
+    if (bits == 8) {
+        launch(prefill_small_kernel<8>, grid, SMALL_THREADS, SmallLds<8>::BYTES, stream, a);
+    } else if (bits == 4) {
+        launch(prefill_small_kernel<4>, grid, SMALL_THREADS, SmallLds<4>::BYTES, stream, a);
+    } else {
+        launch(prefill_small_kernel<16>, grid, SMALL_THREADS, SmallLds<16>::BYTES, stream, a);
     }
-    return f;
-}
-
-size_t workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) {
-    return flash_plan(saetta_flash_params{0, kv_heads, pos, tokens, 0.0f}).bytes();
+    return launch_status(what);
 }
 
 // The launches of a chunk in a workspace of at least plan.plain bytes, plan.bytes() with `split`.
@@ -938,7 +1266,13 @@ int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kda
     if (int rc = check_prefill(bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, what)) return rc;
     if (int rc = ensure_device()) return rc;
     if (p.tokens == 0) return SAETTA_OK;
-    const FlashPlan plan = flash_plan(p);
+    const FlashPlan plan = flash_plan(p.pos, p.tokens, p.kv_heads, bits);
+    if (plan.small) {
+        // (a workspace that is given has to do, whatever the chunk: which launches serve it is no caller's business)
+        SAETTA_REQUIRE(!workspace || workspace_size >= plan.plain, SAETTA_E_SCRATCH, "%s: workspace of %zu bytes, %zu needed", what,
+                       workspace_size, plan.plain);
+        return launch_small(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, what);
+    }
     size_t need = plan.bytes();
     if (workspace && workspace_size < need) need = plan.plain;  // (room for the images only: the keys are not split)
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
@@ -1308,7 +1642,11 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
     if (int rc = acquire_workspace(stream, workspace, workspace_size, need, owned_lock, what, "saetta_attn_gemm_workspace_bytes")) return rc;
     // All of the call: the flash kernel's result is the same and it is there in 0.5 to 0.6 of the time (see above).
-    if (stages == 0) return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, true, flash_plan(p), what);
+    if (stages == 0) {
+        const FlashPlan plan = flash_plan(p.pos, p.tokens, p.kv_heads, bits);
+        if (plan.small) return launch_small(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, what);
+        return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, true, plan, what);
+    }
     const uint32_t nblocks = launch_prepare(stream, bits, kdata, vdata, ks, kz, vs, vz, workspace, p.kv_heads, rows);
 
     const size_t groups = gemm_row_groups(slice) * p.kv_heads;
@@ -1354,6 +1692,9 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
 int setup_prefill() {
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_prefill_kernel<false>))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(prefill_merge_kernel))) return rc;
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<16>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<16>::BYTES))) return rc;
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<8>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<8>::BYTES))) return rc;
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<4>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<4>::BYTES))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_scores_kernel))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_pv_kernel))) return rc;
     if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_prefill_kernel<true>),

@@ -64,12 +64,12 @@ def _stream(stream=None):
         return stream
     if stream is None:
         # the handle of torch's current stream, without the Stream object of torch.cuda.current_stream()
-        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
     return ctypes.c_void_p(stream.cuda_stream)
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()  # (an int: the binding's argument types make the pointer of it)
 
 
 def device_status(clear=False):
@@ -79,7 +79,7 @@ def device_status(clear=False):
 
 
 def _need(t, dtype, what):
-    if not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == dtype and t.is_contiguous()):
+    if not (isinstance(t, torch.Tensor) and t.dtype is dtype and t.is_cuda and t.is_contiguous()):
         raise TypeError(f"{what}: expected a contiguous {dtype} tensor on the GPU")
     return t
 
@@ -358,7 +358,9 @@ def to_half(x, out, stream=None):
     """to_half (kernels/prefill.metal:1428-1432)."""
     _need(x, torch.float32, "to_half x")
     _need(out, torch.float16, "to_half out")
-    ffi.check(ffi.lib().saetta_to_half(_stream(stream), _ptr(x), _ptr(out), x.numel()), "to_half")
+    rc = ffi.lib().saetta_to_half(_stream(stream), x.data_ptr(), out.data_ptr(), x.numel())
+    if rc:
+        ffi.check(rc, "to_half")
 
 
 def _check_shape(heads, kv_heads, head_dim, what):
@@ -766,14 +768,12 @@ def _workspace_or_own(t, p, like, stream):
     return t
 
 
-class FlashParams:
-    """src/attention_prefill.rs:4-14."""
-
-    def __init__(self, heads, kv_heads, pos, tokens, scale):
-        self.heads, self.kv_heads, self.pos, self.tokens, self.scale = heads, kv_heads, pos, tokens, scale
+class FlashParams(ffi.FlashParamsC):
+    """src/attention_prefill.rs:4-14 (heads, kv_heads, pos, tokens, scale): the ABI's own block, so that a call
+    has nothing to convert."""
 
     def c(self):
-        return ffi.FlashParamsC(self.heads, self.kv_heads, self.pos, self.tokens, self.scale)
+        return self
 
 
 class attention_prefill:
@@ -800,10 +800,11 @@ class attention_prefill:
             raise ValueError(f"{kernel} needs 8 q heads per kv head")
         _need(q, torch.float16, "q"), _need(keys, torch.float16, "keys"), _need(values, torch.float16, "values")
         _need(q_and_gate, torch.float32, "q_and_gate"), _need(out, torch.float32, "out")
-        workspace = _workspace_or_own(workspace, p, q, stream)
-        ffi.check(ffi.lib().saetta_attn_prefill(_stream(stream), _ptr(q), _ptr(keys), _ptr(values),
-                                                _ptr(q_and_gate), _ptr(out), p.c(), *_workspace(workspace)),
-                  "attn_prefill")
+        workspace = _need(_workspace_or_own(workspace, p, q, stream), torch.uint8, "workspace")
+        rc = ffi.lib().saetta_attn_prefill(_stream(stream), q.data_ptr(), keys.data_ptr(), values.data_ptr(), q_and_gate.data_ptr(),
+                                           out.data_ptr(), p, workspace.data_ptr(), workspace.numel())
+        if rc:
+            ffi.check(rc, "attn_prefill")
 
     @staticmethod
     def encode_rows2(q, keys, values, q_and_gate, out, p, stream=None, workspace=None):
@@ -871,10 +872,11 @@ class attention_prefill:
         if p.heads != p.kv_heads * 8:
             raise ValueError("prefill attention needs 8 q heads per kv head")
         _need(q, torch.float16, "q"), _need(q_and_gate, torch.float32, "q_and_gate"), _need(out, torch.float32, "out")
-        workspace = _workspace_or_own(workspace, p, q, stream)
-        ffi.check(ffi.lib().saetta_attn_prefill_quant(_stream(stream), keys.bits.value, _ptr(q), keys.c(), values.c(),
-                                                      _ptr(q_and_gate), _ptr(out), p.c(), *_workspace(workspace)),
-                  "attn_prefill_quant")
+        workspace = _need(_workspace_or_own(workspace, p, q, stream), torch.uint8, "workspace")
+        rc = ffi.lib().saetta_attn_prefill_quant(_stream(stream), keys.bits.value, q.data_ptr(), keys.c(), values.c(),
+                                                 q_and_gate.data_ptr(), out.data_ptr(), p, workspace.data_ptr(), workspace.numel())
+        if rc:
+            ffi.check(rc, "attn_prefill_quant")
 
 
 class attention_gemm:

@@ -266,3 +266,22 @@ def test_keys_in_parts(kind, pos, tokens):
         assert np.isfinite(got).all()
         assert oracle.rel_rms(got, want) < REL_RMS
         assert np.abs(got - want).max() < MAX_ABS
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("pos,tokens", [(0, 4), (31, 1), (32, 2), (125, 3), (126, 5), (253, 3), (254, 5), (300, 17), (500, 30)])
+def test_short_chunks_over_short_contexts(kind, pos, tokens):
+    # A workgroup per 4 tokens, its 8 waves on alternate blocks of 32 keys: one block, two, four and five (the waves'
+    # parts are joined in one pass or two), eight and nine (a wave with two blocks), 17; ragged last tokens.
+    rng = np.random.default_rng(1000 * pos + tokens)
+    n = pos + tokens
+    k = rng.standard_normal((n, VALUES)).astype(np.float32)
+    v = rng.standard_normal((n, VALUES)).astype(np.float32)
+    q16 = rng.standard_normal((tokens, H, D)).astype(np.float16)
+    qg = rng.standard_normal((tokens, H, 2 * D)).astype(np.float32)
+    kc, vc, kf, vf = make_cache(kind, k, v, n + 7, chunk_from=pos)
+    got = run(kind, q16, kc, vc, qg, pos, tokens)
+    want = oracle.prefill(q16.astype(np.float32), kf, vf, pos, tokens, q_and_gate=qg, threads=8)
+    assert np.isfinite(got).all()
+    assert oracle.rel_rms(got, want) < REL_RMS
+    assert np.abs(got - want).max() < MAX_ABS
