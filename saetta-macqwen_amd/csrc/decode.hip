@@ -303,7 +303,8 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a) {
     const uint32_t kvh = a.kv_heads;
     const uint32_t real_rows = a.rows * 8;  // (row, head) pairs of this kv head
 
-    // ---- query values: requested first, so that nothing they wait for is behind the cache ----
+    // ---- query values: requested first, so that nothing they wait for is behind the cache (loads return in order: with
+    // two and four tiles, asked for when they are used, they came behind the whole first iteration, 1.5 to 2.4 us) ----
     // Item (tile t, k-step, lane l) is the 8 values that lane l feeds to the MFMA k-step;
     // operand row `on` of tile t: PACKED -> head on & 7, part on >> 3; else (row, head)
     // pair 16t + on, both parts.
@@ -324,11 +325,9 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a) {
             for (int e = 0; e < 8; e++) v[e] = 0.0f;
         }
     };
-    float q_early[TILES == 1 ? 2 : 1][8];
-    if constexpr (TILES == 1) {
-        load_q_item(tid, q_early[0]);
-        load_q_item(tid + THREADS, q_early[1]);
-    }
+    float q_early[TILES * 2][8];
+#pragma unroll
+    for (int k = 0; k < TILES * 2; k++) load_q_item(tid + k * THREADS, q_early[k]);
 
     // ---- the context and this workgroup's share of it -----------------------------
     const uint32_t position = a.tp->position;
@@ -425,13 +424,7 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a) {
             const int item = tid + k * THREADS;
             const int t = item / 512, step = (item / 64) & 7, l = item & 63;
             const int on = l & 15;
-            float v[8];
-            if constexpr (TILES == 1) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = q_early[k][e];
-            } else {
-                load_q_item(item, v);
-            }
+            const float (&v)[8] = q_early[k];
             half8 hi, lo;
             float sum_hi = 0.0f, sum_lo = 0.0f;
 #pragma unroll
@@ -787,14 +780,18 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a) {
             const float zb = QUANT ? zsum_lds[wave * Sh::S_ROWS + pair] * (1.0f / P_UP) : 0.0f;
             const size_t slot = (size_t(vrow) * a.nsplits + split) * a.heads + kv * 8 + head;
             float *dst = a.part_o + slot * DIM + 64 * wave;
+            // (Five to eight rows past the caches: up to 17 MB that the L2s would hold dirty until the kernel's end, 27.0 against
+            // 27.7 us a layer for 8 rows at 7000 tokens.  Fewer rows are read back sooner than they are written out: plain.)
+            auto put = [&](float *to, auto value) {
+                if constexpr (TILES == 4) __builtin_nontemporal_store(value, reinterpret_cast<decltype(value) *>(to));
+                else *reinterpret_cast<decltype(value) *>(to) = value;
+            };
             if constexpr (BITS == 16) {
                 // tile e: dims 32*(e/2) + 2n + e%2
-                *reinterpret_cast<float2 *>(dst + 2 * n) = make_float2(o[0][i] * unscale, o[1][i] * unscale);
-                *reinterpret_cast<float2 *>(dst + 32 + 2 * n) = make_float2(o[2][i] * unscale, o[3][i] * unscale);
+                put(dst + 2 * n, floatx2{o[0][i] * unscale, o[1][i] * unscale});
+                put(dst + 32 + 2 * n, floatx2{o[2][i] * unscale, o[3][i] * unscale});
             } else {
-                *reinterpret_cast<float4 *>(dst + 4 * n) =
-                    make_float4(o[0][i] * unscale + zb, o[1][i] * unscale + zb, o[2][i] * unscale + zb,
-                                o[3][i] * unscale + zb);
+                put(dst + 4 * n, floatx4{o[0][i] * unscale + zb, o[1][i] * unscale + zb, o[2][i] * unscale + zb, o[3][i] * unscale + zb});
             }
         }
     }
@@ -2456,7 +2453,12 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
     // splits of this wave: per_wave (a multiple of 16) from per_wave * wave on; of this lane: slot + 16 i
     const uint32_t per_wave = (a.nsplits + 63) / 64 * 16;
     constexpr int PER_LANE = MAX_SPLITS / 64;
-    // Slots past the splits at work hold old values: they are dropped by select, never multiplied.
+    const uint32_t max_len = min(a.decode_len ? a.tp->kv_len : a.tp->position + a.rows, a.capacity);
+    const uint32_t nblocks = (max_len + BLOCK - 1) / BLOCK;
+    const uint32_t parts = min(a.nsplits, nblocks);
+    // Slots past the splits at work hold old values: they are dropped by select, never multiplied.  (One and two rows read
+    // them all the same: waiting for the length first costs more than up to 2 MB of old partials a row.)
+    const uint32_t limit = a.rows > 2 ? parts : a.nsplits;
     floatx2 mlv[PER_LANE];
     floatx4 pv[PER_LANE];
 #pragma unroll
@@ -2464,16 +2466,13 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
         const uint32_t c = per_wave * wave + slot + 16 * i;
         mlv[i] = floatx2{NO_SCORE, 0.0f};
         pv[i] = floatx4{0, 0, 0, 0};
-        if (16 * uint32_t(i) < per_wave && c < a.nsplits) {
+        if (16 * uint32_t(i) < per_wave && c < limit) {
             mlv[i] = *reinterpret_cast<const floatx2 *>(ml + 2 * (size_t(c) * a.heads + h));
             pv[i] = *reinterpret_cast<const floatx4 *>(po + (size_t(c) * a.heads + h) * DIM + REDUCE_DIMS * slice + 4 * quad);
         }
     }
     const size_t qh = size_t(row) * a.heads + h;
     const float g = tid < REDUCE_DIMS ? a.q_and_gate[qh * 2 * DIM + DIM + REDUCE_DIMS * slice + tid] : 0.0f;
-    const uint32_t max_len = min(a.decode_len ? a.tp->kv_len : a.tp->position + a.rows, a.capacity);
-    const uint32_t nblocks = (max_len + BLOCK - 1) / BLOCK;
-    const uint32_t parts = min(a.nsplits, nblocks);
     float m[PER_LANE], mx = NO_SCORE;
 #pragma unroll
     for (int i = 0; i < PER_LANE; i++) {
