@@ -60,13 +60,18 @@ struct LaunchRecord {
     dim3 grid, block;
     uint32_t lds;
     uint32_t first_arg, args;  // of LaunchList::offsets
+    // What a launch is, for a call that may take launches recorded before it into one of its own.
+    uint32_t kind = 0, bits = 0, rows = 0;
 };
+enum : uint32_t { LAUNCH_PREP = 1, LAUNCH_PARTIAL = 2 };
 // Launches in order; the arguments lie in `bytes`, each at its offset, 16-byte aligned.
 struct LaunchList {
     std::vector<LaunchRecord> launches;
     std::vector<uint32_t> offsets;
     std::vector<unsigned char> bytes;
     int device = 0;
+    template <class T>
+    const T &arg(const LaunchRecord &r, uint32_t i) const { return *reinterpret_cast<const T *>(bytes.data() + offsets[r.first_arg + i]); }
 };
 // The list this thread records into, or nullptr: launches are made.
 LaunchList *&recording();
@@ -91,6 +96,11 @@ void launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t
         return;
     }
     kernel<<<grid, block, lds, stream>>>(std::forward<A>(args)...);
+}
+
+// Says what the launch just recorded is.
+inline void tag_launch(uint32_t kind, uint32_t bits, uint32_t rows) {
+    if (LaunchList *list = recording()) list->launches.back().kind = kind, list->launches.back().bits = bits, list->launches.back().rows = rows;
 }
 
 inline bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }

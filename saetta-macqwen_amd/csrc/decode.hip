@@ -57,7 +57,9 @@
 // Which one runs is decided in run_attention from the launch arguments alone, so that the partial
 // and the reduce stage of a step agree on the number of splits.
 #include "common.hpp"
+#include "kv_quant_device.hpp"
 #include "lanes.hpp"
+#include "prep_device.hpp"
 
 namespace saetta {
 namespace {
@@ -115,6 +117,12 @@ struct PartialArgs {
     const saetta_token_params *tp;
     uint32_t decode_len;  // 1: every row sees min(kv_len, capacity); 0: row r sees position + r + 1
     uint32_t *status;     // the device's sticky status word (pinned host memory)
+};
+// The same with the step before the scores taken in.
+struct TokenArgs {
+    PartialArgs a;        // nsplits: the context's workgroups and one
+    PrepArgs prep;
+    uint32_t new_heads;   // q heads of a row that a workgroup of the new rows takes (register kernels)
 };
 
 __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
@@ -248,6 +256,179 @@ __device__ __forceinline__ float half_bits_to_float(uint32_t bits16) {
     return (float)__builtin_bit_cast(_Float16, uint16_t(bits16));
 }
 
+// ---- the step before the scores, taken in -------------------------------------------------------
+//
+// A token step of a plan records attention_prep_store, the partial and the reduce stage of a layer one after the other.
+// The first is a launch of 2.7 us (20 workgroups and row; 1.6 us is what any launch costs in a graph) for 20 KB of work, so
+// where the three stand next to each other on the same buffers (run_attention looks while they are recorded) the partial
+// stage does it:
+//  * every workgroup of the context norms and rotates the query rows it needs itself, under the first loads of the cache;
+//    its context are the tokens BEFORE the new ones;
+//  * workgroups of their own (behind the context's) make the new keys and values, store them and the query rows, and
+//    write the new tokens' own partial result (the last split), from the values just as the cache holds them, so nobody
+//    in the launch reads what another workgroup of it writes.
+// The keys', values' and codes' bits are those of attention_prep_store_kernel (the same operations in the same order).
+// A workgroup of the new rows takes some rows and some heads of them, and makes the keys and values of all rows up to
+// those for itself.  The loader kernels have 12 waves: one workgroup does it all.  The register kernels have 4, so that a
+// row's heads are dealt out two to a workgroup where CUs are free, and a row has one workgroup where the context would
+// fill them all.  The total stays at one workgroup per CU: where it was 128 per kv head the context gives some up.
+// Measured per layer, ten layers in a graph, against the store as a launch of its own: one row 9.9 against 11.9 us (codes,
+// 300 tokens of 8192), 12.6 against 15.2 (f16, 7000 of 8192), 16.6 against 18.1 (8-bit, 32768), 33 against 35 (4-bit,
+// 150000); two rows 11.7 against 13.7 (f16, 3000), 18 against 20.4 (8-bit, 32768); three 24.1 against 26; four 15.8
+// against 17.2 (8-bit, 3000), 36.2 against 37.7 (60000).
+
+// The other half wavefront's value.
+__device__ __forceinline__ float half_swap(float x, bool lower) {
+    uint32_t u = __builtin_bit_cast(uint32_t, x), v = u;
+    swap_rows32(u, v);  // u = (lower, lower), v = (upper, upper)
+    return __builtin_bit_cast(float, lower ? v : u);
+}
+
+constexpr int NEW_ROWS = 4;  // rows of a token step that takes the store in, at most
+// Tokens of the context before the new ones; new tokens that row `row` sees.
+__device__ __forceinline__ uint32_t tokens_before(const PartialArgs &a, uint32_t position, uint32_t kv_len) {
+    return min(a.decode_len ? min(position, kv_len) : position, a.capacity);
+}
+__device__ __forceinline__ uint32_t tokens_new(const PartialArgs &a, uint32_t position, uint32_t kv_len, uint32_t row) {
+    const uint32_t seen = min(a.decode_len ? min(kv_len, position + 1) : position + row + 1, a.capacity);
+    return seen > position ? seen - position : 0;
+}
+
+__device__ __forceinline__ void wave_sync() {  // LDS written by lanes of the wave and read by others: its accesses run in order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// A workgroup of the new rows: q heads head0 .. head0 + heads - 1 of rows row0 .. row0 + nrows - 1 (of up to R).  A wave takes whole
+// heads: lane l holds dims l, 64 + l, 128 + l, 192 + l.
+template <int BITS, int R>
+__device__ __forceinline__ void new_rows(const PartialArgs &a, const PrepArgs &p, unsigned char *lds, uint32_t waves, uint32_t row0, uint32_t nrows,
+                                         uint32_t head0, uint32_t heads) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63, kv = blockIdx.y, kvh = a.kv_heads, rows = row0 + nrows;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float2 *rope = reinterpret_cast<float2 *>(lds);                                          // [row][32] sine, cosine
+    float *keys = reinterpret_cast<float *>(lds + R * 32 * 8), *values = keys + rows * DIM;  // [row][256]: as the cache gives them
+    float *queries = values + rows * DIM;                                                    // [row][head][256]
+    const uint32_t position = a.tp->position, kv_len = a.tp->kv_len;
+    // items: the rows' keys, their values, then the q heads
+    const uint32_t items = 2 * rows + nrows * heads;
+    float next[4];
+    auto request = [&](uint32_t item) {
+        item = item < items ? item : items - 1;
+        const uint32_t q = item - 2 * rows;
+        const float *src = item < rows       ? p.k + (size_t(item) * kvh + kv) * DIM
+                           : item < 2 * rows ? p.v + (size_t(item - rows) * kvh + kv) * DIM
+                                             : p.q_and_gate + (size_t(row0 + q / heads) * a.heads + kv * 8 + head0 + q % heads) * 2 * DIM;
+#pragma unroll
+        for (int i = 0; i < 4; i++) next[i] = src[64 * i + lane];
+    };
+    request(wave);
+    float qn[4], kn[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) qn[i] = p.q_norm[64 * i + lane], kn[i] = p.k_norm[64 * i + lane];
+    if (tid < 32 * rows) {
+        float s, c;
+        rope_angle(position + (tid >> 5), tid & 31, 32, p.p.log2_theta, s, c);
+        rope[tid] = float2{s, c};
+    }
+    __syncthreads();
+    for (uint32_t item = wave; item < items; item += waves) {
+        const bool is_q = item >= 2 * rows, is_k = item < rows;
+        const uint32_t q = item - 2 * rows, row = is_q ? row0 + q / heads : is_k ? item : item - rows;
+        float x[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = next[i];
+        if (item + waves < items) request(item + waves);
+        if (is_q || is_k) {
+            float sq[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) sq[i] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, square_sum(x[i]))));
+            const float scale = norm_scale((sq[0] + sq[1]) + (sq[2] + sq[3]), p.p.eps);
+#pragma unroll
+            for (int i = 0; i < 4; i++) x[i] = __fmul_rn(x[i], __fmul_rn(scale, is_q ? qn[i] : kn[i]));
+            const float2 sc = rope[row * 32 + (lane & 31)];
+            const float other = half_swap(x[0], lane < 32);
+            x[0] = lane < 32 ? rope_first(x[0], other, sc.x, sc.y) : rope_second(other, x[0], sc.x, sc.y);
+        }
+        if (is_q) {
+            float *dst = p.q_out + (size_t(row) * a.heads + kv * 8 + head0 + q % heads) * DIM, *keep = queries + q * DIM;
+#pragma unroll
+            for (int i = 0; i < 4; i++) dst[64 * i + lane] = x[i], keep[64 * i + lane] = x[i];
+            continue;
+        }
+        const bool mine = row >= row0 && head0 == 0;  // of the workgroups that make it, the one that stores it
+        if (is_k && mine && p.k_back) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) p.k_back[(size_t(row) * kvh + kv) * DIM + 64 * i + lane] = x[i];
+        }
+        const size_t slot = size_t(position + row) * kvh + kv;  // (head row of the cache)
+        const bool stored = mine && position + row < a.capacity;
+        float *keep = (is_k ? keys : values) + row * DIM;
+        if constexpr (BITS == 16) {
+            uint16_t *dst = (is_k ? p.keys_half : p.values_half) + slot * DIM;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const __half h = __float2half_rn(x[i]);
+                if (stored) dst[64 * i + lane] = __half_as_ushort(h);
+                keep[64 * i + lane] = __half2float(h);
+            }
+        } else {
+            // the quantizer wants 32 / BITS neighbouring values per lane: through LDS, where the cache's values then go
+            constexpr uint32_t VPL = 32 / BITS, LANES = SAETTA_QUANT_GROUP / VPL;
+#pragma unroll
+            for (int i = 0; i < 4; i++) keep[64 * i + lane] = x[i];
+            wave_sync();
+            if (lane < DIM / VPL) {
+                float v[VPL];
+#pragma unroll
+                for (uint32_t e = 0; e < VPL; e++) v[e] = keep[lane * VPL + e];
+                __half s, z;
+                const uint32_t word = quantize_lane<BITS>(v, s, z);
+                if (stored) {
+                    const saetta_quant_rows c = is_k ? p.kq : p.vq;
+                    c.data[slot * (DIM / VPL) + lane] = word;
+                    if (lane % LANES == 0) c.scales[slot * 4 + lane / LANES] = __half_as_ushort(s), c.biases[slot * 4 + lane / LANES] = __half_as_ushort(z);
+                }
+                const float sf = __half2float(s), zf = __half2float(z);
+#pragma unroll
+                for (uint32_t e = 0; e < VPL; e++) keep[lane * VPL + e] = fmaf(sf, float((word >> (e * BITS)) & ((1u << BITS) - 1)), zf);
+            }
+        }
+    }
+    __syncthreads();
+    // the new tokens' partial result of every (row, head): scores in units of log2(e), as the other splits'
+    for (uint32_t pair = wave; pair < nrows * heads; pair += waves) {
+        const uint32_t row = row0 + pair / heads, seen = tokens_new(a, position, kv_len, row);
+        float q[4], score[R], m = NO_SCORE, l = 0.0f, o[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; i++) q[i] = queries[pair * DIM + 64 * i + lane] * (a.scale * 1.4426950408889634f);
+#pragma unroll
+        for (uint32_t t = 0; t < uint32_t(R); t++) {
+            score[t] = NO_SCORE;
+            if (t < seen) {
+                float dot = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 4; i++) dot += q[i] * keys[t * DIM + 64 * i + lane];
+                score[t] = group_reduce<64>(dot, SumOp());
+                m = fmaxf(m, score[t]);
+            }
+        }
+#pragma unroll
+        for (uint32_t t = 0; t < uint32_t(R); t++) {
+            if (t < seen) {
+                const float prob = __builtin_amdgcn_exp2f(score[t] - m);
+                l += prob;
+#pragma unroll
+                for (int i = 0; i < 4; i++) o[i] += prob * values[t * DIM + 64 * i + lane];
+            }
+        }
+        const size_t slot = (size_t(row) * a.nsplits + (a.nsplits - 1)) * a.heads + kv * 8 + head0 + pair % heads;
+#pragma unroll
+        for (int i = 0; i < 4; i++) a.part_o[slot * DIM + 64 * i + lane] = o[i];
+        if (lane == 0) *reinterpret_cast<floatx2 *>(a.part_ml + 2 * slot) = floatx2{m, l};
+    }
+}
+
 // TILES: 16-row tiles of query rows (rows * 8 heads, rounded up).  PACKED: one
 // verify row; its 8 heads' hi parts are operand rows 0-7 and lo parts rows 8-15
 // of a single tile.  Otherwise hi and lo are two MFMAs into one accumulator.
@@ -276,10 +457,13 @@ struct Shape {
     static constexpr int QZ_OFF = ALPHA_OFF + S_ROWS * 4;                   // [tile][hi, lo][lane] half8
     static constexpr int ZSUM_OFF = QZ_OFF + TILES * 2 * 64 * 16;           // [wave][S_ROWS] f32
     static constexpr int LDS_BYTES = ZSUM_OFF + 4 * S_ROWS * 4;
+    // the new rows' workgroup of attention_token_kernel_*: the angles, then keys, values and 8 query rows per row
+    static constexpr int ROWS = PACKED ? 1 : 2 * TILES;
+    static_assert(2 * 1024 + ROWS * 10 * 256 * 4 <= LDS_BYTES, "the new rows' workgroup fits");
 };
 
-template <int BITS, int TILES, bool PACKED, int ITB, bool UNCOND>
-__device__ __forceinline__ void attention_partial_body(const PartialArgs &a) {
+template <int BITS, int TILES, bool PACKED, int ITB, bool UNCOND, bool PREP = false>
+__device__ __forceinline__ void attention_partial_body(const PartialArgs &a, const PrepArgs *prep = nullptr, uint32_t new_heads = 8) {
     using Sh = Shape<BITS, TILES, PACKED, ITB>;
     constexpr int IT_BLOCKS = ITB, IT_TOKENS = Sh::IT_TOKENS, SC_STRIDE = Sh::SC_STRIDE;
     constexpr int KROUNDS = ITB / 4, KSTEPS = ITB / 2;
@@ -302,6 +486,14 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a) {
     const uint32_t split = blockIdx.x, kv = blockIdx.y;
     const uint32_t kvh = a.kv_heads;
     const uint32_t real_rows = a.rows * 8;  // (row, head) pairs of this kv head
+    const uint32_t context_splits = PREP ? a.nsplits - 1 : a.nsplits;
+    if constexpr (PREP) {
+        if (split >= context_splits) {
+            const uint32_t per_row = SAETTA_GQA_GROUP / new_heads, at = split - context_splits;
+            new_rows<BITS, PACKED ? 1 : TILES == 1 ? 2 : NEW_ROWS>(a, *prep, lds_raw, THREADS / 64, at / per_row, 1, at % per_row * new_heads, new_heads);
+            return;
+        }
+    }
 
     // ---- query values: requested first, so that nothing they wait for is behind the cache (loads return in order: with
     // two and four tiles, asked for when they are used, they came behind the whole first iteration, 1.5 to 2.4 us) ----
@@ -315,7 +507,8 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a) {
         const int pair = PACKED ? (on & 7) : 16 * t + on;
         if (PACKED || pair < int(real_rows)) {  // (a single row always has its 8 heads)
             const int row = pair >> 3, head = pair & 7;
-            const float *src = a.q + (size_t(row) * a.heads + kv * 8 + head) * DIM + 64 * g + 16 * oj + 8 * ab;
+            const size_t of_head = size_t(row) * a.heads + kv * 8 + head;
+            const float *src = (PREP ? prep->q_and_gate + of_head * 2 * DIM : a.q + of_head * DIM) + 64 * g + 16 * oj + 8 * ab;
             const float4 f0 = *reinterpret_cast<const float4 *>(src);
             const float4 f1 = *reinterpret_cast<const float4 *>(src + 4);
             v[0] = f0.x, v[1] = f0.y, v[2] = f0.z, v[3] = f0.w;
@@ -328,22 +521,32 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a) {
     float q_early[TILES * 2][8];
 #pragma unroll
     for (int k = 0; k < TILES * 2; k++) load_q_item(tid + k * THREADS, q_early[k]);
+    float norm_w[PREP ? 2 : 1][8];  // the norm's weights of the thread's dims (k-steps wave and wave + 4)
+    if constexpr (PREP) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const float4 *src = reinterpret_cast<const float4 *>(prep->q_norm + 64 * ((wave + 4 * k) >> 1) + 16 * j + 8 * (wave & 1));
+            const float4 f0 = src[0], f1 = src[1];
+            norm_w[k][0] = f0.x, norm_w[k][1] = f0.y, norm_w[k][2] = f0.z, norm_w[k][3] = f0.w;
+            norm_w[k][4] = f1.x, norm_w[k][5] = f1.y, norm_w[k][6] = f1.z, norm_w[k][7] = f1.w;
+        }
+    }
 
     // ---- the context and this workgroup's share of it -----------------------------
     const uint32_t position = a.tp->position;
     const uint32_t kv_len = a.tp->kv_len;
-    // Tokens the last row sees; the longest context of the launch.
-    const uint32_t max_len = min(a.decode_len ? kv_len : position + a.rows, a.capacity);
+    // Tokens the last row sees; the longest context of the launch.  (PREP: the tokens before the new ones.)
+    const uint32_t max_len = PREP ? tokens_before(a, position, kv_len) : min(a.decode_len ? kv_len : position + a.rows, a.capacity);
     const uint32_t nblocks = (max_len + BLOCK - 1) / BLOCK;
     uint32_t blk_begin, blk_end;
-    if (nblocks <= a.nsplits) {
+    if (nblocks <= context_splits) {
         blk_begin = split;
         blk_end = split + 1;
         if (split >= nblocks) return;
     } else {
         // (split + 1) * nblocks < 2^32: at most 256 splits and 2^27 blocks (32-bit cache offsets)
-        blk_begin = split * nblocks / a.nsplits;
-        blk_end = (split + 1) * nblocks / a.nsplits;
+        blk_begin = split * nblocks / context_splits;
+        blk_end = (split + 1) * nblocks / context_splits;
     }
     const uint32_t range = blk_end - blk_begin;
     const uint32_t n_it = (range + IT_BLOCKS - 1) / IT_BLOCKS;
@@ -417,6 +620,48 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a) {
 
     // ---- prologue: query rows to f16 hi/lo operands in LDS ------------------------
     // (while the first iteration's keys are in flight; the values are requested after it)
+    if constexpr (PREP) {
+        // the norm (each wave has two of the eight k-steps of a row's dims) and the rotation (dims 0-63: k-steps 0 and 1, the
+        // waves 0 and 1; a pair's values are half a wavefront apart), where the scores will be
+        float *squares = s_lds;                                       // [tile][wave][column]
+        float2 *rope = reinterpret_cast<float2 *>(s_lds + 4 * 4 * 16);  // [row][32]
+#pragma unroll
+        for (int t = 0; t < TILES; t++) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int k = 2 * t; k < 2 * t + 2; k++) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) sum += q_early[k][e] * q_early[k][e];
+            }
+            sum = across_rows<16, 64>(sum, SumOp());
+            if (j == 0) squares[(t * 4 + wave) * 16 + n] = sum;
+        }
+        if (tid < int(32 * a.rows)) {
+            float s, c;
+            rope_angle(position + (tid >> 5), tid & 31, 32, prep->p.log2_theta, s, c);
+            rope[tid] = float2{s, c};
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TILES; t++) {
+            const float *sq = squares + t * 64 + n;
+            const float scale = norm_scale((sq[0] + sq[16]) + (sq[32] + sq[48]), prep->p.eps);
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) q_early[2 * t + k][e] *= scale * norm_w[k][e];
+            }
+            if (wave < 2) {
+                const int row = PACKED ? 0 : min(2 * t + (n >> 3), int(a.rows) - 1);
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float2 sc = rope[row * 32 + 16 * (j & 1) + 8 * wave + e];
+                    const float x = q_early[2 * t][e], other = half_swap(x, j < 2);
+                    q_early[2 * t][e] = j < 2 ? rope_first(x, other, sc.x, sc.y) : rope_second(other, x, sc.x, sc.y);
+                }
+            }
+        }
+    }
     {
         const float qmul = a.scale * 1.4426950408889634f * Q_UP;
 #pragma unroll
@@ -478,7 +723,7 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a) {
     {
         const int vrow = PACKED ? 0 : b_row >> 3;
         const bool real = PACKED || b_row < int(real_rows);
-        const uint32_t len = a.decode_len ? kv_len : position + vrow + 1;
+        const uint32_t len = PREP ? max_len : a.decode_len ? kv_len : position + vrow + 1;
         b_len = real ? min(len, a.capacity) : 0;
     }
     float m_run = NO_SCORE, l_part = 0.0f;
@@ -822,6 +1067,16 @@ __global__ __launch_bounds__(THREADS) void attention_partial_kernel_p(PartialArg
     attention_partial_body<BITS, 1, true, ITB_ONE_PER_CU, true>(a);
 }
 
+// The same with the step before the scores taken in.
+template <int BITS, int TILES>
+__global__ __launch_bounds__(THREADS) void attention_token_kernel_n(TokenArgs t) {
+    attention_partial_body<BITS, TILES, false, itb_rows<TILES>(), TILES == 1, true>(t.a, &t.prep, t.new_heads);
+}
+template <int BITS>
+__global__ __launch_bounds__(THREADS) void attention_token_kernel_p(TokenArgs t) {
+    attention_partial_body<BITS, 1, true, ITB_ONE_PER_CU, true, true>(t.a, &t.prep, t.new_heads);
+}
+
 // What a wave of attention_partial_kernel_s does when a bounded wait on an LDS counter has run out (it never
 // should): one lane stores a code in the device's sticky status word, which the host reads at its next call
 // (a plain vector store to pinned host memory), and the workgroup's partials get l = NaN, so that the
@@ -942,11 +1197,15 @@ struct KeysFirst {
     static constexpr int C_SLOT = 12;   // [5]: value loaders whose values of slot s have landed (2 per round)
     static constexpr int C_MERGE = 20;  // [4]: one row: wave 2g + 1 has written its sums for wave 2g | two pairs of rows: blocks
                                         // whose keys the two waves of scores w % 4 have in registers; then [4] as with one row
+    static constexpr int C_NORM = 28;       // the step before the scores: computing waves that have written their sums of squares
+    static constexpr int C_POSITION = 29;   // (not a counter: the first new token's position)
     static constexpr uint32_t SPIN_LIMIT = 1u << 20;
+    static constexpr int THREADS_ = (LOADERS + WAVES) * 64;
+    static_assert(2 * 1024 + M * 10 * DIM * 4 <= LDS_BYTES, "the new rows' workgroup fits");
 };
 
-template <int BITS, int M>
-__global__ __launch_bounds__((KeysFirst<BITS, M>::LOADERS + KeysFirst<BITS, M>::WAVES) * 64) void attention_partial_kernel_s(PartialArgs a) {
+template <int BITS, int M, bool PREP>
+__device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, const PrepArgs *prep) {
     using W = KeysFirst<BITS, M>;
     constexpr int RB = W::RB_, RT = W::SB_TOKENS, RBK = W::ROUND_BLOCKS;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
@@ -958,11 +1217,19 @@ __global__ __launch_bounds__((KeysFirst<BITS, M>::LOADERS + KeysFirst<BITS, M>::
     const int wave = wave_all - W::LOADERS;          // computing waves: 0..7
     uint32_t *sync_lds = reinterpret_cast<uint32_t *>(lds_raw + W::SYNC_OFF);
     const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(lds_raw));
+    const uint32_t context_splits = PREP ? a.nsplits - 1 : a.nsplits;
+    if constexpr (PREP) {
+        if (split == context_splits) {
+            new_rows<BITS, M>(a, *prep, lds_raw, W::LOADERS + W::WAVES, 0, M, 0, SAETTA_GQA_GROUP);
+            return;
+        }
+    }
 
     // ---- query values: requested first (computing waves: thread = (k-step, lane) item of every row) ----
     auto load_query = [&](int r, float (&v)[8]) {
         const int step = wave, g = step >> 1, ab = step & 1;
-        const float *src = a.q + (size_t(r) * a.heads + kv * 8 + (n & 7)) * DIM + 64 * g + 16 * j + 8 * ab;
+        const size_t of_head = size_t(r) * a.heads + kv * 8 + (n & 7);
+        const float *src = (PREP ? prep->q_and_gate + of_head * 2 * DIM : a.q + of_head * DIM) + 64 * g + 16 * j + 8 * ab;
         const float4 f0 = *reinterpret_cast<const float4 *>(src);
         const float4 f1 = *reinterpret_cast<const float4 *>(src + 4);
         v[0] = f0.x, v[1] = f0.y, v[2] = f0.z, v[3] = f0.w, v[4] = f1.x, v[5] = f1.y, v[6] = f1.z, v[7] = f1.w;
@@ -976,6 +1243,14 @@ __global__ __launch_bounds__((KeysFirst<BITS, M>::LOADERS + KeysFirst<BITS, M>::
 #pragma unroll
         for (int p = 0; p < W::PAIRS; p++) load_query(M == 1 ? 0 : min(2 * p + (n >> 3), M - 1), qv[p]);
     }
+    float norm_w[8];
+    if constexpr (PREP) {
+        if (!loader) {
+            const float4 *src = reinterpret_cast<const float4 *>(prep->q_norm + 64 * (wave >> 1) + 16 * j + 8 * (wave & 1));
+            const float4 f0 = src[0], f1 = src[1];
+            norm_w[0] = f0.x, norm_w[1] = f0.y, norm_w[2] = f0.z, norm_w[3] = f0.w, norm_w[4] = f1.x, norm_w[5] = f1.y, norm_w[6] = f1.z, norm_w[7] = f1.w;
+        }
+    }
 
     // ---- the context and this workgroup's share of it -----------------------------
     // One wave of the workgroup reads the token's parameters and hands them on through LDS.  The
@@ -983,33 +1258,39 @@ __global__ __launch_bounds__((KeysFirst<BITS, M>::LOADERS + KeysFirst<BITS, M>::
     // anybody requests anything of the cache.
     // (the context length of a decode step | the position of the first of a verify step's rows: one scalar load)
     static_assert(offsetof(saetta_token_params, position) == 4 && offsetof(saetta_token_params, kv_len) == 8, "dwords 1 and 2");
-    if (threadIdx.x < 32) sync_lds[threadIdx.x] = threadIdx.x == W::C_LENGTH ? reinterpret_cast<const uint32_t *>(a.tp)[a.decode_len ? 2 : 1] : 0u;
+    if constexpr (PREP) {
+        if (threadIdx.x < 32) {
+            const uint32_t position = reinterpret_cast<const volatile uint32_t *>(a.tp)[1], kv_len = reinterpret_cast<const volatile uint32_t *>(a.tp)[2];
+            sync_lds[threadIdx.x] = threadIdx.x == W::C_LENGTH ? tokens_before(a, position, kv_len) : threadIdx.x == W::C_POSITION ? position : 0u;
+        }
+    } else {
+        if (threadIdx.x < 32) sync_lds[threadIdx.x] = threadIdx.x == W::C_LENGTH ? reinterpret_cast<const uint32_t *>(a.tp)[a.decode_len ? 2 : 1] : 0u;
+    }
     __syncthreads();
     const uint32_t tp_first = __builtin_amdgcn_readfirstlane(sync_lds[W::C_LENGTH]);
     // tokens row r sees; the last row's are the launch's
-    auto len_of = [&](int r) -> uint32_t { return min<uint32_t>(a.decode_len ? tp_first : tp_first + uint32_t(r) + 1, a.capacity); };
+    auto len_of = [&](int r) -> uint32_t { return min<uint32_t>(PREP || a.decode_len ? tp_first : tp_first + uint32_t(r) + 1, a.capacity); };
     const uint32_t max_len = len_of(M - 1);
     const uint32_t nblocks = (max_len + BLOCK - 1) / BLOCK;
     uint32_t blk_begin, blk_end;
-    if (nblocks <= a.nsplits) {
+    if (nblocks <= context_splits) {
         blk_begin = split;
         blk_end = split + 1;
         if (split >= nblocks) return;
     } else {
-        blk_begin = split * nblocks / a.nsplits;
-        blk_end = (split + 1) * nblocks / a.nsplits;
+        blk_begin = split * nblocks / context_splits;
+        blk_end = (split + 1) * nblocks / context_splits;
     }
     const uint32_t limit = min(max_len, blk_end * BLOCK);  // tokens of this share end here
     const uint32_t last_tok = limit - 1;                   // rows past it are never read: loads are clamped to it
     const uint32_t range = blk_end - blk_begin;
-    // rounds of equal size (to within a block), none longer than 17 blocks
+    // rounds of equal size (the last may be shorter), none longer than 17 blocks
     // (several rows: one round of up to 17 blocks, or rounds of up to 8)
     constexpr uint32_t LONG_ROUND = W::ALTERNATE ? W::ALT_BLOCKS : W::SHORT_BLOCKS;
     const uint32_t n_rounds = range > uint32_t(RBK) ? (range + LONG_ROUND - 1) / LONG_ROUND : 1;
     const bool alt = W::ALTERNATE && n_rounds > 1;  // rounds in alternate halves of LDS
     const uint32_t per_round = (range + n_rounds - 1) / n_rounds;
     auto blocks_of = [&](uint32_t round) { return min(range - round * per_round, per_round); };
-
     auto dma = [&](uint32_t lds_addr, uint32_t voff, const void *src) {
         asm volatile("s_mov_b32 m0, %0\n"
                      "s_nop 0\n"
@@ -1260,6 +1541,40 @@ __global__ __launch_bounds__((KeysFirst<BITS, M>::LOADERS + KeysFirst<BITS, M>::
     float *bmax_lds = reinterpret_cast<float *>(lds_raw + W::BMAX_OFF);
     float *bsum_lds = reinterpret_cast<float *>(lds_raw + W::BSUM_OFF);
     float *zs_lds = reinterpret_cast<float *>(lds_raw + W::ZS_OFF);
+    if constexpr (PREP) {
+        // The norm and the rotation of the query rows, while the first keys are on their way: wave w has k-step w of every
+        // row, the waves 0 and 1 the dims 0-63 that are rotated (lane 16 row + i of them computes angle i of the wave's 16).
+        float sine = 0.0f, cosine = 0.0f;
+#pragma unroll
+        for (int p = 0; p < W::PAIRS; p++) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) sum += qv[p][e] * qv[p][e];
+            sum = across_rows<16, 64>(sum, SumOp());
+            if (j == 0) zs_lds[(wave * W::PAIRS + p) * 16 + n] = sum;
+        }
+        raise(W::C_NORM);
+        if (wave < 2) rope_angle(sync_lds[W::C_POSITION] + min(j, M - 1), 16 * (n >> 3) + 8 * wave + (n & 7), 32, prep->p.log2_theta, sine, cosine);
+        await(W::C_NORM, W::WAVES);
+#pragma unroll
+        for (int p = 0; p < W::PAIRS; p++) {
+            float total = 0.0f;
+#pragma unroll
+            for (int w = 0; w < W::WAVES; w++) total += zs_lds[(w * W::PAIRS + p) * 16 + n];
+            const float scale = norm_scale(total, prep->p.eps);
+#pragma unroll
+            for (int e = 0; e < 8; e++) qv[p][e] *= scale * norm_w[e];
+            if (wave < 2) {
+                const int row = M == 1 ? 0 : min(2 * p + (n >> 3), M - 1);
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float s = __shfl(sine, 16 * row + 8 * (j & 1) + e), c = __shfl(cosine, 16 * row + 8 * (j & 1) + e);
+                    const float x = qv[p][e], other = half_swap(x, j < 2);
+                    qv[p][e] = j < 2 ? rope_first(x, other, s, c) : rope_second(other, x, s, c);
+                }
+            }
+        }
+    }
     // the scores of block b, row r: [head][token] f32 over the block's keys
     auto s_block = [&](int b, int r) { return reinterpret_cast<float *>(lds_raw + W::K_OFF + b * W::K_BLOCK_BYTES + r * 512); };
 
@@ -2410,6 +2725,15 @@ __global__ __launch_bounds__((KeysFirst<BITS, M>::LOADERS + KeysFirst<BITS, M>::
     leave();
 }
 
+template <int BITS, int M>
+__global__ __launch_bounds__((KeysFirst<BITS, M>::THREADS_)) void attention_partial_kernel_s(PartialArgs a) {
+    attention_partial_s_body<BITS, M, false>(a, nullptr);
+}
+template <int BITS, int M>
+__global__ __launch_bounds__((KeysFirst<BITS, M>::THREADS_)) void attention_token_kernel_s(TokenArgs t) {
+    attention_partial_s_body<BITS, M, true>(t.a, &t.prep);
+}
+
 // Merges the splits of one (q head, row): weights 2^(m_c - M), then the gate
 // (reference: attention_reduce / attention_reduce_rows,
 // kernels/attention.metal:367-409, kernels/attention_rows.metal:296-342).
@@ -2421,6 +2745,7 @@ struct ReduceArgs {
     uint32_t heads, capacity, nsplits, rows;
     const saetta_token_params *tp;
     uint32_t decode_len;
+    uint32_t last_is_new;  // 1: the last split is the new tokens' (attention_token_kernel_*), the others the context before them
 };
 
 constexpr uint32_t MAX_SPLITS = 256;  // workgroups per kv head: 2 kv heads fill 512 slots of 256 CUs
@@ -2453,9 +2778,10 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
     // splits of this wave: per_wave (a multiple of 16) from per_wave * wave on; of this lane: slot + 16 i
     const uint32_t per_wave = (a.nsplits + 63) / 64 * 16;
     constexpr int PER_LANE = MAX_SPLITS / 64;
-    const uint32_t max_len = min(a.decode_len ? a.tp->kv_len : a.tp->position + a.rows, a.capacity);
+    const uint32_t seen = min(a.decode_len ? a.tp->kv_len : a.tp->position + a.rows, a.capacity);
+    const uint32_t max_len = a.last_is_new ? min(seen, a.tp->position) : seen;
     const uint32_t nblocks = (max_len + BLOCK - 1) / BLOCK;
-    const uint32_t parts = min(a.nsplits, nblocks);
+    const uint32_t parts = min(a.nsplits - a.last_is_new, nblocks), fresh = a.last_is_new ? a.nsplits - 1 : ~0u;
     // Slots past the splits at work hold old values: they are dropped by select, never multiplied.  (One and two rows read
     // them all the same: waiting for the length first costs more than up to 2 MB of old partials a row.)
     const uint32_t limit = a.rows > 2 ? parts : a.nsplits;
@@ -2466,7 +2792,7 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
         const uint32_t c = per_wave * wave + slot + 16 * i;
         mlv[i] = floatx2{NO_SCORE, 0.0f};
         pv[i] = floatx4{0, 0, 0, 0};
-        if (16 * uint32_t(i) < per_wave && c < limit) {
+        if (16 * uint32_t(i) < per_wave && (c < limit || c == fresh)) {
             mlv[i] = *reinterpret_cast<const floatx2 *>(ml + 2 * (size_t(c) * a.heads + h));
             pv[i] = *reinterpret_cast<const floatx4 *>(po + (size_t(c) * a.heads + h) * DIM + REDUCE_DIMS * slice + 4 * quad);
         }
@@ -2476,7 +2802,8 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
     float m[PER_LANE], mx = NO_SCORE;
 #pragma unroll
     for (int i = 0; i < PER_LANE; i++) {
-        const bool live = 16 * uint32_t(i) < per_wave && per_wave * wave + slot + 16 * i < parts;
+        const uint32_t c = per_wave * wave + slot + 16 * i;
+        const bool live = 16 * uint32_t(i) < per_wave && (c < parts || c == fresh);
         m[i] = live ? mlv[i][0] : NO_SCORE;
         if (!live) mlv[i][1] = 0.0f, pv[i] = floatx4{0, 0, 0, 0};
         mx = fmaxf(mx, m[i]);
@@ -2531,16 +2858,19 @@ uint32_t splits_for(uint32_t capacity, uint32_t wanted) {
 // that served there before, 28.3 against 29.7 at 150k, 4-bit, for the two-workgroups-per-CU kernel).
 constexpr uint32_t KEYS_FIRST_FROM = 24 * 1024;
 
+// token: with the step before the scores taken in (nullptr: not)
 template <int BITS, int TILES, bool PACKED>
-void launch_partial(hipStream_t stream, const PartialArgs &a, bool one_per_cu, bool keys_first) {
+void launch_partial(hipStream_t stream, const PartialArgs &a, bool one_per_cu, bool keys_first, const TokenArgs *token) {
     void (*kernel)(PartialArgs);
     int lds_bytes;
+    const dim3 grid(a.nsplits, a.kv_heads);
     if constexpr (BITS != 16) {
         if (keys_first) {
             auto launch_rows = [&](auto rows_c) {
                 constexpr int MR = decltype(rows_c)::value;
                 using W = KeysFirst<BITS, MR>;
-                launch(attention_partial_kernel_s<BITS, MR>, dim3(a.nsplits, a.kv_heads), (W::LOADERS + W::WAVES) * 64, W::LDS_BYTES, stream, a);
+                if (token) launch(attention_token_kernel_s<BITS, MR>, dim3(token->a.nsplits, a.kv_heads), W::THREADS_, W::LDS_BYTES, stream, *token);
+                else launch(attention_partial_kernel_s<BITS, MR>, grid, W::THREADS_, W::LDS_BYTES, stream, a);
             };
             if (a.rows == 1) launch_rows(std::integral_constant<int, 1>());
             else if (a.rows == 2) launch_rows(std::integral_constant<int, 2>());
@@ -2565,20 +2895,59 @@ void launch_partial(hipStream_t stream, const PartialArgs &a, bool one_per_cu, b
         lds_bytes = Shape<BITS, TILES, PACKED, itb_rows<TILES>()>::LDS_BYTES;
     }
     // (the dynamic LDS limit of every variant was raised in setup_decode)
-    launch(kernel, dim3(a.nsplits, a.kv_heads), THREADS, lds_bytes, stream, a);
+    if (token) {
+        const dim3 both(token->a.nsplits - 1 + a.rows * (SAETTA_GQA_GROUP / token->new_heads), a.kv_heads);
+        if constexpr (PACKED) launch(attention_token_kernel_p<BITS>, both, THREADS, lds_bytes, stream, *token);
+        else if constexpr (TILES <= 2) launch(attention_token_kernel_n<BITS, TILES>, both, THREADS, lds_bytes, stream, *token);
+        return;
+    }
+    launch(kernel, grid, THREADS, lds_bytes, stream, a);
 }
 
 template <int BITS>
-void launch_partial_rows(hipStream_t stream, const PartialArgs &a, bool one_per_cu, bool keys_first) {
+void launch_partial_rows(hipStream_t stream, const PartialArgs &a, bool one_per_cu, bool keys_first, const TokenArgs *token = nullptr) {
     if (a.rows == 1) {
-        launch_partial<BITS, 1, true>(stream, a, one_per_cu, keys_first);
+        launch_partial<BITS, 1, true>(stream, a, one_per_cu, keys_first, token);
     } else if (a.rows == 2) {
-        launch_partial<BITS, 1, false>(stream, a, one_per_cu, keys_first);
+        launch_partial<BITS, 1, false>(stream, a, one_per_cu, keys_first, token);
     } else if (a.rows <= 4) {
-        launch_partial<BITS, 2, false>(stream, a, one_per_cu, keys_first);
+        launch_partial<BITS, 2, false>(stream, a, one_per_cu, keys_first, token);
     } else {
-        launch_partial<BITS, 4, false>(stream, a, one_per_cu, keys_first);
+        launch_partial<BITS, 4, false>(stream, a, one_per_cu, keys_first, token);
     }
+}
+
+// Whether the last two launches of a plan in the making are the step before the scores and the partial stage `a` of the
+// same rows over the same buffers, so that the reduce stage about to be recorded makes them one layer's token step, which
+// the kernels of TokenArgs do in one launch less.  They are written for 64 rotary dims, and the new tokens take a split of
+// their own: with fewer than 4 the context would be left with too few workgroups.
+bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const float *q_and_gate, bool keys_first, TokenArgs &token) {
+    const size_t n = list.launches.size();
+    if (n < 2 || a.nsplits < 4) return false;
+    const LaunchRecord &before = list.launches[n - 2], &partial = list.launches[n - 1];
+    if (before.kind != LAUNCH_PREP || partial.kind != LAUNCH_PARTIAL || int(before.bits) != bits || int(partial.bits) != bits || before.rows != a.rows) return false;
+    const PartialArgs &b = list.arg<PartialArgs>(partial, 0);
+    if (b.q != a.q || b.kdata != a.kdata || b.vdata != a.vdata || b.kscales != a.kscales || b.kbiases != a.kbiases || b.vscales != a.vscales || b.vbiases != a.vbiases ||
+        b.part_o != a.part_o || b.part_ml != a.part_ml || b.heads != a.heads || b.kv_heads != a.kv_heads || b.capacity != a.capacity || b.scale != a.scale ||
+        b.rows != a.rows || b.nsplits != a.nsplits || b.tp != a.tp || b.decode_len != a.decode_len) return false;
+    const PrepArgs prep = list.arg<PrepArgs>(before, 0);
+    const bool cache = bits == 16 ? prep.keys_half == a.kdata && prep.values_half == a.vdata
+                                  : prep.kq.data == a.kdata && prep.kq.scales == a.kscales && prep.kq.biases == a.kbiases && prep.vq.data == a.vdata &&
+                                        prep.vq.scales == a.vscales && prep.vq.biases == a.vbiases;
+    if (!(cache && prep.q_out == a.q && prep.q_and_gate == q_and_gate && prep.tp == a.tp && prep.capacity == a.capacity && prep.p.heads == a.heads &&
+          prep.p.kv_heads == a.kv_heads && prep.p.half_dims == 32 && aligned(prep.q_and_gate, 16) && aligned(prep.q_norm, 16))) return false;
+    token = TokenArgs{a, prep, SAETTA_GQA_GROUP};
+    if (!keys_first) {
+        // more rows than four: the workgroups of the new rows need longer than the launch takes (18.7 against 18.2 us per
+        // layer at 8 rows and 300 tokens, f16)
+        if (a.rows > NEW_ROWS) return false;
+        // as many splits as before, one of them the new tokens'.  Their workgroups beside the context's: two heads to one
+        // while all fit one to a CU, a whole row to one where the context gives up CUs for them.
+        const uint32_t room = MAX_SPLITS / 2;
+        if (a.nsplits - 1 + 4 * a.rows <= room) token.new_heads = 2;
+        else if (a.nsplits - 1 + a.rows > room) token.a.nsplits = room - a.rows + 1;
+    }
+    return true;
 }
 
 int run_attention(hipStream_t stream, int bits, const float *q, const void *kdata, const void *vdata,
@@ -2619,19 +2988,33 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
     const bool keys_first = rows <= 4 && bits != 16 && capacity >= KEYS_FIRST_FROM && !(stages & SAETTA_STAGE_NO_LOADERS);
     const bool one_per_cu = rows >= 2 || bits == 16 || capacity <= 80 * 1024 || keys_first;
     if (one_per_cu && nsplits > MAX_SPLITS / 2) nsplits = MAX_SPLITS / 2;
-    if (stages & SAETTA_STAGE_PARTIAL) {
-        PartialArgs a{q,     kdata,    vdata,    ks,    kz,   vs,      vz,   part_o, part_ml,
-                      heads, kv_heads, capacity, scale, rows, nsplits, d_tp, decode_len ? 1u : 0u, device_status_word()};
+    const PartialArgs a{q,     kdata,    vdata,    ks,    kz,   vs,      vz,   part_o, part_ml,
+                        heads, kv_heads, capacity, scale, rows, nsplits, d_tp, decode_len ? 1u : 0u, device_status_word()};
+    auto partial = [&](const TokenArgs *token) {
         if (bits == 8) {
-            launch_partial_rows<8>(stream, a, one_per_cu, keys_first);
+            launch_partial_rows<8>(stream, a, one_per_cu, keys_first, token);
         } else if (bits == 4) {
-            launch_partial_rows<4>(stream, a, one_per_cu, keys_first);
+            launch_partial_rows<4>(stream, a, one_per_cu, keys_first, token);
         } else {
-            launch_partial_rows<16>(stream, a, one_per_cu, keys_first);
+            launch_partial_rows<16>(stream, a, one_per_cu, keys_first, token);
         }
+    };
+    if (stages & SAETTA_STAGE_PARTIAL) {
+        partial(nullptr);
+        tag_launch(LAUNCH_PARTIAL, uint32_t(bits), rows);
     }
     if (stages & SAETTA_STAGE_REDUCE) {
-        ReduceArgs r{part_o, part_ml, q_and_gate, out, heads, capacity, nsplits, rows, d_tp, decode_len ? 1u : 0u};
+        uint32_t last_is_new = 0;
+        if (LaunchList *list = recording()) {
+            TokenArgs token;
+            if (one_per_cu && token_step(*list, a, bits, q_and_gate, keys_first, token)) {
+                list->launches.pop_back(), list->launches.pop_back();
+                partial(&token);
+                last_is_new = 1;
+                nsplits = token.a.nsplits;
+            }
+        }
+        ReduceArgs r{part_o, part_ml, q_and_gate, out, heads, capacity, nsplits, rows, d_tp, decode_len ? 1u : 0u, last_is_new};
         launch(attention_reduce_kernel, dim3(heads, rows, DIM / REDUCE_DIMS), 256, 0, stream, r);
     }
     return launch_status(what);
@@ -2640,8 +3023,8 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
 }  // namespace
 
 namespace {
-template <int BITS, int TILES, bool PACKED, int ITB>
-int raise_lds(void (*kernel)(PartialArgs)) {
+template <int BITS, int TILES, bool PACKED, int ITB, class Args>
+int raise_lds(void (*kernel)(Args)) {
     static_assert(Shape<BITS, TILES, PACKED, ITB>::LDS_BYTES <= 160 * 1024, "LDS of a CU");
     if (Shape<BITS, TILES, PACKED, ITB>::LDS_BYTES <= 48 * 1024) return 0;
     return int(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -2649,12 +3032,17 @@ int raise_lds(void (*kernel)(PartialArgs)) {
 }
 template <int BITS, int M>
 int raise_lds_keys_first() {
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_token_kernel_s<BITS, M>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         KeysFirst<BITS, M>::LDS_BYTES))) return rc;
     return int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_partial_kernel_s<BITS, M>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, KeysFirst<BITS, M>::LDS_BYTES));
 }
 template <int BITS>
 int raise_lds_of_bits() {
     if (int rc = raise_lds<BITS, 1, true, ITB_ONE_PER_CU>(attention_partial_kernel_p<BITS>)) return rc;
+    if (int rc = raise_lds<BITS, 1, true, ITB_ONE_PER_CU>(attention_token_kernel_p<BITS>)) return rc;
+    if (int rc = raise_lds<BITS, 1, false, itb_rows<1>()>(attention_token_kernel_n<BITS, 1>)) return rc;
+    if (int rc = raise_lds<BITS, 2, false, itb_rows<2>()>(attention_token_kernel_n<BITS, 2>)) return rc;
     if (int rc = raise_lds<BITS, 1, false, itb_rows<1>()>(attention_partial_kernel_n<BITS, 1>)) return rc;
     if (int rc = raise_lds<BITS, 2, false, itb_rows<2>()>(attention_partial_kernel_n<BITS, 2>)) return rc;
     return raise_lds<BITS, 4, false, itb_rows<4>()>(attention_partial_kernel_n<BITS, 4>);

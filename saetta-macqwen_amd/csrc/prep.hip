@@ -20,24 +20,12 @@
 #include "common.hpp"
 #include "kv_quant_device.hpp"
 #include "lanes.hpp"
+#include "prep_device.hpp"
 
 namespace saetta {
 namespace {
 
 constexpr int DIM = SAETTA_HEAD_DIM;
-
-struct PrepArgs {
-    const float *q_and_gate;  // [row][heads][2 * dim]
-    const float *k, *v;       // [row][kv_heads][dim]
-    const float *q_norm, *k_norm;
-    float *q_out;             // [row][heads][dim]
-    uint16_t *keys_half, *values_half;  // half cache [capacity][kv_heads][dim], or null
-    saetta_quant_rows kq, vq;           // quantized cache (BITS 8 or 4)
-    float *k_back;                      // [row][kv_heads][dim]: the normed, rotated key in f32, or null
-    saetta_prep_params p;
-    const saetta_token_params *tp;
-    uint32_t capacity;
-};
 
 template <int BITS>
 __global__ __launch_bounds__(256) void attention_prep_store_kernel(PrepArgs a) {
@@ -54,21 +42,20 @@ __global__ __launch_bounds__(256) void attention_prep_store_kernel(PrepArgs a) {
                      : a.v[(size_t(row) * kvh + j) * DIM + i];
     if (is_q || is_k) {
         // x * (1 / sqrt(mean(x^2) + eps)) * w, the product taken as x * (scale * w) like the CPU does
-        const float sq = group_reduce<64>(x * x, SumOp());
+        const float sq = square_sum(x);
         if ((i & 63) == 0) partial[i >> 6] = sq;
         __syncthreads();
         const float total = (partial[0] + partial[1]) + (partial[2] + partial[3]);
-        const float scale = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(total, float(DIM)), a.p.eps)));
+        const float scale = norm_scale(total, a.p.eps);
         x = __fmul_rn(x, __fmul_rn(scale, is_q ? a.q_norm[i] : a.k_norm[i]));
         head[i] = x;
         __syncthreads();
         if (i < 2 * half) {
             const uint32_t r = i < half ? i : i - half;
-            const double freq = exp2(-double(r) / double(half) * double(a.p.log2_theta));
-            const double angle = double(position) * freq;
-            const float s = float(sin(angle)), c = float(cos(angle));
+            float s, c;
+            rope_angle(position, r, half, a.p.log2_theta, s, c);
             const float u = head[r], w = head[r + half];
-            x = i < half ? __fsub_rn(__fmul_rn(u, c), __fmul_rn(w, s)) : __fadd_rn(__fmul_rn(u, s), __fmul_rn(w, c));
+            x = i < half ? rope_first(u, w, s, c) : rope_second(u, w, s, c);
         }
         if (is_q) {
             a.q_out[(size_t(row) * heads + j) * DIM + i] = x;
@@ -136,5 +123,6 @@ extern "C" int saetta_attn_prep_store(saetta_stream_t stream, int bits, const fl
     } else {
         launch(attention_prep_store_kernel<16>, grid, 256, 0, as_stream(stream), a);
     }
+    tag_launch(LAUNCH_PREP, uint32_t(bits), rows);
     return launch_status("attn_prep_store");
 }

@@ -221,8 +221,8 @@ class Built:
             g = torch.cuda.CUDAGraph()
             with torch.cuda.graph(g):
                 s = _stream()
-                for _, launch in ops:
-                    launch(s)
+                for part in self._parts:
+                    part(s)
             self.graph = g
 
     def run(self, stream=None):

@@ -1,0 +1,88 @@
+"""A plan's token step: record_store, then decode or verify attention on the same buffers, which the library's plan
+makes one launch less (the partial stage takes the store in, the new tokens get a partial result of their own).
+Every result against the same ops launched one by one: the outputs to the decode tests' bound, q to rounding, what is
+stored bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_common import D, H, KV, VALUES, dev, host, oracle, saetta
+
+pytestmark = pytest.mark.gpu
+KINDS = [saetta.KvBits.Half, saetta.KvBits.Eight, saetta.KvBits.Four]
+PREP = saetta.PrepParams(H, KV, D, 64, 1e7, 1e-6)
+
+
+class Step:
+    def __init__(self, kind, capacity, rows, seed, rope_dims=64):
+        rng = np.random.default_rng(seed)
+        self.rows, self.kind = rows, kind
+        self.qg = dev(rng.standard_normal((rows, H, 2 * D)).astype(np.float32))
+        self.k, self.v = (dev(rng.standard_normal((rows, VALUES)).astype(np.float32)) for _ in range(2))
+        qn, kn = (dev((1 + 0.1 * rng.standard_normal(D)).astype(np.float32)) for _ in range(2))
+        self.cache = saetta.GpuKvCache.with_bits(H, KV, D, capacity, kind)
+        fill = dev(oracle.noise(self.cache.capacity * VALUES, seed).reshape(self.cache.capacity, VALUES))
+        if kind is saetta.KvBits.Half:
+            self.cache.keys.copy_(fill.flatten().half()), self.cache.values.copy_(fill.flatten().flip(0).half())
+        else:
+            for c, x in zip(self.cache.quant, (fill, fill.flip(0).contiguous())):
+                c.encode(x, 0, self.cache.capacity)
+        keys, values = self.cache.quant or (self.cache.keys, self.cache.values)
+        self.q, self.out, self.back = (torch.zeros(rows, n, device="cuda") for n in (H * D, H * D, VALUES))
+        self.plan = saetta.Plan()
+        saetta.record_store(self.plan, self.qg, self.k, self.v, qn, kn, self.q, keys, values, saetta.PrepParams(H, KV, D, rope_dims, 1e7, 1e-6),
+                            self.cache.capacity, rows=rows, k_back=self.back)
+        if rows == 1:
+            (self.cache.decode.record if kind is saetta.KvBits.Half else self.cache.decode.record_quant)(
+                self.plan, self.q, keys, values, self.qg, self.out)
+        else:
+            att = saetta.AttentionRows(H, KV, self.cache.capacity, rows)
+            (att.record if kind is saetta.KvBits.Half else att.record_quant)(
+                self.plan, rows, self.q, keys, values, self.qg, self.out, [self.plan.params] * rows)
+
+    def run(self, how, position):
+        self.plan.set_params(saetta.TokenParams(0, position))
+        self.q.fill_(float("nan")), self.out.fill_(float("nan")), self.back.fill_(float("nan"))
+        how()
+        return [host(t).copy() for t in (self.out, self.q, self.back)] + [host(b).copy() for b in self.cache.buffers()]
+
+
+def launches(step):
+    built = step.plan.build()
+    built.run()
+    return sum(saetta.ffi.lib().saetta_plan_launches(p.plan) for p in built._parts)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("capacity", [512, 8192, 40960])
+def test_fused_step_equals_the_ops_one_by_one(kind, capacity, rows):
+    # 512: four splits, three of them the context's; 8192: 63 of 64; 40960: 127 of 128, codes through the loader kernels
+    step = Step(kind, capacity, rows, seed=capacity + 10 * rows + kind.value)
+    assert launches(step) == (2 if rows <= 4 else 3)  # (five rows and more keep the store a launch of its own)
+    built = step.plan.build()
+    cap = step.cache.capacity
+    # no context; one block and less; around a block's end; several rounds; the last rows; rows that do not fit
+    for position in (0, 1, 15, 16, 100, cap // 2 + 3, cap - rows, cap - 1, cap + 2):
+        want = step.run(step.plan.run_serial, position)
+        before = [host(b).copy() for b in step.cache.buffers()]
+        got = step.run(built.run, position)
+        if position == 0 or position <= cap - rows:
+            assert np.isfinite(got[0]).all(), position
+        ok = np.isfinite(want[0])
+        assert np.array_equal(ok, np.isfinite(got[0]))
+        assert np.abs(got[0] - want[0])[ok].max(initial=0.0) < 2e-5, position
+        assert np.array_equal(got[1], want[1]), position
+        assert np.array_equal(got[2], want[2]), position
+        for a, b in zip(got[3:], before):
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), position
+
+
+def test_other_steps_keep_their_launches():
+    assert launches(Step(saetta.KvBits.Eight, 256, 1, seed=1)) == 3                   # two splits only
+    assert launches(Step(saetta.KvBits.Eight, 8192, 1, seed=1, rope_dims=32)) == 3    # other rotary dims
+    step = Step(saetta.KvBits.Eight, 8192, 1, seed=1)
+    step.plan.ops.insert(1, ("look", lambda s: None))                                # something between the store and the scores
+    built = step.plan.build()
+    built.run()
+    assert [saetta.ffi.lib().saetta_plan_launches(p.plan) for p in built._parts if not callable(getattr(p, "__code__", None)) and hasattr(p, "plan")] == [1, 2]
