@@ -552,6 +552,12 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
     const uint32_t n_it = (range + IT_BLOCKS - 1) / IT_BLOCKS;
     const uint32_t per_it = (range + n_it - 1) / n_it;
     const uint32_t n_rounds = n_it;
+    // Four splits in a row start a quarter of their share apart, so that shares of nearly a power of two do not meet in the
+    // same memory channels at every moment (see attention_partial_s_body; f16, one row: 68 against 58 us per layer at 131000
+    // tokens, 39 against 33 at 65500, the same in between).  3 and 4 rows are bound by their matrix instructions.
+    constexpr bool STAGGER = TILES != 2;
+    const uint32_t first_round = STAGGER ? (split & 3) * n_it / 4 : 0;
+    auto place = [&](uint32_t it) { return it + first_round < n_it ? it + first_round : it + first_round - n_it; };
 
     const uint32_t cap_rows = a.capacity * kvh;
     const __amdgpu_buffer_rsrc_t k_rsrc = make_rsrc(a.kdata, cap_rows * RB);
@@ -568,9 +574,9 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
     KeyRegs<BITS> kreg[KROUNDS][4];
     ValRegs<BITS> vreg[KSTEPS];
     u32x2 ksr = {0, 0}, kzr = {0, 0}, vsr = {0, 0}, vzr = {0, 0};
-    auto blocks_of = [&](uint32_t it) { return it < n_it ? min(per_it, blk_end - (blk_begin + it * per_it)) : 0u; };
+    auto blocks_of = [&](uint32_t it) { return it < n_it ? min(per_it, blk_end - (blk_begin + place(it) * per_it)) : 0u; };
     auto load_keys = [&](uint32_t it) {
-        const uint32_t base = (blk_begin + it * per_it) * BLOCK, nb = blocks_of(it);
+        const uint32_t base = (blk_begin + place(it) * per_it) * BLOCK, nb = blocks_of(it);
         const int voff = int((base + BLOCK * wave + n) * kvh + kv) * RB + j * key_piece<BITS>();
 #pragma unroll
         for (int i = 0; i < KROUNDS; i++) {
@@ -584,7 +590,7 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
     };
     auto load_scales = [&](uint32_t it) {
         if constexpr (QUANT) {
-            const uint32_t base = (blk_begin + it * per_it) * BLOCK;
+            const uint32_t base = (blk_begin + place(it) * per_it) * BLOCK;
             const bool need = uint32_t(tid) < blocks_of(it) * BLOCK;
             if (UNCOND || need) {
                 const int voff = need ? int((base + tid) * kvh + kv) * 8 : OOB;
@@ -596,7 +602,7 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
         }
     };
     auto load_values = [&](uint32_t it) {
-        const uint32_t base = (blk_begin + it * per_it) * BLOCK, ksteps = (blocks_of(it) + 1) / 2;
+        const uint32_t base = (blk_begin + place(it) * per_it) * BLOCK, ksteps = (blocks_of(it) + 1) / 2;
         const int voff = int((base + 8 * j) * kvh + kv) * RB + val_lane_offset<BITS>(wave, n);
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ks++) {
@@ -739,7 +745,7 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
 
     for (uint32_t round = 0; round < n_rounds; round++) {
         const uint32_t it = round;
-        const uint32_t blk0 = blk_begin + it * per_it;
+        const uint32_t blk0 = blk_begin + place(it) * per_it;
         const uint32_t nb = blocks_of(it);  // blocks of this iteration, 0..ITB
         const uint32_t base = blk0 * BLOCK;
         const uint32_t it_tokens = nb * BLOCK;
@@ -1291,6 +1297,13 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
     const bool alt = W::ALTERNATE && n_rounds > 1;  // rounds in alternate halves of LDS
     const uint32_t per_round = (range + n_rounds - 1) / n_rounds;
     auto blocks_of = [&](uint32_t round) { return min(range - round * per_round, per_round); };
+    // The rounds in the order in which the splits take them: four in a row start a quarter of the share apart.  Started all at
+    // the front they read addresses one share apart at every moment, and shares of nearly a power of two then meet in the
+    // same memory channels: 40.5 us per layer at 131000 tokens (8-bit, one row) against 34.2 so, where 128000 take 32.5
+    // and 33.0.  (Fewer rounds than 8: nothing to gain, and 60000 tokens took 21.8 us instead of 21.3.)
+    const uint32_t first_round = n_rounds >= 8 ? (split & 3) * n_rounds / 4 : 0;
+    auto place = [&](uint32_t round) { return round + first_round < n_rounds ? round + first_round : round + first_round - n_rounds; };
+
     auto dma = [&](uint32_t lds_addr, uint32_t voff, const void *src) {
         asm volatile("s_mov_b32 m0, %0\n"
                      "s_nop 0\n"
@@ -1356,7 +1369,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
             // which lay in the same half, has been used up: its scales are read until every wave has built its operands,
             // its keys until every wave has its scores. ----
             for (uint32_t round = L; round < n_rounds; round += 2) {
-                const uint32_t base = (blk_begin + round * per_round) * BLOCK, nb = blocks_of(round);
+                const uint32_t base = (blk_begin + place(round) * per_round) * BLOCK, nb = blocks_of(place(round));
                 const uint32_t half = L * W::ALT_BLOCKS;  // the blocks of LDS this round goes to start here
                 if (round > 1) await(W::C_BUILT, W::WAVES * (round - 1));
                 if (round > 0) await(W::C_VREQ, round);
@@ -1387,7 +1400,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
         }
         // (one row: more than one round is taken above)
         for (uint32_t round = 0; round < (M == 1 ? 1u : n_rounds); round++) {
-            const uint32_t base = (blk_begin + round * per_round) * BLOCK, nb = blocks_of(round);
+            const uint32_t at = M == 1 ? 0 : place(round), base = (blk_begin + at * per_round) * BLOCK, nb = blocks_of(at);
             // the round before: its scales are read until every wave has built its operands, its keys until every wave has its scores
             if (round > 0) await(W::C_BUILT, W::WAVES * round);
 #pragma unroll
@@ -1455,7 +1468,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
             // ---- alternate halves: loader L takes the values of the rounds L, L + 2, ... whole, each behind its round's
             // keys in the stream, into the half that the round before last has left (every wave through with its values) ----
             for (uint32_t round = L; round < n_rounds; round += 2) {
-                const uint32_t base = (blk_begin + round * per_round) * BLOCK, nb = blocks_of(round);
+                const uint32_t base = (blk_begin + place(round) * per_round) * BLOCK, nb = blocks_of(place(round));
                 const uint32_t half = L * W::ALT_BLOCKS;
                 await(W::C_KEYS, round + 1);
                 if (round > 1) await(W::C_DONE, W::WAVES * (round - 1));
@@ -1478,7 +1491,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
             return;
         }
         for (uint32_t round = 0; round < (M == 1 ? 1u : n_rounds); round++) {
-            const uint32_t base = (blk_begin + round * per_round) * BLOCK, nb = blocks_of(round);
+            const uint32_t at = M == 1 ? 0 : place(round), base = (blk_begin + at * per_round) * BLOCK, nb = blocks_of(at);
             // the keys of the first round have been requested | every wave is through with the values before
             if (round == 0) {
                 await(W::C_KEYS, W::K_LOADERS);
@@ -1692,7 +1705,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
             await(W::C_QUERY, W::WAVES);
 #pragma unroll 1
             for (uint32_t round = 0; round < n_rounds; round++) {
-                const uint32_t base = (blk_begin + round * per_round) * BLOCK, nb = blocks_of(round);
+                const uint32_t base = (blk_begin + place(round) * per_round) * BLOCK, nb = blocks_of(place(round));
                 const uint32_t round_limit = min(limit, base + nb * BLOCK);  // tokens of this round end here
                 const uint32_t live_blocks = (nb + 1) & ~1u;  // k-steps are two blocks: the blocks of the k-steps that have tokens
 
@@ -2255,7 +2268,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
             constexpr int AB = W::ALT_BLOCKS, WAVE_BLOCKS = AB / W::WAVES, WAVE_STEPS = AB / 4;
 #pragma unroll 1
             for (uint32_t round = 0; round < n_rounds; round++) {
-                const uint32_t base = (blk_begin + round * per_round) * BLOCK, nb = blocks_of(round);
+                const uint32_t base = (blk_begin + place(round) * per_round) * BLOCK, nb = blocks_of(place(round));
                 const int half = int(round & 1) * AB;  // the round's first block in LDS
                 const uint32_t round_limit = min(limit, base + nb * BLOCK);  // tokens of this round end here
                 const uint32_t live_blocks = (nb + 1) & ~1u;  // k-steps are two blocks: the blocks of the k-steps that have tokens
