@@ -3,8 +3,8 @@
 //
 // Kernels:
 //   deltanet_conv_kernel, deltanet_step_kernel          one token, the reference's two ops
-//   deltanet_conv_rows_kernel, deltanet_conv_state_kernel,
-//   deltanet_rows_kernel, deltanet_gated_norm_rows_kernel   any number of tokens in order (prefill chunks)
+//   deltanet_conv_rows_kernel, deltanet_rows_kernel,
+//   deltanet_gated_norm_rows_kernel   any number of tokens in order (prefill chunks)
 //   deltanet_rows_small_kernel, deltanet_rows_small_tail_kernel
 //                                                       conv and step together for 1..8 tokens
 //
@@ -36,8 +36,6 @@ constexpr int K_DIM = 128;
 constexpr int STEP_THREADS = 1024;
 constexpr int MAX_ROWS_PER_LANE = 8;  // v_dim up to 256
 
-__device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
-__device__ __forceinline__ float silu_f(float x) { return x * sigmoid_f(x); }
 __device__ __forceinline__ float dot4(float4 a, float4 b) { return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w; }
 
 __global__ __launch_bounds__(256) void deltanet_conv_kernel(const float *__restrict__ x, const float *__restrict__ w,
@@ -143,18 +141,28 @@ __device__ __forceinline__ float conv_input(const float *x, const float *state, 
     return i >= 0 ? x[size_t(i) * p.channels + c] : state[size_t(i + int(p.kernel_size) - 1) * p.channels + c];
 }
 
+// After the outputs the last kernel_size - 1 inputs become the state.  Only the tokens before the window's length
+// read it, and those lie in the first tile: its thread of the channel has read what it needs and moves the rows
+// itself, where a launch of its own took 2.5 us.  Rows are written in ascending order and row j only reads rows above
+// it (or x), so the shift is safe in place.
+__device__ __forceinline__ void conv_state_move(const float *x, float *state, uint32_t c, const saetta_conv_rows_params &p) {
+    const int past = int(p.kernel_size) - 1;
+    for (int j = 0; j < past; j++) state[size_t(j) * p.channels + c] = conv_input(x, state, int(p.tokens) - past + j, c, p);
+}
+
 // The same for four channels a thread (16-byte loads and stores, eight tokens' loads in flight), four taps:
 // every channel's sums are taken in the same order as above, so the results are the same bit for bit.
 constexpr uint32_t CONV4_AHEAD = 8;
 static_assert(CONV_TILE % CONV4_AHEAD == 0, "whole groups of tokens in a tile");
+static_assert(CONV_TILE > 15, "every token that reads the state lies in the first tile");
 __global__ __launch_bounds__(256) void deltanet_conv_rows4_kernel(const float *__restrict__ x, const float *__restrict__ w,
-                                                                  const float *__restrict__ state, float *__restrict__ out,
+                                                                  float *state, float *__restrict__ out,
                                                                   float *__restrict__ snaps, saetta_conv_rows_params p) {
     constexpr int KS = 4;
     const uint32_t c4 = blockIdx.x * 256 + threadIdx.x, quads = p.channels / 4;
     if (c4 >= quads) return;
-    const float4 *x4 = reinterpret_cast<const float4 *>(x), *s4 = reinterpret_cast<const float4 *>(state);
-    float4 *o4 = reinterpret_cast<float4 *>(out);
+    const float4 *x4 = reinterpret_cast<const float4 *>(x);
+    float4 *o4 = reinterpret_cast<float4 *>(out), *s4 = reinterpret_cast<float4 *>(state);
     // taps[j] holds tap j of the four channels (w is [channel][4]: the thread's 16 floats lie in a row)
     float4 taps[KS];
     {
@@ -195,13 +203,17 @@ __global__ __launch_bounds__(256) void deltanet_conv_rows4_kernel(const float *_
             }
         }
     }
+    if (blockIdx.y == 0) {  // (a tile of tokens at least: the new state is all inputs)
+#pragma unroll
+        for (int j = 0; j < KS - 1; j++) s4[size_t(j) * quads + c4] = x4[size_t(p.tokens - (KS - 1) + j) * quads + c4];
+    }
 }
 
 template <int KS>  // taps; 0: any number (read from p), the window is re-read from memory
 __global__ __launch_bounds__(256) void deltanet_conv_rows_kernel(const float *__restrict__ x,
                                                                  const float *__restrict__ w,
-                                                                 const float *__restrict__ state,
-                                                                 float *__restrict__ out, float *__restrict__ snaps,
+                                                                 float *state, float *__restrict__ out,
+                                                                 float *__restrict__ snaps,
                                                                  saetta_conv_rows_params p) {
     const uint32_t c = blockIdx.x * 256 + threadIdx.x;
     if (c >= p.channels) return;
@@ -242,18 +254,7 @@ __global__ __launch_bounds__(256) void deltanet_conv_rows_kernel(const float *__
             }
         }
     }
-}
-
-// After the outputs: the last kernel_size - 1 inputs become the state.  Rows are written in
-// ascending order and row j only reads rows above it (or x), so the shift is safe in place.
-__global__ __launch_bounds__(256) void deltanet_conv_state_kernel(const float *__restrict__ x, float *state,
-                                                                  saetta_conv_rows_params p) {
-    const uint32_t c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= p.channels) return;
-    const int past = int(p.kernel_size) - 1;
-    for (int j = 0; j < past; j++) {
-        state[size_t(j) * p.channels + c] = conv_input(x, state, int(p.tokens) - past + j, c, p);
-    }
+    if (blockIdx.y == 0) conv_state_move(x, state, c, p);
 }
 
 // The delta rule over the tokens, in order.  A workgroup owns a few rows of one value head's state
@@ -959,7 +960,6 @@ extern "C" int saetta_deltanet_conv_rows(saetta_stream_t stream, const float *x,
     } else {
         launch(deltanet_conv_rows_kernel<0>, grid, 256, 0, as_stream(stream), x, w, state, out, snaps, p);
     }
-    launch(deltanet_conv_state_kernel, grid.x, 256, 0, as_stream(stream), x, state, p);
     return launch_status("deltanet_conv_rows");
 }
 

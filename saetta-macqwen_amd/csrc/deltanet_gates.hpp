@@ -1,4 +1,4 @@
-// Shared by the Gated DeltaNet kernel files: the gates of a token and head.
+// Shared by the Gated DeltaNet kernel files: the gates of a token and head, the conv's activation.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -24,5 +24,8 @@ __device__ __forceinline__ void fast_gates(float a_plus_bias, float exp_a_log, f
     g = __expf(lg);
     beta = __builtin_amdgcn_rcpf(1.0f + __expf(-b));
 }
+
+__device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
+__device__ __forceinline__ float silu_f(float x) { return x * sigmoid_f(x); }
 
 }  // namespace saetta
