@@ -953,6 +953,7 @@ extern "C" int saetta_deltanet_conv_rows(saetta_stream_t stream, const float *x,
                          (!p.snapshots || aligned(snaps, 16));
     if (p.kernel_size == 4 && by_four) {
         launch(deltanet_conv_rows4_kernel, dim3((p.channels / 4 + 255) / 256, grid.y), 256, 0, as_stream(stream), x, w, state, out, snaps, p);
+        tag_launch(LAUNCH_CONV, 0, 0);
     } else if (p.kernel_size == 4) {
         launch(deltanet_conv_rows_kernel<4>, grid, 256, 0, as_stream(stream), x, w, state, out, snaps, p);
     } else if (p.kernel_size == 2) {

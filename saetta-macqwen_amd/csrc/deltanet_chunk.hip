@@ -69,7 +69,12 @@ struct ChunkArgs {
     unsigned char *ws;
     uint32_t k_heads, v_heads, v_dim, tokens, channels;
     float eps;
+    // the conv before it, where the prepare kernel makes that too (`mixed` is then its output)
+    const float *x, *conv_w;
+    float *conv_state;
 };
+constexpr int CONV = 4;     // taps of the conv that the prepare kernel makes
+constexpr int CONV_V = 128;  // ... and the value dim it takes
 
 // x as an f16 hi part and an f16 lo part.  The lo part has to complete the hi part that is stored: where x is
 // a product, the compiler may round the exact product to f16 for the one and the f32 product for the other, and
@@ -130,8 +135,46 @@ __device__ __forceinline__ void read_by_column(uint32_t at, uint32_t part_bytes,
     lo = __builtin_bit_cast(half8, u32x4{r[1][0].x, r[1][0].y, r[1][1].x, r[1][1].y});
 }
 
-template <int G>
-__global__ __launch_bounds__(256) void deltanet_chunk_prepare_kernel(ChunkArgs a) {
+// The conv of four channels c4 .. c4 + 3 for the 16 tokens from t0 on, in two parts: the inputs are asked for, and
+// the outputs made, with the sums in the order of deltanet_conv_rows4_kernel (the results are the same bit for bit).
+struct ConvPiece {
+    float4 taps[CONV], in[CONV - 1 + 16];
+    __device__ __forceinline__ void request(const ChunkArgs &a, uint32_t c, uint32_t t0) {
+#pragma unroll
+        for (int j = 0; j < CONV; j++) taps[j] = reinterpret_cast<const float4 *>(a.conv_w + size_t(c) * CONV)[j];  // (by channel)
+#pragma unroll
+        for (int i = 0; i < CONV - 1 + 16; i++) {
+            const int t = int(t0) + i - (CONV - 1);
+            // (a token past the end: unused)
+            const float *row = t >= 0 ? a.x + size_t(min(uint32_t(t), a.tokens - 1)) * a.channels : a.conv_state + (t + CONV - 1) * a.channels;
+            in[i] = *reinterpret_cast<const float4 *>(row + c);
+        }
+    }
+    __device__ __forceinline__ float4 output(int i) const {
+        float4 sum = make_float4(0, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < CONV; j++) {
+            const float4 v = in[i + j];
+            const float w[4] = {j == 0 ? taps[0].x : j == 1 ? taps[0].y : j == 2 ? taps[0].z : taps[0].w, j == 0 ? taps[1].x : j == 1 ? taps[1].y : j == 2 ? taps[1].z : taps[1].w,
+                                j == 0 ? taps[2].x : j == 1 ? taps[2].y : j == 2 ? taps[2].z : taps[2].w, j == 0 ? taps[3].x : j == 1 ? taps[3].y : j == 2 ? taps[3].z : taps[3].w};
+            sum.x += w[0] * v.x, sum.y += w[1] * v.y, sum.z += w[2] * v.z, sum.w += w[3] * v.w;
+        }
+        return make_float4(silu_f(sum.x), silu_f(sum.y), silu_f(sum.z), silu_f(sum.w));
+    }
+    // the first block's piece: the chunk's last inputs become the conv's state, which only that piece has read
+    __device__ __forceinline__ void keep_state(const ChunkArgs &a, uint32_t c) const {
+#pragma unroll
+        for (int j = 0; j < CONV - 1; j++)
+            *reinterpret_cast<float4 *>(a.conv_state + j * a.channels + c) = *reinterpret_cast<const float4 *>(a.x + size_t(a.tokens - (CONV - 1) + j) * a.channels + c);
+    }
+};
+
+// CONVOLVE: the conv before the delta rule is part of it.  The workgroup's channels, q and k of its key head and the
+// values of its heads, are nobody else's.  A thread makes four channels' outputs for 16 tokens, of q or k and then of
+// the values, and stores them as the conv's own kernel does; q and k also go to LDS as f32, over the place of the
+// images, and from there to the threads that normalise them.
+template <int G, bool CONVOLVE>
+__global__ __launch_bounds__(256, 2) void deltanet_chunk_prepare_kernel(ChunkArgs a, float *conv_out) {
     using L = PrepLds<G>;
     constexpr int DROW = L::DROW, HROW = L::HROW;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -153,6 +196,34 @@ __global__ __launch_bounds__(256) void deltanet_chunk_prepare_kernel(ChunkArgs a
     auto ws_v = [&](int hh) { return ws_blk + a.k_heads * KHEAD_BYTES + (h0 + hh) * VHEAD_BYTES; };
     const bool writer = h0 % group == 0;  // one workgroup of the key head's keeps the q / k images
 
+    // ---- the conv (src/cpu/deltanet.rs:69-100) of the workgroup's channels ----
+    constexpr int FROW = 2 * K_DIM + 4;  // f32 per token's q | k in LDS
+    static_assert(C * FROW * 4 <= 4 * K_IMG, "the f32 q and k lie over the images");
+    float *qk_lds = reinterpret_cast<float *>(lds);
+    if constexpr (CONVOLVE) {
+        static_assert(G * CONV_V == 4 * 64, "a wave's lanes take the values of a token");
+        const uint32_t t0 = blk * C + 16 * wave;
+        const uint32_t cqk = (lane < 32 ? 0 : key_size - K_DIM) + khd * K_DIM + 4 * lane;  // q: lanes 0-31, k: lanes 32-63
+        const uint32_t cv = 2 * key_size + h0 * CONV_V + 4 * lane;
+        ConvPiece qk, vs;
+        qk.request(a, cqk, t0);
+        vs.request(a, cv, t0);
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const bool real = t0 + i < a.tokens;
+            const float4 y = real ? qk.output(i) : make_float4(0, 0, 0, 0);
+            *reinterpret_cast<float4 *>(qk_lds + (16 * wave + i) * FROW + 4 * lane) = y;
+            if (real) *reinterpret_cast<float4 *>(conv_out + size_t(t0 + i) * a.channels + cqk) = y;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const float4 y = vs.output(i);
+            if (t0 + i < a.tokens) *reinterpret_cast<float4 *>(conv_out + size_t(t0 + i) * a.channels + cv) = y;
+        }
+        if (t0 == 0) qk.keep_state(a, cqk), vs.keep_state(a, cv);
+        __syncthreads();
+    }
+
     // ---- q and k of the block's tokens, normalised (src/cpu/deltanet.rs:133-146), as hi and lo parts ----
     {
         // thread (token t, part): the 8-value pieces part, part + 4, part + 8, part + 12 of the token's q and k, so
@@ -163,7 +234,11 @@ __global__ __launch_bounds__(256) void deltanet_chunk_prepare_kernel(ChunkArgs a
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             qv[i] = kv[i] = make_float4(0, 0, 0, 0);
-            if (tok < a.tokens) {
+            if (CONVOLVE) {
+                const float *row = qk_lds + t * FROW + 8 * (part + 4 * (i >> 1)) + 4 * (i & 1);
+                qv[i] = *reinterpret_cast<const float4 *>(row);
+                kv[i] = *reinterpret_cast<const float4 *>(row + K_DIM);
+            } else if (tok < a.tokens) {
                 const float *row = a.mixed + size_t(tok) * a.channels + khd * K_DIM + 8 * (part + 4 * (i >> 1)) + 4 * (i & 1);
                 qv[i] = *reinterpret_cast<const float4 *>(row);
                 kv[i] = *reinterpret_cast<const float4 *>(row + key_size);
@@ -171,6 +246,7 @@ __global__ __launch_bounds__(256) void deltanet_chunk_prepare_kernel(ChunkArgs a
             qs += qv[i].x * qv[i].x + qv[i].y * qv[i].y + qv[i].z * qv[i].z + qv[i].w * qv[i].w;
             ks += kv[i].x * kv[i].x + kv[i].y * kv[i].y + kv[i].z * kv[i].z + kv[i].w * kv[i].w;
         }
+        if (CONVOLVE) __syncthreads();  // the f32 q and k are read: the images go over them
         qs = group_reduce<4>(qs, SumOp());
         ks = group_reduce<4>(ks, SumOp());
         const bool real = tok < a.tokens;
@@ -727,13 +803,11 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
 }  // namespace
 
 int setup_deltanet_chunk() {
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(deltanet_chunk_prepare_kernel<1>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, PrepLds<1>::BYTES))) {
-        return rc;
-    }
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(deltanet_chunk_prepare_kernel<2>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, PrepLds<2>::BYTES))) {
-        return rc;
+    const std::pair<const void *, int> prepares[] = {{reinterpret_cast<const void *>(deltanet_chunk_prepare_kernel<1, false>), PrepLds<1>::BYTES},
+                                                     {reinterpret_cast<const void *>(deltanet_chunk_prepare_kernel<2, false>), PrepLds<2>::BYTES},
+                                                     {reinterpret_cast<const void *>(deltanet_chunk_prepare_kernel<2, true>), PrepLds<2>::BYTES}};
+    for (const auto &[kernel, bytes] : prepares) {
+        if (int rc = int(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes))) return rc;
     }
     return int(hipFuncSetAttribute(reinterpret_cast<const void *>(deltanet_chunk_chain_kernel),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, ChainLds::BYTES));
@@ -744,15 +818,59 @@ size_t deltanet_chunk_workspace_bytes(const saetta_rows_step_params &p) {
     return size_t((p.tokens + C - 1) / C) * block_bytes(p.k_heads, p.v_heads);
 }
 
+namespace {
+// Whether the launch recorded last is the conv that made `mixed` for this call; it is then taken off the list and the
+// prepare kernel makes it too.  For a call of its own the conv has run before this call is known.  The conv's inputs
+// are read beside what this call writes and reads here, so buffers that a program lays over each other (a workspace in
+// the place of x, gates in the place of `mixed`) keep the two launches.
+bool take_conv(LaunchList &list, ChunkArgs &args, float *&conv_out) {
+    if (list.launches.empty() || list.launches.back().kind != LAUNCH_CONV) return false;
+    const LaunchRecord &conv = list.launches.back();
+    const float *x = list.arg<const float *>(conv, 0), *w = list.arg<const float *>(conv, 1);
+    float *conv_state = list.arg<float *>(conv, 2), *out = list.arg<float *>(conv, 3);
+    const saetta_conv_rows_params &c = list.arg<saetta_conv_rows_params>(conv, 5);
+    if (c.kernel_size != CONV || c.snapshots || c.channels != args.channels || c.tokens != args.tokens || out != args.mixed) return false;
+    const size_t rows = size_t(args.tokens) * args.channels * sizeof(float), gates = size_t(args.tokens) * args.v_heads * sizeof(float);
+    const std::pair<const void *, size_t> inputs[] = {{x, rows}, {w, size_t(CONV) * args.channels * sizeof(float)}, {args.a, gates}, {args.b, gates},
+                                                      {args.a_log, args.v_heads * sizeof(float)}, {args.dt_bias, args.v_heads * sizeof(float)}},
+        outputs[] = {{out, rows}, {conv_state, size_t(CONV - 1) * args.channels * sizeof(float)},
+                     {args.ws, size_t((args.tokens + C - 1) / C) * block_bytes(args.k_heads, args.v_heads)}};
+    const auto apart = [](const std::pair<const void *, size_t> &p, const std::pair<const void *, size_t> &q) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(p.first), b = reinterpret_cast<uintptr_t>(q.first);
+        return a + p.second <= b || b + q.second <= a;
+    };
+    for (const auto &o : outputs) {
+        for (const auto &i : inputs) {
+            if (!apart(o, i)) return false;
+        }
+        for (const auto &other : outputs) {
+            if (&other != &o && !apart(o, other)) return false;
+        }
+    }
+    args.x = x, args.conv_w = w, args.conv_state = conv_state, conv_out = out;
+    list.launches.pop_back();
+    return true;
+}
+}  // namespace
+
 int run_deltanet_chunk(hipStream_t stream, const float *mixed, const float *a, const float *b, const float *a_log,
                        const float *dt_bias, float *state, float *o, const saetta_rows_step_params &p, uint32_t channels,
                        void *workspace) {
     const uint32_t nblocks = (p.tokens + C - 1) / C;
-    ChunkArgs args{mixed, a, b, a_log, dt_bias, state, o, static_cast<unsigned char *>(workspace), p.k_heads, p.v_heads, p.v_dim, p.tokens, channels, p.eps};
-    if (p.v_heads == 2 * p.k_heads) {
-        launch(deltanet_chunk_prepare_kernel<2>, dim3(nblocks, p.k_heads), 256, PrepLds<2>::BYTES, stream, args);
+    ChunkArgs args{mixed, a, b, a_log, dt_bias, state, o, static_cast<unsigned char *>(workspace), p.k_heads, p.v_heads, p.v_dim, p.tokens, channels, p.eps, nullptr, nullptr, nullptr};
+    const bool two_heads = p.v_heads == 2 * p.k_heads;
+    LaunchList *list = recording();
+    float *conv_out = nullptr;
+    // The conv inside: while the workgroups are all on the machine at once, two to a CU.  Past that the conv's own kernel
+    // is the faster one, whose many waves keep the memory busy (whole chunk, us, inside against apart: 1000 tokens 76.8
+    // and 79, 2048 125 and 131; 3000 209 and 199, 4096 290 and 280).
+    const bool conv_inside = two_heads && p.v_dim == CONV_V && nblocks * p.k_heads <= 2 * 256;
+    if (conv_inside && list && take_conv(*list, args, conv_out)) {
+        launch(deltanet_chunk_prepare_kernel<2, true>, dim3(nblocks, p.k_heads), 256, PrepLds<2>::BYTES, stream, args, conv_out);
+    } else if (two_heads) {
+        launch(deltanet_chunk_prepare_kernel<2, false>, dim3(nblocks, p.k_heads), 256, PrepLds<2>::BYTES, stream, args, conv_out);
     } else {
-        launch(deltanet_chunk_prepare_kernel<1>, dim3(nblocks, p.v_heads), 256, PrepLds<1>::BYTES, stream, args);
+        launch(deltanet_chunk_prepare_kernel<1, false>, dim3(nblocks, p.v_heads), 256, PrepLds<1>::BYTES, stream, args, conv_out);
     }
     launch(deltanet_chunk_chain_kernel, dim3(p.v_dim / DV * p.v_heads), 512, ChainLds::BYTES, stream, args);
     return SAETTA_OK;

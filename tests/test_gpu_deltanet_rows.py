@@ -275,6 +275,50 @@ def test_full_chunk_equals_uneven_pieces():
     assert torch.equal(torch.cat(parts), whole) and torch.equal(state3, state4)
 
 
+@pytest.mark.parametrize("k_heads,v_heads,v_dim,tokens,over,launches", [
+    (1, 2, 128, 128, False, 3), (2, 4, 128, 129, False, 3), (16, 32, 128, 191, False, 3), (2, 4, 128, 1027, False, 3),
+    (2, 4, 128, 200, True, 4),   # the workspace lies where x does: x has to be read before it is written
+    (2, 4, 64, 200, False, 4), (2, 2, 128, 200, False, 4), (2, 4, 128, 127, False, 3)])  # (127: conv, rows, norm)
+def test_a_plan_of_conv_and_chunk_gives_what_the_calls_give(k_heads, v_heads, v_dim, tokens, over, launches):
+    # A recorded plan makes the conv inside the chunk's first kernel, call by call it is a kernel of its own: the same
+    # sums in the same order, so every output and both states are the same bits, also on a second run (from the first
+    # run's states).
+    layer = Layer(k_heads, v_heads, v_dim, 4, seed=tokens + v_dim)
+    x, z, a, b = (dev(np.ascontiguousarray(t)) for t in layer.inputs(tokens))
+    w, a_log, dt_bias, norm = dev(layer.conv_w), dev(layer.a_log), dev(layer.dt_bias), dev(layer.norm)
+    conv0, state0 = (torch.randn_like(t) for t in layer.zero_state())
+    lib, ffi, call = saetta.ffi.lib(), saetta.ffi, saetta.host._Call
+    need = lib.saetta_deltanet_rows_workspace_bytes(ffi.RowsStepParamsC(k_heads, v_heads, v_dim, tokens, EPS, 0))
+    room = torch.empty(max(need, x.numel() * 4), dtype=torch.uint8, device="cuda")
+    got = []
+    for recorded in (False, True):
+        mixed, y = torch.full((tokens, layer.channels), 7.0, device="cuda"), torch.full((tokens, layer.val), 7.0, device="cuda")
+        conv, state = conv0.clone(), state0.clone()
+        xs = room[:x.numel() * 4].view(torch.float32) if over else x
+        calls = [call("saetta_deltanet_conv_rows", "conv", (*[t.data_ptr() for t in (xs, w, conv, mixed)], None,
+                                                             ffi.ConvRowsParamsC(layer.channels, 4, tokens, 0))),
+                 call("saetta_deltanet_rows_ws", "rows", (*[t.data_ptr() for t in (mixed, a, b, a_log, dt_bias, state, z, norm, y)], None,
+                                                           ffi.RowsStepParamsC(k_heads, v_heads, v_dim, tokens, EPS, 0),
+                                                           room.data_ptr() if need else None, need))]
+        plan = saetta.Plan()
+        for c in calls:
+            plan.op(c.what, c)
+        built = plan.build()
+        for run in range(2):
+            xs.copy_(x.reshape(-1) if over else x)
+            built.run() if recorded else plan.run_serial()
+            torch.cuda.synchronize()
+            got.append([t.clone() for t in (mixed, y, conv, state)])
+    for run in range(2):
+        assert [torch.equal(p, q) for p, q in zip(got[run], got[2 + run])] == [True] * 4
+    assert lib.saetta_plan_begin() == 0
+    for c in calls:
+        c(None)
+    made = saetta.ffi.ctypes.c_void_p(lib.saetta_plan_end())
+    assert lib.saetta_plan_launches(made) == launches
+    lib.saetta_plan_free(made)
+
+
 def test_rejections():
     z = torch.zeros(4096, device="cuda")
     plan = saetta.Plan()
