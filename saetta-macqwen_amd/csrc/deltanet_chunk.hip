@@ -451,6 +451,12 @@ __global__ __launch_bounds__(256, 2) void deltanet_chunk_prepare_kernel(ChunkArg
     for (int hh = 0; hh < G; hh++) leave(hh, ws_v(hh));
 }
 
+// ds_read_b64_tr_b16 of the 8 bytes at `at` in LDS
+__device__ __forceinline__ half4 read_transposed(const unsigned char *at) {
+    typedef __fp16 fp16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) fp16x4 *)(at)));
+}
+
 // ---- the chain over the blocks --------------------------------------------------------------------
 // Per block, with S0 [dv][128] the state's slice: P = K S0^T and Q S0^T (rows: tokens); R = V - e^c P;
 // U = T R; O = (e^c (Q S0^T) + M U) / sqrt(128); S1 = e^{c_last} S0 + (e^{c_last - c} U)^T K.
@@ -560,7 +566,7 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
     };
 
     // ---- the state's slice: S [dv][128]; wave w of the first team keeps columns 32 w .. + 31: lane (n, j) the four
-    // rows dv = 16 mt + 4j + i of columns 32 w + 16 nt + n.  Its image for the products lies in LDS as hi and lo parts. ----
+    // columns 32 w + 16 nt + 4j + i of row dv = 16 mt + n.  Its image for the products lies in LDS as hi and lo parts. ----
     float *state = a.state + (size_t(h) * a.v_dim + DV * slice) * K_DIM;
     floatx4 s_reg[NT][2];
     auto publish_state = [&]() {
@@ -568,13 +574,15 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
         for (int mt = 0; mt < NT; mt++) {
 #pragma unroll
             for (int nt = 0; nt < 2; nt++) {
+                half4 sh, sl;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     _Float16 hi, lo;
                     split2(s_reg[mt][nt][i], hi, lo);
-                    const int at = (16 * mt + 4 * j + i) * L::SROW + 32 * wave + 16 * nt + n;
-                    img_w(L::SH)[at] = hi, img_w(L::SL)[at] = lo;
+                    sh[i] = hi, sl[i] = lo;
                 }
+                const int at = (16 * mt + n) * L::SROW + 32 * wave + 16 * nt + 4 * j;
+                *reinterpret_cast<half4 *>(img_w(L::SH) + at) = sh, *reinterpret_cast<half4 *>(img_w(L::SL) + at) = sl;
             }
         }
     };
@@ -582,8 +590,7 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
     for (int mt = 0; mt < NT; mt++) {
 #pragma unroll
         for (int nt = 0; nt < 2; nt++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) s_reg[mt][nt][i] = state_team ? state[(16 * mt + 4 * j + i) * K_DIM + 32 * wave + 16 * nt + n] : 0.0f;
+            s_reg[mt][nt] = state_team ? *reinterpret_cast<const floatx4 *>(state + (16 * mt + n) * K_DIM + 32 * wave + 16 * nt + 4 * j) : floatx4{0, 0, 0, 0};
         }
     }
 
@@ -611,7 +618,8 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
         }
         __syncthreads();  // the block's values and factors, the state's image and the keys are in LDS
 
-        // ---- K S0^T (first team) | Q S0^T (second team): rows t = 16 wave + n, columns dv = 16 vt + n' ----
+        // ---- K S0^T (first team): rows t = 16 wave + n, columns dv = 16 vt + n' | (Q S0^T)^T (second team): the other way
+        // round, so that a lane's results are four value dims of a token, one 16-byte store ----
         floatx4 pkq[NT];
 #pragma unroll
         for (int vt = 0; vt < NT; vt++) pkq[vt] = floatx4{0, 0, 0, 0};
@@ -621,16 +629,41 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
             for (int vt = 0; vt < NT; vt++) {
                 const int bo = (16 * vt + n) * L::SROW + 32 * ks + 8 * j;
                 const half8 bh = *reinterpret_cast<const half8 *>(img(L::SH) + bo), bl = *reinterpret_cast<const half8 *>(img(L::SL) + bo);
-                pkq[vt] = mma3(__builtin_bit_cast(half8, cur.kq[0][ks]), __builtin_bit_cast(half8, cur.kq[1][ks]), bh, bl, pkq[vt]);
+                const half8 ah = __builtin_bit_cast(half8, cur.kq[0][ks]), al = __builtin_bit_cast(half8, cur.kq[1][ks]);
+                pkq[vt] = STATE ? mma3(ah, al, bh, bl, pkq[vt]) : mma3(bh, bl, ah, al, pkq[vt]);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
         request_kq(blk + 2, cur);
         __builtin_amdgcn_sched_barrier(0);
-        // C layout: lane (n, j) holds dv = 16 vt + n of tokens t = 16 wave + 4j + i
+        // The left operands of the state's update, K by key dim: lane (n, j) wants key dim 32 wave + 16 nt + n, tokens
+        // 32 ks + 8j .. + 7.  The transposing read works on 16 lanes: lane a + 4e of them names 8 bytes (4 values of a row),
+        // and lane 4a + c receives value c of the lanes a, a + 4, a + 8, a + 12.  So lane a + 4e names token .. + e, key
+        // dims .. + 4a .. + 3, and lane n = 4a + c receives key dim .. + n of four tokens in a row; two reads an operand.
+        // They are asked for here, two barriers before their use, behind the state's image and beside the arithmetic of R.
+        half4 xr[2][2][2][2];  // [hi | lo][nt][k-step][tokens + 0 | + 4]
+        if constexpr (STATE) {
+            const uint32_t la = lane & 3, le = (lane >> 2) & 3;
+            const unsigned char *kbase = lds + L::KIMG + (blk & 1) * 2 * K_IMG;
+#pragma unroll
+            for (int part = 0; part < 2; part++) {
+#pragma unroll
+                for (int nt = 0; nt < 2; nt++) {
+#pragma unroll
+                    for (int ks = 0; ks < 2; ks++) {
+#pragma unroll
+                        for (int hf = 0; hf < 2; hf++) {
+                            xr[part][nt][ks][hf] = read_transposed(kbase + part * K_IMG + ((32 * ks + 8 * j + 4 * hf + le) * KROW + 32 * wave + 16 * nt + 4 * la) * 2);
+                        }
+                    }
+                }
+            }
+        }
+        // C layout: lane (n, j) holds dv = 16 vt + n of tokens t = 16 wave + 4j + i (second team: dv = 16 vt + 4j + i of
+        // token 16 wave + n)
         const floatx4 gam4 = *reinterpret_cast<const floatx4 *>(gam + 16 * wave + 4 * j);
         const floatx4 gk4 = *reinterpret_cast<const floatx4 *>(gam + C + 16 * wave + 4 * j);
-        const float glast = gam[C - 1];
+        const float glast = gam[C - 1], gam_t = gam[16 * wave + n];
         if constexpr (STATE) {
 #pragma unroll
             for (int vt = 0; vt < NT; vt++) {
@@ -680,39 +713,10 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
         __syncthreads();  // U is whole; every wave is through with the state's image, the values and the factors
 
         if constexpr (STATE) {
-            // ---- S1 = e^{c_last} S0 + (U scaled)^T K: rows dv, columns 32 wave + 16 nt + n, over the 64 tokens ----
-            // The B operands, K by key dim: lane (n, j) wants column 32 wave + 16 nt + n, tokens 32 ks + 8j .. + 7.
-            // ds_read_b64_tr_b16 works on 16 lanes: lane a + 4e of them names 8 bytes (4 values of a row), and lane
-            // 4a + c receives value c of the lanes a, a + 4, a + 8, a + 12.  So lane a + 4e names token .. + e, key
-            // dims .. + 4a .. + 3, and lane n = 4a + c receives key dim .. + n of four tokens in a row; two reads an operand.
-            u32x2 xr[2][2][2][2];  // [hi | lo][nt][k-step][tokens + 0 | + 4]
-            {
-                const uint32_t kbase = uint32_t(reinterpret_cast<uintptr_t>(lds)) + L::KIMG + (blk & 1) * 2 * K_IMG;
-                const uint32_t la = lane & 3, le = (lane >> 2) & 3;
-#pragma unroll
-                for (int part = 0; part < 2; part++) {
-#pragma unroll
-                    for (int nt = 0; nt < 2; nt++) {
-#pragma unroll
-                        for (int ks = 0; ks < 2; ks++) {
-#pragma unroll
-                            for (int hf = 0; hf < 2; hf++) {
-                                const uint32_t at = kbase + part * K_IMG + ((32 * ks + 8 * j + 4 * hf + le) * KROW + 32 * wave + 16 * nt + 4 * la) * 2;
-                                asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(xr[part][nt][ks][hf]) : "v"(at) : "memory");
-                            }
-                        }
-                    }
-                }
-                // (the registers are handed on only behind the wait, in the same straight piece of code)
-                asm volatile("s_waitcnt lgkmcnt(0)"
-                             : "+v"(xr[0][0][0][0]), "+v"(xr[0][0][0][1]), "+v"(xr[0][0][1][0]), "+v"(xr[0][0][1][1]), "+v"(xr[0][1][0][0]),
-                               "+v"(xr[0][1][0][1]), "+v"(xr[0][1][1][0]), "+v"(xr[0][1][1][1]), "+v"(xr[1][0][0][0]), "+v"(xr[1][0][0][1]),
-                               "+v"(xr[1][0][1][0]), "+v"(xr[1][0][1][1]), "+v"(xr[1][1][0][0]), "+v"(xr[1][1][0][1]), "+v"(xr[1][1][1][0]),
-                               "+v"(xr[1][1][1][1])::"memory");
-            }
+            // ---- S1 = e^{c_last} S0 + (U scaled)^T K, over the 64 tokens, taken as its transpose: rows are the key dims
+            // 32 wave + 16 nt + .., columns dv, so that a lane's four results are four columns of a row of S in a row ----
             auto x_operand = [&](int part, int nt, int ks) {
-                const u32x4 v = {xr[part][nt][ks][0].x, xr[part][nt][ks][0].y, xr[part][nt][ks][1].x, xr[part][nt][ks][1].y};
-                return __builtin_bit_cast(half8, v);
+                return __builtin_shufflevector(xr[part][nt][ks][0], xr[part][nt][ks][1], 0, 1, 2, 3, 4, 5, 6, 7);
             };
 #pragma unroll
             for (int nt = 0; nt < 2; nt++) {
@@ -724,8 +728,8 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
 #pragma unroll
                     for (int mt = 0; mt < NT; mt++) {
                         const int ao = (16 * mt + n) * TROW + 32 * ks + 8 * j;
-                        acc[mt] = mma3(*reinterpret_cast<const half8 *>(img(L::WH) + ao), *reinterpret_cast<const half8 *>(img(L::WL) + ao),
-                                       x_operand(0, nt, ks), x_operand(1, nt, ks), acc[mt]);
+                        acc[mt] = mma3(x_operand(0, nt, ks), x_operand(1, nt, ks), *reinterpret_cast<const half8 *>(img(L::WH) + ao),
+                                       *reinterpret_cast<const half8 *>(img(L::WL) + ao), acc[mt]);
                     }
                 }
 #pragma unroll
@@ -744,19 +748,20 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
                 for (int ks = 0; ks < 2; ks++) {
                     if (ks > int(wave) / 2) continue;
                     const int bo = (16 * vt + n) * TROW + 32 * ks + 8 * j;
-                    mu[vt] = mma3(__builtin_bit_cast(half8, cur.tm[0][ks]), __builtin_bit_cast(half8, cur.tm[1][ks]),
-                                  *reinterpret_cast<const half8 *>(img(L::UH) + bo), *reinterpret_cast<const half8 *>(img(L::UL) + bo), mu[vt]);
+                    mu[vt] = mma3(*reinterpret_cast<const half8 *>(img(L::UH) + bo), *reinterpret_cast<const half8 *>(img(L::UL) + bo),
+                                  __builtin_bit_cast(half8, cur.tm[0][ks]), __builtin_bit_cast(half8, cur.tm[1][ks]), mu[vt]);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
             request_tm(blk + 2, cur);
             __builtin_amdgcn_sched_barrier(0);
+            const uint32_t tok = blk * C + 16 * wave + n;
+            if (tok < a.tokens) {
+                float *o = a.o + (size_t(tok) * a.v_heads + h) * a.v_dim + DV * slice + 4 * j;
 #pragma unroll
-            for (int vt = 0; vt < NT; vt++) {
+                for (int vt = 0; vt < NT; vt++) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t tok = blk * C + 16 * wave + 4 * j + i;
-                    if (tok < a.tokens) a.o[(size_t(tok) * a.v_heads + h) * a.v_dim + DV * slice + 16 * vt + n] = Q_SCALE * (gam4[i] * pkq[vt][i] + mu[vt][i]);
+                    for (int i = 0; i < 4; i++) o[16 * vt + i] = Q_SCALE * (gam_t * pkq[vt][i] + mu[vt][i]);
                 }
             }
         }
@@ -783,7 +788,9 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
         }
         if (blk < nblocks) step(team, blk, even, odd);
     };
+    // (the first team is the chain: where both teams' waves of a SIMD are ready, its go first)
     if (state_team) {
+        __builtin_amdgcn_s_setprio(2);
         walk(std::true_type{});
     } else {
         walk(std::false_type{});
@@ -793,8 +800,7 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
         for (int mt = 0; mt < NT; mt++) {
 #pragma unroll
             for (int nt = 0; nt < 2; nt++) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) state[(16 * mt + 4 * j + i) * K_DIM + 32 * wave + 16 * nt + n] = s_reg[mt][nt][i];
+                *reinterpret_cast<floatx4 *>(state + (16 * mt + n) * K_DIM + 32 * wave + 16 * nt + 4 * j) = s_reg[mt][nt];
             }
         }
     }
