@@ -48,7 +48,7 @@
 // Kernels (one body, attention_partial_body, behind template switches):
 //   attention_partial_kernel_p   one query row, one workgroup per CU (all registers)
 //   attention_partial_kernel_1   one query row over codes, two workgroups per CU (long 4-bit caches)
-//   attention_partial_kernel_n   2 rows (1 tile), 3-4 rows (2 tiles), 5-8 rows (4 tiles)
+//   attention_partial_kernel_n   2 rows (1 tile), 3-4 rows (2 tiles), 5-6 (3 tiles), 7-8 (4 tiles)
 //   attention_partial_kernel_s   one to four query rows over codes in large caches: four more waves
 //                                move the codes into LDS (global_load_lds), a whole share at once
 //                                with the keys requested first (longer shares: rounds in alternate
@@ -440,7 +440,7 @@ struct Shape {
     static constexpr int SC_STRIDE = IT_TOKENS + 4;  // floats; keeps rows on different LDS banks
     static constexpr bool QUANT = BITS != 16;
     static constexpr int S_ROWS = 16 * TILES;                  // rows of the score buffer
-    static constexpr int SOFT_ROWS = PACKED ? 8 : 16 * TILES;  // rows phase B walks
+    static constexpr int SOFT_ROWS = PACKED ? 8 : TILES == 3 ? 64 : 16 * TILES;  // rows phase B's threads are dealt to (three tiles: a wave has none)
     static constexpr int TPR = THREADS / SOFT_ROWS;            // threads per row in phase B
     static constexpr int TPT = IT_TOKENS / TPR;                // tokens per thread in phase B
     static constexpr int PARTS = PACKED ? 1 : 2;
@@ -743,6 +743,15 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
         for (int e = 0; e < 4; e++) acc[t][e] = floatx4{0, 0, 0, 0};
     }
 
+    // What phase B leaves for phase C: P * P_UP; over halves, where no scale goes into it, its hi and lo parts side by side
+    // (every wave takes all rows' P: split here, once, it is two permutes for two values there).
+    constexpr bool P_SPLIT = BITS == 16 && !PACKED;
+    auto p_word = [&](float x) {
+        if constexpr (!P_SPLIT) return x;
+        _Float16 h, lw;
+        split_hi_lo(x, h, lw);
+        return __builtin_bit_cast(float, uint32_t(__builtin_bit_cast(uint16_t, h)) | uint32_t(__builtin_bit_cast(uint16_t, lw)) << 16);
+    };
     for (uint32_t round = 0; round < n_rounds; round++) {
         const uint32_t it = round;
         const uint32_t blk0 = blk_begin + place(it) * per_it;
@@ -849,7 +858,8 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
         // Writes P * P_UP over the scores; l sums the plain P.
         {
             float sv[Sh::TPT];
-            float *row = s_lds + b_row * SC_STRIDE + b_part * Sh::TPT;
+            const bool scores = Sh::SOFT_ROWS == Sh::S_ROWS || PACKED || b_row < Sh::S_ROWS;  // (three tiles: the last wave has no rows)
+            float *row = s_lds + (scores ? b_row : 0) * SC_STRIDE + b_part * Sh::TPT;
 #pragma unroll
             for (int i = 0; i < Sh::TPT; i += 2) {
                 floatx2 v = *reinterpret_cast<const floatx2 *>(row + i);
@@ -875,11 +885,13 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
             }
             l_part = l_part * al + sum;
             m_run = nm;
+            if (scores) {
 #pragma unroll
-            for (int i = 0; i < Sh::TPT; i += 2) {
-                *reinterpret_cast<floatx2 *>(row + i) = floatx2{sv[i] * P_UP, sv[i + 1] * P_UP};
+                for (int i = 0; i < Sh::TPT; i += 2) {
+                    *reinterpret_cast<floatx2 *>(row + i) = floatx2{p_word(sv[i] * P_UP), p_word(sv[i + 1] * P_UP)};
+                }
+                if (b_part == 0) alpha_lds[b_row] = al;
             }
-            if (b_part == 0) alpha_lds[b_row] = al;
         }
         __syncthreads();
 
@@ -917,6 +929,14 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
                     o[e / 2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
                 }
                 phi = as_half8(o[0], o[1], o[2], o[3]);
+            } else if constexpr (P_SPLIT) {
+                uint32_t h[4], lw[4];
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {
+                    const uint32_t w0 = __builtin_bit_cast(uint32_t, pv[e]), w1 = __builtin_bit_cast(uint32_t, pv[e + 1]);
+                    h[e / 2] = perm(w1, w0, 0x05040100u), lw[e / 2] = perm(w1, w0, 0x07060302u);
+                }
+                phi = as_half8(h[0], h[1], h[2], h[3]), plo = as_half8(lw[0], lw[1], lw[2], lw[3]);
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
@@ -962,25 +982,30 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
                         }
                     }
                 }
-            } else {
+            }
+        }
+        if constexpr (!PACKED) {
+            // (the k-steps outside: a step's value operands are permuted once for all tiles)
 #pragma unroll
-                for (int ks = 0; ks < KSTEPS; ks++) {
-                    if (uint32_t(ks) >= ksteps) break;
+            for (int ks = 0; ks < KSTEPS; ks++) {
+                if (uint32_t(ks) >= ksteps) break;
+                if constexpr (BITS == 16) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        if (base + 32 * ks + 8 * j + e >= max_len) vreg[ks].w[e] = 0, vreg[ks].w[8 + e] = 0;
+                    }
+                }
+                half8 vop[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) vop[e] = val_operand<BITS>(vreg[ks], e, n);
+#pragma unroll
+                for (int t = 0; t < TILES; t++) {
                     half8 phi, plo;
                     build_p(t, ks, phi, plo);
-                    if constexpr (BITS == 16) {
-                        if (t == 0) {
-#pragma unroll
-                            for (int e = 0; e < 8; e++) {
-                                if (base + 32 * ks + 8 * j + e >= max_len) vreg[ks].w[e] = 0, vreg[ks].w[8 + e] = 0;
-                            }
-                        }
-                    }
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        const half8 vop = val_operand<BITS>(vreg[ks], e, n);
-                        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(phi, vop, acc[t][e], 0, 0, 0);
-                        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(plo, vop, acc[t][e], 0, 0, 0);
+                        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(phi, vop[e], acc[t][e], 0, 0, 0);
+                        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(plo, vop[e], acc[t][e], 0, 0, 0);
                     }
                 }
             }
@@ -1034,7 +1059,7 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
             // (Five to eight rows past the caches: up to 17 MB that the L2s would hold dirty until the kernel's end, 27.0 against
             // 27.7 us a layer for 8 rows at 7000 tokens.  Fewer rows are read back sooner than they are written out: plain.)
             auto put = [&](float *to, auto value) {
-                if constexpr (TILES == 4) __builtin_nontemporal_store(value, reinterpret_cast<decltype(value) *>(to));
+                if constexpr (TILES >= 3) __builtin_nontemporal_store(value, reinterpret_cast<decltype(value) *>(to));
                 else *reinterpret_cast<decltype(value) *>(to) = value;
             };
             if constexpr (BITS == 16) {
@@ -2925,6 +2950,8 @@ void launch_partial_rows(hipStream_t stream, const PartialArgs &a, bool one_per_
         launch_partial<BITS, 1, false>(stream, a, one_per_cu, keys_first, token);
     } else if (a.rows <= 4) {
         launch_partial<BITS, 2, false>(stream, a, one_per_cu, keys_first, token);
+    } else if (a.rows <= 6) {
+        launch_partial<BITS, 3, false>(stream, a, one_per_cu, keys_first, token);
     } else {
         launch_partial<BITS, 4, false>(stream, a, one_per_cu, keys_first, token);
     }
@@ -3058,6 +3085,7 @@ int raise_lds_of_bits() {
     if (int rc = raise_lds<BITS, 2, false, itb_rows<2>()>(attention_token_kernel_n<BITS, 2>)) return rc;
     if (int rc = raise_lds<BITS, 1, false, itb_rows<1>()>(attention_partial_kernel_n<BITS, 1>)) return rc;
     if (int rc = raise_lds<BITS, 2, false, itb_rows<2>()>(attention_partial_kernel_n<BITS, 2>)) return rc;
+    if (int rc = raise_lds<BITS, 3, false, itb_rows<3>()>(attention_partial_kernel_n<BITS, 3>)) return rc;
     return raise_lds<BITS, 4, false, itb_rows<4>()>(attention_partial_kernel_n<BITS, 4>);
 }
 }  // namespace
