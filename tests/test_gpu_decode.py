@@ -324,6 +324,35 @@ def test_several_rows_in_caches_of_65536_and_131072_tokens(kind, m):
             del kc, vc
 
 
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("m", [5, 6, 7, 8])
+def test_three_and_four_tiles_of_query_rows_at_the_edges_of_a_step(kind, m):
+    # One split, so that a workgroup's iterations are what the context makes them: one block and a few tokens (a k-step
+    # half filled), two, just past two, 12 blocks (one whole iteration) and one token more, several iterations with a
+    # short one last.  Five and seven rows leave half of the last tile of query rows empty.  The rows past the context
+    # are poisoned, and in the last iteration no step past its blocks is read.
+    rng = np.random.default_rng(5200 + m)
+    capacity = 640
+    k = rng.standard_normal((capacity, VALUES)).astype(np.float32)
+    v = rng.standard_normal((capacity, VALUES)).astype(np.float32)
+    q = rng.standard_normal((m, H, D)).astype(np.float32)
+    qg = rng.standard_normal((m, H, 2 * D)).astype(np.float32)
+    rows = saetta.AttentionRows(H, KV, capacity, m)
+    rows.splits = 1
+    for tokens in [m, 16, 21, 32, 33, 192, 193, 250, 400, 625]:
+        pos = tokens - m
+        kc, vc, kf, vf = cache_pair(k[:tokens], v[:tokens], kind, capacity, poison=True)
+        out = torch.full((m, H, D), float("nan"), device="cuda")
+        plan = saetta.Plan()
+        params = [saetta.TokenParams(0, pos + r).as_tensor("cuda") for r in range(m)]
+        (rows.record if kind is saetta.KvBits.Half else rows.record_quant)(plan, m, dev(q), kc, vc, dev(qg), out, params)
+        plan.build().run()
+        got = host(out)
+        assert np.isfinite(got).all(), tokens
+        worst = np.abs(got - oracle.rows(q, kf, vf, pos, m, q_and_gate=qg, threads=8, f64=True)).max()
+        assert worst < MAX_ABS_F64, (tokens, worst)
+
+
 @pytest.mark.parametrize("splits", [100, 64, 7])
 def test_several_rows_with_fewer_splits(splits):
     # RowsAttentionParams.splits is an upper bound the caller may lower (src/rows.rs:344-367).  In a
