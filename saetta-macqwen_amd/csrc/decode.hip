@@ -225,13 +225,14 @@ __device__ __forceinline__ half8 val_operand(const ValRegs<BITS> &r, int tile, i
 #pragma unroll
         for (int i = 0; i < 4; i++) o[i] = perm(r.w[2 * i + 1], r.w[2 * i], sel);
     } else if constexpr (BITS == 4) {
-        const uint32_t byte = uint32_t(tile >> 1);
-        const uint32_t sel = 0x0c000c00u | ((4 + byte) << 16) | byte;
-        const uint32_t sh = (n & 1) * 16, up = (tile & 1) ? 0 : 4;
+        // the byte first, by a selector of the lane's own that every word shares, then its nibble: two tiles take the same
+        // byte, so four instructions make two words of operands (nine with the nibbles cut out of each token's word)
+        const uint32_t byte = uint32_t(n & 1) * 2 + uint32_t(tile >> 1);
+        const uint32_t sel = 0x0c040c00u + byte * 0x00010001u;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const uint32_t a = ((r.w[2 * i] >> sh) << up) & 0xf0f0u, b = ((r.w[2 * i + 1] >> sh) << up) & 0xf0f0u;
-            o[i] = perm(b, a, sel);
+            const uint32_t w = perm(r.w[2 * i + 1], r.w[2 * i], sel);
+            o[i] = (tile & 1 ? w : w << 4) & 0x00f000f0u;
         }
     } else {
         const int set = tile >> 1;
