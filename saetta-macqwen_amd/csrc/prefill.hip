@@ -72,6 +72,8 @@ constexpr int BK = 32;                  // keys per block
 constexpr int PART_BYTES = BK * DIM * 2;
 constexpr int IMG_BYTES = 2 * PART_BYTES;
 constexpr float NO_SCORE = -1e30f;
+// (EXACT: not in the first EXACT_BLOCKS blocks of a row's keys, see prefill_tile)
+constexpr uint32_t EXACT_BLOCKS = 8;
 constexpr float TAU = 8.0f;  // the reference max is raised only past this many powers of two
 
 struct PrepareArgs {
@@ -93,7 +95,7 @@ struct PrefillArgs {
     float scale;
     uint32_t nblocks;  // images per kv head
     uint32_t *tiles_taken;  // tiles handed out past every workgroup's first (zero at the start: the prepare kernel's doing)
-    // Split keys (attention_prefill_kernel<true>): a tile's keys are taken in parts of `part_blocks` blocks, each of which
+    // Split keys (attention_prefill_kernel<true, ..>): a tile's keys are taken in parts of `part_blocks` blocks, each of which
     // leaves its unnormalised O and (m, l) in the workspace for prefill_merge_kernel.
     uint32_t part_blocks;
     float *part_o;   // [part][tile][kv head][8 waves][16][64 lanes][4]: the accumulators as they are
@@ -336,7 +338,12 @@ __device__ __host__ __forceinline__ uint32_t tile_blocks(uint32_t pos, uint32_t 
 }
 
 // One tile of TQ tokens x 8 heads of kv head `kv` against the keys it sees, or (SPLIT) against part `part` of them.
-template <bool SPLIT>
+// EXACT: in the first EXACT_BLOCKS blocks the reference maximum is the maximum itself, so that a row's largest probability
+// there is 1, which f16 holds exactly; relative to a maximum up to 2^TAU below it is rounded like the others, which shows
+// in rows of few keys.  For AttGemm, whose passes took every tile's probabilities relative to the tile's own maximum
+// (largest error over the output's r.m.s., 1712 tokens at 37: passes 0.8e-2 to 1.3e-2, without EXACT 1.5e-2, with 0.6e-2; 1 us
+// a tile).
+template <bool SPLIT, bool EXACT>
 __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char *tiles, uint32_t tile, uint32_t kv, uint32_t part_index, bool ask, uint32_t *next_tile) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -438,9 +445,10 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
         return fmaxf(bm * c, NO_SCORE);
     };
     // Raises the reference maximum when a block tops it by more than 2^TAU, rescaling O and l.
-    auto raise_max = [&](float bm) {
-        if (__any(bm > m_ref + TAU)) {
-            const float m_new = bm > m_ref + TAU ? bm : m_ref;
+    auto raise_max = [&](float bm, uint32_t kb) {
+        const float slack = EXACT && block0 + kb < EXACT_BLOCKS ? 0.0f : TAU;
+        if (__any(bm > m_ref + slack)) {
+            const float m_new = bm > m_ref + slack ? bm : m_ref;
             const float alpha = __builtin_amdgcn_exp2f(m_ref - m_new);
             m_ref = m_new;
             l_sum *= alpha;
@@ -489,7 +497,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
             const Copy cp = copy_of(step);
             const uint32_t kb = 2 * step;
             if (kb < wave_blocks) {
-                raise_max(mask_max(s, kb * BK, kb >= full_blocks));
+                raise_max(mask_max(s, kb * BK, kb >= full_blocks), kb);
                 half8 pb[2];
                 exp_pack(s, pb);
                 // (past the wave's last block the scores are of stale keys and never looked at)
@@ -505,7 +513,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
         if (1 < wave_blocks) {
             floatx16 s;
             scores_block(s, qb, lds0 + k_slot(1) + lane16);
-            raise_max(mask_max(s, BK, 1 >= full_blocks));
+            raise_max(mask_max(s, BK, 1 >= full_blocks), 1);
             exp_pack(s, pb);
         }
         __syncthreads();
@@ -520,7 +528,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
                 stream_block(s, acc, qb, pb, lds0 + k_slot(kb + 2) + lane16, lds0 + v_slot(kb) + lane16, cp, lane16);
                 __builtin_amdgcn_s_setprio(0);
                 if (kb + 2 < wave_blocks) {
-                    raise_max(mask_max(s, (kb + 2) * BK, kb + 2 >= full_blocks));
+                    raise_max(mask_max(s, (kb + 2) * BK, kb + 2 >= full_blocks), kb + 2);
                     exp_pack(s, pb);
                 }
             } else {
@@ -658,7 +666,7 @@ __device__ __host__ __forceinline__ uint32_t prefill_items(uint32_t pos, uint32_
 // longest with the shortest, ended 40 us apart: the workgroups' rates differ by a tenth).
 // SPLIT: an item is a part of a tile's keys, parts side by side in tiles and kv heads (workgroups that run together walk
 // the same keys); the tiles that have a part p are the ones from prefill_first_tile(p) on.
-template <bool SPLIT>
+template <bool SPLIT, bool EXACT>
 __global__ __launch_bounds__(THREADS, 2) void attention_prefill_kernel(PrefillArgs a) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char tiles[];
     __shared__ uint32_t next_tile;
@@ -672,7 +680,7 @@ __global__ __launch_bounds__(THREADS, 2) void attention_prefill_kernel(PrefillAr
         if constexpr (SPLIT) {
             for (uint32_t n; at >= (n = ntiles - prefill_first_tile(a.pos, a.tokens, a.part_blocks, part)); part++) at -= n;
         }
-        prefill_tile<SPLIT>(a, tiles, ntiles - 1 - at, idx % a.kv_heads, part, idx + G < total, &next_tile);
+        prefill_tile<SPLIT, EXACT>(a, tiles, ntiles - 1 - at, idx % a.kv_heads, part, idx + G < total, &next_tile);
         lds_barrier();  // the next tile is known; this tile's merge has been read: the next tile's keys may land on it (its stores go on meanwhile)
         idx = next_tile;
     }
@@ -1248,7 +1256,7 @@ int launch_small(hipStream_t stream, int bits, const uint16_t *q, const void *kd
 // The launches of a chunk in a workspace of at least plan.plain bytes, plan.bytes() with `split`.
 int launch_flash(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
                  const uint16_t *kz, const uint16_t *vs, const uint16_t *vz, const float *q_and_gate, float *out,
-                 const saetta_flash_params &p, void *workspace, bool split, const FlashPlan &plan, const char *what) {
+                 const saetta_flash_params &p, void *workspace, bool split, bool exact, const FlashPlan &plan, const char *what) {
     const uint64_t rows = uint64_t(p.pos) + p.tokens;
     unsigned char *ws = static_cast<unsigned char *>(workspace);
     uint32_t *tiles_taken = reinterpret_cast<uint32_t *>(ws + images_bytes(p.pos, p.tokens, p.kv_heads));
@@ -1261,11 +1269,11 @@ int launch_flash(hipStream_t stream, int bits, const uint16_t *q, const void *kd
         a.part_o = reinterpret_cast<float *>(ws + plan.plain);
         a.part_ml = reinterpret_cast<float *>(ws + plan.plain + size_t(plan.nparts) * ntiles * p.kv_heads * PART_O_BYTES);
         const uint32_t total = prefill_items(p.pos, p.tokens, plan.part_blocks) * p.kv_heads;
-        launch(attention_prefill_kernel<true>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
+        launch(exact ? attention_prefill_kernel<true, true> : attention_prefill_kernel<true, false>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
         launch(prefill_merge_kernel, dim3(p.tokens, p.kv_heads), MERGE_THREADS, 0, stream, a);
     } else {
         const uint32_t total = ntiles * p.kv_heads;
-        launch(attention_prefill_kernel<false>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
+        launch(exact ? attention_prefill_kernel<false, true> : attention_prefill_kernel<false, false>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
     }
     return launch_status(what);
 }
@@ -1288,7 +1296,7 @@ int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kda
     if (workspace && workspace_size < need) need = plan.plain;  // (room for the images only: the keys are not split)
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
     if (int rc = acquire_workspace(stream, workspace, workspace_size, need, owned_lock, what, "saetta_prefill_workspace_bytes")) return rc;
-    return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, need >= plan.bytes(), plan, what);
+    return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, need >= plan.bytes(), false, plan, what);
 }
 
 // ---- the same chunk as matrix products over blocks of 1024 keys ---------------------------------
@@ -1656,7 +1664,7 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
     if (stages == 0) {
         const FlashPlan plan = flash_plan(p.pos, p.tokens, p.kv_heads, bits);
         if (plan.small) return launch_small(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, what);
-        return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, true, plan, what);
+        return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, true, true, plan, what);
     }
     const uint32_t nblocks = launch_prepare(stream, bits, kdata, vdata, ks, kz, vs, vz, workspace, p.kv_heads, rows);
 
@@ -1701,17 +1709,17 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
 }  // namespace
 
 int setup_prefill() {
-    if (int rc = load_kernel(reinterpret_cast<const void *>(attention_prefill_kernel<false>))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(prefill_merge_kernel))) return rc;
     if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<16>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<16>::BYTES))) return rc;
     if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<8>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<8>::BYTES))) return rc;
     if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<4>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<4>::BYTES))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_scores_kernel))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_pv_kernel))) return rc;
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_prefill_kernel<true>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES))) return rc;
-    return int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_prefill_kernel<false>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
+    for (const void *kernel : {reinterpret_cast<const void *>(attention_prefill_kernel<true, false>), reinterpret_cast<const void *>(attention_prefill_kernel<true, true>),
+                               reinterpret_cast<const void *>(attention_prefill_kernel<false, false>), reinterpret_cast<const void *>(attention_prefill_kernel<false, true>)}) {
+        if (int rc = int(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES))) return rc;
+    }
+    return 0;
 }
 }  // namespace saetta
 

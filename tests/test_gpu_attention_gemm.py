@@ -241,6 +241,22 @@ def test_other_head_counts_both_routes(kv_heads):
         assert np.abs(got - want).max() < MAX_ABS and oracle.rel_rms(got, want) < REL_RMS
 
 
+@pytest.mark.parametrize("pos,tokens", [(90, 1100), (200, 777)])  # whole tiles; their keys in parts
+def test_a_key_that_stands_out_early_is_not_rounded(pos, tokens):
+    # All scores are 0 but that of key 70, in the third block of keys, 8 x 0.4 above: its probability relative to the
+    # maximum before it, 24.51, is not an f16 number (1e-4 off), relative to its own score it is 1.  Only its value is not
+    # 0, so the output is w / (n - 1 + w) / 2 to f32's accuracy (sums of up to 1200 terms: 1e-5).
+    n = pos + tokens
+    q = torch.full((tokens, H, D), 0.5, dtype=torch.float16, device="cuda")
+    k, v = (torch.zeros(n * VALUES, dtype=torch.float16, device="cuda") for _ in range(2))
+    k[70 * VALUES:71 * VALUES] = 0.4
+    v[70 * VALUES:71 * VALUES] = 1.0
+    got = run(saetta.KvBits.Half, q, k, v, torch.zeros(tokens, H, 2 * D, device="cuda"), pos, tokens).astype(np.float64)
+    w = math.exp(D * 0.5 * float(np.float16(0.4)) / math.sqrt(D))
+    want = 0.5 * w / (pos + 1 + np.arange(tokens) - 1 + w)
+    assert np.abs(got / want[:, None, None] - 1).max() < 1e-5
+
+
 def test_bench_mirrors_the_reference():
     # bench (src/attention_gemm.rs:366-470) at a small shape: both kernels timed at the last and the middle
     # chunk, the passes one by one, and the two outputs compared as the reference prints them.
