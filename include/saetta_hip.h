@@ -194,7 +194,9 @@ int saetta_token_params_set(saetta_stream_t stream, saetta_token_params *d_tp, s
  * them (the stream it is given is not used).  saetta_plan_run makes them on a stream, one after the
  * other, with one call and no further checks: 2 us of host time per launch.  Buffers named in the
  * plan must outlive it.  A plan runs on the device it was recorded on (that device current), from
- * any thread, also on several at once; under stream capture it becomes part of the graph.  begin
+ * any thread, also on several at once; under stream capture it becomes part of the graph.  Launches
+ * recorded one after the other over the same buffers may become one: a token's store, partial and
+ * reduce stage, a DeltaNet conv and the chunk it feeds; what they write is the same.  begin
  * fails while the thread is recording, end returns NULL when it is not. */
 typedef struct saetta_plan saetta_plan;
 int saetta_plan_begin(void);
