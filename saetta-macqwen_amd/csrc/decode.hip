@@ -1218,7 +1218,10 @@ struct KeysFirst {
     // LDS for every pair's query operands to stay ([pair][hi, lo][k-step][lane] half8, then [pair][hi, lo][lane][k-step]
     // f16 of the key bias term), so that they need no registers between one round's scores and the next's.
     // 8-bit codes: over the keys' blocks that short rounds never fill; 4-bit: behind the values.
-    static constexpr int SHORT_BLOCKS = 8;
+    // (4-bit, two pairs: rounds of 12, for which there is room.  A round costs 2.6 us beside its bytes, and with the new
+    // tokens' split taken out of the context's 128 a share of 32 blocks is one of 33, a fifth round of 8: four rows at 65500
+    // tokens 42.3 -> 38.5 us a layer, 120000 60.7 -> 56.0, 262000 114.6 -> 105.5.)
+    static constexpr int SHORT_BLOCKS = BITS == 4 && PAIRS == 2 ? 12 : 8;
     static constexpr int QP_PAIR_BYTES = 2 * 8 * 64 * 16, QPZ_PAIR_BYTES = 2 * 64 * 16;
     static constexpr int QP_BYTES = M > 1 ? PAIRS * (QP_PAIR_BYTES + QPZ_PAIR_BYTES) : 0;
     static constexpr int QP_OFF = BITS == 8 ? K_OFF + SHORT_BLOCKS * K_BLOCK_BYTES : V_OFF + AREA_BLOCKS * K_BLOCK_BYTES;
@@ -1696,7 +1699,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
         auto row_of = [&](int pair, int half) { return min(2 * pair + half, M - 1); };
         if (range > uint32_t(RBK)) {
             // ---- a share of more than one round (a context of more than 17 blocks per split) ----------
-            // Rounds of up to SHORT_BLOCKS blocks, in the blocks 0-7 of the keys' and the values' places.  What
+            // Rounds of up to SHORT_BLOCKS blocks, in the first blocks of the keys' and the values' places.  What
             // a round leaves behind, per column: the maximum so far, the sums so far relative to it (O in
             // registers, l with wave 0), both brought to the new maximum before the next round's values are
             // added.  The query operands of every pair wait in LDS (the blocks that short rounds never fill) and
