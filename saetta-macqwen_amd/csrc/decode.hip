@@ -1218,15 +1218,18 @@ struct KeysFirst {
     // LDS for every pair's query operands to stay ([pair][hi, lo][k-step][lane] half8, then [pair][hi, lo][lane][k-step]
     // f16 of the key bias term), so that they need no registers between one round's scores and the next's.
     // 8-bit codes: over the keys' blocks that short rounds never fill; 4-bit: behind the values.
-    // (4-bit, two pairs: rounds of 12, for which there is room.  A round costs 2.6 us beside its bytes, and with the new
+    // (Two pairs: rounds of 12, for which there is room.  A round costs 2.6 us beside its bytes, and with the new
     // tokens' split taken out of the context's 128 a share of 32 blocks is one of 33, a fifth round of 8: four rows at 65500
-    // tokens 42.3 -> 38.5 us a layer, 120000 60.7 -> 56.0, 262000 114.6 -> 105.5.)
-    static constexpr int SHORT_BLOCKS = BITS == 4 && PAIRS == 2 ? 12 : 8;
+    // tokens, 4-bit, 42.3 -> 38.5 us a layer, 120000 60.7 -> 56.0, 262000 114.6 -> 105.5; 8-bit 42.0 -> 37.7, 57.6 -> 54.5,
+    // 109.3 -> 99.4; behind at some lengths between: 80000 43.9 -> 44.9.)
+    static constexpr int SHORT_BLOCKS = PAIRS == 2 ? 12 : 8;
     static constexpr int QP_PAIR_BYTES = 2 * 8 * 64 * 16, QPZ_PAIR_BYTES = 2 * 64 * 16;
     static constexpr int QP_BYTES = M > 1 ? PAIRS * (QP_PAIR_BYTES + QPZ_PAIR_BYTES) : 0;
     static constexpr int QP_OFF = BITS == 8 ? K_OFF + SHORT_BLOCKS * K_BLOCK_BYTES : V_OFF + AREA_BLOCKS * K_BLOCK_BYTES;
     static constexpr int QPZ_OFF = QP_OFF + PAIRS * QP_PAIR_BYTES;
-    static_assert(BITS != 8 || QP_OFF + QP_BYTES <= V_OFF, "the query operands fit behind the short rounds' keys");
+    // (8-bit, two pairs: they reach into the values' places, whose last SHORT_BLOCKS blocks the short rounds fill then)
+    static constexpr int V_SHORT = BITS == 8 && PAIRS == 2 ? (AREA_BLOCKS - SHORT_BLOCKS) * K_BLOCK_BYTES : 0;
+    static_assert(BITS != 8 || M == 1 || QP_OFF + QP_BYTES <= V_OFF + V_SHORT, "the query operands fit between the short rounds' keys and values");
     static constexpr int LDS_BYTES = (BITS == 8 || M == 1) ? V_OFF + AREA_BLOCKS * K_BLOCK_BYTES : QP_OFF + QP_BYTES;
     // one row: the merge of two waves, [group][lane < 32][4 rows] of 16 bytes, lies over the query operands,
     // which nobody reads after the last scores
@@ -1340,6 +1343,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
     const uint32_t n_rounds = range > uint32_t(RBK) ? (range + LONG_ROUND - 1) / LONG_ROUND : 1;
     const bool alt = W::ALTERNATE && n_rounds > 1;  // rounds in alternate halves of LDS
     const uint32_t per_round = (range + n_rounds - 1) / n_rounds;
+    const uint32_t v_off = W::V_OFF + (M > 1 && n_rounds > 1 ? uint32_t(W::V_SHORT) : 0u);  // where the rounds' values lie
     auto blocks_of = [&](uint32_t round) { return min(range - round * per_round, per_round); };
     // The rounds in the order in which the splits take them: four in a row start a quarter of the share apart.  Started all at
     // the front they read addresses one share apart at every moment, and shares of nearly a power of two then meet in the
@@ -1549,7 +1553,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
                     // of the row, which is rotated by (token / 8) % 4 quarters: the same for the group's tokens)
                     const uint32_t t = BLOCK * blk + W::V_GROUP_TOKENS * i + lane / W::PIECES;  // token of the round
                     const uint32_t piece = (lane % W::PIECES + W::PIECES - ((t >> 3) & 3) * (W::PIECES / 4)) % W::PIECES;
-                    dma(lds0 + W::V_OFF + (W::PER_BLOCK * blk + i) * 1024, (min(base + t, last_tok) * kvh + kv) * RB + piece * 16, a.vdata);
+                    dma(lds0 + v_off + (W::PER_BLOCK * blk + i) * 1024, (min(base + t, last_tok) * kvh + kv) * RB + piece * 16, a.vdata);
                 }
             };
 #pragma unroll
@@ -1639,7 +1643,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
     auto read_values = [&](int ks, int g, ValRegs<BITS> &vreg) {
         const int jj = ks == 8 ? (j & 1) : j;
         // (tokens 8 jj .. 8 jj + 7 of a k-step: their rows are rotated by jj quarters)
-        const unsigned char *vb = lds_raw + W::V_OFF + 8 * jj * RB + ((val_lane_offset<BITS>(g, n) + jj * W::V_ROT) & (RB - 1));
+        const unsigned char *vb = lds_raw + v_off + 8 * jj * RB + ((val_lane_offset<BITS>(g, n) + jj * W::V_ROT) & (RB - 1));
 #pragma unroll
         for (int e = 0; e < 8; e++) vreg.w[e] = *reinterpret_cast<const uint32_t *>(vb + (32 * ks + e) * RB);
     };
