@@ -105,6 +105,17 @@ inline void tag_launch(uint32_t kind, uint32_t bits, uint32_t rows) {
 
 inline bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
+// Memory that a launch reads or writes.  Launches may become one only where what the one reads and writes lies apart: in
+// order of launches a program may lay a buffer over another that is done with, inside one launch nothing is done with.
+struct Span {
+    const void *start;
+    size_t bytes;
+};
+inline bool apart(const Span &p, const Span &q) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(p.start), b = reinterpret_cast<uintptr_t>(q.start);
+    return a + p.bytes <= b || b + q.bytes <= a;
+}
+
 }  // namespace saetta
 
 #define SAETTA_REQUIRE(cond, code, ...)                       \

@@ -266,8 +266,8 @@ __device__ __forceinline__ float half_bits_to_float(uint32_t bits16) {
 //  * every workgroup of the context norms and rotates the query rows it needs itself, under the first loads of the cache;
 //    its context are the tokens BEFORE the new ones;
 //  * workgroups of their own (behind the context's) make the new keys and values, store them and the query rows, and
-//    write the new tokens' own partial result (the last split), from the values just as the cache holds them, so nobody
-//    in the launch reads what another workgroup of it writes.
+//    write the new tokens' own partial result (the last split), from the values just as the cache holds them.  Nobody in
+//    the launch reads what another workgroup of it writes, as long as the step's buffers lie apart (token_step looks).
 // The keys', values' and codes' bits are those of attention_prep_store_kernel (the same operations in the same order).
 // A workgroup of the new rows takes some rows and some heads of them, and makes the keys and values of all rows up to
 // those for itself.  The loader kernels have 12 waves: one workgroup does it all.  The register kernels have 4, so that a
@@ -2999,6 +2999,14 @@ bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const fl
                                         prep.vq.scales == a.vscales && prep.vq.biases == a.vbiases;
     if (!(cache && prep.q_out == a.q && prep.q_and_gate == q_and_gate && prep.tp == a.tp && prep.capacity == a.capacity && prep.p.heads == a.heads &&
           prep.p.kv_heads == a.kv_heads && prep.p.half_dims == 32 && aligned(prep.q_and_gate, 16) && aligned(prep.q_norm, 16))) return false;
+    // Workgroups that make the same key read it while one of them writes it back: `k_back` in the place of `k` (the
+    // reference's in-place key), or of any other input of the step, keeps the launches.
+    const size_t row_kv = size_t(a.rows) * a.kv_heads * DIM * sizeof(float), norm = DIM * sizeof(float);
+    const Span inputs[] = {{prep.q_and_gate, size_t(a.rows) * a.heads * 2 * DIM * sizeof(float)}, {prep.k, row_kv}, {prep.v, row_kv},
+                           {prep.q_norm, norm}, {prep.k_norm, norm}, {a.tp, sizeof(saetta_token_params)}};
+    for (const Span &i : inputs) {
+        if (prep.k_back && !apart({prep.k_back, row_kv}, i)) return false;
+    }
     token = TokenArgs{a, prep, SAETTA_GQA_GROUP};
     if (!keys_first) {
         // more rows than four: the workgroups of the new rows need longer than the launch takes (18.7 against 18.2 us per

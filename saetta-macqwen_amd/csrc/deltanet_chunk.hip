@@ -837,14 +837,10 @@ bool take_conv(LaunchList &list, ChunkArgs &args, float *&conv_out) {
     const saetta_conv_rows_params &c = list.arg<saetta_conv_rows_params>(conv, 5);
     if (c.kernel_size != CONV || c.snapshots || c.channels != args.channels || c.tokens != args.tokens || out != args.mixed) return false;
     const size_t rows = size_t(args.tokens) * args.channels * sizeof(float), gates = size_t(args.tokens) * args.v_heads * sizeof(float);
-    const std::pair<const void *, size_t> inputs[] = {{x, rows}, {w, size_t(CONV) * args.channels * sizeof(float)}, {args.a, gates}, {args.b, gates},
+    const Span inputs[] = {{x, rows}, {w, size_t(CONV) * args.channels * sizeof(float)}, {args.a, gates}, {args.b, gates},
                                                       {args.a_log, args.v_heads * sizeof(float)}, {args.dt_bias, args.v_heads * sizeof(float)}},
         outputs[] = {{out, rows}, {conv_state, size_t(CONV - 1) * args.channels * sizeof(float)},
                      {args.ws, size_t((args.tokens + C - 1) / C) * block_bytes(args.k_heads, args.v_heads)}};
-    const auto apart = [](const std::pair<const void *, size_t> &p, const std::pair<const void *, size_t> &q) {
-        const uintptr_t a = reinterpret_cast<uintptr_t>(p.first), b = reinterpret_cast<uintptr_t>(q.first);
-        return a + p.second <= b || b + q.second <= a;
-    };
     for (const auto &o : outputs) {
         for (const auto &i : inputs) {
             if (!apart(o, i)) return false;

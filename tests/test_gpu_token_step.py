@@ -14,7 +14,7 @@ PREP = saetta.PrepParams(H, KV, D, 64, 1e7, 1e-6)
 
 
 class Step:
-    def __init__(self, kind, capacity, rows, seed, rope_dims=64):
+    def __init__(self, kind, capacity, rows, seed, rope_dims=64, lay=lambda step: None):
         rng = np.random.default_rng(seed)
         self.rows, self.kind = rows, kind
         self.qg = dev(rng.standard_normal((rows, H, 2 * D)).astype(np.float32))
@@ -29,6 +29,8 @@ class Step:
                 c.encode(x, 0, self.cache.capacity)
         keys, values = self.cache.quant or (self.cache.keys, self.cache.values)
         self.q, self.out, self.back = (torch.zeros(rows, n, device="cuda") for n in (H * D, H * D, VALUES))
+        self.k0, self.v0 = self.k.clone(), self.v.clone()
+        lay(self)  # (buffers over others)
         self.plan = saetta.Plan()
         saetta.record_store(self.plan, self.qg, self.k, self.v, qn, kn, self.q, keys, values, saetta.PrepParams(H, KV, D, rope_dims, 1e7, 1e-6),
                             self.cache.capacity, rows=rows, k_back=self.back)
@@ -43,6 +45,7 @@ class Step:
     def run(self, how, position):
         self.plan.set_params(saetta.TokenParams(0, position))
         self.q.fill_(float("nan")), self.out.fill_(float("nan")), self.back.fill_(float("nan"))
+        self.k.copy_(self.k0), self.v.copy_(self.v0)
         how()
         return [host(t).copy() for t in (self.out, self.q, self.back)] + [host(b).copy() for b in self.cache.buffers()]
 
@@ -76,6 +79,31 @@ def test_fused_step_equals_the_ops_one_by_one(kind, capacity, rows):
         assert np.array_equal(got[2], want[2]), position
         for a, b in zip(got[3:], before):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), position
+
+
+def check_laid_over(step, positions):
+    """A step with buffers over each other keeps its launches; outputs as the ops one by one, what is stored bit for bit."""
+    assert launches(step) == 3
+    built = step.plan.build()
+    for position in positions:
+        want, got = step.run(step.plan.run_serial, position), step.run(built.run, position)
+        assert np.isfinite(got[0]).all()
+        for a, b in zip(got, want):
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), position
+
+
+def key_in_place(step):
+    step.back = step.k
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 4])
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("capacity", [512, 8192, 40960])
+def test_a_key_written_back_in_place(kind, capacity, rows):
+    # Several workgroups make a new key; were one to write it back over what the others read, they would take a key
+    # that is normed and rotated already.
+    step = Step(kind, capacity, rows, seed=capacity + 7 * rows + kind.value, lay=key_in_place)
+    check_laid_over(step, (100, step.cache.capacity - rows))
 
 
 def test_other_steps_keep_their_launches():
