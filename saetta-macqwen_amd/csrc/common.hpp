@@ -113,7 +113,7 @@ struct Span {
 };
 inline bool apart(const Span &p, const Span &q) {
     const uintptr_t a = reinterpret_cast<uintptr_t>(p.start), b = reinterpret_cast<uintptr_t>(q.start);
-    return a + p.bytes <= b || b + q.bytes <= a;
+    return p.bytes == 0 || q.bytes == 0 || a + p.bytes <= b || b + q.bytes <= a;
 }
 
 }  // namespace saetta

@@ -2999,13 +2999,24 @@ bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const fl
                                         prep.vq.scales == a.vscales && prep.vq.biases == a.vbiases;
     if (!(cache && prep.q_out == a.q && prep.q_and_gate == q_and_gate && prep.tp == a.tp && prep.capacity == a.capacity && prep.p.heads == a.heads &&
           prep.p.kv_heads == a.kv_heads && prep.p.half_dims == 32 && aligned(prep.q_and_gate, 16) && aligned(prep.q_norm, 16))) return false;
-    // Workgroups that make the same key read it while one of them writes it back: `k_back` in the place of `k` (the
-    // reference's in-place key), or of any other input of the step, keeps the launches.
-    const size_t row_kv = size_t(a.rows) * a.kv_heads * DIM * sizeof(float), norm = DIM * sizeof(float);
-    const Span inputs[] = {{prep.q_and_gate, size_t(a.rows) * a.heads * 2 * DIM * sizeof(float)}, {prep.k, row_kv}, {prep.v, row_kv},
-                           {prep.q_norm, norm}, {prep.k_norm, norm}, {a.tp, sizeof(saetta_token_params)}};
-    for (const Span &i : inputs) {
-        if (prep.k_back && !apart({prep.k_back, row_kv}, i)) return false;
+    // One launch only where its buffers lie apart.  In three, the step's inputs are done with when the store has run, so a
+    // program may write the key back in the place of `k` (the reference's in-place key) or lay the partials over any of
+    // them; in one, workgroups still read the inputs while others write.
+    const size_t row_kv = size_t(a.rows) * a.kv_heads * DIM * sizeof(float), row_q = size_t(a.rows) * a.heads * DIM * sizeof(float);
+    const size_t partials = size_t(a.rows) * a.nsplits * a.heads, cached = size_t(a.capacity) * a.kv_heads * DIM;
+    const size_t data = cached * size_t(bits) / 8, scales = bits == 16 ? 0 : cached / SAETTA_QUANT_GROUP * sizeof(uint16_t);
+    const Span inputs[] = {{prep.q_and_gate, 2 * row_q}, {prep.k, row_kv}, {prep.v, row_kv}, {prep.q_norm, DIM * sizeof(float)},
+                           {prep.k_norm, DIM * sizeof(float)}, {a.tp, sizeof(saetta_token_params)}},
+               outputs[] = {{prep.k_back, prep.k_back ? row_kv : 0}, {prep.q_out, row_q}, {a.part_o, partials * DIM * sizeof(float)},
+                            {a.part_ml, partials * 2 * sizeof(float)}, {a.kdata, data}, {a.vdata, data}, {a.kscales, scales},
+                            {a.kbiases, scales}, {a.vscales, scales}, {a.vbiases, scales}};
+    for (const Span &o : outputs) {
+        for (const Span &i : inputs) {
+            if (!apart(o, i)) return false;
+        }
+        for (const Span &other : outputs) {
+            if (&other != &o && !apart(o, other)) return false;
+        }
     }
     token = TokenArgs{a, prep, SAETTA_GQA_GROUP};
     if (!keys_first) {

@@ -30,7 +30,9 @@ class Step:
         keys, values = self.cache.quant or (self.cache.keys, self.cache.values)
         self.q, self.out, self.back = (torch.zeros(rows, n, device="cuda") for n in (H * D, H * D, VALUES))
         self.k0, self.v0 = self.k.clone(), self.v.clone()
+        self.att = saetta.AttentionRows(H, KV, self.cache.capacity, rows) if rows > 1 else None
         lay(self)  # (buffers over others)
+        self.k.copy_(self.k0), self.v.copy_(self.v0)
         self.plan = saetta.Plan()
         saetta.record_store(self.plan, self.qg, self.k, self.v, qn, kn, self.q, keys, values, saetta.PrepParams(H, KV, D, rope_dims, 1e7, 1e-6),
                             self.cache.capacity, rows=rows, k_back=self.back)
@@ -38,8 +40,7 @@ class Step:
             (self.cache.decode.record if kind is saetta.KvBits.Half else self.cache.decode.record_quant)(
                 self.plan, self.q, keys, values, self.qg, self.out)
         else:
-            att = saetta.AttentionRows(H, KV, self.cache.capacity, rows)
-            (att.record if kind is saetta.KvBits.Half else att.record_quant)(
+            (self.att.record if kind is saetta.KvBits.Half else self.att.record_quant)(
                 self.plan, rows, self.q, keys, values, self.qg, self.out, [self.plan.params] * rows)
 
     def run(self, how, position):
@@ -103,6 +104,32 @@ def test_a_key_written_back_in_place(kind, capacity, rows):
     # Several workgroups make a new key; were one to write it back over what the others read, they would take a key
     # that is normed and rotated already.
     step = Step(kind, capacity, rows, seed=capacity + 7 * rows + kind.value, lay=key_in_place)
+    check_laid_over(step, (100, step.cache.capacity - rows))
+
+
+def partials_over_inputs(step):  # k and v, done with when the store has run, in front of part_o
+    att = step.cache.decode if step.rows == 1 else step.att
+    n = step.rows * VALUES
+    step.k, step.v = (att.part_o[i * n:(i + 1) * n].view(step.rows, VALUES) for i in range(2))
+
+
+def partial_sums_over_the_key(step):
+    att = step.cache.decode if step.rows == 1 else step.att
+    step.k = att.part_ml[:step.rows * VALUES].view(step.rows, VALUES)
+
+
+def partials_over_the_key_written_back(step):  # which this program does not read
+    att = step.cache.decode if step.rows == 1 else step.att
+    step.back = att.part_o[:step.rows * VALUES].view(step.rows, VALUES)
+
+
+@pytest.mark.parametrize("lay", [partials_over_inputs, partial_sums_over_the_key, partials_over_the_key_written_back])
+@pytest.mark.parametrize("rows", [1, 3])
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("capacity", [8192, 40960])
+def test_scratch_laid_over_what_is_done_with(kind, capacity, rows, lay):
+    # The context's workgroups write partials while the new rows' workgroups still read k and v.
+    step = Step(kind, capacity, rows, seed=capacity + 5 * rows + kind.value, lay=lay)
     check_laid_over(step, (100, step.cache.capacity - rows))
 
 
