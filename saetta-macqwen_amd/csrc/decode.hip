@@ -300,6 +300,22 @@ __device__ __forceinline__ void wave_sync() {  // LDS written by lanes of the wa
     __builtin_amdgcn_wave_barrier();
 }
 
+// Dims 64 i + lane of a kv head's row of the cache.
+template <int BITS>
+__device__ __forceinline__ void cached_row(const void *data, const uint16_t *scales, const uint16_t *biases, size_t slot, uint32_t lane, float (&x)[4]) {
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) {
+        const uint32_t d = 64 * i + lane;
+        if constexpr (BITS == 16) {
+            x[i] = half_bits_to_float(static_cast<const uint16_t *>(data)[slot * DIM + d]);
+        } else {
+            constexpr uint32_t VPL = 32 / BITS;
+            const uint32_t word = static_cast<const uint32_t *>(data)[slot * (DIM / VPL) + d / VPL];
+            x[i] = fmaf(half_bits_to_float(scales[slot * 4 + i]), float((word >> (d % VPL * BITS)) & ((1u << BITS) - 1)), half_bits_to_float(biases[slot * 4 + i]));
+        }
+    }
+}
+
 // A workgroup of the new rows: q heads head0 .. head0 + heads - 1 of rows row0 .. row0 + nrows - 1 (of up to R).  A wave takes whole
 // heads: lane l holds dims l, 64 + l, 128 + l, 192 + l.
 template <int BITS, int R>
@@ -421,6 +437,23 @@ __device__ __forceinline__ void new_rows(const PartialArgs &a, const PrepArgs &p
                 l += prob;
 #pragma unroll
                 for (int i = 0; i < 4; i++) o[i] += prob * values[t * DIM + 64 * i + lane];
+            }
+        }
+        if constexpr (R == 1) {
+            // a decode sees min(kv_len, capacity) tokens: where the record's kv_len is not position + 1 but more, rows
+            // of the cache past the new one too.  No step of a model has any, so one after the other will do.
+            const uint32_t end = a.decode_len ? min(kv_len, a.capacity) : 0;
+            for (uint32_t t = position + 1; t < end && position < end; t++) {
+                float x[4], dot = 0.0f;
+                cached_row<BITS>(a.kdata, a.kscales, a.kbiases, size_t(t) * kvh + kv, lane, x);
+#pragma unroll
+                for (int i = 0; i < 4; i++) dot += q[i] * x[i];
+                const float s = group_reduce<64>(dot, SumOp()), top = fmaxf(m, s);
+                const float keep = __builtin_amdgcn_exp2f(m - top), prob = __builtin_amdgcn_exp2f(s - top);
+                cached_row<BITS>(a.vdata, a.vscales, a.vbiases, size_t(t) * kvh + kv, lane, x);
+                m = top, l = l * keep + prob;
+#pragma unroll
+                for (int i = 0; i < 4; i++) o[i] = o[i] * keep + prob * x[i];
             }
         }
         const size_t slot = (size_t(row) * a.nsplits + (a.nsplits - 1)) * a.heads + kv * 8 + head0 + pair % heads;

@@ -43,8 +43,10 @@ class Step:
             (self.att.record if kind is saetta.KvBits.Half else self.att.record_quant)(
                 self.plan, rows, self.q, keys, values, self.qg, self.out, [self.plan.params] * rows)
 
-    def run(self, how, position):
-        self.plan.set_params(saetta.TokenParams(0, position))
+    def run(self, how, position, kv_len=None):
+        params = saetta.TokenParams(0, position)
+        params.kv_len = position + 1 if kv_len is None else kv_len
+        self.plan.set_params(params)
         self.q.fill_(float("nan")), self.out.fill_(float("nan")), self.back.fill_(float("nan"))
         self.k.copy_(self.k0), self.v.copy_(self.v0)
         how()
@@ -80,6 +82,24 @@ def test_fused_step_equals_the_ops_one_by_one(kind, capacity, rows):
         assert np.array_equal(got[2], want[2]), position
         for a, b in zip(got[3:], before):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), position
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("capacity", [512, 8192, 40960])
+def test_a_length_of_the_callers_own(kind, capacity):
+    # A decode sees min(kv_len, capacity) tokens whatever the position is: without the new one, or with rows past it.
+    step = Step(kind, capacity, 1, seed=capacity + kind.value)
+    assert launches(step) == 2
+    built = step.plan.build()
+    for position in (0, 70, capacity - 3):
+        for kv_len in (1, 20, position, position + 1, position + 2, position + 75, capacity + 9):
+            want, got = step.run(step.plan.run_serial, position, kv_len), step.run(built.run, position, kv_len)
+            ok = np.isfinite(want[0])  # (no token at all: no number)
+            assert ok.all() or kv_len == 0
+            assert np.array_equal(ok, np.isfinite(got[0])), (position, kv_len)
+            assert np.abs(got[0] - want[0])[ok].max(initial=0.0) < 2e-5, (position, kv_len)
+            for a, b in zip(got[1:], want[1:]):
+                assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), (position, kv_len)
 
 
 def check_laid_over(step, positions):
