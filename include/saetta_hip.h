@@ -490,7 +490,10 @@ int saetta_attn_prefill_quant(saetta_stream_t stream, int bits, const uint16_t *
  * of saetta_prefill_workspace_bytes, then what AttGemm::new allocates for one
  * slice (src/attention_gemm.rs:118-142): the probabilities of eight blocks of
  * keys, the tile maxima and sums, the output sums
- * and the per-row softmax state; about 19 KB per query row of a slice. */
+ * and the per-row softmax state; about 19 KB per query row of a slice; or, where that is more, room
+ * for partial results of parts of the keys (saetta_prefill_workspace_bytes).  A call given a workspace
+ * sized for a longer chunk that ends at the same key or a later one, in slices of as many tokens, always
+ * runs; where parts of the keys do not fit, without the split. */
 size_t saetta_attn_gemm_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t slice_tokens,
                                         uint32_t kv_heads);
 

@@ -1640,9 +1640,15 @@ uint32_t gemm_slice(uint32_t tokens, uint32_t slice_tokens) {
     return slice_tokens == 0 || slice_tokens > tokens ? tokens : slice_tokens;
 }
 
-// The images and the passes' scratch, or the images and the parts of the flash kernel's keys: what is more.
+// The images and the passes' scratch for slices of `slice` tokens: what a call cannot do with less of.  It grows with the
+// key a chunk ends at and with the slice, so a workspace for a chunk does for every shorter one up to the same key.
+size_t passes_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t slice, uint32_t kv_heads) {
+    return align_up(plain_workspace_bytes(pos, tokens, kv_heads), 256) + gemm_scratch_bytes(slice, kv_heads);
+}
+
+// That, or the images and the parts of the flash kernel's keys: what is more.
 size_t gemm_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t slice_tokens, uint32_t kv_heads) {
-    const size_t passes = align_up(plain_workspace_bytes(pos, tokens, kv_heads), 256) + gemm_scratch_bytes(gemm_slice(tokens, slice_tokens), kv_heads);
+    const size_t passes = passes_workspace_bytes(pos, tokens, gemm_slice(tokens, slice_tokens), kv_heads);
     const size_t flash = workspace_bytes(pos, tokens, kv_heads);
     return passes > flash ? passes : flash;
 }
@@ -1657,15 +1663,19 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
     if (int rc = ensure_device()) return rc;
     if (p.tokens == 0) return SAETTA_OK;
     const uint32_t slice = gemm_slice(p.tokens, slice_tokens);
-    const size_t need = gemm_workspace_bytes(p.pos, p.tokens, slice, p.kv_heads);
+    const size_t need = passes_workspace_bytes(p.pos, p.tokens, slice, p.kv_heads);
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
-    if (int rc = acquire_workspace(stream, workspace, workspace_size, need, owned_lock, what, "saetta_attn_gemm_workspace_bytes")) return rc;
-    // All of the call: the flash kernel's result is the same and it is there in 0.5 to 0.6 of the time (see above).
+    // All of the call: the flash kernel's result is the same and it is there in 0.5 to 0.6 of the time (see above).  The
+    // workspace that the passes want does for it: where that has no room for parts of the keys they are not split.
     if (stages == 0) {
         const FlashPlan plan = flash_plan(p.pos, p.tokens, p.kv_heads, bits);
+        const bool split = !workspace || workspace_size >= plan.bytes();
+        if (int rc = acquire_workspace(stream, workspace, workspace_size, split && plan.bytes() > need ? plan.bytes() : need, owned_lock, what,
+                                       "saetta_attn_gemm_workspace_bytes")) return rc;
         if (plan.small) return launch_small(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, what);
-        return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, true, true, plan, what);
+        return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, split, true, plan, what);
     }
+    if (int rc = acquire_workspace(stream, workspace, workspace_size, need, owned_lock, what, "saetta_attn_gemm_workspace_bytes")) return rc;
     const uint32_t nblocks = launch_prepare(stream, bits, kdata, vdata, ks, kz, vs, vz, workspace, p.kv_heads, rows);
 
     const size_t groups = gemm_row_groups(slice) * p.kv_heads;

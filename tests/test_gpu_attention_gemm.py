@@ -171,6 +171,28 @@ def test_rejections(monkeypatch):
     assert np.abs(host(out) - want).max() < 1e-6
 
 
+@pytest.mark.parametrize("tokens", [50, 300, 1000])
+def test_a_workspace_sized_for_a_longer_chunk_does(tokens):
+    # 4096 tokens behind 4096 in slices of 64, then a shorter chunk up to the same key, whose keys would be split in parts
+    # had the workspace room for them (it has not): the call runs, without the split.
+    end, slice_tokens = 8192, 64
+    lib, ffi = saetta.ffi.lib(), saetta.ffi
+    pos, given = end - tokens, lib.saetta_attn_gemm_workspace_bytes(end - 4096, 4096, slice_tokens, KV)
+    assert lib.saetta_prefill_workspace_bytes(pos, tokens, KV) > given
+    gen = torch.Generator(device="cuda").manual_seed(tokens)
+    kc, vc = (torch.randn(end * VALUES, generator=gen, device="cuda").half() for _ in range(2))
+    q = torch.randn(tokens, H, D, generator=gen, device="cuda").half()
+    qg = torch.randn(tokens, H, 2 * D, generator=gen, device="cuda")
+    p = saetta.FlashParams(H, KV, pos, tokens, 1.0 / math.sqrt(D))
+    out = torch.full((tokens, H, D), float("nan"), device="cuda")
+    ws = torch.empty(given, dtype=torch.uint8, device="cuda")
+    rows = lambda t: ffi.QuantRowsC(t.data_ptr(), None, None)  # noqa: E731
+    ffi.check(lib.saetta_attn_gemm(None, 16, q.data_ptr(), rows(kc), rows(vc), qg.data_ptr(), out.data_ptr(), p.c(), slice_tokens, 0,
+                                   ws.data_ptr(), given), "attn_gemm")
+    want = run_flash(saetta.KvBits.Half, host(q), kc, vc, host(qg), pos, tokens)
+    assert np.abs(host(out) - want).max() < MAX_ABS and oracle.rel_rms(host(out), want) < REL_RMS
+
+
 @pytest.mark.parametrize("seed", [31, 32])
 def test_sweep(seed, monkeypatch):
     rng = np.random.default_rng(seed)
