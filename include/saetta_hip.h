@@ -493,7 +493,9 @@ int saetta_attn_prefill_quant(saetta_stream_t stream, int bits, const uint16_t *
  * and the per-row softmax state; about 19 KB per query row of a slice; or, where that is more, room
  * for partial results of parts of the keys (saetta_prefill_workspace_bytes).  A call given a workspace
  * sized for a longer chunk that ends at the same key or a later one, in slices of as many tokens, always
- * runs; where parts of the keys do not fit, without the split. */
+ * runs; where parts of the keys do not fit, without the split.  A whole call (stages 0) writes no probabilities
+ * and runs in no slices: what slice_tokens 1 gives does for it, whatever slice_tokens it is called with
+ * (26 MB for 4096 tokens at 4096 and 2 kv heads, where one slice of the passes wants 1.2 GB). */
 size_t saetta_attn_gemm_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t slice_tokens,
                                         uint32_t kv_heads);
 

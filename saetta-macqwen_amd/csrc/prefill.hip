@@ -1663,10 +1663,11 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
     if (int rc = ensure_device()) return rc;
     if (p.tokens == 0) return SAETTA_OK;
     const uint32_t slice = gemm_slice(p.tokens, slice_tokens);
-    const size_t need = passes_workspace_bytes(p.pos, p.tokens, slice, p.kv_heads);
+    // (a whole call runs in no slices: it asks for the passes' scratch of the smallest)
+    const size_t need = passes_workspace_bytes(p.pos, p.tokens, stages == 0 ? 1 : slice, p.kv_heads);
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
-    // All of the call: the flash kernel's result is the same and it is there in 0.5 to 0.6 of the time (see above).  The
-    // workspace that the passes want does for it: where that has no room for parts of the keys they are not split.
+    // All of the call: the flash kernel's result is the same and it is there in 0.5 to 0.6 of the time (see above).  Where
+    // the workspace has no room for parts of the keys they are not split.
     if (stages == 0) {
         const FlashPlan plan = flash_plan(p.pos, p.tokens, p.kv_heads, bits);
         const bool split = !workspace || workspace_size >= plan.bytes();

@@ -916,9 +916,11 @@ class attention_gemm:
             self.fused = self.texp = True
             self.stages = 0
             self._workspace = None
+            self._captured, self._held = False, []
 
         def workspace_bytes(self, p):
-            return ffi.lib().saetta_attn_gemm_workspace_bytes(p.pos, p.tokens, self.slice, p.kv_heads)
+            """Bytes that a call with `stages` as it is wants: a whole call (0) runs in no slices."""
+            return ffi.lib().saetta_attn_gemm_workspace_bytes(p.pos, p.tokens, self.slice if self.stages else 1, p.kv_heads)
 
         def encode(self, q, keys, values, quant, q_and_gate, out, f, stream=None):
             """encode (src/attention_gemm.rs:144-188): the same as attention_prefill.encode on the same
@@ -940,7 +942,11 @@ class attention_gemm:
                 bits, k, v = quant[0].bits.value, quant[0].c(), quant[1].c()
             need = self.workspace_bytes(f)
             if self._workspace is None or self._workspace.numel() < need:
+                if self._captured:
+                    self._held.append(self._workspace)  # a graph that holds a call goes on using what it was captured with
+                self._captured = False
                 self._workspace = torch.empty(need, dtype=torch.uint8, device=self.device)
+            self._captured = self._captured or torch.cuda.is_current_stream_capturing()
             ffi.check(ffi.lib().saetta_attn_gemm(_stream(stream), bits, _ptr(q), k, v, _ptr(q_and_gate), _ptr(out),
                                                  f.c(), self.slice, self.stages, *_workspace(self._workspace)),
                       "attn_gemm")

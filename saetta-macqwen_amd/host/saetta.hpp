@@ -753,8 +753,16 @@ struct AttGemm {
             bits = int(kv_quant::bits(quant->first->bits));
             k = quant->first->c(), v = quant->second->c();
         }
-        const size_t need = saetta_attn_gemm_workspace_bytes(f.pos, f.tokens, uint32_t(slice), f.kv_heads);
-        if (workspace_.length() < need) workspace_ = gpu::Buffer(need);
+        // (a whole call runs in no slices)
+        const size_t need = saetta_attn_gemm_workspace_bytes(f.pos, f.tokens, stages ? uint32_t(slice) : 1u, f.kv_heads);
+        if (workspace_.length() < need) {
+            if (captured_) held_.push_back(workspace_);  // a graph that holds a call goes on using what it was captured with
+            captured_ = false;
+            workspace_ = gpu::Buffer(need);
+        }
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        hip_check(hipStreamIsCapturing(gpu.stream(), &capturing), "hipStreamIsCapturing");
+        captured_ = captured_ || capturing != hipStreamCaptureStatusNone;
         check(saetta_attn_gemm(gpu.stream(), bits, q.ptr<uint16_t>(), k, v, q_and_gate.ptr<float>(), out.ptr<float>(), f,
                                uint32_t(slice), stages, workspace_.get(), workspace_.length()),
               "attn_gemm");
@@ -762,6 +770,8 @@ struct AttGemm {
 
   private:
     mutable gpu::Buffer workspace_;
+    mutable std::vector<gpu::Buffer> held_;
+    mutable bool captured_ = false;
 };
 
 }  // namespace attention_gemm

@@ -193,6 +193,34 @@ def test_a_workspace_sized_for_a_longer_chunk_does(tokens):
     assert np.abs(host(out) - want).max() < MAX_ABS and oracle.rel_rms(host(out), want) < REL_RMS
 
 
+def test_a_whole_call_holds_no_scratch_for_the_passes():
+    # 600 tokens: 173 MB for the passes' probabilities, which a whole call (stages 0) does not write.
+    pos, tokens = 0, 600
+    q16, k, v, qg = spread_case(pos, tokens)
+    kc, vc, kf, vf = make_cache(saetta.KvBits.Eight, k, v, 640)
+    q, g, out = dev(q16), dev(qg), torch.full((tokens, H, D), float("nan"), device="cuda")
+    p = saetta.FlashParams(H, KV, pos, tokens, 1.0 / math.sqrt(D))
+    gemm, lib = saetta.attention_gemm.AttGemm(tokens, KV), saetta.ffi.lib()
+    gemm.encode(q, None, None, (kc, vc), g, out, p)
+    smallest = lib.saetta_attn_gemm_workspace_bytes(pos, tokens, 1, KV)
+    assert gemm._workspace.numel() == smallest < lib.saetta_attn_gemm_workspace_bytes(pos, tokens, 0, KV) / 4
+    whole = host(out).copy()
+    # captured in the small workspace; the passes then want a larger one, and the graph's stays
+    plan = saetta.Plan()
+    plan.op("attention_gemm", lambda s: gemm.encode(q, None, None, (kc, vc), g, out, p, stream=s))
+    built = plan.build(graph=True)
+    gemm.stages = 3
+    gemm.encode(q, None, None, (kc, vc), g, out, p)
+    assert gemm._workspace.numel() == lib.saetta_attn_gemm_workspace_bytes(pos, tokens, tokens, KV)
+    assert [t.numel() for t in gemm._held] == [smallest]
+    for _ in range(3):
+        out.fill_(float("nan"))
+        junk = torch.full((smallest,), 255, dtype=torch.uint8, device="cuda")  # where the small one would lie, were it given back
+        built.run()
+        assert np.array_equal(host(out), whole)
+        del junk
+
+
 @pytest.mark.parametrize("seed", [31, 32])
 def test_sweep(seed, monkeypatch):
     rng = np.random.default_rng(seed)
