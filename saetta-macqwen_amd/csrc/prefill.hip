@@ -1311,7 +1311,9 @@ int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kda
 // A whole call (stages 0) does NOT take these passes: what they compute is what attention_prefill_kernel computes, and it
 // needs no trip of the probabilities through memory (2048 tokens at 118784, half cache: 5.98 ms by the passes, scores 2.7
 // + pv 3.2, against 3.6 ms; 64 to 4096 tokens at 0 to 130000: 1.6 to 4 times).  The passes run where a caller asks
-// for them by number (stages 1 to 3), to see what the scores and the second product take by themselves.
+// for them by number (stages 1 to 3), to see what the scores and the second product take by themselves, and to check the
+// flash kernel by: with stages 3 the sums and their state are in the scratch (GemmArgs' o, m, l, in that order behind the
+// tiles' sums), and AttGemm.passes_output of the Python mirror makes the outputs of them.
 //
 // Here the pair of launches takes a span of AG_SPAN blocks (the scratch holds that many blocks'
 // probabilities: q and the output sums then go through memory once per span, and there are as many times
@@ -1517,7 +1519,7 @@ __global__ __launch_bounds__(AG_THREADS, 2) void attention_gemm_pv_kernel(GemmAr
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 31, hf = lane >> 5;
     const uint32_t tok0 = blockIdx.y * AG_TOKENS, kv = blockIdx.z;
     const uint32_t need = ag_tiles(a, tok0);
-    if (need == 0) return;  // nothing of this span (the outputs were written at an earlier one)
+    if (need == 0) return;  // nothing of this span (the sums stand as an earlier one left them)
     const uint32_t rg = blockIdx.y * AG_WAVES + wave;
     const size_t rows = size_t(kv) * a.row_groups + rg;
     const size_t state = rows * 32 + col;

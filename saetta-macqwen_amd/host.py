@@ -951,13 +951,36 @@ class attention_gemm:
                                                  f.c(), self.slice, self.stages, *_workspace(self._workspace)),
                       "attn_gemm")
 
+        def passes_output(self, q_and_gate, f):
+            """The outputs as the passes compute them: what the last call of encode, with `stages` 3 and its tokens in one
+            slice, left in the scratch as running sums, divided and gated by torch.  To check the passes by, and the
+            kernel that serves a whole call, with which they share no loop; no way to the outputs."""
+            if self.stages != 3 or f.tokens > self.slice:
+                raise ValueError("AttGemm.passes_output: after a call with stages 3 in one slice")
+            kv, groups = f.kv_heads, -(-f.tokens // 32) * 8  # row groups of 4 tokens x 8 heads per kv head
+            rows = kv * groups
+            # in front of the sums: the images (32 KB per kv head and 32 keys) and their line, P, the tiles' maxima and sums
+            at = -(-(-(-(f.pos + f.tokens) // 32) * kv * 32768 + 256) // 256) * 256 + rows * 256 * (2048 + 2 * 128)
+
+            def take(n):
+                nonlocal at
+                at += 4 * n
+                return self._workspace[at - 4 * n:at].view(torch.float32)
+
+            # a lane (32 half + column) holds dims 32 tile + 8 quad + 4 half + e of the row group's row `column`
+            o = take(rows * 8192).view(kv, groups, 8, 4, 2, 32, 4).permute(0, 1, 5, 2, 3, 4, 6).reshape(kv, groups * 4, 8, DIM)
+            take(rows * 32)  # the maxima
+            out = o / take(rows * 32).view(kv, groups * 4, 8, 1)
+            gate = q_and_gate.view(-1, f.heads, 2 * DIM)[:f.tokens, :, DIM:]
+            return out.permute(1, 0, 2, 3).reshape(groups * 4, f.heads, DIM)[:f.tokens] * torch.sigmoid(gate)
+
     @staticmethod
     def bench(contexts, chunk, layers, device="cuda"):
         """bench (src/attention_gemm.rs:366-470): for each context the chunk of `chunk` tokens at its end and
         at its middle through attention_prefill.encode_rows2 and through AttGemm, best of 3 after a warm-up;
         the gemm passes of the last chunk one by one as differences of runs that stop early (a whole call does not
         take them, so what it has over them, final_ms, is 0 where it is the faster); the largest and
-        the rms relative difference of the two outputs.  One dict per context."""
+        the rms relative difference of what the passes compute to what encode_rows2 gives.  One dict per context."""
         heads, kv, dim = 16, 2, DIM
         gemm = attention_gemm.AttGemm(chunk, kv, device)
         rows = []
@@ -1013,9 +1036,12 @@ class attention_gemm:
                              "softmax_ms": prefix[2] - prefix[1], "pv_ms": prefix[3] - prefix[2],
                              "pv_TFLOP/s": flops(last) / 2 / max(prefix[3] - prefix[2], 1e-9) / 1e9,
                              "final_ms": max(0.0, whole - prefix[3])}
-            # both outputs are now of the last chunk
             best_ms(False, last)
-            diff = (want - got).double()
+            check = attention_gemm.AttGemm(chunk, kv, device)
+            check.slice, check.stages = chunk, 3
+            p = FlashParams(heads, kv, last, chunk, 1.0 / math.sqrt(dim))
+            check.encode(q, k, v, None, g, got, p)
+            diff = (want - check.passes_output(g, p).view(-1)).double()
             row["rel_rms"] = float((diff.pow(2).sum() / want.double().pow(2).sum()).sqrt())
             row["max_abs"] = float(diff.abs().max())
             rows.append(row)

@@ -135,6 +135,48 @@ def test_stages_stop_early_and_write_no_outputs():
         assert (got == 7.0).all(), stages
 
 
+def passes(kind, q16, kc, vc, qg, pos, tokens):
+    """The outputs as the passes compute them (stages 3), which a whole call does not take."""
+    p = saetta.FlashParams(H, KV, pos, tokens, 1.0 / math.sqrt(D))
+    gemm = saetta.attention_gemm.AttGemm(tokens, KV)
+    gemm.slice, gemm.stages = tokens, 3
+    caches = (kc, vc, None) if kind is saetta.KvBits.Half else (None, None, (kc, vc))
+    gemm.encode(q16, *caches, qg, torch.empty(tokens, H, D, device="cuda"), p)
+    return host(gemm.passes_output(qg, p))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("pos,tokens", SHAPES)
+def test_the_passes_match_cpu(kind, pos, tokens):
+    n = pos + tokens
+    q16, k, v, qg = spread_case(pos, tokens)
+    kc, vc, kf, vf = make_cache(kind, k, v, -(-n // 64) * 64 + 64, chunk_from=pos)
+    got = passes(kind, dev(q16), kc, vc, dev(qg), pos, tokens)
+    want = oracle.prefill(q16.astype(np.float32), kf, vf, pos, tokens, q_and_gate=qg, threads=8)
+    assert np.isfinite(got).all()
+    assert np.abs(got - want).max() < MAX_ABS and oracle.rel_rms(got, want) < REL_RMS
+
+
+@pytest.mark.parametrize("kind,pos,tokens", [(saetta.KvBits.Eight, 4096, 4096), (saetta.KvBits.Four, 20000, 1237), (saetta.KvBits.Half, 30000, 2048)])
+def test_a_whole_call_against_the_passes(kind, pos, tokens):
+    # Two programs that share the key images and no loop, at sizes the oracle is slow at: every output.
+    n = pos + tokens
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    kc, vc = (torch.randn(n * VALUES, generator=gen, device="cuda") for _ in range(2))
+    if kind is saetta.KvBits.Half:
+        kc, vc = kc.half(), vc.half()
+    else:
+        rows = [saetta.QuantRows(kind, VALUES, n) for _ in range(2)]
+        rows[0].encode(kc, 0, n), rows[1].encode(vc, 0, n)
+        kc, vc = rows
+    q16 = torch.randn(tokens, H, D, generator=gen, device="cuda").half()
+    qg = torch.randn(tokens, H, 2 * D, generator=gen, device="cuda")
+    want = passes(kind, q16, kc, vc, qg, pos, tokens)
+    for got in (run(kind, q16, kc, vc, qg, pos, tokens), run_flash(kind, host(q16), kc, vc, host(qg), pos, tokens)):
+        assert np.isfinite(got).all()
+        assert np.abs(got - want).max() < MAX_ABS and oracle.rel_rms(got, want) < REL_RMS
+
+
 def test_rejections(monkeypatch):
     pos, tokens = 10, 20
     q16, k, v, qg = spread_case(pos, tokens)
