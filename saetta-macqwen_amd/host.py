@@ -128,6 +128,15 @@ class _Launches:
             self.free(self.plan)
 
 
+def _zeros(n, device):
+    """n zeros (int32) that are in place on return, for whichever stream reads them first: a plan runs on other streams
+    than the one it was recorded on.  (Under capture the order is the graph's.)"""
+    t = torch.zeros(n, dtype=torch.int32, device=device)
+    if t.is_cuda and not torch.cuda.is_current_stream_capturing():
+        torch.cuda.current_stream(t.device).synchronize()
+    return t
+
+
 class Plan:
     """A list of launches recorded once and run for every token (src/plan.rs:63-146).
 
@@ -136,7 +145,7 @@ class Plan:
 
     def __init__(self, device="cuda"):
         self.device = torch.device(device)
-        self.params = torch.zeros(4, dtype=torch.int32, device=self.device)
+        self.params = _zeros(4, self.device)
         self.ops = []  # (kernel name, callable(stream))
         self._counters = None
 
@@ -146,7 +155,7 @@ class Plan:
     def counters(self, n):
         """n zeros (int32) of this plan's own, for an op whose workgroups count one another."""
         if self._counters is None or self._counters.numel() < n:
-            self._counters = torch.zeros(max(n, 4096), dtype=torch.int32, device=self.device)
+            self._counters = _zeros(max(n, 4096), self.device)
         taken, self._counters = self._counters[:n], self._counters[n:]
         return taken
 

@@ -57,3 +57,32 @@ def test_a_plan_of_calls_and_other_ops_keeps_their_order():
         built.run()
     got = [float(t[8]) for t in seen]
     assert got == [1.0, 2.0, 2.0, 4.0]
+
+
+def test_a_plan_recorded_on_a_busy_stream_first_runs_on_another():
+    # The plan's own buffers (the position's record, the counters of the one-launch DeltaNet token) are zero whichever
+    # stream reads them first: the fills must not stand behind the work of the stream the plan was recorded on.
+    k_heads, v_heads, v_dim, conv = 16, 32, 128, 4
+    channels = 2 * k_heads * 128 + v_heads * v_dim
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    made = [torch.randn(n, generator=gen, device="cuda") for n in (channels, channels * conv, 3 * channels, v_heads, v_heads, v_heads, v_heads,
+                                                                 v_heads * v_dim * 128, v_heads * v_dim, v_dim, v_heads * v_dim)]
+    x, state = made[0], made[2]
+    before = state.clone()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        used = [torch.full((n,), 7, dtype=torch.int32, device="cuda") for n in (4, 4096)]
+        del used  # (memory that holds something else, for the allocator to hand out again)
+        big = torch.ones(8192, 8192, device="cuda")
+        for _ in range(20):
+            big = big @ big  # a few ms at least
+        plan = saetta.Plan()
+        saetta.deltanet_token(plan, *made, k_heads, v_heads, v_dim, conv, 1e-6)
+    built = plan.build()
+    with torch.cuda.stream(b):
+        params = plan.params.clone()
+        built.run()
+    torch.cuda.synchronize()
+    assert not host(params).any()
+    assert torch.equal(state, torch.cat([before[channels:], x]))
