@@ -14,8 +14,8 @@ view with an offset); a Metal encoder is a HIP stream.  Shape violations raise
 """
 import ctypes
 import enum
+import itertools
 import math
-import threading
 import time
 
 import torch
@@ -96,30 +96,24 @@ class _Call:
 
 
 class _Launches:
-    """A run of _Calls as the library's own plan (saetta_plan_*): recorded at the first run, then one call
-    makes all the launches."""
+    """A run of _Calls as the library's own plan (saetta_plan_*), recorded here: one call makes all the launches.  The
+    calls' arguments are checked by this, so what they do not accept raises when the plan is built."""
 
     def __init__(self, calls):
-        self.calls, self.plan, self.lock = calls, None, threading.Lock()
-
-    def _record(self, l, s):
-        with self.lock:
-            if self.plan is not None:
-                return
+        self.calls, self.plan, l = calls, None, ffi.lib()
+        # a plan runs on the device it was recorded on: the buffers', or the current one
+        with torch.cuda.device(next((t.device for call in calls for t in call.keep if t is not None), None)):
             ffi.check(l.saetta_plan_begin(), "plan_begin")
             try:
-                for call in self.calls:
-                    call(s)
+                for call in calls:
+                    call(None)
             except BaseException:
                 l.saetta_plan_free(l.saetta_plan_end())
                 raise
             self.free, self.plan = l.saetta_plan_free, ctypes.c_void_p(l.saetta_plan_end())
 
     def __call__(self, s):
-        l = ffi.lib()
-        if self.plan is None:
-            self._record(l, s)
-        rc = l.saetta_plan_run(s, self.plan)
+        rc = ffi.lib().saetta_plan_run(s, self.plan)
         if rc:
             ffi.check(rc, "plan_run")
 
@@ -198,7 +192,8 @@ class Plan:
         return list(out.items())
 
     def build(self, graph=False):
-        """Plan::build (src/plan.rs:229-235).  graph=True captures the launches into a HIP
+        """Plan::build (src/plan.rs:229-235): records the launches, so arguments that a call does not
+        accept raise here and a first run is like any other.  graph=True captures the launches into a HIP
         graph, the counterpart of the reference's indirect command buffer: one submission
         replays them all, and the position still comes from `params` at run time."""
         return Built(list(self.ops), graph)
@@ -215,13 +210,8 @@ class Built:
         # what a run without a graph does: the library's own calls in runs of one native plan each, any other
         # callable as it is
         self._parts = []
-        for _, launch in ops:
-            if not isinstance(launch, _Call):
-                self._parts.append(launch)
-            elif self._parts and isinstance(self._parts[-1], _Launches):
-                self._parts[-1].calls.append(launch)
-            else:
-                self._parts.append(_Launches([launch]))
+        for native, run in itertools.groupby((launch for _, launch in ops), lambda launch: isinstance(launch, _Call)):
+            self._parts += [_Launches(list(run))] if native else run
         if graph and ops:
             # The library's one-time set-up (code objects, LDS limits) must not happen under capture;
             # the launches themselves are not run here: a plan may hold ops that advance a state.

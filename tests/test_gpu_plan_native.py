@@ -86,3 +86,20 @@ def test_a_plan_recorded_on_a_busy_stream_first_runs_on_another():
     torch.cuda.synchronize()
     assert not host(params).any()
     assert torch.equal(state, torch.cat([before[channels:], x]))
+
+
+def test_build_records_and_refuses_what_a_call_does_not_accept():
+    rows = saetta.QuantRows(saetta.KvBits.Eight, VALUES, 8)
+    x = torch.ones(VALUES, device="cuda")
+    plan = saetta.Plan()
+    for _ in range(3):
+        rows.record(plan, x)
+    (part,) = plan.build()._parts
+    assert saetta.ffi.lib().saetta_plan_launches(part.plan) == 3  # (before any run)
+    y = torch.zeros(4096, device="cuda")
+    saetta.deltanet_step(plan, *[y] * 11, 2, 3, 8, 1e-6)  # three value heads over two key heads
+    with pytest.raises(saetta.ffi.SaettaError, match="value heads"):
+        plan.build()
+    assert saetta.ffi.lib().saetta_plan_begin() == 0  # (the recording that failed is over)
+    saetta.ffi.lib().saetta_plan_free(saetta.ffi.lib().saetta_plan_end())
+    assert not host(rows.data).any()
