@@ -451,7 +451,11 @@ int saetta_deltanet_rows_fused_sync(saetta_stream_t stream, const float *x, cons
  * value tile images of the pos + tokens rows the chunk can see and, for a chunk with too few
  * tokens to fill the GPU, room for partial results of parts of the keys (up to 32 parts of
  * 1 KB + 8 B per query row).  A call given the images' part only (one sized for
- * another chunk of as many rows) runs too, without the split.  The reference
+ * another chunk of as many rows) runs too, without the split.  Its bits are then
+ * others: the probabilities are rounded to f16 relative to a maximum, which with
+ * the split is a part's own.  Both forms are as close to the exact result, but who
+ * wants the same bits from one call to the next gives workspaces that both do, or
+ * both do not, hold what this function returns.  The reference
  * has no counterpart (its kernels dequantize in place); the closest is the
  * half scratch of Prefill::new (src/prefill.rs:1674-1686). */
 size_t saetta_prefill_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads);
@@ -493,7 +497,8 @@ int saetta_attn_prefill_quant(saetta_stream_t stream, int bits, const uint16_t *
  * and the per-row softmax state; about 19 KB per query row of a slice; or, where that is more, room
  * for partial results of parts of the keys (saetta_prefill_workspace_bytes).  A call given a workspace
  * sized for a longer chunk that ends at the same key or a later one, in slices of as many tokens, always
- * runs; where parts of the keys do not fit, without the split.  A whole call (stages 0) writes no probabilities
+ * runs; where parts of the keys do not fit, without the split (and so with other bits, see
+ * saetta_prefill_workspace_bytes).  A whole call (stages 0) writes no probabilities
  * and runs in no slices: what slice_tokens 1 gives does for it, whatever slice_tokens it is called with
  * (26 MB for 4096 tokens at 4096 and 2 kv heads, where one slice of the passes wants 1.2 GB). */
 size_t saetta_attn_gemm_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t slice_tokens,
