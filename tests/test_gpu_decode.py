@@ -296,11 +296,11 @@ def test_large_cache_of_codes_several_rows(kind, m):
 def test_several_rows_in_caches_of_65536_and_131072_tokens(kind, m):
     # The reference's caches are 8192 * 2^k tokens (src/gpu_model.rs:390,406-416): a verify step at 32k
     # tokens runs in a cache of 65536.  The keys-first kernel sees the length when it runs: shares of up to
-    # 17 blocks are one round whatever the capacity is, longer ones rounds of up to 8 blocks with the
-    # maxima and sums carried from round to round.  Positions: the first tokens of a cache; a block per
-    # share; shares of 16 and 17 blocks side by side (one round); 18 to 20 blocks (three rounds of 6 and
-    # 7); 25 blocks (rounds of 7 and 4); the whole capacity (4 and 8 rounds of 8).  The rows past the last
-    # token are poisoned.
+    # 17 blocks are one round whatever the capacity is, longer ones rounds of up to 8 blocks (two rows) or 12
+    # (three and four) with the maxima and sums carried from round to round.  Positions: the first tokens of a
+    # cache; a block per share; shares of 16 and 17 blocks side by side (one round); 18 to 20 blocks (three
+    # rounds of 6 and 7 | two of 9 and 10); 25 blocks (rounds of 7 and 4 | 9 and 7); the whole capacity (4 and 8
+    # rounds of 8 | 3 and 6 of 11).  The rows past the last token are poisoned.
     rng = np.random.default_rng(6500 + m)
     q = rng.standard_normal((m, H, D)).astype(np.float32)
     qg = rng.standard_normal((m, H, 2 * D)).astype(np.float32)
@@ -353,11 +353,37 @@ def test_three_and_four_tiles_of_query_rows_at_the_edges_of_a_step(kind, m):
         assert worst < MAX_ABS_F64, (tokens, worst)
 
 
+@pytest.mark.parametrize("splits", [64, 43, 32])
+@pytest.mark.parametrize("kind", [saetta.KvBits.Eight, saetta.KvBits.Four])
+@pytest.mark.parametrize("m", [3, 4])
+def test_rounds_of_as_many_blocks_as_there_is_room_for(m, kind, splits):
+    # Three and four rows in a cache of 24576 tokens: shares of 24, 36 and 48 blocks are two, three and four rounds of
+    # 12, which fill the keys' places of LDS beside the query operands; one block less ends in a round that does not.
+    rng = np.random.default_rng(4300 + splits)
+    capacity = 24576
+    k, v = (rng.standard_normal((capacity, VALUES)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((m, H, D)).astype(np.float32)
+    qg = rng.standard_normal((m, H, 2 * D)).astype(np.float32)
+    rows = saetta.AttentionRows(H, KV, capacity, m)
+    rows.splits = splits
+    for tokens in [capacity, capacity - splits * 16 - 5]:
+        pos = tokens - m
+        kc, vc, kf, vf = cache_pair(k[:tokens], v[:tokens], kind, capacity, poison=True)
+        out = torch.full((m, H, D), float("nan"), device="cuda")
+        plan = saetta.Plan()
+        rows.record_quant(plan, m, dev(q), kc, vc, dev(qg), out, [saetta.TokenParams(0, pos + r).as_tensor("cuda") for r in range(m)])
+        plan.build().run()
+        got = host(out)
+        assert np.isfinite(got).all(), tokens
+        worst = np.abs(got - oracle.rows(q, kf, vf, pos, m, q_and_gate=qg, threads=8, f64=True)).max()
+        assert worst < MAX_ABS_F64, (tokens, worst)
+
+
 @pytest.mark.parametrize("splits", [100, 64, 7])
 def test_several_rows_with_fewer_splits(splits):
     # RowsAttentionParams.splits is an upper bound the caller may lower (src/rows.rs:344-367).  In a
     # cache of 24576 tokens: 100 splits are shares of 15 and 16 blocks, still one round of the
-    # keys-first kernel; 64 splits are shares of 24 blocks (three rounds of 8) and 7 of 220 (28 rounds).
+    # keys-first kernel; 64 splits are shares of 24 blocks (two rounds of 12) and 7 of 220 (19 rounds).
     rng = np.random.default_rng(4100 + splits)
     capacity, m, kind = 24576, 3, saetta.KvBits.Eight
     k = rng.standard_normal((capacity, VALUES)).astype(np.float32)
