@@ -28,6 +28,8 @@ int launch_status(const char *what);
 // Device address of the current device's sticky status word (pinned host memory): a kernel whose
 // bounded wait runs out stores a non-zero code there.  nullptr before the device's set-up.
 uint32_t *device_status_word();
+// Compute units of the current device (asked for once per device; without a device, the MI355X's 256).
+uint32_t cu_count();
 
 // One-time set-up of a source file's kernels on the current device: loads their code object and
 // raises their dynamic LDS limits, so that a first launch under stream capture has nothing left to

@@ -1371,7 +1371,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
     const uint32_t last_tok = limit - 1;                   // rows past it are never read: loads are clamped to it
     const uint32_t range = blk_end - blk_begin;
     // rounds of equal size (the last may be shorter), none longer than 17 blocks
-    // (several rows: one round of up to 17 blocks, or rounds of up to 8)
+    // (one row and two: one round of up to 17 blocks, or rounds of up to 8; three and four rows: of up to 12)
     constexpr uint32_t LONG_ROUND = W::ALTERNATE ? W::ALT_BLOCKS : W::SHORT_BLOCKS;
     const uint32_t n_rounds = range > uint32_t(RBK) ? (range + LONG_ROUND - 1) / LONG_ROUND : 1;
     const bool alt = W::ALTERNATE && n_rounds > 1;  // rounds in alternate halves of LDS
@@ -3093,13 +3093,14 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
     // One to four rows over codes in a cache of 24k tokens and more go to the kernel with loader waves, a
     // one-workgroup-per-CU kernel at every length: a share of up to 17 blocks (the kernel sees the length
     // when it runs: a step at 32k tokens is one round in a cache of any size) is one round, a longer one
-    // rounds of 8 blocks.  SAETTA_STAGE_NO_LOADERS keeps to the register kernels (the caller's choice of
+    // rounds of 8 blocks (three and four rows: 12).  SAETTA_STAGE_NO_LOADERS keeps to the register kernels (the caller's choice of
     // kernel family, as DecodeAttention.kernel is in the reference, src/attention.rs:36-38).
     // The register kernels: one workgroup per CU (half as many splits, each twice as long) or two.  Two
     // rows and more and a half cache need the whole register file anyway; one row over codes fits two
     // workgroups per CU, which pays only for long contexts: up to 64k tokens the shorter merge of half as
     // many partials is worth more (measured: 19.4 against 20.6 us per layer at 32k, 28.3 against 29.7 at
-    // 64k, but 44 against 35 at 146k, 4-bit).  Both stages derive the same number from the same arguments.
+    // 64k, but 44 against 35 at 146k, 4-bit).  Both stages of a call derive the same number from the same arguments; where
+    // a plan's reduce stage makes a token step of the launches before it, the number is the token step's.
     const bool keys_first = rows <= 4 && bits != 16 && capacity >= KEYS_FIRST_FROM && !(stages & SAETTA_STAGE_NO_LOADERS);
     const bool one_per_cu = rows >= 2 || bits == 16 || capacity <= 80 * 1024 || keys_first;
     if (one_per_cu && nsplits > MAX_SPLITS / 2) nsplits = MAX_SPLITS / 2;

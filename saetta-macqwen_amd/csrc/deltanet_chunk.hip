@@ -866,7 +866,7 @@ int run_deltanet_chunk(hipStream_t stream, const float *mixed, const float *a, c
     // The conv inside: while the workgroups are all on the machine at once, two to a CU.  Past that the conv's own kernel
     // is the faster one, whose many waves keep the memory busy (whole chunk, us, inside against apart: 1000 tokens 76.8
     // and 79, 2048 125 and 131; 3000 209 and 199, 4096 290 and 280).
-    const bool conv_inside = two_heads && p.v_dim == CONV_V && nblocks * p.k_heads <= 2 * 256;
+    const bool conv_inside = two_heads && p.v_dim == CONV_V && nblocks * p.k_heads <= 2 * cu_count();
     if (conv_inside && list && take_conv(*list, args, conv_out)) {
         launch(deltanet_chunk_prepare_kernel<2, true>, dim3(nblocks, p.k_heads), 256, PrepLds<2>::BYTES, stream, args, conv_out);
     } else if (two_heads) {

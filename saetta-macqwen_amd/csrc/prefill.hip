@@ -42,7 +42,6 @@
 #include "common.hpp"
 #include "lanes.hpp"
 
-#include <atomic>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -1072,23 +1071,6 @@ size_t images_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) {
     return blocks * kv_heads * IMG_BYTES;
 }
 size_t plain_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) { return images_bytes(pos, tokens, kv_heads) + 256; }
-
-// Compute units of the current device (asked for once per device).
-uint32_t cu_count() {
-    static std::atomic<int> known[OWNED_DEVICES];
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= OWNED_DEVICES) {
-        (void)hipGetLastError();
-        return 256;
-    }
-    if ((cus = known[dev].load(std::memory_order_relaxed)) > 0) return uint32_t(cus);
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
-        (void)hipGetLastError();
-        return 256;
-    }
-    known[dev].store(cus, std::memory_order_relaxed);
-    return uint32_t(cus);
-}
 
 constexpr size_t PART_O_BYTES = size_t(TQ) * SAETTA_GQA_GROUP * DIM * 4, PART_ML_BYTES = size_t(TQ) * SAETTA_GQA_GROUP * 8;
 size_t parts_bytes(uint32_t tokens, uint32_t kv_heads, uint32_t nparts) {

@@ -1,6 +1,7 @@
 // Error plumbing and device check of the C ABI.
 #include "common.hpp"
 
+#include <atomic>
 #include <cstring>
 #include <mutex>
 
@@ -99,6 +100,22 @@ DeviceSetup *current_setup() {
     return dev >= 0 && dev < MAX_DEVICES ? &g_devices[dev] : nullptr;
 }
 }  // namespace
+
+uint32_t cu_count() {
+    static std::atomic<int> known[MAX_DEVICES];
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) {
+        (void)hipGetLastError();
+        return 256;
+    }
+    if ((cus = known[dev].load(std::memory_order_relaxed)) > 0) return uint32_t(cus);
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
+        (void)hipGetLastError();
+        return 256;
+    }
+    known[dev].store(cus, std::memory_order_relaxed);
+    return uint32_t(cus);
+}
 
 uint32_t *device_status_word() {
     DeviceSetup *d = current_setup();

@@ -474,8 +474,8 @@ def deltanet_step(plan, q, k, v, a, b, a_log, dt_bias, state, z, norm_w, y, k_he
 def deltanet_token(plan, x, w, conv_state, a, b, a_log, dt_bias, state, z, norm_w, y, k_heads, v_heads, v_dim,
                    kernel_size, eps):
     """Records one token of a Gated DeltaNet layer, conv and step (GpuDeltaNet::record,
-    src/gpu_layers.rs:633-684) as one call of two launches: what deltanet_conv + deltanet_step give,
-    without the conv output in between."""
+    src/gpu_layers.rs:633-684) as one call: what deltanet_conv + deltanet_step give, without the conv
+    output in between; one launch where the value dim is 128 and the conv has 4 taps, else two."""
     ts = (x, w, conv_state, a, b, a_log, dt_bias, state, z, norm_w, y)
     for t in ts:
         _need(t, torch.float32, "deltanet_token buffer")
@@ -538,7 +538,7 @@ def deltanet_rows(plan, mixed, a, b, a_log, dt_bias, state, z, norm_w, y, k_head
 
 def deltanet_rows_fused(plan, x, w, conv_state, a, b, a_log, dt_bias, state, z, norm_w, y, k_heads, v_heads, v_dim,
                         kernel_size, rows, eps, conv_snaps=None, state_snaps=None):
-    """Records up to 8 rows of a Gated DeltaNet layer, conv and step, as one call of two launches
+    """Records up to 8 rows of a Gated DeltaNet layer, conv and step, as one call of one launch, or two
     (kernel deltanet_rows, GpuDeltaNet::record_rows with DN_SIMDS = 0, src/gpu_layers.rs:737-757):
     x, z [rows][...] as for deltanet_conv_rows + deltanet_rows, which this equals; with the two
     snapshot buffers the conv and delta states after each row go there too."""
