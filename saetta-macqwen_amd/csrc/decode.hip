@@ -1254,7 +1254,8 @@ struct KeysFirst {
     // (Two pairs: rounds of 12, for which there is room.  A round costs 2.6 us beside its bytes, and with the new
     // tokens' split taken out of the context's 128 a share of 32 blocks is one of 33, a fifth round of 8: four rows at 65500
     // tokens, 4-bit, 42.3 -> 38.5 us a layer, 120000 60.7 -> 56.0, 262000 114.6 -> 105.5; 8-bit 42.0 -> 37.7, 57.6 -> 54.5,
-    // 109.3 -> 99.4; behind at some lengths between: 80000 43.9 -> 44.9.)
+    // 109.3 -> 99.4; behind at some lengths between: 80000 43.9 -> 44.9; and behind without the new tokens' split, where
+    // shares of 32 and 64 blocks are whole rounds of 8: four rows, 8-bit, at 65000 tokens 37.8 -> 38.2, 131000 62.5 -> 64.2.)
     static constexpr int SHORT_BLOCKS = PAIRS == 2 ? 12 : 8;
     static constexpr int QP_PAIR_BYTES = 2 * 8 * 64 * 16, QPZ_PAIR_BYTES = 2 * 64 * 16;
     static constexpr int QP_BYTES = M > 1 ? PAIRS * (QP_PAIR_BYTES + QPZ_PAIR_BYTES) : 0;
