@@ -150,15 +150,19 @@ __device__ __forceinline__ void conv_state_move(const float *x, float *state, ui
     for (int j = 0; j < past; j++) state[size_t(j) * p.channels + c] = conv_input(x, state, int(p.tokens) - past + j, c, p);
 }
 
-// The same for four channels a thread (16-byte loads and stores, eight tokens' loads in flight), four taps:
-// every channel's sums are taken in the same order as above, so the results are the same bit for bit.
-constexpr uint32_t CONV4_AHEAD = 8;
-static_assert(CONV_TILE % CONV4_AHEAD == 0, "whole groups of tokens in a tile");
-static_assert(CONV_TILE > 15, "every token that reads the state lies in the first tile");
+// The same for four channels a thread (16-byte loads and stores, a tile's loads all in flight), four taps: every channel's
+// sums are taken in the same order as above, so the results are the same bit for bit.  Bound by memory over a long chunk,
+// by one trip through memory and the instructions behind it over a short one, so the tiles are short: a tile of 4 tokens
+// reads 7 rows, 3 of them a second time out of the L2, and is done 8 times as soon as one of 32.  Conv alone, tiles of 32
+// -> 4: 40 tokens 13.9 -> 4.6 us, 2100 34.6 -> 27, 4096 50.6 -> 49.9 (268 MB at 5.4 TB/s); whole layer, us, tiles of
+// 32 / 16 / 8 / 4: 40 tokens 25.7 / 21.1 / 18.8 / 17.6, 2100 150 / 147 / 145 / 142, 4095 269 / 273 / 269 / 267.
+constexpr uint32_t CONV4_TILE = 4;
+constexpr uint32_t CONV4_TAPS = 4, CONV4_FROM = SAETTA_MAX_ROWS + 1;  // (taps it is made for; tokens from which it is taken)
+static_assert(CONV4_TILE >= CONV4_TAPS - 1, "every token that reads the state lies in the first tile");
 __global__ __launch_bounds__(256) void deltanet_conv_rows4_kernel(const float *__restrict__ x, const float *__restrict__ w,
                                                                   float *state, float *__restrict__ out,
                                                                   float *__restrict__ snaps, saetta_conv_rows_params p) {
-    constexpr int KS = 4;
+    constexpr int KS = CONV4_TAPS;
     const uint32_t c4 = blockIdx.x * 256 + threadIdx.x, quads = p.channels / 4;
     if (c4 >= quads) return;
     const float4 *x4 = reinterpret_cast<const float4 *>(x);
@@ -171,39 +175,36 @@ __global__ __launch_bounds__(256) void deltanet_conv_rows4_kernel(const float *_
         taps[0] = make_float4(a.x, b.x, c.x, d.x), taps[1] = make_float4(a.y, b.y, c.y, d.y);
         taps[2] = make_float4(a.z, b.z, c.z, d.z), taps[3] = make_float4(a.w, b.w, c.w, d.w);
     }
-    const uint32_t t_begin = blockIdx.y * CONV_TILE, t_end = min(p.tokens, t_begin + CONV_TILE);
-    float4 win[KS - 1];
+    const uint32_t t0 = blockIdx.y * CONV4_TILE;
+    float4 win[KS - 1], xt[CONV4_TILE];
 #pragma unroll
     for (int j = 0; j < KS - 1; j++) {
-        const int i = int(t_begin) - (KS - 1) + j;
+        const int i = int(t0) - (KS - 1) + j;
         win[j] = i >= 0 ? x4[size_t(i) * quads + c4] : s4[size_t(i + KS - 1) * quads + c4];
     }
-    for (uint32_t t0 = t_begin; t0 < t_end; t0 += CONV4_AHEAD) {
-        float4 xt[CONV4_AHEAD];
 #pragma unroll
-        for (uint32_t u = 0; u < CONV4_AHEAD; u++) xt[u] = x4[size_t(min(t0 + u, p.tokens - 1)) * quads + c4];
+    for (uint32_t u = 0; u < CONV4_TILE; u++) xt[u] = x4[size_t(min(t0 + u, p.tokens - 1)) * quads + c4];
 #pragma unroll
-        for (uint32_t u = 0; u < CONV4_AHEAD; u++) {
-            const uint32_t t = t0 + u;
-            if (t >= t_end) break;
-            float4 acc = make_float4(0, 0, 0, 0);
+    for (uint32_t u = 0; u < CONV4_TILE; u++) {
+        const uint32_t t = t0 + u;
+        if (t >= p.tokens) break;
+        float4 acc = make_float4(0, 0, 0, 0);
 #pragma unroll
-            for (int j = 0; j < KS - 1; j++) {
-                acc.x += taps[j].x * win[j].x, acc.y += taps[j].y * win[j].y, acc.z += taps[j].z * win[j].z, acc.w += taps[j].w * win[j].w;
-            }
-            o4[size_t(t) * quads + c4] = make_float4(silu_f(acc.x + taps[KS - 1].x * xt[u].x), silu_f(acc.y + taps[KS - 1].y * xt[u].y),
-                                                     silu_f(acc.z + taps[KS - 1].z * xt[u].z), silu_f(acc.w + taps[KS - 1].w * xt[u].w));
+        for (int j = 0; j < KS - 1; j++) {
+            acc.x += taps[j].x * win[j].x, acc.y += taps[j].y * win[j].y, acc.z += taps[j].z * win[j].z, acc.w += taps[j].w * win[j].w;
+        }
+        o4[size_t(t) * quads + c4] = make_float4(silu_f(acc.x + taps[KS - 1].x * xt[u].x), silu_f(acc.y + taps[KS - 1].y * xt[u].y),
+                                                 silu_f(acc.z + taps[KS - 1].z * xt[u].z), silu_f(acc.w + taps[KS - 1].w * xt[u].w));
 #pragma unroll
-            for (int j = 0; j + 1 < KS - 1; j++) win[j] = win[j + 1];
-            win[KS - 2] = xt[u];
-            if (p.snapshots) {
-                float4 *snap = reinterpret_cast<float4 *>(snaps) + size_t(t) * (KS - 1) * quads;
+        for (int j = 0; j + 1 < KS - 1; j++) win[j] = win[j + 1];
+        win[KS - 2] = xt[u];
+        if (p.snapshots) {
+            float4 *snap = reinterpret_cast<float4 *>(snaps) + size_t(t) * (KS - 1) * quads;
 #pragma unroll
-                for (int j = 0; j < KS - 1; j++) snap[size_t(j) * quads + c4] = win[j];
-            }
+            for (int j = 0; j < KS - 1; j++) snap[size_t(j) * quads + c4] = win[j];
         }
     }
-    if (blockIdx.y == 0) {  // (a tile of tokens at least: the new state is all inputs)
+    if (blockIdx.y == 0) {  // (CONV4_FROM tokens at least: the new state is all inputs)
 #pragma unroll
         for (int j = 0; j < KS - 1; j++) s4[size_t(j) * quads + c4] = x4[size_t(p.tokens - (KS - 1) + j) * quads + c4];
     }
@@ -948,11 +949,11 @@ extern "C" int saetta_deltanet_conv_rows(saetta_stream_t stream, const float *x,
     if (int rc = ensure_device()) return rc;
     if (p.channels == 0 || p.tokens == 0) return SAETTA_OK;
     const dim3 grid((p.channels + 255) / 256, (p.tokens + CONV_TILE - 1) / CONV_TILE);
-    // (four channels a thread pays from a tile of tokens up: a verify step's few rows want the workgroups)
-    const bool by_four = p.tokens >= CONV_TILE && p.channels % 4 == 0 && aligned(x, 16) && aligned(w, 16) && aligned(state, 16) && aligned(out, 16) &&
+    // (four channels a thread: a verify step's few rows want the workgroups; 16 tokens take 4.1 us this way and 6.1 the other)
+    const bool by_four = p.tokens >= CONV4_FROM && p.channels % 4 == 0 && aligned(x, 16) && aligned(w, 16) && aligned(state, 16) && aligned(out, 16) &&
                          (!p.snapshots || aligned(snaps, 16));
-    if (p.kernel_size == 4 && by_four) {
-        launch(deltanet_conv_rows4_kernel, dim3((p.channels / 4 + 255) / 256, grid.y), 256, 0, as_stream(stream), x, w, state, out, snaps, p);
+    if (p.kernel_size == CONV4_TAPS && by_four) {
+        launch(deltanet_conv_rows4_kernel, dim3((p.channels / 4 + 255) / 256, (p.tokens + CONV4_TILE - 1) / CONV4_TILE), 256, 0, as_stream(stream), x, w, state, out, snaps, p);
         tag_launch(LAUNCH_CONV, 0, 0);
     } else if (p.kernel_size == 4) {
         launch(deltanet_conv_rows_kernel<4>, grid, 256, 0, as_stream(stream), x, w, state, out, snaps, p);

@@ -319,6 +319,12 @@ def test_a_plan_of_conv_and_chunk_gives_what_the_calls_give(k_heads, v_heads, v_
     lib.saetta_plan_free(made)
 
 
+@pytest.mark.parametrize("tokens", [8, 9, 11, 12, 13])
+def test_conv_of_four_channels_a_thread_at_the_edges_of_its_tiles(tokens):
+    # from 9 tokens on, in tiles of 4; the last tile has 1 to 4 tokens
+    check_against_oracle(Layer(2, 4, 16, 4, seed=tokens), 2 * tokens, [tokens, tokens], snapshots=True)
+
+
 def test_rejections():
     z = torch.zeros(4096, device="cuda")
     plan = saetta.Plan()
