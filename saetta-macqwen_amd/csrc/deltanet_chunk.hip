@@ -97,17 +97,24 @@ __device__ __forceinline__ floatx4 mma3(half8 ah, half8 al, half8 bh, half8 bl, 
 }
 
 // ---- prepare: everything of a block that does not depend on the state ------------------------------
-// One workgroup takes G value heads of one key head: the q / k images and the k . k and q . k products
-// belong to the key head, the gates, A, M and T to a value head.  (G = 2, the model's two value heads
-// per key head: the four waves take the heads' four diagonal blocks of the triangular solve; G = 1: any
-// other ratio, one workgroup per value head, the first of a key head's writing the key head's images.)
+// One workgroup of eight waves takes G value heads of one key head: the q / k images and the k . k and q . k products
+// belong to the key head, the gates, A, M and T to a value head.  (G = 2: the model's two value heads per key head;
+// G = 1: any other ratio, one workgroup per value head, the first of a key head's writing the key head's images.)
+// What bounds it: a workgroup is a chain of short phases, and with few blocks (up to 1024 tokens: a workgroup to a CU)
+// that chain is the kernel's time, with many the memory (67 MB read and 118 written at 4096 tokens: 3.7 TB/s).  So the phases are
+// spread over two teams of four waves, a row tile of 16 tokens to a wave: one makes A and solves for T, the other makes M
+// and stores it meanwhile; the products are taken as their transposes, so that a lane's four results lie in a row and
+// leave as one 8-byte store; the solve has a lane to a column, with no sums over lanes.
+// Measured, us, against four waves that did it all in order: 1000 tokens 22.7 -> 15.8, 2047 28.3 -> 26.4, 4096 57.4 -> 49.8;
+// with the conv inside, 512 tokens 31.5 -> 20.3.
 // LDS: the four q / k images; once the products are taken, the heads' A (f32) go over kh | kl, their M
-// images and later their T images over qh | ql (and 2 KB more), so that they leave as whole 16-byte stores.
+// images and later their T images over qh | ql (and more), so that they leave as whole 16-byte stores.
+constexpr int PREP_THREADS = 512, PREP_WAVES = PREP_THREADS / 64;
 template <int G>
 struct PrepLds {
     // per head, over kh | kl once the products are taken: the two diagonal 32 x 32 blocks of A as f32, rows of
-    // DROW ([t][q * 16 + m] holds A_t,s of s = 2m + q; the product of the off-diagonal block goes over them
-    // later), then the block below the diagonal and the inverse of the second diagonal block as f16 images
+    // DROW (their inverses go over them, the product of the off-diagonal block over those later), then the
+    // block below the diagonal and the inverse of the second diagonal block as f16 images
     static constexpr int DROW = 32 + 4, D_BYTES = 32 * DROW * 4;
     static constexpr int HROW = 32 + 8, H_IMG = 32 * HROW * 2;  // f16 per row of a 32 x 32 image; bytes of one part
     static constexpr int W_OFF = 0, LBA_OFF = 2 * D_BYTES, XBB_OFF = LBA_OFF + 2 * H_IMG, HEAD_BYTES = XBB_OFF + 2 * H_IMG;
@@ -119,6 +126,21 @@ struct PrepLds {
     static constexpr int BYTES = GATES + G * GATE_BYTES;
     static_assert(2 * BYTES <= 160 * 1024, "two workgroups per CU");
 };
+
+// x of the lane that DPP control CTRL names, zero where there is none or the row is not in ROWS
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_or_zero(double x) {
+    const u32x2 v = __builtin_bit_cast(u32x2, x);
+    return __builtin_bit_cast(double, u32x2{uint32_t(__builtin_amdgcn_update_dpp(0, int(v.x), CTRL, ROWS, 0xf, false)),
+                                            uint32_t(__builtin_amdgcn_update_dpp(0, int(v.y), CTRL, ROWS, 0xf, false))});
+}
+// The inclusive sum over the lanes of a wavefront: inside rows of 16 lanes, then row by row.
+__device__ __forceinline__ double inclusive_sum(double x) {
+    x += dpp_or_zero<0x111, 0xf>(x), x += dpp_or_zero<0x112, 0xf>(x);  // row_shr 1, 2
+    x += dpp_or_zero<0x114, 0xf>(x), x += dpp_or_zero<0x118, 0xf>(x);  // row_shr 4, 8
+    x += dpp_or_zero<0x142, 0xa>(x);                                   // row_bcast 15, to rows 1 and 3
+    return x + dpp_or_zero<0x143, 0xc>(x);                             // row_bcast 31, to rows 2 and 3
+}
 
 // The B operand of a 16-column tile out of a row-major f16 image in LDS (hi part at `at`, lo part `part_bytes`
 // on; `at`: the byte address of row 8j + e, column 4a of the tile for lane a + 4e of its 16): lane (n, j)
@@ -135,15 +157,17 @@ __device__ __forceinline__ void read_by_column(uint32_t at, uint32_t part_bytes,
     lo = __builtin_bit_cast(half8, u32x4{r[1][0].x, r[1][0].y, r[1][1].x, r[1][1].y});
 }
 
-// The conv of four channels c4 .. c4 + 3 for the 16 tokens from t0 on, in two parts: the inputs are asked for, and
+// The conv of four channels c .. c + 3 for the TOKENS tokens from t0 on, in two parts: the inputs are asked for, and
 // the outputs made, with the sums in the order of deltanet_conv_rows4_kernel (the results are the same bit for bit).
+template <int TOKENS>
 struct ConvPiece {
-    float4 taps[CONV], in[CONV - 1 + 16];
+    static_assert(TOKENS >= CONV - 1, "every token that reads the state lies in the first piece");
+    float4 taps[CONV], in[CONV - 1 + TOKENS];
     __device__ __forceinline__ void request(const ChunkArgs &a, uint32_t c, uint32_t t0) {
 #pragma unroll
         for (int j = 0; j < CONV; j++) taps[j] = reinterpret_cast<const float4 *>(a.conv_w + size_t(c) * CONV)[j];  // (by channel)
 #pragma unroll
-        for (int i = 0; i < CONV - 1 + 16; i++) {
+        for (int i = 0; i < CONV - 1 + TOKENS; i++) {
             const int t = int(t0) + i - (CONV - 1);
             // (a token past the end: unused)
             const float *row = t >= 0 ? a.x + size_t(min(uint32_t(t), a.tokens - 1)) * a.channels : a.conv_state + (t + CONV - 1) * a.channels;
@@ -168,13 +192,14 @@ struct ConvPiece {
             *reinterpret_cast<float4 *>(a.conv_state + j * a.channels + c) = *reinterpret_cast<const float4 *>(a.x + size_t(a.tokens - (CONV - 1) + j) * a.channels + c);
     }
 };
+constexpr int CONV_QK = C / PREP_WAVES, CONV_VALUES = 8;  // tokens of a piece of q and k, and of the values
 
-// CONVOLVE: the conv before the delta rule is part of it.  The workgroup's channels, q and k of its key head and the
-// values of its heads, are nobody else's.  A thread makes four channels' outputs for 16 tokens, of q or k and then of
-// the values, and stores them as the conv's own kernel does; q and k also go to LDS as f32, over the place of the
-// images, and from there to the threads that normalise them.
+// CONVOLVE: the conv before the delta rule is part of the launch.  The workgroup of a block makes the q and k of its key
+// head, which are nobody else's: a thread four channels' outputs for CONV_QK tokens, stored as the conv's own kernel does
+// and in LDS as f32, over the place of the images, from where they go to the threads that normalise them.  The values, which
+// nothing in this kernel reads, are made by workgroups of their own behind the blocks' (grid x from the number of blocks on).
 template <int G, bool CONVOLVE>
-__global__ __launch_bounds__(256, 2) void deltanet_chunk_prepare_kernel(ChunkArgs a, float *conv_out) {
+__global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel(ChunkArgs a, float *conv_out) {
     using L = PrepLds<G>;
     constexpr int DROW = L::DROW, HROW = L::HROW;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -196,259 +221,285 @@ __global__ __launch_bounds__(256, 2) void deltanet_chunk_prepare_kernel(ChunkArg
     auto ws_v = [&](int hh) { return ws_blk + a.k_heads * KHEAD_BYTES + (h0 + hh) * VHEAD_BYTES; };
     const bool writer = h0 % group == 0;  // one workgroup of the key head's keeps the q / k images
 
+    if constexpr (CONVOLVE) {
+        const uint32_t nblocks = (a.tokens + C - 1) / C;
+        if (blk >= nblocks) {  // the values' conv: four channels a thread, CONV_VALUES tokens
+            const uint32_t quads = a.v_heads * a.v_dim / 4, columns = (quads + PREP_THREADS - 1) / PREP_THREADS;
+            const uint32_t at = (blk - nblocks) * a.k_heads + blockIdx.y, quad = at % columns * PREP_THREADS + tid, t0 = at / columns * CONV_VALUES;
+            if (quad >= quads || t0 >= a.tokens) return;
+            const uint32_t cv = 2 * key_size + 4 * quad;
+            ConvPiece<CONV_VALUES> values;
+            values.request(a, cv, t0);
+#pragma unroll
+            for (int i = 0; i < CONV_VALUES; i++) {
+                const float4 y = values.output(i);
+                if (t0 + i < a.tokens) *reinterpret_cast<float4 *>(conv_out + size_t(t0 + i) * a.channels + cv) = y;
+            }
+            if (t0 == 0) values.keep_state(a, cv);
+            return;
+        }
+    }
+    // ---- the gates' inputs of head h0 + gate_head, one of the last G waves: asked for first ----
+    const int gate_head = int(wave) - (PREP_WAVES - G);
+    const bool gate_real = blk * C + lane < a.tokens;
+    float gate_a = 0.0f, gate_b = 0.0f, gate_log = 0.0f, gate_bias = 0.0f;
+    if (gate_head >= 0) {
+        const uint32_t tok = min(blk * C + lane, a.tokens - 1), h = h0 + gate_head;
+        gate_a = a.a[size_t(tok) * a.v_heads + h], gate_b = a.b[size_t(tok) * a.v_heads + h], gate_log = a.a_log[h], gate_bias = a.dt_bias[h];
+    }
+    // c_t = sum of log g up to t, beta_t (tokens past the end: g = 1, beta = 0)
+    auto gates = [&]() {
+        if (gate_head < 0) return;
+        float g, beta, lg;
+        fast_gates(gate_a + gate_bias, __expf(gate_log), gate_b, g, beta, &lg);
+        const double c = inclusive_sum(gate_real ? double(lg) : 0.0);
+        cum_lds(gate_head)[lane] = c, beta_lds(gate_head)[lane] = gate_real ? beta : 0.0f;
+        const double last = __shfl(c, 63, 64);
+        float *gam = reinterpret_cast<float *>(ws_v(gate_head) + 4 * T_GL);
+        gam[lane] = __expf(float(c)), gam[C + lane] = __expf(float(last - c));
+    };
+
     // ---- the conv (src/cpu/deltanet.rs:69-100) of the workgroup's channels ----
     constexpr int FROW = 2 * K_DIM + 4;  // f32 per token's q | k in LDS
     static_assert(C * FROW * 4 <= 4 * K_IMG, "the f32 q and k lie over the images");
     float *qk_lds = reinterpret_cast<float *>(lds);
     if constexpr (CONVOLVE) {
-        static_assert(G * CONV_V == 4 * 64, "a wave's lanes take the values of a token");
-        const uint32_t t0 = blk * C + 16 * wave;
+        const uint32_t t0 = blk * C + CONV_QK * wave;
         const uint32_t cqk = (lane < 32 ? 0 : key_size - K_DIM) + khd * K_DIM + 4 * lane;  // q: lanes 0-31, k: lanes 32-63
-        const uint32_t cv = 2 * key_size + h0 * CONV_V + 4 * lane;
-        ConvPiece qk, vs;
+        ConvPiece<CONV_QK> qk;
         qk.request(a, cqk, t0);
-        vs.request(a, cv, t0);
+        gates();
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
+        for (int i = 0; i < CONV_QK; i++) {
             const bool real = t0 + i < a.tokens;
             const float4 y = real ? qk.output(i) : make_float4(0, 0, 0, 0);
-            *reinterpret_cast<float4 *>(qk_lds + (16 * wave + i) * FROW + 4 * lane) = y;
+            *reinterpret_cast<float4 *>(qk_lds + (CONV_QK * wave + i) * FROW + 4 * lane) = y;
             if (real) *reinterpret_cast<float4 *>(conv_out + size_t(t0 + i) * a.channels + cqk) = y;
         }
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const float4 y = vs.output(i);
-            if (t0 + i < a.tokens) *reinterpret_cast<float4 *>(conv_out + size_t(t0 + i) * a.channels + cv) = y;
-        }
-        if (t0 == 0) qk.keep_state(a, cqk), vs.keep_state(a, cv);
+        if (t0 == 0) qk.keep_state(a, cqk);
         __syncthreads();
     }
 
     // ---- q and k of the block's tokens, normalised (src/cpu/deltanet.rs:133-146), as hi and lo parts ----
     {
-        // thread (token t, part): the 8-value pieces part, part + 4, part + 8, part + 12 of the token's q and k, so
-        // that the four threads of a token read 128 bytes in a row with every pair of loads
-        const uint32_t t = tid >> 2, part = tid & 3, tok = blk * C + t;
-        float4 qv[8], kv[8];
-        float qs = 0.0f, ks = 0.0f;
+        // thread (token t, part): the 8-value pieces part and part + 8 of the token's q and k, so that the eight threads
+        // of a token read 256 bytes in a row with every pair of loads
+        const uint32_t t = tid >> 3, part = tid & 7, tok = blk * C + t;
+        const bool real = tok < a.tokens;
+        float4 qv[4], kv[4];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            qv[i] = kv[i] = make_float4(0, 0, 0, 0);
-            if (CONVOLVE) {
-                const float *row = qk_lds + t * FROW + 8 * (part + 4 * (i >> 1)) + 4 * (i & 1);
-                qv[i] = *reinterpret_cast<const float4 *>(row);
-                kv[i] = *reinterpret_cast<const float4 *>(row + K_DIM);
-            } else if (tok < a.tokens) {
-                const float *row = a.mixed + size_t(tok) * a.channels + khd * K_DIM + 8 * (part + 4 * (i >> 1)) + 4 * (i & 1);
+        for (int i = 0; i < 4; i++) {
+            const uint32_t at = 8 * (part + 8 * (i >> 1)) + 4 * (i & 1);
+            if constexpr (CONVOLVE) {
+                qv[i] = *reinterpret_cast<const float4 *>(qk_lds + t * FROW + at);
+                kv[i] = *reinterpret_cast<const float4 *>(qk_lds + t * FROW + K_DIM + at);
+            } else {
+                const float *row = a.mixed + size_t(min(tok, a.tokens - 1)) * a.channels + khd * K_DIM + at;
                 qv[i] = *reinterpret_cast<const float4 *>(row);
                 kv[i] = *reinterpret_cast<const float4 *>(row + key_size);
             }
+        }
+        if constexpr (!CONVOLVE) gates();
+        float qs = 0.0f, ks = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
             qs += qv[i].x * qv[i].x + qv[i].y * qv[i].y + qv[i].z * qv[i].z + qv[i].w * qv[i].w;
             ks += kv[i].x * kv[i].x + kv[i].y * kv[i].y + kv[i].z * kv[i].z + kv[i].w * kv[i].w;
         }
-        if (CONVOLVE) __syncthreads();  // the f32 q and k are read: the images go over them
-        qs = group_reduce<4>(qs, SumOp());
-        ks = group_reduce<4>(ks, SumOp());
-        const bool real = tok < a.tokens;
-        // (q's factor 1 / sqrt(128) is applied to the output: at unit length the lo parts stay clear of the f16 underflow)
-        const float qi = real ? __builtin_amdgcn_rsqf(qs + a.eps) : 0.0f;
-        const float ki = real ? __builtin_amdgcn_rsqf(ks + a.eps) : 0.0f;
+        if constexpr (CONVOLVE) __syncthreads();  // the f32 q and k are read: the images go over them
+        qs = group_reduce<8>(qs, SumOp());
+        ks = group_reduce<8>(ks, SumOp());
+        // (q's factor 1 / sqrt(128) is applied to the output: at unit length the lo parts stay clear of the f16 underflow;
+        // a token past the end: zeros, whatever was loaded)
+        const float qi = __builtin_amdgcn_rsqf(qs + a.eps), ki = __builtin_amdgcn_rsqf(ks + a.eps);
 #pragma unroll
-        for (int i = 0; i < 8; i += 2) {
+        for (int i = 0; i < 4; i += 2) {
             half8 a_qh, a_ql, a_kh, a_kl;
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const float4 qq = qv[i + e / 4], kk = kv[i + e / 4];
-                const float qf = (e % 4 == 0 ? qq.x : e % 4 == 1 ? qq.y : e % 4 == 2 ? qq.z : qq.w) * qi;
-                const float kf = (e % 4 == 0 ? kk.x : e % 4 == 1 ? kk.y : e % 4 == 2 ? kk.z : kk.w) * ki;
+                const float qf = real ? (e % 4 == 0 ? qq.x : e % 4 == 1 ? qq.y : e % 4 == 2 ? qq.z : qq.w) * qi : 0.0f;
+                const float kf = real ? (e % 4 == 0 ? kk.x : e % 4 == 1 ? kk.y : e % 4 == 2 ? kk.z : kk.w) * ki : 0.0f;
                 _Float16 hi, lo;
                 split2(qf, hi, lo);
                 a_qh[e] = hi, a_ql[e] = lo;
                 split2(kf, hi, lo);
                 a_kh[e] = hi, a_kl[e] = lo;
             }
-            const int at = t * KROW + 8 * (part + 2 * i);  // piece part + 4 (i / 2): key dims 32 (i / 2) + 8 part ..
+            const uint32_t piece = part + 4 * i;  // key dims 8 piece ..: k-step piece / 4, lane group piece % 4 of an operand
+            const int at = t * KROW + 8 * piece;
             *reinterpret_cast<half8 *>(kh + at) = a_kh, *reinterpret_cast<half8 *>(kl + at) = a_kl;
             *reinterpret_cast<half8 *>(qh + at) = a_qh, *reinterpret_cast<half8 *>(ql + at) = a_ql;
             if (writer) {
-                // operand (wave t / 16, k-step i / 2), lane (n = t % 16, j = part): a wave's store is one kilobyte in a row
-                unsigned char *g = ws_k + ((((t >> 4) * 4 + (i >> 1)) * 64 + part * 16 + (t & 15)) * 16);
+                // operand (wave t / 16, k-step), lane (n = t % 16, j): eight tokens in a row are whole lines
+                unsigned char *g = ws_k + ((((t >> 4) * 4 + (piece >> 2)) * 64 + (piece & 3) * 16 + (t & 15)) * 16);
                 *reinterpret_cast<half8 *>(g) = a_kh, *reinterpret_cast<half8 *>(g + K_GL) = a_kl;
                 *reinterpret_cast<half8 *>(g + 2 * K_GL) = a_qh, *reinterpret_cast<half8 *>(g + 3 * K_GL) = a_ql;
             }
         }
     }
-    // ---- the gates of head h0 + wave: c_t = sum of log g up to t, beta_t (tokens past the end: g = 1, beta = 0) ----
-    if (wave < G) {
-        const uint32_t tok = blk * C + lane, h = h0 + wave;
-        float lg = 0.0f, beta = 0.0f;
-        if (tok < a.tokens) {
-            float g;
-            fast_gates(a.a[size_t(tok) * a.v_heads + h] + a.dt_bias[h], __expf(a.a_log[h]), a.b[size_t(tok) * a.v_heads + h], g, beta, &lg);
-        }
-        // inclusive sum over the 64 lanes
-        double c = lg;
-#pragma unroll
-        for (int d = 1; d < 64; d *= 2) {
-            const double up = __shfl_up(c, d, 64);
-            if (int(lane) >= d) c += up;
-        }
-        cum_lds(wave)[lane] = c, beta_lds(wave)[lane] = beta;
-        const double last = __shfl(c, 63, 64);
-        float *gam = reinterpret_cast<float *>(ws_v(wave) + 4 * T_GL);
-        gam[lane] = __expf(float(c)), gam[C + lane] = __expf(float(last - c));
-    }
     __syncthreads();
 
-    // ---- k . k and q . k: rows 16 wave .. + 15, the column tiles at and below the diagonal ----
-    floatx4 gk[4], gq[4];
+    // ---- k . k (first team) and q . k (second): wave tw of a team takes the rows t = 16 tw + .., the tiles of 16 columns s
+    // at and below the diagonal, transposed: lane (n, j) holds columns s = 16 nt + 4j + i of row t = 16 tw + n ----
+    const uint32_t team = wave >> 2, tw = wave & 3;
+    floatx4 prod[4];
+    {
+        const _Float16 *rh = team == 0 ? kh : qh, *rl = team == 0 ? kl : ql;
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-        gk[nt] = gq[nt] = floatx4{0, 0, 0, 0};
-        if (nt <= int(wave)) {
+        for (int nt = 0; nt < 4; nt++) {
+            prod[nt] = floatx4{0, 0, 0, 0};
+            if (nt <= int(tw)) {
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                const int ao = (16 * wave + n) * KROW + 32 * ks + 8 * j, bo = (16 * nt + n) * KROW + 32 * ks + 8 * j;
-                const half8 bh = *reinterpret_cast<const half8 *>(kh + bo), bl = *reinterpret_cast<const half8 *>(kl + bo);
-                gk[nt] = mma3(*reinterpret_cast<const half8 *>(kh + ao), *reinterpret_cast<const half8 *>(kl + ao), bh, bl, gk[nt]);
-                gq[nt] = mma3(*reinterpret_cast<const half8 *>(qh + ao), *reinterpret_cast<const half8 *>(ql + ao), bh, bl, gq[nt]);
+                for (int ks = 0; ks < 4; ks++) {
+                    const int to = (16 * tw + n) * KROW + 32 * ks + 8 * j, so = (16 * nt + n) * KROW + 32 * ks + 8 * j;
+                    prod[nt] = mma3(*reinterpret_cast<const half8 *>(kh + so), *reinterpret_cast<const half8 *>(kl + so),
+                                    *reinterpret_cast<const half8 *>(rh + to), *reinterpret_cast<const half8 *>(rl + to), prod[nt]);
+                }
             }
         }
     }
     __syncthreads();  // the images are read: A and M go over them
 
-    // C layout: lane (n, j) holds column s = 16 nt + n of rows t = 16 wave + 4j + i
-#pragma unroll
+    // ---- A and M.  What lies above the diagonal inside the 32 x 32 blocks is zero; the block above them is not read by
+    // anybody and not written. ----
+#pragma unroll 1
     for (int hh = 0; hh < G; hh++) {
+        const uint32_t t = 16 * tw + n;
+        const double ct = cum_lds(hh)[t];
+        const float beta_t = beta_lds(hh)[t];
 #pragma unroll
         for (int nt = 0; nt < 4; nt++) {
-            const uint32_t s = 16 * nt + n;
-            const double cs = cum_lds(hh)[s];
+            if (nt > int(tw | 1)) continue;  // (tile rows 2i and 2i + 1 end with column tile 2i + 1)
+            const uint32_t s0 = 16 * nt + 4 * j;
+            float x[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const uint32_t t = 16 * wave + 4 * j + i;
-                const float decay = s <= t ? __expf(float(cum_lds(hh)[t] - cs)) : 0.0f;
-                const float at_s = s < t ? beta_lds(hh)[t] * decay * gk[nt][i] : 0.0f;
-                if ((nt >> 1) == int(wave >> 1)) {  // a diagonal 32 x 32 block, zeros above the diagonal included
-                    diag_lds(hh, nt >> 1)[(t & 31) * DROW + (s & 1) * 16 + ((s & 31) >> 1)] = at_s;
-                } else if (nt < 2) {  // the block below the diagonal, as an MFMA operand
-                    _Float16 hi, lo;
-                    split2(at_s, hi, lo);
-                    half_img(hh, L::LBA_OFF)[(t - 32) * HROW + s] = hi, half_img(hh, L::LBA_OFF)[32 * HROW + (t - 32) * HROW + s] = lo;
+                const uint32_t s = s0 + i;
+                const float decayed = __expf(float(ct - cum_lds(hh)[s])) * prod[nt][i];
+                x[i] = team == 0 ? (s < t ? beta_t * decayed : 0.0f) : (s <= t ? decayed : 0.0f);
+            }
+            if (team == 0 && (nt >> 1) == int(tw >> 1)) {  // a diagonal 32 x 32 block of A
+                *reinterpret_cast<floatx4 *>(diag_lds(hh, nt >> 1) + (t & 31) * DROW + (s0 & 31)) = floatx4{x[0], x[1], x[2], x[3]};
+            } else {  // M | the block of A below the diagonal, as an MFMA operand
+                half4 hi, lo;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    _Float16 h, l;
+                    split2(x[i], h, l);
+                    hi[i] = h, lo[i] = l;
                 }
-                _Float16 hi, lo;
-                split2(decay * gq[nt][i], hi, lo);
-                m_lds(hh)[t * TROW + s] = hi, m_lds(hh)[C * TROW + t * TROW + s] = lo;
+                _Float16 *dst = team == 0 ? half_img(hh, L::LBA_OFF) + (t - 32) * HROW + s0 : m_lds(hh) + t * TROW + s0;
+                *reinterpret_cast<half4 *>(dst) = hi;
+                *reinterpret_cast<half4 *>(dst + (team == 0 ? 32 * HROW : C * TROW)) = lo;
             }
         }
     }
     __syncthreads();
-    // A staged matrix leaves in operand order, 16 bytes per piece: piece (part hi | lo, wave w, k-step ks, lane (n, j))
-    // is row 16 w + n, columns 32 ks + 8j .. of the part's image
-    auto leave = [&](int hh, unsigned char *dst) {
-        for (uint32_t i = tid; i < 2 * T_GL / 16; i += 256) {
-            const uint32_t part = i >> 9, w = (i >> 7) & 3, ks = (i >> 6) & 1, nn = i & 15, jj = (i >> 4) & 3;
-            reinterpret_cast<u32x4 *>(dst)[i] = *reinterpret_cast<const u32x4 *>(m_lds(hh) + part * C * TROW + (16 * w + nn) * TROW + 32 * ks + 8 * jj);
+    // A staged matrix leaves in operand order, 16 bytes per piece, by `threads` threads: piece (part hi | lo, operand, lane
+    // (n, j)) is row 16 w + n, columns 32 ks + 8j .. of the part's image; the operands are (w, ks) = (0, 0), (1, 0), (2, 0),
+    // (2, 1), (3, 0), (3, 1): nobody reads the other two.
+    auto leave = [&](int hh, unsigned char *dst, uint32_t thread, uint32_t threads) {
+        for (uint32_t i = thread; i < 2 * 6 * 64; i += threads) {
+            const uint32_t part = i >= 6 * 64 ? 1 : 0, op = (i >> 6) - 6 * part, w = op < 2 ? op : op < 4 ? 2 : 3, ks = op < 2 ? 0 : op & 1, nn = i & 15, jj = (i >> 4) & 3;
+            reinterpret_cast<u32x4 *>(dst)[part * (T_GL / 16) + (w * 2 + ks) * 64 + (i & 63)] =
+                *reinterpret_cast<const u32x4 *>(m_lds(hh) + part * C * TROW + (16 * w + nn) * TROW + 32 * ks + 8 * jj);
         }
     };
-#pragma unroll
-    for (int hh = 0; hh < G; hh++) leave(hh, ws_v(hh) + 2 * T_GL);
 
     // ---- T = (I + A)^-1 diag(beta), in 32 x 32 blocks: with L = I + A = [[L_AA, 0], [L_BA, L_BB]],
     //     T_AA = L_AA^-1 diag(beta_A),  T_BB = L_BB^-1 diag(beta_B),  T_BA = -L_BB^-1 (L_BA T_AA).
-    // The diagonal blocks by forward substitution, one wave per (head, block): lane (column c, q) solves
-    // x_t = [t = c] - sum_{s < t} A_ts x_s, lane group q keeps x_s of s = 2m + q in slot m and adds up those s.
+    // The diagonal blocks by forward substitution, one wave per head: lane (column c, block) solves
+    // x_t = [t = c] - sum_{s < t} A_ts x_s and puts its column over A, which the wave has read.  The second team stores M.
     // The block below the diagonal: two products on the matrix cores. ----
+    if (wave < G) {
+        const uint32_t c = lane & 31;
+        float *ad = diag_lds(wave, lane >> 5);
+        float x[32];
+#pragma unroll
+        for (int t = 0; t < 32; t++) {
+            floatx4 part4 = {0, 0, 0, 0};  // (four chains of sums instead of one of up to 31)
+#pragma unroll
+            for (int s4 = 0; 4 * s4 < t; s4++) {
+                const floatx4 av = *reinterpret_cast<const floatx4 *>(ad + t * DROW + 4 * s4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if (4 * s4 + e < t) part4[e] += av[e] * x[4 * s4 + e];
+                }
+            }
+            x[t] = (uint32_t(t) == c ? 1.0f : 0.0f) - ((part4[0] + part4[1]) + (part4[2] + part4[3]));
+        }
+#pragma unroll
+        for (int t = 0; t < 32; t++) ad[t * DROW + c] = x[t];  // (behind the loop: in it, the next row's reads would wait for x_t)
+    } else if (team == 1) {
+#pragma unroll
+        for (int hh = 0; hh < G; hh++) leave(hh, ws_v(hh) + 2 * T_GL, tid - 256, 256);
+    }
+    __syncthreads();  // M has left: T goes over it
+    for (uint32_t i = tid; i < G * 2 * 32 * 8; i += PREP_THREADS) {
+        // four columns c .. of row t of a diagonal block
+        const uint32_t c = (i & 7) * 4, t = (i >> 3) & 31, half = (i >> 8) & 1, hh = G == 2 ? i >> 9 : 0;
+        const floatx4 x = *reinterpret_cast<const floatx4 *>(diag_lds(hh, half) + t * DROW + c);
+        const floatx4 beta = *reinterpret_cast<const floatx4 *>(beta_lds(hh) + 32 * half + c);
+        half4 th, tl, xh, xl;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            _Float16 h, l;
+            split2(x[e] * beta[e], h, l);
+            th[e] = h, tl[e] = l;
+            split2(x[e], h, l);
+            xh[e] = h, xl[e] = l;
+        }
+        _Float16 *dst = m_lds(hh) + (32 * half + t) * TROW + 32 * half + c;
+        *reinterpret_cast<half4 *>(dst) = th, *reinterpret_cast<half4 *>(dst + C * TROW) = tl;
+        if (half) {
+            _Float16 *xd = half_img(hh, L::XBB_OFF) + t * HROW + c;
+            *reinterpret_cast<half4 *>(xd) = xh, *reinterpret_cast<half4 *>(xd + 32 * HROW) = xl;
+        }
+    }
+    __syncthreads();
     {
-        const uint32_t hs = G == 2 ? wave >> 1 : 0, half = wave & 1;  // the wave's head and diagonal block
-        const bool solver = G == 2 || wave < 2;
-        const uint32_t c = lane & 31, q = lane >> 5;
-        float x[16];
-#pragma unroll
-        for (int m = 0; m < 16; m++) x[m] = 0.0f;
-        if (solver) {
-            const float *ad = diag_lds(hs, half) + q * 16;
-#pragma unroll
-            for (int t = 0; t < 32; t++) {
-                floatx4 part4 = {0, 0, 0, 0};  // (four chains of sums instead of one of up to 16)
-#pragma unroll
-                for (int m4 = 0; 8 * m4 < t; m4++) {  // s = 2m + q < t needs m <= (t - 1) / 2
-                    const floatx4 av = *reinterpret_cast<const floatx4 *>(ad + t * DROW + 4 * m4);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) part4[e] += av[e] * x[4 * m4 + e];
-                }
-                const float sum = across_rows<32, 64>((part4[0] + part4[1]) + (part4[2] + part4[3]), SumOp());
-                const float xt = (uint32_t(t) == c ? 1.0f : 0.0f) - sum;
-                if (q == uint32_t(t & 1)) x[t >> 1] = xt;
-            }
-        }
-        __syncthreads();  // M has left: T goes over it
-        if (solver) {
-            const float bc = beta_lds(hs)[32 * half + c];
-            _Float16 *th = m_lds(hs), *tl = th + C * TROW;
-#pragma unroll
-            for (int m = 0; m < 16; m++) {
-                const uint32_t t = 2 * m + q;
-                _Float16 hi, lo;
-                split2(x[m] * bc, hi, lo);
-                th[(32 * half + t) * TROW + 32 * half + c] = hi, tl[(32 * half + t) * TROW + 32 * half + c] = lo;
-                if (half == 0) {
-                    th[t * TROW + 32 + c] = (_Float16)0.0f, tl[t * TROW + 32 + c] = (_Float16)0.0f;  // nothing above the diagonal
-                } else {
-                    split2(x[m], hi, lo);
-                    half_img(hs, L::XBB_OFF)[t * HROW + c] = hi, half_img(hs, L::XBB_OFF)[32 * HROW + t * HROW + c] = lo;
-                }
-            }
-        }
-        __syncthreads();
-        // W = L_BA T_AA and then T_BA = -L_BB^-1 W: a wave takes 16 rows (two column tiles of its head; with one
-        // head, one tile).  The right operands are read by column out of row-major images.
-        const uint32_t r = wave & 1, la = lane & 3, le = (lane >> 2) & 3;
+        // W = L_BA T_AA and then T_BA = -L_BB^-1 W: a wave takes one 16 x 16 tile (rows 16 r, columns 16 ct) of its head,
+        // as its transpose.  The right operands are read by column out of row-major images.
+        const uint32_t hs = wave >> 2, r = (wave >> 1) & 1, ct = wave & 1, la = lane & 3, le = (lane >> 2) & 3;
+        const bool takes = hs < G;
         const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(lds));
-        floatx4 w[2];
-#pragma unroll
-        for (int ct = 0; ct < 2; ct++) {
-            if (G == 1 && ct != int(wave >> 1)) continue;
-            const int ao = (16 * r + n) * HROW + 8 * j;
+        const int ao = (16 * r + n) * HROW + 8 * j, at = (16 * r + n) * HROW + 16 * ct + 4 * j;
+        if (takes) {
             half8 bh, bl;
             read_by_column(lds0 + L::M_OFF + hs * L::M_BYTES + ((8 * j + le) * TROW + 16 * ct + 4 * la) * 2, C * TROW * 2, 4 * TROW * 2, bh, bl);
-            w[ct] = mma3(*reinterpret_cast<const half8 *>(half_img(hs, L::LBA_OFF) + ao),
-                         *reinterpret_cast<const half8 *>(half_img(hs, L::LBA_OFF) + 32 * HROW + ao), bh, bl, floatx4{0, 0, 0, 0});
-        }
-        // (the diagonal blocks were last read before the barrier above)
-#pragma unroll
-        for (int ct = 0; ct < 2; ct++) {
-            if (G == 1 && ct != int(wave >> 1)) continue;
+            const floatx4 w = mma3(bh, bl, *reinterpret_cast<const half8 *>(half_img(hs, L::LBA_OFF) + ao),
+                                   *reinterpret_cast<const half8 *>(half_img(hs, L::LBA_OFF) + 32 * HROW + ao), floatx4{0, 0, 0, 0});
+            // (the inverses of the diagonal blocks were last read before the barrier above)
+            half4 wh, wl;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                _Float16 hi, lo;
-                split2(w[ct][i], hi, lo);
-                const int at = (16 * r + 4 * j + i) * HROW + 16 * ct + n;
-                half_img(hs, L::W_OFF)[at] = hi, half_img(hs, L::W_OFF)[32 * HROW + at] = lo;
+                _Float16 h, l;
+                split2(w[i], h, l);
+                wh[i] = h, wl[i] = l;
             }
+            *reinterpret_cast<half4 *>(half_img(hs, L::W_OFF) + at) = wh, *reinterpret_cast<half4 *>(half_img(hs, L::W_OFF) + 32 * HROW + at) = wl;
         }
         __syncthreads();
-#pragma unroll
-        for (int ct = 0; ct < 2; ct++) {
-            if (G == 1 && ct != int(wave >> 1)) continue;
-            const int ao = (16 * r + n) * HROW + 8 * j;
+        if (takes) {
             half8 bh, bl;
             read_by_column(lds0 + hs * L::HEAD_BYTES + L::W_OFF + ((8 * j + le) * HROW + 16 * ct + 4 * la) * 2, 32 * HROW * 2, 4 * HROW * 2, bh, bl);
-            const floatx4 tba = mma3(*reinterpret_cast<const half8 *>(half_img(hs, L::XBB_OFF) + ao),
-                                     *reinterpret_cast<const half8 *>(half_img(hs, L::XBB_OFF) + 32 * HROW + ao), bh, bl, floatx4{0, 0, 0, 0});
-            _Float16 *th = m_lds(hs), *tl = th + C * TROW;
+            const floatx4 tba = mma3(bh, bl, *reinterpret_cast<const half8 *>(half_img(hs, L::XBB_OFF) + ao),
+                                     *reinterpret_cast<const half8 *>(half_img(hs, L::XBB_OFF) + 32 * HROW + ao), floatx4{0, 0, 0, 0});
+            half4 th, tl;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                _Float16 hi, lo;
-                split2(-tba[i], hi, lo);
-                const int at = (32 + 16 * r + 4 * j + i) * TROW + 16 * ct + n;
-                th[at] = hi, tl[at] = lo;
+                _Float16 h, l;
+                split2(-tba[i], h, l);
+                th[i] = h, tl[i] = l;
             }
+            _Float16 *dst = m_lds(hs) + (32 + 16 * r + n) * TROW + 16 * ct + 4 * j;
+            *reinterpret_cast<half4 *>(dst) = th, *reinterpret_cast<half4 *>(dst + C * TROW) = tl;
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int hh = 0; hh < G; hh++) leave(hh, ws_v(hh));
+    for (int hh = 0; hh < G; hh++) leave(hh, ws_v(hh), tid, PREP_THREADS);
 }
 
 // ds_read_b64_tr_b16 of the 8 bytes at `at` in LDS
@@ -863,16 +914,18 @@ int run_deltanet_chunk(hipStream_t stream, const float *mixed, const float *a, c
     const bool two_heads = p.v_heads == 2 * p.k_heads;
     LaunchList *list = recording();
     float *conv_out = nullptr;
-    // The conv inside: while the workgroups are all on the machine at once, two to a CU.  Past that the conv's own kernel
-    // is the faster one, whose many waves keep the memory busy (whole chunk, us, inside against apart: 1000 tokens 76.8
-    // and 79, 2048 125 and 131; 3000 209 and 199, 4096 290 and 280).
-    const bool conv_inside = two_heads && p.v_dim == CONV_V && nblocks * p.k_heads <= 2 * cu_count();
+    // The conv inside: while every workgroup, the blocks' and the values', has a CU to itself.  Where they share one, a
+    // block's chain of phases is held up by the conv beside it, and the conv's own launch is the better one (whole chunk,
+    // us, inside against apart: 200 tokens 34.2 and 35.3, 333 38.2 and 39.4, 512 43.4 and 45.5; 750 59.5 and 55.6, 1000 70.9
+    // and 66.6, 2047 126 and 120).
+    const uint32_t columns = (p.v_heads * p.v_dim / 4 + PREP_THREADS - 1) / PREP_THREADS, value_groups = columns * ((p.tokens + CONV_VALUES - 1) / CONV_VALUES);
+    const bool conv_inside = two_heads && p.v_dim == CONV_V && nblocks * p.k_heads + value_groups <= cu_count();
     if (conv_inside && list && take_conv(*list, args, conv_out)) {
-        launch(deltanet_chunk_prepare_kernel<2, true>, dim3(nblocks, p.k_heads), 256, PrepLds<2>::BYTES, stream, args, conv_out);
+        launch(deltanet_chunk_prepare_kernel<2, true>, dim3(nblocks + (value_groups + p.k_heads - 1) / p.k_heads, p.k_heads), PREP_THREADS, PrepLds<2>::BYTES, stream, args, conv_out);
     } else if (two_heads) {
-        launch(deltanet_chunk_prepare_kernel<2, false>, dim3(nblocks, p.k_heads), 256, PrepLds<2>::BYTES, stream, args, conv_out);
+        launch(deltanet_chunk_prepare_kernel<2, false>, dim3(nblocks, p.k_heads), PREP_THREADS, PrepLds<2>::BYTES, stream, args, conv_out);
     } else {
-        launch(deltanet_chunk_prepare_kernel<1, false>, dim3(nblocks, p.v_heads), 256, PrepLds<1>::BYTES, stream, args, conv_out);
+        launch(deltanet_chunk_prepare_kernel<1, false>, dim3(nblocks, p.v_heads), PREP_THREADS, PrepLds<1>::BYTES, stream, args, conv_out);
     }
     launch(deltanet_chunk_chain_kernel, dim3(p.v_dim / DV * p.v_heads), 512, ChainLds::BYTES, stream, args);
     return SAETTA_OK;

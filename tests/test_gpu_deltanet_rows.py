@@ -319,6 +319,13 @@ def test_a_plan_of_conv_and_chunk_gives_what_the_calls_give(k_heads, v_heads, v_
     lib.saetta_plan_free(made)
 
 
+@pytest.mark.parametrize("tokens,launches", [(512, 3), (513, 4)])
+def test_the_largest_chunk_with_its_conv_inside_and_the_next(tokens, launches):
+    # 8 blocks x 16 key heads and 2 x 64 tiles of values are 256 workgroups, one to a CU of an MI355X
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        test_a_plan_of_conv_and_chunk_gives_what_the_calls_give(16, 32, 128, tokens, False, launches)
+
+
 @pytest.mark.parametrize("tokens", [8, 9, 11, 12, 13])
 def test_conv_of_four_channels_a_thread_at_the_edges_of_its_tiles(tokens):
     # from 9 tokens on, in tiles of 4; the last tile has 1 to 4 tokens
