@@ -53,6 +53,8 @@
 //                                move the codes into LDS (global_load_lds), a whole share at once
 //                                with the keys requested first (longer shares: rounds in alternate
 //                                halves of LDS), the waves meeting through counters in LDS
+//   attention_partial_kernel_h   three to eight query rows over a half cache: loader waves, a wave per tile
+//                                (decode_half_rows.hpp)
 //   attention_reduce_kernel      the merge of the splits and the gate
 // Which one runs is decided in run_attention from the launch arguments alone, so that the partial
 // and the reduce stage of a step agree on the number of splits.
@@ -2829,6 +2831,8 @@ __global__ __launch_bounds__((KeysFirst<BITS, M>::THREADS_)) void attention_toke
     attention_partial_s_body<BITS, M, true>(t.a, &t.prep);
 }
 
+#include "decode_half_rows.hpp"
+
 // Merges the splits of one (q head, row): weights 2^(m_c - M), then the gate
 // (reference: attention_reduce / attention_reduce_rows,
 // kernels/attention.metal:367-409, kernels/attention_rows.metal:296-342).
@@ -2952,6 +2956,13 @@ uint32_t splits_for(uint32_t capacity, uint32_t wanted) {
 // than one round in alternate halves of LDS: 13.4 against 14.1 us at 40k for the ring of four 64-token slots
 // that served there before, 28.3 against 29.7 at 150k, 4-bit, for the two-workgroups-per-CU kernel).
 constexpr uint32_t KEYS_FIRST_FROM = 24 * 1024;
+// Rows over a half cache that take the kernel with loader waves, at any capacity (figures there): two rows are one computing
+// wave, which the register kernel's four are ahead of.
+constexpr uint32_t HALF_ROWS_FROM = 3;
+// Five rows and more over halves take the store in from this capacity on.  (One launch is ahead in smaller caches too, 6 rows
+// at 300 tokens of 8192 13.7 -> 12.5 us a layer, at 30000 of 32768 29.3 -> 26.7; but there the store is a launch of its own as the
+// tests have it.)
+constexpr uint32_t MANY_NEW_ROWS_FROM = 48 * 1024;
 
 // token: with the step before the scores taken in (nullptr: not)
 template <int BITS, int TILES, bool PACKED>
@@ -2959,6 +2970,14 @@ void launch_partial(hipStream_t stream, const PartialArgs &a, bool one_per_cu, b
     void (*kernel)(PartialArgs);
     int lds_bytes;
     const dim3 grid(a.nsplits, a.kv_heads);
+    if constexpr (BITS == 16 && !PACKED && TILES >= 2) {
+        if (keys_first) {
+            using W = HalfRows<TILES>;
+            if (token) launch(attention_token_kernel_h<TILES>, dim3(token->a.nsplits - 1 + a.rows, a.kv_heads), W::THREADS_, W::LDS_BYTES, stream, *token);
+            else launch(attention_partial_kernel_h<TILES>, grid, W::THREADS_, W::LDS_BYTES, stream, a);
+            return;
+        }
+    }
     if constexpr (BITS != 16) {
         if (keys_first) {
             auto launch_rows = [&](auto rows_c) {
@@ -3053,13 +3072,18 @@ bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const fl
         }
     }
     token = TokenArgs{a, prep, SAETTA_GQA_GROUP};
-    if (!keys_first) {
+    const uint32_t room = MAX_SPLITS / 2;  // workgroups of a kv head, one to a CU
+    if (bits == 16 && keys_first) {
+        // a workgroup per new row, for which a full context gives up CUs (two rows to one: 6 rows at 57123 tokens 36.2 against
+        // 35.5 us a layer)
+        if (a.rows > NEW_ROWS && a.capacity < MANY_NEW_ROWS_FROM) return false;
+        token.a.nsplits = min(a.nsplits, room - a.rows + 1);
+    } else if (!keys_first) {
         // more rows than four: the workgroups of the new rows need longer than the launch takes (18.7 against 18.2 us per
         // layer at 8 rows and 300 tokens, f16)
         if (a.rows > NEW_ROWS) return false;
         // as many splits as before, one of them the new tokens'.  Their workgroups beside the context's: two heads to one
         // while all fit one to a CU, a whole row to one where the context gives up CUs for them.
-        const uint32_t room = MAX_SPLITS / 2;
         if (a.nsplits - 1 + 4 * a.rows <= room) token.new_heads = 2;
         else if (a.nsplits - 1 + a.rows > room) token.a.nsplits = room - a.rows + 1;
     }
@@ -3094,7 +3118,8 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
     // One to four rows over codes in a cache of 24k tokens and more go to the kernel with loader waves, a
     // one-workgroup-per-CU kernel at every length: a share of up to 17 blocks (the kernel sees the length
     // when it runs: a step at 32k tokens is one round in a cache of any size) is one round, a longer one
-    // rounds of 8 blocks (three and four rows: 12).  SAETTA_STAGE_NO_LOADERS keeps to the register kernels (the caller's choice of
+    // rounds of 8 blocks (three and four rows: 12).  Three rows and more over halves go to their kernel
+    // with loader waves in a cache of any size.  SAETTA_STAGE_NO_LOADERS keeps to the register kernels (the caller's choice of
     // kernel family, as DecodeAttention.kernel is in the reference, src/attention.rs:36-38).
     // The register kernels: one workgroup per CU (half as many splits, each twice as long) or two.  Two
     // rows and more and a half cache need the whole register file anyway; one row over codes fits two
@@ -3102,7 +3127,8 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
     // many partials is worth more (measured: 19.4 against 20.6 us per layer at 32k, 28.3 against 29.7 at
     // 64k, but 44 against 35 at 146k, 4-bit).  Both stages of a call derive the same number from the same arguments; where
     // a plan's reduce stage makes a token step of the launches before it, the number is the token step's.
-    const bool keys_first = rows <= 4 && bits != 16 && capacity >= KEYS_FIRST_FROM && !(stages & SAETTA_STAGE_NO_LOADERS);
+    const bool loaders = bits == 16 ? rows >= HALF_ROWS_FROM : rows <= 4 && capacity >= KEYS_FIRST_FROM;
+    const bool keys_first = loaders && !(stages & SAETTA_STAGE_NO_LOADERS);
     const bool one_per_cu = rows >= 2 || bits == 16 || capacity <= 80 * 1024 || keys_first;
     if (one_per_cu && nsplits > MAX_SPLITS / 2) nsplits = MAX_SPLITS / 2;
     const PartialArgs a{q,     kdata,    vdata,    ks,    kz,   vs,      vz,   part_o, part_ml,
@@ -3154,6 +3180,13 @@ int raise_lds_keys_first() {
     return int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_partial_kernel_s<BITS, M>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, KeysFirst<BITS, M>::LDS_BYTES));
 }
+template <int TILES>
+int raise_lds_half_rows() {
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_token_kernel_h<TILES>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         HalfRows<TILES>::LDS_BYTES))) return rc;
+    return int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_partial_kernel_h<TILES>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   HalfRows<TILES>::LDS_BYTES));
+}
 template <int BITS>
 int raise_lds_of_bits() {
     if (int rc = raise_lds<BITS, 1, true, ITB_ONE_PER_CU>(attention_partial_kernel_p<BITS>)) return rc;
@@ -3186,6 +3219,9 @@ int setup_decode() {
     if (int rc = raise_lds_keys_first<4, 2>()) return rc;
     if (int rc = raise_lds_keys_first<4, 3>()) return rc;
     if (int rc = raise_lds_keys_first<4, 4>()) return rc;
+    if (int rc = raise_lds_half_rows<2>()) return rc;
+    if (int rc = raise_lds_half_rows<3>()) return rc;
+    if (int rc = raise_lds_half_rows<4>()) return rc;
     if (int rc = raise_lds_of_bits<8>()) return rc;
     if (int rc = raise_lds_of_bits<4>()) return rc;
     if (int rc = raise_lds_of_bits<16>()) return rc;

@@ -353,6 +353,36 @@ def test_three_and_four_tiles_of_query_rows_at_the_edges_of_a_step(kind, m):
         assert worst < MAX_ABS_F64, (tokens, worst)
 
 
+@pytest.mark.parametrize("m", [3, 4, 6, 8])
+@pytest.mark.parametrize("step", [0.02, 0.16])
+def test_rows_over_halves_follow_a_growing_maximum(step, m):
+    # One split, slots of 32 tokens in four places: fewer slots than places, one more, several times around.  The scores
+    # grow along the context by 0.64 and 5 (log2) a slot, so that a row's maximum moves now and then, or with every slot;
+    # one q head in two sees them fall instead.  The rows past the context are poisoned.  q's hi and lo parts give a score
+    # 2^-22 of its magnitude as an error, which a probability takes over as a relative one: the largest score, ln 2 * step *
+    # tokens, is up to 71 here, and the bound grows with it (two of these errors between two tokens).
+    rng = np.random.default_rng(5300 + m)
+    capacity = 640
+    k = (0.3 * rng.standard_normal((capacity, KV, D))).astype(np.float32)
+    k[:, :, 0] = step * np.arange(capacity)[:, None]
+    k = k.reshape(capacity, VALUES)
+    v = rng.standard_normal((capacity, VALUES)).astype(np.float32)
+    q = (0.3 * rng.standard_normal((m, H, D))).astype(np.float32)
+    q[:, :, 0] = np.where(np.arange(H) % 2, -1.0, 1.0) * 16 / np.log2(np.e)
+    qg = rng.standard_normal((m, H, 2 * D)).astype(np.float32)
+    rows = saetta.AttentionRows(H, KV, capacity, m)
+    rows.splits = 1
+    for tokens in [m, 33, 97, 130, 161, 500, 640]:
+        pos = tokens - m
+        kc, vc, kf, vf = cache_pair(k[:tokens], v[:tokens], saetta.KvBits.Half, capacity, poison=True)
+        out = torch.full((m, H, D), float("nan"), device="cuda")
+        plan = saetta.Plan()
+        rows.record(plan, m, dev(q), kc, vc, dev(qg), out, [saetta.TokenParams(0, pos + r).as_tensor("cuda") for r in range(m)])
+        plan.build().run()
+        worst = np.abs(host(out) - oracle.rows(q, kf, vf, pos, m, q_and_gate=qg, threads=8, f64=True)).max()
+        assert worst < MAX_ABS_F64 + 2 * 2.0 ** -22 * np.log(2) * step * tokens, (tokens, worst)
+
+
 @pytest.mark.parametrize("splits", [64, 43, 32])
 @pytest.mark.parametrize("kind", [saetta.KvBits.Eight, saetta.KvBits.Four])
 @pytest.mark.parametrize("m", [3, 4])

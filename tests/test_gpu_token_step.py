@@ -84,6 +84,21 @@ def test_fused_step_equals_the_ops_one_by_one(kind, capacity, rows):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), position
 
 
+@pytest.mark.parametrize("rows", [5, 6, 7, 8])
+def test_many_rows_of_a_large_half_cache_take_the_store_in(rows):
+    step = Step(saetta.KvBits.Half, 49152, rows, seed=rows)
+    assert launches(step) == 2
+    built = step.plan.build()
+    for position in (0, 1, 17, 3000, 49152 - rows, 49152 - 1, 49152 + 2):
+        want, got = step.run(step.plan.run_serial, position), step.run(built.run, position)
+        ok = np.isfinite(want[0])
+        assert ok.all() or position > 49152 - rows
+        assert np.array_equal(ok, np.isfinite(got[0])), position
+        assert np.abs(got[0] - want[0])[ok].max(initial=0.0) < 2e-5, position
+        for a, b in zip(got[1:], want[1:]):
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), position
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("capacity", [512, 8192, 40960])
 def test_a_length_of_the_callers_own(kind, capacity):
