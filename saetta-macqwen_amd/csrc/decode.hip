@@ -55,6 +55,8 @@
 //                                halves of LDS), the waves meeting through counters in LDS
 //   attention_partial_kernel_h   three to eight query rows over a half cache: loader waves, a wave per tile
 //                                (decode_half_rows.hpp)
+//   attention_partial_kernel_c   the same over codes: two rows and more in the caches that code_rows names
+//                                (decode_code_rows.hpp)
 //   attention_reduce_kernel      the merge of the splits and the gate
 // Which one runs is decided in run_attention from the launch arguments alone, so that the partial
 // and the reduce stage of a step agree on the number of splits.
@@ -2832,6 +2834,7 @@ __global__ __launch_bounds__((KeysFirst<BITS, M>::THREADS_)) void attention_toke
 }
 
 #include "decode_half_rows.hpp"
+#include "decode_code_rows.hpp"
 
 // Merges the splits of one (q head, row): weights 2^(m_c - M), then the gate
 // (reference: attention_reduce / attention_reduce_rows,
@@ -2959,10 +2962,29 @@ constexpr uint32_t KEYS_FIRST_FROM = 24 * 1024;
 // Rows over a half cache that take the kernel with loader waves, at any capacity (figures there): two rows are one computing
 // wave, which the register kernel's four are ahead of.
 constexpr uint32_t HALF_ROWS_FROM = 3;
-// Five rows and more over halves take the store in from this capacity on.  (One launch is ahead in smaller caches too, 6 rows
+// Five rows and more take the store in, where their kernel has loader waves, from this capacity on.  (One launch is ahead in smaller caches too, 6 rows
 // at 300 tokens of 8192 13.7 -> 12.5 us a layer, at 30000 of 32768 29.3 -> 26.7; but there the store is a launch of its own as the
 // tests have it.)
 constexpr uint32_t MANY_NEW_ROWS_FROM = 48 * 1024;
+
+// Rows over codes that take the kernel with waves of their own (attention_partial_kernel_c), by the cache's capacity; us a
+// layer in a plan, the kernel before it -> this one:
+//   two rows from 40k: 36000 of 65536 21.2 -> 19.9, 57123 26.5 -> 23.7 (4-bit 26.6 -> 21.6; 131000 45.8 -> 31.3); behind where a
+//   share is a single round of the keys-first kernel: 32768 18.1 -> 19.0
+//   three and four rows from 24k: 3 rows, 8-bit, 32768 23.6 -> 22.6, 57123 35.5 -> 27.6; 4 rows, 4-bit, 24400 23.0 -> 23.4, 32768
+//   25.1 -> 24.8, 57123 36.6 -> 29.5, 100000 53.3 -> 39.6; even below, but for 4-bit at 12000: 17.8 -> 18.3, 19.1 -> 19.9
+//   five rows and more: 6 rows, 8-bit, 300 16.8 -> 15.4, 12000 26.9 -> 25.7, 57123 47.1 -> 38; 8 rows 19.3 -> 15.6, 31.6 -> 28, 54.8 ->
+//   42; 5 and 6 rows of 4-bit codes from 28k: 4000 20.9 -> 21.4, 30000 34.8 -> 32.9
+// It is ahead in larger caches still (4 rows, 8-bit, at 150000 tokens 66.5 -> 48.4, 8 rows 107 -> 79), but stops at 64k tokens, 2 to
+// 4 rows of 4-bit codes at 128k: the sums of the codes and of the biases nearly cancel, the more the longer the context, and the
+// order in which 32-bit sums are taken shows as 4e-6 to 8e-6 of the results at 64000 tokens, 1.0e-5 to 1.5e-5 at 131000 (2 to 4
+// rows, 4-bit, 7e-6), where 1e-5 is what results may differ by.
+constexpr bool code_rows(int bits, uint32_t rows, uint32_t capacity) {
+    constexpr uint32_t K = 1024;
+    const uint32_t from = rows >= 7 || (rows >= 5 && bits == 8) ? 0 : rows >= 5 ? 28 * K : rows >= 3 ? 24 * K : 40 * K;
+    const uint32_t to = rows <= 4 && bits == 4 ? 128 * K : 64 * K;
+    return bits != 16 && rows >= 2 && capacity >= from && capacity <= to;
+}
 
 // token: with the step before the scores taken in (nullptr: not)
 template <int BITS, int TILES, bool PACKED>
@@ -2975,6 +2997,14 @@ void launch_partial(hipStream_t stream, const PartialArgs &a, bool one_per_cu, b
             using W = HalfRows<TILES>;
             if (token) launch(attention_token_kernel_h<TILES>, dim3(token->a.nsplits - 1 + a.rows, a.kv_heads), W::THREADS_, W::LDS_BYTES, stream, *token);
             else launch(attention_partial_kernel_h<TILES>, grid, W::THREADS_, W::LDS_BYTES, stream, a);
+            return;
+        }
+    }
+    if constexpr (BITS != 16 && !PACKED) {
+        if (keys_first && code_rows(BITS, a.rows, a.capacity)) {
+            using W = CodeRows<BITS, TILES>;
+            if (token) launch(attention_token_kernel_c<BITS, TILES>, dim3(token->a.nsplits - 1 + a.rows, a.kv_heads), W::THREADS_, W::LDS_BYTES, stream, *token);
+            else launch(attention_partial_kernel_c<BITS, TILES>, grid, W::THREADS_, W::LDS_BYTES, stream, a);
             return;
         }
     }
@@ -3073,7 +3103,7 @@ bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const fl
     }
     token = TokenArgs{a, prep, SAETTA_GQA_GROUP};
     const uint32_t room = MAX_SPLITS / 2;  // workgroups of a kv head, one to a CU
-    if (bits == 16 && keys_first) {
+    if (keys_first && (bits == 16 || code_rows(bits, a.rows, a.capacity))) {
         // a workgroup per new row, for which a full context gives up CUs (two rows to one: 6 rows at 57123 tokens 36.2 against
         // 35.5 us a layer)
         if (a.rows > NEW_ROWS && a.capacity < MANY_NEW_ROWS_FROM) return false;
@@ -3118,8 +3148,8 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
     // One to four rows over codes in a cache of 24k tokens and more go to the kernel with loader waves, a
     // one-workgroup-per-CU kernel at every length: a share of up to 17 blocks (the kernel sees the length
     // when it runs: a step at 32k tokens is one round in a cache of any size) is one round, a longer one
-    // rounds of 8 blocks (three and four rows: 12).  Three rows and more over halves go to their kernel
-    // with loader waves in a cache of any size.  SAETTA_STAGE_NO_LOADERS keeps to the register kernels (the caller's choice of
+    // rounds of 8 blocks (three and four rows: 12).  Three rows and more over halves, and the rows over codes that
+    // code_rows names, go to the kernels with a wave per tile.  SAETTA_STAGE_NO_LOADERS keeps to the register kernels (the caller's choice of
     // kernel family, as DecodeAttention.kernel is in the reference, src/attention.rs:36-38).
     // The register kernels: one workgroup per CU (half as many splits, each twice as long) or two.  Two
     // rows and more and a half cache need the whole register file anyway; one row over codes fits two
@@ -3127,7 +3157,7 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
     // many partials is worth more (measured: 19.4 against 20.6 us per layer at 32k, 28.3 against 29.7 at
     // 64k, but 44 against 35 at 146k, 4-bit).  Both stages of a call derive the same number from the same arguments; where
     // a plan's reduce stage makes a token step of the launches before it, the number is the token step's.
-    const bool loaders = bits == 16 ? rows >= HALF_ROWS_FROM : rows <= 4 && capacity >= KEYS_FIRST_FROM;
+    const bool loaders = bits == 16 ? rows >= HALF_ROWS_FROM : code_rows(bits, rows, capacity) || (rows <= 4 && capacity >= KEYS_FIRST_FROM);
     const bool keys_first = loaders && !(stages & SAETTA_STAGE_NO_LOADERS);
     const bool one_per_cu = rows >= 2 || bits == 16 || capacity <= 80 * 1024 || keys_first;
     if (one_per_cu && nsplits > MAX_SPLITS / 2) nsplits = MAX_SPLITS / 2;
@@ -3180,6 +3210,20 @@ int raise_lds_keys_first() {
     return int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_partial_kernel_s<BITS, M>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, KeysFirst<BITS, M>::LDS_BYTES));
 }
+template <int BITS, int TILES>
+int raise_lds_code_rows_of() {
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_token_kernel_c<BITS, TILES>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         CodeRows<BITS, TILES>::LDS_BYTES))) return rc;
+    return int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_partial_kernel_c<BITS, TILES>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   CodeRows<BITS, TILES>::LDS_BYTES));
+}
+template <int BITS>
+int raise_lds_code_rows() {
+    if (int rc = raise_lds_code_rows_of<BITS, 1>()) return rc;
+    if (int rc = raise_lds_code_rows_of<BITS, 2>()) return rc;
+    if (int rc = raise_lds_code_rows_of<BITS, 3>()) return rc;
+    return raise_lds_code_rows_of<BITS, 4>();
+}
 template <int TILES>
 int raise_lds_half_rows() {
     if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_token_kernel_h<TILES>), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -3219,6 +3263,8 @@ int setup_decode() {
     if (int rc = raise_lds_keys_first<4, 2>()) return rc;
     if (int rc = raise_lds_keys_first<4, 3>()) return rc;
     if (int rc = raise_lds_keys_first<4, 4>()) return rc;
+    if (int rc = raise_lds_code_rows<8>()) return rc;
+    if (int rc = raise_lds_code_rows<4>()) return rc;
     if (int rc = raise_lds_half_rows<2>()) return rc;
     if (int rc = raise_lds_half_rows<3>()) return rc;
     if (int rc = raise_lds_half_rows<4>()) return rc;

@@ -17,8 +17,8 @@
 // still brings two whole rows of the cache.
 // Measured per layer in a plan, ten layers in a graph, attention_partial_kernel_n -> this: 6 rows at 57123 tokens 46.8 ->
 // 35.8 us, of which 2.7 the store taken in (a stream of the same loads without the products, 12 MB of partials and the merge
-// are 36.1 with it apart), at 12000 24.6 -> 22.2, 300 15.0 -> 13.8; 8 rows 51.2 -> 38.2, 27.1 -> 24.9, 17.1 -> 15.1; 3 rows
-// 37.4 -> 33.3, 18.6 -> 17.7, 11.7 -> 10.5; 4 rows at 200000 tokens 96.5 -> 82.  Two rows, one computing wave, are behind:
+// are 36.1 with it apart), at 12000 24.6 -> 21.7, 300 15.0 -> 13.4; 8 rows 51.2 -> 38.2, 27.1 -> 24.7, 17.1 -> 15.0; 3 rows
+// 37.4 -> 32.8, 18.6 -> 17.5, 11.7 -> 10.0; 4 rows at 200000 tokens 96.5 -> 82.  Two rows, one computing wave, are behind:
 // 30.7 -> 32.4 at 57123.  Error against 64 bits, rel, means of six seeds: 6 rows at 57123 tokens 4.4e-7 -> 4.3e-7, 3 at
 // 200000 5.8e-7 -> 5.6e-7, 5 at 700 3.2e-7 -> 2.9e-7.
 // Tried: two computing waves a tile on alternate slots (6 rows 39.4: two places are held instead of one, so less is on its
@@ -48,6 +48,12 @@ struct HalfRows {
 // P_UP and the sums so far need no rescaling.  It is followed in whole numbers: what is rescaled, and what
 // the merge multiplies a split with, is a power of two then, and the exponentials' arguments are rounded once.
 constexpr float MAX_SLACK = 1.0f;
+// x * y as f16 hi and lo parts: hi with the product's low mantissa bits cut off, lo what that leaves of the exact product (one
+// fused operation from it to the f16).
+__device__ __forceinline__ void split_product(float x, float y, _Float16 &hi, _Float16 &lo) {
+    hi = (_Float16)__builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x * y) & 0xffffe000u);
+    lo = (_Float16)fmaf(x, y, -(float)hi);
+}
 constexpr float NEVER = -3e38f;  // the score of a masked token: below any maximum, its probability is 0
 
 template <int TILES, bool PREP>
@@ -178,14 +184,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
     } else {
         // ---- the query operands: 16 * scale * log2(e) * q as f16 hi and lo parts ----
         if constexpr (PREP) {
-            float sum = 0.0f;
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) sum += q[s][e] * q[s][e];
-            }
-            const float scale = norm_scale(across_rows<16, 64>(sum, SumOp()), prep->p.eps);
-            // the tile's two rows' angles: an angle a lane; the pairs of dims (r, r + 32) are k-steps 0 and 1 of the same lane
+            // (before anything waits for the query values) the tile's two rows' angles: an angle a lane; the pairs of dims (r, r + 32) are k-steps 0 and 1 of the same lane
             float2 *rope = reinterpret_cast<float2 *>(lds_raw + W::ROPE_OFF + wave * 512);
             {
                 float s, c;
@@ -193,6 +192,13 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
                 rope[lane] = float2{s, c};
             }
             wave_sync();
+            float sum = 0.0f;
+#pragma unroll
+            for (int s = 0; s < 8; s++) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) sum += q[s][e] * q[s][e];
+            }
+            const float scale = norm_scale(across_rows<16, 64>(sum, SumOp()), prep->p.eps);
 #pragma unroll
             for (int s = 0; s < 8; s++) {
                 const float4 *w = reinterpret_cast<const float4 *>(prep->q_norm + 32 * s + 8 * j);
@@ -215,7 +221,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 _Float16 h, lw;
-                split_hi_lo(q[s][e] * qmul, h, lw);
+                split_product(q[s][e], qmul, h, lw);
                 qhi[s][e] = h, qlo[s][e] = lw;
             }
         }

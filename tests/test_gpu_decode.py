@@ -383,6 +383,33 @@ def test_rows_over_halves_follow_a_growing_maximum(step, m):
         assert worst < MAX_ABS_F64 + 2 * 2.0 ** -22 * np.log(2) * step * tokens, (tokens, worst)
 
 
+@pytest.mark.parametrize("m", [2, 3, 5, 8])
+@pytest.mark.parametrize("kind", [saetta.KvBits.Eight, saetta.KvBits.Four])
+def test_rows_over_codes_slot_by_slot(kind, m):
+    # One split of a cache whose rows go to the waves of their own: less than a slot of 32 tokens, one, just past one, fewer
+    # slots than streams, the loaders' whole depth, the ring of 8 or 16 places and around it.  The rows past the context are
+    # poisoned.
+    rng = np.random.default_rng(5400 + m)
+    capacity = 40960
+    k = rng.standard_normal((1100, VALUES)).astype(np.float32)
+    v = rng.standard_normal((1100, VALUES)).astype(np.float32)
+    q = rng.standard_normal((m, H, D)).astype(np.float32)
+    qg = rng.standard_normal((m, H, 2 * D)).astype(np.float32)
+    rows = saetta.AttentionRows(H, KV, capacity, m)
+    rows.splits = 1
+    for tokens in [m, 16, 32, 33, 65, 97, 193, 257, 330, 513, 1090]:
+        pos = tokens - m
+        kc, vc, kf, vf = cache_pair(k[:tokens], v[:tokens], kind, capacity, poison=True)
+        out = torch.full((m, H, D), float("nan"), device="cuda")
+        plan = saetta.Plan()
+        rows.record_quant(plan, m, dev(q), kc, vc, dev(qg), out, [saetta.TokenParams(0, pos + r).as_tensor("cuda") for r in range(m)])
+        plan.build().run()
+        got = host(out)
+        assert np.isfinite(got).all(), tokens
+        worst = np.abs(got - oracle.rows(q, kf, vf, pos, m, q_and_gate=qg, threads=8, f64=True)).max()
+        assert worst < MAX_ABS_F64, (tokens, worst)
+
+
 @pytest.mark.parametrize("splits", [64, 43, 32])
 @pytest.mark.parametrize("kind", [saetta.KvBits.Eight, saetta.KvBits.Four])
 @pytest.mark.parametrize("m", [3, 4])

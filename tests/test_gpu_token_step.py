@@ -84,9 +84,10 @@ def test_fused_step_equals_the_ops_one_by_one(kind, capacity, rows):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), position
 
 
+@pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("rows", [5, 6, 7, 8])
-def test_many_rows_of_a_large_half_cache_take_the_store_in(rows):
-    step = Step(saetta.KvBits.Half, 49152, rows, seed=rows)
+def test_many_rows_of_a_large_cache_take_the_store_in(rows, kind):
+    step = Step(kind, 49152, rows, seed=rows)
     assert launches(step) == 2
     built = step.plan.build()
     for position in (0, 1, 17, 3000, 49152 - rows, 49152 - 1, 49152 + 2):
