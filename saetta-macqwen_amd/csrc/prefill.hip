@@ -764,11 +764,18 @@ __global__ __launch_bounds__(MERGE_THREADS) void prefill_merge_kernel(PrefillArg
 // cache is read where it lies, once per row group: the keys go from memory to MFMA operands in registers, the values to a
 // tile of the wave's own in LDS, row by row as in memory, and come back transposed (ds_read_b64_tr_b16).  Codes are
 // dequantized on the way, with the arithmetic of the prepare kernel.
-// The price is that every row group pulls (and dequantizes) the keys for itself: from some hundred keys on the tiles of 16
+// The price is that every row group pulls (and dequantizes) the keys for itself: from a thousand keys on the tiles of 16
 // tokens and their images win; the line is in flash_plan.
-// Measured, the whole call, halves (tiles before): 16 tokens at 16 18.3 -> 7.5 us, 166 from 0 21.7 -> 10.8, 500 from 0
-// 31.2 -> 19.2.  A block of keys per wave takes 5 us with eight waves at it: 256 KB through the CU's 64 bytes a cycle are
-// 1.8 of them, the values' way through LDS and the query operands 1.4.
+// What bounds a block of halves per wave (4 us for the eight of them): 256 KB through the CU's 64 bytes a cycle are 1.8 of
+// them, the values' way through LDS and the query operands 1.4.  A key's operands straight from its row, 16 bytes a lane,
+// took 5.3 us: such a load is taken a row a cycle, and so four lanes fetch 64 bytes of a row together and turn four rows
+// round in registers.  Codes (5 us): the dequantization.  The values' reads are left to the compiler's counting: a wait for
+// each four of them took 0.3 us of halves' and 0.4 of 8-bit codes' four rounds, and 0.2 less of 4-bit codes'.
+// Measured, the whole call, tiles -> this: halves, 16 tokens at 16 18.3 -> 7.5 us, 166 from 0 21.7 -> 10.8; fetched row by
+// row -> in turns: 16 at 500 20.5 -> 18.1, 500 from 0 23.1 -> 20.5, 500 at 500 32.2 -> 26.4; 8-bit 33.7 -> 32.2.
+// One maximum for the eight blocks of a round, a wave 32 of the dims of all of them and nothing to join at the end took 1
+// to 2.5 us less with codes, but not with its precision: of each block the largest probability is now 1, without a
+// rounding, and with the largest of eight blocks alone an output was up to 1.2 times as far from 64 bits.
 constexpr int SMALL_WAVES = 8, SMALL_THREADS = 64 * SMALL_WAVES;
 
 struct SmallArgs {
@@ -801,7 +808,8 @@ struct SmallLds {
 template <int BITS>
 __device__ __forceinline__ constexpr int small_dim(int st, int hf) {
     constexpr int STEPS = 16 / BITS;  // k-steps per piece
-    return (st / STEPS * 2 + hf) * 8 * STEPS + st % STEPS * 8;
+    const int i = st / STEPS;         // the lane's register
+    return (BITS == 16 ? (i / 4 * 2 + hf) * 4 + i % 4 : i * 2 + hf) * 8 * STEPS + st % STEPS * 8;
 }
 
 template <int BITS>
@@ -822,19 +830,30 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
     const uint32_t vtile = lds0 + L::V_OFF + wave * L::VTILE;
 
     // ---- what a block needs of memory ----
-    u32x4 kreg[PIECES / 2];           // lane (key col, half hf): the pieces 2i + hf of its row
+    // Keys: lane (key col, half hf) multiplies a piece of its row at a time.  Codes: the pieces 2i + hf, fetched as they are
+    // multiplied.  Halves: the pieces 8i + 4 hf .. + 3; four lanes fetch 64 bytes of a row together, a row a register, and
+    // turn them round, for a load of 16 bytes of each of many rows is taken a row a cycle (codes have half and a quarter of
+    // the loads, and no cycles to spare for the turn).
+    u32x4 kreg[PIECES / 2];
     u32x2 kss = {0, 0}, kzs = {0, 0};  // scales and biases of the key's four groups
     constexpr int V_LOADS = BK * PIECES / 64, V_KEYS = 64 / PIECES;  // loads that bring the values; keys of one
     u32x4 vreg[BITS == 16 ? 1 : V_LOADS];
     uint32_t vss[BITS == 16 ? 1 : V_LOADS], vzs[BITS == 16 ? 1 : V_LOADS];
     const uint32_t vp = lane % PIECES, vk = lane / PIECES;  // codes: the lane's piece and key of a load
-    auto row_of = [&](uint32_t key) { return size_t(min(key, keys - 1)) * kvh + kv; };  // (past the end: the last row, masked)
+    auto row_of = [&](uint32_t key) { return min(key, keys - 1) * kvh + kv; };  // (past the end: the last row, masked; a cache is under 2 GB)
     auto fetch_keys = [&](uint32_t b) {
-        const size_t row = row_of(b * BK + col);
-        const u32x4 *src = reinterpret_cast<const u32x4 *>(a.kdata + row * RB) + hf;
+        if constexpr (BITS == 16) {
 #pragma unroll
-        for (int i = 0; i < PIECES / 2; i++) kreg[i] = src[2 * i];
-        if constexpr (BITS != 16) {
+            for (int j = 0; j < 4; j++) {
+                const u32x4 *src = reinterpret_cast<const u32x4 *>(a.kdata + (row_of(b * BK + (col & ~3) + j) * RB + 64 * hf + 16 * (lane & 3)));
+#pragma unroll
+                for (int i = 0; i < PIECES / 8; i++) kreg[4 * i + j] = src[8 * i];
+            }
+        } else {
+            const uint32_t row = row_of(b * BK + col);
+            const u32x4 *src = reinterpret_cast<const u32x4 *>(a.kdata + (row * RB + 16 * hf));
+#pragma unroll
+            for (int i = 0; i < PIECES / 2; i++) kreg[i] = src[2 * i];
             kss = *reinterpret_cast<const u32x2 *>(a.kscales + row * 4);
             kzs = *reinterpret_cast<const u32x2 *>(a.kbiases + row * 4);
         }
@@ -859,8 +878,8 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
         } else {
 #pragma unroll
             for (int u = 0; u < V_LOADS; u++) {
-                const size_t row = row_of(b * BK + u * V_KEYS + vk);
-                vreg[u] = *reinterpret_cast<const u32x4 *>(a.vdata + row * RB + vp * 16);
+                const uint32_t row = row_of(b * BK + u * V_KEYS + vk);
+                vreg[u] = *reinterpret_cast<const u32x4 *>(a.vdata + (row * RB + vp * 16));
                 vss[u] = a.vscales[row * 4 + vp * 4 / PIECES], vzs[u] = a.vbiases[row * 4 + vp * 4 / PIECES];
             }
         }
@@ -879,6 +898,27 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
             }
             return __builtin_bit_cast(half8, u32x4{o[0], o[1], o[2], o[3]});
         }
+    };
+
+    // Registers x[0..3] of four lanes, lane t holding piece t of row j in x[j]: then lane t holds piece j of its row t.
+    const bool odd = lane & 1, high = lane & 2;
+    auto turn = [&](u32x4 *x) {
+#pragma unroll
+        for (int j = 0; j < 4; j += 2)
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                const uint32_t u = x[j][w], v = x[j + 1][w];
+                const uint32_t un = __builtin_amdgcn_mov_dpp(int(u), 0xb1, 0xf, 0xf, true), vn = __builtin_amdgcn_mov_dpp(int(v), 0xb1, 0xf, 0xf, true);
+                x[j][w] = odd ? vn : u, x[j + 1][w] = odd ? v : un;
+            }
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                const uint32_t u = x[j][w], v = x[j + 2][w];
+                const uint32_t un = __builtin_amdgcn_mov_dpp(int(u), 0x4e, 0xf, 0xf, true), vn = __builtin_amdgcn_mov_dpp(int(v), 0x4e, 0xf, 0xf, true);
+                x[j][w] = high ? vn : u, x[j + 2][w] = high ? v : un;
+            }
     };
 
     if (uint32_t(wave) < active) fetch_keys(wave);
@@ -916,6 +956,7 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
                 const int g = i * 2 * VALUES / SAETTA_QUANT_GROUP;
                 ks = h2f(kss[g >> 1] >> (16 * (g & 1))), kz = h2f(kzs[g >> 1] >> (16 * (g & 1)));
             }
+            if (BITS == 16 && st % 4 == 0) turn(&kreg[i]);
             const half8 q = *reinterpret_cast<const half8 *>(lds + L::Q_OFF + st * 1024 + lane * 16);
             s = __builtin_amdgcn_mfma_f32_32x32x16_f16(eight(kreg[i], st % STEPS, ks, kz), q, s, 0, 0, 0);
         }
@@ -968,13 +1009,14 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
         // ---- O^T += V^T P^T: k-step sp, lane half hf: keys 16 sp + 4 hf .. + 3 and 8 further; a wave's LDS accesses run in order ----
         const uint32_t e = (lane >> 2) & 3, dim = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
         const uint32_t vrow = vtile + (4 * hf + e) * L::VROW;
+        typedef short short4 __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) short4 *LdsShort4;
 #pragma unroll
         for (int mt = 0; mt < 8; mt++) {
             const uint32_t d = BITS == 16 ? ((32 * mt + dim) * 2 + 64 * e) & 511 : (32 * mt + dim) * 2;
             u32x2 r[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(r[i]) : "v"(vrow + d + 8 * i * L::VROW) : "memory");
-            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3])::"memory");
+            for (int i = 0; i < 4; i++) r[i] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<LdsShort4>(vrow + d + 8 * i * L::VROW)));
 #pragma unroll
             for (int sp = 0; sp < 2; sp++) {
                 const half8 v = __builtin_bit_cast(half8, u32x4{r[2 * sp].x, r[2 * sp].y, r[2 * sp + 1].x, r[2 * sp + 1].y});
@@ -1094,43 +1136,46 @@ struct FlashPlan {
 // rounds of workgroups would take, in us, unsplit and with the keys in 2 to 32 parts, from figures measured on the MI355X:
 // a workgroup's block of 32 keys takes 0.6 us while the chip has power to spare (up to ~170 workgroups) and the chip as a
 // whole 284 blocks a us beyond that; the ends of an item (its first loads, the store of its part) 12 us, with the gate
-// 14.5; the merge a launch and 128 KB read back per item.  The small kernel's workgroups take as long for a block, with a
-// quarter of the rows, but their ends take 7 us (8.5 with codes) and there are no images to prepare (4 us and more).
+// 14.5; the merge a launch and 128 KB read back per item.  The small kernel's workgroups take 0.5 us for a block
+// (0.8 with codes), with a quarter of the rows, and don't slow each other down; their ends take 5 us (5.5), and there are no
+// images to prepare (5 us and more).
 // Measured, unsplit -> split by this rule, the whole call (8-bit cache): 100 tokens at 10000: 211 -> 47 us, at 100000
 // (4-bit): 1886 -> 225; 500 at 40000: 770 -> 330; 2100 at 9000: 497 -> 405.  A full chunk (4096 tokens: two whole rounds)
-// is never split.  Tiles -> the small kernel: 16 tokens at 16 18.6 -> 8.6, 300 from 0 24.6 -> 16.7, 500 at 500 36.8 -> 30.4;
-// past its line 100 at 1000 would take 29.4 for 27.5, 700 at 700 (halves) 51.5 for 41.9.
+// is never split.  Tiles -> the small kernel, halves and 8-bit: 16 tokens at 500 22.9 -> 18.1, 23.7 -> 22.9; 500 from 0
+// 31.5 -> 20.7, 32.5 -> 24.2; 700 from 0 37.3 -> 27.1, 38.6 -> 31.1; 145 at 839 31.5 -> 23.6, 32.6 -> 30.6; 500 at 800 38.6 ->
+// 30.1, 39.9 -> 38.2.  Past its line 1250 from 0 would take 51.2 for 45.8 (halves); 1000 from 0 43.3 for 41.8, 23 at 858
+// 27.8 for 25.6, 250 at 1300 41.5 for 37.4 (8-bit).
 FlashPlan flash_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, int bits) {
     constexpr float BLOCK_US = 0.6f, CHIP_BLOCKS_PER_US = 284.0f / 256.0f, PART_US = 12.0f, TILE_US = 14.5f, MERGE_US = 4.0f, MERGE_ITEM_US = 0.03f;
-    constexpr float SMALL_US = 7.0f, SMALL_CODES_US = 1.5f, PREPARE_US = 4.0f;
+    constexpr float SMALL_US = 5.0f, SMALL_BLOCK_US = 0.5f, SMALL_CODES_US = 5.5f, SMALL_CODES_BLOCK_US = 0.8f, PREPARE_US = 5.0f;
     FlashPlan f{};
     f.cus = cu_count();
     f.plain = plain_workspace_bytes(pos, tokens, kv_heads);
     if (tokens == 0 || kv_heads == 0) return f;
     const uint32_t ntiles = (tokens + TQ - 1) / TQ;
     const uint32_t longest = tile_blocks(pos, tokens, ntiles - 1), shortest = tile_blocks(pos, tokens, 0);
-    const float per_us = CHIP_BLOCKS_PER_US * float(f.cus);
+    const float chip_us = 1.0f / (CHIP_BLOCKS_PER_US * float(f.cus));
     // n items in order of length, from `high` down to `low` blocks, handed out one by one
-    auto rounds_us = [&](uint32_t n, float high, float low, float ends_us) {
+    auto rounds_us = [&](uint32_t n, float high, float low, float ends_us, float block_us, float chip_us) {
         float us = 0.0f, at = 0.0f;
         for (uint32_t left = n; left > 0;) {
             const uint32_t now = left < f.cus ? left : f.cus;
             const float mid = high - (high - low) * (at + 0.5f * float(now)) / float(n);  // mean length of the round's items
-            const float alone = mid * BLOCK_US, shared = mid * float(now) / per_us;
+            const float alone = mid * block_us, shared = mid * float(now) * chip_us;
             us += (alone > shared ? alone : shared) + ends_us;
             at += float(now), left -= now;
         }
-        const float one = high * BLOCK_US + ends_us;
+        const float one = high * block_us + ends_us;
         return us > one ? us : one;
     };
-    const float unsplit = rounds_us(ntiles * kv_heads, float(longest), float(shortest), TILE_US);
+    const float unsplit = rounds_us(ntiles * kv_heads, float(longest), float(shortest), TILE_US, BLOCK_US, chip_us);
     float best = 0.95f * unsplit;
     for (uint32_t parts = 2; parts <= 32; parts++) {
         const uint32_t pb = ((longest + parts - 1) / parts + 1) / 2 * 2;  // (a step of the kernel is two blocks)
         if (pb < 4 || pb >= longest) continue;
         const uint32_t items = prefill_items(pos, tokens, pb) * kv_heads;
         const float mid = 0.5f * float(longest + shortest) * float(ntiles * kv_heads) / float(items);
-        const float us = rounds_us(items, mid, mid, PART_US) + MERGE_US + MERGE_ITEM_US * float(items);
+        const float us = rounds_us(items, mid, mid, PART_US, BLOCK_US, chip_us) + MERGE_US + MERGE_ITEM_US * float(items);
         if (us < best) best = us, f.part_blocks = pb;
     }
     if (f.part_blocks) {
@@ -1140,7 +1185,9 @@ FlashPlan flash_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, int bits)
         best = unsplit;
     }
     const uint32_t groups = (tokens + 3) / 4 * kv_heads;
-    f.small = rounds_us(groups, float(longest), float(shortest), SMALL_US + (bits == 16 ? 0.0f : SMALL_CODES_US)) < best + PREPARE_US;
+    const bool halves = bits == 16;
+    f.small = rounds_us(groups, float(longest), float(shortest), halves ? SMALL_US : SMALL_CODES_US, halves ? SMALL_BLOCK_US : SMALL_CODES_BLOCK_US, 0.0f) <
+              best + PREPARE_US;
     return f;
 }
 

@@ -285,3 +285,25 @@ def test_short_chunks_over_short_contexts(kind, pos, tokens):
     assert np.isfinite(got).all()
     assert oracle.rel_rms(got, want) < REL_RMS
     assert np.abs(got - want).max() < MAX_ABS
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("pos,tokens", [(255, 1), (256, 1), (509, 3), (510, 6), (640, 9), (150, 600), (0, 701), (740, 7), (900, 150)])
+def test_short_chunks_whose_scores_grow(kind, pos, tokens):
+    # Rounds of 8 blocks, one a wave: one round and two (8 and 9 blocks), 16 and 17 blocks, a row group with a block more
+    # than the one before it, more row groups than CUs (two of them past the line of codes, before that of halves).  The
+    # keys grow with the square of their position, so that later rounds raise a wave's maximum by more than the slack of 8
+    # powers of two (scores to +-11; rounding keys of codes to halves moves those by 4e-4, their standard deviation, and an
+    # output by a quarter of that times the 4 or 5 between two values: within the tolerance of the other tests).
+    rng = np.random.default_rng(1000 * pos + tokens)
+    n = pos + tokens
+    k = (rng.standard_normal((n, VALUES)) * 3.0 * np.linspace(0.2, 1.0, n)[:, None] ** 2).astype(np.float32)
+    v = rng.standard_normal((n, VALUES)).astype(np.float32)
+    q16 = rng.standard_normal((tokens, H, D)).astype(np.float16)
+    qg = rng.standard_normal((tokens, H, 2 * D)).astype(np.float32)
+    kc, vc, kf, vf = make_cache(kind, k, v, n + 7, chunk_from=pos)
+    got = run(kind, q16, kc, vc, qg, pos, tokens)
+    want = oracle.prefill(q16.astype(np.float32), kf, vf, pos, tokens, q_and_gate=qg, threads=8)
+    assert np.isfinite(got).all()
+    assert oracle.rel_rms(got, want) < REL_RMS
+    assert np.abs(got - want).max() < MAX_ABS
