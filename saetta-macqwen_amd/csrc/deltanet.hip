@@ -725,10 +725,16 @@ __global__ __launch_bounds__(256) void deltanet_rows_small_tail_kernel(SmallRows
 // The snapshots are stored past the caches: as plain stores their lines, 2 MB of dirty data in the L2s per token, are
 // written back when the kernel ends (4 rows 10.7 instead of 8.8 us).  More workgroups to a head, each writing a part of
 // the snapshots, are no faster (9.2 us).
-// Measured per layer (30 layers in a graph, with the two-launch form before it): one token 7.1 -> 4.4 us, 4 rows with
-// snapshots 11.3 -> 8.9; 8 rows 14.2 -> 12.8. (A workgroup stores 64 KB a row, at 1 us each.)
+// A further token is vector instructions, sixteen waves' on one CU (without the snapshots' stores 8 rows take as long); a third
+// of them were the three sums of q and k, which every group of lanes made for itself.  From SHARED_SCALES_FROM rows on a wave
+// makes them for a token, for all, at the price of a barrier: 4 rows with snapshots 8.62 -> 8.21 us, 8 rows 12.55 -> 10.94, 2
+// rows 6.48 either way.  (A head by 512 threads, 8 lanes a row, with these sums: 8.37 and 11.27; 2 rows 6.8.  The loop over the
+// tokens rolled: 8.44, 11.55.)
+// Measured per layer (30 layers in a graph, with the two-launch form before it): one token 7.1 -> 4.6 us, 4 rows with
+// snapshots 11.3 -> 8.2; 8 rows 14.2 -> 10.9.
 typedef float nt4 __attribute__((ext_vector_type(4)));
 constexpr int HEAD_THREADS = 1024, HEAD_V_DIM = 128, HEAD_TAPS = 4;
+constexpr int SHARED_SCALES_FROM = 3;
 constexpr int HEAD_QK_WAVES = 2 * K_DIM / 64;  // waves that hold a key head's q and k channels
 
 // M tokens (1..8), 128 value dims, 4 taps.
@@ -738,6 +744,7 @@ __global__ __launch_bounds__(HEAD_THREADS) void deltanet_head_kernel(SmallRowsAr
     __shared__ __attribute__((aligned(16))) float in_lds[M][2 * K_DIM + HEAD_V_DIM];  // conv outputs: q, k, v
     __shared__ float gb_lds[M][2];                                                    // decay, beta
     __shared__ float o_lds[M][HEAD_V_DIM];
+    __shared__ __attribute__((aligned(16))) float scale_lds[M][4];                    // what q and k are multiplied by, q.k
     const uint32_t tid = threadIdx.x, lane = tid & 63, part = lane & 15;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t h = blockIdx.x, v_heads = a.p.v_heads, per_key = v_heads / a.p.k_heads, kh = h / per_key;
@@ -798,6 +805,21 @@ __global__ __launch_bounds__(HEAD_THREADS) void deltanet_head_kernel(SmallRowsAr
     uint32_t before = 0;
     if (wave < HEAD_QK_WAVES && lane == 0) before = atomicAdd(sync + kh * HEAD_QK_WAVES + wave, 1u);
 
+    // |q|^2, |k|^2 and q.k of token t by wave 15 - t (the first have the counters' answers to wait for), for all
+    if constexpr (M >= SHARED_SCALES_FROM) {
+        const uint32_t t = HEAD_THREADS / 64 - 1 - wave;
+        if (t < uint32_t(M)) {
+            const float2 q = *reinterpret_cast<const float2 *>(&in_lds[t][2 * lane]), k = *reinterpret_cast<const float2 *>(&in_lds[t][K_DIM + 2 * lane]);
+            const float qq = group_reduce<64>(q.x * q.x + q.y * q.y, SumOp()), kk = group_reduce<64>(k.x * k.x + k.y * k.y, SumOp());
+            const float kq = group_reduce<64>(q.x * k.x + q.y * k.y, SumOp());
+            if (lane == 0) {
+                *reinterpret_cast<float4 *>(scale_lds[t]) =
+                    make_float4((1.0f / sqrtf(float(K_DIM))) * __builtin_amdgcn_rsqf(qq + a.p.eps), __builtin_amdgcn_rsqf(kk + a.p.eps), kq, 0.0f);
+            }
+        }
+        __syncthreads();
+    }
+
 #pragma unroll
     for (int t = 0; t < M; t++) {
         float4 q[2], k[2];
@@ -807,12 +829,18 @@ __global__ __launch_bounds__(HEAD_THREADS) void deltanet_head_kernel(SmallRowsAr
             k[i] = *reinterpret_cast<const float4 *>(&in_lds[t][K_DIM + 64 * i + part * 4]);
         }
         const float g = gb_lds[t][0], beta = gb_lds[t][1];
-        // One round of 16-lane sums per token: |q|^2, |k|^2, q.k, and S.k and S.q of both rows, S before the decay and
-        // the update: (g S + d k^T) q = g S q + d (k.q).
-        const float qq = group_reduce<16>(dot4(q[0], q[0]) + dot4(q[1], q[1]), SumOp());
-        const float kk = group_reduce<16>(dot4(k[0], k[0]) + dot4(k[1], k[1]), SumOp());
-        const float kq = group_reduce<16>(dot4(k[0], q[0]) + dot4(k[1], q[1]), SumOp());
-        const float qi = (1.0f / sqrtf(float(K_DIM))) * __builtin_amdgcn_rsqf(qq + a.p.eps), ki = __builtin_amdgcn_rsqf(kk + a.p.eps);
+        // One round of 16-lane sums per token: |q|^2, |k|^2, q.k (if they are not there), and S.k and S.q of both rows, S before
+        // the decay and the update: (g S + d k^T) q = g S q + d (k.q).
+        float qi, ki, kq;
+        if constexpr (M >= SHARED_SCALES_FROM) {
+            const float4 x = *reinterpret_cast<const float4 *>(scale_lds[t]);
+            qi = x.x, ki = x.y, kq = x.z;
+        } else {
+            const float qq = group_reduce<16>(dot4(q[0], q[0]) + dot4(q[1], q[1]), SumOp());
+            const float kk = group_reduce<16>(dot4(k[0], k[0]) + dot4(k[1], k[1]), SumOp());
+            kq = group_reduce<16>(dot4(k[0], q[0]) + dot4(k[1], q[1]), SumOp());
+            qi = (1.0f / sqrtf(float(K_DIM))) * __builtin_amdgcn_rsqf(qq + a.p.eps), ki = __builtin_amdgcn_rsqf(kk + a.p.eps);
+        }
 #pragma unroll
         for (int r = 0; r < 2; r++) {
             const float sk = group_reduce<16>(dot4(st[r][0], k[0]) + dot4(st[r][1], k[1]), SumOp());
