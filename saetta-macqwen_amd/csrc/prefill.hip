@@ -769,10 +769,12 @@ __global__ __launch_bounds__(MERGE_THREADS) void prefill_merge_kernel(PrefillArg
 // What bounds a block of halves per wave (4 us for the eight of them): 256 KB through the CU's 64 bytes a cycle are 1.8 of
 // them, the values' way through LDS and the query operands 1.4.  A key's operands straight from its row, 16 bytes a lane,
 // took 5.3 us: such a load is taken a row a cycle, and so four lanes fetch 64 bytes of a row together and turn four rows
-// round in registers.  Codes (5 us): the dequantization.  The values' reads are left to the compiler's counting: a wait for
-// each four of them took 0.3 us of halves' and 0.4 of 8-bit codes' four rounds, and 0.2 less of 4-bit codes'.
+// round in registers.  Codes (4 us, once for every row group): vector instructions, of which a pair of codes is
+// three (8-bit) or four, in packed halves; as f32, seven of them, the eight blocks took 5 us.  The values' reads are left to
+// the compiler's counting: a wait for each four of them took 0.3 us of halves' four rounds.
 // Measured, the whole call, tiles -> this: halves, 16 tokens at 16 18.3 -> 7.5 us, 166 from 0 21.7 -> 10.8; fetched row by
-// row -> in turns: 16 at 500 20.5 -> 18.1, 500 from 0 23.1 -> 20.5, 500 at 500 32.2 -> 26.4; 8-bit 33.7 -> 32.2.
+// row -> in turns: 16 at 500 20.5 -> 18.1, 500 from 0 23.1 -> 20.5, 500 at 500 32.2 -> 26.4; codes as f32 -> as halves: 8-bit
+// 23.8 -> 20.2, 24.9 -> 21.8, 34.4 -> 28.8, 4-bit 23.3 -> 20.2, 23.4 -> 21.4, 33.3 -> 29.4, and no further from 64 bits.
 // One maximum for the eight blocks of a round, a wave 32 of the dims of all of them and nothing to join at the end took 1
 // to 2.5 us less with codes, but not with its precision: of each block the largest probability is now 1, without a
 // rounding, and with the largest of eight blocks alone an output was up to 1.2 times as far from 64 bits.
@@ -833,7 +835,7 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
     // Keys: lane (key col, half hf) multiplies a piece of its row at a time.  Codes: the pieces 2i + hf, fetched as they are
     // multiplied.  Halves: the pieces 8i + 4 hf .. + 3; four lanes fetch 64 bytes of a row together, a row a register, and
     // turn them round, for a load of 16 bytes of each of many rows is taken a row a cycle (codes have half and a quarter of
-    // the loads, and no cycles to spare for the turn).
+    // the loads: turned, 0.3 us of 33 slower).
     u32x4 kreg[PIECES / 2];
     u32x2 kss = {0, 0}, kzs = {0, 0};  // scales and biases of the key's four groups
     constexpr int V_LOADS = BK * PIECES / 64, V_KEYS = 64 / PIECES;  // loads that bring the values; keys of one
@@ -884,17 +886,29 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
             }
         }
     };
-    // The 8 values of sub-step `sub` of a piece, as halves.
-    auto eight = [&](const u32x4 &piece, int sub, float s, float z) {
+    // The 8 values of sub-step `sub` of a piece, as halves; s, z: scale and bias (f16 bits).  A code in the mantissa of 1024 is
+    // 1024 + code; s * code + z is rounded once, as a half (the prepare kernel rounds it to f32 in between: they differ where
+    // that f32 lies on the middle of two halves).
+    auto eight = [&](const u32x4 &piece, int sub, uint32_t s, uint32_t z) {
         if constexpr (BITS == 16) {
             return __builtin_bit_cast(half8, piece);
         } else {
+            const _Float16 sh = __builtin_bit_cast(_Float16, uint16_t(s)), zh = __builtin_bit_cast(_Float16, uint16_t(z));
             uint32_t o[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 constexpr int PER = 32 / BITS;
-                const int at = 8 * sub + 2 * i;
-                o[i] = pack_half2(dequant(s, z, code_of<BITS>(piece[at / PER], at % PER)), dequant(s, z, code_of<BITS>(piece[at / PER], at % PER + 1)));
+                const uint32_t word = piece[(8 * sub + 2 * i) / PER];
+                const uint32_t at = (8 * sub + 2 * i) % PER * BITS / 8;  // the byte of the first code
+                half2_ x;
+                if constexpr (BITS == 8) {
+                    x = __builtin_bit_cast(half2_, __builtin_amdgcn_perm(0x64646464u, word, at | 4u << 8 | (at + 1) << 16 | 4u << 24));
+                    x = x + half2_{(_Float16)-1024.0f, (_Float16)-1024.0f};
+                } else {  // (both nibbles of a byte, the second times 16)
+                    x = __builtin_bit_cast(half2_, (__builtin_amdgcn_perm(word, word, at * 0x01010101u) & 0x00f0000fu) | 0x64006400u);
+                    x = __builtin_elementwise_fma(x, half2_{(_Float16)1.0f, (_Float16)0.0625f}, half2_{(_Float16)-1024.0f, (_Float16)-64.0f});
+                }
+                o[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(x, half2_{sh, sh}, half2_{zh, zh}));
             }
             return __builtin_bit_cast(half8, u32x4{o[0], o[1], o[2], o[3]});
         }
@@ -951,10 +965,10 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
 #pragma unroll
         for (int st = 0; st < 16; st++) {
             const int i = st / STEPS;
-            float ks = 0.0f, kz = 0.0f;
+            uint32_t ks = 0, kz = 0;
             if constexpr (BITS != 16) {
                 const int g = i * 2 * VALUES / SAETTA_QUANT_GROUP;
-                ks = h2f(kss[g >> 1] >> (16 * (g & 1))), kz = h2f(kzs[g >> 1] >> (16 * (g & 1)));
+                ks = kss[g >> 1] >> (16 * (g & 1)), kz = kzs[g >> 1] >> (16 * (g & 1));
             }
             if (BITS == 16 && st % 4 == 0) turn(&kreg[i]);
             const half8 q = *reinterpret_cast<const half8 *>(lds + L::Q_OFF + st * 1024 + lane * 16);
@@ -999,10 +1013,9 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
         if constexpr (BITS != 16) {
 #pragma unroll
             for (int u = 0; u < V_LOADS; u++) {
-                const float vs = h2f(vss[u]), vz = h2f(vzs[u]);
                 half8 *dst = reinterpret_cast<half8 *>(lds + L::V_OFF + wave * L::VTILE + (u * V_KEYS + vk) * L::VROW + vp * VALUES * 2);
 #pragma unroll
-                for (int sub = 0; sub < STEPS; sub++) dst[sub] = eight(vreg[u], sub, vs, vz);
+                for (int sub = 0; sub < STEPS; sub++) dst[sub] = eight(vreg[u], sub, vss[u], vzs[u]);
             }
             if (b + SMALL_WAVES < nblocks) fetch_values(b + SMALL_WAVES);
         }
@@ -1137,17 +1150,17 @@ struct FlashPlan {
 // a workgroup's block of 32 keys takes 0.6 us while the chip has power to spare (up to ~170 workgroups) and the chip as a
 // whole 284 blocks a us beyond that; the ends of an item (its first loads, the store of its part) 12 us, with the gate
 // 14.5; the merge a launch and 128 KB read back per item.  The small kernel's workgroups take 0.5 us for a block
-// (0.8 with codes), with a quarter of the rows, and don't slow each other down; their ends take 5 us (5.5), and there are no
+// (0.6 with codes), with a quarter of the rows, and don't slow each other down; their ends take 5 us, and there are no
 // images to prepare (5 us and more).
 // Measured, unsplit -> split by this rule, the whole call (8-bit cache): 100 tokens at 10000: 211 -> 47 us, at 100000
 // (4-bit): 1886 -> 225; 500 at 40000: 770 -> 330; 2100 at 9000: 497 -> 405.  A full chunk (4096 tokens: two whole rounds)
-// is never split.  Tiles -> the small kernel, halves and 8-bit: 16 tokens at 500 22.9 -> 18.1, 23.7 -> 22.9; 500 from 0
-// 31.5 -> 20.7, 32.5 -> 24.2; 700 from 0 37.3 -> 27.1, 38.6 -> 31.1; 145 at 839 31.5 -> 23.6, 32.6 -> 30.6; 500 at 800 38.6 ->
-// 30.1, 39.9 -> 38.2.  Past its line 1250 from 0 would take 51.2 for 45.8 (halves); 1000 from 0 43.3 for 41.8, 23 at 858
-// 27.8 for 25.6, 250 at 1300 41.5 for 37.4 (8-bit).
+// is never split.  Tiles -> the small kernel, halves and 8-bit: 16 tokens at 500 22.9 -> 18.1, 24.1 -> 20.6; 500 from 0
+// 31.5 -> 20.7, 32.6 -> 21.8; 700 from 0 37.3 -> 27.1, 37.5 -> 28.6; 145 at 839 31.5 -> 23.6, 32.9 -> 26.0; 500 at 800 38.6 ->
+// 30.1, 41.2 -> 32.6.  Past its line 1250 from 0 would take 51.2 for 45.8 (halves); 1100 from 0 46.3 for 44.9, 16 at 1000
+// 25.9 for 25.0 (4-bit 27.0), 250 at 1700 39.7 for 38.2, but 250 at 1300 34.2 for 37.3 (8-bit).
 FlashPlan flash_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, int bits) {
     constexpr float BLOCK_US = 0.6f, CHIP_BLOCKS_PER_US = 284.0f / 256.0f, PART_US = 12.0f, TILE_US = 14.5f, MERGE_US = 4.0f, MERGE_ITEM_US = 0.03f;
-    constexpr float SMALL_US = 5.0f, SMALL_BLOCK_US = 0.5f, SMALL_CODES_US = 5.5f, SMALL_CODES_BLOCK_US = 0.8f, PREPARE_US = 5.0f;
+    constexpr float SMALL_US = 5.0f, SMALL_BLOCK_US = 0.5f, SMALL_CODES_BLOCK_US = 0.6f, PREPARE_US = 5.0f;
     FlashPlan f{};
     f.cus = cu_count();
     f.plain = plain_workspace_bytes(pos, tokens, kv_heads);
@@ -1185,9 +1198,7 @@ FlashPlan flash_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, int bits)
         best = unsplit;
     }
     const uint32_t groups = (tokens + 3) / 4 * kv_heads;
-    const bool halves = bits == 16;
-    f.small = rounds_us(groups, float(longest), float(shortest), halves ? SMALL_US : SMALL_CODES_US, halves ? SMALL_BLOCK_US : SMALL_CODES_BLOCK_US, 0.0f) <
-              best + PREPARE_US;
+    f.small = rounds_us(groups, float(longest), float(shortest), SMALL_US, bits == 16 ? SMALL_BLOCK_US : SMALL_CODES_BLOCK_US, 0.0f) < best + PREPARE_US;
     return f;
 }
 

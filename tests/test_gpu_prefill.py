@@ -307,3 +307,24 @@ def test_short_chunks_whose_scores_grow(kind, pos, tokens):
     assert np.isfinite(got).all()
     assert oracle.rel_rms(got, want) < REL_RMS
     assert np.abs(got - want).max() < MAX_ABS
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("scale", [1e-3, 300.0])
+def test_short_chunks_of_small_and_large_values(kind, scale):
+    # Codes become halves in packed half arithmetic, with scales below the least normal half (8-bit: 1e-3 * 8 / 255 = 3e-5)
+    # and values past 1000 as well.  A value is rounded to 2^-12 of itself, or to 2^-25 below 6e-5, a fiftieth of the values'
+    # size here: outputs are as close, relative to theirs, as at scale 1.
+    rng = np.random.default_rng(int(scale * 1000))
+    pos, tokens = 300, 37
+    n = pos + tokens
+    k = rng.standard_normal((n, VALUES)).astype(np.float32)
+    v = (scale * rng.standard_normal((n, VALUES))).astype(np.float32)
+    q16 = rng.standard_normal((tokens, H, D)).astype(np.float16)
+    qg = rng.standard_normal((tokens, H, 2 * D)).astype(np.float32)
+    kc, vc, kf, vf = make_cache(kind, k, v, n + 7, chunk_from=pos)
+    got = run(kind, q16, kc, vc, qg, pos, tokens)
+    want = oracle.prefill(q16.astype(np.float32), kf, vf, pos, tokens, q_and_gate=qg, threads=8)
+    assert np.isfinite(got).all()
+    assert oracle.rel_rms(got, want) < REL_RMS
+    assert np.abs(got - want).max() < MAX_ABS * scale
