@@ -773,8 +773,10 @@ __global__ __launch_bounds__(MERGE_THREADS) void prefill_merge_kernel(PrefillArg
 // three (8-bit) or four, in packed halves; as f32, seven of them, the eight blocks took 5 us.  The values' reads are left to
 // the compiler's counting: a wait for each four of them took 0.3 us of halves' four rounds.
 // Measured, the whole call, tiles -> this: halves, 16 tokens at 16 18.3 -> 7.5 us, 166 from 0 21.7 -> 10.8; fetched row by
-// row -> in turns: 16 at 500 20.5 -> 18.1, 500 from 0 23.1 -> 20.5, 500 at 500 32.2 -> 26.4; codes as f32 -> as halves: 8-bit
+// row -> in turns: 16 at 500 20.5 -> 18.6, 300 from 0 19.1 -> 17.4, 500 from 0 23.1 -> 20.5, 500 at 500 32.2 -> 26.5; codes as f32 -> as halves: 8-bit
 // 23.8 -> 20.2, 24.9 -> 21.8, 34.4 -> 28.8, 4-bit 23.3 -> 20.2, 23.4 -> 21.4, 33.3 -> 29.4, and no further from 64 bits.
+// Halves fill the registers: what depends on the lane alone is made anew where it is used (`at`), so that nothing spills; three
+// spilled registers cost a launch 1 us (300 from 0 18.3), the instructions 0.1 to 0.5 (16 at 500 18.1).
 // One maximum for the eight blocks of a round, a wave 32 of the dims of all of them and nothing to join at the end took 1
 // to 2.5 us less with codes, but not with its precision: of each block the largest probability is now 1, without a
 // rounding, and with the largest of eight blocks alone an output was up to 1.2 times as far from 64 bits.
@@ -845,9 +847,11 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
     auto row_of = [&](uint32_t key) { return min(key, keys - 1) * kvh + kv; };  // (past the end: the last row, masked; a cache is under 2 GB)
     auto fetch_keys = [&](uint32_t b) {
         if constexpr (BITS == 16) {
+            uint32_t at = lane;  // (not kept in registers across the loop)
+            asm volatile("" : "+v"(at));
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const u32x4 *src = reinterpret_cast<const u32x4 *>(a.kdata + (row_of(b * BK + (col & ~3) + j) * RB + 64 * hf + 16 * (lane & 3)));
+                const u32x4 *src = reinterpret_cast<const u32x4 *>(a.kdata + (row_of(b * BK + (at & 28) + j) * RB + 64 * (at >> 5) + 16 * (at & 3)));
 #pragma unroll
                 for (int i = 0; i < PIECES / 8; i++) kreg[4 * i + j] = src[8 * i];
             }
@@ -863,10 +867,12 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
     auto fetch_values = [&](uint32_t b) {
         if constexpr (BITS == 16) {
             // straight to the tile: place p of row k holds piece p - 4 (k % 4)
+            uint32_t at = lane;
+            asm volatile("" : "+v"(at));
 #pragma unroll
             for (int u = 0; u < V_LOADS; u++) {
-                const uint32_t k = 2 * u + (lane >> 5);
-                const uint64_t src = reinterpret_cast<uint64_t>(a.vdata) + row_of(b * BK + k) * RB + ((lane - 4 * (k & 3)) & 31) * 16;
+                const uint32_t k = 2 * u + (at >> 5);
+                const uint64_t src = reinterpret_cast<uint64_t>(a.vdata) + row_of(b * BK + k) * RB + ((at - 4 * (k & 3)) & 31) * 16;
                 asm volatile("s_mov_b32 m0, %0\n"
                              "s_nop 0\n"
                              "global_load_lds_dwordx4 %1, off\n"
@@ -1020,8 +1026,10 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
             if (b + SMALL_WAVES < nblocks) fetch_values(b + SMALL_WAVES);
         }
         // ---- O^T += V^T P^T: k-step sp, lane half hf: keys 16 sp + 4 hf .. + 3 and 8 further; a wave's LDS accesses run in order ----
-        const uint32_t e = (lane >> 2) & 3, dim = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
-        const uint32_t vrow = vtile + (4 * hf + e) * L::VROW;
+        uint32_t at = lane;
+        if (BITS == 16) asm volatile("" : "+v"(at));
+        const uint32_t e = (at >> 2) & 3, dim = ((at >> 4) & 1) * 16 + (at & 3) * 4;
+        const uint32_t vrow = vtile + (4 * (at >> 5) + e) * L::VROW;
         typedef short short4 __attribute__((ext_vector_type(4)));
         typedef __attribute__((address_space(3))) short4 *LdsShort4;
 #pragma unroll
