@@ -45,7 +45,12 @@ struct CodeRows {
     static_assert(SAETTA_MAX_ROWS * 32 * 8 + SAETTA_MAX_ROWS * 10 * DIM * 4 <= LDS_BYTES, "the new rows' workgroup fits");
 };
 
-constexpr float CODE_MAX_SLACK = 2.0f;  // as MAX_SLACK: the rescaling is 68 instructions
+// As MAX_SLACK: the rescaling is 68 instructions.  A probability is up to 4 P_UP then, and times a scale of its token it has to
+// fit a half: scales below LARGE_SCALE do (1024 * 63.97 = 65504).  Over a slot with a larger one the maximum is followed at
+// once, so that scales fit up to 255, as in the other kernels.  A loader wave looks the slot's scales over and tells with the
+// counter of its keys: a slack of 0 everywhere made 3 rows at 57123 tokens 27.3 -> 27.9 us a layer, 8 rows 45.3 -> 46.0 (4-bit).
+constexpr float CODE_MAX_SLACK = 2.0f;
+constexpr uint32_t LARGE_SCALE = 0x5400, LARGE_SLOT = 1u << 16;  // 64 as a half; what a counter is raised by
 
 template <int BITS, int TILES, bool PREP>
 __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, const PrepArgs *prep) {
@@ -99,9 +104,9 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
         const uint32_t at = u + first_slot < slots ? u + first_slot : u + first_slot - slots;
         return first_tok + at * W::SLOT_TOKENS;
     };
-    auto raise = [&](uint32_t c) {
+    auto raise = [&](uint32_t c, uint32_t by = 1) {
         asm volatile("" ::: "memory");
-        if (lane == 0) __hip_atomic_fetch_add(sync_lds + c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (lane == 0) __hip_atomic_fetch_add(sync_lds + c, by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         asm volatile("" ::: "memory");
     };
     auto peek = [&](uint32_t c) {
@@ -113,15 +118,16 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
     uint32_t lost = 0;
     auto await = [&](uint32_t c, uint32_t want) {
         asm volatile("" ::: "memory");
-        uint32_t left = W::SPIN_LIMIT;
+        uint32_t left = W::SPIN_LIMIT, v;
 #pragma nounroll
         do {
-            const uint32_t v = __hip_atomic_load(sync_lds + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            if (__builtin_amdgcn_readfirstlane(v) >= want) break;
+            v = __builtin_amdgcn_readfirstlane(__hip_atomic_load(sync_lds + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+            if ((v & (LARGE_SLOT - 1)) >= want) break;
             __builtin_amdgcn_s_sleep(1);
         } while (--left);
         if (__builtin_expect(left == 0, 0)) lost = 0x300u + c;
         asm volatile("" ::: "memory");
+        return v;
     };
 
     floatx4 acc[16];  // O^T of the codes: [4 g + e][i] is dim 64 g + 16 i + 4 j + e of the lane's pair
@@ -153,13 +159,13 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
             const uint32_t sc = (min(t0 + (lane >> 1), last) * kvh + kv) * 8 + (lane & 1) * 4;
             dma4(to + W::SC_OFF, sc, a.kscales);
             dma4(to + W::SC_OFF + W::SC_ARRAY, sc, a.kbiases);
+            dma4(to + W::SC_OFF + 2 * W::SC_ARRAY, sc, a.vscales);
+            dma4(to + W::SC_OFF + 3 * W::SC_ARRAY, sc, a.vbiases);
 #pragma unroll
             for (int i = 0; i < W::PART_LOADS; i++) {
                 const uint32_t row = ROWS_EACH * i + sub_row, turn = BITS == 8 ? row & 15 : row >> 1 & 7;
                 dma(to + i * 1024, (min(t0 + row, last) * kvh + kv) * W::ROW + ((unit ^ turn) << 4), a.kdata);
             }
-            dma4(to + W::SC_OFF + 2 * W::SC_ARRAY, sc, a.vscales);
-            dma4(to + W::SC_OFF + 3 * W::SC_ARRAY, sc, a.vbiases);
 #pragma unroll
             for (int i = 0; i < W::PART_LOADS; i++) {
                 const uint32_t row = ROWS_EACH * i + sub_row, turn = (row >> 2 & 3) * (UNITS / 4);
@@ -168,8 +174,14 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
         };
         uint32_t asked = 0, told = 0;  // of this loader's slots: requested, known to have landed
         auto place_of = [&](uint32_t mine) { return (L + mine * W::LOADERS) % W::PLACES; };
+        auto tell_keys = [&]() {
+            asm volatile("" ::: "memory");
+            const uint32_t s = *reinterpret_cast<__attribute__((address_space(3))) const uint32_t *>(lds0 + place_of(told) * W::SLOT + W::SC_OFF + 2 * W::SC_ARRAY + 4 * lane);
+            const bool large = max(s & 0x7fffu, s >> 16 & 0x7fffu) >= LARGE_SCALE;
+            raise(W::C_KEYS + place_of(told), __ballot(large) ? LARGE_SLOT + 1 : 1);
+        };
         auto tell = [&]() {
-            raise(W::C_KEYS + place_of(told)), raise(W::C_VALUES + place_of(told));
+            tell_keys(), raise(W::C_VALUES + place_of(told));
             told++;
         };
         for (uint32_t u = L; u < slots; u += W::LOADERS) {
@@ -190,8 +202,8 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
             constexpr int left = decltype(left_c)::value;  // slots behind this one
             if constexpr (left < W::DEPTH - 1) {
                 if (asked - told == uint32_t(left) + 1) {
-                    __builtin_amdgcn_s_waitcnt(vmcnt_only(left * W::LOADS + W::PART_LOADS + 2));
-                    raise(W::C_KEYS + place_of(told));
+                    __builtin_amdgcn_s_waitcnt(vmcnt_only(left * W::LOADS + W::PART_LOADS));
+                    tell_keys();
                     __builtin_amdgcn_s_waitcnt(vmcnt_only(left * W::LOADS));
                     raise(W::C_VALUES + place_of(told));
                     told++;
@@ -273,7 +285,7 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
         for (uint32_t u = stream; u < slots; u += W::STREAMS) {
             const uint32_t at = u % W::PLACES, use = u / W::PLACES, t0 = start_of(u), here = lds0 + at * W::SLOT;
             // ---- S^T = K Q^T of the slot's two blocks ----
-            await(W::C_KEYS + at, use + 1);
+            const float slack = await(W::C_KEYS + at, use + 1) < LARGE_SLOT ? CODE_MAX_SLACK : 0.0f;
             KeyRegs<BITS> kreg[2][4];
 #pragma unroll
             for (int b = 0; b < 2; b++) {
@@ -330,7 +342,7 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
             // ---- online softmax of the lane's pair (see attention_half_rows_body) ----
             float top = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
             top = across_rows<16, 64>(top, MaxOp());
-            const bool grown = top > m_run + CODE_MAX_SLACK;
+            const bool grown = top > m_run + slack;
             if (__ballot(grown)) {
                 const float to = grown ? ceilf(top) : m_run, keep = __builtin_amdgcn_exp2f(m_run - to);
                 m_run = to, l_run *= keep;

@@ -410,6 +410,38 @@ def test_rows_over_codes_slot_by_slot(kind, m):
         assert worst < MAX_ABS_F64, (tokens, worst)
 
 
+@pytest.mark.parametrize("m", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("kind", [saetta.KvBits.Eight, saetta.KvBits.Four])
+def test_rows_over_codes_of_large_values(kind, m):
+    # Value groups with scales up to 250: times a probability's 256 they just fit a half.  The scores grow along the context by
+    # 0.64 (log2) a slot of 32 tokens, so that a row's largest probability passes through everything between two of its
+    # maxima; one q head in two sees them fall instead.  The bound is that of the other tests, for normal values whose groups
+    # span 4.8, at the span of these; the hi and lo parts of q as in test_rows_over_halves_follow_a_growing_maximum.
+    rng = np.random.default_rng(5500 + m)
+    capacity, step = 40960, 0.02
+    span = 250.0 * (255 if kind is saetta.KvBits.Eight else 15)
+    k = (0.3 * rng.standard_normal((1100, KV, D))).astype(np.float32)
+    k[:, :, 0] = step * np.arange(1100)[:, None]
+    k = k.reshape(1100, VALUES)
+    v = (span * (rng.random((1100, VALUES)) - 0.5)).astype(np.float32)
+    q = (0.3 * rng.standard_normal((m, H, D))).astype(np.float32)
+    q[:, :, 0] = np.where(np.arange(H) % 2, -1.0, 1.0) * 16 / np.log2(np.e)
+    qg = rng.standard_normal((m, H, 2 * D)).astype(np.float32)
+    rows = saetta.AttentionRows(H, KV, capacity, m)
+    rows.splits = 1
+    for tokens in [m, 97, 330, 1090]:
+        pos = tokens - m
+        kc, vc, kf, vf = cache_pair(k[:tokens], v[:tokens], kind, capacity, poison=True)
+        out = torch.full((m, H, D), float("nan"), device="cuda")
+        plan = saetta.Plan()
+        rows.record_quant(plan, m, dev(q), kc, vc, dev(qg), out, [saetta.TokenParams(0, pos + r).as_tensor("cuda") for r in range(m)])
+        plan.build().run()
+        got = host(out)
+        assert np.isfinite(got).all(), tokens
+        worst = np.abs(got - oracle.rows(q, kf, vf, pos, m, q_and_gate=qg, threads=8, f64=True)).max()
+        assert worst < (MAX_ABS_F64 + 2 * 2.0 ** -22 * np.log(2) * step * tokens) * span / 4.8, (tokens, worst)
+
+
 @pytest.mark.parametrize("splits", [64, 43, 32])
 @pytest.mark.parametrize("kind", [saetta.KvBits.Eight, saetta.KvBits.Four])
 @pytest.mark.parametrize("m", [3, 4])
