@@ -344,7 +344,12 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
             top = across_rows<16, 64>(top, MaxOp());
             const bool grown = top > m_run + slack;
             if (__ballot(grown)) {
-                const float to = grown ? ceilf(top) : m_run, keep = __builtin_amdgcn_exp2f(m_run - to);
+                // (Up to four rows: the score itself, so that its token's probability is 1 and its products with the scales are
+                // halves as they are. In whole numbers every product is split, and the lo parts are cut off: rel 3.84e-5 against
+                // 64 bits instead of 3.50e-5 for 2 rows of 4-bit codes at 50000 tokens, 8.9e-5 instead of 8.4e-5 for 3 of 8 bits at
+                // 57123, 30 times as much over equal keys. With lo parts to the nearest whole numbers are ahead, 4.74e-5
+                // against 4.80e-5 for 6 rows of 8 bits there.)
+                const float to = grown ? (TILES >= 3 ? ceilf(top) : top) : m_run, keep = __builtin_amdgcn_exp2f(m_run - to);
                 m_run = to, l_run *= keep;
 #pragma unroll
                 for (int T = 0; T < 16; T++) acc[T] *= keep;

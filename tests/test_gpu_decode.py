@@ -442,6 +442,32 @@ def test_rows_over_codes_of_large_values(kind, m):
         assert worst < (MAX_ABS_F64 + 2 * 2.0 ** -22 * np.log(2) * step * tokens) * span / 4.8, (tokens, worst)
 
 
+@pytest.mark.parametrize("m", [2, 3, 4])
+@pytest.mark.parametrize("kind", [saetta.KvBits.Eight, saetta.KvBits.Four])
+def test_rows_over_codes_of_equal_keys_lose_nothing(kind, m):
+    # All keys equal, so that every token has the largest score: its probability is 1, its product with a scale is a half as
+    # it is, and only the f32 sums round, by half a unit (2^-25) of sums below 2.4.  A maximum that is not the score itself
+    # makes the probabilities' lo parts, cut off, 2^-23 of the codes' part too small, 1.4e-7 with the gate.
+    rng = np.random.default_rng(5600 + m)
+    capacity = 40960
+    rows = saetta.AttentionRows(H, KV, capacity, m)
+    rows.splits = 1
+    for tokens in [64, 160]:
+        k = np.repeat(rng.standard_normal((1, VALUES)), tokens, 0).astype(np.float32)
+        v = rng.standard_normal((tokens, VALUES)).astype(np.float32)
+        q = rng.standard_normal((m, H, D)).astype(np.float32)
+        qg = rng.standard_normal((m, H, 2 * D)).astype(np.float32)
+        kc, vc, _, vf = cache_pair(k, v, kind, capacity, poison=True)
+        out = torch.full((m, H, D), float("nan"), device="cuda")
+        plan = saetta.Plan()
+        rows.record_quant(plan, m, dev(q), kc, vc, dev(qg), out, [saetta.TokenParams(0, tokens - m + r).as_tensor("cuda") for r in range(m)])
+        plan.build().run()
+        means = np.stack([vf.reshape(tokens, KV, D)[:tokens - m + r + 1].astype(np.float64).mean(0).repeat(H // KV, 0) for r in range(m)])
+        error = host(out) - means / (1 + np.exp(-qg[:, :, D:].astype(np.float64)))
+        rms = np.sqrt((error ** 2).mean())
+        assert rms < 2.0 ** -24, (tokens, rms)
+
+
 @pytest.mark.parametrize("splits", [64, 43, 32])
 @pytest.mark.parametrize("kind", [saetta.KvBits.Eight, saetta.KvBits.Four])
 @pytest.mark.parametrize("m", [3, 4])
