@@ -1045,6 +1045,8 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
             }
         }
         if constexpr (BITS == 16) {
+            // (what comes from memory into the tile is not in the order of the wave's LDS accesses: its reads have to be back)
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             if (b + SMALL_WAVES < nblocks) fetch_values(b + SMALL_WAVES);
         }
     }
