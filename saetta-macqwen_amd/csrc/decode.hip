@@ -2969,19 +2969,22 @@ constexpr uint32_t MANY_NEW_ROWS_FROM = 48 * 1024;
 
 // Rows over codes that take the kernel with waves of their own (attention_partial_kernel_c), by the cache's capacity; us a
 // layer in a plan, the kernel before it -> this one:
-//   two rows from 40k: 36000 of 65536 21.2 -> 19.9, 57123 26.5 -> 23.7 (4-bit 26.6 -> 21.6; 131000 45.8 -> 31.3); behind where a
-//   share is a single round of the keys-first kernel: 32768 18.1 -> 19.0
-//   three and four rows from 24k: 3 rows, 8-bit, 32768 23.6 -> 22.6, 57123 35.5 -> 27.6; 4 rows, 4-bit, 24400 23.0 -> 23.4, 32768
-//   25.1 -> 24.8, 57123 36.6 -> 29.5, 100000 53.3 -> 39.6; even below, but for 4-bit at 12000: 17.8 -> 18.3, 19.1 -> 19.9
-//   five rows and more: 6 rows, 8-bit, 300 16.8 -> 15.4, 12000 26.9 -> 25.7, 57123 47.1 -> 38; 8 rows 19.3 -> 15.6, 31.6 -> 28, 54.8 ->
-//   42; 5 and 6 rows of 4-bit codes from 28k: 4000 20.9 -> 21.4, 30000 34.8 -> 32.9
+//   two rows from 48k: behind up to a length of 34k, where a share is a single round of the keys-first kernel (of 65536, 8-bit: 2000 13.4
+//   -> 13.7, 12000 14.7 -> 15.6, 32768 17.4 -> 19.2; 4-bit 13.5 -> 13.9, 14.8 -> 15.5, 17.0 -> 18.9) and ahead from there (37000 21.8 ->
+//   20.1, 44000 22.8 -> 21.2, 57123 26.6 -> 23.7; 20.8 -> 19.6, 21.7 -> 19.7, 26.4 -> 21.6; 131000 45.1 -> 30.6).  The length is not known
+//   where a launch is recorded, and one launch cannot hold both (twelve waves of 168 registers, six of 256): over all lengths that a
+//   cache has room for the two sides weigh the same at 48k.
+//   three and four rows from 24k, at every length but a full 24k of 4-bit codes: 3 rows, 8-bit, 2000 17.5 -> 15.0, 12000 19.4 -> 18.4, 24400
+//   21.7 -> 21.3, 32768 23.6 -> 22.7, 57123 35.7 -> 27.6; 4 rows, 4-bit, 19.0 -> 16.7, 21.3 -> 20.1, 22.9 -> 23.6, 25.0 -> 25.0, 36.7 -> 29.6
+//   five rows and more: 6 rows, 8-bit, 300 16.8 -> 15.4, 12000 26.9 -> 25.7, 57123 47.1 -> 38; 8 rows 19.1 -> 15.6, 31.6 -> 28.6, 54.8 ->
+//   42; 5 and 6 rows of 4-bit codes from 28k: 6 rows 4000 24.0 -> 22.7, 8000 24.9 -> 25.7, 20000 29.5 -> 29.3, 30000 34.8 -> 32.3
 // It is ahead in larger caches still (4 rows, 8-bit, at 150000 tokens 66.5 -> 48.4, 8 rows 107 -> 79), but stops at 64k tokens, 2 to
-// 4 rows of 4-bit codes at 128k: the sums of the codes and of the biases nearly cancel, the more the longer the context, and the
-// order in which 32-bit sums are taken shows as 4e-6 to 8e-6 of the results at 64000 tokens, 1.0e-5 to 1.5e-5 at 131000 (2 to 4
-// rows, 4-bit, 7e-6), where 1e-5 is what results may differ by.
+// 4 rows of 4-bit codes at 128k, so that results stay what they were: the sums of the codes and of the biases nearly cancel, the
+// more the longer the context, and the order in which 32-bit sums are taken shows as 4e-6 to 8e-6 of the results at 64000 tokens,
+// 1.0e-5 to 1.5e-5 at 131000 (2 to 4 rows, 4-bit, 7e-6).  Either kernel is further than that from 64 bits.
 constexpr bool code_rows(int bits, uint32_t rows, uint32_t capacity) {
     constexpr uint32_t K = 1024;
-    const uint32_t from = rows >= 7 || (rows >= 5 && bits == 8) ? 0 : rows >= 5 ? 28 * K : rows >= 3 ? 24 * K : 40 * K;
+    const uint32_t from = rows >= 7 || (rows >= 5 && bits == 8) ? 0 : rows >= 5 ? 28 * K : rows >= 3 ? 24 * K : 48 * K;
     const uint32_t to = rows <= 4 && bits == 4 ? 128 * K : 64 * K;
     return bits != 16 && rows >= 2 && capacity >= from && capacity <= to;
 }
