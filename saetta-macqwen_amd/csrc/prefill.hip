@@ -1161,16 +1161,18 @@ struct FlashPlan {
 // whole 284 blocks a us beyond that; the ends of an item (its first loads, the store of its part) 12 us, with the gate
 // 14.5; the merge a launch and 128 KB read back per item.  The small kernel's workgroups take 0.5 us for a block
 // (0.6 with codes), with a quarter of the rows, and don't slow each other down; their ends take 5 us, and there are no
-// images to prepare (5 us and more).
+// images to prepare (5 us and more).  (Codes: 0.59, for at 0.6 a tie sends 64 tokens at 1000 to the tiles, 27.2 -> 31.4.)
 // Measured, unsplit -> split by this rule, the whole call (8-bit cache): 100 tokens at 10000: 211 -> 47 us, at 100000
 // (4-bit): 1886 -> 225; 500 at 40000: 770 -> 330; 2100 at 9000: 497 -> 405.  A full chunk (4096 tokens: two whole rounds)
-// is never split.  Tiles -> the small kernel, halves and 8-bit: 16 tokens at 500 22.9 -> 18.1, 24.1 -> 20.6; 500 from 0
-// 31.5 -> 20.7, 32.6 -> 21.8; 700 from 0 37.3 -> 27.1, 37.5 -> 28.6; 145 at 839 31.5 -> 23.6, 32.9 -> 26.0; 500 at 800 38.6 ->
-// 30.1, 41.2 -> 32.6.  Past its line 1250 from 0 would take 51.2 for 45.8 (halves); 1100 from 0 46.3 for 44.9, 16 at 1000
-// 25.9 for 25.0 (4-bit 27.0), 250 at 1700 39.7 for 38.2, but 250 at 1300 34.2 for 37.3 (8-bit).
+// is never split.  Tiles -> the small kernel, halves | 8-bit | 4-bit: 16 tokens at 500 22.9 -> 18.3 | 24.0 -> 20.7 | 24.1 -> 20.6; 64 at
+// 1000 30.3 -> 24.5 | 31.4 -> 27.2 | 31.7 -> 28.4; 500 from 0 32.4 -> 20.3 | 33.4 -> 22.0 | 33.5 -> 21.9; 700 from 0 35.9 -> 25.7 | 37.0 ->
+// 28.5 | 37.3 -> 26.6; 500 at 800 39.2 -> 31.0 | 40.9 -> 32.9 | 41.1 -> 33.8.  Past its line: 1250 from 0 46.5 -> 50.3 | 47.8 -> 55.1 | 47.8
+// -> 54.1; 250 at 1700 35.4 -> 37.0 | 36.7 -> 39.3 | 37.2 -> 42.6; 16 at 1000 25.0 -> 25.9 | 24.9 -> 27.0 (codes).  Of 36 chunks on
+// either side of it each, none is sent to the small kernel that it takes longer for; left to the tiles though the small kernel
+// is ahead are 128 tokens at 1500 (33.7 -> 31.8 | 35.7 -> 34.0), 250 at 1300 (36.2 -> 33.9) and 100 at 1300 (33.1 -> 30.4) of 8-bit codes.
 FlashPlan flash_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, int bits) {
     constexpr float BLOCK_US = 0.6f, CHIP_BLOCKS_PER_US = 284.0f / 256.0f, PART_US = 12.0f, TILE_US = 14.5f, MERGE_US = 4.0f, MERGE_ITEM_US = 0.03f;
-    constexpr float SMALL_US = 5.0f, SMALL_BLOCK_US = 0.5f, SMALL_CODES_BLOCK_US = 0.6f, PREPARE_US = 5.0f;
+    constexpr float SMALL_US = 5.0f, SMALL_BLOCK_US = 0.5f, SMALL_CODES_BLOCK_US = 0.59f, PREPARE_US = 5.0f;
     FlashPlan f{};
     f.cus = cu_count();
     f.plain = plain_workspace_bytes(pos, tokens, kv_heads);
