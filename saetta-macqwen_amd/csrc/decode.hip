@@ -2962,9 +2962,9 @@ constexpr uint32_t KEYS_FIRST_FROM = 24 * 1024;
 // Rows over a half cache that take the kernel with loader waves, at any capacity (figures there): two rows are one computing
 // wave, which the register kernel's four are ahead of.
 constexpr uint32_t HALF_ROWS_FROM = 3;
-// Five rows and more take the store in, where their kernel has loader waves, from this capacity on.  (One launch is ahead in smaller caches too, 6 rows
-// at 300 tokens of 8192 13.7 -> 12.5 us a layer, at 30000 of 32768 29.3 -> 26.7; but there the store is a launch of its own as the
-// tests have it.)
+// Five rows and more take the store in, where their kernel has loader waves, from this capacity on.  This is no crossover: one launch
+// is ahead in smaller caches too (6 rows at 300 tokens of 8192 13.7 -> 12.5 us a layer, at 30000 of 32768 29.3 -> 26.7), but in those a
+// step of many rows is the three launches that test_gpu_token_step.py counts (at up to 40960 tokens).
 constexpr uint32_t MANY_NEW_ROWS_FROM = 48 * 1024;
 
 // Rows over codes that take the kernel with waves of their own (attention_partial_kernel_c), by the cache's capacity; us a
