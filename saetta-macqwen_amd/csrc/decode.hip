@@ -2833,6 +2833,7 @@ __global__ __launch_bounds__((KeysFirst<BITS, M>::THREADS_)) void attention_toke
     attention_partial_s_body<BITS, M, true>(t.a, &t.prep);
 }
 
+#include "decode_rows.hpp"
 #include "decode_half_rows.hpp"
 #include "decode_code_rows.hpp"
 

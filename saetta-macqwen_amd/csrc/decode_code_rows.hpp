@@ -89,46 +89,10 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
 
     // ---- the context and this workgroup's share of it, as in attention_partial_body ----
     const uint32_t max_len = PREP ? tokens_before(a, position, kv_len) : min(position + a.rows, a.capacity);
-    const uint32_t nblocks = (max_len + BLOCK - 1) / BLOCK;
-    uint32_t blk_begin = split, blk_end = split + 1;
-    if (nblocks <= context_splits) {
-        if (split >= nblocks) return;
-    } else {
-        blk_begin = split * nblocks / context_splits;
-        blk_end = (split + 1) * nblocks / context_splits;
-    }
-    const uint32_t first_tok = blk_begin * BLOCK, limit = min(max_len, blk_end * BLOCK);
-    const uint32_t slots = (limit - first_tok + W::SLOT_TOKENS - 1) / W::SLOT_TOKENS;
-    const uint32_t first_slot = (split & 3) * slots / 4;
-    auto start_of = [&](uint32_t u) {
-        const uint32_t at = u + first_slot < slots ? u + first_slot : u + first_slot - slots;
-        return first_tok + at * W::SLOT_TOKENS;
-    };
-    auto raise = [&](uint32_t c, uint32_t by = 1) {
-        asm volatile("" ::: "memory");
-        if (lane == 0) __hip_atomic_fetch_add(sync_lds + c, by, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        asm volatile("" ::: "memory");
-    };
-    auto peek = [&](uint32_t c) {
-        asm volatile("" ::: "memory");
-        const uint32_t v = __hip_atomic_load(sync_lds + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        asm volatile("" ::: "memory");
-        return uint32_t(__builtin_amdgcn_readfirstlane(v));
-    };
-    uint32_t lost = 0;
-    auto await = [&](uint32_t c, uint32_t want) {
-        asm volatile("" ::: "memory");
-        uint32_t left = W::SPIN_LIMIT, v;
-#pragma nounroll
-        do {
-            v = __builtin_amdgcn_readfirstlane(__hip_atomic_load(sync_lds + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
-            if ((v & (LARGE_SLOT - 1)) >= want) break;
-            __builtin_amdgcn_s_sleep(1);
-        } while (--left);
-        if (__builtin_expect(left == 0, 0)) lost = 0x300u + c;
-        asm volatile("" ::: "memory");
-        return v;
-    };
+    const SlotShare<W::SLOT_TOKENS> share(max_len, split, context_splits);
+    if (share.empty()) return;
+    const uint32_t limit = share.limit, slots = share.slots;
+    LdsCounters<W::SPIN_LIMIT, 0x300u, LARGE_SLOT - 1> sync{sync_lds, lane};
 
     floatx4 acc[16];  // O^T of the codes: [4 g + e][i] is dim 64 g + 16 i + 4 j + e of the lane's pair
     float zsum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -155,7 +119,7 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
         constexpr uint32_t UNITS = W::ROW / 16, ROWS_EACH = 64 / UNITS;  // 16-byte units of a row, rows a load brings
         const uint32_t last = limit - 1, sub_row = lane / UNITS, unit = lane % UNITS;
         auto request = [&](uint32_t u) {
-            const uint32_t t0 = start_of(u), to = lds0 + (u % W::PLACES) * W::SLOT;
+            const uint32_t t0 = share.start_of(u), to = lds0 + (u % W::PLACES) * W::SLOT;
             const uint32_t sc = (min(t0 + (lane >> 1), last) * kvh + kv) * 8 + (lane & 1) * 4;
             dma4(to + W::SC_OFF, sc, a.kscales);
             dma4(to + W::SC_OFF + W::SC_ARRAY, sc, a.kbiases);
@@ -178,19 +142,19 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
             asm volatile("" ::: "memory");
             const uint32_t s = *reinterpret_cast<__attribute__((address_space(3))) const uint32_t *>(lds0 + place_of(told) * W::SLOT + W::SC_OFF + 2 * W::SC_ARRAY + 4 * lane);
             const bool large = max(s & 0x7fffu, s >> 16 & 0x7fffu) >= LARGE_SCALE;
-            raise(W::C_KEYS + place_of(told), __ballot(large) ? LARGE_SLOT + 1 : 1);
+            sync.raise(W::C_KEYS + place_of(told), __ballot(large) ? LARGE_SLOT + 1 : 1);
         };
         auto tell = [&]() {
-            tell_keys(), raise(W::C_VALUES + place_of(told));
+            tell_keys(), sync.raise(W::C_VALUES + place_of(told));
             told++;
         };
         for (uint32_t u = L; u < slots; u += W::LOADERS) {
             const uint32_t at = u % W::PLACES, use = u / W::PLACES;
-            if (use && peek(W::C_FREE + at) < TILES * use) {
+            if (use && sync.peek(W::C_FREE + at) < TILES * use) {
                 // no place yet: what has been asked for is told of first, nobody else will
                 __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
                 while (told < asked) tell();
-                await(W::C_FREE + at, TILES * use);
+                sync.await(W::C_FREE + at, TILES * use);
             }
             request(u), asked++;
             if (asked - told == uint32_t(W::DEPTH)) {
@@ -205,7 +169,7 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
                     __builtin_amdgcn_s_waitcnt(vmcnt_only(left * W::LOADS + W::PART_LOADS));
                     tell_keys();
                     __builtin_amdgcn_s_waitcnt(vmcnt_only(left * W::LOADS));
-                    raise(W::C_VALUES + place_of(told));
+                    sync.raise(W::C_VALUES + place_of(told));
                     told++;
                 }
             }
@@ -222,25 +186,11 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
                 rope_angle(position + 2 * tile + (lane >> 5), lane & 31, 32, prep->p.log2_theta, s, c);
                 rope[lane] = float2{s, c};
                 wave_sync();
-                if constexpr (W::STREAMS > 1) raise(W::C_ROPE + tile);
+                if constexpr (W::STREAMS > 1) sync.raise(W::C_ROPE + tile);
             } else {
-                await(W::C_ROPE + tile, 1);
+                sync.await(W::C_ROPE + tile, 1);
             }
-            float sum = 0.0f;
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) sum += q[s][e] * q[s][e];
-            }
-            const float scale = norm_scale(across_rows<16, 64>(sum, SumOp()), prep->p.eps);
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-                const float4 *w = reinterpret_cast<const float4 *>(prep->q_norm + 64 * (s >> 1) + 16 * j + 8 * (s & 1));
-                const float4 f0 = w[0], f1 = w[1];
-                const float wv[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
-#pragma unroll
-                for (int e = 0; e < 8; e++) q[s][e] *= scale * wv[e];
-            }
+            norm_query(q, *prep, [&](int s) { return 64 * (s >> 1) + 16 * j + 8 * (s & 1); });
 #pragma unroll
             for (int s = 0; s < 2; s++) {
 #pragma unroll
@@ -283,9 +233,9 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
         const uint32_t v_lane = W::V_OFF + 4 * j * W::ROW + j * (W::ROW / 4) + (BITS == 8 ? pn : pn >> 1) * 4;
         const uint32_t sc_lane = W::SC_OFF + 4 * j * 8;  // scales of tokens 4 j .. + 3: 32 bytes
         for (uint32_t u = stream; u < slots; u += W::STREAMS) {
-            const uint32_t at = u % W::PLACES, use = u / W::PLACES, t0 = start_of(u), here = lds0 + at * W::SLOT;
+            const uint32_t at = u % W::PLACES, use = u / W::PLACES, t0 = share.start_of(u), here = lds0 + at * W::SLOT;
             // ---- S^T = K Q^T of the slot's two blocks ----
-            const float slack = await(W::C_KEYS + at, use + 1) < LARGE_SLOT ? CODE_MAX_SLACK : 0.0f;
+            const float slack = sync.await(W::C_KEYS + at, use + 1) < LARGE_SLOT ? CODE_MAX_SLACK : 0.0f;
             KeyRegs<BITS> kreg[2][4];
 #pragma unroll
             for (int b = 0; b < 2; b++) {
@@ -365,7 +315,7 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
             // 3e-5 away from what they were.)
             constexpr bool LO_NEAREST = TILES >= 3;
             // ---- O^T += V^T P^T, a group of dims at a time: its scale goes into the probabilities, its bias apart ----
-            await(W::C_VALUES + at, use + 1);
+            sync.await(W::C_VALUES + at, use + 1);
             ValRegs<BITS> vreg[2];
             u32x4 vs[2][2], vz[2][2];
 #pragma unroll
@@ -413,7 +363,7 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
                 for (int e = 0; e < 4; e++) acc[4 * g + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[e], plo, acc[4 * g + e], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            raise(W::C_FREE + at);
+            sync.raise(W::C_FREE + at);
         }
         l_run = across_rows<16, 64>(l_run, SumOp());
 #pragma unroll
@@ -438,7 +388,7 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
     const uint32_t streams = min(slots, uint32_t(W::STREAMS));  // that had a slot
     if (W::STREAMS == 1 || streams == 1) {
         if (wave < uint32_t(W::COMPUTE) && stream == 0) {
-            if (real && j == 0) *reinterpret_cast<floatx2 *>(a.part_ml + 2 * slot) = floatx2{m_run, lost ? __builtin_nanf("") : l_run * (1.0f / P_UP)};
+            if (real && j == 0) *reinterpret_cast<floatx2 *>(a.part_ml + 2 * slot) = floatx2{m_run, sync.lost ? __builtin_nanf("") : l_run * (1.0f / P_UP)};
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 if (real) put(i, piece(i));
@@ -449,7 +399,7 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
         floatx2 *xm = reinterpret_cast<floatx2 *>(lds_raw + W::XM_OFF);
         __syncthreads();  // nobody reads a slot any more
         if (wave < uint32_t(W::COMPUTE) && stream < streams) {
-            if (j == 0) xm[wave * 16 + n] = floatx2{m_run, lost ? __builtin_nanf("") : l_run * (1.0f / P_UP)};
+            if (j == 0) xm[wave * 16 + n] = floatx2{m_run, sync.lost ? __builtin_nanf("") : l_run * (1.0f / P_UP)};
 #pragma unroll
             for (int i = 0; i < 16; i++) xo[(wave * 16 + i) * 64 + lane] = piece(i);
         }
@@ -478,7 +428,7 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
             }
         }
     }
-    if (__builtin_expect(lost != 0, 0)) wait_gave_up(a.status, a.part_ml, lost, a.rows, a.nsplits, split, a.heads, kv);
+    if (__builtin_expect(sync.lost != 0, 0)) wait_gave_up(a.status, a.part_ml, sync.lost, a.rows, a.nsplits, split, a.heads, kv);
 }
 
 template <int BITS, int TILES>

@@ -48,13 +48,6 @@ struct HalfRows {
 // P_UP and the sums so far need no rescaling.  It is followed in whole numbers: what is rescaled, and what
 // the merge multiplies a split with, is a power of two then, and the exponentials' arguments are rounded once.
 constexpr float MAX_SLACK = 1.0f;
-// x * y as f16 hi and lo parts: hi with the product's low mantissa bits cut off, lo what that leaves of the exact product (one
-// fused operation from it to the f16).
-__device__ __forceinline__ void split_product(float x, float y, _Float16 &hi, _Float16 &lo) {
-    hi = (_Float16)__builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x * y) & 0xffffe000u);
-    lo = (_Float16)fmaf(x, y, -(float)hi);
-}
-constexpr float NEVER = -3e38f;  // the score of a masked token: below any maximum, its probability is 0
 
 template <int TILES, bool PREP>
 __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, const PrepArgs *prep) {
@@ -93,42 +86,10 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
 
     // ---- the context and this workgroup's share of it, as in attention_partial_body ----
     const uint32_t max_len = PREP ? tokens_before(a, position, kv_len) : min(position + a.rows, a.capacity);
-    const uint32_t nblocks = (max_len + BLOCK - 1) / BLOCK;
-    uint32_t blk_begin = split, blk_end = split + 1;
-    if (nblocks <= context_splits) {
-        if (split >= nblocks) return;
-    } else {
-        blk_begin = split * nblocks / context_splits;
-        blk_end = (split + 1) * nblocks / context_splits;
-    }
-    const uint32_t first_tok = blk_begin * BLOCK, limit = min(max_len, blk_end * BLOCK);  // tokens of this share
-    const uint32_t slots = (limit - first_tok + W::SLOT_TOKENS - 1) / W::SLOT_TOKENS;
-    // four splits in a row start a quarter of their share apart (see attention_partial_body)
-    const uint32_t first_slot = (split & 3) * slots / 4;
-    auto start_of = [&](uint32_t u) {
-        const uint32_t at = u + first_slot < slots ? u + first_slot : u + first_slot - slots;
-        return first_tok + at * W::SLOT_TOKENS;
-    };
-
-    // (counters and bounded waits as in attention_partial_s_body)
-    auto raise = [&](uint32_t c) {
-        asm volatile("" ::: "memory");
-        if (lane == 0) __hip_atomic_fetch_add(sync_lds + c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        asm volatile("" ::: "memory");
-    };
-    uint32_t lost = 0;
-    auto await = [&](uint32_t c, uint32_t want) {
-        asm volatile("" ::: "memory");
-        uint32_t left = W::SPIN_LIMIT;
-#pragma nounroll
-        do {
-            const uint32_t v = __hip_atomic_load(sync_lds + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            if (__builtin_amdgcn_readfirstlane(v) >= want) break;
-            __builtin_amdgcn_s_sleep(1);
-        } while (--left);
-        if (__builtin_expect(left == 0, 0)) lost = 0x200u + c;
-        asm volatile("" ::: "memory");
-    };
+    const SlotShare<W::SLOT_TOKENS> share(max_len, split, context_splits);
+    if (share.empty()) return;
+    const uint32_t limit = share.limit, slots = share.slots;
+    LdsCounters<W::SPIN_LIMIT, 0x200u> sync{sync_lds, lane};
 
     floatx4 acc[16];  // O^T: dims 16 T + 4 j .. + 3 of the lane's pair
     float m_run = NO_SCORE, l_run = 0.0f;
@@ -146,7 +107,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
         // instruction i brings the rows 2 i and 2 i + 1; rows past the share are the last one again (their scores are masked)
         const uint32_t last = limit - 1, half = lane >> 5, piece = lane & 31;
         auto request = [&](uint32_t u, bool values) {
-            const uint32_t t0 = start_of(u), to = lds0 + (u % W::PLACES) * W::SLOT + (values ? W::PART : 0);
+            const uint32_t t0 = share.start_of(u), to = lds0 + (u % W::PLACES) * W::SLOT + (values ? W::PART : 0);
             const void *src = values ? a.vdata : a.kdata;
 #pragma unroll
             for (int i = 0; i < W::LOADS; i++) {
@@ -157,29 +118,29 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
         uint32_t mine = 0;
         for (uint32_t u = L; u < slots; u += W::LOADERS, mine++) {
             const uint32_t at = u % W::PLACES, use = u / W::PLACES, before = (u - W::LOADERS) % W::PLACES;
-            if (use) await(W::C_KFREE + at, TILES * use);
+            if (use) sync.await(W::C_KFREE + at, TILES * use);
             request(u, false);
             if (use == 0) request(u, true);
             if (mine) {
                 if (use == 0) __builtin_amdgcn_s_waitcnt(vmcnt_only(3 * W::LOADS));
                 else __builtin_amdgcn_s_waitcnt(vmcnt_only(2 * W::LOADS));
-                raise(W::C_KEYS + before);
+                sync.raise(W::C_KEYS + before);
             }
             if (use) {
-                await(W::C_VFREE + at, TILES * use);
+                sync.await(W::C_VFREE + at, TILES * use);
                 request(u, true);
             }
             if (mine) {
                 __builtin_amdgcn_s_waitcnt(vmcnt_only(2 * W::LOADS));
-                raise(W::C_VALUES + before);
+                sync.raise(W::C_VALUES + before);
             }
         }
         if (mine) {
             const uint32_t at = (L + (mine - 1) * W::LOADERS) % W::PLACES;
             __builtin_amdgcn_s_waitcnt(vmcnt_only(W::LOADS));
-            raise(W::C_KEYS + at);
+            sync.raise(W::C_KEYS + at);
             __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-            raise(W::C_VALUES + at);
+            sync.raise(W::C_VALUES + at);
         }
     } else {
         // ---- the query operands: 16 * scale * log2(e) * q as f16 hi and lo parts ----
@@ -192,21 +153,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
                 rope[lane] = float2{s, c};
             }
             wave_sync();
-            float sum = 0.0f;
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) sum += q[s][e] * q[s][e];
-            }
-            const float scale = norm_scale(across_rows<16, 64>(sum, SumOp()), prep->p.eps);
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-                const float4 *w = reinterpret_cast<const float4 *>(prep->q_norm + 32 * s + 8 * j);
-                const float4 f0 = w[0], f1 = w[1];
-                const float wv[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
-#pragma unroll
-                for (int e = 0; e < 8; e++) q[s][e] *= scale * wv[e];
-            }
+            norm_query(q, *prep, [&](int s) { return 32 * s + 8 * j; });
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const float2 sc = rope[((pair >> 3) - 2 * tile) * 32 + 8 * j + e];
@@ -237,9 +184,9 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
         const uint32_t k_lane = lds0 + n * W::ROW + ((j ^ n) << 4);  // (16 n' + n: the same turn)
         const uint32_t v_row = 4 * j + (n >> 2), v_lane = lds0 + W::PART + v_row * W::ROW + (v_row << 5) + (n & 3) * 8;
         for (uint32_t u = 0; u < slots; u++) {
-            const uint32_t at = u % W::PLACES, use = u / W::PLACES, t0 = start_of(u);
+            const uint32_t at = u % W::PLACES, use = u / W::PLACES, t0 = share.start_of(u);
             // ---- S^T = K Q^T of the slot's two blocks, hi and lo parts side by side ----
-            await(W::C_KEYS + at, use + 1);
+            sync.await(W::C_KEYS + at, use + 1);
             floatx4 hi[4][2], lo[2];  // [64 dims][block]: two products to a sum of hi parts, as in attention_partial_body
 #pragma unroll
             for (int b = 0; b < 2; b++) hi[0][b] = hi[1][b] = hi[2][b] = hi[3][b] = lo[b] = floatx4{0, 0, 0, 0};
@@ -266,7 +213,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
             float x[8];  // tokens 4 j .. + 3 of block 0, then of block 1
 #pragma unroll
             for (int e = 0; e < 8; e++) x[e] = ((hi[0][e >> 2][e & 3] + hi[1][e >> 2][e & 3]) + (hi[2][e >> 2][e & 3] + hi[3][e >> 2][e & 3])) + lo[e >> 2][e & 3];
-            raise(W::C_KFREE + at);
+            sync.raise(W::C_KFREE + at);
             if (t0 + W::SLOT_TOKENS > seen_by_all) {
 #pragma unroll
                 for (int e = 0; e < 8; e++) x[e] = t0 + 16 * (e >> 2) + 4 * j + (e & 3) < seen ? x[e] : NEVER;
@@ -298,7 +245,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
             }
             const half8 phi = as_half8(ph[0], ph[1], ph[2], ph[3]), plo = as_half8(pl[0], pl[1], pl[2], pl[3]);
             // ---- O^T += V^T P^T ----
-            await(W::C_VALUES + at, use + 1);
+            sync.await(W::C_VALUES + at, use + 1);
             const uint32_t v_at = v_lane + at * W::SLOT;
             half8 vop[2][4];
             auto read_values = [&](int lot) {
@@ -321,7 +268,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
                 for (int i = 0; i < 4; i++) acc[4 * lot + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[lot & 1][i], plo, acc[4 * lot + i], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            raise(W::C_VFREE + at);
+            sync.raise(W::C_VFREE + at);
         }
         l_run = across_rows<16, 64>(l_run, SumOp());
     }
@@ -329,7 +276,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
     // ---- the partial of every pair ----
     if (wave < uint32_t(W::COMPUTE) && 16 * tile + n < real_rows) {
         const size_t slot = (size_t(pair >> 3) * a.nsplits + split) * a.heads + kv * 8 + (pair & 7);
-        if (j == 0) *reinterpret_cast<floatx2 *>(a.part_ml + 2 * slot) = floatx2{m_run, lost ? __builtin_nanf("") : l_run * (1.0f / P_UP)};
+        if (j == 0) *reinterpret_cast<floatx2 *>(a.part_ml + 2 * slot) = floatx2{m_run, sync.lost ? __builtin_nanf("") : l_run * (1.0f / P_UP)};
         float *dst = a.part_o + slot * DIM + 4 * j;
 #pragma unroll
         for (int T = 0; T < 16; T++) {
@@ -339,7 +286,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
             else *reinterpret_cast<floatx4 *>(dst + 16 * T) = value;
         }
     }
-    if (__builtin_expect(lost != 0, 0)) wait_gave_up(a.status, a.part_ml, lost, a.rows, a.nsplits, split, a.heads, kv);
+    if (__builtin_expect(sync.lost != 0, 0)) wait_gave_up(a.status, a.part_ml, sync.lost, a.rows, a.nsplits, split, a.heads, kv);
 }
 
 // (two waves per SIMD: with four waves in all the compiler would take more than 256 registers, half of them through copies)
