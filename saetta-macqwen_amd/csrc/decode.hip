@@ -2969,7 +2969,7 @@ constexpr uint32_t HALF_ROWS_FROM = 3;
 constexpr uint32_t MANY_NEW_ROWS_FROM = 48 * 1024;
 
 // Rows over codes that take the kernel with waves of their own (attention_partial_kernel_c), by the cache's capacity; us a
-// layer in a plan, the kernel before it -> this one:
+// layer in a plan with the store taken in, the kernel before it -> this one:
 //   two rows from 48k: behind up to a length of 34k, where a share is a single round of the keys-first kernel (of 65536, 8-bit: 2000 13.4
 //   -> 13.7, 12000 14.7 -> 15.6, 32768 17.4 -> 19.2; 4-bit 13.5 -> 13.9, 14.8 -> 15.5, 17.0 -> 18.9) and ahead from there (37000 21.8 ->
 //   20.1, 44000 22.8 -> 21.2, 57123 26.6 -> 23.7; 20.8 -> 19.6, 21.7 -> 19.7, 26.4 -> 21.6; 131000 45.1 -> 30.6).  The length is not known
@@ -2979,13 +2979,18 @@ constexpr uint32_t MANY_NEW_ROWS_FROM = 48 * 1024;
 //   21.7 -> 21.3, 32768 23.6 -> 22.7, 57123 35.7 -> 27.6; 4 rows, 4-bit, 19.0 -> 16.7, 21.3 -> 20.1, 22.9 -> 23.6, 25.0 -> 25.0, 36.7 -> 29.6
 //   five rows and more: 6 rows, 8-bit, 300 16.8 -> 15.4, 12000 26.9 -> 25.7, 57123 47.1 -> 38; 8 rows 19.1 -> 15.6, 31.6 -> 28.6, 54.8 ->
 //   42; 5 and 6 rows of 4-bit codes from 28k: 6 rows 4000 24.0 -> 22.7, 8000 24.9 -> 25.7, 20000 29.5 -> 29.3, 30000 34.8 -> 32.3
+// Attention by itself has 128 splits for the context instead of 127 and less, and the keys-first kernel is further ahead in its
+// single round: two rows from 64k (8-bit, 6000 11.7 -> 13.2, 32768 15.5 -> 17.5, 37000 20.0 -> 19.4, 57123 25.1 -> 22.1), four rows of 8
+// bits from 36k (300 12.7 -> 11.2, 12000 18.1 -> 18.0, 24500 19.4 -> 20.1, 32768 20.7 -> 21.6, 34700 22.2 -> 23.4, 37000 26.7 -> 23.5); three
+// rows (8-bit, 24500 18.3 -> 18.8, 32768 20.5 -> 20.5, 37000 25.8 -> 22.2) and 4-bit codes as above.
 // It is ahead in larger caches still (4 rows, 8-bit, at 150000 tokens 66.5 -> 48.4, 8 rows 107 -> 79), but stops at 64k tokens, 2 to
 // 4 rows of 4-bit codes at 128k, so that results stay what they were: the sums of the codes and of the biases nearly cancel, the
 // more the longer the context, and the order in which 32-bit sums are taken shows as 4e-6 to 8e-6 of the results at 64000 tokens,
 // 1.0e-5 to 1.5e-5 at 131000 (2 to 4 rows, 4-bit, 7e-6).  Either kernel is further than that from 64 bits.
-constexpr bool code_rows(int bits, uint32_t rows, uint32_t capacity) {
+constexpr bool code_rows(int bits, uint32_t rows, uint32_t capacity, bool with_store) {
     constexpr uint32_t K = 1024;
-    const uint32_t from = rows >= 7 || (rows >= 5 && bits == 8) ? 0 : rows >= 5 ? 28 * K : rows >= 3 ? 24 * K : 48 * K;
+    const uint32_t few = rows == 2 ? (with_store ? 48 * K : 64 * K) : rows == 4 && bits == 8 && !with_store ? 36 * K : 24 * K;
+    const uint32_t from = rows >= 7 || (rows >= 5 && bits == 8) ? 0 : rows >= 5 ? 28 * K : few;
     const uint32_t to = rows <= 4 && bits == 4 ? 128 * K : 64 * K;
     return bits != 16 && rows >= 2 && capacity >= from && capacity <= to;
 }
@@ -3005,7 +3010,7 @@ void launch_partial(hipStream_t stream, const PartialArgs &a, bool one_per_cu, b
         }
     }
     if constexpr (BITS != 16 && !PACKED) {
-        if (keys_first && code_rows(BITS, a.rows, a.capacity)) {
+        if (keys_first && code_rows(BITS, a.rows, a.capacity, token != nullptr)) {
             using W = CodeRows<BITS, TILES>;
             if (token) launch(attention_token_kernel_c<BITS, TILES>, dim3(token->a.nsplits - 1 + a.rows, a.kv_heads), W::THREADS_, W::LDS_BYTES, stream, *token);
             else launch(attention_partial_kernel_c<BITS, TILES>, grid, W::THREADS_, W::LDS_BYTES, stream, a);
@@ -3107,7 +3112,7 @@ bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const fl
     }
     token = TokenArgs{a, prep, SAETTA_GQA_GROUP};
     const uint32_t room = MAX_SPLITS / 2;  // workgroups of a kv head, one to a CU
-    if (keys_first && (bits == 16 || code_rows(bits, a.rows, a.capacity))) {
+    if (keys_first && (bits == 16 || code_rows(bits, a.rows, a.capacity, true))) {
         // a workgroup per new row, for which a full context gives up CUs (two rows to one: 6 rows at 57123 tokens 36.2 against
         // 35.5 us a layer)
         if (a.rows > NEW_ROWS && a.capacity < MANY_NEW_ROWS_FROM) return false;
@@ -3161,7 +3166,7 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
     // many partials is worth more (measured: 19.4 against 20.6 us per layer at 32k, 28.3 against 29.7 at
     // 64k, but 44 against 35 at 146k, 4-bit).  Both stages of a call derive the same number from the same arguments; where
     // a plan's reduce stage makes a token step of the launches before it, the number is the token step's.
-    const bool loaders = bits == 16 ? rows >= HALF_ROWS_FROM : code_rows(bits, rows, capacity) || (rows <= 4 && capacity >= KEYS_FIRST_FROM);
+    const bool loaders = bits == 16 ? rows >= HALF_ROWS_FROM : code_rows(bits, rows, capacity, false) || (rows <= 4 && capacity >= KEYS_FIRST_FROM);
     const bool keys_first = loaders && !(stages & SAETTA_STAGE_NO_LOADERS);
     const bool one_per_cu = rows >= 2 || bits == 16 || capacity <= 80 * 1024 || keys_first;
     if (one_per_cu && nsplits > MAX_SPLITS / 2) nsplits = MAX_SPLITS / 2;

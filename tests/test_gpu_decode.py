@@ -390,7 +390,7 @@ def test_rows_over_codes_slot_by_slot(kind, m):
     # slots than streams, the loaders' whole depth, the ring of 8 or 16 places and around it.  The rows past the context are
     # poisoned.
     rng = np.random.default_rng(5400 + m)
-    capacity = 49152
+    capacity = 65536
     k = rng.standard_normal((1100, VALUES)).astype(np.float32)
     v = rng.standard_normal((1100, VALUES)).astype(np.float32)
     q = rng.standard_normal((m, H, D)).astype(np.float32)
@@ -418,7 +418,7 @@ def test_rows_over_codes_of_large_values(kind, m):
     # maxima; one q head in two sees them fall instead.  The bound is that of the other tests, for normal values whose groups
     # span 4.8, at the span of these; the hi and lo parts of q as in test_rows_over_halves_follow_a_growing_maximum.
     rng = np.random.default_rng(5500 + m)
-    capacity, step = 49152, 0.02
+    capacity, step = 65536, 0.02
     span = 250.0 * (255 if kind is saetta.KvBits.Eight else 15)
     k = (0.3 * rng.standard_normal((1100, KV, D))).astype(np.float32)
     k[:, :, 0] = step * np.arange(1100)[:, None]
@@ -449,7 +449,7 @@ def test_rows_over_codes_of_equal_keys_lose_nothing(kind, m):
     # it is, and only the f32 sums round, by half a unit (2^-25) of sums below 2.4.  A maximum that is not the score itself
     # makes the probabilities' lo parts, cut off, 2^-23 of the codes' part too small, 1.4e-7 with the gate.
     rng = np.random.default_rng(5600 + m)
-    capacity = 49152
+    capacity = 65536
     rows = saetta.AttentionRows(H, KV, capacity, m)
     rows.splits = 1
     for tokens in [64, 160]:
