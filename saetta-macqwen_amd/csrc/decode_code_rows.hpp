@@ -89,9 +89,22 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
 
     // ---- the context and this workgroup's share of it, as in attention_partial_body ----
     const uint32_t max_len = PREP ? tokens_before(a, position, kv_len) : min(position + a.rows, a.capacity);
-    const SlotShare<W::SLOT_TOKENS> share(max_len, split, context_splits);
-    if (share.empty()) return;
-    const uint32_t limit = share.limit, slots = share.slots;
+    const uint32_t nblocks = (max_len + BLOCK - 1) / BLOCK;
+    uint32_t blk_begin = split, blk_end = split + 1;
+    if (nblocks <= context_splits) {
+        if (split >= nblocks) return;
+    } else {
+        blk_begin = split * nblocks / context_splits;
+        blk_end = (split + 1) * nblocks / context_splits;
+    }
+    const uint32_t first_tok = blk_begin * BLOCK, limit = min(max_len, blk_end * BLOCK);  // tokens of this share
+    const uint32_t slots = (limit - first_tok + W::SLOT_TOKENS - 1) / W::SLOT_TOKENS;
+    // four splits in a row start a quarter of their share apart (see attention_partial_body)
+    const uint32_t first_slot = (split & 3) * slots / 4;
+    auto start_of = [&](uint32_t u) {
+        const uint32_t at = u + first_slot < slots ? u + first_slot : u + first_slot - slots;
+        return first_tok + at * W::SLOT_TOKENS;
+    };
     LdsCounters<W::SPIN_LIMIT, 0x300u, LARGE_SLOT - 1> sync{sync_lds, lane};
 
     floatx4 acc[16];  // O^T of the codes: [4 g + e][i] is dim 64 g + 16 i + 4 j + e of the lane's pair
@@ -119,7 +132,7 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
         constexpr uint32_t UNITS = W::ROW / 16, ROWS_EACH = 64 / UNITS;  // 16-byte units of a row, rows a load brings
         const uint32_t last = limit - 1, sub_row = lane / UNITS, unit = lane % UNITS;
         auto request = [&](uint32_t u) {
-            const uint32_t t0 = share.start_of(u), to = lds0 + (u % W::PLACES) * W::SLOT;
+            const uint32_t t0 = start_of(u), to = lds0 + (u % W::PLACES) * W::SLOT;
             const uint32_t sc = (min(t0 + (lane >> 1), last) * kvh + kv) * 8 + (lane & 1) * 4;
             dma4(to + W::SC_OFF, sc, a.kscales);
             dma4(to + W::SC_OFF + W::SC_ARRAY, sc, a.kbiases);
@@ -233,7 +246,7 @@ __device__ __forceinline__ void attention_code_rows_body(const PartialArgs &a, c
         const uint32_t v_lane = W::V_OFF + 4 * j * W::ROW + j * (W::ROW / 4) + (BITS == 8 ? pn : pn >> 1) * 4;
         const uint32_t sc_lane = W::SC_OFF + 4 * j * 8;  // scales of tokens 4 j .. + 3: 32 bytes
         for (uint32_t u = stream; u < slots; u += W::STREAMS) {
-            const uint32_t at = u % W::PLACES, use = u / W::PLACES, t0 = share.start_of(u), here = lds0 + at * W::SLOT;
+            const uint32_t at = u % W::PLACES, use = u / W::PLACES, t0 = start_of(u), here = lds0 + at * W::SLOT;
             // ---- S^T = K Q^T of the slot's two blocks ----
             const float slack = sync.await(W::C_KEYS + at, use + 1) < LARGE_SLOT ? CODE_MAX_SLACK : 0.0f;
             KeyRegs<BITS> kreg[2][4];

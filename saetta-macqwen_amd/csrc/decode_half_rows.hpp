@@ -86,9 +86,22 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
 
     // ---- the context and this workgroup's share of it, as in attention_partial_body ----
     const uint32_t max_len = PREP ? tokens_before(a, position, kv_len) : min(position + a.rows, a.capacity);
-    const SlotShare<W::SLOT_TOKENS> share(max_len, split, context_splits);
-    if (share.empty()) return;
-    const uint32_t limit = share.limit, slots = share.slots;
+    const uint32_t nblocks = (max_len + BLOCK - 1) / BLOCK;
+    uint32_t blk_begin = split, blk_end = split + 1;
+    if (nblocks <= context_splits) {
+        if (split >= nblocks) return;
+    } else {
+        blk_begin = split * nblocks / context_splits;
+        blk_end = (split + 1) * nblocks / context_splits;
+    }
+    const uint32_t first_tok = blk_begin * BLOCK, limit = min(max_len, blk_end * BLOCK);  // tokens of this share
+    const uint32_t slots = (limit - first_tok + W::SLOT_TOKENS - 1) / W::SLOT_TOKENS;
+    // four splits in a row start a quarter of their share apart (see attention_partial_body)
+    const uint32_t first_slot = (split & 3) * slots / 4;
+    auto start_of = [&](uint32_t u) {
+        const uint32_t at = u + first_slot < slots ? u + first_slot : u + first_slot - slots;
+        return first_tok + at * W::SLOT_TOKENS;
+    };
     LdsCounters<W::SPIN_LIMIT, 0x200u> sync{sync_lds, lane};
 
     floatx4 acc[16];  // O^T: dims 16 T + 4 j .. + 3 of the lane's pair
@@ -107,7 +120,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
         // instruction i brings the rows 2 i and 2 i + 1; rows past the share are the last one again (their scores are masked)
         const uint32_t last = limit - 1, half = lane >> 5, piece = lane & 31;
         auto request = [&](uint32_t u, bool values) {
-            const uint32_t t0 = share.start_of(u), to = lds0 + (u % W::PLACES) * W::SLOT + (values ? W::PART : 0);
+            const uint32_t t0 = start_of(u), to = lds0 + (u % W::PLACES) * W::SLOT + (values ? W::PART : 0);
             const void *src = values ? a.vdata : a.kdata;
 #pragma unroll
             for (int i = 0; i < W::LOADS; i++) {
@@ -184,7 +197,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
         const uint32_t k_lane = lds0 + n * W::ROW + ((j ^ n) << 4);  // (16 n' + n: the same turn)
         const uint32_t v_row = 4 * j + (n >> 2), v_lane = lds0 + W::PART + v_row * W::ROW + (v_row << 5) + (n & 3) * 8;
         for (uint32_t u = 0; u < slots; u++) {
-            const uint32_t at = u % W::PLACES, use = u / W::PLACES, t0 = share.start_of(u);
+            const uint32_t at = u % W::PLACES, use = u / W::PLACES, t0 = start_of(u);
             // ---- S^T = K Q^T of the slot's two blocks, hi and lo parts side by side ----
             sync.await(W::C_KEYS + at, use + 1);
             floatx4 hi[4][2], lo[2];  // [64 dims][block]: two products to a sum of hi parts, as in attention_partial_body
