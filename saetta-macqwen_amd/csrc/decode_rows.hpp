@@ -1,6 +1,6 @@
 // What decode_half_rows.hpp and decode_code_rows.hpp share: counters in LDS, the norm of a computing wave's query values, the
 // split of a product.  Included by decode.hip, inside its namespace.  (A workgroup's share of the context stays in both: as a
-// struct of its own it made the loops of the half rows another 1 % slower, 6 rows at 57123 tokens 35.5 -> 35.9 us a layer.)
+// struct of its own it changed the loops: 6 rows over halves at 57123 tokens 35.5 -> 35.9 us a layer.)
 
 // Counters in LDS through which waves meet (see attention_partial_s_body): one lane adds, the others poll, and every wait is
 // bounded.  `lost`: the counter, behind the kernel's CODE, of a wait that gave up.
