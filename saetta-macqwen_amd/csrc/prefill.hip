@@ -776,7 +776,8 @@ __global__ __launch_bounds__(MERGE_THREADS) void prefill_merge_kernel(PrefillArg
 // row -> in turns: 16 at 500 20.5 -> 18.6, 300 from 0 19.1 -> 17.4, 500 from 0 23.1 -> 20.5, 500 at 500 32.2 -> 26.5; codes as f32 -> as halves: 8-bit
 // 23.8 -> 20.2, 24.9 -> 21.8, 34.4 -> 28.8, 4-bit 23.3 -> 20.2, 23.4 -> 21.4, 33.3 -> 29.4, and no further from 64 bits.
 // Halves fill the registers: what depends on the lane alone is made anew where it is used (`at`), so that nothing spills; three
-// spilled registers cost a launch 1 us (300 from 0 18.3), the instructions 0.1 to 0.5 (16 at 500 18.1).
+// spilled registers cost a launch 1 us (300 from 0 18.3), the instructions 0.1 to 0.5 (16 at 500 18.1).  8-bit codes spill four, stored
+// before the loop and read back behind it.
 // One maximum for the eight blocks of a round, a wave 32 of the dims of all of them and nothing to join at the end took 1
 // to 2.5 us less with codes, but not with its precision: of each block the largest probability is now 1, without a
 // rounding, and with the largest of eight blocks alone an output was up to 1.2 times as far from 64 bits.
