@@ -84,6 +84,12 @@ def test_fused_step_equals_the_ops_one_by_one(kind, capacity, rows):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), position
 
 
+@pytest.mark.parametrize("kind,capacity,rows", [(saetta.KvBits.Eight, 24576, 4), (saetta.KvBits.Eight, 49152, 2), (saetta.KvBits.Four, 49152, 2)])
+def test_fused_step_by_another_kernel_than_the_ops(kind, capacity, rows):
+    # rows over codes whose line between the loader kernels lies lower with the store taken in than for attention by itself
+    test_fused_step_equals_the_ops_one_by_one(kind, capacity, rows)
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("rows", [5, 6, 7, 8])
 def test_many_rows_of_a_large_cache_take_the_store_in(rows, kind):
