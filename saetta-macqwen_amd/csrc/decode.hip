@@ -2867,51 +2867,61 @@ constexpr int STATIC_MAX_DEVICES = 64;
 float *g_static_scratch[STATIC_MAX_DEVICES] = {};
 
 // One workgroup per (q head, row, 16 dims of the head): wave w takes a quarter of the splits, lane
-// (slot = lane / 4, quad = lane % 4) up to four of them and four dims.  Every load is requested before
-// anything is waited for; a wave sums its splits relative to its own maximum, so that the four waves
-// meet once, through LDS.
+// (slot = lane / 4, quad = lane % 4) PER_LANE of them and four dims.  Latency is all there is to it: every load is
+// requested before anything is waited for (buffer loads, whose slots past the last split read zero: with a branch around each
+// the compiler waited for one before it asked for the next, and for the position before the first), a wave sums its splits
+// relative to its own maximum, so that the four waves meet once, through LDS.
+// A layer's token step, us, ten layers in a graph: 8-bit 300 tokens of 8192 9.1 -> 8.6, halves 4096 of 8192 10.9 -> 10.3, 8-bit 32768
+// 16.8 -> 16.0; eight rows at 1000 tokens 18.3 -> 17.3.
+// WAIT: slots past the splits at work are left out of the requests, which have to wait for the position then.  One and two
+// rows read them all the same: the wait costs more than up to 2 MB of old partials a row.
 constexpr int REDUCE_DIMS = 16;
+template <int PER_LANE, bool WAIT>
 __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
     __shared__ float wave_m[4], wave_l[4];
     __shared__ floatx4 wave_o[4][4];
     const uint32_t h = blockIdx.x, row = blockIdx.y, slice = blockIdx.z;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, slot = lane >> 2, quad = lane & 3;
-    const float *ml = a.part_ml + size_t(2) * row * a.nsplits * a.heads;
-    const float *po = a.part_o + size_t(row) * a.nsplits * a.heads * DIM;
-    // splits of this wave: per_wave (a multiple of 16) from per_wave * wave on; of this lane: slot + 16 i
-    const uint32_t per_wave = (a.nsplits + 63) / 64 * 16;
-    constexpr int PER_LANE = MAX_SPLITS / 64;
-    const uint32_t seen = min(a.decode_len ? a.tp->kv_len : a.tp->position + a.rows, a.capacity);
-    const uint32_t max_len = a.last_is_new ? min(seen, a.tp->position) : seen;
-    const uint32_t nblocks = (max_len + BLOCK - 1) / BLOCK;
-    const uint32_t parts = min(a.nsplits - a.last_is_new, nblocks), fresh = a.last_is_new ? a.nsplits - 1 : ~0u;
-    // Slots past the splits at work hold old values: they are dropped by select, never multiplied.  (One and two rows read
-    // them all the same: waiting for the length first costs more than up to 2 MB of old partials a row.)
-    const uint32_t limit = a.rows > 2 ? parts : a.nsplits;
+    const size_t qh = size_t(row) * a.heads + h;
+    const uint32_t position = a.tp->position, kv_len = a.tp->kv_len;
+    uint32_t parts = 0, fresh = 0;
+    auto splits_at_work = [&]() {
+        const uint32_t seen = min(a.decode_len ? kv_len : position + a.rows, a.capacity);
+        const uint32_t max_len = a.last_is_new ? min(seen, position) : seen;
+        parts = min(a.nsplits - a.last_is_new, (max_len + BLOCK - 1) / BLOCK), fresh = a.last_is_new ? a.nsplits - 1 : ~0u;
+    };
+    if constexpr (WAIT) splits_at_work();
+    const uint32_t records = a.nsplits * a.heads;
+    const __amdgpu_buffer_rsrc_t o_rsrc = make_rsrc(a.part_o + size_t(row) * records * DIM, records * DIM * 4);
+    const __amdgpu_buffer_rsrc_t ml_rsrc = make_rsrc(a.part_ml + size_t(row) * records * 2, records * 8);
+    const __amdgpu_buffer_rsrc_t g_rsrc = make_rsrc(a.q_and_gate + (qh * 2 + 1) * DIM, DIM * 4);
+    auto split_of = [&](int i) { return 16 * PER_LANE * wave + slot + 16 * i; };
     floatx2 mlv[PER_LANE];
     floatx4 pv[PER_LANE];
 #pragma unroll
     for (int i = 0; i < PER_LANE; i++) {
-        const uint32_t c = per_wave * wave + slot + 16 * i;
-        mlv[i] = floatx2{NO_SCORE, 0.0f};
-        pv[i] = floatx4{0, 0, 0, 0};
-        if (16 * uint32_t(i) < per_wave && (c < limit || c == fresh)) {
-            mlv[i] = *reinterpret_cast<const floatx2 *>(ml + 2 * (size_t(c) * a.heads + h));
-            pv[i] = *reinterpret_cast<const floatx4 *>(po + (size_t(c) * a.heads + h) * DIM + REDUCE_DIMS * slice + 4 * quad);
-        }
+        const uint32_t c = split_of(i), record = c * a.heads + h;
+        const bool need = c < (WAIT ? parts : a.nsplits) || (WAIT && c == fresh);
+        mlv[i] = __builtin_bit_cast(floatx2, __builtin_amdgcn_raw_buffer_load_b64(ml_rsrc, need ? int(record * 8) : OOB, 0, 0));
+        pv[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(o_rsrc, need ? int(record * (DIM * 4) + (REDUCE_DIMS * slice + 4 * quad) * 4) : OOB, 0, 0));
     }
-    const size_t qh = size_t(row) * a.heads + h;
-    const float g = tid < REDUCE_DIMS ? a.q_and_gate[qh * 2 * DIM + DIM + REDUCE_DIMS * slice + tid] : 0.0f;
+    const float g = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(g_rsrc, tid < REDUCE_DIMS ? int(REDUCE_DIMS * slice + tid) * 4 : OOB, 0, 0));
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!WAIT) splits_at_work();
     float m[PER_LANE], mx = NO_SCORE;
 #pragma unroll
     for (int i = 0; i < PER_LANE; i++) {
-        const uint32_t c = per_wave * wave + slot + 16 * i;
-        const bool live = 16 * uint32_t(i) < per_wave && (c < parts || c == fresh);
+        // (slots past the splits at work hold old values: dropped by select, never multiplied)
+        const uint32_t c = split_of(i);
+        const bool live = c < parts || c == fresh;
         m[i] = live ? mlv[i][0] : NO_SCORE;
         if (!live) mlv[i][1] = 0.0f, pv[i] = floatx4{0, 0, 0, 0};
         mx = fmaxf(mx, m[i]);
     }
-    mx = group_reduce<64>(mx, MaxOp());  // the wave's maximum
+    // the wave's maximum; like the sums, over the 16 slots (lanes 4 apart: two steps inside a row of 16 lanes, two across
+    // rows), the four quads of a slot having the same m and l
+    mx = fmaxf(mx, dpp<0x124>(mx)), mx = fmaxf(mx, dpp<0x128>(mx));  // row_ror 4, row_ror 8
+    mx = across_rows<16, 64>(mx, MaxOp());
     float l = 0.0f;
     floatx4 o = {0, 0, 0, 0};
 #pragma unroll
@@ -2920,8 +2930,7 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
         l += w * mlv[i][1];
         o += pv[i] * w;
     }
-    // over the 16 slots (lanes 4 apart: two steps inside a row of 16 lanes, two across rows); l is the same in the four quads
-    l += dpp<0x124>(l), l += dpp<0x128>(l);  // row_ror 4, row_ror 8
+    l += dpp<0x124>(l), l += dpp<0x128>(l);
     l = across_rows<16, 64>(l, SumOp());
 #pragma unroll
     for (int e = 0; e < 4; e++) {
@@ -2931,6 +2940,7 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
     }
     if (lane == 0) wave_m[wave] = mx, wave_l[wave] = l;
     if (lane < 4) wave_o[wave][lane] = o;  // (lane = quad)
+    const float open = __builtin_amdgcn_rcpf(1.0f + __expf(-g));
     __syncthreads();
     if (tid < REDUCE_DIMS) {
         const float M = fmaxf(fmaxf(wave_m[0], wave_m[1]), fmaxf(wave_m[2], wave_m[3]));
@@ -2941,9 +2951,10 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
             total += f * wave_l[w];
             sum += f * wave_o[w][tid >> 2][tid & 3];
         }
-        a.out[qh * DIM + REDUCE_DIMS * slice + tid] = sum * __builtin_amdgcn_rcpf(total) * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
+        a.out[qh * DIM + REDUCE_DIMS * slice + tid] = sum * __builtin_amdgcn_rcpf(total) * open;
     }
 }
+static_assert(MAX_SPLITS <= 4 * 64, "four splits a lane at most");
 
 uint32_t splits_for(uint32_t capacity, uint32_t wanted) {
     // Never more than the 128-token chunks of the capacity, so that scratch sized as
@@ -3197,7 +3208,10 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
             }
         }
         ReduceArgs r{part_o, part_ml, q_and_gate, out, heads, capacity, nsplits, rows, d_tp, decode_len ? 1u : 0u, last_is_new};
-        launch(attention_reduce_kernel, dim3(heads, rows, DIM / REDUCE_DIMS), 256, 0, stream, r);
+        void (*const reduce[][2])(ReduceArgs) = {{attention_reduce_kernel<1, false>, attention_reduce_kernel<1, true>},
+                                                 {attention_reduce_kernel<2, false>, attention_reduce_kernel<2, true>},
+                                                 {attention_reduce_kernel<4, false>, attention_reduce_kernel<4, true>}};
+        launch(reduce[nsplits <= 64 ? 0 : nsplits <= 128 ? 1 : 2][rows > 2], dim3(heads, rows, DIM / REDUCE_DIMS), 256, 0, stream, r);
     }
     return launch_status(what);
 }
@@ -3254,7 +3268,7 @@ int raise_lds_of_bits() {
 }  // namespace
 
 int setup_decode() {
-    if (int rc = load_kernel(reinterpret_cast<const void *>(attention_reduce_kernel))) return rc;
+    if (int rc = load_kernel(reinterpret_cast<const void *>(attention_reduce_kernel<1, false>))) return rc;
     {
         // (runs once per device, with that device current)
         int dev = 0;

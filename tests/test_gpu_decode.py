@@ -659,3 +659,37 @@ def test_other_head_counts(kind, kv_heads):
         plan.set_params(saetta.TokenParams(0, pos))
         plan.build().run()
         assert np.abs(host(one) - want[0]).max() < MAX_ABS_F64, (kind, kv_heads, ctx)
+
+
+@pytest.mark.parametrize("capacity,splits,rows", [(c, s, r) for c, s in [(128, 1), (8192, 17), (8192, 64), (8320, 65), (16384, 128)] for r in (1, 2, 3, 8)]
+                         + [(131072, 256, 1)])
+def test_merge_of_the_splits_by_itself(capacity, splits, rows):
+    # the reduce stage over partials of the test's own, at the edges of 64, 128 and 256 splits, with as many at work as the
+    # length has blocks, NaN in the others: sum_c 2^(m_c - M) o_c / sum_c 2^(m_c - M) l_c, gated
+    rng = np.random.default_rng(splits + rows)
+    quant = splits == 256  # (one row over codes)
+    o, l = rng.standard_normal((rows, splits, H, D)).astype(np.float32), rng.uniform(1, 100, (rows, splits, H)).astype(np.float32)
+    m, qg = rng.uniform(-30, 30, (rows, splits, H)).astype(np.float32), rng.standard_normal((rows, H, 2 * D)).astype(np.float32)
+    any_cache, out = torch.zeros(64, device="cuda"), torch.empty(rows, H, D, device="cuda")
+    dqg, lib, f = dev(qg), saetta.ffi.lib(), saetta.ffi
+    p = f.RowsParamsC(H, KV, capacity, 1.0 / 16.0, rows, splits)
+    for position in sorted({0, 15, 16, 16 * splits - rows - 17, 16 * splits - rows, capacity - rows}):
+        if position < 0:
+            continue
+        work = min(splits, -(-(position + rows) // 16))
+        po, pml = o.copy(), np.stack([m, l], -1)
+        po[:, work:], pml[:, work:] = np.nan, np.nan
+        do, dml, tp = dev(po), dev(pml), saetta.TokenParams(0, position).as_tensor("cuda")
+        out.fill_(float("nan"))
+        a, stream = any_cache.data_ptr(), saetta.host._stream()
+        rest = (do.data_ptr(), dml.data_ptr(), dqg.data_ptr(), out.data_ptr(), p, tp.data_ptr(), f.STAGE_REDUCE | f.STAGE_NO_LOADERS)
+        if quant:
+            c = f.QuantRowsC(a, a, a)
+            f.check(lib.saetta_attn_rows_quant(stream, 8, a, c, c, *rest), "attn_rows_quant")
+        else:
+            f.check(lib.saetta_attn_rows(stream, a, a, a, *rest), "attn_rows")
+        w = np.exp2(m[:, :work].astype(np.float64) - m[:, :work].max(1, keepdims=True))
+        want = np.einsum("rch,rchd->rhd", w, o[:, :work].astype(np.float64)) / np.einsum("rch,rch->rh", w, l[:, :work].astype(np.float64))[..., None]
+        want /= 1 + np.exp(-qg[:, :, D:].astype(np.float64))
+        # 32-bit sums of up to 256 terms, two reciprocals and two exponentials of an ulp or so
+        assert np.abs(host(out) - want).max() <= 4e-6 * np.abs(want).max(), position
