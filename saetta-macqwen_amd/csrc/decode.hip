@@ -349,7 +349,7 @@ __device__ __forceinline__ void new_rows(const PartialArgs &a, const PrepArgs &p
     for (int i = 0; i < 4; i++) qn[i] = p.q_norm[64 * i + lane], kn[i] = p.k_norm[64 * i + lane];
     if (tid < 32 * rows) {
         float s, c;
-        rope_angle(position + (tid >> 5), tid & 31, 32, p.p.log2_theta, s, c);
+        rope_angle(position + (tid >> 5), rope_frequency(tid & 31, 32, p.p.log2_theta), s, c);
         rope[tid] = float2{s, c};
     }
     __syncthreads();
@@ -556,6 +556,7 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
             for (int e = 0; e < 8; e++) v[e] = 0.0f;
         }
     };
+    const uint32_t position = a.tp->position, kv_len = a.tp->kv_len;
     float q_early[TILES * 2][8];
 #pragma unroll
     for (int k = 0; k < TILES * 2; k++) load_q_item(tid + k * THREADS, q_early[k]);
@@ -570,9 +571,13 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
         }
     }
 
+    double frequency = 0.0;
+    if constexpr (PREP) {  // (while the position is on its way)
+        frequency = rope_frequency(tid & 31, 32, prep->p.log2_theta);
+        asm volatile("" : "+v"(frequency));
+    }
+
     // ---- the context and this workgroup's share of it -----------------------------
-    const uint32_t position = a.tp->position;
-    const uint32_t kv_len = a.tp->kv_len;
     // Tokens the last row sees; the longest context of the launch.  (PREP: the tokens before the new ones.)
     const uint32_t max_len = PREP ? tokens_before(a, position, kv_len) : min(a.decode_len ? kv_len : position + a.rows, a.capacity);
     const uint32_t nblocks = (max_len + BLOCK - 1) / BLOCK;
@@ -682,14 +687,14 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
         }
         if (tid < int(32 * a.rows)) {
             float s, c;
-            rope_angle(position + (tid >> 5), tid & 31, 32, prep->p.log2_theta, s, c);
+            rope_angle(position + (tid >> 5), frequency, s, c);
             rope[tid] = float2{s, c};
         }
         __syncthreads();
 #pragma unroll
         for (int t = 0; t < TILES; t++) {
             const float *sq = squares + t * 64 + n;
-            const float scale = norm_scale((sq[0] + sq[16]) + (sq[32] + sq[48]), prep->p.eps);
+            const float scale = query_scale((sq[0] + sq[16]) + (sq[32] + sq[48]), prep->p.eps);
 #pragma unroll
             for (int k = 0; k < 2; k++) {
 #pragma unroll
@@ -1653,14 +1658,14 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
             if (j == 0) zs_lds[(wave * W::PAIRS + p) * 16 + n] = sum;
         }
         raise(W::C_NORM);
-        if (wave < 2) rope_angle(sync_lds[W::C_POSITION] + min(j, M - 1), 16 * (n >> 3) + 8 * wave + (n & 7), 32, prep->p.log2_theta, sine, cosine);
+        if (wave < 2) rope_angle(sync_lds[W::C_POSITION] + min(j, M - 1), rope_frequency(16 * (n >> 3) + 8 * wave + (n & 7), 32, prep->p.log2_theta), sine, cosine);
         await(W::C_NORM, W::WAVES);
 #pragma unroll
         for (int p = 0; p < W::PAIRS; p++) {
             float total = 0.0f;
 #pragma unroll
             for (int w = 0; w < W::WAVES; w++) total += zs_lds[(w * W::PAIRS + p) * 16 + n];
-            const float scale = norm_scale(total, prep->p.eps);
+            const float scale = query_scale(total, prep->p.eps);
 #pragma unroll
             for (int e = 0; e < 8; e++) qv[p][e] *= scale * norm_w[e];
             if (wave < 2) {

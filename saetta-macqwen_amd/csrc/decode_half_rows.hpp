@@ -162,7 +162,7 @@ __device__ __forceinline__ void attention_half_rows_body(const PartialArgs &a, c
             float2 *rope = reinterpret_cast<float2 *>(lds_raw + W::ROPE_OFF + wave * 512);
             {
                 float s, c;
-                rope_angle(position + 2 * tile + (lane >> 5), lane & 31, 32, prep->p.log2_theta, s, c);
+                rope_angle(position + 2 * tile + (lane >> 5), rope_frequency(lane & 31, 32, prep->p.log2_theta), s, c);
                 rope[lane] = float2{s, c};
             }
             wave_sync();

@@ -46,7 +46,7 @@ __device__ __forceinline__ void norm_query(float (&q)[8][8], const PrepArgs &pre
 #pragma unroll
         for (int e = 0; e < 8; e++) sum += q[s][e] * q[s][e];
     }
-    const float scale = norm_scale(across_rows<16, 64>(sum, SumOp()), prep.p.eps);
+    const float scale = query_scale(across_rows<16, 64>(sum, SumOp()), prep.p.eps);
 #pragma unroll
     for (int s = 0; s < 8; s++) {
         const float4 *w = reinterpret_cast<const float4 *>(prep.q_norm + dim_of(s));

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256) void attention_prep_store_kernel(PrepArgs a) {
         if (i < 2 * half) {
             const uint32_t r = i < half ? i : i - half;
             float s, c;
-            rope_angle(position, r, half, a.p.log2_theta, s, c);
+            rope_angle(position, rope_frequency(r, half, a.p.log2_theta), s, c);
             const float u = head[r], w = head[r + half];
             x = i < half ? rope_first(u, w, s, c) : rope_second(u, w, s, c);
         }

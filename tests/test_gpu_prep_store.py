@@ -107,6 +107,30 @@ def test_rotation_is_the_cpus_when_log2_theta_is_exact():
     assert np.allclose(host(k_back).reshape(KV, D)[:, ROPE_DIMS:], wk.reshape(KV, D)[:, ROPE_DIMS:], rtol=4e-7, atol=0)
 
 
+def test_angles_of_any_position():
+    # theta = 2^32: the frequencies are 2^-i and the angles exact.  A key whose values are all alike, x behind the norm (dims
+    # past the rotary ones), gives x c - x s and x s + x c, with s and c the f64 values rounded once.
+    ones, keys = torch.ones(D, device="cuda"), make_cache(saetta.KvBits.Half, 16)
+    k, qg = torch.ones(8 * KV * D, device="cuda"), torch.ones(8 * H * 2 * D, device="cuda")
+    q_out, k_back = torch.empty(8 * H * D, device="cuda"), torch.empty(8, KV, D, device="cuda")
+    plan = saetta.Plan()
+    saetta.record_store(plan, qg, k, k, ones, ones, q_out, *keys, saetta.PrepParams(H, KV, D, ROPE_DIMS, float(2 ** 32), EPS), 16, rows=8, k_back=k_back)
+    built, same, total = plan.build(), 0, 0
+    rng = np.random.default_rng(1)
+    positions = [0, 11, 355, 103993, 262136, 2 ** 30, 2 ** 31 - 8, 2 ** 32 - 9] + [int(2.0 ** e) for e in rng.uniform(0, 32, 60)]
+    for pos in positions:
+        plan.set_params(saetta.TokenParams(0, pos))
+        built.run()
+        got = host(k_back)[:, 0]
+        x = got[:, ROPE_DIMS:ROPE_DIMS + 1].astype(np.float64)
+        angle = (pos + np.arange(8, dtype=np.float64))[:, None] * np.exp2(-np.arange(32.0))
+        s, c = np.sin(angle).astype(np.float32).astype(np.float64), np.cos(angle).astype(np.float32).astype(np.float64)
+        want = np.concatenate([x * c - (x * s).astype(np.float32), x * s + (x * c).astype(np.float32)], 1).astype(np.float32)
+        assert np.abs(got[:, :64] - want).max() <= 2.5e-7, pos  # (an ulp of one of the two, and of the result)
+        same, total = same + (got[:, :64] == want).sum(), total + want.size
+    assert same > 0.9999 * total
+
+
 @pytest.mark.parametrize("kind", [saetta.KvBits.Eight, saetta.KvBits.Half])
 def test_verify_rows_and_decode_after_store(kind):
     # m rows at positions pos..pos+m-1 in one launch, then attention over the cache it wrote:
