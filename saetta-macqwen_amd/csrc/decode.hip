@@ -663,9 +663,15 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
             }
         }
     };
-    load_scales(0);  // first: loads return in order, and the barrier that publishes the scales must not wait for the keys
-    load_keys(0);
-    load_values(0);
+    // Loads return in order: the scales first, since the barrier that publishes them must not wait for the keys, the values
+    // last.  (One row: left to itself the compiler asked for the values before the keys; with the epilogue's exchanges 8-bit 300
+    // tokens of 8192 8.4 -> 8.0 us a layer, halves 4096 10.0 -> 9.8.  Two rows in this order 8.9 -> 9.0, so they keep the compiler's.)
+    auto in_order = [] {
+        if constexpr (PACKED) __builtin_amdgcn_sched_barrier(0);
+    };
+    load_scales(0), in_order();
+    load_keys(0), in_order();
+    load_values(0), in_order();
 
     // ---- prologue: query rows to f16 hi/lo operands in LDS ------------------------
     // (while the first iteration's keys are in flight; the values are requested after it)
@@ -1095,22 +1101,27 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
     constexpr float unscale = code_up<BITS>() / P_UP;
 #pragma unroll
     for (int t = 0; t < TILES; t++) {
+        // PACKED: rows 8-15 hold the lo part of rows 0-7, lanes j + 2 those of lanes j: the sums of register i end up in the lanes
+        // j = 0, 1 and those of register i + 2 in the lanes 2, 3 (one exchange and one addition for both, and every lane stores).
         floatx4 o[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             o[e] = acc[t][e];
             if constexpr (PACKED) {
-                // rows 8-15 hold the lo part of rows 0-7: lanes j and j + 2.
 #pragma unroll
-                for (int i = 0; i < 4; i++) o[e][i] = across_rows<32, 64>(o[e][i], SumOp());
+                for (int i = 0; i < 2; i++) {
+                    // (the builtin: what reads a matrix instruction's result has to be an instruction that the compiler knows)
+                    const float first = o[e][i], third = o[e][i + 2];
+                    const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, first), __builtin_bit_cast(uint32_t, third), false, false);
+                    o[e][i] = __builtin_bit_cast(float, uint32_t(both[0])) + __builtin_bit_cast(float, uint32_t(both[1]));
+                }
             }
         }
-        if (PACKED && j >= 2) continue;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int pair = 16 * t + 4 * j + i;  // (row, head) pair of this accumulator row
-            if (pair >= int(real_rows)) continue;
-            const int vrow = pair >> 3, head = pair & 7;
+        for (int i = 0; i < (PACKED ? 2 : 4); i++) {
+            const int pair = PACKED ? 4 * (j & 1) + 2 * (j >> 1) + i : 16 * t + 4 * j + i;  // (row, head) pair of this accumulator row
+            if (!PACKED && pair >= int(real_rows)) continue;
+            const int vrow = PACKED ? 0 : pair >> 3, head = pair & 7;
             const float zb = QUANT ? zsum_lds[wave * Sh::S_ROWS + pair] * (1.0f / P_UP) : 0.0f;
             const size_t slot = (size_t(vrow) * a.nsplits + split) * a.heads + kv * 8 + head;
             float *dst = a.part_o + slot * DIM + 64 * wave;
