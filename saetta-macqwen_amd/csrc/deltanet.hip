@@ -727,11 +727,14 @@ __global__ __launch_bounds__(256) void deltanet_rows_small_tail_kernel(SmallRows
 // the snapshots, are no faster (9.2 us).
 // A further token is vector instructions, sixteen waves' on one CU (without the snapshots' stores 8 rows take as long); a third
 // of them were the three sums of q and k, which every group of lanes made for itself.  From SHARED_SCALES_FROM rows on a wave
-// makes them for a token, for all, at the price of a barrier: 4 rows with snapshots 8.62 -> 8.21 us, 8 rows 12.55 -> 10.94, 2
-// rows 6.48 either way.  (A head by 512 threads, 8 lanes a row, with these sums: 8.37 and 11.27; 2 rows 6.8.  The loop over the
-// tokens rolled: 8.44, 11.55.)
-// Measured per layer (30 layers in a graph, with the two-launch form before it): one token 7.1 -> 4.6 us, 4 rows with
-// snapshots 11.3 -> 8.2; 8 rows 14.2 -> 10.9.
+// makes them for a token, for all, at the price of a barrier (4 rows with snapshots 8.62 -> 8.21 us, 8 rows 12.55 -> 10.94); one and
+// two rows' are made by the waves of the conv.  (A head by 512 threads, 8 lanes a row: 11.27 for 8 rows, 2 rows slower.  The
+// loop over the tokens rolled: 8.44, 11.55.)
+// A launch this short is its chain of latencies, so what the chain waits for is looked at in the compiled code: the arguments
+// come in one fetch, no load's use moves up between the requests, and nobody waits for a counter's answer but at the end.
+// Measured per layer (30 layers in a graph, with the two-launch form before it): one token 7.1 -> 4.2 us (3.1 of them in the kernel, by
+// clock stamps: 1.2 until the last wave has asked for its rows, 0.5 of which is their 64 KB at 64 bytes a cycle, 1.0 in the loop, 0.3
+// for the norm, 0.3 until the stores are out), 4 rows with snapshots 11.3 -> 7.3; 8 rows 14.2 -> 10.3.
 typedef float nt4 __attribute__((ext_vector_type(4)));
 constexpr int HEAD_THREADS = 1024, HEAD_V_DIM = 128, HEAD_TAPS = 4;
 constexpr int SHARED_SCALES_FROM = 3;
@@ -744,33 +747,69 @@ __global__ __launch_bounds__(HEAD_THREADS) void deltanet_head_kernel(SmallRowsAr
     __shared__ __attribute__((aligned(16))) float in_lds[M][2 * K_DIM + HEAD_V_DIM];  // conv outputs: q, k, v
     __shared__ float gb_lds[M][2];                                                    // decay, beta
     __shared__ float o_lds[M][HEAD_V_DIM];
-    __shared__ __attribute__((aligned(16))) float scale_lds[M][4];                    // what q and k are multiplied by, q.k
+    __shared__ __attribute__((aligned(16))) float scale_lds[M][4];                    // a token's factors, see Factors
+    __shared__ __attribute__((aligned(16))) float sum_lds[M][2][4];                   // PAIRED: |q|^2, |k|^2 and q.k of a wave's channels
+    // One and two rows: a thread has the q and the k channel of a dim, so that the waves of the conv make the sums of q and k
+    // too, half of a key head's channels each (made in the loop by every group of lanes they were a quarter of its instructions).
+    constexpr bool PAIRED = M < SHARED_SCALES_FROM;
+    constexpr uint32_t QK_WAVES = PAIRED ? HEAD_QK_WAVES / 2 : HEAD_QK_WAVES;
     const uint32_t tid = threadIdx.x, lane = tid & 63, part = lane & 15;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t h = blockIdx.x, v_heads = a.p.v_heads, per_key = v_heads / a.p.k_heads, kh = h / per_key;
-    const uint32_t key_size = a.p.k_heads * K_DIM, channels = a.channels;
+    const uint32_t v_heads = a.p.v_heads, per_key = gridDim.y, kh = blockIdx.x, h = kh * per_key + blockIdx.y;
+    // (the arguments at once: left alone the compiler fetches them in four lots, each waited for)
+    asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.conv_state), "s"(a.a), "s"(a.b), "s"(a.a_log), "s"(a.dt_bias), "s"(a.state), "s"(a.z), "s"(a.norm_w), "s"(sync),
+                 "s"(a.p.k_heads), "s"(v_heads), "s"(per_key), "s"(a.channels), "s"(a.p.snapshots), "s"(a.p.eps));
+    const uint32_t key_size = a.p.k_heads * K_DIM;
     const size_t value_size = size_t(v_heads) * HEAD_V_DIM;
-    constexpr uint32_t CONV_WAVES = (2 * K_DIM + HEAD_V_DIM) / 64;
-    const bool conv = wave < CONV_WAVES;  // thread = channel: q (waves 0, 1), k (2, 3), v (4, 5)
-    const uint32_t c = tid < K_DIM       ? kh * K_DIM + tid
-                       : tid < 2 * K_DIM ? key_size + kh * K_DIM + (tid - K_DIM)
-                                         : 2 * key_size + h * HEAD_V_DIM + (tid - 2 * K_DIM);
+    constexpr uint32_t CONV_WAVES = QK_WAVES + HEAD_V_DIM / 64;
+    const bool conv = wave < CONV_WAVES;  // thread = channel: q (the first two waves), k (the next two; PAIRED: q and k), v (two)
+    const uint32_t k_channel = key_size + kh * K_DIM + (tid & 127);
+    const uint32_t c = wave < 2 ? kh * K_DIM + tid : wave < QK_WAVES ? k_channel : 2 * key_size + h * HEAD_V_DIM + (tid & 127);
+    const uint32_t slot = wave < QK_WAVES ? tid : 2 * K_DIM + (tid & 127);
 
     // Everything is requested before anything is used, the conv's inputs first: loads return in order.
-    float seq[PAST + M];  // stored inputs, oldest first, then the new ones
-    float4 taps;
-    if (conv) {
-        taps = *reinterpret_cast<const float4 *>(a.w + size_t(c) * HEAD_TAPS);
+    struct Channel {
+        float seq[PAST + M];  // stored inputs, oldest first, then the new ones
+        float4 taps;
+        __device__ __forceinline__ void request(const SmallRowsArgs &a, uint32_t c) {
+            taps = *reinterpret_cast<const float4 *>(a.w + size_t(c) * HEAD_TAPS);
 #pragma unroll
-        for (int k = 0; k < PAST; k++) seq[k] = a.conv_state[size_t(k) * channels + c];
+            for (int k = 0; k < PAST; k++) seq[k] = a.conv_state[size_t(k) * a.channels + c];
 #pragma unroll
-        for (int t = 0; t < M; t++) seq[PAST + t] = a.x[size_t(t) * channels + c];
-    }
-    float gate_a = 0.0f, gate_b = 0.0f, gate_log = 0.0f, gate_bias = 0.0f;
+            for (int t = 0; t < M; t++) seq[PAST + t] = a.x[size_t(t) * a.channels + c];
+        }
+        __device__ __forceinline__ float output(int t) const {  // (the sum as the single-token conv adds it: oldest first)
+            float acc = taps.x * seq[t];
+            acc += taps.y * seq[t + 1];
+            acc += taps.z * seq[t + 2];
+            return silu_f(acc + taps.w * seq[t + 3]);
+        }
+        __device__ __forceinline__ void keep_snapshots(const SmallRowsArgs &a, uint32_t c) const {
+            // after token t the conv state is the inputs t + 1 .. t + PAST of the sequence
+#pragma unroll
+            for (int t = 0; t < M; t++) {
+#pragma unroll
+                for (int j = 0; j < PAST; j++) __builtin_nontemporal_store(seq[t + 1 + j], a.conv_snaps + (size_t(t) * PAST + j) * a.channels + c);
+            }
+        }
+        __device__ __forceinline__ void keep_state(const SmallRowsArgs &a, uint32_t c) const {
+#pragma unroll
+            for (int j = 0; j < PAST; j++) a.conv_state[size_t(j) * a.channels + c] = seq[M + j];
+        }
+    };
+    Channel own, key;  // (key: PAIRED, the k channel beside the q channel)
+    const bool paired = PAIRED && wave < QK_WAVES;
+    if (conv) own.request(a, c);
+    if (paired) key.request(a, k_channel);
+    float gate_a, gate_b, gate_log, gate_bias;
+    asm("" : "=v"(gate_a), "=v"(gate_b), "=v"(gate_log), "=v"(gate_bias));  // (no constants: sums of them would move into the branch, behind a wait)
     const bool gates = wave == CONV_WAVES && lane < M;
     if (gates) {
-        gate_a = a.a[size_t(lane) * v_heads + h], gate_b = a.b[size_t(lane) * v_heads + h];
-        gate_log = a.a_log[h], gate_bias = a.dt_bias[h];
+        // (vector loads: a scalar load is waited for on the spot, and the wave's rows of the state are asked for behind it)
+        uint32_t gate_h = h;
+        asm volatile("" : "+v"(gate_h));
+        gate_a = a.a[size_t(lane) * v_heads + gate_h], gate_b = a.b[size_t(lane) * v_heads + gate_h];
+        gate_log = a.a_log[gate_h], gate_bias = a.dt_bias[gate_h];
     }
     // 16 lanes a row of the state, dims 4 part .. + 3 and 64 + 4 part .. + 3; rows 8 wave + lane / 16 and four further
     const uint32_t row = 8 * wave + (lane >> 4);
@@ -788,23 +827,35 @@ __global__ __launch_bounds__(HEAD_THREADS) void deltanet_head_kernel(SmallRowsAr
         norm = a.norm_w[out_d];
     }
 
-    if (conv) {
+    if (paired) {
 #pragma unroll
         for (int t = 0; t < M; t++) {
-            // (the sum as the single-token conv adds it: oldest first)
-            float acc = taps.x * seq[t];
-            acc += taps.y * seq[t + 1];
-            acc += taps.z * seq[t + 2];
-            in_lds[t][tid] = silu_f(acc + taps.w * seq[t + 3]);
+            const float y = own.output(t), k = key.output(t);
+            in_lds[t][slot] = y, in_lds[t][K_DIM + slot] = k;
+            const float qq = group_reduce<64>(y * y, SumOp()), kk = group_reduce<64>(k * k, SumOp()), kq = group_reduce<64>(y * k, SumOp());
+            if (lane == 0) *reinterpret_cast<float4 *>(sum_lds[t][wave]) = make_float4(qq, kk, kq, 0.0f);
         }
+    } else if (conv) {
+#pragma unroll
+        for (int t = 0; t < M; t++) in_lds[t][slot] = own.output(t);
     }
     if (gates) fast_gates(gate_a + gate_bias, __expf(gate_log), gate_b, gb_lds[lane][0], gb_lds[lane][1]);
     __syncthreads();
 
     // This wave's conv inputs are in registers (its outputs above were made of them).
-    uint32_t before = 0;
-    if (wave < HEAD_QK_WAVES && lane == 0) before = atomicAdd(sync + kh * HEAD_QK_WAVES + wave, 1u);
+    // (The counter's place as a lane's own: where it is known to be the wave's the compiler adds for all lanes at once and
+    // hands the answer out right there, which makes the wave wait for it.)
+    uint32_t before = 0, counter = kh * HEAD_QK_WAVES + wave;
+    asm volatile("" : "+v"(counter));
+    if (wave < QK_WAVES && lane == 0) before = atomicAdd(sync + counter, 1u);
 
+    // With q and k as the conv gives them, ki and qi what they are multiplied by:  delta / ki = (v - x S.k) y,
+    // o = z S.q + w delta,  S = g S + delta k  for x = g ki, y = beta ki, z = qi g, w = qi (k.q)  (o of the updated state: (g S +
+    // delta k^T) q = g S q + delta (k.q)).
+    auto factors = [&](float qq, float kk, float kq, float g, float beta) {
+        const float qi = (1.0f / sqrtf(float(K_DIM))) * __builtin_amdgcn_rsqf(qq + a.p.eps), ki = __builtin_amdgcn_rsqf(kk + a.p.eps);
+        return make_float4(g * ki, beta * ki, qi * g, qi * kq);
+    };
     // |q|^2, |k|^2 and q.k of token t by wave 15 - t (the first have the counters' answers to wait for), for all
     if constexpr (M >= SHARED_SCALES_FROM) {
         const uint32_t t = HEAD_THREADS / 64 - 1 - wave;
@@ -812,10 +863,7 @@ __global__ __launch_bounds__(HEAD_THREADS) void deltanet_head_kernel(SmallRowsAr
             const float2 q = *reinterpret_cast<const float2 *>(&in_lds[t][2 * lane]), k = *reinterpret_cast<const float2 *>(&in_lds[t][K_DIM + 2 * lane]);
             const float qq = group_reduce<64>(q.x * q.x + q.y * q.y, SumOp()), kk = group_reduce<64>(k.x * k.x + k.y * k.y, SumOp());
             const float kq = group_reduce<64>(q.x * k.x + q.y * k.y, SumOp());
-            if (lane == 0) {
-                *reinterpret_cast<float4 *>(scale_lds[t]) =
-                    make_float4((1.0f / sqrtf(float(K_DIM))) * __builtin_amdgcn_rsqf(qq + a.p.eps), __builtin_amdgcn_rsqf(kk + a.p.eps), kq, 0.0f);
-            }
+            if (lane == 0) *reinterpret_cast<float4 *>(scale_lds[t]) = factors(qq, kk, kq, gb_lds[t][0], gb_lds[t][1]);
         }
         __syncthreads();
     }
@@ -828,32 +876,29 @@ __global__ __launch_bounds__(HEAD_THREADS) void deltanet_head_kernel(SmallRowsAr
             q[i] = *reinterpret_cast<const float4 *>(&in_lds[t][64 * i + part * 4]);
             k[i] = *reinterpret_cast<const float4 *>(&in_lds[t][K_DIM + 64 * i + part * 4]);
         }
-        const float g = gb_lds[t][0], beta = gb_lds[t][1];
-        // One round of 16-lane sums per token: |q|^2, |k|^2, q.k (if they are not there), and S.k and S.q of both rows, S before
-        // the decay and the update: (g S + d k^T) q = g S q + d (k.q).
-        float qi, ki, kq;
-        if constexpr (M >= SHARED_SCALES_FROM) {
-            const float4 x = *reinterpret_cast<const float4 *>(scale_lds[t]);
-            qi = x.x, ki = x.y, kq = x.z;
+        const float g = gb_lds[t][0];
+        float4 f;
+        if constexpr (PAIRED) {
+            const float4 x = *reinterpret_cast<const float4 *>(sum_lds[t][0]), y = *reinterpret_cast<const float4 *>(sum_lds[t][1]);
+            f = factors(x.x + y.x, x.y + y.y, x.z + y.z, g, gb_lds[t][1]);
         } else {
-            const float qq = group_reduce<16>(dot4(q[0], q[0]) + dot4(q[1], q[1]), SumOp());
-            const float kk = group_reduce<16>(dot4(k[0], k[0]) + dot4(k[1], k[1]), SumOp());
-            kq = group_reduce<16>(dot4(k[0], q[0]) + dot4(k[1], q[1]), SumOp());
-            qi = (1.0f / sqrtf(float(K_DIM))) * __builtin_amdgcn_rsqf(qq + a.p.eps), ki = __builtin_amdgcn_rsqf(kk + a.p.eps);
+            f = *reinterpret_cast<const float4 *>(scale_lds[t]);
         }
+        // One round of 16-lane sums per token: S.k and S.q of both rows, S before the decay and the update.
+        auto along = [&](const float4 (&s)[2], const float4 (&x)[2]) { return group_reduce<16>(dot4(s[0], x[0]) + dot4(s[1], x[1]), SumOp()); };
+        float o[2];
 #pragma unroll
         for (int r = 0; r < 2; r++) {
-            const float sk = group_reduce<16>(dot4(st[r][0], k[0]) + dot4(st[r][1], k[1]), SumOp());
-            const float sq = group_reduce<16>(dot4(st[r][0], q[0]) + dot4(st[r][1], q[1]), SumOp());
-            const float delta = (in_lds[t][2 * K_DIM + row + 4 * r] - g * ki * sk) * beta * ki;
-            const float o = qi * (g * sq + delta * kq);
+            const float sk = along(st[r], k), sq = along(st[r], q);
+            const float delta = (in_lds[t][2 * K_DIM + row + 4 * r] - f.x * sk) * f.y;
+            o[r] = f.z * sq + f.w * delta;
 #pragma unroll
             for (int i = 0; i < 2; i++) {
                 st[r][i].x = g * st[r][i].x + delta * k[i].x, st[r][i].y = g * st[r][i].y + delta * k[i].y;
                 st[r][i].z = g * st[r][i].z + delta * k[i].z, st[r][i].w = g * st[r][i].w + delta * k[i].w;
             }
-            if (part == 0) o_lds[t][row + 4 * r] = o;
         }
+        if (part < 2) o_lds[t][row + 4 * part] = part == 0 ? o[0] : o[1];
         if (a.p.snapshots) {
             float *snap = a.state_snaps + size_t(t) * value_size * K_DIM + (size_t(h) * HEAD_V_DIM + row) * K_DIM + part * 4;
 #pragma unroll
@@ -868,28 +913,26 @@ __global__ __launch_bounds__(HEAD_THREADS) void deltanet_head_kernel(SmallRowsAr
 #pragma unroll
         for (int i = 0; i < 2; i++) *reinterpret_cast<float4 *>(sp + r * 4 * K_DIM + i * 64) = st[r][i];
     }
+    float gate = silu_f(z);
+    asm volatile("" : "+v"(gate));  // (here, and not behind the barrier)
     __syncthreads();
     if (out_t < M) {
         // the head's outputs of the token, two per lane of either of its waves
         const float o0 = o_lds[out_t][lane], o1 = o_lds[out_t][lane + 64];
         const float total = group_reduce<64>(o0 * o0 + o1 * o1, SumOp());
-        const float inv = 1.0f / sqrtf(total / float(HEAD_V_DIM) + a.p.eps);
-        a.y[size_t(out_t) * value_size + size_t(h) * HEAD_V_DIM + out_d] = (out_d < 64 ? o0 : o1) * (inv * norm) * silu_f(z);
+        const float inv = inverse_root(total * (1.0f / float(HEAD_V_DIM)) + a.p.eps);
+        a.y[size_t(out_t) * value_size + size_t(h) * HEAD_V_DIM + out_d] = (out_d < 64 ? o0 : o1) * (inv * norm) * gate;
     }
     if (conv) {
-        // after token t the conv state is the inputs t + 1 .. t + PAST of the sequence
-        const bool own = wave >= HEAD_QK_WAVES;
-        if (a.p.snapshots && (own || h == kh * per_key)) {
-#pragma unroll
-            for (int t = 0; t < M; t++) {
-#pragma unroll
-                for (int j = 0; j < PAST; j++) __builtin_nontemporal_store(seq[t + 1 + j], a.conv_snaps + (size_t(t) * PAST + j) * channels + c);
-            }
+        const bool mine = wave >= QK_WAVES;
+        if (a.p.snapshots && (mine || h == kh * per_key)) {
+            own.keep_snapshots(a, c);
+            if (paired) key.keep_snapshots(a, k_channel);
         }
-        if (own || uint32_t(__builtin_amdgcn_readfirstlane(before)) == per_key - 1) {
-#pragma unroll
-            for (int j = 0; j < PAST; j++) a.conv_state[size_t(j) * channels + c] = seq[M + j];
-            if (!own && lane == 0) __hip_atomic_store(sync + kh * HEAD_QK_WAVES + wave, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (mine || uint32_t(__builtin_amdgcn_readfirstlane(before)) == per_key - 1) {
+            own.keep_state(a, c);
+            if (paired) key.keep_state(a, k_channel);
+            if (!mine && lane == 0) __hip_atomic_store(sync + kh * HEAD_QK_WAVES + wave, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
@@ -897,7 +940,7 @@ __global__ __launch_bounds__(HEAD_THREADS) void deltanet_head_kernel(SmallRowsAr
 template <int M>
 void launch_head_rows(const SmallRowsArgs &args, uint32_t *sync, hipStream_t stream) {
     if (args.p.rows == uint32_t(M)) {
-        launch(deltanet_head_kernel<M>, dim3(args.p.v_heads), HEAD_THREADS, 0, stream, args, sync);
+        launch(deltanet_head_kernel<M>, dim3(args.p.k_heads, args.p.v_heads / args.p.k_heads), HEAD_THREADS, 0, stream, args, sync);
     } else if constexpr (M < SMALL_ROWS_MAX) {
         launch_head_rows<M + 1>(args, sync, stream);
     }
@@ -905,7 +948,7 @@ void launch_head_rows(const SmallRowsArgs &args, uint32_t *sync, hipStream_t str
 
 void launch_small_rows(const SmallRowsArgs &args, uint32_t *sync, hipStream_t stream) {
     const saetta_rows_fused_params &p = args.p;
-    if (sync && p.v_dim == HEAD_V_DIM && p.kernel_size == HEAD_TAPS && aligned(args.w, 16)) {
+    if (sync && p.v_dim == HEAD_V_DIM && p.kernel_size == HEAD_TAPS && aligned(args.w, 16) && p.v_heads / p.k_heads < 65536) {
         launch_head_rows<1>(args, sync, stream);
         return;
     }

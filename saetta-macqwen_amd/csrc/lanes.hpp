@@ -51,4 +51,11 @@ __device__ __forceinline__ float group_reduce(float x, Op op) {
     return across_rows<16, WIDTH>(x, op);
 }
 
+// 1 / sqrt(x): the hardware's, an ulp off, and one Newton step (as near as the root and the division rounded one after the
+// other, which are thirty instructions).  0 and infinity, where the step has no value, as they are.
+__device__ __forceinline__ float inverse_root(float x) {
+    const float y = __builtin_amdgcn_rsqf(x), off = fmaf(-x * y, y, 1.0f);
+    return off == off ? fmaf(0.5f * y, off, y) : y;
+}
+
 }  // namespace saetta

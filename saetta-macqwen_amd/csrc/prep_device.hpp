@@ -35,12 +35,8 @@ __device__ __forceinline__ float norm_scale(float total, float eps) {
     return __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(total, float(SAETTA_HEAD_DIM)), eps)));
 }
 
-// The same for query values that nobody stores (a workgroup of the context makes its own): the hardware's reciprocal root and
-// one Newton step, an ulp or so of f32, where the roundings above are a chain of forty instructions.
-__device__ __forceinline__ float query_scale(float total, float eps) {
-    const float x = fmaf(total, 1.0f / float(SAETTA_HEAD_DIM), eps), y = __builtin_amdgcn_rsqf(x);
-    return fmaf(0.5f * y, fmaf(-x * y, y, 1.0f), y);
-}
+// The same for query values that nobody stores (a workgroup of the context makes its own), in a fifth of the instructions.
+__device__ __forceinline__ float query_scale(float total, float eps) { return inverse_root(fmaf(total, 1.0f / float(SAETTA_HEAD_DIM), eps)); }
 
 // Sine and cosine of rotary pair r of half_dims at a position, as on the CPU in f64 and rounded: the pair's frequency, which
 // a kernel makes before it knows the position, then the two of the angle.

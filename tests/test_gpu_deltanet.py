@@ -133,3 +133,22 @@ def test_token_call_matches_conv_then_step(k_heads, v_heads, v_dim, kernel):
         assert np.array_equal(host(conv_gpu).reshape(kernel - 1, channels), conv_cpu), t
         assert np.abs(host(y) - want_y).max() <= 2e-5 * max(1.0, np.abs(want_y).max()), t
         assert np.abs(host(state_gpu) - state_cpu).max() <= 2e-5 * max(1.0, np.abs(state_cpu).max()), t
+
+
+def test_activation_over_the_whole_range():
+    # the conv with a last tap of one is its activation, x / (1 + e^-x): two ulps of f32 wherever the result is a normal
+    # number, zero below 2^-119, where e^-x nears the end of f32, and the limits
+    x = np.concatenate([np.linspace(-100, 100, 2001), -np.logspace(-30, 2, 500), np.logspace(-30, 38, 500), [0.0, -87.0, -88.0, -89.0, -1e30]]).astype(np.float32)
+    special = np.array([np.inf, -np.inf, np.nan], np.float32)
+    xs = np.concatenate([x, special])
+    w = np.zeros((xs.size, 4), np.float32)
+    w[:, 3] = 1
+    state, out = torch.zeros(3, xs.size, device="cuda"), torch.empty(xs.size, device="cuda")
+    plan = saetta.Plan()
+    saetta.deltanet_conv(plan, dev(xs), dev(w), state, out, xs.size, 4)
+    plan.build().run()
+    got, x64 = host(out), x.astype(np.float64)
+    with np.errstate(over="ignore"):
+        want = x64 / (1 + np.exp(-x64))
+    assert (np.abs(got[:x.size] - want) <= 2.4e-7 * np.abs(want) + 2.0 ** -119).all()
+    assert got[-3] == np.inf and np.isnan(got[-1]) and not got[-2] > 0
