@@ -97,7 +97,11 @@ void launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t
         (record_arg<std::remove_cv_t<P>>(*list, static_cast<P>(args)), ...);
         return;
     }
-    kernel<<<grid, block, lds, stream>>>(std::forward<A>(args)...);
+    std::tuple<std::remove_cv_t<P>...> values(static_cast<P>(args)...);
+    std::apply([&](auto &...value) {
+        void *pointers[] = {&value...};
+        (void)hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, pointers, lds, stream);  // (its status: launch_status)
+    }, values);
 }
 
 // Says what the launch just recorded is.

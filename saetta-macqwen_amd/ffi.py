@@ -1,9 +1,14 @@
-"""ctypes binding of include/saetta_hip.h.  One function per exported symbol."""
+"""ctypes binding of include/saetta_hip.h.  One function per exported symbol.
+
+The calls that a program makes per chunk and per token go through an extension module instead (`calls`)."""
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("SAETTA_HIP_LIB") or os.path.join(_HERE, "lib", "libsaetta_hip.so")
+CALLS_PATH = os.path.join(_HERE, "lib", "_saetta_calls.so")
 
 # Every symbol include/saetta_hip.h declares; tests check the library exports each.
 SYMBOLS = [
@@ -48,6 +53,24 @@ class QuantRowsC(ctypes.Structure):
 
 class SaettaError(RuntimeError):
     """A non-zero return of the C ABI (the reference panics in these places)."""
+
+
+class _Missing:
+    """What stands for the extension module where it has not been built: importing works, a call raises."""
+
+    def __getattr__(self, name):
+        raise SaettaError(f"{CALLS_PATH} is missing: run __graft_entry__.build() (make -C csrc)")
+
+
+def calls():
+    """The extension module of csrc/calls.cpp, set up for this copy of the package.  (It wants torch to be imported.)"""
+    if not os.path.exists(CALLS_PATH):
+        return _Missing()
+    loader = importlib.machinery.ExtensionFileLoader("_saetta_calls", CALLS_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_saetta_calls", CALLS_PATH, loader=loader))
+    loader.exec_module(module)
+    module.setup(LIB_PATH, SaettaError, FlashParamsC)
+    return module
 
 
 _lib = None

@@ -22,6 +22,7 @@ import torch
 
 from . import ffi
 
+_calls = ffi.calls()
 GROUP = 64      # src/kv_quant.rs:9
 MAX_ROWS = 8    # src/rows.rs:9
 DIM = 256
@@ -66,6 +67,13 @@ def _stream(stream=None):
         # the handle of torch's current stream, without the Stream object of torch.cuda.current_stream()
         return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
     return ctypes.c_void_p(stream.cuda_stream)
+
+
+def _handle(stream):
+    """What the extension's calls take: None for torch's current stream, or the handle of another as a number."""
+    if stream is None:
+        return None
+    return (stream.value or 0) if isinstance(stream, ctypes.c_void_p) else stream.cuda_stream
 
 
 def _ptr(t):
@@ -113,9 +121,7 @@ class _Launches:
             self.free, self.plan = l.saetta_plan_free, ctypes.c_void_p(l.saetta_plan_end())
 
     def __call__(self, s):
-        rc = ffi.lib().saetta_plan_run(s, self.plan)
-        if rc:
-            ffi.check(rc, "plan_run")
+        _calls.plan_run(self.plan.value, _handle(s))
 
     def __del__(self):
         if self.plan is not None:
@@ -156,8 +162,7 @@ class Plan:
     def set_params(self, tp):
         """Plan::set_params (src/plan.rs:144-146): one small launch on the current stream that carries the
         values (a copy from pinned memory took 10 us of the host and 7 us of the stream, this 3 and 1.6)."""
-        ffi.check(ffi.lib().saetta_token_params_set(_stream(), _ptr(self.params), ffi.TokenParamsC(
-            tp.token, tp.position, tp.kv_len, tp.pad)), "token_params_set")
+        _calls.token_params_set(self.params, tp.token, tp.position, tp.kv_len, tp.pad)
 
     def __len__(self):
         return len(self.ops)
@@ -212,6 +217,8 @@ class Built:
         self._parts = []
         for native, run in itertools.groupby((launch for _, launch in ops), lambda launch: isinstance(launch, _Call)):
             self._parts += [_Launches(list(run))] if native else run
+        # the native plan of ops that are nothing else
+        self._native = self._parts[0].plan if len(self._parts) == 1 and isinstance(self._parts[0], _Launches) else None
         if graph and ops:
             # The library's one-time set-up (code objects, LDS limits) must not happen under capture;
             # the launches themselves are not run here: a plan may hold ops that advance a state.
@@ -234,7 +241,10 @@ class Built:
                 raise ValueError("Built.run: a captured plan replays on the current stream; make the stream current instead of passing it")
             self.graph.replay()
             return
-        s = _stream(stream)
+        s = None if self._native else _stream(stream)
+        if s is None:
+            _calls.plan_run(self._native.value, _handle(stream))
+            return
         for part in self._parts:
             part(s)
 
@@ -289,12 +299,7 @@ class QuantRows:
             bits, _ptr(x), self.c(), p, _ptr(params), 0), (x, params, *self.tensors())))
 
     def encode(self, x, pos, tokens, stream=None):
-        _need(x, torch.float32, "QuantRows.encode x")
-        if pos + tokens > self.capacity or x.numel() < tokens * self.per_token * GROUP:
-            raise ValueError("QuantRows.encode: tokens do not fit")
-        p = ffi.KvQuantParamsC(self.per_token * tokens, self.per_token)
-        ffi.check(ffi.lib().saetta_kv_quantize(_stream(stream), self.bits.value, _ptr(x), self.c(), p, None, pos),
-                  "kv_quantize")
+        _calls.kv_encode(self.bits._value_, self.per_token, self.capacity, self.data, self.scales, self.biases, x, pos, tokens, _handle(stream))
 
     def encode_dequantize(self, out, tokens, stream=None):
         _need(out, torch.float16, "QuantRows.encode_dequantize out")
@@ -355,11 +360,7 @@ def test_slack(bits):
 
 def to_half(x, out, stream=None):
     """to_half (kernels/prefill.metal:1428-1432)."""
-    _need(x, torch.float32, "to_half x")
-    _need(out, torch.float16, "to_half out")
-    rc = ffi.lib().saetta_to_half(_stream(stream), x.data_ptr(), out.data_ptr(), x.numel())
-    if rc:
-        ffi.check(rc, "to_half")
+    _calls.to_half(x, out, _handle(stream))
 
 
 def _check_shape(heads, kv_heads, head_dim, what):
@@ -755,13 +756,12 @@ def _workspace(t):
     return _ptr(t), t.numel()
 
 
-def _workspace_or_own(t, p, like, stream):
-    """The caller's workspace for the chunk of FlashParams p, or a tensor of this call's own from torch's allocator (which hands a
+def _own_workspace(q, p, stream):
+    """A workspace for the chunk of FlashParams p as a tensor of the call's own from torch's allocator (which hands a
     block out again only behind the work queued on its stream): the library's own workspace, which a
     NULL pointer would select, is one per device and stream that stays for the life of the process."""
-    if t is not None:
-        return t
-    t = torch.empty(attention_prefill.workspace_bytes(p), dtype=torch.uint8, device=like.device)
+    _need(q, torch.float16, "q")
+    t = torch.empty(attention_prefill.workspace_bytes(p), dtype=torch.uint8, device=q.device)
     if isinstance(stream, torch.cuda.Stream):
         t.record_stream(stream)
     return t
@@ -795,15 +795,7 @@ class attention_prefill:
         call's own (a caller that times the call, or records it, brings its own)."""
         if kernel not in attention_prefill.KERNELS:
             raise ValueError(f"no prefill attention kernel {kernel}")
-        if p.heads != p.kv_heads * 8:
-            raise ValueError(f"{kernel} needs 8 q heads per kv head")
-        _need(q, torch.float16, "q"), _need(keys, torch.float16, "keys"), _need(values, torch.float16, "values")
-        _need(q_and_gate, torch.float32, "q_and_gate"), _need(out, torch.float32, "out")
-        workspace = _need(_workspace_or_own(workspace, p, q, stream), torch.uint8, "workspace")
-        rc = ffi.lib().saetta_attn_prefill(_stream(stream), q.data_ptr(), keys.data_ptr(), values.data_ptr(), q_and_gate.data_ptr(),
-                                           out.data_ptr(), p, workspace.data_ptr(), workspace.numel())
-        if rc:
-            ffi.check(rc, "attn_prefill")
+        _calls.prefill(kernel, q, keys, values, q_and_gate, out, p, workspace if workspace is not None else _own_workspace(q, p, stream), _handle(stream))
 
     @staticmethod
     def encode_rows2(q, keys, values, q_and_gate, out, p, stream=None, workspace=None):
@@ -868,14 +860,8 @@ class attention_prefill:
     @staticmethod
     def encode_quant(q, keys, values, q_and_gate, out, p, stream=None, workspace=None):
         """The chunk over a quantized cache read in place (src/prefill.rs:1735-1776)."""
-        if p.heads != p.kv_heads * 8:
-            raise ValueError("prefill attention needs 8 q heads per kv head")
-        _need(q, torch.float16, "q"), _need(q_and_gate, torch.float32, "q_and_gate"), _need(out, torch.float32, "out")
-        workspace = _need(_workspace_or_own(workspace, p, q, stream), torch.uint8, "workspace")
-        rc = ffi.lib().saetta_attn_prefill_quant(_stream(stream), keys.bits.value, q.data_ptr(), keys.c(), values.c(),
-                                                 q_and_gate.data_ptr(), out.data_ptr(), p, workspace.data_ptr(), workspace.numel())
-        if rc:
-            ffi.check(rc, "attn_prefill_quant")
+        _calls.prefill_quant(keys.bits._value_, q, keys.data, keys.scales, keys.biases, values.data, values.scales, values.biases, q_and_gate, out, p,
+                             workspace if workspace is not None else _own_workspace(q, p, stream), _handle(stream))
 
 
 class attention_gemm:

@@ -141,6 +141,31 @@ def test_without_a_gpu_the_library_refuses_to_run():
     assert ffi.lib().saetta_last_error()
 
 
+def test_calls_check_what_they_are_given():
+    import torch
+    # what the extension refuses before it asks for a stream: types, layouts, sizes, each copy of the package with its own error
+    x, h, ap, p = torch.zeros(512), torch.zeros(512, dtype=torch.float16), saetta.attention_prefill, saetta.FlashParams(16, 2, 0, 1, 0.0625)
+    for bad in (x, x.numpy(), None, "x"):
+        with pytest.raises(TypeError, match=r"to_half x: expected a contiguous torch.float32 tensor on the GPU"):
+            saetta.to_half(bad, h)
+    rows = saetta.QuantRows(saetta.KvBits.Eight, 512, 4, "cpu")
+    with pytest.raises(TypeError, match="QuantRows.encode x"):
+        rows.encode(x, 0, 1)
+    with pytest.raises(ValueError, match="no prefill attention kernel"):
+        ap.encode("attention_fa3", h, h, h, x, x, p, workspace=x)
+    with pytest.raises(ValueError, match="attention_fa4 needs 8 q heads per kv head"):
+        ap.encode("attention_fa4", h, h, h, x, x, saetta.FlashParams(15, 2, 0, 1, 0.0625), workspace=x)
+    with pytest.raises(TypeError, match="q: expected a contiguous torch.float16"):
+        ap.encode("attention_fa8", h, h, h, x, x, p, workspace=x)
+    calls = saetta.host._calls
+    with pytest.raises(TypeError, match="expected FlashParams"):
+        calls.prefill("attention_fa8", h, h, h, x, x, "p", x, None)
+    with pytest.raises(TypeError, match="takes 3 arguments"):
+        calls.to_half(x, h)
+    with pytest.raises(saetta.ffi.SaettaError, match="plan_run: .*code"):
+        calls.plan_run(0, 0)
+
+
 def test_kv_bits_mirror():
     # src/kv_quant.rs:11-50
     K = saetta.KvBits

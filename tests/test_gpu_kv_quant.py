@@ -135,6 +135,30 @@ def test_to_half_rounds_to_nearest_even():
     assert np.array_equal(host(out).view(np.uint16), oracle.f32_to_f16_bits(x))
 
 
+def test_calls_run_on_the_stream_they_are_given():
+    # the current stream, a stream that is not current, the default stream beside a current one: behind what that stream
+    # holds, which is long enough for a call on another stream to be there first
+    x, a, b = torch.ones(1 << 20, device="cuda"), torch.randn(4096, 4096, device="cuda"), torch.empty(4096, 4096, device="cuda")
+    side, default = torch.cuda.Stream(), torch.cuda.default_stream()
+    rows = saetta.QuantRows(saetta.KvBits.Eight, 512, 2048)
+    for current, given in ((side, None), (default, side), (side, default), (default, None)):
+        out = torch.empty(1 << 20, dtype=torch.float16, device="cuda")
+        used = current if given is None else given
+        for value in (2.0, 3.0):
+            x.fill_(1.0), out.zero_(), rows.biases.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(used):
+                for _ in range(8):
+                    torch.mm(a, a, out=b)
+                x.fill_(value)
+            with torch.cuda.stream(current):
+                saetta.to_half(x, out, *([given] if given is not None else []))
+                rows.encode(x, 0, 2048, stream=given)
+            used.synchronize()
+            assert host(out).min() == host(out).max() == value
+            assert host(rows.biases).min() == host(rows.biases).max() == value
+
+
 @pytest.mark.parametrize("kind", KINDS)
 def test_module_functions_match_cpu(kind):
     # quantize / dequantize / round_trip / round_trip_as_half of src/kv_quant.rs:54-125 as device functions.
