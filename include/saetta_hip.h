@@ -449,8 +449,8 @@ int saetta_deltanet_rows_fused_sync(saetta_stream_t stream, const float *x, cons
 
 /* Bytes of workspace a prefill chunk at (pos, tokens) wants: the f16 key and
  * value tile images of the pos + tokens rows the chunk can see and, for a chunk with too few
- * tokens to fill the GPU, room for partial results of parts of the keys (up to 32 parts of
- * 1 KB + 8 B per query row).  A call given the images' part only (one sized for
+ * tokens to fill the GPU, room for partial results of parts of the keys (up to 64 parts of
+ * 1 KB + 8 B per query row; where no images are made, instead of them).  A call given the images' part only (one sized for
  * another chunk of as many rows) runs too, without the split.  Its bits are then
  * others: the probabilities are rounded to f16 relative to a maximum, which with
  * the split is a part's own.  Both forms are as close to the exact result, but who

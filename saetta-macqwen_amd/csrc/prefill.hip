@@ -764,8 +764,9 @@ __global__ __launch_bounds__(MERGE_THREADS) void prefill_merge_kernel(PrefillArg
 // cache is read where it lies, once per row group: the keys go from memory to MFMA operands in registers, the values to a
 // tile of the wave's own in LDS, row by row as in memory, and come back transposed (ds_read_b64_tr_b16).  Codes are
 // dequantized on the way, with the arithmetic of the prepare kernel.
-// The price is that every row group pulls (and dequantizes) the keys for itself: from a thousand keys on the tiles of 16
-// tokens and their images win; the line is in flash_plan.
+// The price is that every row group pulls (and dequantizes) the keys for itself: with many tokens the tiles of 16 and their
+// images win, and with few over a long context a row group's keys go to several workgroups (SPLIT), whose parts the
+// tiles' merge joins; the lines are in choose_small.
 // What bounds a block of halves per wave (4 us for the eight of them): 256 KB through the CU's 64 bytes a cycle are 1.8 of
 // them, the values' way through LDS and the query operands 1.4.  A key's operands straight from its row, 16 bytes a lane,
 // took 5.3 us: such a load is taken a row a cycle, and so four lanes fetch 64 bytes of a row together and turn four rows
@@ -791,6 +792,9 @@ struct SmallArgs {
     float *out;
     uint32_t heads, kv_heads, pos, tokens;
     float scale;
+    // SPLIT: the keys in `nparts` parts of `part_blocks` blocks, a workgroup each; their O, m and l as PrefillArgs' parts
+    uint32_t part_blocks, nparts;
+    float *part_o, *part_ml;
 };
 
 template <int BITS>
@@ -817,20 +821,40 @@ __device__ __forceinline__ constexpr int small_dim(int st, int hf) {
     return (BITS == 16 ? (i / 4 * 2 + hf) * 4 + i % 4 : i * 2 + hf) * 8 * STEPS + st % STEPS * 8;
 }
 
-template <int BITS>
+template <int BITS, bool SPLIT>
 __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallArgs a) {
     using L = SmallLds<BITS>;
     constexpr int RB = row_bytes<BITS>(), PIECES = RB / 16, STEPS = 16 / BITS, VALUES = 128 / BITS;  // pieces of a row; values of one
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hf = lane >> 5;
-    const uint32_t kv = blockIdx.y, kvh = a.kv_heads;
-    const uint32_t tok0 = (gridDim.x - 1 - blockIdx.x) * 4;  // (the row groups that see the most keys first)
+    const uint32_t kvh = a.kv_heads, groups = (a.tokens + 3) / 4;
+    uint32_t kv = blockIdx.y, at_group = blockIdx.x, part = 0;
+    if constexpr (SPLIT) {
+        // Workgroups go to the 8 XCDs in turn, and each XCD has its own L2: an XCD takes an eighth of the (part, kv head, row
+        // group) in a row, since the row groups of a part read the same keys.
+        const uint32_t item = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8, pair = item / groups;
+        if (pair >= a.nparts * kvh) return;
+        at_group = item % groups, kv = pair % kvh, part = pair / kvh;
+    }
+    const uint32_t tok0 = (groups - 1 - at_group) * 4;  // (the row groups that see the most keys first)
     const uint32_t tok = tok0 + (col >> 3), head = kv * SAETTA_GQA_GROUP + (col & 7);
     const float c = a.scale * 1.4426950408889634f;
     const uint32_t keys = a.pos + min(tok0 + 4, a.tokens);  // what the last of its tokens sees
-    const uint32_t nblocks = (keys + BK - 1) / BK;
-    const uint32_t active = min(nblocks, uint32_t(SMALL_WAVES));  // waves that have a block
+    const uint32_t first = SPLIT ? part * a.part_blocks : 0;         // blocks of keys: this workgroup's are first .. nblocks - 1
+    uint32_t nblocks = (keys + BK - 1) / BK;
+    if constexpr (SPLIT) {
+        if (nblocks <= first) {
+            // a part of its tile that this row group sees no key of: no weight in the merge (which multiplies what lies there)
+            const size_t item = (size_t(part) * ((a.tokens + TQ - 1) / TQ) + tok0 / TQ) * kvh + kv;
+            float4 *po = reinterpret_cast<float4 *>(a.part_o) + (item * WAVES + tok0 % TQ / 4 * 2) * 16 * 64;
+            for (uint32_t i = tid; i < 2 * 16 * 64; i += SMALL_THREADS) po[i] = float4{0, 0, 0, 0};
+            if (tid < 32) *reinterpret_cast<float2 *>(a.part_ml + ((item * 4 + tok0 % TQ / 4) * 32 + tid) * 2) = float2{4.0f * NO_SCORE, 0.0f};
+            return;
+        }
+        nblocks = min(nblocks, first + a.part_blocks);
+    }
+    const uint32_t active = min(nblocks - first, uint32_t(SMALL_WAVES));  // waves that have a block
     const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(lds));
     const uint32_t vtile = lds0 + L::V_OFF + wave * L::VTILE;
 
@@ -942,7 +966,7 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
             }
     };
 
-    if (uint32_t(wave) < active) fetch_keys(wave);
+    if (uint32_t(wave) < active) fetch_keys(first + wave);
     // Q^T operands: through LDS, where all waves read them
     {
         half8 qv[2];
@@ -951,7 +975,7 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
             const int st = 2 * wave + i;
             qv[i] = *reinterpret_cast<const half8 *>(a.q + (size_t(min(tok, a.tokens - 1)) * a.heads + head) * DIM + small_dim<BITS>(st, hf));
         }
-        if (uint32_t(wave) < active) fetch_values(wave);
+        if (uint32_t(wave) < active) fetch_values(first + wave);
 #pragma unroll
         for (int i = 0; i < 2; i++) *reinterpret_cast<half8 *>(lds + L::Q_OFF + (2 * wave + i) * 1024 + lane * 16) = qv[i];
     }
@@ -964,7 +988,7 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
         for (int r = 0; r < 16; r++) acc[mt][r] = 0.0f;
     }
     float m = 0.25f * NO_SCORE * c, l = 0.0f;  // (above a masked score, as in the kernel above)
-    for (uint32_t b = wave; b < nblocks; b += SMALL_WAVES) {
+    for (uint32_t b = first + wave; b < nblocks; b += SMALL_WAVES) {
         // ---- S^T = K Q^T ----
         floatx16 s;
 #pragma unroll
@@ -1055,8 +1079,10 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
     // ---- the waves' parts joined: wave w finishes dims 32 w .. 32 w + 31 ----
     const size_t row = size_t(min(tok, a.tokens - 1)) * a.heads + head;
     float4 g[4];
+    if constexpr (!SPLIT) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) g[i] = *reinterpret_cast<const float4 *>(a.q_and_gate + row * 2 * DIM + DIM + 32 * wave + 8 * i + 4 * hf);
+        for (int i = 0; i < 4; i++) g[i] = *reinterpret_cast<const float4 *>(a.q_and_gate + row * 2 * DIM + DIM + 32 * wave + 8 * i + 4 * hf);
+    }
     lds_barrier();  // every wave is through with its tile and the query operands
     float2 *ml = reinterpret_cast<float2 *>(lds + L::ML_OFF);
     const float l_row = l + __shfl_xor(l, 32);
@@ -1072,16 +1098,16 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
             for (int i = 0; i < 4; i++) tile_of(wave, mt)[i * 64] = float4{acc[mt][4 * i], acc[mt][4 * i + 1], acc[mt][4 * i + 2], acc[mt][4 * i + 3]};
         }
     };
-    float weight[SMALL_WAVES], l_all = 0.0f;
-    auto take_in = [&](int first) {  // the dims this wave finishes, from waves first .. first + 3
+    float weight[SMALL_WAVES], l_all = 0.0f, top = 4.0f * NO_SCORE;
+    auto take_in = [&](int from) {  // the dims this wave finishes, from waves from .. from + 3
 #pragma unroll
         for (int w = 0; w < 4; w++) {
-            if (uint32_t(first + w) < active) {
+            if (uint32_t(from + w) < active) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const float4 x = tile_of(w, wave)[i * 64];
-                    fin[4 * i] += x.x * weight[first + w], fin[4 * i + 1] += x.y * weight[first + w];
-                    fin[4 * i + 2] += x.z * weight[first + w], fin[4 * i + 3] += x.w * weight[first + w];
+                    fin[4 * i] += x.x * weight[from + w], fin[4 * i + 1] += x.y * weight[from + w];
+                    fin[4 * i + 2] += x.z * weight[from + w], fin[4 * i + 3] += x.w * weight[from + w];
                 }
             }
         }
@@ -1090,7 +1116,6 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
     lds_barrier();
     {
         float2 x[SMALL_WAVES];
-        float top = 4.0f * NO_SCORE;
 #pragma unroll
         for (int w = 0; w < SMALL_WAVES; w++) x[w] = ml[w * 32 + col];  // (a wave without a block: l = 0)
 #pragma unroll
@@ -1104,6 +1129,16 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
         if (wave >= 4 && uint32_t(wave) < active) hand_out();
         lds_barrier();
         take_in(4);
+    }
+    if constexpr (SPLIT) {
+        // (rows past the chunk's end leave what their masked lanes hold; nothing reads it)
+        const size_t item = (size_t(part) * ((a.tokens + TQ - 1) / TQ) + tok0 / TQ) * kvh + kv;
+        const uint32_t group = tok0 % TQ / 4;
+        float4 *po = reinterpret_cast<float4 *>(a.part_o) + ((item * WAVES + group * 2 + (wave >> 2)) * 16 + (wave & 3) * 4) * 64 + lane;
+#pragma unroll
+        for (int i = 0; i < 4; i++) po[i * 64] = float4{fin[4 * i], fin[4 * i + 1], fin[4 * i + 2], fin[4 * i + 3]};
+        if (wave == 0 && hf == 0) *reinterpret_cast<float2 *>(a.part_ml + ((item * 4 + group) * 32 + col) * 2) = float2{top, l_all};
+        return;
     }
     if (tok < a.tokens) {
         const float inv = 1.0f / l_all;
@@ -1139,6 +1174,7 @@ size_t images_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) {
 size_t plain_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) { return images_bytes(pos, tokens, kv_heads) + 256; }
 
 constexpr size_t PART_O_BYTES = size_t(TQ) * SAETTA_GQA_GROUP * DIM * 4, PART_ML_BYTES = size_t(TQ) * SAETTA_GQA_GROUP * 8;
+constexpr uint32_t SMALL_MAX_PARTS = 64;
 size_t parts_bytes(uint32_t tokens, uint32_t kv_heads, uint32_t nparts) {
     return size_t((tokens + TQ - 1) / TQ) * kv_heads * nparts * (PART_O_BYTES + PART_ML_BYTES);
 }
@@ -1146,13 +1182,15 @@ uint32_t parts_of(uint32_t pos, uint32_t tokens, uint32_t part_blocks) {
     return (uint32_t((uint64_t(pos) + tokens + BK - 1) / BK) + part_blocks - 1) / part_blocks;
 }
 
-// How a chunk's launches are laid out: the row groups' own launch (small), or tiles, with their keys in parts of
-// `part_blocks` blocks where that is not 0.
+// How a chunk's launches are laid out: the row groups' own launch (small), with their keys in parts of `small_part_blocks`
+// blocks where that is not 0 and there is room for them; or tiles, with their keys in parts of `part_blocks` blocks where
+// that is not 0.
 struct FlashPlan {
-    bool small;
-    uint32_t cus, part_blocks, nparts;
-    size_t plain, parts;  // bytes of workspace: the images and the tile count; the parts behind them
-    size_t bytes() const { return plain + parts; }
+    bool small;  // without parts, the row groups' launch is ahead of the tiles
+    uint32_t small_part_blocks, cus, part_blocks, nparts;
+    size_t plain, parts, small_parts;  // bytes of workspace: the images and the tile count; the parts behind them; the row groups' parts, instead of both
+    size_t tiles() const { return plain + parts; }
+    size_t bytes() const { return tiles() > small_parts ? tiles() : small_parts; }
 };
 
 // A tile is one workgroup's work, and 16 tokens of 2 kv heads are all a CU gets of it: chunks under 2048 tokens leave CUs
@@ -1160,48 +1198,45 @@ struct FlashPlan {
 // rounds of workgroups would take, in us, unsplit and with the keys in 2 to 32 parts, from figures measured on the MI355X:
 // a workgroup's block of 32 keys takes 0.6 us while the chip has power to spare (up to ~170 workgroups) and the chip as a
 // whole 284 blocks a us beyond that; the ends of an item (its first loads, the store of its part) 12 us, with the gate
-// 14.5; the merge a launch and 128 KB read back per item.  The small kernel's workgroups take 0.5 us for a block
-// (0.6 with codes), with a quarter of the rows, and don't slow each other down; their ends take 5 us, and there are no
-// images to prepare (5 us and more).  (Codes: 0.59, for at 0.6 a tie sends 64 tokens at 1000 to the tiles, 27.2 -> 31.4.)
+// 14.5; the merge a launch and 128 KB read back per item; the images 4.5 us and 0.3 ns a key and kv head.
 // Measured, unsplit -> split by this rule, the whole call (8-bit cache): 100 tokens at 10000: 211 -> 47 us, at 100000
 // (4-bit): 1886 -> 225; 500 at 40000: 770 -> 330; 2100 at 9000: 497 -> 405.  A full chunk (4096 tokens: two whole rounds)
-// is never split.  Tiles -> the small kernel, halves | 8-bit | 4-bit: 16 tokens at 500 22.9 -> 18.3 | 24.0 -> 20.7 | 24.1 -> 20.6; 64 at
-// 1000 30.3 -> 24.5 | 31.4 -> 27.2 | 31.7 -> 28.4; 500 from 0 32.4 -> 20.3 | 33.4 -> 22.0 | 33.5 -> 21.9; 700 from 0 35.9 -> 25.7 | 37.0 ->
-// 28.5 | 37.3 -> 26.6; 500 at 800 39.2 -> 31.0 | 40.9 -> 32.9 | 41.1 -> 33.8.  Past its line: 1250 from 0 46.5 -> 50.3 | 47.8 -> 55.1 | 47.8
-// -> 54.1; 250 at 1700 35.4 -> 37.0 | 36.7 -> 39.3 | 37.2 -> 42.6; 16 at 1000 25.0 -> 25.9 | 24.9 -> 27.0 (codes).  Of 36 chunks on
-// either side of it each, none is sent to the small kernel that it takes longer for; left to the tiles though the small kernel
-// is ahead are 128 tokens at 1500 (33.7 -> 31.8 | 35.7 -> 34.0), 250 at 1300 (36.2 -> 33.9) and 100 at 1300 (33.1 -> 30.4) of 8-bit codes.
-FlashPlan flash_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, int bits) {
-    constexpr float BLOCK_US = 0.6f, CHIP_BLOCKS_PER_US = 284.0f / 256.0f, PART_US = 12.0f, TILE_US = 14.5f, MERGE_US = 4.0f, MERGE_ITEM_US = 0.03f;
-    constexpr float SMALL_US = 5.0f, SMALL_BLOCK_US = 0.5f, SMALL_CODES_BLOCK_US = 0.59f, PREPARE_US = 5.0f;
+// is never split.
+constexpr float MERGE_ITEM_US = 0.03f;
+// n items in order of length, from `high` down to `low` blocks, handed out one by one to `cus` workgroups: us, if a block
+// takes block_us alone and chip_us of the whole chip
+float rounds_us(uint32_t cus, uint32_t n, float high, float low, float ends_us, float block_us, float chip_us) {
+    float us = 0.0f, at = 0.0f;
+    for (uint32_t left = n; left > 0;) {
+        const uint32_t now = left < cus ? left : cus;
+        const float mid = high - (high - low) * (at + 0.5f * float(now)) / float(n);  // mean length of the round's items
+        const float alone = mid * block_us, shared = mid * float(now) * chip_us;
+        us += (alone > shared ? alone : shared) + ends_us;
+        at += float(now), left -= now;
+    }
+    const float one = high * block_us + ends_us;
+    return us > one ? us : one;
+}
+// The tiles' part of the plan; tiles_us: what they would take, images and all.
+FlashPlan tiles_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, float &tiles_us) {
+    constexpr float BLOCK_US = 0.6f, CHIP_BLOCKS_PER_US = 284.0f / 256.0f, PART_US = 12.0f, TILE_US = 14.5f, MERGE_US = 4.0f;
+    constexpr float PREPARE_US = 4.5f, PREPARE_KEY_US = 0.0003f;
     FlashPlan f{};
     f.cus = cu_count();
     f.plain = plain_workspace_bytes(pos, tokens, kv_heads);
+    tiles_us = 0.0f;
     if (tokens == 0 || kv_heads == 0) return f;
     const uint32_t ntiles = (tokens + TQ - 1) / TQ;
     const uint32_t longest = tile_blocks(pos, tokens, ntiles - 1), shortest = tile_blocks(pos, tokens, 0);
     const float chip_us = 1.0f / (CHIP_BLOCKS_PER_US * float(f.cus));
-    // n items in order of length, from `high` down to `low` blocks, handed out one by one
-    auto rounds_us = [&](uint32_t n, float high, float low, float ends_us, float block_us, float chip_us) {
-        float us = 0.0f, at = 0.0f;
-        for (uint32_t left = n; left > 0;) {
-            const uint32_t now = left < f.cus ? left : f.cus;
-            const float mid = high - (high - low) * (at + 0.5f * float(now)) / float(n);  // mean length of the round's items
-            const float alone = mid * block_us, shared = mid * float(now) * chip_us;
-            us += (alone > shared ? alone : shared) + ends_us;
-            at += float(now), left -= now;
-        }
-        const float one = high * block_us + ends_us;
-        return us > one ? us : one;
-    };
-    const float unsplit = rounds_us(ntiles * kv_heads, float(longest), float(shortest), TILE_US, BLOCK_US, chip_us);
+    const float unsplit = rounds_us(f.cus, ntiles * kv_heads, float(longest), float(shortest), TILE_US, BLOCK_US, chip_us);
     float best = 0.95f * unsplit;
     for (uint32_t parts = 2; parts <= 32; parts++) {
         const uint32_t pb = ((longest + parts - 1) / parts + 1) / 2 * 2;  // (a step of the kernel is two blocks)
         if (pb < 4 || pb >= longest) continue;
         const uint32_t items = prefill_items(pos, tokens, pb) * kv_heads;
         const float mid = 0.5f * float(longest + shortest) * float(ntiles * kv_heads) / float(items);
-        const float us = rounds_us(items, mid, mid, PART_US, BLOCK_US, chip_us) + MERGE_US + MERGE_ITEM_US * float(items);
+        const float us = rounds_us(f.cus, items, mid, mid, PART_US, BLOCK_US, chip_us) + MERGE_US + MERGE_ITEM_US * float(items);
         if (us < best) best = us, f.part_blocks = pb;
     }
     if (f.part_blocks) {
@@ -1210,12 +1245,61 @@ FlashPlan flash_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, int bits)
     } else {
         best = unsplit;
     }
-    const uint32_t groups = (tokens + 3) / 4 * kv_heads;
-    f.small = rounds_us(groups, float(longest), float(shortest), SMALL_US, bits == 16 ? SMALL_BLOCK_US : SMALL_CODES_BLOCK_US, 0.0f) < best + PREPARE_US;
+    tiles_us = best + PREPARE_US + PREPARE_KEY_US * float(pos + tokens) * float(kv_heads);
     return f;
 }
 
-size_t workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) { return flash_plan(pos, tokens, kv_heads, 16).bytes(); }
+// The row groups' part, for one kind of cache.  Without parts their workgroups take 0.5 us for a block (0.6 with codes), with a
+// quarter of a tile's rows, and don't slow each other down; their ends take 5 us, and there are no images to prepare.  (Codes:
+// 0.59, for at 0.6 a tie sends 64 tokens at 1000 to the tiles, 27.2 -> 31.4.)  Tiles -> row groups, halves | 8-bit | 4-bit: 16 tokens
+// at 500 22.9 -> 18.3 | 24.0 -> 20.7 | 24.1 -> 20.6; 500 from 0 32.4 -> 20.3 | 33.4 -> 22.0 | 33.5 -> 21.9; 700 from 0 35.9 -> 25.7 | 37.0 -> 28.5 |
+// 37.3 -> 26.6; 500 at 800 39.2 -> 31.0 | 40.9 -> 32.9 | 41.1 -> 33.8.  Past the line: 1250 from 0 46.5 -> 50.3 | 47.8 -> 55.1 | 47.8 -> 54.1.
+// With their keys in parts, a multiple of 8 blocks (a round of a workgroup's waves) each, a workgroup has a part of a row
+// group's keys: the few tokens of a short turn behind a long prefix then fill the chip, each CU reading a part of the cache where
+// it lies, where the tiles would write and read the images of all of it for two or four of them.  0.36 us a block up to some
+// 200 workgroups, the chip 590 blocks a us; parts are some 7 us of ends, the merge 4.2 and a little for each part.  Two rounds of
+// workgroups at most, so that row groups of up to 64 tokens of 2 kv heads have parts to choose from and those of up to 256 two.
+// The whole call, halves, what it was -> parts: 7 tokens at 3000 31.3 -> 19.5 us, at 20000 49.8 -> 29.9, at 100000 186 -> 54.6; 30 at 3000 34.1 ->
+// 22.2, at 40000 79.0 -> 54.4; 64 at 1500 32.7 -> 20.9, at 20000 64.6 -> 52.8; 128 at 1000 25.0 -> 22.8, at 3000 35.6 -> 31.6; 250 at 1500
+// 36.2 -> 31.9.  Left alone: 128 at 10000 54.1 and 53.5, 250 at 4000 46.8 and 52.1 (with codes 49.3 and 53.8).
+void choose_small(FlashPlan &f, uint32_t pos, uint32_t tokens, uint32_t kv_heads, int bits, float tiles_us) {
+    const bool codes = bits != 16;
+    const float SMALL_US = 5.0f, BLOCK_US = codes ? 0.59f : 0.5f;
+    const float PART_US = codes ? 7.5f : 6.5f, PART_BLOCK_US = codes ? 0.37f : 0.36f, CHIP_BLOCKS_PER_US = (codes ? 570.0f : 590.0f) / 256.0f;
+    constexpr float MERGE_US = 4.2f, MERGE_PART_US = 0.1f;
+    if (tokens == 0 || kv_heads == 0) return;
+    const uint32_t longest = tile_blocks(pos, tokens, (tokens - 1) / TQ), shortest = tile_blocks(pos, tokens, 0);
+    const uint32_t groups = (tokens + 3) / 4 * kv_heads;
+    const float small_us = rounds_us(f.cus, groups, float(longest), float(shortest), SMALL_US, BLOCK_US, 0.0f);
+    f.small = small_us < tiles_us;
+    if (2 * uint64_t(groups) > f.cus) return;
+    float best = 0.95f * (f.small ? small_us : tiles_us);
+    const uint32_t least = (longest + SMALL_MAX_PARTS - 1) / SMALL_MAX_PARTS;
+    for (uint32_t pb = (least + SMALL_WAVES - 1) / SMALL_WAVES * SMALL_WAVES; pb < longest; pb += SMALL_WAVES) {
+        const uint32_t nparts = (longest + pb - 1) / pb, items = groups * nparts;
+        if (items > 2 * f.cus) continue;
+        const float us = rounds_us(f.cus, items, float(pb), float(pb), PART_US, PART_BLOCK_US, 1.0f / (CHIP_BLOCKS_PER_US * float(f.cus))) +
+                         MERGE_US + MERGE_PART_US * float(nparts) + 0.25f * MERGE_ITEM_US * float(items);
+        if (us < best) best = us, f.small_part_blocks = pb;
+        if (3 * items <= f.cus) break;  // (longer parts leave more of the chip idle)
+    }
+    if (f.small_part_blocks) f.small_parts = parts_bytes(tokens, kv_heads, parts_of(pos, tokens, f.small_part_blocks));
+}
+
+FlashPlan flash_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, int bits) {
+    float tiles_us;
+    FlashPlan f = tiles_plan(pos, tokens, kv_heads, tiles_us);
+    choose_small(f, pos, tokens, kv_heads, bits, tiles_us);
+    return f;
+}
+
+// (for either kind of cache)
+size_t workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads) {
+    float tiles_us;
+    FlashPlan halves = tiles_plan(pos, tokens, kv_heads, tiles_us), codes = halves;
+    choose_small(halves, pos, tokens, kv_heads, 16, tiles_us), choose_small(codes, pos, tokens, kv_heads, 8, tiles_us);
+    return halves.bytes() > codes.bytes() ? halves.bytes() : codes.bytes();
+}
 
 // The checks both prefill paths share.
 int check_prefill(int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
@@ -1291,22 +1375,36 @@ uint32_t launch_prepare(hipStream_t stream, int bits, const void *kdata, const v
     return nblocks;
 }
 
+// The row groups' launch; with part_blocks, their keys in parts that lie at the start of the workspace, and the merge.
 int launch_small(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
                  const uint16_t *kz, const uint16_t *vs, const uint16_t *vz, const float *q_and_gate, float *out,
-                 const saetta_flash_params &p, const char *what) {
-    SmallArgs a{q, static_cast<const unsigned char *>(kdata), static_cast<const unsigned char *>(vdata), ks, kz, vs, vz, q_and_gate, out, p.heads, p.kv_heads, p.pos, p.tokens, p.scale};
-    const dim3 grid((p.tokens + 3) / 4, p.kv_heads);
-    if (bits == 8) {
-        launch(prefill_small_kernel<8>, grid, SMALL_THREADS, SmallLds<8>::BYTES, stream, a);
-    } else if (bits == 4) {
-        launch(prefill_small_kernel<4>, grid, SMALL_THREADS, SmallLds<4>::BYTES, stream, a);
-    } else {
-        launch(prefill_small_kernel<16>, grid, SMALL_THREADS, SmallLds<16>::BYTES, stream, a);
+                 const saetta_flash_params &p, uint32_t part_blocks, void *workspace, const char *what) {
+    SmallArgs a{q, static_cast<const unsigned char *>(kdata), static_cast<const unsigned char *>(vdata), ks, kz, vs, vz, q_and_gate, out, p.heads, p.kv_heads, p.pos, p.tokens, p.scale, 0, 0, nullptr, nullptr};
+    auto kernels = [&](auto split, dim3 grid) {
+        constexpr bool SPLIT = decltype(split)::value;
+        if (bits == 8) {
+            launch(prefill_small_kernel<8, SPLIT>, grid, SMALL_THREADS, SmallLds<8>::BYTES, stream, a);
+        } else if (bits == 4) {
+            launch(prefill_small_kernel<4, SPLIT>, grid, SMALL_THREADS, SmallLds<4>::BYTES, stream, a);
+        } else {
+            launch(prefill_small_kernel<16, SPLIT>, grid, SMALL_THREADS, SmallLds<16>::BYTES, stream, a);
+        }
+    };
+    const uint32_t groups = (p.tokens + 3) / 4;
+    if (!part_blocks) {
+        kernels(std::false_type{}, dim3(groups, p.kv_heads));
+        return launch_status(what);
     }
+    a.part_blocks = part_blocks, a.nparts = parts_of(p.pos, p.tokens, part_blocks);
+    a.part_o = static_cast<float *>(workspace);
+    a.part_ml = a.part_o + size_t(a.nparts) * ((p.tokens + TQ - 1) / TQ) * p.kv_heads * (PART_O_BYTES / 4);
+    kernels(std::true_type{}, dim3((a.nparts * p.kv_heads * groups + 7) / 8 * 8));
+    PrefillArgs m{q, nullptr, q_and_gate, out, p.heads, p.kv_heads, p.pos, p.tokens, p.scale, 0, nullptr, part_blocks, a.part_o, a.part_ml};
+    launch(prefill_merge_kernel, dim3(p.tokens, p.kv_heads), MERGE_THREADS, 0, stream, m);
     return launch_status(what);
 }
 
-// The launches of a chunk in a workspace of at least plan.plain bytes, plan.bytes() with `split`.
+// The tiles' launches in a workspace of at least plan.plain bytes, plan.tiles() with `split`.
 int launch_flash(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
                  const uint16_t *kz, const uint16_t *vs, const uint16_t *vz, const float *q_and_gate, float *out,
                  const saetta_flash_params &p, void *workspace, bool split, bool exact, const FlashPlan &plan, const char *what) {
@@ -1331,6 +1429,18 @@ int launch_flash(hipStream_t stream, int bits, const uint16_t *q, const void *kd
     return launch_status(what);
 }
 
+// The chunk in a workspace of `have` bytes (none: 0, for the row groups without parts only; else at least plan.plain): the plan's
+// layout as far as there is room for its parts.
+int launch_chunk(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
+                 const uint16_t *kz, const uint16_t *vs, const uint16_t *vz, const float *q_and_gate, float *out,
+                 const saetta_flash_params &p, void *workspace, size_t have, bool exact, const FlashPlan &plan, const char *what) {
+    const bool small_parts = plan.small_part_blocks && have >= plan.small_parts;
+    if (small_parts || plan.small) {
+        return launch_small(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, small_parts ? plan.small_part_blocks : 0, workspace, what);
+    }
+    return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, have >= plan.tiles(), exact, plan, what);
+}
+
 int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata,
                 const uint16_t *ks, const uint16_t *kz, const uint16_t *vs, const uint16_t *vz,
                 const float *q_and_gate, float *out, saetta_flash_params p, void *workspace, size_t workspace_size,
@@ -1339,17 +1449,15 @@ int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kda
     if (int rc = ensure_device()) return rc;
     if (p.tokens == 0) return SAETTA_OK;
     const FlashPlan plan = flash_plan(p.pos, p.tokens, p.kv_heads, bits);
-    if (plan.small) {
-        // (a workspace that is given has to do, whatever the chunk: which launches serve it is no caller's business)
-        SAETTA_REQUIRE(!workspace || workspace_size >= plan.plain, SAETTA_E_SCRATCH, "%s: workspace of %zu bytes, %zu needed", what,
-                       workspace_size, plan.plain);
-        return launch_small(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, what);
-    }
-    size_t need = plan.bytes();
-    if (workspace && workspace_size < need) need = plan.plain;  // (room for the images only: the keys are not split)
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
-    if (int rc = acquire_workspace(stream, workspace, workspace_size, need, owned_lock, what, "saetta_prefill_workspace_bytes")) return rc;
-    return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, need >= plan.bytes(), false, plan, what);
+    size_t have = workspace ? workspace_size : 0;
+    // (a workspace that is given has to do for the images, whatever the chunk: which launches serve it is no caller's business.
+    // One of the library's is taken where the chunk does not do without.)
+    if (workspace || !plan.small) {
+        if (!workspace) have = plan.bytes();
+        if (int rc = acquire_workspace(stream, workspace, workspace_size, workspace ? plan.plain : have, owned_lock, what, "saetta_prefill_workspace_bytes")) return rc;
+    }
+    return launch_chunk(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, have, false, plan, what);
 }
 
 // ---- the same chunk as matrix products over blocks of 1024 keys ---------------------------------
@@ -1725,11 +1833,9 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
     // the workspace has no room for parts of the keys they are not split.
     if (stages == 0) {
         const FlashPlan plan = flash_plan(p.pos, p.tokens, p.kv_heads, bits);
-        const bool split = !workspace || workspace_size >= plan.bytes();
-        if (int rc = acquire_workspace(stream, workspace, workspace_size, split && plan.bytes() > need ? plan.bytes() : need, owned_lock, what,
-                                       "saetta_attn_gemm_workspace_bytes")) return rc;
-        if (plan.small) return launch_small(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, what);
-        return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, split, true, plan, what);
+        const size_t have = workspace ? workspace_size : plan.bytes() > need ? plan.bytes() : need;
+        if (int rc = acquire_workspace(stream, workspace, workspace_size, workspace ? need : have, owned_lock, what, "saetta_attn_gemm_workspace_bytes")) return rc;
+        return launch_chunk(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, have, true, plan, what);
     }
     if (int rc = acquire_workspace(stream, workspace, workspace_size, need, owned_lock, what, "saetta_attn_gemm_workspace_bytes")) return rc;
     const uint32_t nblocks = launch_prepare(stream, bits, kdata, vdata, ks, kz, vs, vz, workspace, p.kv_heads, rows);
@@ -1776,9 +1882,12 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
 
 int setup_prefill() {
     if (int rc = load_kernel(reinterpret_cast<const void *>(prefill_merge_kernel))) return rc;
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<16>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<16>::BYTES))) return rc;
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<8>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<8>::BYTES))) return rc;
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<4>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<4>::BYTES))) return rc;
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<16, false>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<16>::BYTES))) return rc;
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<16, true>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<16>::BYTES))) return rc;
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<8, false>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<8>::BYTES))) return rc;
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<8, true>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<8>::BYTES))) return rc;
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<4, false>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<4>::BYTES))) return rc;
+    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<4, true>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<4>::BYTES))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_scores_kernel))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_pv_kernel))) return rc;
     for (const void *kernel : {reinterpret_cast<const void *>(attention_prefill_kernel<true, false>), reinterpret_cast<const void *>(attention_prefill_kernel<true, true>),

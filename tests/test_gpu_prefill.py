@@ -268,6 +268,48 @@ def test_keys_in_parts(kind, pos, tokens):
         assert np.abs(got - want).max() < MAX_ABS
 
 
+def attention_64(q16, k, v, qg, pos):
+    """out [tokens][heads][256] in 64 bits, k and v [pos + tokens][kv][256] as the cache stands for them."""
+    tokens, heads, kv = q16.shape[0], q16.shape[1], k.shape[1]
+    q = q16.double().view(tokens, kv, 8, D).permute(1, 2, 0, 3).reshape(kv, 8 * tokens, D)
+    s = torch.matmul(q, k.double().permute(1, 2, 0).contiguous()) / 16
+    sees = torch.arange(pos + tokens, device="cuda")[None] <= pos + torch.arange(tokens, device="cuda")[:, None]
+    p = torch.softmax(s.view(kv, 8, tokens, -1).masked_fill(~sees, float("-inf")), -1).view(kv, 8 * tokens, -1)
+    o = torch.matmul(p, v.double().permute(1, 0, 2).contiguous()).view(kv, 8, tokens, D).permute(2, 0, 1, 3).reshape(tokens, heads, D)
+    return o * torch.sigmoid(qg.double().view(tokens, heads, 2 * D)[:, :, D:])
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("pos,tokens,kv", [(505, 1, 1), (767, 2, 2), (1020, 9, 2), (1279, 30, 3), (1800, 64, 2), (2047, 130, 2), (3000, 250, 2), (6100, 33, 1),
+                                           (9000, 7, 5), (20001, 30, 2), (50000, 5, 2)])
+def test_row_groups_with_their_keys_in_parts(kind, pos, tokens, kv):
+    # A part is a multiple of 8 blocks of 32 keys: a row group that sees no key of a part that its tile has (1020, 1279, 2047),
+    # one block of the last, parts of one round and of many, two rounds of workgroups, as many as 64 parts, kv heads that an
+    # eighth of the workgroups does not divide; in a workspace of NaN of just the size, and with room for the images only.
+    heads, n = 8 * kv, pos + tokens
+    gen = torch.Generator(device="cuda").manual_seed(pos)
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device="cuda")  # noqa: E731
+    k, v, q16, qg = normal(n, kv * D), normal(n, kv * D), normal(tokens, heads, D).half(), normal(tokens, heads, 2 * D)
+    if kind is saetta.KvBits.Half:
+        kc, vc = k.half(), v.half()
+        kf, vf = kc, vc
+    else:
+        kc, vc = saetta.QuantRows(kind, kv * D, n), saetta.QuantRows(kind, kv * D, n)
+        kc.encode(k.view(-1), 0, n), vc.encode(v.view(-1), 0, n)
+        kf, vf = (saetta.dequantize(*c.tensors(), kind) for c in (kc, vc))
+    want = attention_64(q16, kf.view(n, kv, D), vf.view(n, kv, D), qg, pos)
+    p = saetta.FlashParams(heads, kv, pos, tokens, 1.0 / 16)
+    for nbytes in (saetta.attention_prefill.workspace_bytes(p), -(-n // 32) * kv * 32768 + 256):
+        ws, out = torch.full((nbytes,), 0xff, dtype=torch.uint8, device="cuda"), torch.full((tokens, heads, D), float("nan"), device="cuda")
+        if kind is saetta.KvBits.Half:
+            saetta.attention_prefill.encode(saetta.attention_prefill.DEFAULT, q16, kc, vc, qg, out, p, workspace=ws)
+        else:
+            saetta.attention_prefill.encode_quant(q16, kc, vc, qg, out, p, workspace=ws)
+        off = (out.double() - want).norm() / want.norm()
+        assert float(off) < REL_RMS, float(off)
+        assert float((out - want).abs().max()) < MAX_ABS
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("pos,tokens", [(0, 4), (31, 1), (32, 2), (125, 3), (126, 5), (253, 3), (254, 5), (300, 17), (500, 30)])
 def test_short_chunks_over_short_contexts(kind, pos, tokens):
