@@ -353,7 +353,6 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
 
     // Row of this lane: token tok0 + col / 8, head col % 8.
     const uint32_t tok = tok0 + (col >> 3);
-    const uint32_t head = kv * 8 + (col & 7);
 
     // Keys this workgroup walks: up to what its last token sees; what this wave needs.  A part's keys count from its
     // first block on: key0 is that block's first key, and a row of the tile may see none of the part (the tile's tokens
@@ -388,29 +387,56 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     //   parity 1:  O(2s+1) + S(2s+3)         | softmax(2s+3)
     // During step s the workgroup copies what step s + 1 reads: K(2s+4), K(2s+5), V(2s+2),
     // V(2s+3); wave w takes half (w % 2) of part w / 2 of that list.  Before the loop: K(0..3),
-    // V(0), V(1), twelve kilobytes per wave.
-    for (int i = wave; i < 48; i += WAVES) {
-        const int part = i >> 3, v = part >= 4;
-        const uint32_t b = v ? part - 4 : part;
-        Copy cp = piece(b, v, 0);
-        cp.src += (i & 7) * 2048, cp.dst += (i & 7) * 2048;
+    // V(0), V(1), in front of them the queries.
+    auto copy2k = [&](uint64_t src, uint32_t dst) {
         asm volatile(
             "s_mov_b32 m0, %[dst]\n"
             "s_nop 0\n"
             "global_load_lds_dwordx4 %[off], %[src]\n"
             "global_load_lds_dwordx4 %[off], %[src] offset:1024\n"
             :
-            : [off] "v"(lane16), [src] "s"(cp.src), [dst] "s"(cp.dst)
+            : [off] "v"(lane16), [src] "s"(src), [dst] "s"(dst)
+            : "memory", "m0");
+    };
+    // Q^T operands: lane (col, hf), k-step st: dims 16 st + 8 hf .. + 7 of its row.  They come through LDS, in the places of
+    // V(0..3): a load of 16 bytes of each of 32 rows is taken a row a cycle, and 16 of them in eight waves were 4 us in front of a
+    // tile (1470 tokens from 0: first keys and queries there after 5.2 us, now 2.7).  A row group's 16 KB as they lie in memory, half
+    // by each of its two waves; place p of row r holds the row's 16-byte piece (p - 4 (r / 4) mod 32) ^ (r % 4), which puts what
+    // 16 lanes read on different banks and keeps every 64 bytes of memory together.
+    uint32_t at = lane;  // (what depends on the lane is made where it is used, not kept in registers from tile to tile)
+    asm volatile("" : "+v"(at));
+    const uint32_t q_place = lds0 + v_slot(0) + group * (32 * DIM * 2);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const uint32_t k = 8 * parity + i;  // rows 2k and 2k + 1
+        const uint32_t tk = min(tok0 + k / 4, a.tokens - 1);
+        const uint64_t src = reinterpret_cast<uint64_t>(a.q) + ((size_t(tk) * a.heads + kv * SAETTA_GQA_GROUP + 2 * k % 8) * DIM) * 2;
+        const uint32_t off = (at >> 5) * 512 + (((at - 4 * (i >> 1 & 3)) & 31) ^ (2 * (i & 1) + (at >> 5))) * 16;
+        asm volatile(
+            "s_mov_b32 m0, %[dst]\n"
+            "s_nop 0\n"
+            "global_load_lds_dwordx4 %[off], %[src]\n"
+            :
+            : [off] "v"(off), [src] "s"(src), [dst] "s"(q_place + k * 1024)
             : "memory", "m0");
     }
-
-    // Q^T operands: lane (col, hf), k-step st: dims 16 st + 8 hf .. + 7 of its row.
-    half8 qb[16];
-    {
-        const uint32_t tk = min(tok, a.tokens - 1);
-        const u32x4 *src = reinterpret_cast<const u32x4 *>(a.q + (size_t(tk) * a.heads + head) * DIM + 8 * hf);
 #pragma unroll
-        for (int st = 0; st < 16; st++) qb[st] = __builtin_bit_cast(half8, src[2 * st]);
+    for (int i = 0; i < 4; i++) {  // K(0..3): wave w takes 2 KB of each
+        const Copy cp = piece(i, 0, 0);
+        copy2k(cp.src + wave * 2048, cp.dst + wave * 2048);
+    }
+    asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");  // (the keys stay on their way)
+    half8 qb[16];
+#pragma unroll
+    for (int st = 0; st < 16; st++) {
+        const uint32_t place = 4 * (((st >> 1) + (at >> 2 & 3)) & 7) + ((2 * (st & 1) + (at >> 5)) ^ (at & 3));
+        qb[st] = *reinterpret_cast<const half8 *>(tiles + v_slot(0) + group * (32 * DIM * 2) + (at & 31) * (DIM * 2) + place * 16);
+    }
+    lds_barrier();  // the queries have been read: the values may land there
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const Copy cp = piece(i, 1, 0);
+        copy2k(cp.src + wave * 2048, cp.dst + wave * 2048);
     }
 
     floatx16 acc[8];
@@ -477,8 +503,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
         }
     };
 
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();  // K(0..3), V(0), V(1) are in LDS
+    asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");  // K(0..3) are in LDS, V(0) and V(1) on their way
 
     const uint32_t nsteps = (nblocks + 1) / 2;
     const int part = wave >> 1, half = wave & 1;  // what the wave copies in every step
@@ -491,7 +516,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
 #pragma unroll
         for (int r = 0; r < 16; r++) s[r] = 0.0f;
         if (0 < wave_blocks) scores_block(s, qb, lds0 + k_slot(0) + lane16);
-        __syncthreads();  // the first step's copies overwrite K(0) and K(1)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();  // V(0) and V(1) are there; the first step's copies overwrite K(0) and K(1)
         for (uint32_t step = 0; step < nsteps; step++) {
             const Copy cp = copy_of(step);
             const uint32_t kb = 2 * step;
@@ -515,6 +541,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
             raise_max(mask_max(s, BK, 1 >= full_blocks), 1);
             exp_pack(s, pb);
         }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         for (uint32_t step = 0; step < nsteps; step++) {
             const Copy cp = copy_of(step);
@@ -547,43 +574,48 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     if (ask && tid == 0) got = gridDim.x + atomicAdd(a.tiles_taken, 1u);
 
     // The gate values of this wave's half of the dims, asked for before the merge below so that they travel while
-    // it runs (scattered 16-byte pieces, one round trip for the lot; a token past the end: the last token's, unused).
+    // it runs: two rows of 512 bytes a load, as the outputs are stored (a token past the end: the last token's, unused).
+    asm volatile("" : "+v"(at));
     float4 g[16];
+    const uint32_t half_row = at >> 5, in_row = 4 * (at & 31);  // a lane's row of two; its dims of the half
+    auto first_row = [&](int i) { return size_t(min(tok0 + i / 4, a.tokens - 1)) * a.heads + kv * SAETTA_GQA_GROUP + 2 * i % 8; };
     if constexpr (!SPLIT) {
-        const size_t grow = size_t(min(tok, a.tokens - 1)) * a.heads + head;
-        const float *gate = a.q_and_gate + grow * 2 * DIM + DIM + 128 * parity;
 #pragma unroll
-        for (int i = 0; i < 16; i++) g[i] = *reinterpret_cast<const float4 *>(gate + 32 * (i >> 2) + 8 * (i & 3) + 4 * hf);
+        for (int i = 0; i < 16; i++) g[i] = *reinterpret_cast<const float4 *>(a.q_and_gate + first_row(i) * 2 * DIM + DIM + 128 * parity + (half_row * 2 * DIM + in_row));
     }
     // ---- the two waves of a row group merge their halves of the keys ----------------------
     // Each wave finishes half of the dims: parity 0 the accumulators 0..3 (dims 0..127), parity 1
     // the rest.  It hands the other half, m and l to its partner through LDS (the tiles are done
-    // with: the loop ended on a barrier); element e of lane L sits at word e * 64 + L.
-    float *mine_out = reinterpret_cast<float *>(tiles + wave * MERGE_WAVE_BYTES) + lane;
-    const float *theirs_in = reinterpret_cast<const float *>(tiles + (wave ^ 4) * MERGE_WAVE_BYTES) + lane;
+    // with: the loop ended on a barrier), four accumulator registers of a lane side by side.
+    float4 *mine_out = reinterpret_cast<float4 *>(tiles + wave * MERGE_WAVE_BYTES) + at;
+    unsigned char *theirs_base = tiles + (wave ^ 4) * MERGE_WAVE_BYTES;
+    const float4 *theirs_in = reinterpret_cast<const float4 *>(theirs_base) + at;
     floatx16 fin[4];
+    auto hand_over = [&](const floatx16 &x, int i) {
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++) mine_out[(4 * i + q4) * 64] = float4{x[4 * q4], x[4 * q4 + 1], x[4 * q4 + 2], x[4 * q4 + 3]};
+    };
     if (parity == 0) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            fin[i] = acc[i];
-#pragma unroll
-            for (int r = 0; r < 16; r++) mine_out[(16 * i + r) * 64] = acc[4 + i][r];
-        }
+        for (int i = 0; i < 4; i++) fin[i] = acc[i], hand_over(acc[4 + i], i);
     } else {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            fin[i] = acc[4 + i];
-#pragma unroll
-            for (int r = 0; r < 16; r++) mine_out[(16 * i + r) * 64] = acc[i][r];
-        }
+        for (int i = 0; i < 4; i++) fin[i] = acc[4 + i], hand_over(acc[i], i);
     }
-    mine_out[64 * 64] = m_ref;
-    mine_out[65 * 64] = l_sum;
+    float2 *ml_out = reinterpret_cast<float2 *>(tiles + wave * MERGE_WAVE_BYTES + 16 * 1024) + at;
+    *ml_out = float2{m_ref, l_sum};
     lds_barrier();  // (the gate values stay on their way)
-    const float m_other = theirs_in[64 * 64], l_other = theirs_in[65 * 64];
+    const float2 ml_other = *(reinterpret_cast<const float2 *>(theirs_base + 16 * 1024) + at);
+    const float m_other = ml_other.x, l_other = ml_other.y;
     const float m_new = fmaxf(m_ref, m_other);
     const float mine = __builtin_amdgcn_exp2f(m_ref - m_new), theirs = __builtin_amdgcn_exp2f(m_other - m_new);
     l_sum = l_sum * mine + l_other * theirs;
+    auto joined = [&](int i) {
+        const int mt = i >> 2, q4 = i & 3;
+        const float4 x = theirs_in[i * 64];
+        return float4{fin[mt][4 * q4] * mine + x.x * theirs, fin[mt][4 * q4 + 1] * mine + x.y * theirs,
+                      fin[mt][4 * q4 + 2] * mine + x.z * theirs, fin[mt][4 * q4 + 3] * mine + x.w * theirs};
+    };
 
     if constexpr (SPLIT) {
         // The part's O, m and l as they are, a contiguous kilobyte per store of a wave.  (Rows past the chunk's end leave
@@ -594,12 +626,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
         float *po = a.part_o + ((item * WAVES + group * 2 + parity) * 16 * 64 + lane) * 4;
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            const int mt = i >> 2, q4 = i & 3;
-            float4 w;
-            w.x = fin[mt][4 * q4] * mine + theirs_in[(16 * mt + 4 * q4) * 64] * theirs;
-            w.y = fin[mt][4 * q4 + 1] * mine + theirs_in[(16 * mt + 4 * q4 + 1) * 64] * theirs;
-            w.z = fin[mt][4 * q4 + 2] * mine + theirs_in[(16 * mt + 4 * q4 + 2) * 64] * theirs;
-            w.w = fin[mt][4 * q4 + 3] * mine + theirs_in[(16 * mt + 4 * q4 + 3) * 64] * theirs;
+            const float4 w = joined(i);
             *reinterpret_cast<float4 *>(po + i * 64 * 4) = w;
         }
         if (parity == 0 && hf == 0) {
@@ -613,26 +640,30 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     // ---- out = O / l * sigmoid(gate) ---------------------------------------------------
     // The lane's row sum is split over the two lane halves (each saw half the keys).
     const float l = l_sum + __shfl_xor(l_sum, 32);
-    if (tok < a.tokens) {
-        const float inv = 1.0f / l;
-        const size_t row = size_t(tok) * a.heads + head;
-        float *out = a.out + row * DIM + 128 * parity;
+    // Through LDS once more, so that a wave stores whole lines: 16 bytes of each of 32 rows are taken a row a cycle, gates
+    // and outputs both (8 us of a tile's end, 1470 tokens from 0; now 4.2).  A lane's four dims of its row are a piece; the
+    // pieces of the same dims lie side by side, 528 bytes from the next dims', in the place of what the partner handed over,
+    // which nobody else reads (a wave's LDS accesses run in order).
+    const float inv = 1.0f / l;
+    float4 o[16];
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int mt = i >> 2, q4 = i & 3;
-            float o[4];
+    for (int i = 0; i < 16; i++) {
+        o[i] = joined(i);
+        o[i].x *= inv, o[i].y *= inv, o[i].z *= inv, o[i].w *= inv;
+    }
+    constexpr int PIECE = 32 * 16 + 16;
+    static_assert(32 * PIECE <= MERGE_WAVE_BYTES, "the pieces of 32 rows");
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int r = 4 * q4 + e;
-                o[e] = (fin[mt][r] * mine + theirs_in[(16 * mt + r) * 64] * theirs) * inv;
-            }
-            float4 w;
-            w.x = o[0] * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].x));
-            w.y = o[1] * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].y));
-            w.z = o[2] * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].z));
-            w.w = o[3] * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].w));
-            *reinterpret_cast<float4 *>(out + 32 * mt + 8 * q4 + 4 * hf) = w;
-        }
+    for (int i = 0; i < 16; i++) *reinterpret_cast<float4 *>(theirs_base + (2 * i + (at >> 5)) * PIECE + (at & 31) * 16) = o[i];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const float4 x = *reinterpret_cast<const float4 *>(theirs_base + in_row / 4 * PIECE + (2 * i + half_row) * 16);
+        float4 w;
+        w.x = x.x * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].x));
+        w.y = x.y * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].y));
+        w.z = x.z * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].z));
+        w.w = x.w * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].w));
+        if (tok0 + i / 4 < a.tokens) *reinterpret_cast<float4 *>(a.out + first_row(i) * DIM + 128 * parity + (half_row * DIM + in_row)) = w;
     }
     if (tid == 0) *next_tile = got;
 }
