@@ -716,72 +716,137 @@ __global__ __launch_bounds__(THREADS, 2) void attention_prefill_kernel(PrefillAr
     }
 }
 
+// Registers x[0..3] of four lanes, lane t holding piece t of row j in x[j]: then lane t holds piece j of its row t.
+__device__ __forceinline__ void turn(u32x4 *x, int lane) {
+    const bool odd = lane & 1, high = lane & 2;
+#pragma unroll
+    for (int j = 0; j < 4; j += 2)
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const uint32_t u = x[j][w], v = x[j + 1][w];
+            const uint32_t un = __builtin_amdgcn_mov_dpp(int(u), 0xb1, 0xf, 0xf, true), vn = __builtin_amdgcn_mov_dpp(int(v), 0xb1, 0xf, 0xf, true);
+            x[j][w] = odd ? vn : u, x[j + 1][w] = odd ? v : un;
+        }
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const uint32_t u = x[j][w], v = x[j + 2][w];
+            const uint32_t un = __builtin_amdgcn_mov_dpp(int(u), 0x4e, 0xf, 0xf, true), vn = __builtin_amdgcn_mov_dpp(int(v), 0x4e, 0xf, 0xf, true);
+            x[j][w] = high ? vn : u, x[j + 2][w] = high ? v : un;
+        }
+}
+
 // Joins the parts of every tile: out = sum_p 2^(m_p - m) O_p / sum_p 2^(m_p - m) l_p * sigmoid(gate).  A workgroup takes
-// one token of one kv head: 8 rows x 256 dims, two float4 per thread.  The parts lie in accumulator order, where the 8
-// rows' pieces of four dims are one line of 128 bytes: 8 neighbouring lanes take a line of a part and 16 bytes each of
-// 8 rows of `out`, of which a wave writes 128 bytes (a lane per piece of ONE row made every lane of a load its own
-// line: 22 us for 50 MB of parts).
-constexpr int MERGE_THREADS = 256;
-__global__ __launch_bounds__(MERGE_THREADS) void prefill_merge_kernel(PrefillArgs a) {
+// one token of one kv head: 8 rows x 256 dims, four float4 per thread.  The parts lie in accumulator order, where the 8
+// rows' pieces of four dims are one line of 128 bytes: 8 neighbouring lanes take a line of a part (a lane per piece of ONE
+// row made every lane of a load its own line: 22 us for 50 MB of parts).  Then four lanes turn their four pieces of four rows
+// round, so that gates and outputs move 512 bytes of a row at a time and not 16 of each of eight, which are taken a row a
+// cycle (the whole call: 1032 tokens at 38 41.1 -> 40.3 us, 150 at 9000 50.2 -> 49.0, 7 at 3000 19.0 -> 18.2).
+// TEAMS: more than eight parts are dealt to four teams of 128 threads, joined through LDS: one team's batches come one after
+// another, a trip through memory each (the whole call: 7 tokens at 3000 18.2 -> 17.4 us, 10 at 103706 63.5 -> 61.3; from 9 parts on
+// four teams are ahead or even: 55 tokens at 17388 47.0 both).
+constexpr int MERGE_THREADS = 128, MERGE_TEAMS = 4;
+template <int TEAMS>
+__global__ __launch_bounds__(MERGE_THREADS * TEAMS, 4) void prefill_merge_kernel(PrefillArgs a) {
+    __shared__ floatx4 team_o[TEAMS > 1 ? TEAMS - 1 : 1][4][MERGE_THREADS];
+    __shared__ float2 team_ml[TEAMS > 1 ? TEAMS - 1 : 1][8];
+    const uint32_t tid = TEAMS > 1 ? threadIdx.x % MERGE_THREADS : threadIdx.x, team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / MERGE_THREADS) : 0;
     const uint32_t tok = blockIdx.x, kv = blockIdx.y, tile = tok / TQ, group = (tok % TQ) / 4;
     const uint32_t ntiles = (a.tokens + TQ - 1) / TQ;
     const uint32_t parts = (tile_blocks(a.pos, a.tokens, tile) + a.part_blocks - 1) / a.part_blocks;
     const size_t item_stride = size_t(ntiles) * a.kv_heads, item0 = size_t(tile) * a.kv_heads + kv;
-    const uint32_t h = threadIdx.x & 7;
+    const uint32_t h = tid & 7, four = tid >> 3, col = (tok % 4) * 8 + h;  // pieces 4 four .. + 3 of row h
+    // gates and outputs: piece 4 four + h % 4 of rows h / 4 * 4 .. + 3
+    const size_t row = size_t(tok) * a.heads + kv * SAETTA_GQA_GROUP + (h & 4);
+    const uint32_t dim = 16 * four + 4 * (h & 3);
+    float4 g[4];
+    if (team == 0) {
 #pragma unroll
-    for (int half = 0; half < 2; half++) {
-        const uint32_t piece = 32 * half + (threadIdx.x >> 3);       // dims 4 piece .. + 3 of the row
-        const uint32_t i = (piece >> 1) & 15, parity = piece >> 5;   // mt % 4 and q4; which half of the dims
-        const uint32_t col = (tok % 4) * 8 + h, lane = (piece & 1) * 32 + col;
-        const size_t row = size_t(tok) * a.heads + kv * SAETTA_GQA_GROUP + h;
-        const float4 g = *reinterpret_cast<const float4 *>(a.q_and_gate + row * 2 * DIM + DIM + 4 * piece);
-        const float *ml = a.part_ml + ((item0 * 4 + group) * 32 + col) * 2;
-        const float *po = a.part_o + (((item0 * WAVES + group * 2 + parity) * 16 + i) * 64 + lane) * 4;
-        float m = 4.0f * NO_SCORE, l = 0.0f;
-        float4 o = {0.0f, 0.0f, 0.0f, 0.0f};
-        // BATCH parts at a time, all of their loads requested before the first is used (past the last part: the last part
-        // again, with no weight: in batches of 8 whatever the number, a tile of two parts asked for each of them four times;
-        // 777 tokens from 0 12.1 -> 8.9 us, 2300 at 10000 36.4 -> 31.0, which is 4.8 TB/s of parts, gates and outputs)
-        auto join = [&](auto batch) {
-            constexpr int BATCH = decltype(batch)::value;
-            for (uint32_t p0 = 0; p0 < parts; p0 += BATCH) {
-                float2 x[BATCH];
-                float4 y[BATCH];
+        for (int j = 0; j < 4; j++) g[j] = *reinterpret_cast<const float4 *>(a.q_and_gate + (row + j) * 2 * DIM + DIM + dim);
+    }
+    const float *ml = a.part_ml + ((item0 * 4 + group) * 32 + col) * 2;
+    // (pieces 2i and 2i + 1 are accumulator registers 4i .. 4i + 3 of the lanes col and col + 32)
+    const float *po = a.part_o + (((item0 * WAVES + group * 2 + (four >> 3)) * 16 + 2 * (four & 7)) * 64 + col) * 4;
+    float m = 4.0f * NO_SCORE, l = 0.0f;
+    floatx4 o[4] = {};
+    // BATCH parts at a time, all of their loads requested before the first is used (past the last part: the last part
+    // again, with no weight: in batches of 8 whatever the number, a tile of two parts asked for each of them four times;
+    // 777 tokens from 0 12.1 -> 8.9 us, 2300 at 10000 36.4 -> 31.0, which is 4.8 TB/s of parts, gates and outputs)
+    auto join = [&](auto batch) {
+        constexpr int BATCH = decltype(batch)::value;
+        for (uint32_t p0 = team * BATCH; p0 < parts; p0 += TEAMS * BATCH) {
+            float2 x[BATCH];
+            floatx4 y[BATCH][4];
 #pragma unroll
-                for (int j = 0; j < BATCH; j++) {
-                    const uint32_t p = min(p0 + j, parts - 1);
-                    x[j] = *reinterpret_cast<const float2 *>(ml + p * item_stride * (4 * 32 * 2));
-                    y[j] = *reinterpret_cast<const float4 *>(po + p * item_stride * (WAVES * 16 * 64 * 4));
-                }
-                float m_new = m;
+            for (int j = 0; j < BATCH; j++) {
+                const uint32_t p = min(p0 + j, parts - 1);
+                x[j] = *reinterpret_cast<const float2 *>(ml + p * item_stride * (4 * 32 * 2));
 #pragma unroll
-                for (int j = 0; j < BATCH; j++) m_new = fmaxf(m_new, x[j].x);
-                const float old = __builtin_amdgcn_exp2f(m - m_new);
-                m = m_new;
-                l *= old;
-                o.x *= old, o.y *= old, o.z *= old, o.w *= old;
-#pragma unroll
-                for (int j = 0; j < BATCH; j++) {
-                    const float now = p0 + j < parts ? __builtin_amdgcn_exp2f(x[j].x - m_new) : 0.0f;
-                    l += x[j].y * now;
-                    o.x += y[j].x * now, o.y += y[j].y * now, o.z += y[j].z * now, o.w += y[j].w * now;
-                }
+                for (int k = 0; k < 4; k++) y[j][k] = *reinterpret_cast<const floatx4 *>(po + p * item_stride * (WAVES * 16 * 64 * 4) + ((k >> 1) * 64 + (k & 1) * 32) * 4);
             }
-        };
-        if (parts <= 2) {
-            join(std::integral_constant<int, 2>{});
-        } else if (parts <= 4) {
-            join(std::integral_constant<int, 4>{});
-        } else {
-            join(std::integral_constant<int, 8>{});
+            float m_new = m;
+#pragma unroll
+            for (int j = 0; j < BATCH; j++) m_new = fmaxf(m_new, x[j].x);
+            const float old = __builtin_amdgcn_exp2f(m - m_new);
+            m = m_new;
+            l *= old;
+#pragma unroll
+            for (int k = 0; k < 4; k++) o[k] *= old;
+#pragma unroll
+            for (int j = 0; j < BATCH; j++) {
+                const float now = p0 + j < parts ? __builtin_amdgcn_exp2f(x[j].x - m_new) : 0.0f;
+                l += x[j].y * now;
+#pragma unroll
+                for (int k = 0; k < 4; k++) o[k] += y[j][k] * now;
+            }
         }
-        const float inv = 1.0f / l;
-        float4 w;
-        w.x = o.x * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.x));
-        w.y = o.y * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.y));
-        w.z = o.z * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.z));
-        w.w = o.w * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g.w));
-        *reinterpret_cast<float4 *>(a.out + row * DIM + 4 * piece) = w;
+    };
+    if constexpr (TEAMS > 1) {
+        if (parts <= 4 * TEAMS) join(std::integral_constant<int, 4>{});
+        else join(std::integral_constant<int, 8>{});
+        if (team > 0) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) team_o[team - 1][k][tid] = o[k];
+            if (four == 0) team_ml[team - 1][h] = float2{m, l};
+        }
+        __syncthreads();
+        if (team > 0) return;
+        float top = m;
+#pragma unroll
+        for (int t = 0; t < TEAMS - 1; t++) top = fmaxf(top, team_ml[t][h].x);
+        const float own = __builtin_amdgcn_exp2f(m - top);
+        l *= own;
+#pragma unroll
+        for (int k = 0; k < 4; k++) o[k] *= own;
+#pragma unroll
+        for (int t = 0; t < TEAMS - 1; t++) {  // (a team without a part: l = 0, o = 0)
+            const float now = __builtin_amdgcn_exp2f(team_ml[t][h].x - top);
+            l += team_ml[t][h].y * now;
+#pragma unroll
+            for (int k = 0; k < 4; k++) o[k] += team_o[t][k][tid] * now;
+        }
+    } else if (parts <= 2) {
+        join(std::integral_constant<int, 2>{});
+    } else if (parts <= 4) {
+        join(std::integral_constant<int, 4>{});
+    } else {
+        join(std::integral_constant<int, 8>{});
+    }
+    const float inv = 1.0f / l;
+    u32x4 w[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) w[k] = __builtin_bit_cast(u32x4, o[k] * inv);
+    turn(w, tid);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const floatx4 x = __builtin_bit_cast(floatx4, w[j]);
+        float4 r;
+        r.x = x[0] * __builtin_amdgcn_rcpf(1.0f + __expf(-g[j].x));
+        r.y = x[1] * __builtin_amdgcn_rcpf(1.0f + __expf(-g[j].y));
+        r.z = x[2] * __builtin_amdgcn_rcpf(1.0f + __expf(-g[j].z));
+        r.w = x[3] * __builtin_amdgcn_rcpf(1.0f + __expf(-g[j].w));
+        *reinterpret_cast<float4 *>(a.out + (row + j) * DIM + dim) = r;
     }
 }
 
@@ -976,27 +1041,6 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
         }
     };
 
-    // Registers x[0..3] of four lanes, lane t holding piece t of row j in x[j]: then lane t holds piece j of its row t.
-    const bool odd = lane & 1, high = lane & 2;
-    auto turn = [&](u32x4 *x) {
-#pragma unroll
-        for (int j = 0; j < 4; j += 2)
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-                const uint32_t u = x[j][w], v = x[j + 1][w];
-                const uint32_t un = __builtin_amdgcn_mov_dpp(int(u), 0xb1, 0xf, 0xf, true), vn = __builtin_amdgcn_mov_dpp(int(v), 0xb1, 0xf, 0xf, true);
-                x[j][w] = odd ? vn : u, x[j + 1][w] = odd ? v : un;
-            }
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-                const uint32_t u = x[j][w], v = x[j + 2][w];
-                const uint32_t un = __builtin_amdgcn_mov_dpp(int(u), 0x4e, 0xf, 0xf, true), vn = __builtin_amdgcn_mov_dpp(int(v), 0x4e, 0xf, 0xf, true);
-                x[j][w] = high ? vn : u, x[j + 2][w] = high ? v : un;
-            }
-    };
-
     if (uint32_t(wave) < active) fetch_keys(first + wave);
     // Q^T operands: through LDS, where all waves read them
     {
@@ -1032,7 +1076,7 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
                 const int g = i * 2 * VALUES / SAETTA_QUANT_GROUP;
                 ks = kss[g >> 1] >> (16 * (g & 1)), kz = kzs[g >> 1] >> (16 * (g & 1));
             }
-            if (BITS == 16 && st % 4 == 0) turn(&kreg[i]);
+            if (BITS == 16 && st % 4 == 0) turn(&kreg[i], lane);
             const half8 q = *reinterpret_cast<const half8 *>(lds + L::Q_OFF + st * 1024 + lane * 16);
             s = __builtin_amdgcn_mfma_f32_32x32x16_f16(eight(kreg[i], st % STEPS, ks, kz), q, s, 0, 0, 0);
         }
@@ -1406,6 +1450,12 @@ uint32_t launch_prepare(hipStream_t stream, int bits, const void *kdata, const v
     return nblocks;
 }
 
+void launch_merge(hipStream_t stream, const PrefillArgs &a, uint32_t nparts) {
+    const dim3 grid(a.tokens, a.kv_heads);
+    if (nparts > 8) launch(prefill_merge_kernel<MERGE_TEAMS>, grid, MERGE_THREADS * MERGE_TEAMS, 0, stream, a);
+    else launch(prefill_merge_kernel<1>, grid, MERGE_THREADS, 0, stream, a);
+}
+
 // The row groups' launch; with part_blocks, their keys in parts that lie at the start of the workspace, and the merge.
 int launch_small(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
                  const uint16_t *kz, const uint16_t *vs, const uint16_t *vz, const float *q_and_gate, float *out,
@@ -1431,7 +1481,7 @@ int launch_small(hipStream_t stream, int bits, const uint16_t *q, const void *kd
     a.part_ml = a.part_o + size_t(a.nparts) * ((p.tokens + TQ - 1) / TQ) * p.kv_heads * (PART_O_BYTES / 4);
     kernels(std::true_type{}, dim3((a.nparts * p.kv_heads * groups + 7) / 8 * 8));
     PrefillArgs m{q, nullptr, q_and_gate, out, p.heads, p.kv_heads, p.pos, p.tokens, p.scale, 0, nullptr, part_blocks, a.part_o, a.part_ml};
-    launch(prefill_merge_kernel, dim3(p.tokens, p.kv_heads), MERGE_THREADS, 0, stream, m);
+    launch_merge(stream, m, a.nparts);
     return launch_status(what);
 }
 
@@ -1452,7 +1502,7 @@ int launch_flash(hipStream_t stream, int bits, const uint16_t *q, const void *kd
         a.part_ml = reinterpret_cast<float *>(ws + plan.plain + size_t(plan.nparts) * ntiles * p.kv_heads * PART_O_BYTES);
         const uint32_t total = prefill_items(p.pos, p.tokens, plan.part_blocks) * p.kv_heads;
         launch(exact ? attention_prefill_kernel<true, true> : attention_prefill_kernel<true, false>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
-        launch(prefill_merge_kernel, dim3(p.tokens, p.kv_heads), MERGE_THREADS, 0, stream, a);
+        launch_merge(stream, a, plan.nparts);
     } else {
         const uint32_t total = ntiles * p.kv_heads;
         launch(exact ? attention_prefill_kernel<false, true> : attention_prefill_kernel<false, false>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
@@ -1912,7 +1962,7 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
 }  // namespace
 
 int setup_prefill() {
-    if (int rc = load_kernel(reinterpret_cast<const void *>(prefill_merge_kernel))) return rc;
+    if (int rc = load_kernel(reinterpret_cast<const void *>(prefill_merge_kernel<1>))) return rc;
     if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<16, false>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<16>::BYTES))) return rc;
     if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<16, true>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<16>::BYTES))) return rc;
     if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<8, false>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<8>::BYTES))) return rc;

@@ -310,6 +310,12 @@ def test_row_groups_with_their_keys_in_parts(kind, pos, tokens, kv):
         assert float((out - want).abs().max()) < MAX_ABS
 
 
+@pytest.mark.parametrize("pos,tokens", [(2045, 3), (2300, 4), (4200, 3), (8186, 5), (8200, 4), (16300, 2)])
+def test_many_parts_are_merged_by_teams(pos, tokens):
+    # 8 parts of 8 blocks and one team, 9 and more and four: teams without a part, one batch each and two, a last batch of one
+    test_row_groups_with_their_keys_in_parts(saetta.KvBits.Half, pos, tokens, 2)
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("pos,tokens", [(0, 4), (31, 1), (32, 2), (125, 3), (126, 5), (253, 3), (254, 5), (300, 17), (500, 30)])
 def test_short_chunks_over_short_contexts(kind, pos, tokens):
