@@ -909,12 +909,13 @@ struct SmallLds {
     static_assert(BYTES <= 160 * 1024, "LDS of a CU");
 };
 
-// Which dims MFMA k-step st holds in lane half hf (8 of them): what a 16-byte piece of a row gives, whatever a value's size.
+// Where dims 8 u .. + 7 of the 32 query rows lie in LDS, [k-step][half][row][16 bytes]: MFMA k-step and lane half are those in which a
+// key's lane holds the same dims, which is what a 16-byte piece of its row gives, whatever a value's size.
 template <int BITS>
-__device__ __forceinline__ constexpr int small_dim(int st, int hf) {
-    constexpr int STEPS = 16 / BITS;  // k-steps per piece
-    const int i = st / STEPS;         // the lane's register
-    return (BITS == 16 ? (i / 4 * 2 + hf) * 4 + i % 4 : i * 2 + hf) * 8 * STEPS + st % STEPS * 8;
+__device__ __forceinline__ uint32_t small_place(uint32_t u) {
+    constexpr uint32_t STEPS = 16 / BITS;
+    const uint32_t st = BITS == 16 ? u / 8 * 4 + u % 4 : u / (2 * STEPS) * STEPS + u % STEPS, hf = BITS == 16 ? u / 4 % 2 : u / STEPS % 2;
+    return st * 1024 + hf * 512;
 }
 
 template <int BITS, bool SPLIT>
@@ -934,7 +935,7 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
         at_group = item % groups, kv = pair % kvh, part = pair / kvh;
     }
     const uint32_t tok0 = (groups - 1 - at_group) * 4;  // (the row groups that see the most keys first)
-    const uint32_t tok = tok0 + (col >> 3), head = kv * SAETTA_GQA_GROUP + (col & 7);
+    const uint32_t tok = tok0 + (col >> 3);
     const float c = a.scale * 1.4426950408889634f;
     const uint32_t keys = a.pos + min(tok0 + 4, a.tokens);  // what the last of its tokens sees
     const uint32_t first = SPLIT ? part * a.part_blocks : 0;         // blocks of keys: this workgroup's are first .. nblocks - 1
@@ -1042,17 +1043,17 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
     };
 
     if (uint32_t(wave) < active) fetch_keys(first + wave);
-    // Q^T operands: through LDS, where all waves read them
+    // Q^T operands: through LDS, where all waves read them.  Wave w fetches 64 bytes of each row, four lanes a row.
     {
         half8 qv[2];
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            const int st = 2 * wave + i;
-            qv[i] = *reinterpret_cast<const half8 *>(a.q + (size_t(min(tok, a.tokens - 1)) * a.heads + head) * DIM + small_dim<BITS>(st, hf));
+            const uint32_t r = 16 * i + (lane >> 2);
+            qv[i] = *reinterpret_cast<const half8 *>(a.q + (size_t(min(tok0 + (r >> 3), a.tokens - 1)) * a.heads + kv * SAETTA_GQA_GROUP + (r & 7)) * DIM + 32 * wave + 8 * (lane & 3));
         }
         if (uint32_t(wave) < active) fetch_values(first + wave);
 #pragma unroll
-        for (int i = 0; i < 2; i++) *reinterpret_cast<half8 *>(lds + L::Q_OFF + (2 * wave + i) * 1024 + lane * 16) = qv[i];
+        for (int i = 0; i < 2; i++) *reinterpret_cast<half8 *>(lds + L::Q_OFF + small_place<BITS>(4 * wave + (lane & 3)) + (16 * i + (lane >> 2)) * 16) = qv[i];
     }
     lds_barrier();
 
@@ -1152,11 +1153,14 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
     }
 
     // ---- the waves' parts joined: wave w finishes dims 32 w .. 32 w + 31 ----
-    const size_t row = size_t(min(tok, a.tokens - 1)) * a.heads + head;
+    // Gates and outputs: lane l has dims 4 (l % 8) .. + 3 of those of rows 8 j + l / 8 (a row group's rows 8 j .. + 7 are a
+    // token's), 128 bytes of a row a load or store.  16 bytes of each of 32 rows, as the accumulators lie, are taken a row a cycle.
     float4 g[4];
+    const uint32_t in_token = (lane >> 3) * DIM + 32 * wave + 4 * (lane & 7);
+    auto first_row = [&](int j) { return size_t(min(tok0 + j, a.tokens - 1)) * a.heads + kv * SAETTA_GQA_GROUP; };
     if constexpr (!SPLIT) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) g[i] = *reinterpret_cast<const float4 *>(a.q_and_gate + row * 2 * DIM + DIM + 32 * wave + 8 * i + 4 * hf);
+        for (int j = 0; j < 4; j++) g[j] = *reinterpret_cast<const float4 *>(a.q_and_gate + first_row(j) * 2 * DIM + DIM + ((lane >> 3) * DIM + in_token));
     }
     lds_barrier();  // every wave is through with its tile and the query operands
     float2 *ml = reinterpret_cast<float2 *>(lds + L::ML_OFF);
@@ -1215,18 +1219,25 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
         if (wave == 0 && hf == 0) *reinterpret_cast<float2 *>(a.part_ml + ((item * 4 + group) * 32 + col) * 2) = float2{top, l_all};
         return;
     }
-    if (tok < a.tokens) {
-        const float inv = 1.0f / l_all;
-        float *out = a.out + row * DIM + 32 * wave + 4 * hf;
+    // Turned round in the place of what the first wave handed to this one, which nobody else reads: piece p (dims 4 p .. + 3) of row
+    // r at 16 ((r + 2 p) % 32) of the piece's 512 bytes, so that neither side meets in its banks.
+    const float inv = 1.0f / l_all;
+    unsigned char *turned = lds + wave * 4096;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float4 w;
-            w.x = fin[4 * i] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].x));
-            w.y = fin[4 * i + 1] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].y));
-            w.z = fin[4 * i + 2] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].z));
-            w.w = fin[4 * i + 3] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-g[i].w));
-            *reinterpret_cast<float4 *>(out + 8 * i) = w;
-        }
+    for (int i = 0; i < 4; i++) {
+        const uint32_t piece = 2 * i + hf;
+        *reinterpret_cast<float4 *>(turned + piece * 512 + (col + 2 * piece) % 32 * 16) = float4{fin[4 * i] * inv, fin[4 * i + 1] * inv, fin[4 * i + 2] * inv, fin[4 * i + 3] * inv};
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t piece = lane & 7;
+        const float4 x = *reinterpret_cast<const float4 *>(turned + piece * 512 + (8 * j + (lane >> 3) + 2 * piece) % 32 * 16);
+        float4 w;
+        w.x = x.x * __builtin_amdgcn_rcpf(1.0f + __expf(-g[j].x));
+        w.y = x.y * __builtin_amdgcn_rcpf(1.0f + __expf(-g[j].y));
+        w.z = x.z * __builtin_amdgcn_rcpf(1.0f + __expf(-g[j].z));
+        w.w = x.w * __builtin_amdgcn_rcpf(1.0f + __expf(-g[j].w));
+        if (tok0 + j < a.tokens) *reinterpret_cast<float4 *>(a.out + first_row(j) * DIM + in_token) = w;
     }
 }
 
