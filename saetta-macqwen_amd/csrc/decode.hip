@@ -470,7 +470,7 @@ __device__ __forceinline__ void new_rows(const PartialArgs &a, const PrepArgs &p
 // TILES: 16-row tiles of query rows (rows * 8 heads, rounded up).  PACKED: one
 // verify row; its 8 heads' hi parts are operand rows 0-7 and lo parts rows 8-15
 // of a single tile.  Otherwise hi and lo are two MFMAs into one accumulator.
-// ITB: blocks per iteration of a workgroup (a multiple of 4: one block per wave and round).
+// ITB: blocks per iteration of a workgroup (a multiple of 4: one block per wave and round), at most (walk).
 template <int BITS, int TILES, bool PACKED, int ITB>
 struct Shape {
     static constexpr int IT_BLOCKS = ITB;
@@ -502,24 +502,11 @@ struct Shape {
 
 template <int BITS, int TILES, bool PACKED, int ITB, bool UNCOND, bool PREP = false>
 __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, const PrepArgs *prep = nullptr, uint32_t new_heads = 8) {
-    using Sh = Shape<BITS, TILES, PACKED, ITB>;
-    constexpr int IT_BLOCKS = ITB, IT_TOKENS = Sh::IT_TOKENS, SC_STRIDE = Sh::SC_STRIDE;
-    constexpr int KROUNDS = ITB / 4, KSTEPS = ITB / 2;
-    constexpr bool QUANT = Sh::QUANT;
-    constexpr int PARTS = Sh::PARTS;
+    constexpr bool QUANT = BITS != 16;
+    constexpr int PARTS = PACKED ? 1 : 2;
     constexpr int RB = row_bytes<BITS>();
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     const int tid = int(threadIdx.x), lane = tid & 63, wave = tid >> 6;
-    half8 *q_lds = reinterpret_cast<half8 *>(lds_raw + Sh::Q_OFF);
-    float *s_lds = reinterpret_cast<float *>(lds_raw + Sh::S_OFF);
-    uint16_t *ks_lds = reinterpret_cast<uint16_t *>(lds_raw + Sh::KS_OFF);
-    uint16_t *kz_lds = reinterpret_cast<uint16_t *>(lds_raw + Sh::KZ_OFF);
-    uint16_t *vs_lds = reinterpret_cast<uint16_t *>(lds_raw + Sh::VS_OFF);
-    uint16_t *vz_lds = reinterpret_cast<uint16_t *>(lds_raw + Sh::VZ_OFF);
-    float *alpha_lds = reinterpret_cast<float *>(lds_raw + Sh::ALPHA_OFF);
-    _Float16 *qz_lds = reinterpret_cast<_Float16 *>(lds_raw + Sh::QZ_OFF);
-    float *zsum_lds = reinterpret_cast<float *>(lds_raw + Sh::ZSUM_OFF);
-
     const int n = lane & 15, j = lane >> 4;
     const uint32_t split = blockIdx.x, kv = blockIdx.y;
     const uint32_t kvh = a.kv_heads;
@@ -592,553 +579,585 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
         blk_end = (split + 1) * nblocks / context_splits;
     }
     const uint32_t range = blk_end - blk_begin;
-    const uint32_t n_it = (range + IT_BLOCKS - 1) / IT_BLOCKS;
-    const uint32_t per_it = (range + n_it - 1) / n_it;
-    const uint32_t n_rounds = n_it;
-    // Four splits in a row start a quarter of their share apart, so that shares of nearly a power of two do not meet in the
-    // same memory channels at every moment (see attention_partial_s_body; f16, one row: 68 against 58 us per layer at 131000
-    // tokens, 39 against 33 at 65500, the same in between).  3 and 4 rows are bound by their matrix instructions.
-    constexpr bool STAGGER = TILES != 2;
-    const uint32_t first_round = STAGGER ? (split & 3) * n_it / 4 : 0;
-    auto place = [&](uint32_t it) { return it + first_round < n_it ? it + first_round : it + first_round - n_it; };
 
-    const uint32_t cap_rows = a.capacity * kvh;
-    const __amdgpu_buffer_rsrc_t k_rsrc = make_rsrc(a.kdata, cap_rows * RB);
-    const __amdgpu_buffer_rsrc_t v_rsrc = make_rsrc(a.vdata, cap_rows * RB);
-    const __amdgpu_buffer_rsrc_t ks_rsrc = make_rsrc(a.kscales, QUANT ? cap_rows * 8 : 0);
-    const __amdgpu_buffer_rsrc_t kz_rsrc = make_rsrc(a.kbiases, QUANT ? cap_rows * 8 : 0);
-    const __amdgpu_buffer_rsrc_t vs_rsrc = make_rsrc(a.vscales, QUANT ? cap_rows * 8 : 0);
-    const __amdgpu_buffer_rsrc_t vz_rsrc = make_rsrc(a.vbiases, QUANT ? cap_rows * 8 : 0);
-    const int tok_stride = int(kvh) * RB;  // bytes between tokens of one kv head
+    // ---- the share in iterations of at most `blocks` blocks, of whose values `value_steps` k-steps are asked for ----
+    // One and two rows ask for all an iteration may need, what it does not need out of range (see load_keys): the compiler then
+    // knows how many loads are in flight at each wait, but each such load still costs its turn, eight of them 0.2 to 0.5 us.  So
+    // the shares of up to 4 and up to 6 blocks have code of their own.  Us a layer, ten layers in a graph, 8192 tokens of capacity
+    // (halves, 8-bit, 4-bit): 1000 tokens (2 blocks) one row 8.9 -> 7.9, 8.5 -> 8.1, 8.6 -> 8.1, two rows 10.1 -> 9.3, 9.6 -> 9.2, 9.7 -> 9.3;
+    // 6000 tokens (6) one row 10.1 -> 9.6, 9.7 -> 9.3, 9.5 -> 9.1, two rows of halves 11.7 -> 11.3 (of codes 11.1 -> 11.3, so they go on
+    // with all four k-steps); from 7 blocks on as before within 1 % (two rows 1.5 %).  Twelve blocks in one iteration, for shares
+    // of 9 to 12, were ahead of two by 0.3 us and took as much from the shares of 7 and 8.
+    auto walk = [&](auto blocks, auto value_steps) __attribute__((always_inline)) {
+        using Sh = Shape<BITS, TILES, PACKED, decltype(blocks)::value>;
+        constexpr int IT_BLOCKS = Sh::IT_BLOCKS, IT_TOKENS = Sh::IT_TOKENS, SC_STRIDE = Sh::SC_STRIDE;
+        constexpr int KROUNDS = IT_BLOCKS / 4, KSTEPS = decltype(value_steps)::value;
+        half8 *q_lds = reinterpret_cast<half8 *>(lds_raw + Sh::Q_OFF);
+        float *s_lds = reinterpret_cast<float *>(lds_raw + Sh::S_OFF);
+        uint16_t *ks_lds = reinterpret_cast<uint16_t *>(lds_raw + Sh::KS_OFF);
+        uint16_t *kz_lds = reinterpret_cast<uint16_t *>(lds_raw + Sh::KZ_OFF);
+        uint16_t *vs_lds = reinterpret_cast<uint16_t *>(lds_raw + Sh::VS_OFF);
+        uint16_t *vz_lds = reinterpret_cast<uint16_t *>(lds_raw + Sh::VZ_OFF);
+        float *alpha_lds = reinterpret_cast<float *>(lds_raw + Sh::ALPHA_OFF);
+        _Float16 *qz_lds = reinterpret_cast<_Float16 *>(lds_raw + Sh::QZ_OFF);
+        float *zsum_lds = reinterpret_cast<float *>(lds_raw + Sh::ZSUM_OFF);
+        const uint32_t n_it = (range + IT_BLOCKS - 1) / IT_BLOCKS;
+        const uint32_t per_it = (range + n_it - 1) / n_it;
+        const uint32_t n_rounds = n_it;
+        // Four splits in a row start a quarter of their share apart, so that shares of nearly a power of two do not meet in the
+        // same memory channels at every moment (see attention_partial_s_body; f16, one row: 68 against 58 us per layer at 131000
+        // tokens, 39 against 33 at 65500, the same in between).  3 and 4 rows are bound by their matrix instructions.
+        constexpr bool STAGGER = TILES != 2;
+        const uint32_t first_round = STAGGER ? (split & 3) * n_it / 4 : 0;
+        auto place = [&](uint32_t it) { return it + first_round < n_it ? it + first_round : it + first_round - n_it; };
 
-    // ---- the loads of one iteration ------------------------------------------------
-    // Everything an iteration reads is requested before anything is computed: keys first
-    // (phase A needs them first), then the small scale/bias rows, then the values.
-    KeyRegs<BITS> kreg[KROUNDS][4];
-    ValRegs<BITS> vreg[KSTEPS];
-    u32x2 ksr = {0, 0}, kzr = {0, 0}, vsr = {0, 0}, vzr = {0, 0};
-    auto blocks_of = [&](uint32_t it) { return it < n_it ? min(per_it, blk_end - (blk_begin + place(it) * per_it)) : 0u; };
-    auto load_keys = [&](uint32_t it) {
-        const uint32_t base = (blk_begin + place(it) * per_it) * BLOCK, nb = blocks_of(it);
-        const int voff = int((base + BLOCK * wave + n) * kvh + kv) * RB + j * key_piece<BITS>();
-#pragma unroll
-        for (int i = 0; i < KROUNDS; i++) {
-            const bool need = uint32_t(wave + 4 * i) < nb;
-            if (UNCOND || need) {
-                const int off = need ? voff : OOB;
-#pragma unroll
-                for (int g = 0; g < 4; g++) kreg[i][g] = load_key<BITS>(k_rsrc, off, i * 64 * tok_stride, g);
-            }
-        }
-    };
-    auto load_scales = [&](uint32_t it) {
-        if constexpr (QUANT) {
-            const uint32_t base = (blk_begin + place(it) * per_it) * BLOCK;
-            const bool need = uint32_t(tid) < blocks_of(it) * BLOCK;
-            if (UNCOND || need) {
-                const int voff = need ? int((base + tid) * kvh + kv) * 8 : OOB;
-                ksr = __builtin_amdgcn_raw_buffer_load_b64(ks_rsrc, voff, 0, 0);
-                kzr = __builtin_amdgcn_raw_buffer_load_b64(kz_rsrc, voff, 0, 0);
-                vsr = __builtin_amdgcn_raw_buffer_load_b64(vs_rsrc, voff, 0, 0);
-                vzr = __builtin_amdgcn_raw_buffer_load_b64(vz_rsrc, voff, 0, 0);
-            }
-        }
-    };
-    auto load_values = [&](uint32_t it) {
-        const uint32_t base = (blk_begin + place(it) * per_it) * BLOCK, ksteps = (blocks_of(it) + 1) / 2;
-        const int voff = int((base + 8 * j) * kvh + kv) * RB + val_lane_offset<BITS>(wave, n);
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ks++) {
-            const bool need = uint32_t(ks) < ksteps;
-            if (UNCOND || need) {
-                const int off = need ? voff : OOB;
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int soff = (32 * ks + e) * tok_stride;
-                    vreg[ks].w[e] = __builtin_amdgcn_raw_buffer_load_b32(v_rsrc, off, soff, 0);
-                    if constexpr (BITS == 16) {
-                        vreg[ks].w[8 + e] = __builtin_amdgcn_raw_buffer_load_b32(v_rsrc, off + 64, soff, 0);
-                    }
-                }
-            }
-        }
-    };
-    // Loads return in order: the scales first, since the barrier that publishes them must not wait for the keys, the values
-    // last.  (One row: left to itself the compiler asked for the values before the keys; with the epilogue's exchanges 8-bit 300
-    // tokens of 8192 8.4 -> 8.0 us a layer, halves 4096 10.0 -> 9.8.  Two rows in this order 8.9 -> 9.0, so they keep the compiler's.)
-    auto in_order = [] {
-        if constexpr (PACKED) __builtin_amdgcn_sched_barrier(0);
-    };
-    load_scales(0), in_order();
-    load_keys(0), in_order();
-    load_values(0), in_order();
+        const uint32_t cap_rows = a.capacity * kvh;
+        const __amdgpu_buffer_rsrc_t k_rsrc = make_rsrc(a.kdata, cap_rows * RB);
+        const __amdgpu_buffer_rsrc_t v_rsrc = make_rsrc(a.vdata, cap_rows * RB);
+        const __amdgpu_buffer_rsrc_t ks_rsrc = make_rsrc(a.kscales, QUANT ? cap_rows * 8 : 0);
+        const __amdgpu_buffer_rsrc_t kz_rsrc = make_rsrc(a.kbiases, QUANT ? cap_rows * 8 : 0);
+        const __amdgpu_buffer_rsrc_t vs_rsrc = make_rsrc(a.vscales, QUANT ? cap_rows * 8 : 0);
+        const __amdgpu_buffer_rsrc_t vz_rsrc = make_rsrc(a.vbiases, QUANT ? cap_rows * 8 : 0);
+        const int tok_stride = int(kvh) * RB;  // bytes between tokens of one kv head
 
-    // ---- prologue: query rows to f16 hi/lo operands in LDS ------------------------
-    // (while the first iteration's keys are in flight; the values are requested after it)
-    if constexpr (PREP) {
-        // the norm (each wave has two of the eight k-steps of a row's dims) and the rotation (dims 0-63: k-steps 0 and 1, the
-        // waves 0 and 1; a pair's values are half a wavefront apart), where the scores will be
-        float *squares = s_lds;                                       // [tile][wave][column]
-        float2 *rope = reinterpret_cast<float2 *>(s_lds + 4 * 4 * 16);  // [row][32]
-#pragma unroll
-        for (int t = 0; t < TILES; t++) {
-            float sum = 0.0f;
-#pragma unroll
-            for (int k = 2 * t; k < 2 * t + 2; k++) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) sum += q_early[k][e] * q_early[k][e];
-            }
-            sum = across_rows<16, 64>(sum, SumOp());
-            if (j == 0) squares[(t * 4 + wave) * 16 + n] = sum;
-        }
-        if (tid < int(32 * a.rows)) {
-            float s, c;
-            rope_angle(position + (tid >> 5), frequency, s, c);
-            rope[tid] = float2{s, c};
-        }
-        __syncthreads();
-#pragma unroll
-        for (int t = 0; t < TILES; t++) {
-            const float *sq = squares + t * 64 + n;
-            const float scale = query_scale((sq[0] + sq[16]) + (sq[32] + sq[48]), prep->p.eps);
-#pragma unroll
-            for (int k = 0; k < 2; k++) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) q_early[2 * t + k][e] *= scale * norm_w[k][e];
-            }
-            if (wave < 2) {
-                const int row = PACKED ? 0 : min(2 * t + (n >> 3), int(a.rows) - 1);
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const float2 sc = rope[row * 32 + 16 * (j & 1) + 8 * wave + e];
-                    const float x = q_early[2 * t][e], other = half_swap(x, j < 2);
-                    q_early[2 * t][e] = j < 2 ? rope_first(x, other, sc.x, sc.y) : rope_second(other, x, sc.x, sc.y);
-                }
-            }
-        }
-    }
-    {
-        const float qmul = a.scale * 1.4426950408889634f * Q_UP;
-#pragma unroll
-        for (int k = 0; k < TILES * 2; k++) {
-            const int item = tid + k * THREADS;
-            const int t = item / 512, step = (item / 64) & 7, l = item & 63;
-            const int on = l & 15;
-            const float (&v)[8] = q_early[k];
-            half8 hi, lo;
-            float sum_hi = 0.0f, sum_lo = 0.0f;
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                _Float16 h, lw;
-                split_hi_lo(v[key_slot_dim<BITS>(e)] * qmul, h, lw);
-                hi[e] = h;
-                lo[e] = lw;
-                sum_hi += (float)h;
-                sum_lo += (float)lw;
-            }
-            float sum;
-            if constexpr (PACKED) {
-                q_lds[step * 64 + l] = (on < 8) ? hi : lo;
-                sum = (on < 8) ? sum_hi : sum_lo;
-            } else {
-                q_lds[((t * 2 + 0) * 8 + step) * 64 + l] = hi;
-                q_lds[((t * 2 + 1) * 8 + step) * 64 + l] = lo;
-                sum = sum_hi + sum_lo;
-            }
-            // The key bias term sum_g z_g * sum_{d in g} q_d is one more MFMA over the same 32
-            // (lane group, slot) pairs: its B operand holds, in lane l and slot `step`, the sum of
-            // the 8 operand values this item made (divided by Q_UP, as hi and lo halves), and its
-            // A operand holds z_g of the step's group.
-            if constexpr (QUANT) {
-                _Float16 h, lw;
-                split_hi_lo(sum * (1.0f / Q_UP), h, lw);
-                qz_lds[((t * 2 + 0) * 64 + l) * 8 + step] = h;
-                qz_lds[((t * 2 + 1) * 64 + l) * 8 + step] = lw;
-            }
-        }
-    }
-    __syncthreads();
-
-    // Query operands of a single tile live in registers for the whole kernel.
-    half8 q_reg[TILES == 1 ? PARTS * 8 : 1];
-    half8 qz_reg[2] = {{0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0, 0, 0}};
-    if constexpr (TILES == 1) {
-#pragma unroll
-        for (int i = 0; i < PARTS * 8; i++) q_reg[i] = q_lds[i * 64 + lane];
-        if constexpr (QUANT) {
-            qz_reg[0] = *reinterpret_cast<const half8 *>(qz_lds + lane * 8);
-            qz_reg[1] = *reinterpret_cast<const half8 *>(qz_lds + (64 + lane) * 8);
-        }
-    }
-
-    // ---- running state -------------------------------------------------------------
-    // Phase B: thread (row, part) of SOFT_ROWS x TPR.
-    const int b_row = tid / Sh::TPR, b_part = tid % Sh::TPR;
-    uint32_t b_len;  // tokens row b_row sees
-    {
-        const int vrow = PACKED ? 0 : b_row >> 3;
-        const bool real = PACKED || b_row < int(real_rows);
-        const uint32_t len = PREP ? max_len : a.decode_len ? kv_len : position + vrow + 1;
-        b_len = real ? min(len, a.capacity) : 0;
-    }
-    float m_run = NO_SCORE, l_part = 0.0f;
-    // Phase C: accumulators of this wave's 64 dims, per tile 4 output tiles of 16 dims.
-    floatx4 acc[TILES][4];
-    float zacc[TILES];
-#pragma unroll
-    for (int t = 0; t < TILES; t++) {
-        zacc[t] = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 4; e++) acc[t][e] = floatx4{0, 0, 0, 0};
-    }
-
-    // What phase B leaves for phase C: P * P_UP; over halves, where no scale goes into it, its hi and lo parts side by side
-    // (every wave takes all rows' P: split here, once, it is two permutes for two values there).
-    constexpr bool P_SPLIT = BITS == 16 && !PACKED;
-    auto p_word = [&](float x) {
-        if constexpr (!P_SPLIT) return x;
-        _Float16 h, lw;
-        split_hi_lo(x, h, lw);
-        return __builtin_bit_cast(float, uint32_t(__builtin_bit_cast(uint16_t, h)) | uint32_t(__builtin_bit_cast(uint16_t, lw)) << 16);
-    };
-    for (uint32_t round = 0; round < n_rounds; round++) {
-        const uint32_t it = round;
-        const uint32_t blk0 = blk_begin + place(it) * per_it;
-        const uint32_t nb = blocks_of(it);  // blocks of this iteration, 0..ITB
-        const uint32_t base = blk0 * BLOCK;
-        const uint32_t it_tokens = nb * BLOCK;
-        const uint32_t ksteps = (nb + 1) / 2;
-
-        // Scales and biases of the iteration's tokens to LDS: thread = token, 4 groups each.  The key
-        // ones before the barrier (phase A reads them); the value ones after it: a wave may still be
-        // reading the previous iteration's in its phase C until every wave has arrived here.
-        if constexpr (QUANT) {
-            if (tid < IT_TOKENS) {
-                *reinterpret_cast<u32x2 *>(ks_lds + 4 * tid) = ksr;
-                *reinterpret_cast<u32x2 *>(kz_lds + 4 * tid) = kzr;
-            }
-        }
-        __syncthreads();  // key scales visible; the previous iteration's phase C is over
-        if constexpr (QUANT) {
-            if (tid < IT_TOKENS) {
-                // Tokens past the context or the iteration get value scale 0 and bias 0, so that
-                // whatever their rows hold stays out of O (their probabilities are 0 as well).
-                if (uint32_t(tid) >= it_tokens || base + tid >= max_len) vsr = u32x2{0, 0}, vzr = u32x2{0, 0};
-                vs_lds[0 * IT_TOKENS + tid] = uint16_t(vsr.x), vs_lds[1 * IT_TOKENS + tid] = uint16_t(vsr.x >> 16);
-                vs_lds[2 * IT_TOKENS + tid] = uint16_t(vsr.y), vs_lds[3 * IT_TOKENS + tid] = uint16_t(vsr.y >> 16);
-                vz_lds[0 * IT_TOKENS + tid] = uint16_t(vzr.x), vz_lds[1 * IT_TOKENS + tid] = uint16_t(vzr.x >> 16);
-                vz_lds[2 * IT_TOKENS + tid] = uint16_t(vzr.y), vz_lds[3 * IT_TOKENS + tid] = uint16_t(vzr.y >> 16);
-            }
-        }
-        // ---- phase A: scores -------------------------------------------------------
-#pragma unroll
-        for (int t = 0; t < TILES; t++) {
-            half8 qt[PARTS * 8];
-            half8 qz[2] = {qz_reg[0], qz_reg[1]};
-            if constexpr (TILES == 1) {
-#pragma unroll
-                for (int i = 0; i < PARTS * 8; i++) qt[i] = q_reg[i];
-            } else {
-#pragma unroll
-                for (int i = 0; i < PARTS * 8; i++) qt[i] = q_lds[(t * PARTS * 8 + i) * 64 + lane];
-                if constexpr (QUANT) {
-                    qz[0] = *reinterpret_cast<const half8 *>(qz_lds + ((t * 2 + 0) * 64 + lane) * 8);
-                    qz[1] = *reinterpret_cast<const half8 *>(qz_lds + ((t * 2 + 1) * 64 + lane) * 8);
-                }
-            }
+        // ---- the loads of one iteration ------------------------------------------------
+        // Everything an iteration reads is requested before anything is computed: keys first
+        // (phase A needs them first), then the small scale/bias rows, then the values.
+        KeyRegs<BITS> kreg[KROUNDS][4];
+        ValRegs<BITS> vreg[KSTEPS];
+        u32x2 ksr = {0, 0}, kzr = {0, 0}, vsr = {0, 0}, vzr = {0, 0};
+        auto blocks_of = [&](uint32_t it) { return it < n_it ? min(per_it, blk_end - (blk_begin + place(it) * per_it)) : 0u; };
+        auto load_keys = [&](uint32_t it) {
+            const uint32_t base = (blk_begin + place(it) * per_it) * BLOCK, nb = blocks_of(it);
+            const int voff = int((base + BLOCK * wave + n) * kvh + kv) * RB + j * key_piece<BITS>();
 #pragma unroll
             for (int i = 0; i < KROUNDS; i++) {
-                const int blk = wave + 4 * i;
-                if (uint32_t(blk) >= nb) break;
-                const int tok0 = BLOCK * blk + 4 * j;  // this lane's 4 tokens in C layout
-                floatx4 s = {0, 0, 0, 0};
-                if constexpr (QUANT) {
-                    // bias term: slot e of every lane group belongs to group e / 2 of token n
-                    const u32x2 zr = *reinterpret_cast<const u32x2 *>(kz_lds + 4 * (BLOCK * blk + n));
-                    const half8 zop = as_half8(perm(0, zr.x, 0x01000100u), perm(0, zr.x, 0x03020302u),
-                                               perm(0, zr.y, 0x01000100u), perm(0, zr.y, 0x03020302u));
-                    s = __builtin_amdgcn_mfma_f32_16x16x32_f16(zop, qz[0], s, 0, 0, 0);
-                    s = __builtin_amdgcn_mfma_f32_16x16x32_f16(zop, qz[1], s, 0, 0, 0);
-                }
-                floatx4 r[4];
+                const bool need = uint32_t(wave + 4 * i) < nb;
+                if (UNCOND || need) {
+                    const int off = need ? voff : OOB;
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    r[g] = floatx4{0, 0, 0, 0};
-#pragma unroll
-                    for (int ab = 0; ab < 2; ab++) {
-                        const half8 kop = key_operand<BITS>(kreg[i][g], ab);
-#pragma unroll
-                        for (int part = 0; part < PARTS; part++) {
-                            r[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop, qt[part * 8 + g * 2 + ab], r[g], 0,
-                                                                          0, 0);
-                        }
-                    }
-                }
-                if constexpr (QUANT) {
-                    // scales of tokens tok0..tok0+3, 4 groups each: 32 contiguous bytes
-                    const u32x4 s01 = *reinterpret_cast<const u32x4 *>(ks_lds + 4 * tok0);
-                    const u32x4 s23 = *reinterpret_cast<const u32x4 *>(ks_lds + 4 * tok0 + 8);
-                    const uint32_t sw[8] = {s01.x, s01.y, s01.z, s01.w, s23.x, s23.y, s23.z, s23.w};
-                    constexpr float C1 = code_up<BITS>() / Q_UP;
-#pragma unroll
-                    for (int tk = 0; tk < 4; tk++) {
-                        float d = 0.0f;
-#pragma unroll
-                        for (int g = 0; g < 4; g++) {
-                            d += half_bits_to_float(sw[2 * tk + (g >> 1)] >> (16 * (g & 1))) * r[g][tk];
-                        }
-                        s[tk] += d * C1;
-                    }
-                } else {
-#pragma unroll
-                    for (int tk = 0; tk < 4; tk++) s[tk] = (r[0][tk] + r[1][tk] + r[2][tk] + r[3][tk]) * (1.0f / Q_UP);
-                }
-                *reinterpret_cast<floatx4 *>(s_lds + (16 * t + n) * SC_STRIDE + tok0) = s;
-            }
-        }
-        // The key registers and the scale registers are free: request the next iteration's.
-        if (it + 1 < n_it) {
-            load_scales(it + 1);
-            load_keys(it + 1);
-        }
-        __syncthreads();
-
-        // ---- phase B: online softmax per row ---------------------------------------
-        // Writes P * P_UP over the scores; l sums the plain P.
-        {
-            // A thread's tokens: TPT in a row, or (three and four tiles, 48 of them) CH in a row of every 32, so that a k-step
-            // without tokens is no work for anyone (8 rows at 300 tokens, 8-bit 23.7 -> 23.1 us a layer; two rows 12.0 -> 12.3).
-            constexpr bool BY_STEP = TILES >= 3;
-            constexpr int CH = BY_STEP ? 32 / Sh::TPR : Sh::TPT, STEP = CH % 4 == 0 ? 4 : 2;
-            static_assert(CH % STEP == 0, "whole pieces");
-            typedef float piece __attribute__((ext_vector_type(STEP)));
-            float sv[Sh::TPT];
-            const bool scores = Sh::SOFT_ROWS == Sh::S_ROWS || PACKED || b_row < Sh::S_ROWS;  // (three tiles: the last wave has no rows)
-            float *row = s_lds + (scores ? b_row : 0) * SC_STRIDE + b_part * CH;
-            const uint32_t tok0 = b_part * CH;
-            // tokens of this row in this iteration: inside the iteration and inside the row's context
-            const uint32_t lim = b_len > base ? min(b_len - base, it_tokens) : 0;
-            auto steps = [&](bool all, auto f) {  // f(index of the thread's value, the token's place in the iteration)
-#pragma unroll
-                for (int i = 0; i < Sh::TPT; i += CH) {
-                    const int at = i / CH * 32;
-                    if (BY_STEP && !all && uint32_t(i / CH) >= ksteps) break;
-#pragma unroll
-                    for (int k = 0; k < CH; k += STEP) f(i + k, at + k);
-                }
-            };
-            float cm = NO_SCORE;
-            steps(true, [&](int i, int at) {
-                piece v = *reinterpret_cast<const piece *>(row + at);
-                if constexpr (PACKED) v += *reinterpret_cast<const piece *>(row + 8 * SC_STRIDE + at);
-#pragma unroll
-                for (int e = 0; e < STEP; e++) {
-                    sv[i + e] = v[e];
-                    cm = (tok0 + at + e < lim) ? fmaxf(cm, v[e]) : cm;
-                }
-            });
-            cm = group_reduce<Sh::TPR>(cm, MaxOp());
-            const float nm = fmaxf(m_run, cm);
-            const float al = __builtin_amdgcn_exp2f(m_run - nm);
-            float sum = 0.0f;
-            steps(false, [&](int i, int at) {
-                piece v;
-#pragma unroll
-                for (int e = 0; e < STEP; e++) {
-                    const float x = (tok0 + at + e < lim) ? __builtin_amdgcn_exp2f(sv[i + e] - nm) : 0.0f;
-                    sum += x;
-                    v[e] = p_word(x * P_UP);
-                }
-                if (scores) *reinterpret_cast<piece *>(row + at) = v;
-            });
-            l_part = l_part * al + sum;
-            m_run = nm;
-            if (scores) {
-                if (b_part == 0) alpha_lds[b_row] = al;
-            }
-        }
-        __syncthreads();
-
-        // ---- phase C: O += P V for this wave's group -------------------------------
-        // The probability operands need only P and the value scales, so they are all built
-        // before the first value code is touched: what is left to do once the (large,
-        // last-requested) value loads land is the byte permutes and the MFMAs.
-        auto build_p = [&](int t, int ks, half8 &phi, half8 &plo) {
-            const float *prow = s_lds + (PACKED ? (n & 7) : 16 * t + n) * SC_STRIDE;
-            const int tk = 32 * ks + 8 * j;
-            const floatx4 p0 = *reinterpret_cast<const floatx4 *>(prow + tk);
-            const floatx4 p1 = *reinterpret_cast<const floatx4 *>(prow + tk + 4);
-            float pv[8] = {p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]};
-            if constexpr (QUANT) {
-                const u32x4 sr = *reinterpret_cast<const u32x4 *>(vs_lds + wave * IT_TOKENS + tk);
-                const u32x4 zr = *reinterpret_cast<const u32x4 *>(vz_lds + wave * IT_TOKENS + tk);
-                const uint32_t sw[4] = {sr.x, sr.y, sr.z, sr.w}, zw[4] = {zr.x, zr.y, zr.z, zr.w};
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    zacc[t] += pv[e] * half_bits_to_float(zw[e >> 1] >> (16 * (e & 1)));
-                    pv[e] *= half_bits_to_float(sw[e >> 1] >> (16 * (e & 1)));
-                }
-            }
-            if constexpr (PACKED) {
-                // hi lanes (n < 8) keep x and let the conversion truncate it to its hi part;
-                // lo lanes subtract the hi part first.
-                const uint32_t lo_mask = (n >= 8) ? 0xffffe000u : 0u;
-                uint32_t o[4];
-#pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    const float x0 = pv[e] - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, pv[e]) & lo_mask);
-                    const float x1 =
-                        pv[e + 1] - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, pv[e + 1]) & lo_mask);
-                    // round toward zero: exact truncation to the hi part in hi lanes
-                    o[e / 2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
-                }
-                phi = as_half8(o[0], o[1], o[2], o[3]);
-            } else if constexpr (P_SPLIT) {
-                uint32_t h[4], lw[4];
-#pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    const uint32_t w0 = __builtin_bit_cast(uint32_t, pv[e]), w1 = __builtin_bit_cast(uint32_t, pv[e + 1]);
-                    h[e / 2] = perm(w1, w0, 0x05040100u), lw[e / 2] = perm(w1, w0, 0x07060302u);
-                }
-                phi = as_half8(h[0], h[1], h[2], h[3]), plo = as_half8(lw[0], lw[1], lw[2], lw[3]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    _Float16 h, lw;
-                    split_hi_lo(pv[e], h, lw);
-                    phi[e] = h;
-                    plo[e] = lw;
+                    for (int g = 0; g < 4; g++) kreg[i][g] = load_key<BITS>(k_rsrc, off, i * 64 * tok_stride, g);
                 }
             }
         };
+        auto load_scales = [&](uint32_t it) {
+            if constexpr (QUANT) {
+                const uint32_t base = (blk_begin + place(it) * per_it) * BLOCK;
+                const bool need = uint32_t(tid) < blocks_of(it) * BLOCK;
+                if (UNCOND || need) {
+                    const int voff = need ? int((base + tid) * kvh + kv) * 8 : OOB;
+                    ksr = __builtin_amdgcn_raw_buffer_load_b64(ks_rsrc, voff, 0, 0);
+                    kzr = __builtin_amdgcn_raw_buffer_load_b64(kz_rsrc, voff, 0, 0);
+                    vsr = __builtin_amdgcn_raw_buffer_load_b64(vs_rsrc, voff, 0, 0);
+                    vzr = __builtin_amdgcn_raw_buffer_load_b64(vz_rsrc, voff, 0, 0);
+                }
+            }
+        };
+        auto load_values = [&](uint32_t it) {
+            const uint32_t base = (blk_begin + place(it) * per_it) * BLOCK, ksteps = (blocks_of(it) + 1) / 2;
+            const int voff = int((base + 8 * j) * kvh + kv) * RB + val_lane_offset<BITS>(wave, n);
+#pragma unroll
+            for (int ks = 0; ks < KSTEPS; ks++) {
+                const bool need = uint32_t(ks) < ksteps;
+                if (UNCOND || need) {
+                    const int off = need ? voff : OOB;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const int soff = (32 * ks + e) * tok_stride;
+                        vreg[ks].w[e] = __builtin_amdgcn_raw_buffer_load_b32(v_rsrc, off, soff, 0);
+                        if constexpr (BITS == 16) {
+                            vreg[ks].w[8 + e] = __builtin_amdgcn_raw_buffer_load_b32(v_rsrc, off + 64, soff, 0);
+                        }
+                    }
+                }
+            }
+        };
+        // Loads return in order: the scales first, since the barrier that publishes them must not wait for the keys, the values
+        // last.  (One row: left to itself the compiler asked for the values before the keys; with the epilogue's exchanges 8-bit 300
+        // tokens of 8192 8.4 -> 8.0 us a layer, halves 4096 10.0 -> 9.8.  Two rows in this order 8.9 -> 9.0, so they keep the compiler's.)
+        auto in_order = [] {
+            if constexpr (PACKED) __builtin_amdgcn_sched_barrier(0);
+        };
+        load_scales(0), in_order();
+        load_keys(0), in_order();
+        load_values(0), in_order();
+
+        // ---- prologue: query rows to f16 hi/lo operands in LDS ------------------------
+        // (while the first iteration's keys are in flight; the values are requested after it)
+        if constexpr (PREP) {
+            // the norm (each wave has two of the eight k-steps of a row's dims) and the rotation (dims 0-63: k-steps 0 and 1, the
+            // waves 0 and 1; a pair's values are half a wavefront apart), where the scores will be
+            float *squares = s_lds;                                       // [tile][wave][column]
+            float2 *rope = reinterpret_cast<float2 *>(s_lds + 4 * 4 * 16);  // [row][32]
+#pragma unroll
+            for (int t = 0; t < TILES; t++) {
+                float sum = 0.0f;
+#pragma unroll
+                for (int k = 2 * t; k < 2 * t + 2; k++) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) sum += q_early[k][e] * q_early[k][e];
+                }
+                sum = across_rows<16, 64>(sum, SumOp());
+                if (j == 0) squares[(t * 4 + wave) * 16 + n] = sum;
+            }
+            if (tid < int(32 * a.rows)) {
+                float s, c;
+                rope_angle(position + (tid >> 5), frequency, s, c);
+                rope[tid] = float2{s, c};
+            }
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < TILES; t++) {
+                const float *sq = squares + t * 64 + n;
+                const float scale = query_scale((sq[0] + sq[16]) + (sq[32] + sq[48]), prep->p.eps);
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) q_early[2 * t + k][e] *= scale * norm_w[k][e];
+                }
+                if (wave < 2) {
+                    const int row = PACKED ? 0 : min(2 * t + (n >> 3), int(a.rows) - 1);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const float2 sc = rope[row * 32 + 16 * (j & 1) + 8 * wave + e];
+                        const float x = q_early[2 * t][e], other = half_swap(x, j < 2);
+                        q_early[2 * t][e] = j < 2 ? rope_first(x, other, sc.x, sc.y) : rope_second(other, x, sc.x, sc.y);
+                    }
+                }
+            }
+        }
+        {
+            const float qmul = a.scale * 1.4426950408889634f * Q_UP;
+#pragma unroll
+            for (int k = 0; k < TILES * 2; k++) {
+                const int item = tid + k * THREADS;
+                const int t = item / 512, step = (item / 64) & 7, l = item & 63;
+                const int on = l & 15;
+                const float (&v)[8] = q_early[k];
+                half8 hi, lo;
+                float sum_hi = 0.0f, sum_lo = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    _Float16 h, lw;
+                    split_hi_lo(v[key_slot_dim<BITS>(e)] * qmul, h, lw);
+                    hi[e] = h;
+                    lo[e] = lw;
+                    sum_hi += (float)h;
+                    sum_lo += (float)lw;
+                }
+                float sum;
+                if constexpr (PACKED) {
+                    q_lds[step * 64 + l] = (on < 8) ? hi : lo;
+                    sum = (on < 8) ? sum_hi : sum_lo;
+                } else {
+                    q_lds[((t * 2 + 0) * 8 + step) * 64 + l] = hi;
+                    q_lds[((t * 2 + 1) * 8 + step) * 64 + l] = lo;
+                    sum = sum_hi + sum_lo;
+                }
+                // The key bias term sum_g z_g * sum_{d in g} q_d is one more MFMA over the same 32
+                // (lane group, slot) pairs: its B operand holds, in lane l and slot `step`, the sum of
+                // the 8 operand values this item made (divided by Q_UP, as hi and lo halves), and its
+                // A operand holds z_g of the step's group.
+                if constexpr (QUANT) {
+                    _Float16 h, lw;
+                    split_hi_lo(sum * (1.0f / Q_UP), h, lw);
+                    qz_lds[((t * 2 + 0) * 64 + l) * 8 + step] = h;
+                    qz_lds[((t * 2 + 1) * 64 + l) * 8 + step] = lw;
+                }
+            }
+        }
+        __syncthreads();
+
+        // Query operands of a single tile live in registers for the whole kernel.
+        half8 q_reg[TILES == 1 ? PARTS * 8 : 1];
+        half8 qz_reg[2] = {{0, 0, 0, 0, 0, 0, 0, 0}, {0, 0, 0, 0, 0, 0, 0, 0}};
+        if constexpr (TILES == 1) {
+#pragma unroll
+            for (int i = 0; i < PARTS * 8; i++) q_reg[i] = q_lds[i * 64 + lane];
+            if constexpr (QUANT) {
+                qz_reg[0] = *reinterpret_cast<const half8 *>(qz_lds + lane * 8);
+                qz_reg[1] = *reinterpret_cast<const half8 *>(qz_lds + (64 + lane) * 8);
+            }
+        }
+
+        // ---- running state -------------------------------------------------------------
+        // Phase B: thread (row, part) of SOFT_ROWS x TPR.
+        const int b_row = tid / Sh::TPR, b_part = tid % Sh::TPR;
+        uint32_t b_len;  // tokens row b_row sees
+        {
+            const int vrow = PACKED ? 0 : b_row >> 3;
+            const bool real = PACKED || b_row < int(real_rows);
+            const uint32_t len = PREP ? max_len : a.decode_len ? kv_len : position + vrow + 1;
+            b_len = real ? min(len, a.capacity) : 0;
+        }
+        float m_run = NO_SCORE, l_part = 0.0f;
+        // Phase C: accumulators of this wave's 64 dims, per tile 4 output tiles of 16 dims.
+        floatx4 acc[TILES][4];
+        float zacc[TILES];
 #pragma unroll
         for (int t = 0; t < TILES; t++) {
-            // Rescale what was summed so far.  Accumulator rows (C layout) are 4j..4j+3.
-            if (round > 0) {
-                const int arow = PACKED ? ((4 * j) & 7) : 16 * t + 4 * j;
-                const floatx4 al = *reinterpret_cast<const floatx4 *>(alpha_lds + arow);
+            zacc[t] = 0.0f;
 #pragma unroll
-                for (int e = 0; e < 4; e++) acc[t][e] *= al;
-                zacc[t] *= alpha_lds[PACKED ? (n & 7) : 16 * t + n];
-            }
-            if constexpr (PACKED) {
-                half8 phi[KSTEPS], plo[KSTEPS];
-#pragma unroll
-                for (int ks = 0; ks < KSTEPS; ks++) {
-                    if (uint32_t(ks) < ksteps) build_p(t, ks, phi[ks], plo[ks]);
+            for (int e = 0; e < 4; e++) acc[t][e] = floatx4{0, 0, 0, 0};
+        }
+
+        // What phase B leaves for phase C: P * P_UP; over halves, where no scale goes into it, its hi and lo parts side by side
+        // (every wave takes all rows' P: split here, once, it is two permutes for two values there).
+        constexpr bool P_SPLIT = BITS == 16 && !PACKED;
+        auto p_word = [&](float x) {
+            if constexpr (!P_SPLIT) return x;
+            _Float16 h, lw;
+            split_hi_lo(x, h, lw);
+            return __builtin_bit_cast(float, uint32_t(__builtin_bit_cast(uint16_t, h)) | uint32_t(__builtin_bit_cast(uint16_t, lw)) << 16);
+        };
+        for (uint32_t round = 0; round < n_rounds; round++) {
+            const uint32_t it = round;
+            const uint32_t blk0 = blk_begin + place(it) * per_it;
+            const uint32_t nb = blocks_of(it);  // blocks of this iteration, 0..ITB
+            const uint32_t base = blk0 * BLOCK;
+            const uint32_t it_tokens = nb * BLOCK;
+            const uint32_t ksteps = (nb + 1) / 2;
+
+            // Scales and biases of the iteration's tokens to LDS: thread = token, 4 groups each.  The key
+            // ones before the barrier (phase A reads them); the value ones after it: a wave may still be
+            // reading the previous iteration's in its phase C until every wave has arrived here.
+            if constexpr (QUANT) {
+                if (tid < IT_TOKENS) {
+                    *reinterpret_cast<u32x2 *>(ks_lds + 4 * tid) = ksr;
+                    *reinterpret_cast<u32x2 *>(kz_lds + 4 * tid) = kzr;
                 }
+            }
+            __syncthreads();  // key scales visible; the previous iteration's phase C is over
+            if constexpr (QUANT) {
+                if (tid < IT_TOKENS) {
+                    // Tokens past the context or the iteration get value scale 0 and bias 0, so that
+                    // whatever their rows hold stays out of O (their probabilities are 0 as well).
+                    if (uint32_t(tid) >= it_tokens || base + tid >= max_len) vsr = u32x2{0, 0}, vzr = u32x2{0, 0};
+                    vs_lds[0 * IT_TOKENS + tid] = uint16_t(vsr.x), vs_lds[1 * IT_TOKENS + tid] = uint16_t(vsr.x >> 16);
+                    vs_lds[2 * IT_TOKENS + tid] = uint16_t(vsr.y), vs_lds[3 * IT_TOKENS + tid] = uint16_t(vsr.y >> 16);
+                    vz_lds[0 * IT_TOKENS + tid] = uint16_t(vzr.x), vz_lds[1 * IT_TOKENS + tid] = uint16_t(vzr.x >> 16);
+                    vz_lds[2 * IT_TOKENS + tid] = uint16_t(vzr.y), vz_lds[3 * IT_TOKENS + tid] = uint16_t(vzr.y >> 16);
+                }
+            }
+            // ---- phase A: scores -------------------------------------------------------
+#pragma unroll
+            for (int t = 0; t < TILES; t++) {
+                half8 qt[PARTS * 8];
+                half8 qz[2] = {qz_reg[0], qz_reg[1]};
+                if constexpr (TILES == 1) {
+#pragma unroll
+                    for (int i = 0; i < PARTS * 8; i++) qt[i] = q_reg[i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < PARTS * 8; i++) qt[i] = q_lds[(t * PARTS * 8 + i) * 64 + lane];
+                    if constexpr (QUANT) {
+                        qz[0] = *reinterpret_cast<const half8 *>(qz_lds + ((t * 2 + 0) * 64 + lane) * 8);
+                        qz[1] = *reinterpret_cast<const half8 *>(qz_lds + ((t * 2 + 1) * 64 + lane) * 8);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < KROUNDS; i++) {
+                    const int blk = wave + 4 * i;
+                    if (uint32_t(blk) >= nb) break;
+                    const int tok0 = BLOCK * blk + 4 * j;  // this lane's 4 tokens in C layout
+                    floatx4 s = {0, 0, 0, 0};
+                    if constexpr (QUANT) {
+                        // bias term: slot e of every lane group belongs to group e / 2 of token n
+                        const u32x2 zr = *reinterpret_cast<const u32x2 *>(kz_lds + 4 * (BLOCK * blk + n));
+                        const half8 zop = as_half8(perm(0, zr.x, 0x01000100u), perm(0, zr.x, 0x03020302u),
+                                                   perm(0, zr.y, 0x01000100u), perm(0, zr.y, 0x03020302u));
+                        s = __builtin_amdgcn_mfma_f32_16x16x32_f16(zop, qz[0], s, 0, 0, 0);
+                        s = __builtin_amdgcn_mfma_f32_16x16x32_f16(zop, qz[1], s, 0, 0, 0);
+                    }
+                    floatx4 r[4];
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        r[g] = floatx4{0, 0, 0, 0};
+#pragma unroll
+                        for (int ab = 0; ab < 2; ab++) {
+                            const half8 kop = key_operand<BITS>(kreg[i][g], ab);
+#pragma unroll
+                            for (int part = 0; part < PARTS; part++) {
+                                r[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop, qt[part * 8 + g * 2 + ab], r[g], 0,
+                                                                              0, 0);
+                            }
+                        }
+                    }
+                    if constexpr (QUANT) {
+                        // scales of tokens tok0..tok0+3, 4 groups each: 32 contiguous bytes
+                        const u32x4 s01 = *reinterpret_cast<const u32x4 *>(ks_lds + 4 * tok0);
+                        const u32x4 s23 = *reinterpret_cast<const u32x4 *>(ks_lds + 4 * tok0 + 8);
+                        const uint32_t sw[8] = {s01.x, s01.y, s01.z, s01.w, s23.x, s23.y, s23.z, s23.w};
+                        constexpr float C1 = code_up<BITS>() / Q_UP;
+#pragma unroll
+                        for (int tk = 0; tk < 4; tk++) {
+                            float d = 0.0f;
+#pragma unroll
+                            for (int g = 0; g < 4; g++) {
+                                d += half_bits_to_float(sw[2 * tk + (g >> 1)] >> (16 * (g & 1))) * r[g][tk];
+                            }
+                            s[tk] += d * C1;
+                        }
+                    } else {
+#pragma unroll
+                        for (int tk = 0; tk < 4; tk++) s[tk] = (r[0][tk] + r[1][tk] + r[2][tk] + r[3][tk]) * (1.0f / Q_UP);
+                    }
+                    *reinterpret_cast<floatx4 *>(s_lds + (16 * t + n) * SC_STRIDE + tok0) = s;
+                }
+            }
+            // The key registers and the scale registers are free: request the next iteration's.
+            if (it + 1 < n_it) {
+                load_scales(it + 1);
+                load_keys(it + 1);
+            }
+            __syncthreads();
+
+            // ---- phase B: online softmax per row ---------------------------------------
+            // Writes P * P_UP over the scores; l sums the plain P.
+            {
+                // A thread's tokens: TPT in a row, or (three and four tiles, 48 of them) CH in a row of every 32, so that a k-step
+                // without tokens is no work for anyone (8 rows at 300 tokens, 8-bit 23.7 -> 23.1 us a layer; two rows 12.0 -> 12.3).
+                constexpr bool BY_STEP = TILES >= 3;
+                constexpr int CH = BY_STEP ? 32 / Sh::TPR : Sh::TPT, STEP = CH % 4 == 0 ? 4 : 2;
+                static_assert(CH % STEP == 0, "whole pieces");
+                typedef float piece __attribute__((ext_vector_type(STEP)));
+                float sv[Sh::TPT];
+                const bool scores = Sh::SOFT_ROWS == Sh::S_ROWS || PACKED || b_row < Sh::S_ROWS;  // (three tiles: the last wave has no rows)
+                float *row = s_lds + (scores ? b_row : 0) * SC_STRIDE + b_part * CH;
+                const uint32_t tok0 = b_part * CH;
+                // tokens of this row in this iteration: inside the iteration and inside the row's context
+                const uint32_t lim = b_len > base ? min(b_len - base, it_tokens) : 0;
+                auto steps = [&](bool all, auto f) {  // f(index of the thread's value, the token's place in the iteration)
+#pragma unroll
+                    for (int i = 0; i < Sh::TPT; i += CH) {
+                        const int at = i / CH * 32;
+                        if (BY_STEP && !all && uint32_t(i / CH) >= ksteps) break;
+#pragma unroll
+                        for (int k = 0; k < CH; k += STEP) f(i + k, at + k);
+                    }
+                };
+                float cm = NO_SCORE;
+                steps(true, [&](int i, int at) {
+                    piece v = *reinterpret_cast<const piece *>(row + at);
+                    if constexpr (PACKED) v += *reinterpret_cast<const piece *>(row + 8 * SC_STRIDE + at);
+#pragma unroll
+                    for (int e = 0; e < STEP; e++) {
+                        sv[i + e] = v[e];
+                        cm = (tok0 + at + e < lim) ? fmaxf(cm, v[e]) : cm;
+                    }
+                });
+                cm = group_reduce<Sh::TPR>(cm, MaxOp());
+                const float nm = fmaxf(m_run, cm);
+                const float al = __builtin_amdgcn_exp2f(m_run - nm);
+                float sum = 0.0f;
+                steps(false, [&](int i, int at) {
+                    piece v;
+#pragma unroll
+                    for (int e = 0; e < STEP; e++) {
+                        const float x = (tok0 + at + e < lim) ? __builtin_amdgcn_exp2f(sv[i + e] - nm) : 0.0f;
+                        sum += x;
+                        v[e] = p_word(x * P_UP);
+                    }
+                    if (scores) *reinterpret_cast<piece *>(row + at) = v;
+                });
+                l_part = l_part * al + sum;
+                m_run = nm;
+                if (scores) {
+                    if (b_part == 0) alpha_lds[b_row] = al;
+                }
+            }
+            __syncthreads();
+
+            // ---- phase C: O += P V for this wave's group -------------------------------
+            // The probability operands need only P and the value scales, so they are all built
+            // before the first value code is touched: what is left to do once the (large,
+            // last-requested) value loads land is the byte permutes and the MFMAs.
+            auto build_p = [&](int t, int ks, half8 &phi, half8 &plo) {
+                const float *prow = s_lds + (PACKED ? (n & 7) : 16 * t + n) * SC_STRIDE;
+                const int tk = 32 * ks + 8 * j;
+                const floatx4 p0 = *reinterpret_cast<const floatx4 *>(prow + tk);
+                const floatx4 p1 = *reinterpret_cast<const floatx4 *>(prow + tk + 4);
+                float pv[8] = {p0[0], p0[1], p0[2], p0[3], p1[0], p1[1], p1[2], p1[3]};
+                if constexpr (QUANT) {
+                    const u32x4 sr = *reinterpret_cast<const u32x4 *>(vs_lds + wave * IT_TOKENS + tk);
+                    const u32x4 zr = *reinterpret_cast<const u32x4 *>(vz_lds + wave * IT_TOKENS + tk);
+                    const uint32_t sw[4] = {sr.x, sr.y, sr.z, sr.w}, zw[4] = {zr.x, zr.y, zr.z, zr.w};
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        zacc[t] += pv[e] * half_bits_to_float(zw[e >> 1] >> (16 * (e & 1)));
+                        pv[e] *= half_bits_to_float(sw[e >> 1] >> (16 * (e & 1)));
+                    }
+                }
+                if constexpr (PACKED) {
+                    // hi lanes (n < 8) keep x and let the conversion truncate it to its hi part;
+                    // lo lanes subtract the hi part first.
+                    const uint32_t lo_mask = (n >= 8) ? 0xffffe000u : 0u;
+                    uint32_t o[4];
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2) {
+                        const float x0 = pv[e] - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, pv[e]) & lo_mask);
+                        const float x1 =
+                            pv[e + 1] - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, pv[e + 1]) & lo_mask);
+                        // round toward zero: exact truncation to the hi part in hi lanes
+                        o[e / 2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
+                    }
+                    phi = as_half8(o[0], o[1], o[2], o[3]);
+                } else if constexpr (P_SPLIT) {
+                    uint32_t h[4], lw[4];
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2) {
+                        const uint32_t w0 = __builtin_bit_cast(uint32_t, pv[e]), w1 = __builtin_bit_cast(uint32_t, pv[e + 1]);
+                        h[e / 2] = perm(w1, w0, 0x05040100u), lw[e / 2] = perm(w1, w0, 0x07060302u);
+                    }
+                    phi = as_half8(h[0], h[1], h[2], h[3]), plo = as_half8(lw[0], lw[1], lw[2], lw[3]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        _Float16 h, lw;
+                        split_hi_lo(pv[e], h, lw);
+                        phi[e] = h;
+                        plo[e] = lw;
+                    }
+                }
+            };
+#pragma unroll
+            for (int t = 0; t < TILES; t++) {
+                // Rescale what was summed so far.  Accumulator rows (C layout) are 4j..4j+3.
+                if (round > 0) {
+                    const int arow = PACKED ? ((4 * j) & 7) : 16 * t + 4 * j;
+                    const floatx4 al = *reinterpret_cast<const floatx4 *>(alpha_lds + arow);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[t][e] *= al;
+                    zacc[t] *= alpha_lds[PACKED ? (n & 7) : 16 * t + n];
+                }
+                if constexpr (PACKED) {
+                    half8 phi[KSTEPS], plo[KSTEPS];
+#pragma unroll
+                    for (int ks = 0; ks < KSTEPS; ks++) {
+                        if (uint32_t(ks) < ksteps) build_p(t, ks, phi[ks], plo[ks]);
+                    }
+#pragma unroll
+                    for (int ks = 0; ks < KSTEPS; ks++) {
+                        if (uint32_t(ks) >= ksteps) break;
+                        if constexpr (BITS == 16) {
+                            // Rows past the context may hold anything, NaN included: 0 * NaN must not reach O.
+#pragma unroll
+                            for (int e = 0; e < 8; e++) {
+                                if (base + 32 * ks + 8 * j + e >= max_len) vreg[ks].w[e] = 0, vreg[ks].w[8 + e] = 0;
+                            }
+                        }
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const half8 vop = val_operand<BITS>(vreg[ks], e, n);
+                            acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(phi[ks], vop, acc[t][e], 0, 0, 0);
+                            if constexpr (!PACKED) {
+                                acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(plo[ks], vop, acc[t][e], 0, 0, 0);
+                            }
+                        }
+                    }
+                }
+            }
+            if constexpr (!PACKED) {
+                // (the k-steps outside: a step's value operands are permuted once for all tiles)
 #pragma unroll
                 for (int ks = 0; ks < KSTEPS; ks++) {
                     if (uint32_t(ks) >= ksteps) break;
                     if constexpr (BITS == 16) {
-                        // Rows past the context may hold anything, NaN included: 0 * NaN must not reach O.
 #pragma unroll
                         for (int e = 0; e < 8; e++) {
                             if (base + 32 * ks + 8 * j + e >= max_len) vreg[ks].w[e] = 0, vreg[ks].w[8 + e] = 0;
                         }
                     }
+                    half8 vop[4];
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const half8 vop = val_operand<BITS>(vreg[ks], e, n);
-                        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(phi[ks], vop, acc[t][e], 0, 0, 0);
-                        if constexpr (!PACKED) {
-                            acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(plo[ks], vop, acc[t][e], 0, 0, 0);
+                    for (int e = 0; e < 4; e++) vop[e] = val_operand<BITS>(vreg[ks], e, n);
+#pragma unroll
+                    for (int t = 0; t < TILES; t++) {
+                        half8 phi, plo;
+                        build_p(t, ks, phi, plo);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(phi, vop[e], acc[t][e], 0, 0, 0);
+                            acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(plo, vop[e], acc[t][e], 0, 0, 0);
                         }
                     }
                 }
             }
+            if (it + 1 < n_it) load_values(it + 1);
         }
-        if constexpr (!PACKED) {
-            // (the k-steps outside: a step's value operands are permuted once for all tiles)
-#pragma unroll
-            for (int ks = 0; ks < KSTEPS; ks++) {
-                if (uint32_t(ks) >= ksteps) break;
-                if constexpr (BITS == 16) {
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        if (base + 32 * ks + 8 * j + e >= max_len) vreg[ks].w[e] = 0, vreg[ks].w[8 + e] = 0;
-                    }
-                }
-                half8 vop[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) vop[e] = val_operand<BITS>(vreg[ks], e, n);
-#pragma unroll
-                for (int t = 0; t < TILES; t++) {
-                    half8 phi, plo;
-                    build_p(t, ks, phi, plo);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(phi, vop[e], acc[t][e], 0, 0, 0);
-                        acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(plo, vop[e], acc[t][e], 0, 0, 0);
-                    }
-                }
-            }
-        }
-        if (it + 1 < n_it) load_values(it + 1);
-    }
 
-    // ---- epilogue: one partial per (row, head) ------------------------------------
-    // m and l from the phase B threads.
-    l_part = group_reduce<Sh::TPR>(l_part, SumOp());
-    if (b_part == 0 && (PACKED || b_row < int(real_rows))) {
-        const int vrow = PACKED ? 0 : b_row >> 3, head = b_row & 7;
-        const size_t slot = (size_t(vrow) * a.nsplits + split) * a.heads + kv * 8 + head;
-        *reinterpret_cast<floatx2 *>(a.part_ml + 2 * slot) = floatx2{m_run, l_part};
-    }
-    // Bias sums: reduce over the 4 lane groups, hand to the C-layout lanes through LDS.
-    if constexpr (QUANT) {
+        // ---- epilogue: one partial per (row, head) ------------------------------------
+        // m and l from the phase B threads.
+        l_part = group_reduce<Sh::TPR>(l_part, SumOp());
+        if (b_part == 0 && (PACKED || b_row < int(real_rows))) {
+            const int vrow = PACKED ? 0 : b_row >> 3, head = b_row & 7;
+            const size_t slot = (size_t(vrow) * a.nsplits + split) * a.heads + kv * 8 + head;
+            *reinterpret_cast<floatx2 *>(a.part_ml + 2 * slot) = floatx2{m_run, l_part};
+        }
+        // Bias sums: reduce over the 4 lane groups, hand to the C-layout lanes through LDS.
+        if constexpr (QUANT) {
+#pragma unroll
+            for (int t = 0; t < TILES; t++) {
+                float z = zacc[t];
+                z = across_rows<16, 64>(z, SumOp());
+                // One copy per wave: the sum of wave w's group lives at [w][row].
+                if (j == 0 && (!PACKED || n < 8)) zsum_lds[wave * Sh::S_ROWS + 16 * t + n] = z;
+            }
+            // written and read by lanes of the same wave: no workgroup barrier
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+        constexpr float unscale = code_up<BITS>() / P_UP;
 #pragma unroll
         for (int t = 0; t < TILES; t++) {
-            float z = zacc[t];
-            z = across_rows<16, 64>(z, SumOp());
-            // One copy per wave: the sum of wave w's group lives at [w][row].
-            if (j == 0 && (!PACKED || n < 8)) zsum_lds[wave * Sh::S_ROWS + 16 * t + n] = z;
-        }
-        // written and read by lanes of the same wave: no workgroup barrier
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
-    constexpr float unscale = code_up<BITS>() / P_UP;
+            // PACKED: rows 8-15 hold the lo part of rows 0-7, lanes j + 2 those of lanes j: the sums of register i end up in the lanes
+            // j = 0, 1 and those of register i + 2 in the lanes 2, 3 (one exchange and one addition for both, and every lane stores).
+            floatx4 o[4];
 #pragma unroll
-    for (int t = 0; t < TILES; t++) {
-        // PACKED: rows 8-15 hold the lo part of rows 0-7, lanes j + 2 those of lanes j: the sums of register i end up in the lanes
-        // j = 0, 1 and those of register i + 2 in the lanes 2, 3 (one exchange and one addition for both, and every lane stores).
-        floatx4 o[4];
+            for (int e = 0; e < 4; e++) {
+                o[e] = acc[t][e];
+                if constexpr (PACKED) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            o[e] = acc[t][e];
-            if constexpr (PACKED) {
+                    for (int i = 0; i < 2; i++) {
+                        // (the builtin: what reads a matrix instruction's result has to be an instruction that the compiler knows)
+                        const float first = o[e][i], third = o[e][i + 2];
+                        const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, first), __builtin_bit_cast(uint32_t, third), false, false);
+                        o[e][i] = __builtin_bit_cast(float, uint32_t(both[0])) + __builtin_bit_cast(float, uint32_t(both[1]));
+                    }
+                }
+            }
 #pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    // (the builtin: what reads a matrix instruction's result has to be an instruction that the compiler knows)
-                    const float first = o[e][i], third = o[e][i + 2];
-                    const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, first), __builtin_bit_cast(uint32_t, third), false, false);
-                    o[e][i] = __builtin_bit_cast(float, uint32_t(both[0])) + __builtin_bit_cast(float, uint32_t(both[1]));
+            for (int i = 0; i < (PACKED ? 2 : 4); i++) {
+                const int pair = PACKED ? 4 * (j & 1) + 2 * (j >> 1) + i : 16 * t + 4 * j + i;  // (row, head) pair of this accumulator row
+                if (!PACKED && pair >= int(real_rows)) continue;
+                const int vrow = PACKED ? 0 : pair >> 3, head = pair & 7;
+                const float zb = QUANT ? zsum_lds[wave * Sh::S_ROWS + pair] * (1.0f / P_UP) : 0.0f;
+                const size_t slot = (size_t(vrow) * a.nsplits + split) * a.heads + kv * 8 + head;
+                float *dst = a.part_o + slot * DIM + 64 * wave;
+                // (Five to eight rows past the caches: up to 17 MB that the L2s would hold dirty until the kernel's end, 27.0 against
+                // 27.7 us a layer for 8 rows at 7000 tokens.  Fewer rows are read back sooner than they are written out: plain.)
+                auto put = [&](float *to, auto value) {
+                    if constexpr (TILES >= 3) __builtin_nontemporal_store(value, reinterpret_cast<decltype(value) *>(to));
+                    else *reinterpret_cast<decltype(value) *>(to) = value;
+                };
+                if constexpr (BITS == 16) {
+                    // tile e: dims 32*(e/2) + 2n + e%2
+                    put(dst + 2 * n, floatx2{o[0][i] * unscale, o[1][i] * unscale});
+                    put(dst + 32 + 2 * n, floatx2{o[2][i] * unscale, o[3][i] * unscale});
+                } else {
+                    put(dst + 4 * n, floatx4{o[0][i] * unscale + zb, o[1][i] * unscale + zb, o[2][i] * unscale + zb, o[3][i] * unscale + zb});
                 }
             }
         }
-#pragma unroll
-        for (int i = 0; i < (PACKED ? 2 : 4); i++) {
-            const int pair = PACKED ? 4 * (j & 1) + 2 * (j >> 1) + i : 16 * t + 4 * j + i;  // (row, head) pair of this accumulator row
-            if (!PACKED && pair >= int(real_rows)) continue;
-            const int vrow = PACKED ? 0 : pair >> 3, head = pair & 7;
-            const float zb = QUANT ? zsum_lds[wave * Sh::S_ROWS + pair] * (1.0f / P_UP) : 0.0f;
-            const size_t slot = (size_t(vrow) * a.nsplits + split) * a.heads + kv * 8 + head;
-            float *dst = a.part_o + slot * DIM + 64 * wave;
-            // (Five to eight rows past the caches: up to 17 MB that the L2s would hold dirty until the kernel's end, 27.0 against
-            // 27.7 us a layer for 8 rows at 7000 tokens.  Fewer rows are read back sooner than they are written out: plain.)
-            auto put = [&](float *to, auto value) {
-                if constexpr (TILES >= 3) __builtin_nontemporal_store(value, reinterpret_cast<decltype(value) *>(to));
-                else *reinterpret_cast<decltype(value) *>(to) = value;
-            };
-            if constexpr (BITS == 16) {
-                // tile e: dims 32*(e/2) + 2n + e%2
-                put(dst + 2 * n, floatx2{o[0][i] * unscale, o[1][i] * unscale});
-                put(dst + 32 + 2 * n, floatx2{o[2][i] * unscale, o[3][i] * unscale});
-            } else {
-                put(dst + 4 * n, floatx4{o[0][i] * unscale + zb, o[1][i] * unscale + zb, o[2][i] * unscale + zb, o[3][i] * unscale + zb});
-            }
-        }
+    };
+    if constexpr (UNCOND) {
+        using std::integral_constant;
+        constexpr bool HAS_3 = PACKED || BITS == 16;
+        if (__builtin_expect(range > (HAS_3 ? 6 : 4), 1)) walk(integral_constant<int, ITB>(), integral_constant<int, ITB / 2>());
+        else if (HAS_3 && range > 4) walk(integral_constant<int, ITB>(), integral_constant<int, HAS_3 ? 3 : ITB / 2>());
+        else walk(integral_constant<int, 4>(), integral_constant<int, 2>());
+    } else {
+        walk(std::integral_constant<int, ITB>(), std::integral_constant<int, ITB / 2>());
     }
 }
 

@@ -353,6 +353,33 @@ def test_three_and_four_tiles_of_query_rows_at_the_edges_of_a_step(kind, m):
         assert worst < MAX_ABS_F64, (tokens, worst)
 
 
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("m", [1, 2])
+def test_one_and_two_rows_at_the_edges_of_a_share(kind, m):
+    # Two splits, shares of 1 to 17 blocks: up to 4 blocks and two k-steps of values, 5 and 6 and three, 7 and more and four, a
+    # second iteration from 9 on; the splits' shares on either side of such a line, rows past the context poisoned.
+    rng = np.random.default_rng(5300 + m)
+    capacity = 640
+    k = rng.standard_normal((capacity, VALUES)).astype(np.float32)
+    v = rng.standard_normal((capacity, VALUES)).astype(np.float32)
+    q = rng.standard_normal((m, H, D)).astype(np.float32)
+    qg = rng.standard_normal((m, H, 2 * D)).astype(np.float32)
+    rows = saetta.AttentionRows(H, KV, capacity, m)
+    rows.splits = 2
+    for tokens in [m, 17, 64, 100, 128, 129, 145, 160, 177, 192, 193, 209, 256, 257, 289, 513, 530]:
+        pos = tokens - m
+        kc, vc, kf, vf = cache_pair(k[:tokens], v[:tokens], kind, capacity, poison=True)
+        out = torch.full((m, H, D), float("nan"), device="cuda")
+        plan = saetta.Plan()
+        params = [saetta.TokenParams(0, pos + r).as_tensor("cuda") for r in range(m)]
+        (rows.record if kind is saetta.KvBits.Half else rows.record_quant)(plan, m, dev(q), kc, vc, dev(qg), out, params)
+        plan.build().run()
+        got = host(out)
+        assert np.isfinite(got).all(), tokens
+        worst = np.abs(got - oracle.rows(q, kf, vf, pos, m, q_and_gate=qg, threads=8, f64=True)).max()
+        assert worst < MAX_ABS_F64, (tokens, worst)
+
+
 @pytest.mark.parametrize("m", [3, 4, 6, 8])
 @pytest.mark.parametrize("step", [0.02, 0.16])
 def test_rows_over_halves_follow_a_growing_maximum(step, m):
