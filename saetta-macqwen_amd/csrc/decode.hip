@@ -81,7 +81,7 @@ constexpr int BLOCK = 16;                     // tokens per MFMA block
 // memory.  With UNCOND, loads that an iteration does not need are issued with it instead of being
 // branched around, so that the number of loads in flight at every wait is known when the kernel is
 // compiled: loads return in order, and a wait whose count is not known has to wait for all of them.
-// (Measured per kernel: it pays for one and two query rows, not for the larger tiles.)
+// (Measured per kernel: it pays for up to four query rows, not for the larger tiles.)
 constexpr int OOB = int(0x80000000u);
 // s_waitcnt operand that waits for the vector memory counter only (gfx9 encoding: vmcnt in bits
 // 3:0 and 15:14, the other counters at their maxima).
@@ -581,13 +581,15 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
     const uint32_t range = blk_end - blk_begin;
 
     // ---- the share in iterations of at most `blocks` blocks, of whose values `value_steps` k-steps are asked for ----
-    // One and two rows ask for all an iteration may need, what it does not need out of range (see load_keys): the compiler then
+    // Up to four rows ask for all an iteration may need, what it does not need out of range (see load_keys): the compiler then
     // knows how many loads are in flight at each wait, but each such load still costs its turn, eight of them 0.2 to 0.5 us.  So
     // the shares of up to 4 and up to 6 blocks have code of their own.  Us a layer, ten layers in a graph, 8192 tokens of capacity
     // (halves, 8-bit, 4-bit): 1000 tokens (2 blocks) one row 8.9 -> 7.9, 8.5 -> 8.1, 8.6 -> 8.1, two rows 10.1 -> 9.3, 9.6 -> 9.2, 9.7 -> 9.3;
     // 6000 tokens (6) one row 10.1 -> 9.6, 9.7 -> 9.3, 9.5 -> 9.1, two rows of halves 11.7 -> 11.3 (of codes 11.1 -> 11.3, so they go on
     // with all four k-steps); from 7 blocks on as before within 1 % (two rows 1.5 %).  Twelve blocks in one iteration, for shares
-    // of 9 to 12, were ahead of two by 0.3 us and took as much from the shares of 7 and 8.
+    // of 9 to 12, were ahead of two by 0.3 us and took as much from the shares of 7 and 8.  Three and four rows, whose iterations are of 12
+    // blocks, have code for up to 4 and up to 8 (3 rows, 8-bit and 4-bit: 1000 tokens 12.9 -> 12.4 and 12.9 -> 12.3, 8000, of 8 blocks, 15.9 ->
+    // 15.1 and 16.0 -> 14.7); from 9 blocks on within 1 %, 2656 tokens of 2688 1.7 %.
     auto walk = [&](auto blocks, auto value_steps) __attribute__((always_inline)) {
         using Sh = Shape<BITS, TILES, PACKED, decltype(blocks)::value>;
         constexpr int IT_BLOCKS = Sh::IT_BLOCKS, IT_TOKENS = Sh::IT_TOKENS, SC_STRIDE = Sh::SC_STRIDE;
@@ -1150,14 +1152,18 @@ __device__ __forceinline__ void attention_partial_body(const PartialArgs &a, con
             }
         }
     };
-    if constexpr (UNCOND) {
-        using std::integral_constant;
+    using std::integral_constant;
+    if constexpr (UNCOND && TILES == 2) {
+        if (range <= 4) walk(integral_constant<int, 4>(), integral_constant<int, 2>());
+        else if (range <= 8) walk(integral_constant<int, 8>(), integral_constant<int, 4>());
+        else walk(integral_constant<int, ITB>(), integral_constant<int, ITB / 2>());
+    } else if constexpr (UNCOND) {
         constexpr bool HAS_3 = PACKED || BITS == 16;
         if (__builtin_expect(range > (HAS_3 ? 6 : 4), 1)) walk(integral_constant<int, ITB>(), integral_constant<int, ITB / 2>());
         else if (HAS_3 && range > 4) walk(integral_constant<int, ITB>(), integral_constant<int, HAS_3 ? 3 : ITB / 2>());
         else walk(integral_constant<int, 4>(), integral_constant<int, 2>());
     } else {
-        walk(std::integral_constant<int, ITB>(), std::integral_constant<int, ITB / 2>());
+        walk(integral_constant<int, ITB>(), integral_constant<int, ITB / 2>());
     }
 }
 
@@ -1178,7 +1184,7 @@ __global__ __launch_bounds__(THREADS, 2) void attention_partial_kernel_1(Partial
 
 template <int BITS, int TILES>
 __global__ __launch_bounds__(THREADS) void attention_partial_kernel_n(PartialArgs a) {
-    attention_partial_body<BITS, TILES, false, itb_rows<TILES>(), TILES == 1>(a);
+    attention_partial_body<BITS, TILES, false, itb_rows<TILES>(), TILES <= 2>(a);
 }
 
 template <int BITS>
@@ -1189,7 +1195,7 @@ __global__ __launch_bounds__(THREADS) void attention_partial_kernel_p(PartialArg
 // The same with the step before the scores taken in.
 template <int BITS, int TILES>
 __global__ __launch_bounds__(THREADS) void attention_token_kernel_n(TokenArgs t) {
-    attention_partial_body<BITS, TILES, false, itb_rows<TILES>(), TILES == 1, true>(t.a, &t.prep, t.new_heads);
+    attention_partial_body<BITS, TILES, false, itb_rows<TILES>(), TILES <= 2, true>(t.a, &t.prep, t.new_heads);
 }
 template <int BITS>
 __global__ __launch_bounds__(THREADS) void attention_token_kernel_p(TokenArgs t) {

@@ -354,10 +354,11 @@ def test_three_and_four_tiles_of_query_rows_at_the_edges_of_a_step(kind, m):
 
 
 @pytest.mark.parametrize("kind", KINDS)
-@pytest.mark.parametrize("m", [1, 2])
-def test_one_and_two_rows_at_the_edges_of_a_share(kind, m):
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+def test_up_to_four_rows_at_the_edges_of_a_share(kind, m):
     # Two splits, shares of 1 to 17 blocks: up to 4 blocks and two k-steps of values, 5 and 6 and three, 7 and more and four, a
-    # second iteration from 9 on; the splits' shares on either side of such a line, rows past the context poisoned.
+    # second iteration from 9 on (three and four rows: iterations of 12); the splits' shares on either side of such a line,
+    # rows past the context poisoned.
     rng = np.random.default_rng(5300 + m)
     capacity = 640
     k = rng.standard_normal((capacity, VALUES)).astype(np.float32)
@@ -366,7 +367,7 @@ def test_one_and_two_rows_at_the_edges_of_a_share(kind, m):
     qg = rng.standard_normal((m, H, 2 * D)).astype(np.float32)
     rows = saetta.AttentionRows(H, KV, capacity, m)
     rows.splits = 2
-    for tokens in [m, 17, 64, 100, 128, 129, 145, 160, 177, 192, 193, 209, 256, 257, 289, 513, 530]:
+    for tokens in [m, 17, 64, 100, 128, 129, 145, 160, 177, 192, 193, 209, 256, 257, 289, 385, 513, 530]:
         pos = tokens - m
         kc, vc, kf, vf = cache_pair(k[:tokens], v[:tokens], kind, capacity, poison=True)
         out = torch.full((m, H, D), float("nan"), device="cuda")
