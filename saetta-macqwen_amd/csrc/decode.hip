@@ -1176,6 +1176,11 @@ template <int TILES>
 constexpr int itb_rows() {
     return TILES == 1 ? 8 : 12;
 }
+// UNCOND of each kernel (three and four rows over halves come to theirs with SAETTA_STAGE_NO_LOADERS only, and stay as they were)
+template <int BITS, int TILES>
+constexpr bool all_asked() {
+    return TILES == 1 || (TILES == 2 && BITS != 16);
+}
 
 template <int BITS>
 __global__ __launch_bounds__(THREADS, 2) void attention_partial_kernel_1(PartialArgs a) {
@@ -1184,7 +1189,7 @@ __global__ __launch_bounds__(THREADS, 2) void attention_partial_kernel_1(Partial
 
 template <int BITS, int TILES>
 __global__ __launch_bounds__(THREADS) void attention_partial_kernel_n(PartialArgs a) {
-    attention_partial_body<BITS, TILES, false, itb_rows<TILES>(), TILES <= 2>(a);
+    attention_partial_body<BITS, TILES, false, itb_rows<TILES>(), all_asked<BITS, TILES>()>(a);
 }
 
 template <int BITS>
@@ -1195,7 +1200,7 @@ __global__ __launch_bounds__(THREADS) void attention_partial_kernel_p(PartialArg
 // The same with the step before the scores taken in.
 template <int BITS, int TILES>
 __global__ __launch_bounds__(THREADS) void attention_token_kernel_n(TokenArgs t) {
-    attention_partial_body<BITS, TILES, false, itb_rows<TILES>(), TILES <= 2, true>(t.a, &t.prep, t.new_heads);
+    attention_partial_body<BITS, TILES, false, itb_rows<TILES>(), all_asked<BITS, TILES>(), true>(t.a, &t.prep, t.new_heads);
 }
 template <int BITS>
 __global__ __launch_bounds__(THREADS) void attention_token_kernel_p(TokenArgs t) {
