@@ -28,15 +28,17 @@ __device__ __forceinline__ void fast_gates(float a_plus_bias, float exp_a_log, f
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
 // x / (1 + e^-x): the exponent as a product and what its rounding leaves out, the hardware's exp2, and the quotient by the
 // hardware's reciprocal and one step on what the product with it leaves of x (no further off than expf and a division, on the
-// average nearer; zero where 1 + e^-x is beyond 2^126).  The library's two, thirty instructions in a row, stood twice on the path
-// of a DeltaNet token's one launch.
+// average nearer; zero where e^-x is beyond f32).  From e^-x = 2^64 on the divisor is taken 2^64 smaller and the quotient by as much
+// too large, for from 2^126 on the hardware's reciprocal is zero.  The library's two calls, thirty instructions in a row, stood
+// twice on the path of a DeltaNet token's one launch.
 __device__ __forceinline__ float silu_f(float x) {
     constexpr float LOG2_E = 0x1.715476p+0f, LOG2_E_REST = 0x1.4ae0cp-26f, LN_2 = 0x1.62e43p-1f;
-    const float at = -LOG2_E * x, near = __builtin_amdgcn_fmed3f(x, -128.0f, 128.0f);  // (infinities: no rest)
-    const float rest = fmaf(-LOG2_E_REST, near, fmaf(-LOG2_E, near, LOG2_E * near));
-    const float e = __builtin_amdgcn_exp2f(at), d = 1.0f + fmaf(e, LN_2 * rest, e), r = at > 126.0f ? 0.0f : __builtin_amdgcn_rcpf(d);
-    const float y = x * r, off = fmaf(-d, y, x);
-    return at > 126.0f || !(off == off) ? y : fmaf(off, r, y);
+    const float at = -LOG2_E * x, rest = fmaf(-LOG2_E_REST, x, fmaf(-LOG2_E, x, LOG2_E * x));
+    // (where e^-x is zero or infinite no rest, but not zero, which times an infinity is NaN)
+    const float tail = fabsf(at) < 128.0f ? LN_2 * rest : 0x1p-64f, down = at > 64.0f ? 0x1p-64f : 1.0f;
+    const float e = __builtin_amdgcn_exp2f(at), d = fmaf(fmaf(e, tail, e), down, down), r = __builtin_amdgcn_rcpf(d);
+    const float y = x * r, off = fmaf(-d, y, x), y_down = y * down;
+    return off == off ? fmaf(off, r * down, y_down) : y_down;
 }
 
 }  // namespace saetta

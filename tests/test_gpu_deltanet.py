@@ -136,8 +136,8 @@ def test_token_call_matches_conv_then_step(k_heads, v_heads, v_dim, kernel):
 
 
 def test_activation_over_the_whole_range():
-    # the conv with a last tap of one is its activation, x / (1 + e^-x): two ulps of f32 wherever the result is a normal
-    # number, zero below 2^-119, where e^-x nears the end of f32, and the limits
+    # the conv with a last tap of one is its activation, x / (1 + e^-x): two ulps of f32 (below 2^-119 see the next test), and the
+    # limits
     x = np.concatenate([np.linspace(-100, 100, 2001), -np.logspace(-30, 2, 500), np.logspace(-30, 38, 500), [0.0, -87.0, -88.0, -89.0, -1e30]]).astype(np.float32)
     special = np.array([np.inf, -np.inf, np.nan], np.float32)
     xs = np.concatenate([x, special])
@@ -152,3 +152,20 @@ def test_activation_over_the_whole_range():
         want = x64 / (1 + np.exp(-x64))
     assert (np.abs(got[:x.size] - want) <= 2.4e-7 * np.abs(want) + 2.0 ** -119).all()
     assert got[-3] == np.inf and np.isnan(got[-1]) and not got[-2] > 0
+
+
+def test_activation_down_to_the_end_of_its_exponential():
+    # up to where e^-x leaves f32 (x = -88.7228) two ulps, whatever its reciprocal; zero or the number it is from there on
+    x = -np.concatenate([np.linspace(44, 130, 8001), [44.361419, 87.336544, 88.02969, 88.7227, 103.97208, 1e3, 1e30, 3.4e38]]).astype(np.float32)
+    w = np.zeros((x.size, 4), np.float32)
+    w[:, 3] = 1
+    state, out = torch.zeros(3, x.size, device="cuda"), torch.empty(x.size, device="cuda")
+    plan = saetta.Plan()
+    saetta.deltanet_conv(plan, dev(x), dev(w), state, out, x.size, 4)
+    plan.build().run()
+    x64 = x.astype(np.float64)
+    with np.errstate(over="ignore"):
+        want = x64 / (1 + np.exp(-x64))
+    allowed = np.where(x64 > -88.7228, 2.4e-7, 1.0) * np.abs(want) + 2.0 ** -149
+    worst = (np.abs(host(out) - want) - allowed).argmax()
+    assert abs(host(out)[worst] - want[worst]) <= allowed[worst], (x[worst], host(out)[worst], want[worst])
