@@ -53,7 +53,9 @@ __global__ __launch_bounds__(256) void attention_prep_store_kernel(PrepArgs a) {
         if (i < 2 * half) {
             const uint32_t r = i < half ? i : i - half;
             float s, c;
-            rope_angle(position, rope_frequency(r, half, a.p.log2_theta), s, c);
+            const double frequency = rope_frequency(r, half, a.p.log2_theta);
+            if (a.p.log2_theta >= 0.0f) rope_angle(position, frequency, s, c);
+            else library_angle(position, frequency, s, c);
             const float u = head[r], w = head[r + half];
             x = i < half ? rope_first(u, w, s, c) : rope_second(u, w, s, c);
         }

@@ -44,9 +44,10 @@ __device__ __forceinline__ float query_scale(float total, float eps) { return in
 // sin() and cos() of the library, one after the other, stood in front of a token step's first scores (their code holds a
 // reduction for any argument, twice).  Here the angle is reduced once: n quarter turns off it with pi / 2 as the sum of two
 // doubles, fma by fma.  The first difference is exact (a multiple of the angle's or pi / 2's last place, below 2), so what is
-// left is good to an ulp or so of f64 for angles up to 2^50; then the series of both to where the next term is below 2^-53 at
-// pi / 4, rounded to f32.  A layer's token step, us, with the norm below, ten layers in a graph: 8-bit 300 tokens of 8192
-// 8.6 -> 8.4, 6000 10.2 -> 9.7, halves 20000 of 32768 16.3 -> 15.8, four rows over 4-bit codes at 1000 tokens 14.0 -> 13.2.
+// left is good to an ulp or so of f64 for angles up to 2^50 (frequencies of at most 1, a theta from 1 on, give angles below 2^32; any
+// other theta takes library_angle); then the series of both to where the next term is below 2^-53 at pi / 4, rounded to f32.
+// A layer's token step, us, with the norm below, ten layers in a graph: 8-bit 300 tokens of 8192 8.6 -> 8.4, 6000
+// 10.2 -> 9.7, halves 20000 of 32768 16.3 -> 15.8, four rows over 4-bit codes at 1000 tokens 14.0 -> 13.2.
 __device__ __forceinline__ double rope_frequency(uint32_t r, uint32_t half_dims, float log2_theta) {
     return exp2(-double(r) / double(half_dims) * double(log2_theta));
 }
@@ -65,6 +66,11 @@ __device__ __forceinline__ void rope_angle(uint32_t position, double frequency, 
     const int quarter = int(n - 4.0 * floor(0.25 * n));
     const float fs = float(sine), fc = float(cosine), s0 = quarter & 1 ? fc : fs, c0 = quarter & 1 ? fs : fc;
     s = quarter & 2 ? -s0 : s0, c = (quarter + 1) & 2 ? -c0 : c0;
+}
+// The same for any frequency.
+__device__ __forceinline__ void library_angle(uint32_t position, double frequency, float &s, float &c) {
+    const double angle = double(position) * frequency;
+    s = float(sin(angle)), c = float(cos(angle));
 }
 // Values u (index r) and w (index r + half) of a pair: the rotated first and second (one product rounded, the other fused).
 __device__ __forceinline__ float rope_first(float u, float w, float s, float c) { return fmaf(u, c, -__fmul_rn(w, s)); }

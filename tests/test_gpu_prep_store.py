@@ -131,6 +131,27 @@ def test_angles_of_any_position():
     assert same > 0.9999 * total
 
 
+@pytest.mark.parametrize("log2_theta", [-16, -32, -64])
+def test_angles_beyond_2_to_32(log2_theta):
+    # a theta below 1, with frequencies of up to 2^15.5, 2^31 and 2^62: sines and cosines of the angles as f64 holds them
+    ones, keys = torch.ones(D, device="cuda"), make_cache(saetta.KvBits.Half, 16)
+    k, qg = torch.ones(8 * KV * D, device="cuda"), torch.ones(8 * H * 2 * D, device="cuda")
+    q_out, k_back = torch.empty(8 * H * D, device="cuda"), torch.empty(8, KV, D, device="cuda")
+    plan = saetta.Plan()
+    saetta.record_store(plan, qg, k, k, ones, ones, q_out, *keys, saetta.PrepParams(H, KV, D, ROPE_DIMS, 2.0 ** log2_theta, EPS), 16, rows=8, k_back=k_back)
+    built = plan.build()
+    even = slice(0, 32, 2 if log2_theta == -16 else 1)  # (frequencies that are whole powers of two)
+    for pos in [0, 1, 2, 355, 4096, 103993, 262136, 2 ** 30 + 1, 2 ** 31 + 12345, 2 ** 32 - 9]:
+        plan.set_params(saetta.TokenParams(0, pos))
+        built.run()
+        got = host(k_back)[:, 0]
+        x = got[:, ROPE_DIMS:ROPE_DIMS + 1].astype(np.float64)
+        angle = (pos + np.arange(8, dtype=np.float64))[:, None] * np.exp2(-np.arange(32.0) / 32 * log2_theta)
+        s, c = np.sin(angle), np.cos(angle)
+        off = np.abs(got[:, :64] - np.concatenate([x * c - x * s, x * s + x * c], 1)).reshape(8, 2, 32)[:, :, even]
+        assert off.max() <= 3e-7, pos  # (an ulp of the products and of the result)
+
+
 @pytest.mark.parametrize("kind", [saetta.KvBits.Eight, saetta.KvBits.Half])
 def test_verify_rows_and_decode_after_store(kind):
     # m rows at positions pos..pos+m-1 in one launch, then attention over the cache it wrote:

@@ -14,7 +14,7 @@ PREP = saetta.PrepParams(H, KV, D, 64, 1e7, 1e-6)
 
 
 class Step:
-    def __init__(self, kind, capacity, rows, seed, rope_dims=64, lay=lambda step: None):
+    def __init__(self, kind, capacity, rows, seed, rope_dims=64, lay=lambda step: None, theta=1e7):
         rng = np.random.default_rng(seed)
         self.rows, self.kind = rows, kind
         self.qg = dev(rng.standard_normal((rows, H, 2 * D)).astype(np.float32))
@@ -34,7 +34,7 @@ class Step:
         lay(self)  # (buffers over others)
         self.k.copy_(self.k0), self.v.copy_(self.v0)
         self.plan = saetta.Plan()
-        saetta.record_store(self.plan, self.qg, self.k, self.v, qn, kn, self.q, keys, values, saetta.PrepParams(H, KV, D, rope_dims, 1e7, 1e-6),
+        saetta.record_store(self.plan, self.qg, self.k, self.v, qn, kn, self.q, keys, values, saetta.PrepParams(H, KV, D, rope_dims, theta, 1e-6),
                             self.cache.capacity, rows=rows, k_back=self.back)
         if rows == 1:
             (self.cache.decode.record if kind is saetta.KvBits.Half else self.cache.decode.record_quant)(
@@ -173,6 +173,20 @@ def test_scratch_laid_over_what_is_done_with(kind, capacity, rows, lay):
     # The context's workgroups write partials while the new rows' workgroups still read k and v.
     step = Step(kind, capacity, rows, seed=capacity + 5 * rows + kind.value, lay=lay)
     check_laid_over(step, (100, step.cache.capacity - rows))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("rows", [1, 3])
+def test_a_theta_below_one_keeps_its_launches(kind, rows):
+    # angles of up to 2^31 times the position: the step that takes the store in is written for frequencies of at most 1
+    step = Step(kind, 8192, rows, seed=rows, theta=2.0 ** -32)
+    assert launches(step) == 3
+    built = step.plan.build()
+    for position in (0, 5, 3001, 8192 - rows):
+        want, got = step.run(step.plan.run_serial, position), step.run(built.run, position)
+        assert np.isfinite(want[0]).all() and np.abs(want[1]).max() < 20  # (a rotation keeps the norm)
+        for a, b in zip(got, want):
+            assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), position
 
 
 def test_other_steps_keep_their_launches():
