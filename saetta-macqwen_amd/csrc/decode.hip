@@ -3131,9 +3131,10 @@ void launch_partial_rows(hipStream_t stream, const PartialArgs &a, bool one_per_
 
 // Whether the last two launches of a plan in the making are the step before the scores and the partial stage `a` of the
 // same rows over the same buffers, so that the reduce stage about to be recorded makes them one layer's token step, which
-// the kernels of TokenArgs do in one launch less.  They are written for 64 rotary dims and rope_angle's frequencies, and the new
-// tokens take a split of their own: with fewer than 4 the context would be left with too few workgroups.  (The branch to the
-// library's sine and cosine inside them was 1 to 1.6 % of a step at 32768 tokens of 8 bits, taken or not.)
+// the kernels of TokenArgs do in one launch less.  They are written for 64 rotary dims and for what rope_angle and
+// inverse_root take, and the new tokens take a split of their own: with fewer than 4 the context would be left with too few
+// workgroups.  (The branch to the library's sine and cosine inside them was 1 to 1.6 % of a step at 32768 tokens of 8 bits,
+// taken or not.)
 bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const float *q_and_gate, bool keys_first, TokenArgs &token) {
     const size_t n = list.launches.size();
     if (n < 2 || a.nsplits < 4) return false;
@@ -3148,7 +3149,8 @@ bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const fl
                                   : prep.kq.data == a.kdata && prep.kq.scales == a.kscales && prep.kq.biases == a.kbiases && prep.vq.data == a.vdata &&
                                         prep.vq.scales == a.vscales && prep.vq.biases == a.vbiases;
     if (!(cache && prep.q_out == a.q && prep.q_and_gate == q_and_gate && prep.tp == a.tp && prep.capacity == a.capacity && prep.p.heads == a.heads &&
-          prep.p.kv_heads == a.kv_heads && prep.p.half_dims == 32 && prep.p.log2_theta >= 0.0f && aligned(prep.q_and_gate, 16) && aligned(prep.q_norm, 16))) return false;
+          prep.p.kv_heads == a.kv_heads && prep.p.half_dims == 32 && prep.p.log2_theta >= 0.0f && prep.p.eps >= INVERSE_ROOT_FROM &&
+          aligned(prep.q_and_gate, 16) && aligned(prep.q_norm, 16))) return false;
     // One launch only where its buffers lie apart.  In three, the step's inputs are done with when the store has run, so a
     // program may write the key back in the place of `k` (the reference's in-place key) or lay the partials over any of
     // them; in one, workgroups still read the inputs while others write.

@@ -948,7 +948,7 @@ void launch_head_rows(const SmallRowsArgs &args, uint32_t *sync, hipStream_t str
 
 void launch_small_rows(const SmallRowsArgs &args, uint32_t *sync, hipStream_t stream) {
     const saetta_rows_fused_params &p = args.p;
-    if (sync && p.v_dim == HEAD_V_DIM && p.kernel_size == HEAD_TAPS && aligned(args.w, 16) && p.v_heads / p.k_heads < 65536) {
+    if (sync && p.v_dim == HEAD_V_DIM && p.kernel_size == HEAD_TAPS && aligned(args.w, 16) && p.v_heads / p.k_heads < 65536 && p.eps >= INVERSE_ROOT_FROM) {
         launch_head_rows<1>(args, sync, stream);
         return;
     }

@@ -52,7 +52,10 @@ __device__ __forceinline__ float group_reduce(float x, Op op) {
 }
 
 // 1 / sqrt(x): the hardware's, an ulp off, and one Newton step (as near as the root and the division rounded one after the
-// other, which are thirty instructions).  0 and infinity, where the step has no value, as they are.
+// other, which are thirty instructions).  0 and infinity, where the step has no value, as they are; not for numbers below
+// INVERSE_ROOT_FROM, whose root the hardware takes for that of 0: the eps under a norm's root keeps those away, and who takes
+// a smaller eps goes by kernels without this.
+constexpr float INVERSE_ROOT_FROM = 0x1p-126f;
 __device__ __forceinline__ float inverse_root(float x) {
     const float y = __builtin_amdgcn_rsqf(x), off = fmaf(-x * y, y, 1.0f);
     return off == off ? fmaf(0.5f * y, off, y) : y;

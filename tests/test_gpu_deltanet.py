@@ -135,6 +135,43 @@ def test_token_call_matches_conv_then_step(k_heads, v_heads, v_dim, kernel):
         assert np.abs(host(state_gpu) - state_cpu).max() <= 2e-5 * max(1.0, np.abs(state_cpu).max()), t
 
 
+@pytest.mark.parametrize("rows", [1, 4])
+def test_norm_of_outputs_whose_mean_square_is_below_the_normal_numbers(rows):
+    # values of 1e-18 and no eps: outputs whose mean square is 1e-42 to 1e-38, which the hardware's reciprocal root takes for 0;
+    # against the same in 64 bits, to half a step of 2^-149 of the 128 squares and of their mean
+    rng = np.random.default_rng(rows)
+    k_heads, v_heads, v_dim = 2, 4, 128
+    key, val = k_heads * K_DIM, v_heads * v_dim
+    x = rng.standard_normal((rows, 2 * key + val)).astype(np.float32)
+    x[:, 2 * key:] *= 5e-18
+    z, a, b = (rng.standard_normal((rows, n)).astype(np.float32) for n in (val, v_heads, v_heads))
+    a_log, dt_bias, norm = rng.uniform(-1, 1, v_heads).astype(np.float32), rng.standard_normal(v_heads).astype(np.float32), np.ones(v_dim, np.float32)
+    w = np.zeros((x.shape[1], 4), np.float32)
+    w[:, 3] = 1
+    conv, state, y = torch.zeros(3, x.shape[1], device="cuda"), torch.zeros(val * K_DIM, device="cuda"), torch.empty(rows, val, device="cuda")
+    buffers = (dev(x), dev(w), conv, dev(a), dev(b), dev(a_log), dev(dt_bias), state, dev(z), dev(norm), y)
+    plan = saetta.Plan()
+    if rows == 1:
+        saetta.deltanet_token(plan, *buffers, k_heads, v_heads, v_dim, 4, 0.0)
+    else:
+        saetta.deltanet_rows_fused(plan, *buffers, k_heads, v_heads, v_dim, 4, rows, 0.0)
+    plan.build().run()
+    sigmoid = lambda u: 1 / (1 + np.exp(-u.astype(np.float64)))  # noqa: E731
+    m, s = x * sigmoid(x), np.zeros((v_heads, v_dim, K_DIM))
+    for t in range(rows):
+        for h in range(v_heads):
+            q, k = (m[t, o + h // 2 * K_DIM:o + (h // 2 + 1) * K_DIM] for o in (0, key))
+            q, k = q / np.linalg.norm(q) / np.sqrt(K_DIM), k / np.linalg.norm(k)
+            g = np.exp(-np.exp(np.float64(a_log[h])) * np.logaddexp(0, np.float64(a[t, h]) + dt_bias[h]))
+            v = m[t, 2 * key + h * v_dim:2 * key + (h + 1) * v_dim]
+            s[h] = g * s[h]
+            s[h] += np.outer((v - s[h] @ k) * sigmoid(b[t, h:h + 1]), k)
+            o = s[h] @ q
+            want = o / np.sqrt(np.mean(o * o)) * z[t, h * v_dim:(h + 1) * v_dim] * sigmoid(z[t, h * v_dim:(h + 1) * v_dim])
+            got = host(y)[t, h * v_dim:(h + 1) * v_dim]
+            assert np.mean(o * o) < 2.0 ** -120 and np.abs(got - want).max() < (1e-5 + 2.0 ** -149 / np.mean(o * o)) * np.abs(want).max(), (t, h)
+
+
 def test_activation_over_the_whole_range():
     # the conv with a last tap of one is its activation, x / (1 + e^-x): two ulps of f32 (below 2^-119 see the next test), and the
     # limits

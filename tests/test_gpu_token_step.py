@@ -14,7 +14,7 @@ PREP = saetta.PrepParams(H, KV, D, 64, 1e7, 1e-6)
 
 
 class Step:
-    def __init__(self, kind, capacity, rows, seed, rope_dims=64, lay=lambda step: None, theta=1e7):
+    def __init__(self, kind, capacity, rows, seed, rope_dims=64, lay=lambda step: None, theta=1e7, eps=1e-6):
         rng = np.random.default_rng(seed)
         self.rows, self.kind = rows, kind
         self.qg = dev(rng.standard_normal((rows, H, 2 * D)).astype(np.float32))
@@ -34,7 +34,7 @@ class Step:
         lay(self)  # (buffers over others)
         self.k.copy_(self.k0), self.v.copy_(self.v0)
         self.plan = saetta.Plan()
-        saetta.record_store(self.plan, self.qg, self.k, self.v, qn, kn, self.q, keys, values, saetta.PrepParams(H, KV, D, rope_dims, theta, 1e-6),
+        saetta.record_store(self.plan, self.qg, self.k, self.v, qn, kn, self.q, keys, values, saetta.PrepParams(H, KV, D, rope_dims, theta, eps),
                             self.cache.capacity, rows=rows, k_back=self.back)
         if rows == 1:
             (self.cache.decode.record if kind is saetta.KvBits.Half else self.cache.decode.record_quant)(
@@ -187,6 +187,19 @@ def test_a_theta_below_one_keeps_its_launches(kind, rows):
         assert np.isfinite(want[0]).all() and np.abs(want[1]).max() < 20  # (a rotation keeps the norm)
         for a, b in zip(got, want):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), position
+
+
+@pytest.mark.parametrize("rows", [1, 3])
+@pytest.mark.parametrize("capacity", [8192, 40960])
+def test_queries_whose_mean_square_is_below_the_normal_numbers(capacity, rows):
+    # 1e-20 and no eps: the norm's root is of 1e-40 (with some 16 bits), which the hardware's reciprocal root takes for 0
+    step, plain = (Step(saetta.KvBits.Eight, capacity, rows, seed=rows, eps=0.0) for _ in range(2))
+    step.qg[:, :, :D] *= 1e-20
+    built, ref = step.plan.build(), plain.plan.build()
+    for position in (0, 100, 3001):
+        got, want = step.run(built.run, position), plain.run(ref.run, position)
+        assert np.isfinite(got[0]).all() and np.isfinite(got[1]).all(), position
+        assert np.abs(got[0] - want[0]).max() < 1e-3 and np.abs(got[1] - want[1]).max() < 1e-3, position
 
 
 def test_other_steps_keep_their_launches():
