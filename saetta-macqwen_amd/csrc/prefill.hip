@@ -1334,7 +1334,10 @@ FlashPlan tiles_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, float &ti
     } else {
         best = unsplit;
     }
-    tiles_us = best + PREPARE_US + PREPARE_KEY_US * float(pos + tokens) * float(kv_heads);
+    // (never less than 5 us, what short contexts' images were counted at when the row groups came in: a chunk that goes to them
+    // without parts needs no workspace, and who calls it without one, recording or under capture, goes on to)
+    const float prepare_us = PREPARE_US + PREPARE_KEY_US * float(pos + tokens) * float(kv_heads);
+    tiles_us = best + (prepare_us > 5.0f ? prepare_us : 5.0f);
     return f;
 }
 

@@ -5,6 +5,7 @@ Restates tests/attention_prefill.rs (spread data; (pos, tokens) = (0,1), (0,7), 
 f32 CPU attention as the other side (src/prefill.rs:2489-2495 defines the chunk that way), over a
 half cache and over 8/4-bit caches read in place; bar of this build: rel-RMS <= 1e-3.
 """
+import ctypes
 import math
 
 import numpy as np
@@ -308,6 +309,49 @@ def test_row_groups_with_their_keys_in_parts(kind, pos, tokens, kv):
         off = (out.double() - want).norm() / want.norm()
         assert float(off) < REL_RMS, float(off)
         assert float((out - want).abs().max()) < MAX_ABS
+
+
+def chunk(kind, pos, tokens, kv):
+    """Inputs of a chunk, what the cache stands for in 64 bits, and the C call of it in a workspace (address, bytes)."""
+    heads, n = 8 * kv, pos + tokens
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device="cuda")  # noqa: E731
+    k, v, q16, qg = normal(n, kv * D), normal(n, kv * D), normal(tokens, heads, D).half(), normal(tokens, heads, 2 * D)
+    lib, p, out = saetta.ffi.lib(), saetta.FlashParams(heads, kv, pos, tokens, 1.0 / 16), torch.empty(tokens, heads, D, device="cuda")
+    if kind is saetta.KvBits.Half:
+        keys, values = k.half(), v.half()
+        kf, vf = keys, values
+        call = lambda ws, size: lib.saetta_attn_prefill(saetta.host._stream(), q16.data_ptr(), keys.data_ptr(), values.data_ptr(), qg.data_ptr(),  # noqa: E731
+                                                        out.data_ptr(), p, ws, size)
+    else:
+        keys, values = saetta.QuantRows(kind, kv * D, n), saetta.QuantRows(kind, kv * D, n)
+        keys.encode(k.view(-1), 0, n), values.encode(v.view(-1), 0, n)
+        kf, vf = (saetta.dequantize(*c.tensors(), kind) for c in (keys, values))
+        call = lambda ws, size: lib.saetta_attn_prefill_quant(saetta.host._stream(), kind.value, q16.data_ptr(), keys.c(), values.c(),  # noqa: E731
+                                                              qg.data_ptr(), out.data_ptr(), p, ws, size)
+    return call, out, p, attention_64(q16, kf.view(n, kv, D), vf.view(n, kv, D), qg, pos)
+
+
+@pytest.mark.parametrize("kind,pos,tokens,kv", [(saetta.KvBits.Half, 1166, 1, 1), (saetta.KvBits.Half, 1166, 85, 1), (saetta.KvBits.Half, 1203, 183, 1),
+                                                (saetta.KvBits.Half, 315, 1317, 1), (saetta.KvBits.Eight, 981, 134, 1), (saetta.KvBits.Four, 759, 638, 1),
+                                                (saetta.KvBits.Eight, 95, 1401, 1), (saetta.KvBits.Half, 767, 2, 2), (saetta.KvBits.Four, 200, 30, 2)])
+def test_short_chunks_are_recorded_without_a_workspace(kind, pos, tokens, kv):
+    # what the row groups take without parts needs none; sizes at the line to the tiles, which a recorded call without a
+    # workspace is refused
+    call, out, _, want = chunk(kind, pos, tokens, kv)
+    lib, results = saetta.ffi.lib(), []
+    assert lib.saetta_plan_begin() == 0
+    results.append(call(None, 0))
+    plan = ctypes.c_void_p(lib.saetta_plan_end())
+    try:
+        assert results == [0], lib.saetta_last_error()
+        out.fill_(float("nan"))
+        assert lib.saetta_plan_run(saetta.host._stream(), plan) == 0
+        assert float((out.double() - want).norm() / want.norm()) < REL_RMS
+        assert float((out - want).abs().max()) < MAX_ABS
+    finally:
+        torch.cuda.synchronize()
+        lib.saetta_plan_free(plan)
 
 
 @pytest.mark.parametrize("pos,tokens", [(2045, 3), (2300, 4), (4200, 3), (8186, 5), (8200, 4), (16300, 2)])
