@@ -450,12 +450,11 @@ int saetta_deltanet_rows_fused_sync(saetta_stream_t stream, const float *x, cons
 /* Bytes of workspace a prefill chunk at (pos, tokens) wants: the f16 key and
  * value tile images of the pos + tokens rows the chunk can see and, for a chunk with too few
  * tokens to fill the GPU, room for partial results of parts of the keys (up to 64 parts of
- * 1 KB + 8 B per query row; where no images are made, instead of them).  A call given the images' part only (one sized for
- * another chunk of as many rows) runs too, without the split.  Its bits are then
+ * 1 KB + 8 B per query row; where no images are made, instead of them).  A call given less, but room for the images (one
+ * sized for another chunk of as many rows), runs too, and without the split if the parts do not fit.  Its bits are then
  * others: the probabilities are rounded to f16 relative to a maximum, which with
  * the split is a part's own.  Both forms are as close to the exact result, but who
- * wants the same bits from one call to the next gives workspaces that both do, or
- * both do not, hold what this function returns.  The reference
+ * wants the same bits from one call to the next gives workspaces that hold what this function returns.  The reference
  * has no counterpart (its kernels dequantize in place); the closest is the
  * half scratch of Prefill::new (src/prefill.rs:1674-1686). */
 size_t saetta_prefill_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv_heads);
@@ -468,7 +467,8 @@ size_t saetta_prefill_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv
  * saetta_prefill_workspace_bytes(pos, tokens, kv_heads) bytes (at least the images), 16-byte
  * aligned, overwritten by the call; NULL makes the library use one of its own
  * per device and stream, which it grows with hipMalloc when needed (so not
- * under stream capture) and keeps until the process ends.  Kernel replaced:
+ * under stream capture, and not when recorded) and keeps until the process ends; where it
+ * cannot have one, a chunk that is short enough to do without runs without the split, any other is refused.  Kernel replaced:
  * attention_fa{4,8} (kernels/attention_prefill.metal:38-169). */
 int saetta_attn_prefill(saetta_stream_t stream, const uint16_t *q_f16, const uint16_t *keys,
                         const uint16_t *values, const float *q_and_gate, float *out,

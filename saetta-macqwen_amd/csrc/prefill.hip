@@ -1548,12 +1548,16 @@ int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kda
     if (p.tokens == 0) return SAETTA_OK;
     const FlashPlan plan = flash_plan(p.pos, p.tokens, p.kv_heads, bits);
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
-    size_t have = workspace ? workspace_size : 0;
     // (a workspace that is given has to do for the images, whatever the chunk: which launches serve it is no caller's business.
-    // One of the library's is taken where the chunk does not do without.)
-    if (workspace || !plan.small) {
-        if (!workspace) have = plan.bytes();
-        if (int rc = acquire_workspace(stream, workspace, workspace_size, workspace ? plan.plain : have, owned_lock, what, "saetta_prefill_workspace_bytes")) return rc;
+    // One of the library's is taken where the chunk has a use for one, so that it runs as in one of the caller's; where there
+    // is none to be had, a chunk that can do without does.)
+    size_t have = workspace ? workspace_size : plan.small ? plan.small_parts : plan.bytes();
+    if (workspace || have > 0) {
+        if (int rc = acquire_workspace(stream, workspace, workspace_size, workspace ? plan.plain : have, owned_lock, what, "saetta_prefill_workspace_bytes")) {
+            if (workspace || !plan.small) return rc;
+            (void)hipGetLastError();
+            have = 0;
+        }
     }
     return launch_chunk(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, have, false, plan, what);
 }

@@ -354,6 +354,25 @@ def test_short_chunks_are_recorded_without_a_workspace(kind, pos, tokens, kv):
         lib.saetta_plan_free(plan)
 
 
+@pytest.mark.parametrize("kind,pos,tokens,kv", [(saetta.KvBits.Half, 767, 2, 2), (saetta.KvBits.Half, 1020, 9, 2), (saetta.KvBits.Half, 961, 139, 2),
+                                                (saetta.KvBits.Eight, 767, 2, 2), (saetta.KvBits.Four, 767, 2, 2), (saetta.KvBits.Half, 2300, 4, 2),
+                                                (saetta.KvBits.Half, 200, 30, 2)])
+def test_no_workspace_is_as_good_as_one(kind, pos, tokens, kv):
+    # the library's own holds the parts of a chunk that could do without too: the same bits as in a workspace of just the size;
+    # one that does not hold the images is refused
+    call, out, p, want = chunk(kind, pos, tokens, kv)
+    size = saetta.attention_prefill.workspace_bytes(p)
+    ws, results = torch.full((size,), 0xff, dtype=torch.uint8, device="cuda"), []
+    for args in ((ws.data_ptr(), size), (None, 0)):
+        out.fill_(float("nan"))
+        assert call(*args) == 0, saetta.ffi.lib().saetta_last_error()
+        results.append(host(out))
+        assert float((out.double() - want).norm() / want.norm()) < REL_RMS
+    assert np.array_equal(*results)
+    for nbytes in (0, 1, -(-(pos + tokens) // 32) * kv * 32768):
+        assert call(ws.data_ptr(), nbytes) == -6  # SAETTA_E_SCRATCH
+
+
 @pytest.mark.parametrize("pos,tokens", [(2045, 3), (2300, 4), (4200, 3), (8186, 5), (8200, 4), (16300, 2)])
 def test_many_parts_are_merged_by_teams(pos, tokens):
     # 8 parts of 8 blocks and one team, 9 and more and four: teams without a part, one batch each and two, a last batch of one
