@@ -299,11 +299,6 @@ __device__ __forceinline__ uint32_t tokens_new(const PartialArgs &a, uint32_t po
     return seen > position ? seen - position : 0;
 }
 
-__device__ __forceinline__ void wave_sync() {  // LDS written by lanes of the wave and read by others: its accesses run in order
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // Dims 64 i + lane of a kv head's row of the cache.
 template <int BITS>
 __device__ __forceinline__ void cached_row(const void *data, const uint16_t *scales, const uint16_t *biases, size_t slot, uint32_t lane, float (&x)[4]) {

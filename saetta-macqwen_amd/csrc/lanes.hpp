@@ -61,4 +61,11 @@ __device__ __forceinline__ float inverse_root(float x) {
     return off == off ? fmaf(0.5f * y, off, y) : y;
 }
 
+// Between accesses of LDS by lanes of a wave to what others of its lanes access: the hardware runs a wave's in order, and this
+// keeps the compiler, which sees one lane's addresses, from moving them past each other.  (No instruction.)
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 }  // namespace saetta

@@ -653,8 +653,10 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     }
     constexpr int PIECE = 32 * 16 + 16;
     static_assert(32 * PIECE <= MERGE_WAVE_BYTES, "the pieces of 32 rows");
+    wave_sync();  // every lane has taken what the partner handed over
 #pragma unroll
     for (int i = 0; i < 16; i++) *reinterpret_cast<float4 *>(theirs_base + (2 * i + (at >> 5)) * PIECE + (at & 31) * 16) = o[i];
+    wave_sync();
 #pragma unroll
     for (int i = 0; i < 16; i++) {
         const float4 x = *reinterpret_cast<const float4 *>(theirs_base + in_row / 4 * PIECE + (2 * i + half_row) * 16);
@@ -1223,11 +1225,13 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
     // r at 16 ((r + 2 p) % 32) of the piece's 512 bytes, so that neither side meets in its banks.
     const float inv = 1.0f / l_all;
     unsigned char *turned = lds + wave * 4096;
+    wave_sync();  // every lane has taken what was handed over
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const uint32_t piece = 2 * i + hf;
         *reinterpret_cast<float4 *>(turned + piece * 512 + (col + 2 * piece) % 32 * 16) = float4{fin[4 * i] * inv, fin[4 * i + 1] * inv, fin[4 * i + 2] * inv, fin[4 * i + 3] * inv};
     }
+    wave_sync();
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const uint32_t piece = lane & 7;
