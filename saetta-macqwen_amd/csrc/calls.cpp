@@ -80,10 +80,14 @@ template <class T>
 T *pointer(const at::Tensor &t) {
     return static_cast<T *>(t.data_ptr());
 }
-template <class T = void>
+// A tensor that a kernel can reach.
+template <class T>
 T *pointer_of(PyObject *o, const char *what) {
-    if (!THPVariable_Check(o)) raise(PyExc_TypeError, "%s: expected a tensor", what);
-    return pointer<T>(THPVariable_Unpack(o));
+    if (THPVariable_Check(o)) {
+        const at::Tensor &t = THPVariable_Unpack(o);
+        if (t.is_cuda() || t.is_pinned()) return pointer<T>(t);
+    }
+    raise(PyExc_TypeError, "%s: expected a tensor on the GPU or in pinned memory", what);
 }
 
 long long integer(PyObject *o) {
@@ -157,6 +161,7 @@ PyObject *setup(PyObject *module, PyObject *const *a, Py_ssize_t n) {
 PyObject *to_half(PyObject *module, PyObject *const *a, Py_ssize_t n) {
     return guarded(n, 3, "to_half", [&] {
         const at::Tensor &x = need(a[0], at::kFloat, "to_half x"), &out = need(a[1], at::kHalf, "to_half out");
+        if (out.numel() < x.numel()) raise(PyExc_ValueError, "to_half: out does not hold x's values");
         State &st = state_of(module);
         const Library &lib = library(st);
         const saetta_stream_t s = stream_of(a[2]);
@@ -170,14 +175,16 @@ PyObject *to_half(PyObject *module, PyObject *const *a, Py_ssize_t n) {
 // kv_encode(bits, per_token, capacity, data, scales, biases, x, pos, tokens, stream)
 PyObject *kv_encode(PyObject *module, PyObject *const *a, Py_ssize_t n) {
     return guarded(n, 10, "kv_encode", [&] {
-        const at::Tensor &x = need(a[6], at::kFloat, "QuantRows.encode x");
         const long long per_token = integer(a[1]), capacity = integer(a[2]), pos = integer(a[7]), tokens = integer(a[8]);
-        if (pos + tokens > capacity || x.numel() < tokens * per_token * SAETTA_QUANT_GROUP) raise(PyExc_ValueError, "QuantRows.encode: tokens do not fit");
+        const bool fit = tokens >= 0 && tokens <= capacity && pos >= 0 && pos <= capacity - tokens;
+        if (!fit) raise(PyExc_ValueError, "QuantRows.encode: tokens do not fit");
+        const at::Tensor &x = need(a[6], at::kFloat, "QuantRows.encode x");
+        if (x.numel() < tokens * per_token * SAETTA_QUANT_GROUP) raise(PyExc_ValueError, "QuantRows.encode: tokens do not fit");
+        const saetta_quant_rows rows{pointer_of<uint32_t>(a[3], "QuantRows.encode data"), pointer_of<uint16_t>(a[4], "QuantRows.encode scales"),
+                                     pointer_of<uint16_t>(a[5], "QuantRows.encode biases")};
         State &st = state_of(module);
         const Library &lib = library(st);
         const saetta_stream_t s = stream_of(a[9]);
-        const saetta_quant_rows rows{pointer_of<uint32_t>(a[3], "QuantRows.encode data"), pointer_of<uint16_t>(a[4], "QuantRows.encode scales"),
-                                     pointer_of<uint16_t>(a[5], "QuantRows.encode biases")};
         const saetta_kv_quant_params p{uint32_t(per_token * tokens), uint32_t(per_token)};
         const int bits = int(integer(a[0]));
         const float *from = pointer<float>(x);
@@ -212,10 +219,10 @@ PyObject *prefill_quant(PyObject *module, PyObject *const *a, Py_ssize_t n) {
         if (p.heads != p.kv_heads * SAETTA_GQA_GROUP) raise(PyExc_ValueError, "prefill attention needs 8 q heads per kv head");
         const at::Tensor &q = need(a[1], at::kHalf, "q"), &qg = need(a[8], at::kFloat, "q_and_gate"), &out = need(a[9], at::kFloat, "out"),
                          &ws = need(a[11], at::kByte, "workspace");
-        const Library &lib = library(st);
-        const saetta_stream_t s = stream_of(a[12]);
         const saetta_quant_rows keys{pointer_of<uint32_t>(a[2], "keys"), pointer_of<uint16_t>(a[3], "keys"), pointer_of<uint16_t>(a[4], "keys")},
             values{pointer_of<uint32_t>(a[5], "values"), pointer_of<uint16_t>(a[6], "values"), pointer_of<uint16_t>(a[7], "values")};
+        const Library &lib = library(st);
+        const saetta_stream_t s = stream_of(a[12]);
         const int bits = int(integer(a[0]));
         const uint16_t *q_ptr = pointer<uint16_t>(q);
         const float *g = pointer<float>(qg);

@@ -151,6 +151,9 @@ def test_calls_check_what_they_are_given():
     rows = saetta.QuantRows(saetta.KvBits.Eight, 512, 4, "cpu")
     with pytest.raises(TypeError, match="QuantRows.encode x"):
         rows.encode(x, 0, 1)
+    for pos, tokens in ((-1, 1), (-4, 8), (0, -1), (3, -1), (4, 1), (0, 5), (2**63 - 1, 1), (-2**63, 0)):
+        with pytest.raises(ValueError, match="tokens do not fit"):
+            rows.encode(x, pos, tokens)
     with pytest.raises(ValueError, match="no prefill attention kernel"):
         ap.encode("attention_fa3", h, h, h, x, x, p, workspace=x)
     with pytest.raises(ValueError, match="attention_fa4 needs 8 q heads per kv head"):
@@ -158,6 +161,8 @@ def test_calls_check_what_they_are_given():
     with pytest.raises(TypeError, match="q: expected a contiguous torch.float16"):
         ap.encode("attention_fa8", h, h, h, x, x, p, workspace=x)
     calls = saetta.host._calls
+    with pytest.raises(TypeError, match="token_params_set params: expected a tensor on the GPU"):
+        calls.token_params_set(x, 0, 0, 0, 0)
     with pytest.raises(TypeError, match="expected FlashParams"):
         calls.prefill("attention_fa8", h, h, h, x, x, "p", x, None)
     with pytest.raises(TypeError, match="takes 3 arguments"):

@@ -135,6 +135,26 @@ def test_to_half_rounds_to_nearest_even():
     assert np.array_equal(host(out).view(np.uint16), oracle.f32_to_f16_bits(x))
 
 
+def test_buffers_too_small_or_elsewhere_are_refused():
+    x = torch.zeros(1024, device="cuda")
+    with pytest.raises(ValueError, match="out does not hold"):
+        saetta.to_half(x, torch.empty(1023, dtype=torch.float16, device="cuda"))
+    with pytest.raises(ValueError, match="tokens do not fit"):
+        saetta.QuantRows(saetta.KvBits.Eight, 512, 4).encode(x, 0, 3)
+    with pytest.raises(TypeError, match="QuantRows.encode data: expected a tensor on the GPU"):
+        saetta.QuantRows(saetta.KvBits.Eight, 512, 4, "cpu").encode(x, 0, 2)
+    pinned, there = saetta.QuantRows(saetta.KvBits.Eight, 512, 4, "cpu"), saetta.QuantRows(saetta.KvBits.Eight, 512, 4)
+    pinned.data, pinned.scales, pinned.biases = (t.pin_memory() for t in pinned.tensors())  # (new tensors, made in pinned memory)
+    for rows in (pinned, there):
+        rows.encode(torch.arange(1024.0, device="cuda"), 2, 2)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b.cpu()) for a, b in zip(pinned.tensors(), there.tensors()))
+    plan = saetta.Plan()
+    plan.params = plan.params.cpu()
+    with pytest.raises(TypeError, match="token_params_set params: expected a tensor on the GPU"):
+        plan.set_params(saetta.TokenParams(0, 0))
+
+
 def test_calls_run_on_the_stream_they_are_given():
     # the current stream, a stream that is not current, the default stream beside a current one: behind what that stream
     # holds, which is long enough for a call on another stream to be there first
