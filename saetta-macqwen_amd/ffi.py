@@ -55,23 +55,28 @@ class SaettaError(RuntimeError):
     """A non-zero return of the C ABI (the reference panics in these places)."""
 
 
-class _Missing:
-    """What stands for the extension module where it has not been built: importing works, a call raises."""
+class _Calls:
+    """The extension module of csrc/calls.cpp, set up for this copy of the package, and loaded when the first of its calls is
+    made: one that is built after the package was imported does, and where there is none, or one that does not load, importing
+    works and a call raises.  (It wants torch to be imported.)"""
 
     def __getattr__(self, name):
-        raise SaettaError(f"{CALLS_PATH} is missing: run __graft_entry__.build() (make -C csrc)")
+        if name.startswith("__"):
+            raise AttributeError(name)
+        if not os.path.exists(CALLS_PATH):
+            raise SaettaError(f"{CALLS_PATH} is missing: run __graft_entry__.build() (make -C csrc)")
+        loader = importlib.machinery.ExtensionFileLoader("_saetta_calls", CALLS_PATH)
+        try:
+            module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_saetta_calls", CALLS_PATH, loader=loader))
+            loader.exec_module(module)
+        except ImportError as e:
+            raise SaettaError(f"{CALLS_PATH} does not load (built for another Python or torch?): run __graft_entry__.build() (make -C csrc): {e}") from e
+        module.setup(LIB_PATH, SaettaError, FlashParamsC)
+        vars(self).update((k, v) for k, v in vars(module).items() if not k.startswith("__"))  # (found there from now on)
+        return getattr(module, name)
 
 
-def calls():
-    """The extension module of csrc/calls.cpp, set up for this copy of the package.  (It wants torch to be imported.)"""
-    if not os.path.exists(CALLS_PATH):
-        return _Missing()
-    loader = importlib.machinery.ExtensionFileLoader("_saetta_calls", CALLS_PATH)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_saetta_calls", CALLS_PATH, loader=loader))
-    loader.exec_module(module)
-    module.setup(LIB_PATH, SaettaError, FlashParamsC)
-    return module
-
+calls = _Calls()
 
 _lib = None
 

@@ -171,6 +171,36 @@ def test_calls_check_what_they_are_given():
         calls.plan_run(0, 0)
 
 
+def test_the_calls_extension_is_looked_for_when_it_is_called(tmp_path):
+    # a package imported before its extension is there: importing works, a call says what is missing, and works once it is
+    # built; one that does not load is an error of the call, too
+    import shutil
+    import sys
+    src = os.path.dirname(ffi.__file__)
+    shutil.copytree(src, tmp_path / "pkg", ignore=shutil.ignore_patterns("*.so", "*.o", "__pycache__", "csrc"))
+    os.makedirs(tmp_path / "pkg" / "lib", exist_ok=True)
+    code = f"""
+import os, shutil, torch, pkg
+x = torch.zeros(64)
+def raised():
+    try:
+        pkg.to_half(x, x)
+    except Exception as e:
+        return e
+e = raised()
+assert isinstance(e, pkg.ffi.SaettaError) and "is missing" in str(e), e
+with open(pkg.ffi.CALLS_PATH, "w") as f:
+    f.write("not a library")
+e = raised()
+assert isinstance(e, pkg.ffi.SaettaError) and "does not load" in str(e), e
+os.remove(pkg.ffi.CALLS_PATH)
+shutil.copy({ffi.CALLS_PATH!r}, pkg.ffi.CALLS_PATH)
+e = raised()
+assert type(e) is TypeError and "to_half x" in str(e), e
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=tmp_path, env=dict(os.environ, PYTHONPATH=str(tmp_path)))
+
+
 def test_kv_bits_mirror():
     # src/kv_quant.rs:11-50
     K = saetta.KvBits
