@@ -201,6 +201,26 @@ assert type(e) is TypeError and "to_half x" in str(e), e
     subprocess.run([sys.executable, "-c", code], check=True, cwd=tmp_path, env=dict(os.environ, PYTHONPATH=str(tmp_path)))
 
 
+def test_the_library_is_built_without_torch(tmp_path):
+    # what make would do: with a Python that finds no torch, or none at all, the C library and nothing else
+    import sys
+
+    def steps(python, *goals):
+        r = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "saetta-macqwen_amd", "csrc"), f"PYTHON={python}", *goals], capture_output=True, text=True)
+        return r.returncode, r.stdout + r.stderr
+
+    bare = tmp_path / "bare"
+    bare.write_text(f'#!/bin/sh\nexec {sys.executable} -S -I "$@"\n')  # (without site-packages)
+    bare.chmod(0o755)
+    for python in (bare, tmp_path / "none"):
+        rc, text = steps(python)
+        assert rc == 0 and "libsaetta_hip.so" in text and "calls" not in text, text
+        rc, text = steps(python, "calls")
+        assert rc != 0 and "need torch" in text
+    rc, text = steps(sys.executable)
+    assert rc == 0 and os.path.basename(ffi.CALLS_PATH) in text and "libsaetta_hip.so" in text
+
+
 def test_kv_bits_mirror():
     # src/kv_quant.rs:11-50
     K = saetta.KvBits
