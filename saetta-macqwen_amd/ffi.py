@@ -5,10 +5,11 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import sysconfig
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("SAETTA_HIP_LIB") or os.path.join(_HERE, "lib", "libsaetta_hip.so")
-CALLS_PATH = os.path.join(_HERE, "lib", "_saetta_calls.so")
+CALLS_PATH = os.path.join(_HERE, "lib", "_saetta_calls" + sysconfig.get_config_var("EXT_SUFFIX"))  # (of this Python)
 
 # Every symbol include/saetta_hip.h declares; tests check the library exports each.
 SYMBOLS = [

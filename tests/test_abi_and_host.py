@@ -202,7 +202,8 @@ assert type(e) is TypeError and "to_half x" in str(e), e
 
 
 def test_the_library_is_built_without_torch(tmp_path):
-    # what make would do: with a Python that finds no torch, or none at all, the C library and nothing else
+    # what make would do: with a Python that finds no torch, or none at all, the C library and nothing else; the extension by the
+    # Python that is asked for, under the name which that Python looks for
     import sys
 
     def steps(python, *goals):
@@ -219,6 +220,17 @@ def test_the_library_is_built_without_torch(tmp_path):
         assert rc != 0 and "need torch" in text
     rc, text = steps(sys.executable)
     assert rc == 0 and os.path.basename(ffi.CALLS_PATH) in text and "libsaetta_hip.so" in text
+
+
+def test_the_extension_is_this_pythons(monkeypatch):
+    # built by the Python that runs build(), whatever python3 is on the path, and under a name that no other loads
+    import sys
+    import sysconfig
+    made = []
+    monkeypatch.setattr(entry.subprocess, "run", lambda command, **_: made.append(command))
+    entry.build()
+    assert f"PYTHON={sys.executable}" in made[0] and "calls" in made[0]
+    assert ffi.CALLS_PATH.endswith("_saetta_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
 def test_kv_bits_mirror():
