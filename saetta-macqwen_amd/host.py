@@ -756,10 +756,12 @@ def _workspace(t):
     return _ptr(t), t.numel()
 
 
-def _own_workspace(q, p, stream):
+def _own_workspace(what, q, p, stream):
     """A workspace for the chunk of FlashParams p as a tensor of the call's own from torch's allocator (which hands a
     block out again only behind the work queued on its stream): the library's own workspace, which a
     NULL pointer would select, is one per device and stream that stays for the life of the process."""
+    if p.heads != p.kv_heads * 8:  # (what the call would say once it has its workspace)
+        raise ValueError(f"{what} needs 8 q heads per kv head")
     _need(q, torch.float16, "q")
     t = torch.empty(attention_prefill.workspace_bytes(p), dtype=torch.uint8, device=q.device)
     if isinstance(stream, torch.cuda.Stream):
@@ -795,7 +797,7 @@ class attention_prefill:
         call's own (a caller that times the call, or records it, brings its own)."""
         if kernel not in attention_prefill.KERNELS:
             raise ValueError(f"no prefill attention kernel {kernel}")
-        _calls.prefill(kernel, q, keys, values, q_and_gate, out, p, workspace if workspace is not None else _own_workspace(q, p, stream), _handle(stream))
+        _calls.prefill(kernel, q, keys, values, q_and_gate, out, p, workspace if workspace is not None else _own_workspace(kernel, q, p, stream), _handle(stream))
 
     @staticmethod
     def encode_rows2(q, keys, values, q_and_gate, out, p, stream=None, workspace=None):
@@ -861,7 +863,7 @@ class attention_prefill:
     def encode_quant(q, keys, values, q_and_gate, out, p, stream=None, workspace=None):
         """The chunk over a quantized cache read in place (src/prefill.rs:1735-1776)."""
         _calls.prefill_quant(keys.bits._value_, q, keys.data, keys.scales, keys.biases, values.data, values.scales, values.biases, q_and_gate, out, p,
-                             workspace if workspace is not None else _own_workspace(q, p, stream), _handle(stream))
+                             workspace if workspace is not None else _own_workspace("prefill attention", q, p, stream), _handle(stream))
 
 
 class attention_gemm:

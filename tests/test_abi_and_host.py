@@ -158,6 +158,10 @@ def test_calls_check_what_they_are_given():
         ap.encode("attention_fa3", h, h, h, x, x, p, workspace=x)
     with pytest.raises(ValueError, match="attention_fa4 needs 8 q heads per kv head"):
         ap.encode("attention_fa4", h, h, h, x, x, saetta.FlashParams(15, 2, 0, 1, 0.0625), workspace=x)
+    with pytest.raises(ValueError, match="attention_fa4 needs 8 q heads per kv head"):  # ... before there is a workspace
+        ap.encode("attention_fa4", h, h, h, x, x, saetta.FlashParams(15, 2, 0, 1, 0.0625))
+    with pytest.raises(ValueError, match="prefill attention needs 8 q heads per kv head"):
+        ap.encode_quant(h, rows, rows, x, x, saetta.FlashParams(15, 2, 0, 1, 0.0625))
     with pytest.raises(TypeError, match="q: expected a contiguous torch.float16"):
         ap.encode("attention_fa8", h, h, h, x, x, p, workspace=x)
     calls = saetta.host._calls
