@@ -1354,7 +1354,8 @@ FlashPlan tiles_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, float &ti
 // group's keys: the few tokens of a short turn behind a long prefix then fill the chip, each CU reading a part of the cache where
 // it lies, where the tiles would write and read the images of all of it for two or four of them.  0.36 us a block up to some
 // 200 workgroups, the chip 590 blocks a us; parts are some 7 us of ends, the merge 4.2 and a little for each part.  Two rounds of
-// workgroups at most, so that row groups of up to 64 tokens of 2 kv heads have parts to choose from and those of up to 256 two.
+// workgroups at most (one, nearly always), and row groups for half of the CUs: 64 tokens of 2 kv heads may have up to 16 parts, 256
+// tokens 2 to 4.
 // The whole call, halves, what it was -> parts: 7 tokens at 3000 31.3 -> 19.5 us, at 20000 49.8 -> 29.9, at 100000 186 -> 54.6; 30 at 3000 34.1 ->
 // 22.2, at 40000 79.0 -> 54.4; 64 at 1500 32.7 -> 20.9, at 20000 64.6 -> 52.8; 128 at 1000 25.0 -> 22.8, at 3000 35.6 -> 31.6; 250 at 1500
 // 36.2 -> 31.9.  Left alone: 128 at 10000 54.1 and 53.5, 250 at 4000 46.8 and 52.1 (with codes 49.3 and 53.8).

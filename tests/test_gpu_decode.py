@@ -101,7 +101,7 @@ def test_verify_rows_match_single_row_decodes(kind, m):
 @pytest.mark.parametrize("kind,m", [(saetta.KvBits.Eight, 2), (saetta.KvBits.Eight, 3), (saetta.KvBits.Eight, 4),
                                     (saetta.KvBits.Four, 1)])
 def test_long_context_with_outlier_channels(kind, m):
-    # configs[1] in full: 8-bit at 32768 + m rows for m = 2, 3, 4 (m = 1 at this size is in
+    # 8-bit at 32768 + m rows for m = 2, 3, 4 (m = 1 at this size is in
     # test_large_cache_of_codes_one_row); 4-bit at 20000 with 1 % of channels x8; the new tokens are
     # quantized on the device into the rows after the context.
     rng = np.random.default_rng(8 + m)
@@ -143,7 +143,7 @@ def poison_from(cache, bits, token):
 
 
 def test_four_bit_150k_tokens_with_append():
-    # configs[3] in full: one query token over 150 000 cached tokens of 4-bit codes with 1 % of the
+    # one query token over 150 000 cached tokens of 4-bit codes with 1 % of the
     # channels scaled x8, capacity 150 016, the step's 4 new tokens quantized on the device into
     # the rows after them.  A one-row launch over 4-bit codes in a cache this large takes the
     # two-workgroups-per-CU kernel and 256 splits.  Then two shorter contexts in the same cache

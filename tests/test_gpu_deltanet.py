@@ -1,7 +1,7 @@
 """Gated DeltaNet decode step on the GPU (deltanet_conv + deltanet_step) against the oracle.
 
 The oracle is pinned by the reference's MLX golden vectors at dims 8 (tests/test_oracle_deltanet.py);
-here the kernels run the real shape (16 key / 32 value heads of 128, conv kernel 4, configs[4]) and
+here the kernels run the real shape (16 key / 32 value heads of 128, conv kernel 4) and
 smaller value dims over several tokens, with the states carried along on both sides.  Dot products
 are summed in another order than on the CPU: 2e-5 relative on y and the state, 2e-6 on the conv.
 """

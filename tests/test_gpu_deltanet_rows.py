@@ -105,7 +105,7 @@ def check_against_oracle(layer, tokens, pieces, snapshots, tol=2e-5):
 
 
 def test_real_shape_verify_rows_with_snapshots():
-    # configs[4]: 16 key / 32 value heads of 128, conv kernel 4; 1..4 rows as the verify step has
+    # 16 key / 32 value heads of 128, conv kernel 4; 1..4 rows as the verify step has
     layer = Layer(16, 32, 128, 4, seed=11)
     check_against_oracle(layer, 10, [1, 2, 3, 4], snapshots=True)
 

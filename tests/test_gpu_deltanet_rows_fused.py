@@ -63,7 +63,7 @@ def check(layer, pieces, snapshots):
 
 @pytest.mark.parametrize("snapshots", [False, True])
 def test_real_shape_one_to_eight_rows(snapshots):
-    # configs[4]: 16 key / 32 value heads of 128, conv kernel 4; every row count the call takes
+    # 16 key / 32 value heads of 128, conv kernel 4; every row count the call takes
     layer = Layer(16, 32, 128, 4, seed=41 + snapshots)
     check(layer, [1, 2, 3, 4, 5, 6, 7, 8], snapshots)
 

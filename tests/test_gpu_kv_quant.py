@@ -98,7 +98,7 @@ def test_extreme_groups_are_bit_exact(kind):
 
 @pytest.mark.parametrize("kind", KINDS)
 def test_outlier_channels_and_a_full_chunk(kind):
-    # configs[3]/[2]: N(0,1) with 1 % of channels x8; a 4096-token append in one launch.
+    # N(0,1) with 1 % of channels x8; a 4096-token append in one launch.
     rng = np.random.default_rng(23)
     tokens = 4096
     x = rng.standard_normal((tokens, VALUES)).astype(np.float32)

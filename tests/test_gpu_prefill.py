@@ -79,7 +79,7 @@ def test_matches_cpu_on_spread_data(kind, pos, tokens):
 
 @pytest.mark.parametrize("kind", KINDS)
 def test_gaussian_chunk_with_cached_prefix(kind):
-    # configs[2] in shape, scaled to what the CPU finishes in seconds: bf16-exact N(0,1) q, a cached
+    # a chunk behind a prefix of its length, scaled to what the CPU finishes in seconds: bf16-exact N(0,1) q, a cached
     # prefix quantized on the host, the chunk's K/V quantized on the device, gate N(0,1).
     rng = np.random.default_rng(12)
     pos, tokens = 300, 200
@@ -282,11 +282,13 @@ def attention_64(q16, k, v, qg, pos):
 
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("pos,tokens,kv", [(505, 1, 1), (767, 2, 2), (1020, 9, 2), (1279, 30, 3), (1800, 64, 2), (2047, 130, 2), (3000, 250, 2), (6100, 33, 1),
-                                           (9000, 7, 5), (20001, 30, 2), (50000, 5, 2)])
+                                           (9000, 7, 5), (20001, 30, 2), (50000, 5, 2), (32510, 1, 2), (33998, 49, 5)])
 def test_row_groups_with_their_keys_in_parts(kind, pos, tokens, kv):
     # A part is a multiple of 8 blocks of 32 keys: a row group that sees no key of a part that its tile has (1020, 1279, 2047),
-    # one block of the last, parts of one round and of many, two rounds of workgroups, as many as 64 parts, kv heads that an
-    # eighth of the workgroups does not divide; in a workspace of NaN of just the size, and with room for the images only.
+    # one block of the last, parts of one round and of many, two rounds of workgroups (33998, halves), as many as 64 parts
+    # (32510), kv heads that an eighth of the workgroups does not divide; in a workspace of NaN of just the size, and in one with
+    # room for the images, which holds the parts too where there are few rows to a key (767, 1020, from 9000 on) and elsewhere
+    # makes it the layout without them.
     heads, n = 8 * kv, pos + tokens
     gen = torch.Generator(device="cuda").manual_seed(pos)
     normal = lambda *shape: torch.randn(*shape, generator=gen, device="cuda")  # noqa: E731
