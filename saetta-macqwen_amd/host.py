@@ -22,7 +22,7 @@ import torch
 
 from . import ffi
 
-_calls = ffi.calls
+_calls = ffi.calls.ready()
 GROUP = 64      # src/kv_quant.rs:9
 MAX_ROWS = 8    # src/rows.rs:9
 DIM = 256

@@ -176,8 +176,9 @@ def test_calls_check_what_they_are_given():
 
 
 def test_the_calls_extension_is_looked_for_when_it_is_called(tmp_path):
-    # a package imported before its extension is there: importing works, a call says what is missing, and works once it is
-    # built; one that does not load is an error of the call, too
+    # loaded by the import where it is there; a package imported before its extension is there: importing works, a call says
+    # what is missing, and works once it is built; one that does not load is an error of the call, too
+    assert "to_half" in vars(ffi.calls)
     import shutil
     import sys
     src = os.path.dirname(ffi.__file__)
