@@ -89,6 +89,23 @@ __device__ __forceinline__ void split2(float x, _Float16 &hi, _Float16 &lo) {
     lo = (_Float16)(x - h);
 }
 
+typedef _Float16 half2_ __attribute__((ext_vector_type(2)));
+// The same of four values, two to a conversion; a lo part is what one multiply-add leaves of x and the hi part as stored.
+template <class F>
+__device__ __forceinline__ void split4(F &&value, half4 &hi, half4 &lo) {
+    half2_ h[2], l[2];
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        float x = value(2 * p), y = value(2 * p + 1);
+        asm("" : "+v"(x), "+v"(y));
+        uint32_t both = __builtin_bit_cast(uint32_t, half2_{(_Float16)x, (_Float16)y});
+        asm("" : "+v"(both));
+        h[p] = __builtin_bit_cast(half2_, both);
+        l[p] = half2_{(_Float16)__builtin_fmaf((float)h[p][0], -1.0f, x), (_Float16)__builtin_fmaf((float)h[p][1], -1.0f, y)};
+    }
+    hi = __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3), lo = __builtin_shufflevector(l[0], l[1], 0, 1, 2, 3);
+}
+
 // acc += A B with both operands in hi and lo parts
 __device__ __forceinline__ floatx4 mma3(half8 ah, half8 al, half8 bh, half8 bl, floatx4 acc) {
     acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh, acc, 0, 0, 0);
@@ -515,10 +532,17 @@ __device__ __forceinline__ half4 read_transposed(const unsigned char *at) {
 // Per block, with S0 [dv][128] the state's slice: P = K S0^T and Q S0^T (rows: tokens); R = V - e^c P;
 // U = T R; O = (e^c (Q S0^T) + M U) / sqrt(128); S1 = e^{c_last} S0 + (e^{c_last - c} U)^T K.
 // A wave takes 16 tokens' rows of K, Q, T and M, and nobody else reads those: they come from the workspace
-// straight into its registers, a whole block ahead, as the MFMA operands they are.  LDS holds what the
+// straight into its registers, two blocks ahead, as the MFMA operands they are.  LDS holds what the
 // waves hand to each other: the state's image, R, U and the scaled U, the block's values and decay
 // factors, and the block's keys, which the state's update contracts over the tokens: every wave puts
 // its rows there, and ds_read_b64_tr_b16 hands them out by key dim.
+// What bounds it: a block is three phases between barriers, each a trip through LDS, a few dependent products and a trip back,
+// and 92 KB of operands through the CU's 64 bytes a cycle, 1500 cycles of loads that a wave stands still at when they come all at
+// once.  A block took 4050 cycles, a state wave 450 of them at its eight loads behind K S0^T and 580 waiting for the output waves, who
+// stood at theirs.  So each team works where the other leaves LDS and the memory pipe alone: the outputs' M U and
+// stores under the next block's K S0^T, their Q S0^T under U, their loads under the state's update; the state's
+// loads two at a time between its dependent products.  (The output waves' loads under U: 246 us instead of 230.)
+// Measured, whole chunk, us: 1000 tokens 65.4 -> 61.2, 2300 140.3 -> 128.7, 4096 253.3 -> 230.4; results bit for bit the same.
 struct ChainLds {
     static constexpr int GAM = 0;                          // e^{c_t}, e^{c_last - c_t}: 128 f32
     static constexpr int V = GAM + 2 * C * 4;              // [token][DV] f32
@@ -527,15 +551,17 @@ struct ChainLds {
     static constexpr int RH = SL + DV * SROW * 2;          // [dv][64 tokens] images, rows of TROW f16: R, U, U scaled
     static constexpr int RL = RH + DV * TROW * 2, UH = RL + DV * TROW * 2, UL = UH + DV * TROW * 2;
     static constexpr int WH = UL + DV * TROW * 2, WL = WH + DV * TROW * 2;
-    // the block's keys [token][128] as hi and lo images, two sets for alternate blocks: every wave puts its 16
-    // rows there, and the state's update reads them by key dim (transposing reads)
-    static constexpr int KIMG = (WL + DV * TROW * 2 + 15) / 16 * 16;
-    static constexpr int BYTES = KIMG + 4 * K_IMG;
+    // the block's keys [token][128] as hi and lo images: every wave puts its 16 rows there, and the state's update reads
+    // them by key dim (transposing reads).  Piece p (8 key dims) of token t lies at place p ^ key_piece(t) of the token's 256
+    // bytes: 16 rows' pieces fall on all banks, and so do what half a wave reads, four tokens in a row and four 8 further.
+    static constexpr int KIMG = (WL + DV * TROW * 2 + 15) / 16 * 16, K_BYTES = C * K_DIM * 2;
+    static __device__ __forceinline__ uint32_t key_piece(uint32_t t) { return (t & 3) << 1 | (t & 8) | (t >> 2 & 1); }
+    static constexpr int BYTES = KIMG + 2 * K_BYTES;
 };
 
 // Eight waves in two teams.  Waves 0-3 carry the state: K S0^T, R, U and the state's update, each for 16 of
 // the block's tokens (the update: for 32 key dims).  Waves 4-7 make the outputs, which nothing in the chain
-// waits for: Q S0^T beside the first team's K S0^T, M U beside its update of the state, and the stores.
+// waits for: Q S0^T beside the first team's U, M U and the stores beside its K S0^T of the next block.
 // What a wave reads of a block: its 16 rows of K (or Q) and of T (or M), 12 operands at most, and, in the
 // first team, its share of the block's values and factors.
 struct ChainBlock {
@@ -543,8 +569,17 @@ struct ChainBlock {
     u32x4 tm[2][2];  // [hi | lo][k-step]: rows 16 w + n of T | M
     static constexpr int V_LOADS = C * DV * 4 / 16 / 256;  // 16-byte pieces per thread of the block's [token][DV] values
     u32x4 v[V_LOADS], gam;   // ...; 16 bytes of the 128 factors (threads 0-31)
+    uint32_t touched[2];     // AHEAD: what `touch` has loaded
 };
 
+// AHEAD: the operands of the block AHEAD_BLOCKS on are brought into the L2 by the workgroups that share them, each a piece
+// (`touch`).  What the conv and the prepare kernel have just written is served from the memory's cache (256 MB) while it fits, fast
+// enough for loads two blocks ahead, and the pieces are an eighth more traffic: whole chunk, us, without -> with: 1000 tokens 61.2
+// -> 62.8, 2300 128.9 -> 133.5, 3200 180.6 -> 182.0; past it the first of a line's readers waits for memory: 3500 205.1 -> 199.9, 4096
+// 248.0 -> 230.5 (6 blocks ahead 232.3, without the values' lines 238.7).
+constexpr uint32_t AHEAD_BLOCKS = 3;
+constexpr size_t AHEAD_FROM = size_t(208) << 20;  // bytes of `mixed` and the workspace: 3300 tokens of the model's shape
+template <bool AHEAD>
 __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) {
     using L = ChainLds;
     constexpr int NT = DV / 16;  // 16-wide tiles of value dims
@@ -571,18 +606,21 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
     const float *gam = reinterpret_cast<const float *>(lds + L::GAM);
     float *v_lds = reinterpret_cast<float *>(lds + L::V);
 
-    // A block's operands are asked for in three lots, each as soon as the registers it goes to have been read
+    // A block's operands are asked for in three lots, each when the registers it goes to have been read
     // for the block two before: the rows of K | Q, the rows of T | M, the block's values and factors.
     auto clamp_block = [&](uint32_t blk) { return blk < nblocks ? blk : nblocks - 1; };  // (past the last block: its operands again, unused)
+    // (the second team's operands lie two parts on: Q behind K, M behind T)
+    auto rows_of = [&](uint32_t at) {
+        return reinterpret_cast<const u32x4 *>(a.ws + size_t(clamp_block(at)) * per_block + khd * KHEAD_BYTES + (state_team ? 0 : 2 * K_GL)) + wave * 4 * 64 + lane;
+    };
+    auto request_kq_step = [&](const u32x4 *wk, int ks, ChainBlock &b) {
+#pragma unroll
+        for (int part = 0; part < 2; part++) b.kq[part][ks] = wk[(part * K_GL) / 16 + ks * 64];
+    };
     auto request_kq = [&](uint32_t at, ChainBlock &b) {
-        const uint32_t blk = clamp_block(at);
-        // (the second team's operands lie two parts on: Q behind K, M behind T)
-        const u32x4 *wk = reinterpret_cast<const u32x4 *>(a.ws + size_t(blk) * per_block + khd * KHEAD_BYTES + (state_team ? 0 : 2 * K_GL));
+        const u32x4 *wk = rows_of(at);
 #pragma unroll
-        for (int part = 0; part < 2; part++) {
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) b.kq[part][ks] = wk[(part * K_GL) / 16 + (wave * 4 + ks) * 64 + lane];
-        }
+        for (int ks = 0; ks < 4; ks++) request_kq_step(wk, ks, b);
     };
     auto request_tm = [&](uint32_t at, ChainBlock &b) {
         const uint32_t blk = clamp_block(at);
@@ -629,12 +667,7 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
 #pragma unroll
             for (int nt = 0; nt < 2; nt++) {
                 half4 sh, sl;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    _Float16 hi, lo;
-                    split2(s_reg[mt][nt][i], hi, lo);
-                    sh[i] = hi, sl[i] = lo;
-                }
+                split4([&](int i) { return s_reg[mt][nt][i]; }, sh, sl);
                 const int at = (16 * mt + n) * L::SROW + 32 * wave + 16 * nt + 4 * j;
                 *reinterpret_cast<half4 *>(img_w(L::SH) + at) = sh, *reinterpret_cast<half4 *>(img_w(L::SL) + at) = sl;
             }
@@ -653,52 +686,131 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
     // blocks' time to come back (one block's time is less than the 2.9 us a wave's batch takes under this load).
     // (the team is a type, so that a team's blocks are one piece of code: what one team asks for is not taken to be
     // in flight where the other team waits)
-    auto step = [&](auto team, uint32_t blk, ChainBlock &cur, const ChainBlock &next) {
-        constexpr bool STATE = decltype(team)::value;
-        const uint32_t nxt = blk + 1 < nblocks ? blk + 1 : blk;
-        if constexpr (STATE) {
-            request_values(blk + 2, cur);  // (this block's values went to LDS during the block before)
-            __builtin_amdgcn_sched_barrier(0);
-            // this wave's rows of the block's keys, for the state's update (the set of two blocks ago is read no more:
-            // every wave has been through the three barriers of the block between)
-            _Float16 *kimg = img_w(L::KIMG + int(blk & 1) * 2 * K_IMG);
+    // AHEAD: the lines of a block's operands that this workgroup brings into its XCD's L2 for all that read them: a sixteenth of
+    // the key head's rows (an eighth per value head), an eighth of T and M, and of the values, whose lines two slices share,
+    // half of its own.  One load names a line every four (values: eight) lanes.
+    auto touch = [&](uint32_t at, ChainBlock &b) {
+        asm volatile("" ::"v"(b.touched[0]), "v"(b.touched[1]));  // (two blocks old: there)
+        const uint32_t blk = clamp_block(at), line = (wave & 1) * 16 + (lane >> 2);
+        const unsigned char *base = a.ws + size_t(blk) * per_block;
+        const unsigned char *rows = base + khd * KHEAD_BYTES + (((h % group) * slices + slice) * 32 + line) * 128 % KHEAD_BYTES;
+        const unsigned char *tm = base + a.k_heads * KHEAD_BYTES + h * VHEAD_BYTES + (slice * 32 + line) * 128 % (4 * T_GL);
+        b.touched[0] = *reinterpret_cast<const uint32_t *>(wave < 2 ? rows : tm);
+        const uint32_t tok = min(blk * C + (slice & 1) * 32 + wave * 8 + (lane >> 3), a.tokens - 1);
+        b.touched[1] = *reinterpret_cast<const uint32_t *>(a.mixed + size_t(tok) * a.channels + 2 * a.k_heads * K_DIM + h * a.v_dim + DV * slice);
+    };
+    // ---- O = (e^c (Q S0^T) + M U) / sqrt(128) of block `blk`, whose Q S0^T and e^c the second team's waves hold ----
+    floatx4 held[NT];
+    float held_gam = 0.0f;
 #pragma unroll
-            for (int part = 0; part < 2; part++) {
+    for (int vt = 0; vt < NT; vt++) held[vt] = floatx4{0, 0, 0, 0};
+    auto outputs = [&](uint32_t blk, bool real, ChainBlock &b) {
+        floatx4 mu[NT];
 #pragma unroll
-                for (int ks = 0; ks < 4; ks++) {
-                    *reinterpret_cast<u32x4 *>(kimg + part * C * KROW + (16 * wave + n) * KROW + 32 * ks + 8 * j) = cur.kq[part][ks];
-                }
+        for (int vt = 0; vt < NT; vt++) {
+            mu[vt] = floatx4{0, 0, 0, 0};
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+                if (ks > int(wave) / 2) continue;
+                const int bo = (16 * vt + n) * TROW + 32 * ks + 8 * j;
+                mu[vt] = mma3(*reinterpret_cast<const half8 *>(img(L::UH) + bo), *reinterpret_cast<const half8 *>(img(L::UL) + bo),
+                              __builtin_bit_cast(half8, b.tm[0][ks]), __builtin_bit_cast(half8, b.tm[1][ks]), mu[vt]);
             }
         }
-        __syncthreads();  // the block's values and factors, the state's image and the keys are in LDS
-
-        // ---- K S0^T (first team): rows t = 16 wave + n, columns dv = 16 vt + n' | (Q S0^T)^T (second team): the other way
-        // round, so that a lane's results are four value dims of a token, one 16-byte store ----
-        floatx4 pkq[NT];
-#pragma unroll
-        for (int vt = 0; vt < NT; vt++) pkq[vt] = floatx4{0, 0, 0, 0};
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
+        __builtin_amdgcn_sched_barrier(0);
+        request_tm(blk + 2, b);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t tok = blk * C + 16 * wave + n;
+        if (real && tok < a.tokens) {
+            float *o = a.o + (size_t(tok) * a.v_heads + h) * a.v_dim + DV * slice + 4 * j;
 #pragma unroll
             for (int vt = 0; vt < NT; vt++) {
-                const int bo = (16 * vt + n) * L::SROW + 32 * ks + 8 * j;
-                const half8 bh = *reinterpret_cast<const half8 *>(img(L::SH) + bo), bl = *reinterpret_cast<const half8 *>(img(L::SL) + bo);
-                const half8 ah = __builtin_bit_cast(half8, cur.kq[0][ks]), al = __builtin_bit_cast(half8, cur.kq[1][ks]);
-                pkq[vt] = STATE ? mma3(ah, al, bh, bl, pkq[vt]) : mma3(bh, bl, ah, al, pkq[vt]);
+#pragma unroll
+                for (int i = 0; i < 4; i++) o[16 * vt + i] = Q_SCALE * (held_gam * held[vt][i] + mu[vt][i]);
             }
         }
+    };
+
+    auto step = [&](auto team, uint32_t blk, ChainBlock &cur, ChainBlock &next) {
+        constexpr bool STATE = decltype(team)::value;
+        const uint32_t nxt = blk + 1 < nblocks ? blk + 1 : blk;
+        if constexpr (STATE) request_values(blk + 2, cur);  // (this block's values went to LDS during the block before)
         __builtin_amdgcn_sched_barrier(0);
-        request_kq(blk + 2, cur);
-        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();  // the block's values and factors and the state's image are in LDS
+
+        // K S0^T (first team): rows t = 16 wave + n, columns dv = 16 vt + n' | (Q S0^T)^T (second team): the other way round,
+        // so that a lane's results are four value dims of a token, one 16-byte store.  As a k-step's rows have been read, the first
+        // team puts them into LDS (the image was last read two barriers ago) and asks for the block after next's.
+        floatx4 pkq[NT];
+        const u32x4 *const wk = rows_of(blk + 2);
+        auto by_state = [&]() {
+            half8 image[4][NT][2];
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+#pragma unroll
+                for (int vt = 0; vt < NT; vt++) {
+                    const int bo = (16 * vt + n) * L::SROW + 32 * ks + 8 * j;
+                    image[ks][vt][0] = *reinterpret_cast<const half8 *>(img(L::SH) + bo), image[ks][vt][1] = *reinterpret_cast<const half8 *>(img(L::SL) + bo);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+#pragma unroll
+                for (int vt = 0; vt < NT; vt++) {
+                    const half8 bh = image[ks][vt][0], bl = image[ks][vt][1];
+                    const half8 ah = __builtin_bit_cast(half8, cur.kq[0][ks]), al = __builtin_bit_cast(half8, cur.kq[1][ks]);
+                    pkq[vt] = STATE ? mma3(ah, al, bh, bl, pkq[vt]) : mma3(bh, bl, ah, al, pkq[vt]);
+                }
+                if constexpr (STATE) {
+#pragma unroll
+                    for (int part = 0; part < 2; part++)
+                        *reinterpret_cast<u32x4 *>(lds + L::KIMG + part * L::K_BYTES + (16 * wave + n) * 256 + ((4 * ks + j) ^ L::key_piece(n)) * 16) = cur.kq[part][ks];
+                    __builtin_amdgcn_sched_barrier(0);
+                    request_kq_step(wk, ks, cur);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        };
+#pragma unroll
+        for (int vt = 0; vt < NT; vt++) pkq[vt] = floatx4{0, 0, 0, 0};
+        // C layout: lane (n, j) holds dv = 16 vt + n of tokens t = 16 wave + 4j + i (second team: dv = 16 vt + 4j + i of
+        // token 16 wave + n)
+        floatx4 gk4 = {0, 0, 0, 0};
+        float glast = 0.0f;
+        if constexpr (STATE) {
+            const floatx4 gam4 = *reinterpret_cast<const floatx4 *>(gam + 16 * wave + 4 * j);
+            gk4 = *reinterpret_cast<const floatx4 *>(gam + C + 16 * wave + 4 * j);
+            glast = gam[C - 1];
+            float v4[NT][4];
+#pragma unroll
+            for (int vt = 0; vt < NT; vt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) v4[vt][i] = v_lds[(16 * wave + 4 * j + i) * DV + 16 * vt + n];
+            by_state();
+#pragma unroll
+            for (int vt = 0; vt < NT; vt++) {
+                // R = V - e^c (K S0^T), as the [dv][token] image
+                half4 rh, rl;
+                split4([&](int i) { return v4[vt][i] - gam4[i] * pkq[vt][i]; }, rh, rl);
+                const int at = (16 * vt + n) * TROW + 16 * wave + 4 * j;
+                *reinterpret_cast<half4 *>(img_w(L::RH) + at) = rh, *reinterpret_cast<half4 *>(img_w(L::RL) + at) = rl;
+            }
+        }
+        if constexpr (!STATE) {
+            outputs(blk - 1, blk > 0, next);
+            if constexpr (AHEAD) touch(blk + AHEAD_BLOCKS, cur);
+        }
+        __syncthreads();  // R and the block's keys are whole
         // The left operands of the state's update, K by key dim: lane (n, j) wants key dim 32 wave + 16 nt + n, tokens
         // 32 ks + 8j .. + 7.  The transposing read works on 16 lanes: lane a + 4e of them names 8 bytes (4 values of a row),
         // and lane 4a + c receives value c of the lanes a, a + 4, a + 8, a + 12.  So lane a + 4e names token .. + e, key
         // dims .. + 4a .. + 3, and lane n = 4a + c receives key dim .. + n of four tokens in a row; two reads an operand.
-        // They are asked for here, two barriers before their use, behind the state's image and beside the arithmetic of R.
+        // They are asked for behind R, a barrier before their use.
         half4 xr[2][2][2][2];  // [hi | lo][nt][k-step][tokens + 0 | + 4]
-        if constexpr (STATE) {
-            const uint32_t la = lane & 3, le = (lane >> 2) & 3;
-            const unsigned char *kbase = lds + L::KIMG + (blk & 1) * 2 * K_IMG;
+        auto read_keys = [&]() {
+            const uint32_t la = lane & 3, le = (lane >> 2) & 3, x = (4 * wave + (la >> 1)) ^ L::key_piece(8 * (j & 1) + le);
+            const unsigned char *kbase = lds + L::KIMG + (8 * j + le) * 256 + (la & 1) * 8;
 #pragma unroll
             for (int part = 0; part < 2; part++) {
 #pragma unroll
@@ -707,55 +819,38 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
                     for (int ks = 0; ks < 2; ks++) {
 #pragma unroll
                         for (int hf = 0; hf < 2; hf++) {
-                            xr[part][nt][ks][hf] = read_transposed(kbase + part * K_IMG + ((32 * ks + 8 * j + 4 * hf + le) * KROW + 32 * wave + 16 * nt + 4 * la) * 2);
+                            xr[part][nt][ks][hf] = read_transposed(kbase + part * L::K_BYTES + (32 * ks + 4 * hf) * 256 + (x ^ (2 * nt + hf)) * 16);
                         }
                     }
                 }
             }
-        }
-        // C layout: lane (n, j) holds dv = 16 vt + n of tokens t = 16 wave + 4j + i (second team: dv = 16 vt + 4j + i of
-        // token 16 wave + n)
-        const floatx4 gam4 = *reinterpret_cast<const floatx4 *>(gam + 16 * wave + 4 * j);
-        const floatx4 gk4 = *reinterpret_cast<const floatx4 *>(gam + C + 16 * wave + 4 * j);
-        const float glast = gam[C - 1], gam_t = gam[16 * wave + n];
-        if constexpr (STATE) {
-#pragma unroll
-            for (int vt = 0; vt < NT; vt++) {
-                // R = V - e^c (K S0^T), as the [dv][token] image
-                half4 rh, rl;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    _Float16 hi, lo;
-                    split2(v_lds[(16 * wave + 4 * j + i) * DV + 16 * vt + n] - gam4[i] * pkq[vt][i], hi, lo);
-                    rh[i] = hi, rl[i] = lo;
-                }
-                const int at = (16 * vt + n) * TROW + 16 * wave + 4 * j;
-                *reinterpret_cast<half4 *>(img_w(L::RH) + at) = rh, *reinterpret_cast<half4 *>(img_w(L::RL) + at) = rl;
-            }
-        }
-        __syncthreads();  // R is whole
+        };
 
         if constexpr (STATE) {
             // ---- U = T R (T is lower triangular: k-steps up to the row tile's own) ----
 #pragma unroll
             for (int vt = 0; vt < NT; vt++) {
                 floatx4 u = {0, 0, 0, 0};
+                half8 r[2][2];  // [k-step][hi | lo]
 #pragma unroll
                 for (int ks = 0; ks < 2; ks++) {
                     if (ks > int(wave) / 2) continue;
                     const int bo = (16 * vt + n) * TROW + 32 * ks + 8 * j;
-                    u = mma3(__builtin_bit_cast(half8, cur.tm[0][ks]), __builtin_bit_cast(half8, cur.tm[1][ks]),
-                             *reinterpret_cast<const half8 *>(img(L::RH) + bo), *reinterpret_cast<const half8 *>(img(L::RL) + bo), u);
+                    r[ks][0] = *reinterpret_cast<const half8 *>(img(L::RH) + bo), r[ks][1] = *reinterpret_cast<const half8 *>(img(L::RL) + bo);
+                }
+                if (vt == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    read_keys();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int ks = 0; ks < 2; ks++) {
+                    if (ks > int(wave) / 2) continue;
+                    u = mma3(__builtin_bit_cast(half8, cur.tm[0][ks]), __builtin_bit_cast(half8, cur.tm[1][ks]), r[ks][0], r[ks][1], u);
                 }
                 half4 uh, ul, wh, wl;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    _Float16 hi, lo;
-                    split2(u[i], hi, lo);
-                    uh[i] = hi, ul[i] = lo;
-                    split2(u[i] * gk4[i], hi, lo);  // scaled by e^{c_last - c_t} for the state
-                    wh[i] = hi, wl[i] = lo;
-                }
+                split4([&](int i) { return u[i]; }, uh, ul);
+                split4([&](int i) { return u[i] * gk4[i]; }, wh, wl);  // scaled by e^{c_last - c_t} for the state
                 const int at = (16 * vt + n) * TROW + 16 * wave + 4 * j;
                 *reinterpret_cast<half4 *>(img_w(L::UH) + at) = uh, *reinterpret_cast<half4 *>(img_w(L::UL) + at) = ul;
                 *reinterpret_cast<half4 *>(img_w(L::WH) + at) = wh, *reinterpret_cast<half4 *>(img_w(L::WL) + at) = wl;
@@ -763,6 +858,12 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
             __builtin_amdgcn_sched_barrier(0);
             request_tm(blk + 2, cur);
             __builtin_amdgcn_sched_barrier(0);
+        } else {
+            // (here, where the first team does not want the LDS that both teams' reads of the state's image would share)
+            by_state();
+            held_gam = gam[16 * wave + n];
+#pragma unroll
+            for (int vt = 0; vt < NT; vt++) held[vt] = pkq[vt];
         }
         __syncthreads();  // U is whole; every wave is through with the state's image, the values and the factors
 
@@ -793,42 +894,21 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
             publish_state();
             place(nxt, next);
         } else {
-            // ---- O = (e^c (Q S0^T) + M U) / sqrt(128) ----
-            floatx4 mu[NT];
-#pragma unroll
-            for (int vt = 0; vt < NT; vt++) {
-                mu[vt] = floatx4{0, 0, 0, 0};
-#pragma unroll
-                for (int ks = 0; ks < 2; ks++) {
-                    if (ks > int(wave) / 2) continue;
-                    const int bo = (16 * vt + n) * TROW + 32 * ks + 8 * j;
-                    mu[vt] = mma3(*reinterpret_cast<const half8 *>(img(L::UH) + bo), *reinterpret_cast<const half8 *>(img(L::UL) + bo),
-                                  __builtin_bit_cast(half8, cur.tm[0][ks]), __builtin_bit_cast(half8, cur.tm[1][ks]), mu[vt]);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            request_tm(blk + 2, cur);
-            __builtin_amdgcn_sched_barrier(0);
-            const uint32_t tok = blk * C + 16 * wave + n;
-            if (tok < a.tokens) {
-                float *o = a.o + (size_t(tok) * a.v_heads + h) * a.v_dim + DV * slice + 4 * j;
-#pragma unroll
-                for (int vt = 0; vt < NT; vt++) {
-#pragma unroll
-                    for (int i = 0; i < 4; i++) o[16 * vt + i] = Q_SCALE * (gam_t * pkq[vt][i] + mu[vt][i]);
-                }
-            }
+            request_kq(blk + 2, cur);
         }
     };
     // (two sets of operand registers that change roles, so that nothing is copied from one to the other)
     auto walk = [&](auto team) {
         constexpr bool STATE = decltype(team)::value;
         ChainBlock even, odd;
+        even.touched[0] = even.touched[1] = odd.touched[0] = odd.touched[1] = 0;
         // (in the order the blocks ask in, so that the first blocks' waits are those of every block)
         if constexpr (STATE) request_values(0, even);
         request_kq(0, even), request_tm(0, even);
         if constexpr (STATE) request_values(1, odd);
-        request_kq(1, odd), request_tm(1, odd);
+        request_kq(1, odd);
+        if constexpr (STATE) request_tm(1, odd);
+        else odd.tm[0][0] = odd.tm[0][1] = odd.tm[1][0] = odd.tm[1][1] = u32x4{0, 0, 0, 0};
         if constexpr (STATE) {
             publish_state();
             place(0, even);
@@ -841,6 +921,7 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
             step(team, blk + 1, odd, even);
         }
         if (blk < nblocks) step(team, blk, even, odd);
+        if constexpr (!STATE) outputs(nblocks - 1, true, nblocks % 2 ? even : odd);
     };
     // (the first team is the chain: where both teams' waves of a SIMD are ready, its go first)
     if (state_team) {
@@ -869,8 +950,10 @@ int setup_deltanet_chunk() {
     for (const auto &[kernel, bytes] : prepares) {
         if (int rc = int(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes))) return rc;
     }
-    return int(hipFuncSetAttribute(reinterpret_cast<const void *>(deltanet_chunk_chain_kernel),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, ChainLds::BYTES));
+    for (const void *kernel : {reinterpret_cast<const void *>(deltanet_chunk_chain_kernel<false>), reinterpret_cast<const void *>(deltanet_chunk_chain_kernel<true>)}) {
+        if (int rc = int(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, ChainLds::BYTES))) return rc;
+    }
+    return 0;
 }
 
 size_t deltanet_chunk_workspace_bytes(const saetta_rows_step_params &p) {
@@ -930,7 +1013,8 @@ int run_deltanet_chunk(hipStream_t stream, const float *mixed, const float *a, c
     } else {
         launch(deltanet_chunk_prepare_kernel<1, false>, dim3(nblocks, p.v_heads), PREP_THREADS, PrepLds<1>::BYTES, stream, args, conv_out);
     }
-    launch(deltanet_chunk_chain_kernel, dim3(p.v_dim / DV * p.v_heads), 512, ChainLds::BYTES, stream, args);
+    const bool ahead = size_t(p.tokens) * channels * sizeof(float) + deltanet_chunk_workspace_bytes(p) >= AHEAD_FROM;
+    launch(ahead ? deltanet_chunk_chain_kernel<true> : deltanet_chunk_chain_kernel<false>, dim3(p.v_dim / DV * p.v_heads), 512, ChainLds::BYTES, stream, args);
     return SAETTA_OK;
 }
 

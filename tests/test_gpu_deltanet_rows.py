@@ -334,6 +334,32 @@ def test_conv_of_four_channels_a_thread_at_the_edges_of_its_tiles(tokens):
     check_against_oracle(Layer(2, 4, 16, 4, seed=tokens), 2 * tokens, [tokens, tokens], snapshots=True)
 
 
+@pytest.mark.parametrize("k_heads,v_heads,v_dim,first,second", [(16, 32, 128, 3264, 129), (8, 16, 256, 5248, 190), (32, 32, 64, 2368, 131)])
+def test_a_chunk_past_the_memorys_cache_equals_its_pieces(k_heads, v_heads, v_dim, first, second):
+    # From 208 MB of `mixed` and workspace on, the chain's operands are brought into L2 ahead of their use: the one call is past that
+    # line, its two pieces, cut between two blocks, are below it.  The arithmetic is the same, so the bits are.
+    layer = Layer(k_heads, v_heads, v_dim, 4, seed=first)
+    tokens = first + second
+    gen = torch.Generator(device="cuda").manual_seed(first)
+    x, z, a, b = (torch.randn(tokens, n, generator=gen, device="cuda") for n in (layer.channels, layer.val, v_heads, v_heads))
+    weights = [dev(w) for w in (layer.conv_w, layer.a_log, layer.dt_bias, layer.norm)]
+
+    def run(pieces):
+        conv, state = layer.zero_state()
+        mixed, y, at = torch.empty_like(x), torch.empty_like(z), 0
+        for n in pieces:
+            i, at = slice(at, at + n), at + n
+            plan = saetta.Plan()
+            saetta.deltanet_conv_rows(plan, x[i], weights[0], conv, mixed[i], layer.channels, layer.kernel, n)
+            saetta.deltanet_rows(plan, mixed[i], a[i], b[i], weights[1], weights[2], state, z[i], weights[3], y[i], k_heads, v_heads, v_dim, n, EPS)
+            plan.build().run()
+            torch.cuda.synchronize()
+        return mixed, y, conv, state
+
+    for one, two in zip(run([tokens]), run([first, second])):
+        assert torch.isfinite(one).all() and torch.equal(one, two)
+
+
 def test_rejections():
     z = torch.zeros(4096, device="cuda")
     plan = saetta.Plan()
