@@ -76,21 +76,12 @@ struct ChunkArgs {
 constexpr int CONV = 4;     // taps of the conv that the prepare kernel makes
 constexpr int CONV_V = 128;  // ... and the value dim it takes
 
-// x as an f16 hi part and an f16 lo part.  The lo part has to complete the hi part that is stored: where x is
+// Four values as f16 hi parts and f16 lo parts.  A lo part has to complete the hi part that is stored: where x is
 // a product, the compiler may round the exact product to f16 for the one and the f32 product for the other, and
 // next to a midpoint between two f16 numbers the two roundings differ by an ulp of the hi part (one value in
 // some thousands: an error of 2^-11 of it instead of 2^-22).  So x is pinned as the f32 number it is, and the
-// hi part as the number that the lo part is taken against.
-__device__ __forceinline__ void split2(float x, _Float16 &hi, _Float16 &lo) {
-    asm volatile("" : "+v"(x));
-    float h = (float)(_Float16)x;
-    asm volatile("" : "+v"(h));
-    hi = (_Float16)h;  // (exact)
-    lo = (_Float16)(x - h);
-}
-
+// hi parts, two to a conversion, as the numbers that the lo parts are taken against.
 typedef _Float16 half2_ __attribute__((ext_vector_type(2)));
-// The same of four values, two to a conversion; a lo part is what one multiply-add leaves of x and the hi part as stored.
 template <class F>
 __device__ __forceinline__ void split4(F &&value, half4 &hi, half4 &lo) {
     half2_ h[2], l[2];
@@ -101,7 +92,7 @@ __device__ __forceinline__ void split4(F &&value, half4 &hi, half4 &lo) {
         uint32_t both = __builtin_bit_cast(uint32_t, half2_{(_Float16)x, (_Float16)y});
         asm("" : "+v"(both));
         h[p] = __builtin_bit_cast(half2_, both);
-        l[p] = half2_{(_Float16)__builtin_fmaf((float)h[p][0], -1.0f, x), (_Float16)__builtin_fmaf((float)h[p][1], -1.0f, y)};
+        l[p] = half2_{(_Float16)(x - (float)h[p][0]), (_Float16)(y - (float)h[p][1])};
     }
     hi = __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3), lo = __builtin_shufflevector(l[0], l[1], 0, 1, 2, 3);
 }
@@ -331,18 +322,15 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
         const float qi = __builtin_amdgcn_rsqf(qs + a.eps), ki = __builtin_amdgcn_rsqf(ks + a.eps);
 #pragma unroll
         for (int i = 0; i < 4; i += 2) {
-            half8 a_qh, a_ql, a_kh, a_kl;
+            half4 h[2][2], l[2][2];  // [q | k][half of the piece]
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float4 qq = qv[i + e / 4], kk = kv[i + e / 4];
-                const float qf = real ? (e % 4 == 0 ? qq.x : e % 4 == 1 ? qq.y : e % 4 == 2 ? qq.z : qq.w) * qi : 0.0f;
-                const float kf = real ? (e % 4 == 0 ? kk.x : e % 4 == 1 ? kk.y : e % 4 == 2 ? kk.z : kk.w) * ki : 0.0f;
-                _Float16 hi, lo;
-                split2(qf, hi, lo);
-                a_qh[e] = hi, a_ql[e] = lo;
-                split2(kf, hi, lo);
-                a_kh[e] = hi, a_kl[e] = lo;
+            for (int e = 0; e < 2; e++) {
+                const float4 qq = qv[i + e], kk = kv[i + e];
+                split4([&](int c) { return real ? (c == 0 ? qq.x : c == 1 ? qq.y : c == 2 ? qq.z : qq.w) * qi : 0.0f; }, h[0][e], l[0][e]);
+                split4([&](int c) { return real ? (c == 0 ? kk.x : c == 1 ? kk.y : c == 2 ? kk.z : kk.w) * ki : 0.0f; }, h[1][e], l[1][e]);
             }
+            auto joined = [](const half4 (&x)[2]) { return __builtin_shufflevector(x[0], x[1], 0, 1, 2, 3, 4, 5, 6, 7); };
+            const half8 a_qh = joined(h[0]), a_ql = joined(l[0]), a_kh = joined(h[1]), a_kl = joined(l[1]);
             const uint32_t piece = part + 4 * i;  // key dims 8 piece ..: k-step piece / 4, lane group piece % 4 of an operand
             const int at = t * KROW + 8 * piece;
             *reinterpret_cast<half8 *>(kh + at) = a_kh, *reinterpret_cast<half8 *>(kl + at) = a_kl;
@@ -400,12 +388,7 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
                 *reinterpret_cast<floatx4 *>(diag_lds(hh, nt >> 1) + (t & 31) * DROW + (s0 & 31)) = floatx4{x[0], x[1], x[2], x[3]};
             } else {  // M | the block of A below the diagonal, as an MFMA operand
                 half4 hi, lo;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    _Float16 h, l;
-                    split2(x[i], h, l);
-                    hi[i] = h, lo[i] = l;
-                }
+                split4([&](int i) { return x[i]; }, hi, lo);
                 _Float16 *dst = team == 0 ? half_img(hh, L::LBA_OFF) + (t - 32) * HROW + s0 : m_lds(hh) + t * TROW + s0;
                 *reinterpret_cast<half4 *>(dst) = hi;
                 *reinterpret_cast<half4 *>(dst + (team == 0 ? 32 * HROW : C * TROW)) = lo;
@@ -462,14 +445,8 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
         const floatx4 x = *reinterpret_cast<const floatx4 *>(diag_lds(hh, half) + t * DROW + c);
         const floatx4 beta = *reinterpret_cast<const floatx4 *>(beta_lds(hh) + 32 * half + c);
         half4 th, tl, xh, xl;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            _Float16 h, l;
-            split2(x[e] * beta[e], h, l);
-            th[e] = h, tl[e] = l;
-            split2(x[e], h, l);
-            xh[e] = h, xl[e] = l;
-        }
+        split4([&](int e) { return x[e] * beta[e]; }, th, tl);
+        split4([&](int e) { return x[e]; }, xh, xl);
         _Float16 *dst = m_lds(hh) + (32 * half + t) * TROW + 32 * half + c;
         *reinterpret_cast<half4 *>(dst) = th, *reinterpret_cast<half4 *>(dst + C * TROW) = tl;
         if (half) {
@@ -492,12 +469,7 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
                                    *reinterpret_cast<const half8 *>(half_img(hs, L::LBA_OFF) + 32 * HROW + ao), floatx4{0, 0, 0, 0});
             // (the inverses of the diagonal blocks were last read before the barrier above)
             half4 wh, wl;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                _Float16 h, l;
-                split2(w[i], h, l);
-                wh[i] = h, wl[i] = l;
-            }
+            split4([&](int i) { return w[i]; }, wh, wl);
             *reinterpret_cast<half4 *>(half_img(hs, L::W_OFF) + at) = wh, *reinterpret_cast<half4 *>(half_img(hs, L::W_OFF) + 32 * HROW + at) = wl;
         }
         __syncthreads();
@@ -507,12 +479,7 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
             const floatx4 tba = mma3(bh, bl, *reinterpret_cast<const half8 *>(half_img(hs, L::XBB_OFF) + ao),
                                      *reinterpret_cast<const half8 *>(half_img(hs, L::XBB_OFF) + 32 * HROW + ao), floatx4{0, 0, 0, 0});
             half4 th, tl;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                _Float16 h, l;
-                split2(-tba[i], h, l);
-                th[i] = h, tl[i] = l;
-            }
+            split4([&](int i) { return -tba[i]; }, th, tl);
             _Float16 *dst = m_lds(hs) + (32 + 16 * r + n) * TROW + 16 * ct + 4 * j;
             *reinterpret_cast<half4 *>(dst) = th, *reinterpret_cast<half4 *>(dst + C * TROW) = tl;
         }
