@@ -857,15 +857,14 @@ __global__ __launch_bounds__(MERGE_THREADS * TEAMS, 4) void prefill_merge_kernel
 // A chunk of 166 tokens is 22 workgroups of the kernel above, which then walk their 166 keys in three steps behind a
 // prologue and an epilogue of 7 us, and the prepare kernel is 3.8 us more before them: 22 us in all for 2 us of work.
 // Here a workgroup takes ONE row group (4 tokens x 8 heads = 32 rows) of a kv head, eight times as many workgroups, and
-// its 8 waves take alternate blocks of 32 keys, so that 256 keys are one step; each wave keeps its own (m, l, O) and they
-// are joined at the end, each wave finishing 32 of the 256 dims.  Nothing of a block is shared between waves, so the
+// its 8 waves take alternate blocks of 32 keys, so that 256 keys are one round; each wave finishes 32 of the 256 dims.  The
 // cache is read where it lies, once per row group: the keys go from memory to MFMA operands in registers, the values to a
 // tile of the wave's own in LDS, row by row as in memory, and come back transposed (ds_read_b64_tr_b16).  Codes are
 // dequantized on the way, with the arithmetic of the prepare kernel.
 // The price is that every row group pulls (and dequantizes) the keys for itself: with many tokens the tiles of 16 and their
 // images win, and with few over a long context a row group's keys go to several workgroups (SPLIT), whose parts the
 // tiles' merge joins; the lines are in choose_small.
-// What bounds a block of halves per wave (4 us for the eight of them): 256 KB through the CU's 64 bytes a cycle are 1.8 of
+// What bounds a block of halves per wave, each with all dims of its own blocks (4 us for the eight of them): 256 KB through the CU's 64 bytes a cycle are 1.8 of
 // them, the values' way through LDS and the query operands 1.4.  A key's operands straight from its row, 16 bytes a lane,
 // took 5.3 us: such a load is taken a row a cycle, and so four lanes fetch 64 bytes of a row together and turn four rows
 // round in registers.  Codes (4 us, once for every row group): vector instructions, of which a pair of codes is
@@ -874,13 +873,24 @@ __global__ __launch_bounds__(MERGE_THREADS * TEAMS, 4) void prefill_merge_kernel
 // Measured, the whole call, tiles -> this: halves, 16 tokens at 16 18.3 -> 7.5 us, 166 from 0 21.7 -> 10.8; fetched row by
 // row -> in turns: 16 at 500 20.5 -> 18.6, 300 from 0 19.1 -> 17.4, 500 from 0 23.1 -> 20.5, 500 at 500 32.2 -> 26.5; codes as f32 -> as halves: 8-bit
 // 23.8 -> 20.2, 24.9 -> 21.8, 34.4 -> 28.8, 4-bit 23.3 -> 20.2, 23.4 -> 21.4, 33.3 -> 29.4, and no further from 64 bits.
-// Halves fill the registers: what depends on the lane alone is made anew where it is used (`at`), so that nothing spills; three
-// spilled registers cost a launch 1 us (300 from 0 18.3), the instructions 0.1 to 0.5 (16 at 500 18.1).  8-bit codes spill four, stored
-// before the loop and read back behind it.
-// One maximum for the eight blocks of a round, a wave 32 of the dims of all of them and nothing to join at the end took 1
-// to 2.5 us less with codes, but not with its precision: of each block the largest probability is now 1, without a
-// rounding, and with the largest of eight blocks alone an output was up to 1.2 times as far from 64 bits.
+// Halves fill the registers there: what depends on the lane alone is made anew where it is used (`at`), so that nothing spills; three
+// spilled registers cost a launch 1 us (300 from 0 18.3), the instructions 0.1 to 0.5 (16 at 500 18.1).
+// One maximum for the eight blocks of a round was faster with codes, but not with this precision: of each block the largest probability
+// is now 1, without a rounding, and with the largest of eight blocks alone an output was up to 1.2 times as far from 64 bits.
 constexpr int SMALL_WAVES = 8, SMALL_THREADS = 64 * SMALL_WAVES;
+// How the waves divide the work on O.  OWN_BLOCKS: each all dims of its own blocks, joined at the end through LDS: 32 KB a wave
+// written and read, in two rounds, 3000 of the 13900 cycles that a workgroup of 166 tokens took, and 128 registers of sums that
+// the scores and the loads have to do without.  ONE_ROUND, SHARED_ROUNDS: the waves make the probabilities of a round's
+// eight blocks, relative to each block's own maximum, and hand them round (2 KB a block); then each makes 32 dims of O over all of them, 16
+// registers, with 2^(m_b - m) a factor of the block's product in 32 bits.  Nothing is joined, the values travel under the scores and
+// the queries stay in registers, but a round's loads wait for the end of the round before, and its phases don't overlap.
+// Whole call, us, OWN_BLOCKS -> ONE_ROUND (8 blocks at most): 166 from 0 13.4 -> 10.8 (halves), 14.7 -> 12.7 (8-bit), 14.8 -> 12.7 (4-bit); in parts of 8
+// blocks, 10 at 3000, 17.7 -> 15.0, 19.5 -> 17.0, 19.2 -> 16.7.  -> SHARED_ROUNDS, halves: 300 from 0 16.8 -> 14.0, 700 25.4 -> 22.2, 900 32.2 -> 29.0,
+// 30 at 500 17.8 -> 16.8, 500 at 300 23.4 -> 23.5, 500 at 800 29.7 -> 32.1; 4-bit: 300 from 0 17.6 -> 16.8, 520 21.8 -> 21.9, 766 28.7 -> 25.7, 30 at
+// 500 20.2 -> 20.2, 500 at 300 25.5 -> 26.7; 8-bit spills 26 registers that way (300 from 0 17.8 -> 18.9) and has none.  So the line lies at the
+// keys that a row group sees in the mean.  Distance from 64 bits: the same or less (halves, 500 at 300: 1.66e-4 -> 1.13e-4).
+constexpr int OWN_BLOCKS = 0, ONE_ROUND = 1, SHARED_ROUNDS = 2;
+constexpr uint32_t SHARED_KEYS_HALF = 544, SHARED_KEYS_4 = 464;
 
 struct SmallArgs {
     const uint16_t *q;  // f16 [tokens][heads][256]
@@ -895,16 +905,18 @@ struct SmallArgs {
     float *part_o, *part_ml;
 };
 
-template <int BITS>
+template <int BITS, bool SHARED>
 struct SmallLds {
     // the values of a wave's block: f16 rows as in memory.  Codes: rows of 576 bytes, halves (copied in by 16-byte pieces in
     // whole kilobytes): rows of 512 rotated by 64 bytes per row; either way the four rows of a transposing read, 32 bytes
     // each, and those of its neighbours fall on different banks.
-    static constexpr int VROW = BITS == 16 ? 512 : 576;
+    static constexpr int VROW = BITS == 16 || SHARED ? 512 : 576;
     static constexpr int VTILE = BK * VROW;
     static constexpr int Q_OFF = 0, V_OFF = 16 * 1024;
+    // SHARED: the blocks' probabilities, two operands of 64 lanes x 16 bytes each, take the place of a tile or of the queries
+    static_assert(SMALL_WAVES * 2 * 64 * 16 <= VTILE && SMALL_WAVES * 2 * 64 * 16 <= V_OFF, "the probabilities");
     // the merge, over both: four waves' O at a time, [wave][8 dim tiles][4][64 lanes][16 bytes], and [wave][row][m, l]
-    static constexpr int ML_OFF = 4 * 32 * 1024;
+    static constexpr int ML_OFF = SHARED ? V_OFF + SMALL_WAVES * VTILE : 4 * 32 * 1024;
     static constexpr int MERGE_BYTES = ML_OFF + SMALL_WAVES * 32 * 8;
     static constexpr int TILES_BYTES = V_OFF + SMALL_WAVES * VTILE;
     static constexpr int BYTES = TILES_BYTES > MERGE_BYTES ? TILES_BYTES : MERGE_BYTES;
@@ -920,11 +932,17 @@ __device__ __forceinline__ uint32_t small_place(uint32_t u) {
     return st * 1024 + hf * 512;
 }
 
-template <int BITS, bool SPLIT>
+template <int BITS, bool SPLIT, int ROUNDS>
 __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallArgs a) {
-    using L = SmallLds<BITS>;
+    constexpr bool ONE = ROUNDS == ONE_ROUND, SHARED = ROUNDS != OWN_BLOCKS;
+    using L = SmallLds<BITS, SHARED>;
     constexpr int RB = row_bytes<BITS>(), PIECES = RB / 16, STEPS = 16 / BITS, VALUES = 128 / BITS;  // pieces of a row; values of one
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    if constexpr (SHARED) {  // (every argument is asked for here, in one trip: the compiler asks for each where it is used)
+        asm volatile("" ::"s"(a.q), "s"(a.kdata), "s"(a.vdata), "s"(a.q_and_gate), "s"(a.out), "s"(a.heads), "s"(a.kv_heads), "s"(a.pos), "s"(a.tokens), "s"(a.scale));
+        if constexpr (BITS != 16) asm volatile("" ::"s"(a.kscales), "s"(a.kbiases), "s"(a.vscales), "s"(a.vbiases));
+        if constexpr (SPLIT) asm volatile("" ::"s"(a.part_blocks), "s"(a.nparts), "s"(a.part_o), "s"(a.part_ml));
+    }
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hf = lane >> 5;
     const uint32_t kvh = a.kv_heads, groups = (a.tokens + 3) / 4;
@@ -988,22 +1006,23 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
             kzs = *reinterpret_cast<const u32x2 *>(a.kbiases + row * 4);
         }
     };
+    // halves: load u of the block's values, straight to the tile: place p of row k holds piece p - 4 (k % 4)
+    auto fetch_value = [&](uint32_t b, int u, uint32_t at) {
+        const uint32_t k = 2 * u + (at >> 5);
+        const uint64_t src = reinterpret_cast<uint64_t>(a.vdata) + row_of(b * BK + k) * RB + ((at - 4 * (k & 3)) & 31) * 16;
+        asm volatile("s_mov_b32 m0, %0\n"
+                     "s_nop 0\n"
+                     "global_load_lds_dwordx4 %1, off\n"
+                     :
+                     : "s"(vtile + u * 1024), "v"(src)
+                     : "memory", "m0");
+    };
     auto fetch_values = [&](uint32_t b) {
         if constexpr (BITS == 16) {
-            // straight to the tile: place p of row k holds piece p - 4 (k % 4)
             uint32_t at = lane;
             asm volatile("" : "+v"(at));
 #pragma unroll
-            for (int u = 0; u < V_LOADS; u++) {
-                const uint32_t k = 2 * u + (at >> 5);
-                const uint64_t src = reinterpret_cast<uint64_t>(a.vdata) + row_of(b * BK + k) * RB + ((at - 4 * (k & 3)) & 31) * 16;
-                asm volatile("s_mov_b32 m0, %0\n"
-                             "s_nop 0\n"
-                             "global_load_lds_dwordx4 %1, off\n"
-                             :
-                             : "s"(vtile + u * 1024), "v"(src)
-                             : "memory", "m0");
-            }
+            for (int u = 0; u < V_LOADS; u++) fetch_value(b, u, at);
             // (loads into registers and into LDS do not come back in one order, and the compiler counts only the former:
             // all that is out is waited for here, in front of anything it may do with the keys)
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1044,30 +1063,10 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
         }
     };
 
-    if (uint32_t(wave) < active) fetch_keys(first + wave);
-    // Q^T operands: through LDS, where all waves read them.  Wave w fetches 64 bytes of each row, four lanes a row.
-    {
-        half8 qv[2];
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const uint32_t r = 16 * i + (lane >> 2);
-            qv[i] = *reinterpret_cast<const half8 *>(a.q + (size_t(min(tok0 + (r >> 3), a.tokens - 1)) * a.heads + kv * SAETTA_GQA_GROUP + (r & 7)) * DIM + 32 * wave + 8 * (lane & 3));
-        }
-        if (uint32_t(wave) < active) fetch_values(first + wave);
-#pragma unroll
-        for (int i = 0; i < 2; i++) *reinterpret_cast<half8 *>(lds + L::Q_OFF + small_place<BITS>(4 * wave + (lane & 3)) + (16 * i + (lane >> 2)) * 16) = qv[i];
-    }
-    lds_barrier();
-
-    floatx16 acc[8];
-#pragma unroll
-    for (int mt = 0; mt < 8; mt++) {
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[mt][r] = 0.0f;
-    }
-    float m = 0.25f * NO_SCORE * c, l = 0.0f;  // (above a masked score, as in the kernel above)
-    for (uint32_t b = first + wave; b < nblocks; b += SMALL_WAVES) {
-        // ---- S^T = K Q^T ----
+    typedef short short4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) short4 *LdsShort4;
+    // ---- S^T = K Q^T of the block whose keys are in registers ----
+    auto scores = [&](auto &&query) {
         floatx16 s;
 #pragma unroll
         for (int r = 0; r < 16; r++) s[r] = 0.0f;
@@ -1080,136 +1079,310 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
                 ks = kss[g >> 1] >> (16 * (g & 1)), kz = kzs[g >> 1] >> (16 * (g & 1));
             }
             if (BITS == 16 && st % 4 == 0) turn(&kreg[i], lane);
-            const half8 q = *reinterpret_cast<const half8 *>(lds + L::Q_OFF + st * 1024 + lane * 16);
-            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(eight(kreg[i], st % STEPS, ks, kz), q, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(eight(kreg[i], st % STEPS, ks, kz), query(st), s, 0, 0, 0);
         }
-        if (b + SMALL_WAVES < nblocks) fetch_keys(b + SMALL_WAVES);
-        // ---- softmax: register r is key 4 hf + r % 4 + 8 (r / 4) of the block, the lane's row col ----
+        return s;
+    };
+    // register r of a block's scores is key 4 hf + r % 4 + 8 (r / 4) of the block, the lane's row col
+    auto mask = [&](floatx16 &s, uint32_t b) {
         const uint32_t key0 = b * BK;
         if (key0 + BK > a.pos + tok0 + 1) {
             const uint32_t len = a.pos + tok + 1, vis = len > key0 ? len - key0 : 0;
 #pragma unroll
             for (int r = 0; r < 16; r++) s[r] = uint32_t(4 * hf + (r & 3) + 8 * (r >> 2)) < vis ? s[r] : NO_SCORE;
         }
-        float bm = s[0];
+    };
+    // the operand of k-step sp, its sum added to l
+    auto probabilities = [&](const floatx16 &s, int sp, float m, float &l) {
+        uint32_t w[4];
 #pragma unroll
-        for (int r = 1; r < 16; r++) bm = fmaxf(bm, s[r]);
-        bm = fmaxf(max_across_halves(bm) * c, NO_SCORE);
-        if (__any(bm > m + TAU)) {
-            const float m_new = bm > m + TAU ? bm : m, alpha = __builtin_amdgcn_exp2f(m - m_new);
-            m = m_new, l *= alpha;
-#pragma unroll
-            for (int mt = 0; mt < 8; mt++) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[mt][r] *= alpha;
-            }
+        for (int i = 0; i < 4; i++) {
+            const float x = __builtin_amdgcn_exp2f(fmaf(s[8 * sp + 2 * i], c, -m)), y = __builtin_amdgcn_exp2f(fmaf(s[8 * sp + 2 * i + 1], c, -m));
+            l += x + y;
+            w[i] = pack_half2(x, y);
         }
-        half8 p[2];
-        float sum = 0.0f;
-#pragma unroll
-        for (int sp = 0; sp < 2; sp++) {
-            uint32_t w[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float x = __builtin_amdgcn_exp2f(fmaf(s[8 * sp + 2 * i], c, -m)), y = __builtin_amdgcn_exp2f(fmaf(s[8 * sp + 2 * i + 1], c, -m));
-                sum += x + y;
-                w[i] = pack_half2(x, y);
-            }
-            p[sp] = __builtin_bit_cast(half8, u32x4{w[0], w[1], w[2], w[3]});
-        }
-        l += sum;
-        // ---- the values to the wave's tile (halves: they are there) ----
+        return __builtin_bit_cast(half8, u32x4{w[0], w[1], w[2], w[3]});
+    };
+    // codes: the block's values to the wave's tile
+    auto store_values = [&]() {
         if constexpr (BITS != 16) {
 #pragma unroll
             for (int u = 0; u < V_LOADS; u++) {
-                half8 *dst = reinterpret_cast<half8 *>(lds + L::V_OFF + wave * L::VTILE + (u * V_KEYS + vk) * L::VROW + vp * VALUES * 2);
+                const uint32_t in_row = SHARED ? (vp * VALUES * 2 + 64 * (vk & 3)) & 511 : vp * VALUES * 2;
+                half8 *dst = reinterpret_cast<half8 *>(lds + L::V_OFF + wave * L::VTILE + (u * V_KEYS + vk) * L::VROW + in_row);
 #pragma unroll
                 for (int sub = 0; sub < STEPS; sub++) dst[sub] = eight(vreg[u], sub, vss[u], vzs[u]);
             }
-            if (b + SMALL_WAVES < nblocks) fetch_values(b + SMALL_WAVES);
         }
-        // ---- O^T += V^T P^T: k-step sp, lane half hf: keys 16 sp + 4 hf .. + 3 and 8 further; a wave's LDS accesses run in order ----
-        uint32_t at = lane;
-        if (BITS == 16) asm volatile("" : "+v"(at));
-        const uint32_t e = (at >> 2) & 3, dim = ((at >> 4) & 1) * 16 + (at & 3) * 4;
-        const uint32_t vrow = vtile + (4 * (at >> 5) + e) * L::VROW;
-        typedef short short4 __attribute__((ext_vector_type(4)));
-        typedef __attribute__((address_space(3))) short4 *LdsShort4;
+    };
+    // What a wave finishes: O^T of dims 32 wave .. + 31, relative to `top`, with the sums l_all (the lane's row col)
+    floatx16 fin;
 #pragma unroll
-        for (int mt = 0; mt < 8; mt++) {
-            const uint32_t d = BITS == 16 ? ((32 * mt + dim) * 2 + 64 * e) & 511 : (32 * mt + dim) * 2;
-            u32x2 r[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) r[i] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<LdsShort4>(vrow + d + 8 * i * L::VROW)));
-#pragma unroll
-            for (int sp = 0; sp < 2; sp++) {
-                const half8 v = __builtin_bit_cast(half8, u32x4{r[2 * sp].x, r[2 * sp].y, r[2 * sp + 1].x, r[2 * sp + 1].y});
-                acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, p[sp], acc[mt], 0, 0, 0);
-            }
-        }
-        if constexpr (BITS == 16) {
-            // (what comes from memory into the tile is not in the order of the wave's LDS accesses: its reads have to be back)
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            if (b + SMALL_WAVES < nblocks) fetch_values(b + SMALL_WAVES);
-        }
-    }
-
-    // ---- the waves' parts joined: wave w finishes dims 32 w .. 32 w + 31 ----
+    for (int r = 0; r < 16; r++) fin[r] = 0.0f;
+    const float least = 0.25f * NO_SCORE * c;  // (above a masked score, as in the kernel above)
+    float top = SHARED ? least : 4.0f * NO_SCORE, l_all = 0.0f;
+    float2 *ml = reinterpret_cast<float2 *>(lds + L::ML_OFF);
     // Gates and outputs: lane l has dims 4 (l % 8) .. + 3 of those of rows 8 j + l / 8 (a row group's rows 8 j .. + 7 are a
     // token's), 128 bytes of a row a load or store.  16 bytes of each of 32 rows, as the accumulators lie, are taken a row a cycle.
     float4 g[4];
     const uint32_t in_token = (lane >> 3) * DIM + 32 * wave + 4 * (lane & 7);
     auto first_row = [&](int j) { return size_t(min(tok0 + j, a.tokens - 1)) * a.heads + kv * SAETTA_GQA_GROUP; };
-    if constexpr (!SPLIT) {
+    auto ask_gates = [&]() {
+        if constexpr (!SPLIT) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) g[j] = *reinterpret_cast<const float4 *>(a.q_and_gate + first_row(j) * 2 * DIM + DIM + ((lane >> 3) * DIM + in_token));
-    }
-    lds_barrier();  // every wave is through with its tile and the query operands
-    float2 *ml = reinterpret_cast<float2 *>(lds + L::ML_OFF);
-    const float l_row = l + __shfl_xor(l, 32);
-    if (hf == 0) ml[wave * 32 + col] = float2{m, l_row};
-    auto tile_of = [&](int w, int mt) { return reinterpret_cast<float4 *>(lds + (w & 3) * 32768 + mt * 4096) + lane; };
-    floatx16 fin;
+            for (int j = 0; j < 4; j++) g[j] = *reinterpret_cast<const float4 *>(a.q_and_gate + first_row(j) * 2 * DIM + DIM + ((lane >> 3) * DIM + in_token));
+        }
+    };
+
+    if constexpr (SHARED) {
+        // ---- the waves share the probabilities and the values of a round's blocks, and each makes 32 dims of O ----
+        // Q^T operands: to registers by way of LDS.  Wave w fetches 64 bytes of each row, four lanes a row.
+        half8 q[16];
+        {
+            half8 qv[2];
 #pragma unroll
-    for (int r = 0; r < 16; r++) fin[r] = 0.0f;
-    auto hand_out = [&]() {  // this wave's O, all dims
+            for (int i = 0; i < 2; i++) {
+                const uint32_t r = 16 * i + (lane >> 2);
+                qv[i] = *reinterpret_cast<const half8 *>(a.q + (size_t(min(tok0 + (r >> 3), a.tokens - 1)) * a.heads + kv * SAETTA_GQA_GROUP + (r & 7)) * DIM + 32 * wave + 8 * (lane & 3));
+            }
+            auto put = [&]() {
+#pragma unroll
+                for (int i = 0; i < 2; i++) *reinterpret_cast<half8 *>(lds + L::Q_OFF + small_place<BITS>(4 * wave + (lane & 3)) + (16 * i + (lane >> 2)) * 16) = qv[i];
+            };
+            if (uint32_t(wave) < active) {  // (each side with its own wait: behind a branch the compiler would wait for the keys too)
+                fetch_keys(first + wave);
+                put();
+                if constexpr (BITS != 16) fetch_values(first + wave);
+                asm volatile("; keys on their way" ::: "memory");
+            } else {
+                put();
+                asm volatile("; no keys" ::: "memory");
+            }
+            lds_barrier();
+            if constexpr (ONE) ask_gates();
+            if (uint32_t(wave) < active) {
+#pragma unroll
+                for (int st = 0; st < 16; st++) q[st] = *reinterpret_cast<const half8 *>(lds + L::Q_OFF + st * 1024 + lane * 16);
+            }
+            if (!ONE || active == SMALL_WAVES) lds_barrier();  // the probabilities go over them
+        }
+        // the blocks' probabilities: in the place of the last wave's values, or, where it has some, of the queries
+        const uint32_t p_at = !ONE || active == SMALL_WAVES ? L::Q_OFF : L::V_OFF + (SMALL_WAVES - 1) * L::VTILE;
+        for (uint32_t b0 = first;;) {
+            const uint32_t b = b0 + wave, here = ONE ? active : min(nblocks - b0, uint32_t(SMALL_WAVES));
+            const bool mine = uint32_t(wave) < here, more = !ONE && b + SMALL_WAVES < nblocks;
+            if (mine) {
+                if constexpr (BITS == 16) {
+                    // Loads into registers and into LDS do not come back in one order, and the compiler counts only the former: the
+                    // keys are waited for here, in front of the values, which travel under the scores.
+#pragma unroll
+                    for (int i = 0; i < PIECES / 2; i++) asm volatile("" : "+v"(kreg[i]));
+                }
+                if constexpr (BITS != 16) asm volatile("" : "+v"(kss), "+v"(kzs));  // (nothing of them before the queries have left)
+                floatx16 s = scores([&](int st) {
+                    if constexpr (BITS == 16) fetch_value(b, st, lane);  // (a load beside each product)
+                    return q[st];
+                });
+                if constexpr (BITS != 16) {
+                    if (more) fetch_keys(b + SMALL_WAVES);
+                }
+                mask(s, b);
+                // relative to the block's own maximum, so that a row's largest probability in it is 1, which f16 holds exactly
+                float m = s[0];
+#pragma unroll
+                for (int r = 1; r < 16; r++) m = fmaxf(m, s[r]);
+                m = fmaxf(max_across_halves(m) * c, least);
+                float l = 0.0f;
+#pragma unroll
+                for (int sp = 0; sp < 2; sp++) *reinterpret_cast<half8 *>(lds + p_at + (2 * wave + sp) * 1024 + lane * 16) = probabilities(s, sp, m, l);
+                l += __shfl_xor(l, 32);
+                if (hf == 0) ml[wave * 32 + col] = float2{m, l};
+                if constexpr (BITS != 16) {
+                    store_values();
+                    if (more) fetch_values(b + SMALL_WAVES);
+                } else {
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                }
+            }
+            lds_barrier();  // the probabilities and the values are in LDS
+            if constexpr (BITS == 16) {
+                if (more) fetch_keys(b + SMALL_WAVES);
+            }
+            if (!ONE && b0 + SMALL_WAVES >= nblocks) ask_gates();
+            // ---- O^T = sum over the blocks of 2^(m_b - top) V_b^T P_b^T ----
+            float weight[SMALL_WAVES];
+            {
+                float2 x[SMALL_WAVES];
+                const float before = top;
+#pragma unroll
+                for (int w = 0; w < SMALL_WAVES; w++) {
+                    x[w] = ml[w * 32 + col];
+                    if (uint32_t(w) >= here) x[w] = float2{4.0f * NO_SCORE, 0.0f};
+                    top = fmaxf(top, x[w].x);
+                }
+                if constexpr (!ONE) {
+                    const float alpha = __builtin_amdgcn_exp2f(before - top);
+                    l_all *= alpha;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) fin[r] *= alpha;
+                }
+#pragma unroll
+                for (int w = 0; w < SMALL_WAVES; w++) weight[w] = __builtin_amdgcn_exp2f(x[w].x - top), l_all += x[w].y * weight[w];
+            }
+            // k-step sp, lane half hf: keys 16 sp + 4 hf .. + 3 and 8 further
+            const uint32_t e = (lane >> 2) & 3, dim = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+            const uint32_t vrow = lds0 + L::V_OFF + (4 * hf + e) * L::VROW + (((32 * wave + dim) * 2 + 64 * e) & 511);
+            auto block = [&](uint32_t w) {
+                floatx16 t;
+#pragma unroll
+                for (int r = 0; r < 16; r++) t[r] = 0.0f;
+                u32x2 r[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) r[i] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<LdsShort4>(vrow + w * L::VTILE + 8 * i * L::VROW)));
+#pragma unroll
+                for (int sp = 0; sp < 2; sp++) {
+                    const half8 p = *reinterpret_cast<const half8 *>(lds + p_at + (2 * w + sp) * 1024 + lane * 16);
+                    const half8 v = __builtin_bit_cast(half8, u32x4{r[2 * sp].x, r[2 * sp].y, r[2 * sp + 1].x, r[2 * sp + 1].y});
+                    t = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, p, t, 0, 0, 0);
+                }
+                return t;
+            };
+#pragma unroll
+            for (int w = 0; w < SMALL_WAVES; w += 2) {
+                if (uint32_t(w) >= here) break;
+                if constexpr (!ONE) __builtin_amdgcn_sched_barrier(0);  // (no reads of the next pair's before this one's are used)
+                const floatx16 t0 = block(w);
+                if (uint32_t(w + 1) < here) {
+                    const floatx16 t1 = block(w + 1);
+#pragma unroll
+                    for (int r = 0; r < 16; r++) fin[r] += t0[r] * weight[w] + t1[r] * weight[w + 1];
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) fin[r] += t0[r] * weight[w];
+                }
+            }
+            if (ONE || (b0 += SMALL_WAVES) >= nblocks) break;
+            lds_barrier();  // the round has been read
+        }
+    } else {
+        if (uint32_t(wave) < active) fetch_keys(first + wave);
+        // Q^T operands: through LDS, where all waves read them.  Wave w fetches 64 bytes of each row, four lanes a row.
+        {
+            half8 qv[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const uint32_t r = 16 * i + (lane >> 2);
+                qv[i] = *reinterpret_cast<const half8 *>(a.q + (size_t(min(tok0 + (r >> 3), a.tokens - 1)) * a.heads + kv * SAETTA_GQA_GROUP + (r & 7)) * DIM + 32 * wave + 8 * (lane & 3));
+            }
+            if (uint32_t(wave) < active) fetch_values(first + wave);
+#pragma unroll
+            for (int i = 0; i < 2; i++) *reinterpret_cast<half8 *>(lds + L::Q_OFF + small_place<BITS>(4 * wave + (lane & 3)) + (16 * i + (lane >> 2)) * 16) = qv[i];
+        }
+        lds_barrier();
+
+        floatx16 acc[8];
 #pragma unroll
         for (int mt = 0; mt < 8; mt++) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) tile_of(wave, mt)[i * 64] = float4{acc[mt][4 * i], acc[mt][4 * i + 1], acc[mt][4 * i + 2], acc[mt][4 * i + 3]};
+            for (int r = 0; r < 16; r++) acc[mt][r] = 0.0f;
         }
-    };
-    float weight[SMALL_WAVES], l_all = 0.0f, top = 4.0f * NO_SCORE;
-    auto take_in = [&](int from) {  // the dims this wave finishes, from waves from .. from + 3
+        float m = least, l = 0.0f;
+        for (uint32_t b = first + wave; b < nblocks; b += SMALL_WAVES) {
+            floatx16 s = scores([&](int st) { return *reinterpret_cast<const half8 *>(lds + L::Q_OFF + st * 1024 + lane * 16); });
+            if (b + SMALL_WAVES < nblocks) fetch_keys(b + SMALL_WAVES);
+            mask(s, b);
+            float bm = s[0];
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
-            if (uint32_t(from + w) < active) {
+            for (int r = 1; r < 16; r++) bm = fmaxf(bm, s[r]);
+            bm = fmaxf(max_across_halves(bm) * c, NO_SCORE);
+            if (__any(bm > m + TAU)) {
+                const float m_new = bm > m + TAU ? bm : m, alpha = __builtin_amdgcn_exp2f(m - m_new);
+                m = m_new, l *= alpha;
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float4 x = tile_of(w, wave)[i * 64];
-                    fin[4 * i] += x.x * weight[from + w], fin[4 * i + 1] += x.y * weight[from + w];
-                    fin[4 * i + 2] += x.z * weight[from + w], fin[4 * i + 3] += x.w * weight[from + w];
+                for (int mt = 0; mt < 8; mt++) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[mt][r] *= alpha;
                 }
             }
+            half8 p[2];
+            float sum = 0.0f;
+#pragma unroll
+            for (int sp = 0; sp < 2; sp++) p[sp] = probabilities(s, sp, m, sum);
+            l += sum;
+            // ---- the values to the wave's tile (halves: they are there) ----
+            if constexpr (BITS != 16) {
+                store_values();
+                if (b + SMALL_WAVES < nblocks) fetch_values(b + SMALL_WAVES);
+            }
+            // ---- O^T += V^T P^T: k-step sp, lane half hf: keys 16 sp + 4 hf .. + 3 and 8 further; a wave's LDS accesses run in order ----
+            uint32_t at = lane;
+            if (BITS == 16) asm volatile("" : "+v"(at));
+            const uint32_t e = (at >> 2) & 3, dim = ((at >> 4) & 1) * 16 + (at & 3) * 4;
+            const uint32_t vrow = vtile + (4 * (at >> 5) + e) * L::VROW;
+#pragma unroll
+            for (int mt = 0; mt < 8; mt++) {
+                const uint32_t d = BITS == 16 ? ((32 * mt + dim) * 2 + 64 * e) & 511 : (32 * mt + dim) * 2;
+                u32x2 r[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) r[i] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<LdsShort4>(vrow + d + 8 * i * L::VROW)));
+#pragma unroll
+                for (int sp = 0; sp < 2; sp++) {
+                    const half8 v = __builtin_bit_cast(half8, u32x4{r[2 * sp].x, r[2 * sp].y, r[2 * sp + 1].x, r[2 * sp + 1].y});
+                    acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, p[sp], acc[mt], 0, 0, 0);
+                }
+            }
+            if constexpr (BITS == 16) {
+                // (what comes from memory into the tile is not in the order of the wave's LDS accesses: its reads have to be back)
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                if (b + SMALL_WAVES < nblocks) fetch_values(b + SMALL_WAVES);
+            }
         }
-    };
-    if (wave < 4 && uint32_t(wave) < active) hand_out();
-    lds_barrier();
-    {
-        float2 x[SMALL_WAVES];
+
+        // ---- the waves' parts joined: wave w finishes dims 32 w .. 32 w + 31 ----
+        ask_gates();
+        lds_barrier();  // every wave is through with its tile and the query operands
+        const float l_row = l + __shfl_xor(l, 32);
+        if (hf == 0) ml[wave * 32 + col] = float2{m, l_row};
+        auto tile_of = [&](int w, int mt) { return reinterpret_cast<float4 *>(lds + (w & 3) * 32768 + mt * 4096) + lane; };
+        auto hand_out = [&]() {  // this wave's O, all dims
 #pragma unroll
-        for (int w = 0; w < SMALL_WAVES; w++) x[w] = ml[w * 32 + col];  // (a wave without a block: l = 0)
+            for (int mt = 0; mt < 8; mt++) {
 #pragma unroll
-        for (int w = 0; w < SMALL_WAVES; w++) top = fmaxf(top, x[w].x);
+                for (int i = 0; i < 4; i++) tile_of(wave, mt)[i * 64] = float4{acc[mt][4 * i], acc[mt][4 * i + 1], acc[mt][4 * i + 2], acc[mt][4 * i + 3]};
+            }
+        };
+        float weight[SMALL_WAVES];
+        auto take_in = [&](int from) {  // the dims this wave finishes, from waves from .. from + 3
 #pragma unroll
-        for (int w = 0; w < SMALL_WAVES; w++) weight[w] = __builtin_amdgcn_exp2f(x[w].x - top), l_all += x[w].y * weight[w];
-    }
-    take_in(0);
-    if (active > 4) {
+            for (int w = 0; w < 4; w++) {
+                if (uint32_t(from + w) < active) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float4 x = tile_of(w, wave)[i * 64];
+                        fin[4 * i] += x.x * weight[from + w], fin[4 * i + 1] += x.y * weight[from + w];
+                        fin[4 * i + 2] += x.z * weight[from + w], fin[4 * i + 3] += x.w * weight[from + w];
+                    }
+                }
+            }
+        };
+        if (wave < 4 && uint32_t(wave) < active) hand_out();
         lds_barrier();
-        if (wave >= 4 && uint32_t(wave) < active) hand_out();
-        lds_barrier();
-        take_in(4);
+        {
+            float2 x[SMALL_WAVES];
+#pragma unroll
+            for (int w = 0; w < SMALL_WAVES; w++) x[w] = ml[w * 32 + col];  // (a wave without a block: l = 0)
+#pragma unroll
+            for (int w = 0; w < SMALL_WAVES; w++) top = fmaxf(top, x[w].x);
+#pragma unroll
+            for (int w = 0; w < SMALL_WAVES; w++) weight[w] = __builtin_amdgcn_exp2f(x[w].x - top), l_all += x[w].y * weight[w];
+        }
+        take_in(0);
+        if (active > 4) {
+            lds_barrier();
+            if (wave >= 4 && uint32_t(wave) < active) hand_out();
+            lds_barrier();
+            take_in(4);
+        }
     }
     if constexpr (SPLIT) {
         // (rows past the chunk's end leave what their masked lanes hold; nothing reads it)
@@ -1221,11 +1394,12 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
         if (wave == 0 && hf == 0) *reinterpret_cast<float2 *>(a.part_ml + ((item * 4 + group) * 32 + col) * 2) = float2{top, l_all};
         return;
     }
-    // Turned round in the place of what the first wave handed to this one, which nobody else reads: piece p (dims 4 p .. + 3) of row
+    // Turned round (in the place of what the first wave handed to this one, which nobody else reads): piece p (dims 4 p .. + 3) of row
     // r at 16 ((r + 2 p) % 32) of the piece's 512 bytes, so that neither side meets in its banks.
     const float inv = 1.0f / l_all;
     unsigned char *turned = lds + wave * 4096;
-    wave_sync();  // every lane has taken what was handed over
+    if constexpr (SHARED) lds_barrier();  // the values have been read
+    else wave_sync();  // every lane has taken what was handed over
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const uint32_t piece = 2 * i + hf;
@@ -1483,25 +1657,34 @@ int launch_small(hipStream_t stream, int bits, const uint16_t *q, const void *kd
                  const uint16_t *kz, const uint16_t *vs, const uint16_t *vz, const float *q_and_gate, float *out,
                  const saetta_flash_params &p, uint32_t part_blocks, void *workspace, const char *what) {
     SmallArgs a{q, static_cast<const unsigned char *>(kdata), static_cast<const unsigned char *>(vdata), ks, kz, vs, vz, q_and_gate, out, p.heads, p.kv_heads, p.pos, p.tokens, p.scale, 0, 0, nullptr, nullptr};
-    auto kernels = [&](auto split, dim3 grid) {
+    auto kernels = [&](auto split, dim3 grid, uint32_t blocks) {  // blocks: the most of a workgroup
         constexpr bool SPLIT = decltype(split)::value;
-        if (bits == 8) {
-            launch(prefill_small_kernel<8, SPLIT>, grid, SMALL_THREADS, SmallLds<8>::BYTES, stream, a);
-        } else if (bits == 4) {
-            launch(prefill_small_kernel<4, SPLIT>, grid, SMALL_THREADS, SmallLds<4>::BYTES, stream, a);
-        } else {
-            launch(prefill_small_kernel<16, SPLIT>, grid, SMALL_THREADS, SmallLds<16>::BYTES, stream, a);
+        auto variant = [&](auto rounds) {
+            constexpr int ROUNDS = decltype(rounds)::value;
+            constexpr bool SHARED = ROUNDS != OWN_BLOCKS;
+            if (bits == 8) {
+                if constexpr (ROUNDS != SHARED_ROUNDS) launch(prefill_small_kernel<8, SPLIT, ROUNDS>, grid, SMALL_THREADS, SmallLds<8, SHARED>::BYTES, stream, a);
+            } else if (bits == 4) {
+                launch(prefill_small_kernel<4, SPLIT, ROUNDS>, grid, SMALL_THREADS, SmallLds<4, SHARED>::BYTES, stream, a);
+            } else {
+                launch(prefill_small_kernel<16, SPLIT, ROUNDS>, grid, SMALL_THREADS, SmallLds<16, SHARED>::BYTES, stream, a);
+            }
+        };
+        if (blocks <= SMALL_WAVES) return variant(std::integral_constant<int, ONE_ROUND>{});
+        if constexpr (!SPLIT) {
+            if (bits != 8 && p.pos + p.tokens / 2 <= (bits == 16 ? SHARED_KEYS_HALF : SHARED_KEYS_4)) return variant(std::integral_constant<int, SHARED_ROUNDS>{});
         }
+        variant(std::integral_constant<int, OWN_BLOCKS>{});
     };
     const uint32_t groups = (p.tokens + 3) / 4;
     if (!part_blocks) {
-        kernels(std::false_type{}, dim3(groups, p.kv_heads));
+        kernels(std::false_type{}, dim3(groups, p.kv_heads), (p.pos + p.tokens + BK - 1) / BK);
         return launch_status(what);
     }
     a.part_blocks = part_blocks, a.nparts = parts_of(p.pos, p.tokens, part_blocks);
     a.part_o = static_cast<float *>(workspace);
     a.part_ml = a.part_o + size_t(a.nparts) * ((p.tokens + TQ - 1) / TQ) * p.kv_heads * (PART_O_BYTES / 4);
-    kernels(std::true_type{}, dim3((a.nparts * p.kv_heads * groups + 7) / 8 * 8));
+    kernels(std::true_type{}, dim3((a.nparts * p.kv_heads * groups + 7) / 8 * 8), part_blocks);
     PrefillArgs m{q, nullptr, q_and_gate, out, p.heads, p.kv_heads, p.pos, p.tokens, p.scale, 0, nullptr, part_blocks, a.part_o, a.part_ml};
     launch_merge(stream, m, a.nparts);
     return launch_status(what);
@@ -1989,12 +2172,22 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
 
 int setup_prefill() {
     if (int rc = load_kernel(reinterpret_cast<const void *>(prefill_merge_kernel<1>))) return rc;
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<16, false>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<16>::BYTES))) return rc;
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<16, true>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<16>::BYTES))) return rc;
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<8, false>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<8>::BYTES))) return rc;
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<8, true>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<8>::BYTES))) return rc;
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<4, false>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<4>::BYTES))) return rc;
-    if (int rc = int(hipFuncSetAttribute(reinterpret_cast<const void *>(prefill_small_kernel<4, true>), hipFuncAttributeMaxDynamicSharedMemorySize, SmallLds<4>::BYTES))) return rc;
+    auto raise_small = [](auto bits_c) {
+        constexpr int BITS = decltype(bits_c)::value;
+        std::vector<std::pair<const void *, int>> kernels = {
+            {reinterpret_cast<const void *>(prefill_small_kernel<BITS, false, OWN_BLOCKS>), SmallLds<BITS, false>::BYTES},
+            {reinterpret_cast<const void *>(prefill_small_kernel<BITS, true, OWN_BLOCKS>), SmallLds<BITS, false>::BYTES},
+            {reinterpret_cast<const void *>(prefill_small_kernel<BITS, false, ONE_ROUND>), SmallLds<BITS, true>::BYTES},
+            {reinterpret_cast<const void *>(prefill_small_kernel<BITS, true, ONE_ROUND>), SmallLds<BITS, true>::BYTES}};
+        if constexpr (BITS != 8) kernels.push_back({reinterpret_cast<const void *>(prefill_small_kernel<BITS, false, SHARED_ROUNDS>), SmallLds<BITS, true>::BYTES});
+        for (const auto &[kernel, bytes] : kernels) {
+            if (int rc = int(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes))) return rc;
+        }
+        return 0;
+    };
+    if (int rc = raise_small(std::integral_constant<int, 16>{})) return rc;
+    if (int rc = raise_small(std::integral_constant<int, 8>{})) return rc;
+    if (int rc = raise_small(std::integral_constant<int, 4>{})) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_scores_kernel))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_pv_kernel))) return rc;
     for (const void *kernel : {reinterpret_cast<const void *>(attention_prefill_kernel<true, false>), reinterpret_cast<const void *>(attention_prefill_kernel<true, true>),
