@@ -81,7 +81,7 @@ __global__ __launch_bounds__(THREADS, 2) void calib_mfma_stream_kernel(const uns
         Copy cp;
         cp.src = reinterpret_cast<uint64_t>(operands) + uint64_t(at) * PART_BYTES + (wave & 1) * 8192;
         cp.dst = lds0 + ((wave >> 1) + 4 * h) * PART_BYTES + (wave & 1) * 8192;
-        copy_plain(cp, lane16);
+        copy_plain<false>(cp, lane16);
         at = at + 1 < parts ? at + 1 : 0;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(THREADS, 2) void calib_mfma_stream_kernel(const uns
         Copy cp;
         cp.src = reinterpret_cast<uint64_t>(operands) + uint64_t((at + (wave >> 1)) % parts) * PART_BYTES + (wave & 1) * 8192;
         cp.dst = lds0 + ((((wave >> 1) & 1) * 4) + ((2 * step + 2 + (wave >> 2)) & 3)) * PART_BYTES + (wave & 1) * 8192;
-        stream_block(s, o, q, p, lds0 + slot * PART_BYTES + lane16, lds0 + (4 + slot) * PART_BYTES + lane16, cp, lane16);
+        stream_block<false>(s, o, q, p, lds0 + slot * PART_BYTES + lane16, lds0 + (4 + slot) * PART_BYTES + lane16, cp, lane16);
         at = at + 4 < parts ? at + 4 : at + 4 - parts;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();

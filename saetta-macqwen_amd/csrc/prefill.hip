@@ -62,6 +62,7 @@ constexpr int PREP_THREADS = 256;       // the prepare kernel's workgroup
 constexpr int WAVES = 8;                // 4 row groups x 2 waves that take alternate key blocks
 constexpr int THREADS = 64 * WAVES;
 constexpr int TQ = 16;                  // tokens per workgroup: a row group is 4 tokens x 8 heads = 32 rows
+constexpr int WIDE_TQ = 32;             // ... of a wide tile, a row group a wave
 constexpr int BK = 32;                  // keys per block
 // One key block's image: the K tile and the V^T tile in MFMA fragment order, 16 KB each.  A
 // fragment is what one ds_read_b128 of a wave fetches: 64 lanes x 16 bytes, lane (col, hf) at
@@ -330,25 +331,30 @@ constexpr int LDS_BYTES = 8 * MERGE_WAVE_BYTES > 8 * PART_BYTES ? 8 * MERGE_WAVE
 __device__ __forceinline__ uint32_t k_slot(uint32_t b) { return (b & 3) * PART_BYTES; }
 __device__ __forceinline__ uint32_t v_slot(uint32_t b) { return (4 + (b & 3)) * PART_BYTES; }
 
-// Blocks of keys that tile `tile` sees.
-__device__ __host__ __forceinline__ uint32_t tile_blocks(uint32_t pos, uint32_t tokens, uint32_t tile) {
-    const uint32_t end = tile * TQ + TQ < tokens ? tile * TQ + TQ : tokens;
+// Blocks of keys that tile `tile` of `tq` tokens sees.
+__device__ __host__ __forceinline__ uint32_t tile_blocks(uint32_t pos, uint32_t tokens, uint32_t tile, uint32_t tq = TQ) {
+    const uint32_t end = tile * tq + tq < tokens ? tile * tq + tq : tokens;
     return (pos + end + BK - 1) / BK;
 }
 
 // One tile of TQ tokens x 8 heads of kv head `kv` against the keys it sees, or (SPLIT) against part `part` of them.
+// WIDE: of WIDE_TQ tokens.  A wave has a row group of its own and takes every block, a block a step, and what the workgroup
+// copies for a step, 32 KB instead of 64, serves twice the rows.  The copies are what the clock pays for most after the products: the kernel's
+// streams by themselves run at 1370 to 1384 TFLOP/s with half of them and at 1290 with all.  Where a wide tile is taken: tiles_plan.
 // EXACT: in the first EXACT_BLOCKS blocks the reference maximum is the maximum itself, so that a row's largest probability
 // there is 1, which f16 holds exactly; relative to a maximum up to 2^TAU below it is rounded like the others, which shows
 // in rows of few keys.  For AttGemm, whose passes took every tile's probabilities relative to the tile's own maximum
 // (largest error over the output's r.m.s., 1712 tokens at 37: passes 0.8e-2 to 1.3e-2, without EXACT 1.5e-2, with 0.6e-2; 1 us
 // a tile).
-template <bool SPLIT, bool EXACT>
+template <bool SPLIT, bool EXACT, bool WIDE>
 __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char *tiles, uint32_t tile, uint32_t kv, uint32_t part_index, bool ask, uint32_t *next_tile) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hf = lane >> 5;
-    const int group = wave & 3, parity = wave >> 2;  // the wave's rows; which key blocks it takes
-    const uint32_t tok0 = tile * TQ + 4 * group;    // this wave's first token
+    static_assert(SPLIT || !WIDE, "wide tiles leave parts");
+    constexpr uint32_t TILE = WIDE ? WIDE_TQ : TQ, STRIDE = WIDE ? 1 : 2;  // tokens; blocks from one of a wave's to its next
+    const int group = WIDE ? wave : wave & 3, parity = wave >> 2;  // the wave's rows; which key blocks it takes (WIDE: all), and its order
+    const uint32_t tok0 = tile * TILE + 4 * group;  // this wave's first token
     const float c = a.scale * 1.4426950408889634f;  // scores are kept in units of log2(e)
 
     // Row of this lane: token tok0 + col / 8, head col % 8.
@@ -358,7 +364,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     // first block on: key0 is that block's first key, and a row of the tile may see none of the part (the tile's tokens
     // cross a block's end where the last part begins).
     const uint32_t block0 = SPLIT ? part_index * a.part_blocks : 0, key_base = block0 * BK;
-    const uint32_t all_blocks = tile_blocks(a.pos, a.tokens, tile) - block0;
+    const uint32_t all_blocks = tile_blocks(a.pos, a.tokens, tile, TILE) - block0;
     const uint32_t nblocks = SPLIT ? min(all_blocks, a.part_blocks) : all_blocks;
     auto from_base = [&](uint32_t keys) { return SPLIT ? (keys > key_base ? keys - key_base : 0) : keys; };
     const uint32_t wave_first_len = from_base(a.pos + tok0 + 1);            // keys the wave's first token sees
@@ -405,10 +411,11 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     // 16 lanes read on different banks and keeps every 64 bytes of memory together.
     uint32_t at = lane;  // (what depends on the lane is made where it is used, not kept in registers from tile to tile)
     asm volatile("" : "+v"(at));
-    const uint32_t q_place = lds0 + v_slot(0) + group * (32 * DIM * 2);
+    // (WIDE: eight row groups fill all places, the keys' too, and come before them)
+    const uint32_t q_at = (WIDE ? 0 : v_slot(0)) + group * (32 * DIM * 2), q_place = lds0 + q_at;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const uint32_t k = 8 * parity + i;  // rows 2k and 2k + 1
+    for (int i = 0; i < (WIDE ? 16 : 8); i++) {
+        const uint32_t k = WIDE ? i : 8 * parity + i;  // rows 2k and 2k + 1
         const uint32_t tk = min(tok0 + k / 4, a.tokens - 1);
         const uint64_t src = reinterpret_cast<uint64_t>(a.q) + ((size_t(tk) * a.heads + kv * SAETTA_GQA_GROUP + 2 * k % 8) * DIM) * 2;
         const uint32_t off = (at >> 5) * 512 + (((at - 4 * (i >> 1 & 3)) & 31) ^ (2 * (i & 1) + (at >> 5))) * 16;
@@ -420,21 +427,32 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
             : [off] "v"(off), [src] "s"(src), [dst] "s"(q_place + k * 1024)
             : "memory", "m0");
     }
+    if constexpr (!WIDE) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {  // K(0..3): wave w takes 2 KB of each
-        const Copy cp = piece(i, 0, 0);
-        copy2k(cp.src + wave * 2048, cp.dst + wave * 2048);
+        for (int i = 0; i < 4; i++) {  // K(0..3): wave w takes 2 KB of each
+            const Copy cp = piece(i, 0, 0);
+            copy2k(cp.src + wave * 2048, cp.dst + wave * 2048);
+        }
+        asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");  // (the keys stay on their way)
+    } else {
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     }
-    asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");  // (the keys stay on their way)
     half8 qb[16];
 #pragma unroll
     for (int st = 0; st < 16; st++) {
         const uint32_t place = 4 * (((st >> 1) + (at >> 2 & 3)) & 7) + ((2 * (st & 1) + (at >> 5)) ^ (at & 3));
-        qb[st] = *reinterpret_cast<const half8 *>(tiles + v_slot(0) + group * (32 * DIM * 2) + (at & 31) * (DIM * 2) + place * 16);
+        qb[st] = *reinterpret_cast<const half8 *>(tiles + q_at + (at & 31) * (DIM * 2) + place * 16);
     }
     lds_barrier();  // the queries have been read: the values may land there
+    if constexpr (WIDE) {
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < 2; i++) {  // K(0), K(1)
+            const Copy cp = piece(i, 0, 0);
+            copy2k(cp.src + wave * 2048, cp.dst + wave * 2048);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < (WIDE ? 1 : 2); i++) {
         const Copy cp = piece(i, 1, 0);
         copy2k(cp.src + wave * 2048, cp.dst + wave * 2048);
     }
@@ -503,11 +521,18 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
         }
     };
 
-    asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");  // K(0..3) are in LDS, V(0) and V(1) on their way
+    // K(0..3) are in LDS, V(0) and V(1) on their way (WIDE: K(0) and K(1), V(0))
+    if constexpr (WIDE) asm volatile("s_waitcnt vmcnt(2)\n\ts_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");
 
-    const uint32_t nsteps = (nblocks + 1) / 2;
+    const uint32_t nsteps = WIDE ? nblocks : (nblocks + 1) / 2;
     const int part = wave >> 1, half = wave & 1;  // what the wave copies in every step
     auto copy_of = [&](uint32_t step) {
+        if constexpr (WIDE) {  // a quarter of K(s + 2) or of V(s + 1)
+            Copy cp = piece(step + 2 - parity, parity, 0);
+            cp.src += (wave & 3) * 4096, cp.dst += (wave & 3) * 4096;
+            return cp;
+        }
         const uint32_t cb = part == 0 ? 2 * step + 4 : part == 1 ? 2 * step + 5 : part == 2 ? 2 * step + 2 : 2 * step + 3;
         return piece(cb, part >= 2, half);
     };
@@ -520,45 +545,46 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
         __syncthreads();  // V(0) and V(1) are there; the first step's copies overwrite K(0) and K(1)
         for (uint32_t step = 0; step < nsteps; step++) {
             const Copy cp = copy_of(step);
-            const uint32_t kb = 2 * step;
+            const uint32_t kb = STRIDE * step;
             if (kb < wave_blocks) {
                 raise_max(mask_max(s, kb * BK, kb >= full_blocks), kb);
                 half8 pb[2];
                 exp_pack(s, pb);
                 // (past the wave's last block the scores are of stale keys and never looked at)
-                stream_block(s, acc, qb, pb, lds0 + k_slot(kb + 2) + lane16, lds0 + v_slot(kb) + lane16, cp, lane16);
+                stream_block<WIDE>(s, acc, qb, pb, lds0 + k_slot(kb + STRIDE) + lane16, lds0 + v_slot(kb) + lane16, cp, lane16);
             } else {
-                copy_plain(cp, lane16);
+                copy_plain<WIDE>(cp, lane16);
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
         }
     } else {
+        constexpr uint32_t FIRST = WIDE ? 0 : 1;
         half8 pb[2] = {};
-        if (1 < wave_blocks) {
+        if (FIRST < wave_blocks) {
             floatx16 s;
-            scores_block(s, qb, lds0 + k_slot(1) + lane16);
-            raise_max(mask_max(s, BK, 1 >= full_blocks), 1);
+            scores_block(s, qb, lds0 + k_slot(FIRST) + lane16);
+            raise_max(mask_max(s, FIRST * BK, FIRST >= full_blocks), FIRST);
             exp_pack(s, pb);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         for (uint32_t step = 0; step < nsteps; step++) {
             const Copy cp = copy_of(step);
-            const uint32_t kb = 2 * step + 1;
+            const uint32_t kb = STRIDE * step + FIRST;
             if (kb < wave_blocks) {
                 // This wave's stream comes before its softmax, the other wave's of the SIMD after: let
                 // this one's MFMAs go first, so that its softmax still finds the other's to run under.
                 floatx16 s;
                 __builtin_amdgcn_s_setprio(2);
-                stream_block(s, acc, qb, pb, lds0 + k_slot(kb + 2) + lane16, lds0 + v_slot(kb) + lane16, cp, lane16);
+                stream_block<WIDE>(s, acc, qb, pb, lds0 + k_slot(kb + STRIDE) + lane16, lds0 + v_slot(kb) + lane16, cp, lane16);
                 __builtin_amdgcn_s_setprio(0);
-                if (kb + 2 < wave_blocks) {
-                    raise_max(mask_max(s, (kb + 2) * BK, kb + 2 >= full_blocks), kb + 2);
+                if (kb + STRIDE < wave_blocks) {
+                    raise_max(mask_max(s, (kb + STRIDE) * BK, kb + STRIDE >= full_blocks), kb + STRIDE);
                     exp_pack(s, pb);
                 }
             } else {
-                copy_plain(cp, lane16);
+                copy_plain<WIDE>(cp, lane16);
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
@@ -572,6 +598,24 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     // live with them costs 150 bytes of spills.)
     uint32_t got = ask ? 0u : 0xffffffffu;
     if (ask && tid == 0) got = gridDim.x + atomicAdd(a.tiles_taken, 1u);
+    if constexpr (WIDE) {
+        // Nothing to join: the part's O, m and l leave as two tiles of TQ tokens would leave them (a second one past the chunk's end
+        // has no place).
+        const float l = l_sum + __shfl_xor(l_sum, 32);
+        const uint32_t ntiles = (a.tokens + TQ - 1) / TQ, narrow = 2 * tile + (group >> 2);
+        if (narrow < ntiles) {
+            const size_t item = (size_t(part_index) * ntiles + narrow) * a.kv_heads + kv;
+#pragma unroll
+            for (int i = 0; i < 32; i++) {
+                float *po = a.part_o + ((item * WAVES + (group & 3) * 2 + (i >> 4)) * 16 * 64 + lane) * 4;
+                const int mt = i >> 2, q4 = i & 3;
+                *reinterpret_cast<float4 *>(po + (i & 15) * 64 * 4) = float4{acc[mt][4 * q4], acc[mt][4 * q4 + 1], acc[mt][4 * q4 + 2], acc[mt][4 * q4 + 3]};
+            }
+            if (hf == 0) *reinterpret_cast<float2 *>(a.part_ml + ((item * 4 + (group & 3)) * 32 + col) * 2) = float2{m_ref, l};
+        }
+        if (tid == 0) *next_tile = got;
+        return;
+    }
 
     // The gate values of this wave's half of the dims, asked for before the merge below so that they travel while
     // it runs: two rows of 512 bytes a load, as the outputs are stored (a token past the end: the last token's, unused).
@@ -672,20 +716,20 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
 
 // The first tile that has a part `part` of part_blocks blocks (tiles see more keys the later they are), and how many
 // (tile, part) pairs there are.
-__device__ __host__ __forceinline__ uint32_t prefill_first_tile(uint32_t pos, uint32_t tokens, uint32_t part_blocks, uint32_t part) {
-    const uint32_t ntiles = (tokens + TQ - 1) / TQ;
+__device__ __host__ __forceinline__ uint32_t prefill_first_tile(uint32_t pos, uint32_t tokens, uint32_t part_blocks, uint32_t part, uint32_t tq = TQ) {
+    const uint32_t ntiles = (tokens + tq - 1) / tq;
     const uint32_t keys = part * part_blocks * BK;  // a tile has the part if it sees more keys than these
     if (pos + tokens <= keys) return ntiles;
-    if (pos + TQ > keys) return 0;
-    const uint32_t t = (keys - pos) / TQ;  // tokens up to keys - pos see no key of it
+    if (pos + tq > keys) return 0;
+    const uint32_t t = (keys - pos) / tq;  // tokens up to keys - pos see no key of it
     return t < ntiles ? t : ntiles - 1;
 }
-__device__ __host__ __forceinline__ uint32_t prefill_items(uint32_t pos, uint32_t tokens, uint32_t part_blocks) {
-    const uint32_t ntiles = (tokens + TQ - 1) / TQ;
+__device__ __host__ __forceinline__ uint32_t prefill_items(uint32_t pos, uint32_t tokens, uint32_t part_blocks, uint32_t tq = TQ) {
+    const uint32_t ntiles = (tokens + tq - 1) / tq;
     // the parts that begin at a key the first tile sees are every tile's
-    const uint32_t whole = (pos + (tokens < TQ ? tokens : TQ) - 1) / (part_blocks * BK) + 1;
+    const uint32_t whole = (pos + (tokens < tq ? tokens : tq) - 1) / (part_blocks * BK) + 1;
     uint32_t n = whole * ntiles;
-    for (uint32_t p = whole, first; (first = prefill_first_tile(pos, tokens, part_blocks, p)) < ntiles; p++) n += ntiles - first;
+    for (uint32_t p = whole, first; (first = prefill_first_tile(pos, tokens, part_blocks, p, tq)) < ntiles; p++) n += ntiles - first;
     return n;
 }
 
@@ -698,21 +742,22 @@ __device__ __host__ __forceinline__ uint32_t prefill_items(uint32_t pos, uint32_
 // longest with the shortest, ended 40 us apart: the workgroups' rates differ by a tenth).
 // SPLIT: an item is a part of a tile's keys, parts side by side in tiles and kv heads (workgroups that run together walk
 // the same keys); the tiles that have a part p are the ones from prefill_first_tile(p) on.
-template <bool SPLIT, bool EXACT>
+template <bool SPLIT, bool EXACT, bool WIDE>
 __global__ __launch_bounds__(THREADS, 2) void attention_prefill_kernel(PrefillArgs a) {
+    constexpr uint32_t TILE = WIDE ? WIDE_TQ : TQ;
     extern __shared__ __attribute__((aligned(1024))) unsigned char tiles[];
     __shared__ uint32_t next_tile;
-    const uint32_t ntiles = (a.tokens + TQ - 1) / TQ, G = gridDim.x;
+    const uint32_t ntiles = (a.tokens + TILE - 1) / TILE, G = gridDim.x;
     uint32_t total = ntiles * a.kv_heads;
-    if constexpr (SPLIT) total = prefill_items(a.pos, a.tokens, a.part_blocks) * a.kv_heads;
+    if constexpr (SPLIT) total = prefill_items(a.pos, a.tokens, a.part_blocks, TILE) * a.kv_heads;
     for (uint32_t idx = blockIdx.x; idx < total;) {
         // (the tiles from G on are handed out by one question each: the tiles before the last G ask one, when they end,
         // and the last G none: nothing is left by then, and the kernel's last epilogues do not wait for an answer)
         uint32_t at = idx / a.kv_heads, part = 0;
         if constexpr (SPLIT) {
-            for (uint32_t n; at >= (n = ntiles - prefill_first_tile(a.pos, a.tokens, a.part_blocks, part)); part++) at -= n;
+            for (uint32_t n; at >= (n = ntiles - prefill_first_tile(a.pos, a.tokens, a.part_blocks, part, TILE)); part++) at -= n;
         }
-        prefill_tile<SPLIT, EXACT>(a, tiles, ntiles - 1 - at, idx % a.kv_heads, part, idx + G < total, &next_tile);
+        prefill_tile<SPLIT, EXACT, WIDE>(a, tiles, ntiles - 1 - at, idx % a.kv_heads, part, idx + G < total, &next_tile);
         lds_barrier();  // the next tile is known; this tile's merge has been read: the next tile's keys may land on it (its stores go on meanwhile)
         idx = next_tile;
     }
@@ -1452,6 +1497,7 @@ uint32_t parts_of(uint32_t pos, uint32_t tokens, uint32_t part_blocks) {
 struct FlashPlan {
     bool small;  // without parts, the row groups' launch is ahead of the tiles
     uint32_t small_part_blocks, cus, part_blocks, nparts;
+    bool wide;  // the parts are those of tiles of WIDE_TQ tokens
     size_t plain, parts, small_parts;  // bytes of workspace: the images and the tile count; the parts behind them; the row groups' parts, instead of both
     size_t tiles() const { return plain + parts; }
     size_t bytes() const { return tiles() > small_parts ? tiles() : small_parts; }
@@ -1466,6 +1512,11 @@ struct FlashPlan {
 // (The ends have become 6 and 2.5 us shorter since, the merge 1; with these figures the rule still takes what is the fastest or
 // within 2 % of it at 33 of 38 sizes from 20 to 3500 tokens, 0 to 10000 keys before them, both kinds of cache; the furthest off are
 // 2300 tokens at 3000, 216 us instead of 201 in two parts, and 128 at 4000, 36 instead of 33.)
+// Wide tiles (WIDE_TQ tokens, a row group a wave; always in parts, so that there are as many items): a copied part of keys or values serves eight
+// row groups instead of four, half the global -> LDS copies, and the chip, which is bound by its power, does 5 % more blocks; a block
+// alone takes 1.3 us for twice the rows and an item's ends 18.  Whole call, us, without -> with: 2048 tokens at 118784 (AttGemm) 3568 -> 3397, 1237 at
+// 60007 (4-bit) 1142 -> 1082, 800 at 80000 1018 -> 978, 1024 at 30000 481 -> 465, 2300 at 3000 218 -> 205, 2100 at 1000 114 -> 106, 4096 at 20000 1307 ->
+// 1254.  Not where the parts' merge costs more than that: 4096 at 4096 would take 467 instead of 387, 2048 at 10000 (355) is even.
 // Measured, unsplit -> split by this rule, the whole call (8-bit cache): 100 tokens at 10000: 211 -> 47 us, at 100000
 // (4-bit): 1886 -> 225; 500 at 40000: 770 -> 330; 2100 at 9000: 497 -> 405.  A full chunk (4096 tokens: two whole rounds)
 // is never split.
@@ -1488,6 +1539,7 @@ float rounds_us(uint32_t cus, uint32_t n, float high, float low, float ends_us, 
 FlashPlan tiles_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, float &tiles_us) {
     constexpr float BLOCK_US = 0.6f, CHIP_BLOCKS_PER_US = 284.0f / 256.0f, PART_US = 12.0f, TILE_US = 14.5f, MERGE_US = 4.0f;
     constexpr float PREPARE_US = 4.5f, PREPARE_KEY_US = 0.0003f;
+    constexpr float WIDE_PART_US = 18.0f, WIDE_BLOCK_US = 1.3f, WIDE_GAIN = 0.95f;
     FlashPlan f{};
     f.cus = cu_count();
     f.plain = plain_workspace_bytes(pos, tokens, kv_heads);
@@ -1498,24 +1550,34 @@ FlashPlan tiles_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, float &ti
     const float chip_us = 1.0f / (CHIP_BLOCKS_PER_US * float(f.cus));
     const float unsplit = rounds_us(f.cus, ntiles * kv_heads, float(longest), float(shortest), TILE_US, BLOCK_US, chip_us);
     float best = 0.95f * unsplit;
-    for (uint32_t parts = 2; parts <= 32; parts++) {
-        const uint32_t pb = ((longest + parts - 1) / parts + 1) / 2 * 2;  // (a step of the kernel is two blocks)
-        if (pb < 4 || pb >= longest) continue;
-        const uint32_t items = prefill_items(pos, tokens, pb) * kv_heads;
-        const float mid = 0.5f * float(longest + shortest) * float(ntiles * kv_heads) / float(items);
-        const float us = rounds_us(f.cus, items, mid, mid, PART_US, BLOCK_US, chip_us) + MERGE_US + MERGE_ITEM_US * float(items);
-        if (us < best) best = us, f.part_blocks = pb;
-    }
+    auto in_parts = [&](bool wide) {
+        const uint32_t tq = wide ? WIDE_TQ : TQ, n = (tokens + tq - 1) / tq;
+        const float high = float(tile_blocks(pos, tokens, n - 1, tq)), low = float(tile_blocks(pos, tokens, 0, tq));
+        for (uint32_t parts = 2; parts <= 32; parts++) {
+            const uint32_t pb = ((longest + parts - 1) / parts + 1) / 2 * 2;  // (a step of the kernel is two blocks)
+            if (pb < 4 || pb >= longest) continue;
+            const uint32_t items = prefill_items(pos, tokens, pb, tq) * kv_heads;
+            const float mid = 0.5f * (high + low) * float(n * kv_heads) / float(items);
+            const float us = (wide ? rounds_us(f.cus, items, mid, mid, WIDE_PART_US, WIDE_BLOCK_US, WIDE_GAIN * 2.0f * chip_us) : rounds_us(f.cus, items, mid, mid, PART_US, BLOCK_US, chip_us)) +
+                             MERGE_US + (wide ? 2.0f : 1.0f) * MERGE_ITEM_US * float(items);
+            if (us < best) best = us, f.part_blocks = pb, f.wide = wide;
+        }
+    };
+    in_parts(false);
+    if (!f.part_blocks) best = unsplit;
+    // (what the row groups are weighed against stays what it was before there were wide tiles: which chunks need no workspace is
+    // decided there)
+    const float narrow = best;
+    best *= 0.985f;
+    in_parts(true);
     if (f.part_blocks) {
         f.nparts = parts_of(pos, tokens, f.part_blocks);
         f.parts = parts_bytes(tokens, kv_heads, f.nparts);
-    } else {
-        best = unsplit;
     }
     // (never less than 5 us, what short contexts' images were counted at when the row groups came in: a chunk that goes to them
     // without parts needs no workspace, and who calls it without one, recording or under capture, goes on to)
     const float prepare_us = PREPARE_US + PREPARE_KEY_US * float(pos + tokens) * float(kv_heads);
-    tiles_us = best + (prepare_us > 5.0f ? prepare_us : 5.0f);
+    tiles_us = narrow + (prepare_us > 5.0f ? prepare_us : 5.0f);
     return f;
 }
 
@@ -1705,12 +1767,14 @@ int launch_flash(hipStream_t stream, int bits, const uint16_t *q, const void *kd
         a.part_blocks = plan.part_blocks;
         a.part_o = reinterpret_cast<float *>(ws + plan.plain);
         a.part_ml = reinterpret_cast<float *>(ws + plan.plain + size_t(plan.nparts) * ntiles * p.kv_heads * PART_O_BYTES);
-        const uint32_t total = prefill_items(p.pos, p.tokens, plan.part_blocks) * p.kv_heads;
-        launch(exact ? attention_prefill_kernel<true, true> : attention_prefill_kernel<true, false>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
+        const uint32_t total = prefill_items(p.pos, p.tokens, plan.part_blocks, plan.wide ? WIDE_TQ : TQ) * p.kv_heads;
+        auto *kernel = plan.wide ? (exact ? attention_prefill_kernel<true, true, true> : attention_prefill_kernel<true, false, true>)
+                                 : (exact ? attention_prefill_kernel<true, true, false> : attention_prefill_kernel<true, false, false>);
+        launch(kernel, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
         launch_merge(stream, a, plan.nparts);
     } else {
         const uint32_t total = ntiles * p.kv_heads;
-        launch(exact ? attention_prefill_kernel<false, true> : attention_prefill_kernel<false, false>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
+        launch(exact ? attention_prefill_kernel<false, true, false> : attention_prefill_kernel<false, false, false>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
     }
     return launch_status(what);
 }
@@ -2190,8 +2254,9 @@ int setup_prefill() {
     if (int rc = raise_small(std::integral_constant<int, 4>{})) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_scores_kernel))) return rc;
     if (int rc = load_kernel(reinterpret_cast<const void *>(attention_gemm_pv_kernel))) return rc;
-    for (const void *kernel : {reinterpret_cast<const void *>(attention_prefill_kernel<true, false>), reinterpret_cast<const void *>(attention_prefill_kernel<true, true>),
-                               reinterpret_cast<const void *>(attention_prefill_kernel<false, false>), reinterpret_cast<const void *>(attention_prefill_kernel<false, true>)}) {
+    for (const void *kernel : {reinterpret_cast<const void *>(attention_prefill_kernel<true, false, false>), reinterpret_cast<const void *>(attention_prefill_kernel<true, true, false>),
+                               reinterpret_cast<const void *>(attention_prefill_kernel<true, false, true>), reinterpret_cast<const void *>(attention_prefill_kernel<true, true, true>),
+                               reinterpret_cast<const void *>(attention_prefill_kernel<false, false, false>), reinterpret_cast<const void *>(attention_prefill_kernel<false, true, false>)}) {
         if (int rc = int(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES))) return rc;
     }
     return 0;

@@ -438,6 +438,26 @@ def test_short_chunks_whose_waves_share_their_blocks(kind, pos, tokens, kv):
     assert float((out - want).abs().max()) < MAX_ABS
 
 
+@pytest.mark.parametrize("kind,pos,tokens,kv", [(saetta.KvBits.Half, 1000, 2100, 2), (saetta.KvBits.Eight, 1003, 2113, 2), (saetta.KvBits.Four, 9990, 2309, 2),
+                                                (saetta.KvBits.Half, 2991, 4177, 1), (saetta.KvBits.Half, 3000, 1441, 3)])
+def test_wide_tiles(kind, pos, tokens, kv):
+    # tiles of 32 tokens, their keys in parts: whole tiles; a last one with 1, 5, 17 tokens (its second half of no place, or of one token);
+    # parts that begin between a tile's tokens; 1 and 3 kv heads
+    call, out, p, want = chunk(kind, pos, tokens, kv)
+    size = saetta.attention_prefill.workspace_bytes(p)
+    ws = torch.full((size,), 0xff, dtype=torch.uint8, device="cuda")
+    out.fill_(float("nan"))
+    assert call(ws.data_ptr(), size) == 0, saetta.ffi.lib().saetta_last_error()
+    got = out.clone()
+    assert float((got.double() - want).norm() / want.norm()) < REL_RMS
+    assert float((got - want).abs().max()) < MAX_ABS
+    # without room for the parts: tiles of 16, the same to the rounding of the probabilities
+    out.fill_(float("nan"))
+    plain = -(-(pos + tokens) // 32) * kv * 32768 + 256
+    assert call(ws.data_ptr(), plain) == 0, saetta.ffi.lib().saetta_last_error()
+    assert float((out.double() - want).norm() / want.norm()) < REL_RMS
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("scale", [1e-3, 300.0])
 def test_short_chunks_of_small_and_large_values(kind, scale):
