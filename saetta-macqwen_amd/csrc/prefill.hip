@@ -933,9 +933,11 @@ constexpr int SMALL_WAVES = 8, SMALL_THREADS = 64 * SMALL_WAVES;
 // blocks, 10 at 3000, 17.7 -> 15.0, 19.5 -> 17.0, 19.2 -> 16.7.  -> SHARED_ROUNDS, halves: 300 from 0 16.8 -> 14.0, 700 25.4 -> 22.2, 900 32.2 -> 29.0,
 // 30 at 500 17.8 -> 16.8, 500 at 300 23.4 -> 23.5, 500 at 800 29.7 -> 32.1; 4-bit: 300 from 0 17.6 -> 16.8, 520 21.8 -> 21.9, 766 28.7 -> 25.7, 30 at
 // 500 20.2 -> 20.2, 500 at 300 25.5 -> 26.7; 8-bit spills 26 registers that way (300 from 0 17.8 -> 18.9) and has none.  So the line lies at the
-// keys that a row group sees in the mean.  Distance from 64 bits: the same or less (halves, 500 at 300: 1.66e-4 -> 1.13e-4).
+// keys that a row group sees in the mean, and in parts, whose row groups all see the same, at the blocks of a part: of 16 blocks halves 12 at
+// 20000 26.1 -> 23.6, 64 at 2000 22.5 -> 19.4, 4-bit 28.4 -> 26.7, 24.2 -> 22.7 (8-bit 28.2 -> 27.1, but 23.5 -> 24.8), of 24 7 at 40000 34.0 -> 31.5 and 32.9 ->
+// 32.5, of 32 120 at 3000 29.2 -> 28.9 and 32.4 -> 32.8, of 40 30 at 16000 32.4 -> 33.7, of 72 55 at 17388 43.8 -> 50.6.  Distance from 64 bits: the same or less (halves, 500 at 300: 1.66e-4 -> 1.13e-4).
 constexpr int OWN_BLOCKS = 0, ONE_ROUND = 1, SHARED_ROUNDS = 2;
-constexpr uint32_t SHARED_KEYS_HALF = 544, SHARED_KEYS_4 = 464;
+constexpr uint32_t SHARED_KEYS_HALF = 544, SHARED_KEYS_4 = 464, SHARED_PART_HALF = 32, SHARED_PART_4 = 24;
 
 struct SmallArgs {
     const uint16_t *q;  // f16 [tokens][heads][256]
@@ -1733,9 +1735,8 @@ int launch_small(hipStream_t stream, int bits, const uint16_t *q, const void *kd
             }
         };
         if (blocks <= SMALL_WAVES) return variant(std::integral_constant<int, ONE_ROUND>{});
-        if constexpr (!SPLIT) {
-            if (bits != 8 && p.pos + p.tokens / 2 <= (bits == 16 ? SHARED_KEYS_HALF : SHARED_KEYS_4)) return variant(std::integral_constant<int, SHARED_ROUNDS>{});
-        }
+        const bool shared = SPLIT ? blocks <= (bits == 16 ? SHARED_PART_HALF : SHARED_PART_4) : p.pos + p.tokens / 2 <= (bits == 16 ? SHARED_KEYS_HALF : SHARED_KEYS_4);
+        if (shared && bits != 8) return variant(std::integral_constant<int, SHARED_ROUNDS>{});
         variant(std::integral_constant<int, OWN_BLOCKS>{});
     };
     const uint32_t groups = (p.tokens + 3) / 4;
@@ -2243,7 +2244,10 @@ int setup_prefill() {
             {reinterpret_cast<const void *>(prefill_small_kernel<BITS, true, OWN_BLOCKS>), SmallLds<BITS, false>::BYTES},
             {reinterpret_cast<const void *>(prefill_small_kernel<BITS, false, ONE_ROUND>), SmallLds<BITS, true>::BYTES},
             {reinterpret_cast<const void *>(prefill_small_kernel<BITS, true, ONE_ROUND>), SmallLds<BITS, true>::BYTES}};
-        if constexpr (BITS != 8) kernels.push_back({reinterpret_cast<const void *>(prefill_small_kernel<BITS, false, SHARED_ROUNDS>), SmallLds<BITS, true>::BYTES});
+        if constexpr (BITS != 8) {
+            kernels.push_back({reinterpret_cast<const void *>(prefill_small_kernel<BITS, false, SHARED_ROUNDS>), SmallLds<BITS, true>::BYTES});
+            kernels.push_back({reinterpret_cast<const void *>(prefill_small_kernel<BITS, true, SHARED_ROUNDS>), SmallLds<BITS, true>::BYTES});
+        }
         for (const auto &[kernel, bytes] : kernels) {
             if (int rc = int(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes))) return rc;
         }

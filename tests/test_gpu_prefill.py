@@ -424,11 +424,11 @@ def test_short_chunks_whose_scores_grow(kind, pos, tokens):
 
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("pos,tokens,kv", [(0, 1, 3), (190, 34, 1), (193, 31, 2), (225, 31, 3), (226, 31, 2), (207, 512, 2), (208, 514, 1), (288, 512, 2), (289, 512, 2),
-                                           (1, 900, 2), (4095, 1, 2), (4090, 12, 1)])
+                                           (1, 900, 2), (4095, 1, 2), (4090, 12, 1), (20000, 12, 2), (1997, 64, 2), (40000, 7, 2), (3000, 120, 2)])
 def test_short_chunks_whose_waves_share_their_blocks(kind, pos, tokens, kv):
     # one block; the last round with 6, 7 and 8 blocks (where the probabilities lie differs from the eighth on) and with the ninth
     # in a second round; the keys in the mean at which the rounds of 4-bit codes and of halves stop being shared, and one past them;
-    # parts of 8 blocks; 1, 2 and 3 kv heads
+    # parts of 8, 16, 24 and 32 blocks; 1, 2 and 3 kv heads
     call, out, p, want = chunk(kind, pos, tokens, kv)
     out.fill_(float("nan"))
     size = saetta.attention_prefill.workspace_bytes(p)
