@@ -171,15 +171,18 @@ template <int TOKENS>
 struct ConvPiece {
     static_assert(TOKENS >= CONV - 1, "every token that reads the state lies in the first piece");
     float4 taps[CONV], in[CONV - 1 + TOKENS];
-    __device__ __forceinline__ void request(const ChunkArgs &a, uint32_t c, uint32_t t0) {
+    __device__ __forceinline__ void request_taps(const ChunkArgs &a, uint32_t c) {
 #pragma unroll
         for (int j = 0; j < CONV; j++) taps[j] = reinterpret_cast<const float4 *>(a.conv_w + size_t(c) * CONV)[j];  // (by channel)
+    }
+    __device__ __forceinline__ void request_inputs(const ChunkArgs &a, uint32_t c, uint32_t t0) {
 #pragma unroll
         for (int i = 0; i < CONV - 1 + TOKENS; i++) {
             const int t = int(t0) + i - (CONV - 1);
             // (a token past the end: unused)
-            const float *row = t >= 0 ? a.x + size_t(min(uint32_t(t), a.tokens - 1)) * a.channels : a.conv_state + (t + CONV - 1) * a.channels;
-            in[i] = *reinterpret_cast<const float4 *>(row + c);
+            const float *from = t >= 0 ? a.x : a.conv_state;
+            const uint32_t row = t >= 0 ? min(uint32_t(t), a.tokens - 1) : uint32_t(t + CONV - 1);
+            in[i] = *reinterpret_cast<const float4 *>(from + size_t(row) * a.channels + c);
         }
     }
     __device__ __forceinline__ float4 output(int i) const {
@@ -237,7 +240,8 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
             if (quad >= quads || t0 >= a.tokens) return;
             const uint32_t cv = 2 * key_size + 4 * quad;
             ConvPiece<CONV_VALUES> values;
-            values.request(a, cv, t0);
+            values.request_taps(a, cv);
+            values.request_inputs(a, cv, t0);
 #pragma unroll
             for (int i = 0; i < CONV_VALUES; i++) {
                 const float4 y = values.output(i);
@@ -258,6 +262,7 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
     // c_t = sum of log g up to t, beta_t (tokens past the end: g = 1, beta = 0)
     auto gates = [&]() {
         if (gate_head < 0) return;
+        asm volatile("" : "+v"(gate_a), "+v"(gate_b), "+v"(gate_log), "+v"(gate_bias));  // (their first use is here: the loads that follow them wait for nothing)
         float g, beta, lg;
         fast_gates(gate_a + gate_bias, __expf(gate_log), gate_b, g, beta, &lg);
         const double c = inclusive_sum(gate_real ? double(lg) : 0.0);
@@ -274,15 +279,31 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
     if constexpr (CONVOLVE) {
         const uint32_t t0 = blk * C + CONV_QK * wave;
         const uint32_t cqk = (lane < 32 ? 0 : key_size - K_DIM) + khd * K_DIM + 4 * lane;  // q: lanes 0-31, k: lanes 32-63
+        // The taps, which are the same in all waves, go through LDS: channel c's four to piece c / 4 of plane c % 4.
+        constexpr int TAP_PLANE = 64 * 16 + 64;
+        static_assert(C * FROW * 4 + CONV * TAP_PLANE <= L::GATES, "the taps lie behind the f32 q and k");
+        unsigned char *taps_lds = lds + C * FROW * 4;
+        float4 tap = make_float4(0, 0, 0, 0);
+        if (tid < 2 * K_DIM) tap = reinterpret_cast<const float4 *>(a.conv_w)[(tid < K_DIM ? 0 : key_size - K_DIM) + khd * K_DIM + tid];
         ConvPiece<CONV_QK> qk;
-        qk.request(a, cqk, t0);
+        qk.request_inputs(a, cqk, t0);
+        if (tid < 2 * K_DIM) *reinterpret_cast<float4 *>(taps_lds + (tid & 3) * TAP_PLANE + (tid >> 2) * 16) = tap;
         gates();
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < CONV; j++) qk.taps[j] = *reinterpret_cast<const float4 *>(taps_lds + j * TAP_PLANE + lane * 16);
+        // (Every token's output, and all of them before the first store: loads and stores count in one order, and a load whose value
+        // nobody had taken would be waited for, behind all stores, at the next use of its registers.)
+        float4 y[CONV_QK];
 #pragma unroll
         for (int i = 0; i < CONV_QK; i++) {
-            const bool real = t0 + i < a.tokens;
-            const float4 y = real ? qk.output(i) : make_float4(0, 0, 0, 0);
-            *reinterpret_cast<float4 *>(qk_lds + (CONV_QK * wave + i) * FROW + 4 * lane) = y;
-            if (real) *reinterpret_cast<float4 *>(conv_out + size_t(t0 + i) * a.channels + cqk) = y;
+            const float4 made = qk.output(i);
+            y[i] = t0 + i < a.tokens ? made : make_float4(0, 0, 0, 0);
+            *reinterpret_cast<float4 *>(qk_lds + (CONV_QK * wave + i) * FROW + 4 * lane) = y[i];
+        }
+#pragma unroll
+        for (int i = 0; i < CONV_QK; i++) {
+            if (t0 + i < a.tokens) *reinterpret_cast<float4 *>(conv_out + size_t(t0 + i) * a.channels + cqk) = y[i];
         }
         if (t0 == 0) qk.keep_state(a, cqk);
         __syncthreads();
@@ -307,7 +328,13 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
                 kv[i] = *reinterpret_cast<const float4 *>(row + key_size);
             }
         }
-        if constexpr (!CONVOLVE) gates();
+        if constexpr (!CONVOLVE) {
+            gates();
+            if ((blk + 1) * C > a.tokens && !real) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) qv[i] = kv[i] = make_float4(0, 0, 0, 0);
+            }
+        }
         float qs = 0.0f, ks = 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -318,16 +345,16 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
         qs = group_reduce<8>(qs, SumOp());
         ks = group_reduce<8>(ks, SumOp());
         // (q's factor 1 / sqrt(128) is applied to the output: at unit length the lo parts stay clear of the f16 underflow;
-        // a token past the end: zeros, whatever was loaded)
-        const float qi = __builtin_amdgcn_rsqf(qs + a.eps), ki = __builtin_amdgcn_rsqf(ks + a.eps);
+        // a token past the end is zeros and stays so, whatever eps is)
+        const float qi = real ? __builtin_amdgcn_rsqf(qs + a.eps) : 0.0f, ki = real ? __builtin_amdgcn_rsqf(ks + a.eps) : 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; i += 2) {
             half4 h[2][2], l[2][2];  // [q | k][half of the piece]
 #pragma unroll
             for (int e = 0; e < 2; e++) {
                 const float4 qq = qv[i + e], kk = kv[i + e];
-                split4([&](int c) { return real ? (c == 0 ? qq.x : c == 1 ? qq.y : c == 2 ? qq.z : qq.w) * qi : 0.0f; }, h[0][e], l[0][e]);
-                split4([&](int c) { return real ? (c == 0 ? kk.x : c == 1 ? kk.y : c == 2 ? kk.z : kk.w) * ki : 0.0f; }, h[1][e], l[1][e]);
+                split4([&](int c) { return (c == 0 ? qq.x : c == 1 ? qq.y : c == 2 ? qq.z : qq.w) * qi; }, h[0][e], l[0][e]);
+                split4([&](int c) { return (c == 0 ? kk.x : c == 1 ? kk.y : c == 2 ? kk.z : kk.w) * ki; }, h[1][e], l[1][e]);
             }
             auto joined = [](const half4 (&x)[2]) { return __builtin_shufflevector(x[0], x[1], 0, 1, 2, 3, 4, 5, 6, 7); };
             const half8 a_qh = joined(h[0]), a_ql = joined(l[0]), a_kh = joined(h[1]), a_kl = joined(l[1]);
@@ -346,55 +373,75 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
     __syncthreads();
 
     // ---- k . k (first team) and q . k (second): wave tw of a team takes the rows t = 16 tw + .., the tiles of 16 columns s
-    // at and below the diagonal, transposed: lane (n, j) holds columns s = 16 nt + 4j + i of row t = 16 tw + n ----
-    const uint32_t team = wave >> 2, tw = wave & 3;
+    // at and below the diagonal, transposed: lane (n, j) holds columns s = 16 nt + 4j + i of row t = 16 tw + n.  The tiles go two
+    // by two, the columns of the first 32 tokens and, for the rows of the last 32, those of the last; what of a pair lies above the
+    // diagonal is masked.  The two waves of a SIMD, w and w + 4, have six tiles between them: the second team's rows go upwards.
+    // The decays e^(c_t - c_s), which wait for no product, are made between them. ----
+    const uint32_t team = wave >> 2, tw = team == 0 ? wave & 3 : 3 - (wave & 3), t_row = 16 * tw + n;
     floatx4 prod[4];
-    {
+    float decay[G][4][4];
+    auto products = [&](auto half) {
+        constexpr int nt0 = 2 * decltype(half)::value;
         const _Float16 *rh = team == 0 ? kh : qh, *rl = team == 0 ? kl : ql;
+        prod[nt0] = prod[nt0 + 1] = floatx4{0, 0, 0, 0};
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) {
-            prod[nt] = floatx4{0, 0, 0, 0};
-            if (nt <= int(tw)) {
+        for (int ks = 0; ks < 4; ks++) {
+            const int to = t_row * KROW + 32 * ks + 8 * j;
+            const half8 th = *reinterpret_cast<const half8 *>(rh + to), tl = *reinterpret_cast<const half8 *>(rl + to);
 #pragma unroll
-                for (int ks = 0; ks < 4; ks++) {
-                    const int to = (16 * tw + n) * KROW + 32 * ks + 8 * j, so = (16 * nt + n) * KROW + 32 * ks + 8 * j;
-                    prod[nt] = mma3(*reinterpret_cast<const half8 *>(kh + so), *reinterpret_cast<const half8 *>(kl + so),
-                                    *reinterpret_cast<const half8 *>(rh + to), *reinterpret_cast<const half8 *>(rl + to), prod[nt]);
-                }
+            for (int nt = nt0; nt < nt0 + 2; nt++) {
+                const int so = (16 * nt + n) * KROW + 32 * ks + 8 * j;
+                prod[nt] = mma3(*reinterpret_cast<const half8 *>(kh + so), *reinterpret_cast<const half8 *>(kl + so), th, tl, prod[nt]);
             }
         }
-    }
+#pragma unroll
+        for (int hh = 0; hh < G; hh++) {
+            const double ct = cum_lds(hh)[t_row];
+#pragma unroll
+            for (int nt = nt0; nt < nt0 + 2; nt++) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) decay[hh][nt][i] = __expf(float(ct - cum_lds(hh)[16 * nt + 4 * j + i]));
+            }
+        }
+    };
+    products(std::integral_constant<int, 0>());
+    if (tw >= 2) products(std::integral_constant<int, 1>());
     __syncthreads();  // the images are read: A and M go over them
 
     // ---- A and M.  What lies above the diagonal inside the 32 x 32 blocks is zero; the block above them is not read by
     // anybody and not written. ----
-#pragma unroll 1
-    for (int hh = 0; hh < G; hh++) {
-        const uint32_t t = 16 * tw + n;
-        const double ct = cum_lds(hh)[t];
-        const float beta_t = beta_lds(hh)[t];
+    auto matrices = [&](auto half) {
+        constexpr int nt0 = 2 * decltype(half)::value;
+        const bool diagonal = team == 0 && (nt0 == 2 || tw < 2);  // a diagonal 32 x 32 block of A
+        const uint32_t end = t_row + team;  // A has s < t, M s <= t
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) {
-            if (nt > int(tw | 1)) continue;  // (tile rows 2i and 2i + 1 end with column tile 2i + 1)
-            const uint32_t s0 = 16 * nt + 4 * j;
-            float x[4];
+        for (int hh = 0; hh < G; hh++) {
+            const float beta_t = team == 0 ? beta_lds(hh)[t_row] : 1.0f;
+            float x[2][4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const uint32_t s = s0 + i;
-                const float decayed = __expf(float(ct - cum_lds(hh)[s])) * prod[nt][i];
-                x[i] = team == 0 ? (s < t ? beta_t * decayed : 0.0f) : (s <= t ? decayed : 0.0f);
+            for (int e = 0; e < 2; e++) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[e][i] = 16 * (nt0 + e) + 4 * j + i < end ? beta_t * (decay[hh][nt0 + e][i] * prod[nt0 + e][i]) : 0.0f;
             }
-            if (team == 0 && (nt >> 1) == int(tw >> 1)) {  // a diagonal 32 x 32 block of A
-                *reinterpret_cast<floatx4 *>(diag_lds(hh, nt >> 1) + (t & 31) * DROW + (s0 & 31)) = floatx4{x[0], x[1], x[2], x[3]};
+            if (diagonal) {
+                float *dst = diag_lds(hh, nt0 / 2) + (t_row & 31) * DROW + 4 * j;
+                *reinterpret_cast<floatx4 *>(dst) = floatx4{x[0][0], x[0][1], x[0][2], x[0][3]};
+                *reinterpret_cast<floatx4 *>(dst + 16) = floatx4{x[1][0], x[1][1], x[1][2], x[1][3]};
             } else {  // M | the block of A below the diagonal, as an MFMA operand
-                half4 hi, lo;
-                split4([&](int i) { return x[i]; }, hi, lo);
-                _Float16 *dst = team == 0 ? half_img(hh, L::LBA_OFF) + (t - 32) * HROW + s0 : m_lds(hh) + t * TROW + s0;
-                *reinterpret_cast<half4 *>(dst) = hi;
-                *reinterpret_cast<half4 *>(dst + (team == 0 ? 32 * HROW : C * TROW)) = lo;
+                _Float16 *dst = team == 0 ? half_img(hh, L::LBA_OFF) + (t_row - 32) * HROW : m_lds(hh) + t_row * TROW;
+                const int lo_part = team == 0 ? 32 * HROW : C * TROW;
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    half4 hi, lo;
+                    split4([&](int i) { return x[e][i]; }, hi, lo);
+                    *reinterpret_cast<half4 *>(dst + 16 * (nt0 + e) + 4 * j) = hi;
+                    *reinterpret_cast<half4 *>(dst + 16 * (nt0 + e) + 4 * j + lo_part) = lo;
+                }
             }
         }
-    }
+    };
+    matrices(std::integral_constant<int, 0>());
+    if (tw >= 2) matrices(std::integral_constant<int, 1>());
     __syncthreads();
     // A staged matrix leaves in operand order, 16 bytes per piece, by `threads` threads: piece (part hi | lo, operand, lane
     // (n, j)) is row 16 w + n, columns 32 ks + 8j .. of the part's image; the operands are (w, ks) = (0, 0), (1, 0), (2, 0),
