@@ -123,7 +123,8 @@ struct PrepLds {
     // per head, over kh | kl once the products are taken: the two diagonal 32 x 32 blocks of A as f32, rows of
     // DROW (their inverses go over them, the product of the off-diagonal block over those later), then the
     // block below the diagonal and the inverse of the second diagonal block as f16 images
-    static constexpr int DROW = 32 + 4, D_BYTES = 32 * DROW * 4;
+    // (a diagonal block is 128 bytes longer than its rows: what the four 16 x 16 blocks of a solve read at once lies in different banks)
+    static constexpr int DROW = 32 + 4, D_BYTES = 32 * DROW * 4 + 128;
     static constexpr int HROW = 32 + 8, H_IMG = 32 * HROW * 2;  // f16 per row of a 32 x 32 image; bytes of one part
     static constexpr int W_OFF = 0, LBA_OFF = 2 * D_BYTES, XBB_OFF = LBA_OFF + 2 * H_IMG, HEAD_BYTES = XBB_OFF + 2 * H_IMG;
     static_assert(2 * H_IMG <= 2 * D_BYTES, "the product's images fit over the diagonal blocks");
@@ -456,20 +457,19 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
 
     // ---- T = (I + A)^-1 diag(beta), in 32 x 32 blocks: with L = I + A = [[L_AA, 0], [L_BA, L_BB]],
     //     T_AA = L_AA^-1 diag(beta_A),  T_BB = L_BB^-1 diag(beta_B),  T_BA = -L_BB^-1 (L_BA T_AA).
-    // The diagonal blocks by forward substitution, one wave per head: lane (column c, block) solves
-    // x_t = [t = c] - sum_{s < t} A_ts x_s and puts its column over A, which the wave has read.  The second team stores M.
-    // The block below the diagonal: two products on the matrix cores. ----
+    // A diagonal block's inverse goes over it, one wave per head, in the same way from 16 x 16 blocks: lane (column c = n, block j)
+    // solves x_t = [t = c] - sum_{s < t} A_ts x_s of its block, and the block below is two f32 products on the matrix cores.  The
+    // second team stores M meanwhile.  Then T_BA: two products in hi and lo parts. ----
     if (wave < G) {
-        const uint32_t c = lane & 31;
-        float *ad = diag_lds(wave, lane >> 5);
-        float x[32];
-        floatx4 av[2][8];  // a row and the next: no row waits for its own reads (the whole chunk, 262 tokens 34.9 -> 34.2 us)
+        float *ad = diag_lds(wave, j >> 1) + (j & 1) * (16 * DROW + 16);
+        float x[16];
+        floatx4 av[2][4];  // a row and the next: no row waits for its own reads
 #pragma unroll
-        for (int t = 0; t < 32; t++) {
+        for (int t = 0; t < 16; t++) {
 #pragma unroll
-            for (int s4 = 0; t < 31 && 4 * s4 <= t; s4++) av[(t + 1) & 1][s4] = *reinterpret_cast<const floatx4 *>(ad + (t + 1) * DROW + 4 * s4);
+            for (int s4 = 0; t < 15 && 4 * s4 <= t; s4++) av[(t + 1) & 1][s4] = *reinterpret_cast<const floatx4 *>(ad + (t + 1) * DROW + 4 * s4);
             __builtin_amdgcn_sched_barrier(0);
-            floatx4 part4 = {0, 0, 0, 0};  // (four chains of sums instead of one of up to 31)
+            floatx4 part4 = {0, 0, 0, 0};  // (four chains of sums instead of one of up to 15)
 #pragma unroll
             for (int s4 = 0; 4 * s4 < t; s4++) {
 #pragma unroll
@@ -477,10 +477,32 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
                     if (4 * s4 + e < t) part4[e] += av[t & 1][s4][e] * x[4 * s4 + e];
                 }
             }
-            x[t] = (uint32_t(t) == c ? 1.0f : 0.0f) - ((part4[0] + part4[1]) + (part4[2] + part4[3]));
+            x[t] = (uint32_t(t) == n ? 1.0f : 0.0f) - ((part4[0] + part4[1]) + (part4[2] + part4[3]));
         }
 #pragma unroll
-        for (int t = 0; t < 32; t++) ad[t * DROW + c] = x[t];  // (behind the loop: in it, the next row's reads would wait for x_t)
+        for (int t = 0; t < 16; t++) ad[t * DROW + n] = x[t];  // (behind the loop: in it, the next row's reads would wait for x_t)
+        // the block below them, for both halves: k index 4j + i in step i, so that the first product's result is the second's operand
+        floatx4 w[2], y[2];
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            const float *d = diag_lds(wave, half);
+            const floatx4 below = *reinterpret_cast<const floatx4 *>(d + (16 + n) * DROW + 4 * j);
+            w[half] = floatx4{0, 0, 0, 0};
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(below[i], d[(4 * j + i) * DROW + n], w[half], 0, 0, 0);
+        }
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            const floatx4 second = *reinterpret_cast<const floatx4 *>(diag_lds(wave, half) + (16 + n) * DROW + 16 + 4 * j);
+            y[half] = floatx4{0, 0, 0, 0};
+#pragma unroll
+            for (int i = 0; i < 4; i++) y[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(second[i], w[half][i], y[half], 0, 0, 0);
+        }
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) diag_lds(wave, half)[(16 + 4 * j + i) * DROW + n] = -y[half][i];
+        }
     } else if (team == 1) {
 #pragma unroll
         for (int hh = 0; hh < G; hh++) leave(hh, ws_v(hh) + 2 * T_GL, tid - 256, 256);
