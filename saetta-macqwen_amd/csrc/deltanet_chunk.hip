@@ -85,6 +85,8 @@ typedef _Float16 half2_ __attribute__((ext_vector_type(2)));
 template <class F>
 __device__ __forceinline__ void split4(F &&value, half4 &hi, half4 &lo) {
     half2_ h[2], l[2];
+    float minus = -1.0f;  // not as a constant: x - hi is then one v_fma_mix, taken from and rounded to f16, and not three instructions
+    asm("" : "+s"(minus));
 #pragma unroll
     for (int p = 0; p < 2; p++) {
         float x = value(2 * p), y = value(2 * p + 1);
@@ -92,7 +94,7 @@ __device__ __forceinline__ void split4(F &&value, half4 &hi, half4 &lo) {
         uint32_t both = __builtin_bit_cast(uint32_t, half2_{(_Float16)x, (_Float16)y});
         asm("" : "+v"(both));
         h[p] = __builtin_bit_cast(half2_, both);
-        l[p] = half2_{(_Float16)(x - (float)h[p][0]), (_Float16)(y - (float)h[p][1])};
+        l[p] = half2_{(_Float16)__builtin_fmaf((float)h[p][0], minus, x), (_Float16)__builtin_fmaf((float)h[p][1], minus, y)};
     }
     hi = __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3), lo = __builtin_shufflevector(l[0], l[1], 0, 1, 2, 3);
 }
@@ -363,12 +365,6 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
             const int at = t * KROW + 8 * piece;
             *reinterpret_cast<half8 *>(kh + at) = a_kh, *reinterpret_cast<half8 *>(kl + at) = a_kl;
             *reinterpret_cast<half8 *>(qh + at) = a_qh, *reinterpret_cast<half8 *>(ql + at) = a_ql;
-            if (writer) {
-                // operand (wave t / 16, k-step), lane (n = t % 16, j): eight tokens in a row are whole lines
-                unsigned char *g = ws_k + ((((t >> 4) * 4 + (piece >> 2)) * 64 + (piece & 3) * 16 + (t & 15)) * 16);
-                *reinterpret_cast<half8 *>(g) = a_kh, *reinterpret_cast<half8 *>(g + K_GL) = a_kl;
-                *reinterpret_cast<half8 *>(g + 2 * K_GL) = a_qh, *reinterpret_cast<half8 *>(g + 3 * K_GL) = a_ql;
-            }
         }
     }
     __syncthreads();
@@ -389,6 +385,10 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
         for (int ks = 0; ks < 4; ks++) {
             const int to = t_row * KROW + 32 * ks + 8 * j;
             const half8 th = *reinterpret_cast<const half8 *>(rh + to), tl = *reinterpret_cast<const half8 *>(rl + to);
+            if (nt0 == 0 && writer) {  // the rows' operands are what the chain kernel reads: operand (wave tw, k-step), whole lines a store
+                unsigned char *g = ws_k + team * (2 * K_GL) + ((tw * 4 + ks) * 64 + lane) * 16;
+                *reinterpret_cast<half8 *>(g) = th, *reinterpret_cast<half8 *>(g + K_GL) = tl;
+            }
 #pragma unroll
             for (int nt = nt0; nt < nt0 + 2; nt++) {
                 const int so = (16 * nt + n) * KROW + 32 * ks + 8 * j;
