@@ -254,8 +254,9 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
             return;
         }
     }
-    // ---- the gates' inputs of head h0 + gate_head, one of the last G waves: asked for first ----
-    const int gate_head = int(wave) - (PREP_WAVES - G);
+    // ---- the gates' inputs of head h0 + gate_head, one of the first G waves: asked for first, and used when the wave has made its
+    // q and k: the first wave of a SIMD, which has precedence, then waits for the second ----
+    const int gate_head = wave < G ? int(wave) : -1;
     const bool gate_real = blk * C + lane < a.tokens;
     float gate_a = 0.0f, gate_b = 0.0f, gate_log = 0.0f, gate_bias = 0.0f;
     if (gate_head >= 0) {
@@ -291,7 +292,6 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
         ConvPiece<CONV_QK> qk;
         qk.request_inputs(a, cqk, t0);
         if (tid < 2 * K_DIM) *reinterpret_cast<float4 *>(taps_lds + (tid & 3) * TAP_PLANE + (tid >> 2) * 16) = tap;
-        gates();
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < CONV; j++) qk.taps[j] = *reinterpret_cast<const float4 *>(taps_lds + j * TAP_PLANE + lane * 16);
@@ -309,6 +309,7 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
             if (t0 + i < a.tokens) *reinterpret_cast<float4 *>(conv_out + size_t(t0 + i) * a.channels + cqk) = y[i];
         }
         if (t0 == 0) qk.keep_state(a, cqk);
+        gates();
         __syncthreads();
     }
 
@@ -332,7 +333,6 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
             }
         }
         if constexpr (!CONVOLVE) {
-            gates();
             if ((blk + 1) * C > a.tokens && !real) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) qv[i] = kv[i] = make_float4(0, 0, 0, 0);
@@ -366,6 +366,7 @@ __global__ __launch_bounds__(PREP_THREADS, 4) void deltanet_chunk_prepare_kernel
             *reinterpret_cast<half8 *>(kh + at) = a_kh, *reinterpret_cast<half8 *>(kl + at) = a_kl;
             *reinterpret_cast<half8 *>(qh + at) = a_qh, *reinterpret_cast<half8 *>(ql + at) = a_ql;
         }
+        if constexpr (!CONVOLVE) gates();
     }
     __syncthreads();
 
