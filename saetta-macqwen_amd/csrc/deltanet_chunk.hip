@@ -116,7 +116,9 @@ __device__ __forceinline__ floatx4 mma3(half8 ah, half8 al, half8 bh, half8 bl, 
 // and stores it meanwhile; the products are taken as their transposes, so that a lane's four results lie in a row and
 // leave as one 8-byte store; the solve has a lane to a column, with no sums over lanes.
 // Measured, us, against four waves that did it all in order: 1000 tokens 22.7 -> 15.8, 2047 28.3 -> 26.4, 4096 57.4 -> 49.8;
-// with the conv inside, 512 tokens 31.5 -> 20.3.
+// with the conv inside, 512 tokens 31.5 -> 20.3.  Of the 34 000 cycles of a block with its conv most were waits for something that
+// need not be waited for, or one wave's work: without them 25 000, and 20 400 of 25 900 without the conv (whole chunk: 130
+// tokens 28.9 -> 25.3, 500 38.7 -> 35.6, 1000 60.2 -> 57.9, 2300 127.2 -> 121.4, 4096 230.3 -> 223.3).
 // LDS: the four q / k images; once the products are taken, the heads' A (f32) go over kh | kl, their M
 // images and later their T images over qh | ql (and more), so that they leave as whole 16-byte stores.
 constexpr int PREP_THREADS = 512, PREP_WAVES = PREP_THREADS / 64;
@@ -197,7 +199,7 @@ struct ConvPiece {
                                 j == 0 ? taps[2].x : j == 1 ? taps[2].y : j == 2 ? taps[2].z : taps[2].w, j == 0 ? taps[3].x : j == 1 ? taps[3].y : j == 2 ? taps[3].z : taps[3].w};
             sum.x += w[0] * v.x, sum.y += w[1] * v.y, sum.z += w[2] * v.z, sum.w += w[3] * v.w;
         }
-        return make_float4(silu_f(sum.x), silu_f(sum.y), silu_f(sum.z), silu_f(sum.w));
+        return silu4_f(sum);
     }
     // the first block's piece: the chunk's last inputs become the conv's state, which only that piece has read
     __device__ __forceinline__ void keep_state(const ChunkArgs &a, uint32_t c) const {

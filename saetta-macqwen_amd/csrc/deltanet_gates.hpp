@@ -40,5 +40,18 @@ __device__ __forceinline__ float silu_f(float x) {
     const float y = x * r, off = fmaf(-d, y, x), y_down = y * down;
     return off == off ? fmaf(off, r * down, y_down) : y_down;
 }
+// silu_f of four values: where none of the wavefront's is beyond +-44, and none therefore meets a bound above, the same steps
+// without the bounds (eleven instructions a value, not eighteen; the same bits).
+__device__ __forceinline__ float4 silu4_f(float4 x) {
+    if (__any(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))) > 44.0f)) return make_float4(silu_f(x.x), silu_f(x.y), silu_f(x.z), silu_f(x.w));
+    auto inside = [](float v) {
+        constexpr float LOG2_E = 0x1.715476p+0f, LOG2_E_REST = 0x1.4ae0cp-26f, LN_2 = 0x1.62e43p-1f;
+        const float at = -LOG2_E * v, rest = fmaf(-LOG2_E_REST, v, fmaf(-LOG2_E, v, LOG2_E * v));
+        const float e = __builtin_amdgcn_exp2f(at), d = fmaf(e, LN_2 * rest, e) + 1.0f, r = __builtin_amdgcn_rcpf(d);
+        const float y = v * r;
+        return fmaf(fmaf(-d, y, v), r, y);
+    };
+    return make_float4(inside(x.x), inside(x.y), inside(x.z), inside(x.w));
+}
 
 }  // namespace saetta

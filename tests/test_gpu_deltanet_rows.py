@@ -334,6 +334,34 @@ def test_conv_of_four_channels_a_thread_at_the_edges_of_its_tiles(tokens):
     check_against_oracle(Layer(2, 4, 16, 4, seed=tokens), 2 * tokens, [tokens, tokens], snapshots=True)
 
 
+@pytest.mark.parametrize("tokens", [128, 135, 191, 512])
+def test_the_conv_inside_a_chunk_gives_the_convs_bits(tokens):
+    # The conv's activation has a short form for wavefronts without a value beyond +-44: values on both sides of that line and of
+    # the exponential's own ends, infinities and NaN, in some wavefronts and not in others.
+    layer = Layer(4, 8, 128, 4, seed=tokens)
+    gen = torch.Generator(device="cuda").manual_seed(tokens)
+    x, z, a, b = (torch.randn(tokens, n, generator=gen, device="cuda") for n in (layer.channels, layer.val, 8, 8))
+    x[5::9, 3::50] *= 30
+    x[11::17, ::77] *= 400
+    x[tokens // 2, 40], x[tokens // 2 + 20, 1500], x[tokens - 1, 700] = float("inf"), -float("inf"), float("nan")
+    weights = [dev(w) for w in (layer.conv_w, layer.a_log, layer.dt_bias, layer.norm)]
+
+    def run(inside):
+        conv, state = layer.zero_state()
+        mixed, y, plan = torch.empty_like(x), torch.empty_like(z), saetta.Plan()
+        saetta.deltanet_conv_rows(plan, x, weights[0], conv, mixed, layer.channels, layer.kernel, tokens)
+        if inside:
+            saetta.deltanet_rows(plan, mixed, a, b, weights[1], weights[2], state, z, weights[3], y, 4, 8, 128, tokens, EPS)
+        plan.build().run()
+        torch.cuda.synchronize()
+        return mixed, conv
+
+    inside, alone = run(True), run(False)
+    assert (inside[0].abs() > 44).any() and inside[0].isnan().any()
+    for one, two in zip(inside, alone):
+        assert torch.equal(one.isnan(), two.isnan()) and torch.equal(one.nan_to_num(7.0), two.nan_to_num(7.0))
+
+
 @pytest.mark.parametrize("k_heads,v_heads,v_dim,first,second", [(16, 32, 128, 3264, 129), (8, 16, 256, 5248, 190), (32, 32, 64, 2368, 131)])
 def test_a_chunk_past_the_memorys_cache_equals_its_pieces(k_heads, v_heads, v_dim, first, second):
     # From 208 MB of `mixed` and workspace on, the chain's operands are brought into L2 ahead of their use: the one call is past that
