@@ -759,14 +759,23 @@ __global__ __launch_bounds__(512) void deltanet_chunk_chain_kernel(ChunkArgs a) 
         __builtin_amdgcn_sched_barrier(0);
         request_tm(blk + 2, b);
         __builtin_amdgcn_sched_barrier(0);
-        const uint32_t tok = blk * C + 16 * wave + n;
-        if (real && tok < a.tokens) {
-            float *o = a.o + (size_t(tok) * a.v_heads + h) * a.v_dim + DV * slice + 4 * j;
+        // AHEAD: lane 4t + p takes piece p of token t's 64 bytes, so that four lanes store them in a row (a store of 64 lanes that
+        // are apart takes the memory pipe 64 cycles and not 16, and leaves in more pieces: 4096 tokens 224.2 -> 220.6 us, 3500 192.7 ->
+        // 190.3; where the memory's cache takes the stores it gives nothing, 2300 121.2 -> 121.3, 130 25.5 -> 25.6)
+        const uint32_t row = AHEAD ? lane >> 2 : n, piece = AHEAD ? lane & 3 : j, tok = blk * C + 16 * wave + row;
+        floatx4 out[NT];
 #pragma unroll
-            for (int vt = 0; vt < NT; vt++) {
+        for (int vt = 0; vt < NT; vt++) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) o[16 * vt + i] = Q_SCALE * (held_gam * held[vt][i] + mu[vt][i]);
+            for (int i = 0; i < 4; i++) {
+                const float x = Q_SCALE * (held_gam * held[vt][i] + mu[vt][i]);
+                out[vt][i] = AHEAD ? __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(int(4 * (16 * piece + row)), __builtin_bit_cast(int, x))) : x;
             }
+        }
+        if (real && tok < a.tokens) {
+            float *o = a.o + (size_t(tok) * a.v_heads + h) * a.v_dim + DV * slice + 4 * piece;
+#pragma unroll
+            for (int vt = 0; vt < NT; vt++) *reinterpret_cast<floatx4 *>(o + 16 * vt) = out[vt];
         }
     };
 
@@ -1041,8 +1050,9 @@ int run_deltanet_chunk(hipStream_t stream, const float *mixed, const float *a, c
     float *conv_out = nullptr;
     // The conv inside: while every workgroup, the blocks' and the values', has a CU to itself.  Where they share one, a
     // block's chain of phases is held up by the conv beside it, and the conv's own launch is the better one (whole chunk,
-    // us, inside against apart: 200 tokens 34.2 and 35.3, 333 38.2 and 39.4, 512 43.4 and 45.5; 750 59.5 and 55.6, 1000 70.9
-    // and 66.6, 2047 126 and 120).
+    // us, inside against apart: 512 tokens 35.8 and 39.3; 513 41.8 and 39.3, 640 45.2 and 43.4, 800 50.7 and 50.4, 1000 58.3 and 58.1,
+    // 2047 126 and 120; the values' conv alone as a launch of its own: 513 41.8, 1000 57.4, 2300 124.7 instead of 122.0, 4096 226.7
+    // instead of 222.6).
     const uint32_t columns = (p.v_heads * p.v_dim / 4 + PREP_THREADS - 1) / PREP_THREADS, value_groups = columns * ((p.tokens + CONV_VALUES - 1) / CONV_VALUES);
     const bool conv_inside = two_heads && p.v_dim == CONV_V && nblocks * p.k_heads + value_groups <= cu_count();
     if (conv_inside && list && take_conv(*list, args, conv_out)) {
