@@ -156,6 +156,9 @@ __device__ __forceinline__ void conv_state_move(const float *x, float *state, ui
 // reads 7 rows, 3 of them a second time out of the L2, and is done 8 times as soon as one of 32.  Conv alone, tiles of 32
 // -> 4: 40 tokens 13.9 -> 4.6 us, 2100 34.6 -> 27, 4096 50.6 -> 49.9 (268 MB at 5.4 TB/s); whole layer, us, tiles of
 // 32 / 16 / 8 / 4: 40 tokens 25.7 / 21.1 / 18.8 / 17.6, 2100 150 / 147 / 145 / 142, 4095 269 / 273 / 269 / 267.
+// Vector instructions are issued for half of its time: the activation's short form takes 0.2 to 1 us of the layer (40 tokens 16.85 -> 16.65,
+// 513 39.3 -> 39.1, 2300 121.7 -> 120.9, 4096 221.6 -> 220.5; the norm's 2300 120.9 -> 120.7).  The taps by way of LDS, whole lines to a load
+// instead of 64 bytes to a lane, give nothing (40 tokens 16.9, 2300 121.5).
 constexpr uint32_t CONV4_TILE = 4;
 constexpr uint32_t CONV4_TAPS = 4, CONV4_FROM = SAETTA_MAX_ROWS + 1;  // (taps it is made for; tokens from which it is taken)
 static_assert(CONV4_TILE >= CONV4_TAPS - 1, "every token that reads the state lies in the first tile");
@@ -193,8 +196,8 @@ __global__ __launch_bounds__(256) void deltanet_conv_rows4_kernel(const float *_
         for (int j = 0; j < KS - 1; j++) {
             acc.x += taps[j].x * win[j].x, acc.y += taps[j].y * win[j].y, acc.z += taps[j].z * win[j].z, acc.w += taps[j].w * win[j].w;
         }
-        o4[size_t(t) * quads + c4] = make_float4(silu_f(acc.x + taps[KS - 1].x * xt[u].x), silu_f(acc.y + taps[KS - 1].y * xt[u].y),
-                                                 silu_f(acc.z + taps[KS - 1].z * xt[u].z), silu_f(acc.w + taps[KS - 1].w * xt[u].w));
+        o4[size_t(t) * quads + c4] = silu4_f(make_float4(acc.x + taps[KS - 1].x * xt[u].x, acc.y + taps[KS - 1].y * xt[u].y,
+                                                         acc.z + taps[KS - 1].z * xt[u].z, acc.w + taps[KS - 1].w * xt[u].w));
 #pragma unroll
         for (int j = 0; j + 1 < KS - 1; j++) win[j] = win[j + 1];
         win[KS - 2] = xt[u];
@@ -474,7 +477,8 @@ __global__ __launch_bounds__(256) void deltanet_gated_norm_wide_kernel(float *y,
     const float4 o = *yp, g = reinterpret_cast<const float4 *>(z)[size_t(pair) * LP + part], w = reinterpret_cast<const float4 *>(norm_w)[part];
     const float total = group_reduce<LP>(o.x * o.x + o.y * o.y + o.z * o.z + o.w * o.w, SumOp());
     const float inv = 1.0f / sqrtf(total / float(4 * LP) + eps);
-    *yp = make_float4(o.x * (inv * w.x) * silu_f(g.x), o.y * (inv * w.y) * silu_f(g.y), o.z * (inv * w.z) * silu_f(g.z), o.w * (inv * w.w) * silu_f(g.w));
+    const float4 open = silu4_f(g);
+    *yp = make_float4(o.x * (inv * w.x) * open.x, o.y * (inv * w.y) * open.y, o.z * (inv * w.z) * open.z, o.w * (inv * w.w) * open.w);
 }
 
 // y = o / sqrt(mean(o^2) + eps) * norm_w * silu(z) per (token, value head), in place on y:

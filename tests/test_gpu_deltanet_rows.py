@@ -334,32 +334,59 @@ def test_conv_of_four_channels_a_thread_at_the_edges_of_its_tiles(tokens):
     check_against_oracle(Layer(2, 4, 16, 4, seed=tokens), 2 * tokens, [tokens, tokens], snapshots=True)
 
 
-@pytest.mark.parametrize("tokens", [128, 135, 191, 512])
-def test_the_conv_inside_a_chunk_gives_the_convs_bits(tokens):
-    # The conv's activation has a short form for wavefronts without a value beyond +-44: values on both sides of that line and of
-    # the exponential's own ends, infinities and NaN, in some wavefronts and not in others.
+@pytest.mark.parametrize("tokens", [9, 128, 135, 191, 512, 517])
+def test_the_conv_of_a_chunk_gives_the_bits_of_few_rows(tokens):
+    # The activation of four channels a thread has a short form for wavefronts without a value beyond +-44: values on both sides of
+    # that line and of the exponential's own ends, infinities and NaN, in some wavefronts and not in others.
     layer = Layer(4, 8, 128, 4, seed=tokens)
     gen = torch.Generator(device="cuda").manual_seed(tokens)
     x, z, a, b = (torch.randn(tokens, n, generator=gen, device="cuda") for n in (layer.channels, layer.val, 8, 8))
     x[5::9, 3::50] *= 30
-    x[11::17, ::77] *= 400
-    x[tokens // 2, 40], x[tokens // 2 + 20, 1500], x[tokens - 1, 700] = float("inf"), -float("inf"), float("nan")
+    x[3::17, ::77] *= 400
+    x[tokens // 2, 40], x[tokens // 3, 1500], x[tokens - 1, 700] = float("inf"), -float("inf"), float("nan")
     weights = [dev(w) for w in (layer.conv_w, layer.a_log, layer.dt_bias, layer.norm)]
 
-    def run(inside):
+    def run(rows):
         conv, state = layer.zero_state()
         mixed, y, plan = torch.empty_like(x), torch.empty_like(z), saetta.Plan()
-        saetta.deltanet_conv_rows(plan, x, weights[0], conv, mixed, layer.channels, layer.kernel, tokens)
-        if inside:
+        for at in range(0, tokens, rows):
+            n = min(rows, tokens - at)
+            saetta.deltanet_conv_rows(plan, x[at:at + n], weights[0], conv, mixed[at:at + n], layer.channels, layer.kernel, n)
+        if rows == tokens:
             saetta.deltanet_rows(plan, mixed, a, b, weights[1], weights[2], state, z, weights[3], y, 4, 8, 128, tokens, EPS)
         plan.build().run()
         torch.cuda.synchronize()
         return mixed, conv
 
-    inside, alone = run(True), run(False)
-    assert (inside[0].abs() > 44).any() and inside[0].isnan().any()
-    for one, two in zip(inside, alone):
+    whole, few = run(tokens), run(8)
+    assert (whole[0].abs() > 44).any() and whole[0].isnan().any()
+    for one, two in zip(whole, few):
         assert torch.equal(one.isnan(), two.isnan()) and torch.equal(one.nan_to_num(7.0), two.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("tokens", [40, 130])
+def test_the_gate_of_a_chunk_over_all_of_its_range(tokens):
+    # y = n silu(z), with n the same whatever z is: against z = 1, in 64 bits.  Each side rounds n, silu and their product: 4 ulp each.
+    layer = Layer(2, 4, 128, 4, seed=tokens)
+    gen = torch.Generator(device="cuda").manual_seed(tokens)
+    mixed, a, b = (torch.randn(tokens, n, generator=gen, device="cuda") for n in (layer.channels, 4, 4))
+    weights = [dev(w) for w in (layer.a_log, layer.dt_bias, layer.norm)]
+    z = torch.randn(tokens, layer.val, generator=gen, device="cuda")
+    z[1::2] *= 20  # (beyond +-44 in some wavefronts only)
+    z[5] = torch.linspace(-100, 100, layer.val, device="cuda")
+
+    def run(z):
+        _, state = layer.zero_state()
+        y, plan = torch.empty_like(z), saetta.Plan()
+        saetta.deltanet_rows(plan, mixed, a, b, weights[0], weights[1], state, z, weights[2], y, 2, 4, 128, tokens, EPS)
+        plan.build().run()
+        torch.cuda.synchronize()
+        return y.double()
+
+    silu = lambda t: t.double() * torch.sigmoid(t.double())
+    one = torch.ones_like(z)
+    want = run(one) / silu(one) * silu(z)
+    assert ((run(z) - want).abs() <= 8 * 2.0 ** -23 * want.abs() + 1e-36).all()
 
 
 @pytest.mark.parametrize("k_heads,v_heads,v_dim,first,second", [(16, 32, 128, 3264, 129), (8, 16, 256, 5248, 190), (32, 32, 64, 2368, 131)])
