@@ -615,7 +615,8 @@ struct ChainBlock {
 // (`touch`).  What the conv and the prepare kernel have just written is served from the memory's cache (256 MB) while it fits, fast
 // enough for loads two blocks ahead, and the pieces are an eighth more traffic: whole chunk, us, without -> with: 1000 tokens 61.2
 // -> 62.8, 2300 128.9 -> 133.5, 3200 180.6 -> 182.0; past it the first of a line's readers waits for memory: 3500 205.1 -> 199.9, 4096
-// 248.0 -> 230.5 (6 blocks ahead 232.3, without the values' lines 238.7).
+// 248.0 -> 230.5 (6 blocks ahead 232.3, without the values' lines 238.7).  With the rest as it is now: 2300 123.8 -> 127.0, 3000 159.3 ->
+// 160.9, 3150 171.7 -> 171.7, 3250 177.7 -> 176.3.
 constexpr uint32_t AHEAD_BLOCKS = 3;
 constexpr size_t AHEAD_FROM = size_t(208) << 20;  // bytes of `mixed` and the workspace: 3300 tokens of the model's shape
 template <bool AHEAD>
