@@ -1493,16 +1493,25 @@ uint32_t parts_of(uint32_t pos, uint32_t tokens, uint32_t part_blocks) {
     return (uint32_t((uint64_t(pos) + tokens + BK - 1) / BK) + part_blocks - 1) / part_blocks;
 }
 
+// The tiles' keys in parts of `blocks` blocks, n of them at most, which take `bytes` behind the images; not in parts where blocks is 0.
+struct TileParts {
+    uint32_t blocks, n;
+    size_t bytes;
+};
 // How a chunk's launches are laid out: the row groups' own launch (small), with their keys in parts of `small_part_blocks`
-// blocks where that is not 0 and there is room for them; or tiles, with their keys in parts of `part_blocks` blocks where
-// that is not 0.
+// blocks where that is not 0 and there is room for them; or tiles, with their keys in the parts of tiles of WIDE_TQ tokens (wide) where
+// those are ahead and there is room for them, else in those of tiles of TQ (narrow) where there is room for these, else whole.  Wide parts
+// are often more than narrow ones, for a few per cent; whole keys are 1.2 to 5 times as slow (halves, wide | narrow | whole: 447 tokens at
+// 86225 616 us in 229 MB | 632 in 207 | 1870, 288 at 129584 641 in 318 MB | 730 in 290 | 3130, 2210 at 5272 261 in 126 MB | 266 in 89 | 307).
 struct FlashPlan {
     bool small;  // without parts, the row groups' launch is ahead of the tiles
-    uint32_t small_part_blocks, cus, part_blocks, nparts;
-    bool wide;  // the parts are those of tiles of WIDE_TQ tokens
-    size_t plain, parts, small_parts;  // bytes of workspace: the images and the tile count; the parts behind them; the row groups' parts, instead of both
-    size_t tiles() const { return plain + parts; }
+    uint32_t small_part_blocks, cus;
+    TileParts narrow, wide;
+    size_t plain, small_parts;  // bytes of workspace: the images and the tile count; the row groups' parts, instead of the images and all
+    size_t tiles() const { return plain + (wide.blocks ? wide.bytes : narrow.bytes); }
     size_t bytes() const { return tiles() > small_parts ? tiles() : small_parts; }
+    bool takes_wide(size_t have) const { return wide.blocks && have >= plain + wide.bytes; }
+    bool takes_narrow(size_t have) const { return narrow.blocks && have >= plain + narrow.bytes; }
 };
 
 // A tile is one workgroup's work, and 16 tokens of 2 kv heads are all a CU gets of it: chunks under 2048 tokens leave CUs
@@ -1552,7 +1561,7 @@ FlashPlan tiles_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, float &ti
     const float chip_us = 1.0f / (CHIP_BLOCKS_PER_US * float(f.cus));
     const float unsplit = rounds_us(f.cus, ntiles * kv_heads, float(longest), float(shortest), TILE_US, BLOCK_US, chip_us);
     float best = 0.95f * unsplit;
-    auto in_parts = [&](bool wide) {
+    auto in_parts = [&](bool wide, TileParts &of) {
         const uint32_t tq = wide ? WIDE_TQ : TQ, n = (tokens + tq - 1) / tq;
         const float high = float(tile_blocks(pos, tokens, n - 1, tq)), low = float(tile_blocks(pos, tokens, 0, tq));
         for (uint32_t parts = 2; parts <= 32; parts++) {
@@ -1562,20 +1571,19 @@ FlashPlan tiles_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, float &ti
             const float mid = 0.5f * (high + low) * float(n * kv_heads) / float(items);
             const float us = (wide ? rounds_us(f.cus, items, mid, mid, WIDE_PART_US, WIDE_BLOCK_US, WIDE_GAIN * 2.0f * chip_us) : rounds_us(f.cus, items, mid, mid, PART_US, BLOCK_US, chip_us)) +
                              MERGE_US + (wide ? 2.0f : 1.0f) * MERGE_ITEM_US * float(items);
-            if (us < best) best = us, f.part_blocks = pb, f.wide = wide;
+            if (us < best) best = us, of.blocks = pb;
         }
+        if (!of.blocks) return;
+        of.n = parts_of(pos, tokens, of.blocks);
+        of.bytes = parts_bytes(tokens, kv_heads, of.n);
     };
-    in_parts(false);
-    if (!f.part_blocks) best = unsplit;
+    in_parts(false, f.narrow);
+    if (!f.narrow.blocks) best = unsplit;
     // (what the row groups are weighed against stays what it was before there were wide tiles: which chunks need no workspace is
     // decided there)
     const float narrow = best;
     best *= 0.985f;
-    in_parts(true);
-    if (f.part_blocks) {
-        f.nparts = parts_of(pos, tokens, f.part_blocks);
-        f.parts = parts_bytes(tokens, kv_heads, f.nparts);
-    }
+    in_parts(true, f.wide);
     // (never less than 5 us, what short contexts' images were counted at when the row groups came in: a chunk that goes to them
     // without parts needs no workspace, and who calls it without one, recording or under capture, goes on to)
     const float prepare_us = PREPARE_US + PREPARE_KEY_US * float(pos + tokens) * float(kv_heads);
@@ -1753,10 +1761,10 @@ int launch_small(hipStream_t stream, int bits, const uint16_t *q, const void *kd
     return launch_status(what);
 }
 
-// The tiles' launches in a workspace of at least plan.plain bytes, plan.tiles() with `split`.
+// The tiles' launches in a workspace of `have` bytes, plan.plain at least.
 int launch_flash(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata, const uint16_t *ks,
                  const uint16_t *kz, const uint16_t *vs, const uint16_t *vz, const float *q_and_gate, float *out,
-                 const saetta_flash_params &p, void *workspace, bool split, bool exact, const FlashPlan &plan, const char *what) {
+                 const saetta_flash_params &p, void *workspace, size_t have, bool exact, const FlashPlan &plan, const char *what) {
     const uint64_t rows = uint64_t(p.pos) + p.tokens;
     unsigned char *ws = static_cast<unsigned char *>(workspace);
     uint32_t *tiles_taken = reinterpret_cast<uint32_t *>(ws + images_bytes(p.pos, p.tokens, p.kv_heads));
@@ -1764,15 +1772,17 @@ int launch_flash(hipStream_t stream, int bits, const uint16_t *q, const void *kd
     const uint32_t ntiles = (p.tokens + TQ - 1) / TQ;
     PrefillArgs a{q, ws, q_and_gate, out, p.heads, p.kv_heads, p.pos, p.tokens, p.scale, nblocks, tiles_taken, 0, nullptr, nullptr};
     // one workgroup per CU at most: a workgroup's LDS ring fills a CU, and further tiles are taken in the kernel
-    if (split && plan.part_blocks) {
-        a.part_blocks = plan.part_blocks;
+    const bool wide = plan.takes_wide(have);
+    if (wide || plan.takes_narrow(have)) {
+        const TileParts &parts = wide ? plan.wide : plan.narrow;
+        a.part_blocks = parts.blocks;
         a.part_o = reinterpret_cast<float *>(ws + plan.plain);
-        a.part_ml = reinterpret_cast<float *>(ws + plan.plain + size_t(plan.nparts) * ntiles * p.kv_heads * PART_O_BYTES);
-        const uint32_t total = prefill_items(p.pos, p.tokens, plan.part_blocks, plan.wide ? WIDE_TQ : TQ) * p.kv_heads;
-        auto *kernel = plan.wide ? (exact ? attention_prefill_kernel<true, true, true> : attention_prefill_kernel<true, false, true>)
-                                 : (exact ? attention_prefill_kernel<true, true, false> : attention_prefill_kernel<true, false, false>);
+        a.part_ml = reinterpret_cast<float *>(ws + plan.plain + size_t(parts.n) * ntiles * p.kv_heads * PART_O_BYTES);
+        const uint32_t total = prefill_items(p.pos, p.tokens, parts.blocks, wide ? WIDE_TQ : TQ) * p.kv_heads;
+        auto *kernel = wide ? (exact ? attention_prefill_kernel<true, true, true> : attention_prefill_kernel<true, false, true>)
+                            : (exact ? attention_prefill_kernel<true, true, false> : attention_prefill_kernel<true, false, false>);
         launch(kernel, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
-        launch_merge(stream, a, plan.nparts);
+        launch_merge(stream, a, parts.n);
     } else {
         const uint32_t total = ntiles * p.kv_heads;
         launch(exact ? attention_prefill_kernel<false, true, false> : attention_prefill_kernel<false, false, false>, dim3(total < plan.cus ? total : plan.cus), THREADS, LDS_BYTES, stream, a);
@@ -1789,7 +1799,7 @@ int launch_chunk(hipStream_t stream, int bits, const uint16_t *q, const void *kd
     if (small_parts || plan.small) {
         return launch_small(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, small_parts ? plan.small_part_blocks : 0, workspace, what);
     }
-    return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, have >= plan.tiles(), exact, plan, what);
+    return launch_flash(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, have, exact, plan, what);
 }
 
 int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kdata, const void *vdata,

@@ -458,6 +458,36 @@ def test_wide_tiles(kind, pos, tokens, kv):
     assert float((out.double() - want).norm() / want.norm()) < REL_RMS
 
 
+PART_O, PART_ML = 16 * 8 * D * 4, 16 * 8 * 8  # bytes of a tile's part (16 tokens, 8 heads): its sums; its maxima and their sums
+
+
+def parts_written(ws, plain, tokens, kv, parts):
+    """[part][tile of 16 tokens]: whether a call left sums there, in a workspace of 0xff with `parts` parts behind `plain` bytes."""
+    items = parts * -(-tokens // 16) * kv
+    sums = ws[plain + items * PART_O:plain + items * (PART_O + PART_ML)].view(torch.int32).view(parts, -1, kv * 16 * 8 * 2)
+    return (sums != -1).any(2)
+
+
+@pytest.mark.parametrize("kind,pos,tokens,kv,wide,narrow", [(saetta.KvBits.Half, 5499, 1379, 3, 3, 2), (saetta.KvBits.Four, 36049, 1236, 1, 5, 3),
+                                                            (saetta.KvBits.Eight, 5272, 2210, 2, 3, 2)])
+def test_a_workspace_without_room_for_wide_tiles_parts(kind, pos, tokens, kv, wide, narrow):
+    # wide tiles leave more parts than tiles of 16 would: in a workspace that holds only the latter's, those are made, and only
+    # where it holds neither are the keys not split
+    call, out, p, want = chunk(kind, pos, tokens, kv)
+    plain = -(-(pos + tokens) // 32) * kv * 32768 + 256
+    bytes_of = lambda n: plain + n * -(-tokens // 16) * kv * (PART_O + PART_ML)  # noqa: E731
+    assert saetta.attention_prefill.workspace_bytes(p) == bytes_of(wide)
+    ws = torch.empty(bytes_of(wide), dtype=torch.uint8, device="cuda")
+    for size, parts in ((bytes_of(wide), wide), (bytes_of(wide) - 1, narrow), (bytes_of(narrow), narrow), (bytes_of(narrow) - 1, 0), (plain, 0)):
+        ws.fill_(0xff), out.fill_(float("nan"))
+        assert call(ws.data_ptr(), size) == 0, saetta.ffi.lib().saetta_last_error()
+        assert float((out.double() - want).norm() / want.norm()) < REL_RMS
+        assert float((out - want).abs().max()) < MAX_ABS
+        assert bool((ws[plain:] == 0xff).all()) == (parts == 0)
+        if parts:
+            assert bool((ws[bytes_of(parts):] == 0xff).all()) and bool(parts_written(ws, plain, tokens, kv, parts)[0].all())
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("scale", [1e-3, 300.0])
 def test_short_chunks_of_small_and_large_values(kind, scale):
