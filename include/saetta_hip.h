@@ -449,9 +449,10 @@ int saetta_deltanet_rows_fused_sync(saetta_stream_t stream, const float *x, cons
 
 /* Bytes of workspace a prefill chunk at (pos, tokens) wants: the f16 key and
  * value tile images of the pos + tokens rows the chunk can see and, for a chunk with too few
- * tokens to fill the GPU, room for partial results of parts of the keys (up to 64 parts of
- * 1 KB + 8 B per query row; where no images are made, instead of them).  A call given less, but room for the images (one
- * sized for another chunk of as many rows), runs too, and without the split if the parts do not fit.  Its bits are then
+ * tokens to fill the GPU evenly, or of any length behind a long prefix, room for partial results of parts of the keys (up to 64 parts of
+ * 1 KB + 8 B per query row; where no images are made, instead of them).  With 2 kv heads 4096 tokens at 4096 want 17 MB, at 20000
+ * 185, 2300 at 3000 163: it is not the longest chunk that wants most.  A call given less, but room for the images (one
+ * sized for another chunk of as many rows), runs too, with fewer parts or without if the parts do not fit: 1.05 to 5 times as long.  Its bits are then
  * others: the probabilities are rounded to f16 relative to a maximum, which with
  * the split is a part's own.  Both forms are as close to the exact result, but who
  * wants the same bits from one call to the next gives workspaces that hold what this function returns.  The reference
@@ -468,7 +469,8 @@ size_t saetta_prefill_workspace_bytes(uint32_t pos, uint32_t tokens, uint32_t kv
  * aligned, overwritten by the call; NULL makes the library use one of its own
  * per device and stream, which it grows with hipMalloc when needed (so not
  * under stream capture, and not when recorded) and keeps until the process ends; where it
- * cannot have one, a chunk that is short enough to do without runs without the split, any other is refused.  Kernel replaced:
+ * cannot have so much, it is of fewer parts, or of the images; where it cannot have these, a chunk that is short enough to do without
+ * runs without the split, any other is refused.  Kernel replaced:
  * attention_fa{4,8} (kernels/attention_prefill.metal:38-169). */
 int saetta_attn_prefill(saetta_stream_t stream, const uint16_t *q_f16, const uint16_t *keys,
                         const uint16_t *values, const float *q_and_gate, float *out,
@@ -497,7 +499,7 @@ int saetta_attn_prefill_quant(saetta_stream_t stream, int bits, const uint16_t *
  * and the per-row softmax state; about 19 KB per query row of a slice; or, where that is more, room
  * for partial results of parts of the keys (saetta_prefill_workspace_bytes).  A call given a workspace
  * sized for a longer chunk that ends at the same key or a later one, in slices of as many tokens, always
- * runs; where parts of the keys do not fit, without the split (and so with other bits, see
+ * runs; where parts of the keys do not fit, with fewer or without (and so with other bits, see
  * saetta_prefill_workspace_bytes).  A whole call (stages 0) writes no probabilities
  * and runs in no slices: what slice_tokens 1 gives does for it, whatever slice_tokens it is called with
  * (26 MB for 4096 tokens at 4096 and 2 kv heads, where one slice of the passes wants 1.2 GB). */

@@ -41,7 +41,10 @@
 // there are two per CU, which evens out the causal imbalance.
 #include "common.hpp"
 #include "lanes.hpp"
+#include "owned_workspace.hpp"
 
+#include <algorithm>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -1469,10 +1472,6 @@ __global__ __launch_bounds__(SMALL_THREADS, 2) void prefill_small_kernel(SmallAr
 // Workspaces the library owns when the caller passes none: one per (device, stream), grown on demand,
 // so that calls on different streams never share one (work on one stream runs in order).  They are
 // kept until the process ends: a caller with many short-lived streams passes its own.
-struct OwnedWorkspace {
-    void *ptr = nullptr;
-    size_t bytes = 0;
-};
 constexpr int OWNED_DEVICES = 64;  // as many devices as the library's set-up admits
 std::map<std::pair<int, hipStream_t>, OwnedWorkspace> g_owned;
 std::mutex g_owned_mutex;
@@ -1663,40 +1662,42 @@ int check_prefill(int bits, const uint16_t *q, const void *kdata, const void *vd
 }
 
 // The caller's workspace if it gave one of at least `need` bytes, else the library's own for this device
-// and stream, grown to `need`.  The library's own is held under the lock until the launches that use it
+// and stream, grown to the first of `wants` bytes (in falling order) that can be had; `have`: the bytes of either.  The
+// library's own is held under the lock until the launches that use it
 // are queued (the caller keeps `owned_lock` until then): a second host thread on the same stream that has
 // to grow it waits for them (hipStreamSynchronize) before it frees.
-int acquire_workspace(hipStream_t stream, void *&workspace, size_t workspace_size, size_t need,
+int acquire_workspace(hipStream_t stream, void *&workspace, size_t &have, size_t need, std::initializer_list<size_t> wants,
                       std::unique_lock<std::mutex> &owned_lock, const char *what, const char *sizer) {
     if (workspace) {
-        SAETTA_REQUIRE(workspace_size >= need, SAETTA_E_SCRATCH, "%s: workspace of %zu bytes, %zu needed", what,
-                       workspace_size, need);
+        SAETTA_REQUIRE(have >= need, SAETTA_E_SCRATCH, "%s: workspace of %zu bytes, %zu needed", what, have, need);
         return SAETTA_OK;
     }
+    const size_t want = *wants.begin();
     // No workspace given: use (and grow) the library's own for this stream.  This may allocate, which a
     // stream under capture cannot do; and a plan outlives the buffer, which a later call may grow.
-    SAETTA_REQUIRE(!recording(), SAETTA_E_SCRATCH, "%s: a recorded call needs a workspace of the caller's (%zu bytes, %s)", what, need, sizer);
+    SAETTA_REQUIRE(!recording(), SAETTA_E_SCRATCH, "%s: a recorded call needs a workspace of the caller's (%zu bytes, %s)", what, want, sizer);
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) (void)hipGetLastError();
     SAETTA_REQUIRE(capturing == hipStreamCaptureStatusNone, SAETTA_E_SCRATCH,
-                   "%s: a stream under capture needs a workspace of the caller's (%zu bytes, %s)", what, need, sizer);
+                   "%s: a stream under capture needs a workspace of the caller's (%zu bytes, %s)", what, want, sizer);
     int dev = 0;
     if (hipError_t e = hipGetDevice(&dev)) return fail(int(e), "%s: %s", what, hipGetErrorString(e));
     SAETTA_REQUIRE(dev >= 0 && dev < OWNED_DEVICES, SAETTA_E_DEVICE, "%s: device index %d (up to %d)", what, dev, OWNED_DEVICES - 1);
     owned_lock.lock();
     OwnedWorkspace &w = g_owned[std::make_pair(dev, stream)];
-    if (w.bytes < need) {
-        if (w.ptr) {
-            (void)hipStreamSynchronize(stream);
-            (void)hipFree(w.ptr);
-        }
-        w.ptr = nullptr;
-        w.bytes = 0;
-        hipError_t e = hipMalloc(&w.ptr, need);
-        if (e != hipSuccess) return fail(int(e), "%s: workspace of %zu bytes: %s", what, need, hipGetErrorString(e));
-        w.bytes = need;
-    }
-    workspace = w.ptr;
+    hipError_t e = hipSuccess;
+    auto alloc = [&](size_t bytes) -> void * {
+        void *at = nullptr;
+        if ((e = hipMalloc(&at, bytes)) == hipSuccess) return at;
+        (void)hipGetLastError();  // (or the launches' status would be this)
+        return nullptr;
+    };
+    auto release = [&](void *at) {
+        (void)hipStreamSynchronize(stream);
+        (void)hipFree(at);
+    };
+    if (!w.take(wants, alloc, release)) return fail(int(e), "%s: workspace of %zu bytes: %s", what, *(wants.end() - 1), hipGetErrorString(e));
+    workspace = w.ptr, have = w.bytes;
     return SAETTA_OK;
 }
 
@@ -1813,14 +1814,15 @@ int run_prefill(hipStream_t stream, int bits, const uint16_t *q, const void *kda
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
     // (a workspace that is given has to do for the images, whatever the chunk: which launches serve it is no caller's business.
     // One of the library's is taken where the chunk has a use for one, so that it runs as in one of the caller's; where there
-    // is none to be had, a chunk that can do without does.)
-    size_t have = workspace ? workspace_size : plan.small ? plan.small_parts : plan.bytes();
-    if (workspace || have > 0) {
-        if (int rc = acquire_workspace(stream, workspace, workspace_size, workspace ? plan.plain : have, owned_lock, what, "saetta_prefill_workspace_bytes")) {
-            if (workspace || !plan.small) return rc;
-            (void)hipGetLastError();
-            have = 0;
-        }
+    // is none to be had, it is one of fewer parts, or of the images alone, and a chunk that can do without does.)
+    size_t have = workspace ? workspace_size : 0;
+    auto acquire = [&](std::initializer_list<size_t> wants) {
+        return acquire_workspace(stream, workspace, have, plan.plain, wants, owned_lock, what, "saetta_prefill_workspace_bytes");
+    };
+    if (workspace || !plan.small) {
+        if (int rc = acquire({plan.bytes(), plan.plain + plan.narrow.bytes, plan.plain})) return rc;
+    } else if (plan.small_parts > 0) {
+        (void)acquire({plan.small_parts});
     }
     return launch_chunk(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, have, false, plan, what);
 }
@@ -2193,16 +2195,16 @@ int run_gemm(hipStream_t stream, int bits, const uint16_t *q, const void *kdata,
     const uint32_t slice = gemm_slice(p.tokens, slice_tokens);
     // (a whole call runs in no slices: it asks for the passes' scratch of the smallest)
     const size_t need = passes_workspace_bytes(p.pos, p.tokens, stages == 0 ? 1 : slice, p.kv_heads);
+    size_t have = workspace ? workspace_size : 0;
     std::unique_lock<std::mutex> owned_lock(g_owned_mutex, std::defer_lock);
     // All of the call: the flash kernel's result is the same and it is there in 0.5 to 0.6 of the time (see above).  Where
     // the workspace has no room for parts of the keys they are not split.
     if (stages == 0) {
         const FlashPlan plan = flash_plan(p.pos, p.tokens, p.kv_heads, bits);
-        const size_t have = workspace ? workspace_size : plan.bytes() > need ? plan.bytes() : need;
-        if (int rc = acquire_workspace(stream, workspace, workspace_size, workspace ? need : have, owned_lock, what, "saetta_attn_gemm_workspace_bytes")) return rc;
+        if (int rc = acquire_workspace(stream, workspace, have, need, {std::max(plan.bytes(), need), std::max(plan.plain + plan.narrow.bytes, need), need}, owned_lock, what, "saetta_attn_gemm_workspace_bytes")) return rc;
         return launch_chunk(stream, bits, q, kdata, vdata, ks, kz, vs, vz, q_and_gate, out, p, workspace, have, true, plan, what);
     }
-    if (int rc = acquire_workspace(stream, workspace, workspace_size, need, owned_lock, what, "saetta_attn_gemm_workspace_bytes")) return rc;
+    if (int rc = acquire_workspace(stream, workspace, have, need, {need}, owned_lock, what, "saetta_attn_gemm_workspace_bytes")) return rc;
     const uint32_t nblocks = launch_prepare(stream, bits, kdata, vdata, ks, kz, vs, vz, workspace, p.kv_heads, rows);
 
     const size_t groups = gemm_row_groups(slice) * p.kv_heads;

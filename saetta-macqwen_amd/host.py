@@ -759,11 +759,16 @@ def _workspace(t):
 def _own_workspace(what, q, p, stream):
     """A workspace for the chunk of FlashParams p as a tensor of the call's own from torch's allocator (which hands a
     block out again only behind the work queued on its stream): the library's own workspace, which a
-    NULL pointer would select, is one per device and stream that stays for the life of the process."""
+    NULL pointer would select, is one per device and stream that stays for the life of the process.  Where there is no room
+    for the parts that the chunk wants: with the images of a chunk of one token that ends where this one does, which are the same."""
     if p.heads != p.kv_heads * 8:  # (what the call would say once it has its workspace)
         raise ValueError(f"{what} needs 8 q heads per kv head")
     _need(q, torch.float16, "q")
-    t = torch.empty(attention_prefill.workspace_bytes(p), dtype=torch.uint8, device=q.device)
+    try:
+        t = torch.empty(attention_prefill.workspace_bytes(p), dtype=torch.uint8, device=q.device)
+    except torch.OutOfMemoryError:
+        least = ffi.lib().saetta_prefill_workspace_bytes(max(p.pos + p.tokens, 1) - 1, 1, p.kv_heads)
+        t = torch.empty(least, dtype=torch.uint8, device=q.device)
     if isinstance(stream, torch.cuda.Stream):
         t.record_stream(stream)
     return t
@@ -903,6 +908,7 @@ class attention_gemm:
             self.fused = self.texp = True
             self.stages = 0
             self._workspace = None
+            self._refused = math.inf  # bytes: the least that could not be had
             self._captured, self._held = False, []
 
         def workspace_bytes(self, p):
@@ -929,14 +935,32 @@ class attention_gemm:
                 bits, k, v = quant[0].bits.value, quant[0].c(), quant[1].c()
             need = self.workspace_bytes(f)
             if self._workspace is None or self._workspace.numel() < need:
-                if self._captured:
-                    self._held.append(self._workspace)  # a graph that holds a call goes on using what it was captured with
-                self._captured = False
-                self._workspace = torch.empty(need, dtype=torch.uint8, device=self.device)
+                self._grow(need, f)
             self._captured = self._captured or torch.cuda.is_current_stream_capturing()
             ffi.check(ffi.lib().saetta_attn_gemm(_stream(stream), bits, _ptr(q), k, v, _ptr(q_and_gate), _ptr(out),
                                                  f.c(), self.slice, self.stages, *_workspace(self._workspace)),
                       "attn_gemm")
+
+        def _grow(self, need, f):
+            """A workspace of `need` bytes; where there is no room for it, of what a chunk of one token that ends where f does
+            wants, which does for f without the parts of its keys.  What was refused is asked for again only where that does not
+            do: each try has torch give back what it holds."""
+            least = ffi.lib().saetta_attn_gemm_workspace_bytes(max(f.pos + f.tokens, 1) - 1, 1, self.slice if self.stages else 1, f.kv_heads)
+            had = 0 if self._workspace is None else self._workspace.numel()
+            t = None
+            if need < self._refused or had < least:
+                try:
+                    t = torch.empty(need, dtype=torch.uint8, device=self.device)
+                    self._refused = self._refused if need < self._refused else math.inf
+                except torch.OutOfMemoryError:
+                    self._refused = min(need, self._refused)
+                    t = torch.empty(least, dtype=torch.uint8, device=self.device) if had < least else None
+            if t is None:
+                return
+            if self._captured:
+                self._held.append(self._workspace)  # a graph that holds a call goes on using what it was captured with
+            self._captured = False
+            self._workspace = t
 
         def passes_output(self, q_and_gate, f):
             """The outputs as the passes compute them: what the last call of encode, with `stages` 3 and its tokens in one

@@ -755,11 +755,7 @@ struct AttGemm {
         }
         // (a whole call runs in no slices)
         const size_t need = saetta_attn_gemm_workspace_bytes(f.pos, f.tokens, stages ? uint32_t(slice) : 1u, f.kv_heads);
-        if (workspace_.length() < need) {
-            if (captured_) held_.push_back(workspace_);  // a graph that holds a call goes on using what it was captured with
-            captured_ = false;
-            workspace_ = gpu::Buffer(need);
-        }
+        if (workspace_.length() < need) grow(need, f);
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         hip_check(hipStreamIsCapturing(gpu.stream(), &capturing), "hipStreamIsCapturing");
         captured_ = captured_ || capturing != hipStreamCaptureStatusNone;
@@ -769,7 +765,30 @@ struct AttGemm {
     }
 
   private:
+    // A workspace of `need` bytes; where there is no room for it, of what a chunk of one token that ends where f does wants, which
+    // does for f without the parts of its keys.
+    void grow(size_t need, const attention_prefill::FlashParams &f) const {
+        const uint32_t end = f.pos + f.tokens;
+        const size_t least = saetta_attn_gemm_workspace_bytes(end ? end - 1 : 0, 1, stages ? uint32_t(slice) : 1u, f.kv_heads);
+        gpu::Buffer grown;
+        if (need < refused_ || workspace_.length() < least) {
+            try {
+                grown = gpu::Buffer(need);
+                if (need >= refused_) refused_ = SIZE_MAX;
+            } catch (const std::runtime_error &) {
+                (void)hipGetLastError();
+                if (need < refused_) refused_ = need;
+                if (workspace_.length() < least) grown = gpu::Buffer(least);
+            }
+        }
+        if (!grown.length()) return;
+        if (captured_) held_.push_back(workspace_);  // a graph that holds a call goes on using what it was captured with
+        captured_ = false;
+        workspace_ = grown;
+    }
+
     mutable gpu::Buffer workspace_;
+    mutable size_t refused_ = SIZE_MAX;  // bytes: the least that could not be had
     mutable std::vector<gpu::Buffer> held_;
     mutable bool captured_ = false;
 };

@@ -7,7 +7,17 @@
 #include <cstdio>
 #include <cstdlib>
 
+#include <hip/hip_runtime.h>
+
+// Device memory for the host mirror, of malloc_limit bytes at most.
+static size_t malloc_limit = SIZE_MAX;
+template <class T>
+static hipError_t limited_malloc(T **p, size_t bytes) {
+    return bytes > malloc_limit ? hipErrorOutOfMemory : hipMalloc(p, bytes);
+}
+#define hipMalloc limited_malloc
 #include "../../saetta-macqwen_amd/host/saetta.hpp"
+#undef hipMalloc
 
 extern "C" {  // oracle/saetta_oracle.c (the checker)
 int orc_quantize(const float *x, size_t n, int bits, uint32_t *data, uint16_t *scales, uint16_t *biases);
@@ -390,6 +400,23 @@ int main() {
         }
         std::printf("prefill (1000, 64): flash worst %.2e, gemm worst %.2e\n", worst_a, worst_b);
         EXPECT(worst_a < 2e-3f && worst_b < 2e-3f, "prefill chunk: flash %g gemm %g", worst_a, worst_b);
+    }
+    {   // AttGemm without room for parts of the keys does with less, and gives the same to the rounding of its probabilities
+        const size_t pos = 2000, tokens = 128, n = pos + tokens;
+        View q(gpu.buffer_from(attention_prefill::spread(tokens * HEADS * DIM, 1))), k(gpu.buffer_from(attention_prefill::spread(n * VALUES, 2)));
+        View v(gpu.buffer_from(attention_prefill::spread(n * VALUES, 3))), g(gpu.buffer_from(std::vector<float>(tokens * HEADS * 2 * DIM, 1.0f)));
+        View roomy(gpu.buffer(tokens * HEADS * DIM * 4)), tight(gpu.buffer(tokens * HEADS * DIM * 4));
+        const attention_prefill::FlashParams f{uint32_t(HEADS), uint32_t(KV), uint32_t(pos), uint32_t(tokens), 1.0f / 16.0f};
+        const attention_gemm::AttGemm one(gpu, tokens, KV), two(gpu, tokens, KV);
+        one.encode(gpu, q, k, v, nullptr, g, roomy, f);
+        malloc_limit = saetta_attn_gemm_workspace_bytes(f.pos, f.tokens, 1, f.kv_heads) - 1;
+        for (int i = 0; i < 2; i++) two.encode(gpu, q, k, v, nullptr, g, tight, f);
+        malloc_limit = SIZE_MAX;
+        gpu.sync();
+        const auto a = gpu::contents<float>(roomy.buffer, tokens * HEADS * DIM), b = gpu::contents<float>(tight.buffer, a.size());
+        float worst = 0.0f;
+        for (size_t i = 0; i < a.size(); i++) worst = std::max(worst, std::fabs(a[i] - b[i]));
+        EXPECT(worst < 4e-3f, "AttGemm in less memory: %g", worst);
     }
     // shape checks panic (throw) as the reference asserts
     bool threw = false;

@@ -269,3 +269,42 @@ def test_plan_records_and_filters_ops_without_a_device():
     built = plan.build_where(lambda name: name == "attention_reduce")
     assert [k for k, _ in built.ops] == ["attention_reduce"]
     assert [k for k, _ in plan.build().ops] == ["attention_partial_mma_q8", "attention_reduce"]
+
+
+def test_the_librarys_own_workspace_takes_less_where_there_is_less(tmp_path):
+    # (its memory comes from a function of the caller's: here one that has a limit and counts)
+    src, exe = tmp_path / "take.cc", tmp_path / "take"
+    src.write_text("""
+#include "owned_workspace.hpp"
+#include <cstdio>
+static size_t limit = SIZE_MAX, held = 0;
+static int asked = 0, given_back = 0;
+static char memory[1];
+int main() {
+    saetta::OwnedWorkspace w;
+    auto take = [&](std::initializer_list<size_t> wants) {
+        asked = given_back = 0;
+        const bool ok = w.take(wants, [](size_t n) -> void * { asked++; return held || n > limit ? nullptr : (held = n, memory); },
+                               [](void *) { given_back++; held = 0; });
+        printf("%d %zu %d %d\\n", ok, w.bytes, asked, given_back);
+        if (ok != (w.ptr != nullptr) || held != w.bytes) puts("wrong");
+    };
+    take({100, 50, 40});   // the first
+    take({90, 50, 40});    // is there
+    limit = 120;
+    take({200, 120, 110}); // refused: the second
+    take({200, 120, 110}); // not asked for again
+    take({300, 200, 110}); // nor is more
+    limit = 130;
+    take({200, 130});      // the last is more than is held
+    take({150, 140});      // not even the last: nothing is held
+    take({150, 60});       // 60 of it
+    limit = 1000;
+    take({150, 145});      // what was refused may be there by now, where nothing else does
+    take({500, 400});      // and then anything is asked for
+    take({500, 0});
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "saetta-macqwen_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    said = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split("\n")[:-1]
+    assert said == ["1 100 1 0", "1 100 0 0", "1 120 2 1", "1 120 0 0", "1 120 0 0", "1 130 1 1", "0 0 2 1", "1 60 1 0", "1 145 1 1", "1 500 1 1", "1 500 0 0"]

@@ -488,6 +488,39 @@ def test_a_workspace_without_room_for_wide_tiles_parts(kind, pos, tokens, kv, wi
             assert bool((ws[bytes_of(parts):] == 0xff).all()) and bool(parts_written(ws, plain, tokens, kv, parts)[0].all())
 
 
+@pytest.mark.parametrize("kind,pos,tokens,kv", [(saetta.KvBits.Half, 2097, 2148, 2), (saetta.KvBits.Four, 5499, 1379, 3)])
+def test_calls_without_room_for_their_parts(kind, pos, tokens, kv, monkeypatch):
+    # 151 and 125 MB of workspace are wanted and 9 and 21 needed: a call that makes its own, and AttGemm, do with what there is
+    _, out, p, want = chunk(kind, pos, tokens, kv)
+    gen, heads, n = torch.Generator(device="cuda").manual_seed(pos + tokens), 8 * kv, pos + tokens  # (chunk's own inputs again)
+    k, v = (torch.randn(n, kv * D, generator=gen, device="cuda") for _ in range(2))
+    q16, qg = torch.randn(tokens, heads, D, generator=gen, device="cuda").half(), torch.randn(tokens, heads, 2 * D, generator=gen, device="cuda")
+    if kind is saetta.KvBits.Half:
+        keys, values = k.half(), v.half()
+        flash = lambda: saetta.attention_prefill.encode(saetta.attention_prefill.DEFAULT, q16, keys, values, qg, out, p)  # noqa: E731
+    else:
+        keys, values = (saetta.QuantRows(kind, kv * D, n) for _ in range(2))
+        keys.encode(k.view(-1), 0, n), values.encode(v.view(-1), 0, n)
+        flash = lambda: saetta.attention_prefill.encode_quant(q16, keys, values, qg, out, p)  # noqa: E731
+    gemm = saetta.attention_gemm.AttGemm(tokens, kv)
+    quant = None if kind is saetta.KvBits.Half else (keys, values)
+    empty, refused = torch.empty, []
+
+    def limited(size, **options):
+        if options.get("dtype") is torch.uint8 and size > 80e6:
+            refused.append(size)
+            raise torch.OutOfMemoryError
+        return empty(size, **options)
+
+    monkeypatch.setattr(torch, "empty", limited)
+    encode = lambda: gemm.encode(q16, keys, values, quant, qg, out, p)  # noqa: E731
+    for call in (flash, encode, encode):
+        out.fill_(float("nan"))
+        call()
+        assert float((out.double() - want).norm() / want.norm()) < REL_RMS
+    assert refused == [saetta.attention_prefill.workspace_bytes(p), gemm.workspace_bytes(p)]
+
+
 @pytest.mark.parametrize("kind", KINDS)
 @pytest.mark.parametrize("scale", [1e-3, 300.0])
 def test_short_chunks_of_small_and_large_values(kind, scale):
