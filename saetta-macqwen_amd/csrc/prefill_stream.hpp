@@ -196,7 +196,7 @@ __device__ __forceinline__ void stream_block(floatx16 &s, floatx16 (&o)[8], cons
     [q10] "v"(q[10]), [q11] "v"(q[11]), [q12] "v"(q[12]), [q13] "v"(q[13]), [q14] "v"(q[14]), [q15] "v"(q[15]), \
     [p0] "v"(p[0]), [p1] "v"(p[1]), [off] "v"(lane16), [src] "s"(c.src), [src2] "s"(c.src + 4096), \
     [dst] "s"(c.dst) \
-    : "memory", "m0"
+    : "memory", "m0", "scc"
     if constexpr (HALF) {
         asm volatile(SAETTA_STREAM(SAETTA_COPY(src, 0), "", SAETTA_COPY(src, 1024), "", "", SAETTA_COPY(src, 2048), "", SAETTA_COPY(src, 3072), "")
                      SAETTA_OPERANDS);

@@ -308,3 +308,18 @@ int main() {
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "saetta-macqwen_amd", "csrc"), str(src), "-o", str(exe)], check=True)
     said = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split("\n")[:-1]
     assert said == ["1 100 1 0", "1 100 0 0", "1 120 2 1", "1 120 0 0", "1 120 0 0", "1 130 1 1", "0 0 2 1", "1 60 1 0", "1 145 1 1", "1 500 1 1", "1 500 0 0"]
+
+
+def test_asm_that_changes_scc_says_so(tmp_path):
+    # Most scalar arithmetic writes SCC, where the compiler may keep a comparison across a statement that does not name it.
+    writes = re.compile(r"\bs_(add|sub|min|max|and|or|xor|not|andn2|orn2|nand|nor|xnor|lshl|lshr|ashr|bfe|bcnt|abs|cmp|bitcmp|wqm|quadmask|ff0|flbit|addk|cmpk)[a-z0-9]*_")
+    folder, seen = os.path.join(ROOT, "saetta-macqwen_amd", "csrc"), 0
+    for name in sorted(n for n in os.listdir(folder) if n.endswith((".hip", ".hpp"))):
+        with open(os.path.join(folder, name)) as f:
+            text = re.sub(r"(?m)^\s*#\s*(include|pragma).*$", "", f.read())  # (asm text is made of a file's own macros)
+        text = subprocess.run(["g++", "-E", "-P", "-x", "c++", "-"], input=text, capture_output=True, text=True, check=True).stdout
+        for at in re.finditer(r"\basm\b\s*(volatile\b\s*)?\(", text):
+            statement = text[at.end():text.index(");", at.end())]
+            seen += 1
+            assert not writes.search(statement) or '"scc"' in statement, f"{name}: {statement}"
+    assert seen > 50
