@@ -1561,15 +1561,28 @@ FlashPlan tiles_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, float &ti
     const float unsplit = rounds_us(f.cus, ntiles * kv_heads, float(longest), float(shortest), TILE_US, BLOCK_US, chip_us);
     float best = 0.95f * unsplit;
     auto in_parts = [&](bool wide, TileParts &of) {
-        const uint32_t tq = wide ? WIDE_TQ : TQ, n = (tokens + tq - 1) / tq;
+        const uint32_t tq = wide ? WIDE_TQ : TQ, n = (tokens + tq - 1) / tq, seen_by_all = pos + (tokens < tq ? tokens : tq) - 1;
         const float high = float(tile_blocks(pos, tokens, n - 1, tq)), low = float(tile_blocks(pos, tokens, 0, tq));
+        const float blocks = 0.5f * (high + low) * float(n * kv_heads), chip = wide ? WIDE_GAIN * 2.0f * chip_us : chip_us;
+        const float ends_us = wide ? WIDE_PART_US : PART_US, block_us = wide ? WIDE_BLOCK_US : BLOCK_US, item_us = (wide ? 2.0f : 1.0f) * MERGE_ITEM_US;
+        // What `rounds` rounds of `items` items take is no less than this, and more with every further part: where it is no gain, nothing
+        // further is.  (The rounds one by one are most of what the plan costs the host.)
+        auto no_gain = [&](uint32_t rounds, uint32_t items) {
+            return 0.999f * (blocks * chip + float(rounds) * ends_us + MERGE_US + item_us * float(items)) >= best;
+        };
+        if (no_gain(1, n * kv_heads)) return;
+        uint32_t last = 0;
         for (uint32_t parts = 2; parts <= 32; parts++) {
             const uint32_t pb = ((longest + parts - 1) / parts + 1) / 2 * 2;  // (a step of the kernel is two blocks)
-            if (pb < 4 || pb >= longest) continue;
+            if (pb < 4 || pb >= longest || pb == last) continue;
+            last = pb;
+            if (n * kv_heads * parts > f.cus) {  // (not a round, and short)
+                const uint32_t least = (seen_by_all / (pb * BK) + 1) * n * kv_heads;
+                if (no_gain((least + f.cus - 1) / f.cus, least)) break;
+            }
             const uint32_t items = prefill_items(pos, tokens, pb, tq) * kv_heads;
-            const float mid = 0.5f * (high + low) * float(n * kv_heads) / float(items);
-            const float us = (wide ? rounds_us(f.cus, items, mid, mid, WIDE_PART_US, WIDE_BLOCK_US, WIDE_GAIN * 2.0f * chip_us) : rounds_us(f.cus, items, mid, mid, PART_US, BLOCK_US, chip_us)) +
-                             MERGE_US + (wide ? 2.0f : 1.0f) * MERGE_ITEM_US * float(items);
+            const float mid = blocks / float(items);
+            const float us = rounds_us(f.cus, items, mid, mid, ends_us, block_us, chip) + MERGE_US + item_us * float(items);
             if (us < best) best = us, of.blocks = pb;
         }
         if (!of.blocks) return;
@@ -1582,7 +1595,7 @@ FlashPlan tiles_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, float &ti
     // decided there)
     const float narrow = best;
     best *= 0.985f;
-    in_parts(true, f.wide);
+    if (tokens > TQ) in_parts(true, f.wide);  // (of one tile a wide one takes twice a block's time for nothing)
     // (never less than 5 us, what short contexts' images were counted at when the row groups came in: a chunk that goes to them
     // without parts needs no workspace, and who calls it without one, recording or under capture, goes on to)
     const float prepare_us = PREPARE_US + PREPARE_KEY_US * float(pos + tokens) * float(kv_heads);

@@ -6,6 +6,7 @@ import ctypes
 import os
 import re
 import subprocess
+import timeit
 
 import pytest
 
@@ -269,6 +270,21 @@ def test_plan_records_and_filters_ops_without_a_device():
     built = plan.build_where(lambda name: name == "attention_reduce")
     assert [k for k, _ in built.ops] == ["attention_reduce"]
     assert [k for k, _ in plan.build().ops] == ["attention_partial_mma_q8", "attention_reduce"]
+
+
+@pytest.mark.parametrize("pos,tokens,kv,parts", [(4096, 4096, 2, 0), (2048, 2048, 2, 0), (300, 16, 1, 3), (20000, 4096, 2, 2), (118784, 2048, 2, 2),
+                                                 (60007, 1237, 2, 3), (3000, 2300, 2, 4), (86225, 447, 2, 7), (10000, 100, 2, 12), (20000, 12, 2, 32)])
+def test_parts_of_a_chunks_keys(pos, tokens, kv, parts):
+    # what the layouts' estimates come to on 256 CUs: whole keys, wide tiles in 2 to 7 parts, tiles of 16 in 3 to 32
+    images = -(-(pos + tokens) // 32) * kv * 32768 + 256
+    assert ffi.lib().saetta_prefill_workspace_bytes(pos, tokens, kv) - images == parts * -(-tokens // 16) * kv * 16 * 8 * (1024 + 8)
+
+
+def test_the_plan_of_a_long_chunk_costs_the_host_no_more_than_a_short_ones():
+    # every call makes one: few layouts of many rounds are worked out to their end
+    size = ffi.lib().saetta_prefill_workspace_bytes
+    of = lambda *chunk: min(timeit.repeat(lambda: size(*chunk), number=500, repeat=20))  # noqa: E731
+    assert of(20000, 4096, 2) < 2 * of(20000, 12, 2)
 
 
 def test_the_librarys_own_workspace_takes_less_where_there_is_less(tmp_path):
