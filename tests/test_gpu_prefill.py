@@ -438,26 +438,6 @@ def test_short_chunks_whose_waves_share_their_blocks(kind, pos, tokens, kv):
     assert float((out - want).abs().max()) < MAX_ABS
 
 
-@pytest.mark.parametrize("kind,pos,tokens,kv", [(saetta.KvBits.Half, 1000, 2100, 2), (saetta.KvBits.Eight, 1003, 2113, 2), (saetta.KvBits.Four, 9990, 2309, 2),
-                                                (saetta.KvBits.Half, 2991, 4177, 1), (saetta.KvBits.Half, 3000, 1441, 3)])
-def test_wide_tiles(kind, pos, tokens, kv):
-    # tiles of 32 tokens, their keys in parts: whole tiles; a last one with 1, 5, 17 tokens (its second half of no place, or of one token);
-    # parts that begin between a tile's tokens; 1 and 3 kv heads
-    call, out, p, want = chunk(kind, pos, tokens, kv)
-    size = saetta.attention_prefill.workspace_bytes(p)
-    ws = torch.full((size,), 0xff, dtype=torch.uint8, device="cuda")
-    out.fill_(float("nan"))
-    assert call(ws.data_ptr(), size) == 0, saetta.ffi.lib().saetta_last_error()
-    got = out.clone()
-    assert float((got.double() - want).norm() / want.norm()) < REL_RMS
-    assert float((got - want).abs().max()) < MAX_ABS
-    # without room for the parts: tiles of 16, the same to the rounding of the probabilities
-    out.fill_(float("nan"))
-    plain = -(-(pos + tokens) // 32) * kv * 32768 + 256
-    assert call(ws.data_ptr(), plain) == 0, saetta.ffi.lib().saetta_last_error()
-    assert float((out.double() - want).norm() / want.norm()) < REL_RMS
-
-
 PART_O, PART_ML = 16 * 8 * D * 4, 16 * 8 * 8  # bytes of a tile's part (16 tokens, 8 heads): its sums; its maxima and their sums
 
 
@@ -466,6 +446,32 @@ def parts_written(ws, plain, tokens, kv, parts):
     items = parts * -(-tokens // 16) * kv
     sums = ws[plain + items * PART_O:plain + items * (PART_O + PART_ML)].view(torch.int32).view(parts, -1, kv * 16 * 8 * 2)
     return (sums != -1).any(2)
+
+
+@pytest.mark.parametrize("kind,pos,tokens,kv,blocks", [(saetta.KvBits.Half, 1000, 2100, 2, 50), (saetta.KvBits.Eight, 1003, 2113, 2, 50), (saetta.KvBits.Four, 9990, 2309, 2, 130),
+                                                       (saetta.KvBits.Half, 2991, 4177, 1, 112), (saetta.KvBits.Half, 3000, 1441, 3, 36), (saetta.KvBits.Eight, 1000, 2112, 2, 50),
+                                                       (saetta.KvBits.Four, 1005, 2080, 2, 50)])
+def test_wide_tiles(kind, pos, tokens, kv, blocks):
+    # tiles of 32 tokens, their keys in parts of `blocks` blocks: a last one with 20, 1, 5, 17, 1 tokens (its second half of no place, or of one
+    # token), and whole; parts that begin between a tile's tokens; 1 and 3 kv heads
+    call, out, p, want = chunk(kind, pos, tokens, kv)
+    size, plain = saetta.attention_prefill.workspace_bytes(p), -(-(pos + tokens) // 32) * kv * 32768 + 256
+    ws = torch.full((size,), 0xff, dtype=torch.uint8, device="cuda")
+    out.fill_(float("nan"))
+    assert call(ws.data_ptr(), size) == 0, saetta.ffi.lib().saetta_last_error()
+    # a tile leaves the parts that its last token sees: the second half of a wide one is in the same as the first
+    begins, tile = torch.arange(0, pos + tokens, 32 * blocks), torch.arange(-(-tokens // 16))
+    left = lambda tq: pos + torch.clamp((16 * tile // tq + 1) * tq, max=tokens)[None] > begins[:, None]  # noqa: E731
+    assert size == plain + len(begins) * len(tile) * kv * (PART_O + PART_ML)
+    assert torch.equal(parts_written(ws, plain, tokens, kv, len(begins)).cpu(), left(32))
+    assert torch.equal(left(32), left(16)) == (pos in (9990, 3000))  # (elsewhere tiles of 16 would leave fewer)
+    got = out.clone()
+    assert float((got.double() - want).norm() / want.norm()) < REL_RMS
+    assert float((got - want).abs().max()) < MAX_ABS
+    # without room for the parts: tiles of 16, the same to the rounding of the probabilities
+    out.fill_(float("nan"))
+    assert call(ws.data_ptr(), plain) == 0, saetta.ffi.lib().saetta_last_error()
+    assert float((out.double() - want).norm() / want.norm()) < REL_RMS
 
 
 @pytest.mark.parametrize("kind,pos,tokens,kv,wide,narrow", [(saetta.KvBits.Half, 5499, 1379, 3, 3, 2), (saetta.KvBits.Four, 36049, 1236, 1, 5, 3),
