@@ -111,14 +111,15 @@ __device__ __forceinline__ floatx4 mma3(half8 ah, half8 al, half8 bh, half8 bl, 
 // belong to the key head, the gates, A, M and T to a value head.  (G = 2: the model's two value heads per key head;
 // G = 1: any other ratio, one workgroup per value head, the first of a key head's writing the key head's images.)
 // What bounds it: a workgroup is a chain of short phases, and with few blocks (up to 1024 tokens: a workgroup to a CU)
-// that chain is the kernel's time, with many the memory (67 MB read and 118 written at 4096 tokens: 3.7 TB/s).  So the phases are
+// that chain is the kernel's time, with many the memory (69 MB read and 118 written at 4096 tokens in 40 us: 4.7 TB/s).  So the phases are
 // spread over two teams of four waves, a row tile of 16 tokens to a wave: one makes A and solves for T, the other makes M
 // and stores it meanwhile; the products are taken as their transposes, so that a lane's four results lie in a row and
 // leave as one 8-byte store; the solve has a lane to a column, with no sums over lanes.
 // Measured, us, against four waves that did it all in order: 1000 tokens 22.7 -> 15.8, 2047 28.3 -> 26.4, 4096 57.4 -> 49.8;
-// with the conv inside, 512 tokens 31.5 -> 20.3.  Of the 34 000 cycles of a block with its conv most were waits for something that
+// with the conv inside, 512 tokens 31.5 -> 20.3; then 4096 49.8 -> 40: of the 34 000 cycles of a block with its conv most were waits for something that
 // need not be waited for, or one wave's work: without them 25 000, and 20 400 of 25 900 without the conv (whole chunk: 130
-// tokens 28.9 -> 25.3, 500 38.7 -> 35.6, 1000 60.2 -> 57.9, 2300 127.2 -> 121.4, 4096 230.3 -> 223.3).
+// tokens 28.9 -> 25.3, 500 38.7 -> 35.6, 1000 60.2 -> 57.9, 2300 127.2 -> 121.4, 4096 230.3 -> 223.3, with the chain's outputs
+// in whole lines and the conv's and norm's short activation 219).
 // LDS: the four q / k images; once the products are taken, the heads' A (f32) go over kh | kl, their M
 // images and later their T images over qh | ql (and more), so that they leave as whole 16-byte stores.
 constexpr int PREP_THREADS = 512, PREP_WAVES = PREP_THREADS / 64;
@@ -581,7 +582,8 @@ __device__ __forceinline__ half4 read_transposed(const unsigned char *at) {
 // stood at theirs.  So each team works where the other leaves LDS and the memory pipe alone: the outputs' M U and
 // stores under the next block's K S0^T, their Q S0^T under U, their loads under the state's update; the state's
 // loads two at a time between its dependent products.  (The output waves' loads under U: 246 us instead of 230.)
-// Measured, whole chunk, us: 1000 tokens 65.4 -> 61.2, 2300 140.3 -> 128.7, 4096 253.3 -> 230.4; results bit for bit the same.
+// Measured, whole chunk, us: 1000 tokens 65.4 -> 61.2, 2300 140.3 -> 128.7, 4096 253.3 -> 230.4 (this kernel 132 -> 109,
+// with the outputs in whole lines); results bit for bit the same.
 struct ChainLds {
     static constexpr int GAM = 0;                          // e^{c_t}, e^{c_last - c_t}: 128 f32
     static constexpr int V = GAM + 2 * C * 4;              // [token][DV] f32

@@ -11,7 +11,7 @@
 // cache is seen "through half": every value is f16(f32(s)*code + f32(z)),
 // exactly what round_trip_as_half (src/kv_quant.rs:119-125) gives the CPU path.
 //
-// Two kernels, and a third where a tile's keys are taken in parts (further down: the passes of the reference's other
+// Two kernels, and a third where a tile's keys are taken in parts; prefill_small_kernel instead of them for short chunks (further down: the passes of the reference's other
 // route to the same output, AttGemm of src/attention_gemm.rs, on the same images, block by block of 1024 keys).
 //
 // prefill_prepare_kernel<16|8|4> turns the keys and values the chunk can see into
@@ -22,23 +22,19 @@
 // exactly the arithmetic of round_trip_as_half, instead of once per workgroup that walks
 // the key; it costs one pass over the cache (a few microseconds).
 //
-// attention_prefill_kernel: workgroup (token tile of 16, kv head), 4 waves (one per SIMD);
-// wave w owns 4 tokens x 8 heads = 32 query rows, one 32-row MFMA tile.  Keys are walked in
-// blocks of 32 whose images are copied global -> LDS by global_load_lds_dwordx4 (no vector
-// registers, no vector ALU) into three rotating buffers, two blocks ahead.  Every wave
-// computes with v_mfma_f32_32x32x16_f16
+// attention_prefill_kernel: workgroup (token tile of 16 or 32, kv head), 8 waves, two to a SIMD; a row group is 4 tokens x 8 heads =
+// 32 query rows, one 32-row MFMA tile, and belongs to two waves that take alternate key blocks, or, in a tile of 32, to one.  Keys are
+// walked in blocks of 32 whose images are copied global -> LDS by global_load_lds_dwordx4 (no vector registers, no vector ALU) into a
+// ring of four places for K parts and four for V^T parts.  Every wave computes with v_mfma_f32_32x32x16_f16
 //     S^T = K Q^T      (A = K rows from LDS, B = Q^T held in registers)
 //     O^T += V^T P^T   (A = V^T rows from LDS, B = P^T from the S^T registers)
 // Both products are transposed so that a lane always owns one query row: in the 32x32
 // accumulator layout a lane holds column l % 32, so the row's running max and sum, the
 // rescale of O and the final 1/l and gate are plain per-lane values and the softmax needs one
-// cross-lane exchange per block.  The loop is software-pipelined inside each wave, because
-// MFMA and vector instructions of one wave run side by side when they are independent:
-//   stage A   MFMA: S^T of block kb+1      |  VALU: exp / sum / pack of block kb
-//   stage B   MFMA: O^T += V^T P^T (kb)    |  VALU: scale and row max of block kb+1
-// with one barrier per block.  The running max is only raised when a block exceeds it by
-// more than 2^8 (lazy rescale), so O is rarely rescaled.  Tiles are issued heaviest first and
-// there are two per CU, which evens out the causal imbalance.
+// cross-lane exchange per block.  A wave's step is its block's softmax (vector ALU) and one stream of MFMAs that adds the block to
+// O and makes the scores of its next; the two waves of a SIMD take them in opposite order, so that one's softmax runs
+// under the other's MFMAs, with one barrier per step.  The running max is only raised when a block exceeds it by
+// more than 2^8 (lazy rescale), so O is rarely rescaled.  Tiles are taken heaviest first, one workgroup per CU, on demand.
 #include "common.hpp"
 #include "lanes.hpp"
 #include "owned_workspace.hpp"
@@ -396,7 +392,14 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
     //   parity 1:  O(2s+1) + S(2s+3)         | softmax(2s+3)
     // During step s the workgroup copies what step s + 1 reads: K(2s+4), K(2s+5), V(2s+2),
     // V(2s+3); wave w takes half (w % 2) of part w / 2 of that list.  Before the loop: K(0..3),
-    // V(0), V(1), in front of them the queries.
+    // V(0), V(1), in front of them the queries.  K(2s+4) and K(2s+5) land on K(2s) and K(2s+1), which step s - 1 read, V(2s+2) and
+    // V(2s+3) on V(2s-2) and V(2s-1), the same: the barrier between the steps is all they wait for.
+    // WIDE: step s works on block s, in all eight waves:
+    //   parity 0:  softmax(s)                | O(s) + S(s+1)
+    //   parity 1:  O(s) + S(s+1)             | softmax(s+1)
+    // During step s, which reads V(s) and K(s+1), the workgroup copies V(s+1) and K(s+2), a quarter a wave, parity 0 the keys.  They
+    // land on V(s-3) and K(s-2), last read in step s - 3.  Before the loop: K(0), K(1) and V(0), behind the queries, which
+    // had all of the places.
     auto copy2k = [&](uint64_t src, uint32_t dst) {
         asm volatile(
             "s_mov_b32 m0, %[dst]\n"
@@ -545,7 +548,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs &a, unsigned char
         for (int r = 0; r < 16; r++) s[r] = 0.0f;
         if (0 < wave_blocks) scores_block(s, qb, lds0 + k_slot(0) + lane16);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();  // V(0) and V(1) are there; the first step's copies overwrite K(0) and K(1)
+        __syncthreads();  // V(0) and V(1) are there; the first step's copies overwrite K(0) and K(1) (WIDE: V(0); nothing)
         for (uint32_t step = 0; step < nsteps; step++) {
             const Copy cp = copy_of(step);
             const uint32_t kb = STRIDE * step;
@@ -957,9 +960,10 @@ struct SmallArgs {
 
 template <int BITS, bool SHARED>
 struct SmallLds {
-    // the values of a wave's block: f16 rows as in memory.  Codes: rows of 576 bytes, halves (copied in by 16-byte pieces in
-    // whole kilobytes): rows of 512 rotated by 64 bytes per row; either way the four rows of a transposing read, 32 bytes
-    // each, and those of its neighbours fall on different banks.
+    // the values of a wave's block: f16 rows as in memory.  Halves (copied in by 16-byte pieces in whole kilobytes), and codes where the
+    // values are SHARED (rows of 576 would leave the maxima no room): rows of 512 bytes, row k rotated by 64 (k % 4); codes of a wave's own
+    // blocks: rows of 576.  Either way the four rows of a transposing read, 32 bytes each, and those of its neighbours fall on different
+    // banks.
     static constexpr int VROW = BITS == 16 || SHARED ? 512 : 576;
     static constexpr int VTILE = BK * VROW;
     static constexpr int Q_OFF = 0, V_OFF = 16 * 1024;
@@ -1519,17 +1523,18 @@ struct FlashPlan {
 // a workgroup's block of 32 keys takes 0.6 us while the chip has power to spare (up to ~170 workgroups) and the chip as a
 // whole 284 blocks a us beyond that; the ends of an item (its first loads, the store of its part) 12 us, with the gate
 // 14.5; the merge a launch and 128 KB read back per item; the images 4.5 us and 0.3 ns a key and kv head.
-// (The ends have become 6 and 2.5 us shorter since, the merge 1; with these figures the rule still takes what is the fastest or
-// within 2 % of it at 33 of 38 sizes from 20 to 3500 tokens, 0 to 10000 keys before them, both kinds of cache; the furthest off are
-// 2300 tokens at 3000, 216 us instead of 201 in two parts, and 128 at 4000, 36 instead of 33.)
+// (The ends have become 6 and 2.5 us shorter since, the merge 1; with these figures and narrow tiles alone the rule takes what is the fastest
+// or within 2 % of it at 33 of 38 sizes from 20 to 3500 tokens, 0 to 10000 keys before them, both kinds of cache; the furthest off were
+// 2300 tokens at 3000, 216 us instead of 201 in two parts, which wide tiles now take in 205, and 128 at 4000, 36 instead of 33, which
+// row groups in parts now take.)
 // Wide tiles (WIDE_TQ tokens, a row group a wave; always in parts, so that there are as many items): a copied part of keys or values serves eight
 // row groups instead of four, half the global -> LDS copies, and the chip, which is bound by its power, does 5 % more blocks; a block
 // alone takes 1.3 us for twice the rows and an item's ends 18.  Whole call, us, without -> with: 2048 tokens at 118784 (AttGemm) 3568 -> 3397, 1237 at
 // 60007 (4-bit) 1142 -> 1082, 800 at 80000 1018 -> 978, 1024 at 30000 481 -> 465, 2300 at 3000 218 -> 205, 2100 at 1000 114 -> 106, 4096 at 20000 1307 ->
 // 1254.  Not where the parts' merge costs more than that: 4096 at 4096 would take 467 instead of 387, 2048 at 10000 (355) is even.
 // Measured, unsplit -> split by this rule, the whole call (8-bit cache): 100 tokens at 10000: 211 -> 47 us, at 100000
-// (4-bit): 1886 -> 225; 500 at 40000: 770 -> 330; 2100 at 9000: 497 -> 405.  A full chunk (4096 tokens: two whole rounds)
-// is never split.
+// (4-bit): 1886 -> 225; 500 at 40000: 770 -> 330; 2100 at 9000: 497 -> 405.  A full chunk (4096 tokens of 2 kv heads: two whole rounds) is
+// split from some 19300 keys before it on, into two parts of wide tiles.
 constexpr float MERGE_ITEM_US = 0.03f;
 // n items in order of length, from `high` down to `low` blocks, handed out one by one to `cus` workgroups: us, if a block
 // takes block_us alone and chip_us of the whole chip
