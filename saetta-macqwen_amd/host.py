@@ -942,10 +942,10 @@ class attention_gemm:
                       "attn_gemm")
 
         def _grow(self, need, f):
-            """A workspace of `need` bytes; where there is no room for it, of what a chunk of one token that ends where f does
-            wants, which does for f without the parts of its keys.  What was refused is asked for again only where that does not
-            do: each try has torch give back what it holds."""
-            least = ffi.lib().saetta_attn_gemm_workspace_bytes(max(f.pos + f.tokens, 1) - 1, 1, self.slice if self.stages else 1, f.kv_heads)
+            """A workspace of `need` bytes; where there is no room for it, a whole call's (stages 0) is of what a chunk of one token
+            that ends where f does wants, which does for f without the parts of its keys.  What was refused is asked for again
+            only where that does not do: each try has torch give back what it holds."""
+            least = need if self.stages else ffi.lib().saetta_attn_gemm_workspace_bytes(max(f.pos + f.tokens, 1) - 1, 1, 1, f.kv_heads)
             had = 0 if self._workspace is None else self._workspace.numel()
             t = None
             if need < self._refused or had < least:

@@ -765,11 +765,11 @@ struct AttGemm {
     }
 
   private:
-    // A workspace of `need` bytes; where there is no room for it, of what a chunk of one token that ends where f does wants, which
-    // does for f without the parts of its keys.
+    // A workspace of `need` bytes; where there is no room for it, a whole call's (stages 0) is of what a chunk of one token that ends
+    // where f does wants, which does for f without the parts of its keys.
     void grow(size_t need, const attention_prefill::FlashParams &f) const {
         const uint32_t end = f.pos + f.tokens;
-        const size_t least = saetta_attn_gemm_workspace_bytes(end ? end - 1 : 0, 1, stages ? uint32_t(slice) : 1u, f.kv_heads);
+        const size_t least = stages ? need : saetta_attn_gemm_workspace_bytes(end ? end - 1 : 0, 1, 1, f.kv_heads);
         gpu::Buffer grown;
         if (need < refused_ || workspace_.length() < least) {
             try {

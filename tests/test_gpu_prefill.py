@@ -525,6 +525,10 @@ def test_calls_without_room_for_their_parts(kind, pos, tokens, kv, monkeypatch):
         call()
         assert float((out.double() - want).norm() / want.norm()) < REL_RMS
     assert refused == [saetta.attention_prefill.workspace_bytes(p), gemm.workspace_bytes(p)]
+    gemm.stages = 3  # the passes cannot do with less
+    for _ in range(2):
+        with pytest.raises(torch.OutOfMemoryError):
+            encode()
 
 
 @pytest.mark.parametrize("kind", KINDS)
