@@ -452,7 +452,7 @@ int saetta_deltanet_rows_fused_sync(saetta_stream_t stream, const float *x, cons
  * tokens to fill the GPU evenly, or of any length behind a long prefix, room for partial results of parts of the keys (up to 64 parts of
  * 1 KB + 8 B per query row; where no images are made, instead of them).  With 2 kv heads 4096 tokens at 4096 want 17 MB, at 20000
  * 185, 2300 at 3000 163: it is not the longest chunk that wants most.  A call given less, but room for the images (one
- * sized for another chunk of as many rows), runs too, with fewer parts or without if the parts do not fit: 1.05 to 5 times as long.  Its bits are then
+ * sized for another chunk of as many rows), runs too, with fewer parts or without if the parts do not fit: 1.04 to 5 times as long.  Its bits are then
  * others: the probabilities are rounded to f16 relative to a maximum, which with
  * the split is a part's own.  Both forms are as close to the exact result, but who
  * wants the same bits from one call to the next gives workspaces that hold what this function returns.  The reference
