@@ -1327,6 +1327,8 @@ struct KeysFirst {
     static constexpr int C_QREAD = 7;   // computing waves that have a row's query operands in registers (several rows)
     static constexpr int C_KPART = 8;   // [3]: key loaders whose blocks 0-7 and scales | blocks 8-15 | block 16 have landed (2 per round)
     static constexpr int C_SLOT = 12;   // [5]: value loaders whose values of slot s have landed (2 per round)
+    // (alternating rounds: C_KPART, C_SLOT [2]: rounds of key | value loader L that have landed.  A counter for both loaders would not
+    // say which of two rounds on their way it was.)
     static constexpr int C_MERGE = 20;  // [4]: one row: wave 2g + 1 has written its sums for wave 2g | two pairs of rows: blocks
                                         // whose keys the two waves of scores w % 4 have in registers; then [4] as with one row
     static constexpr int C_NORM = 28;       // the step before the scores: computing waves that have written their sums of squares
@@ -1520,7 +1522,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
                 }
                 raise(W::C_KEYS);
                 __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-                raise(W::C_KPART + 0);
+                raise(W::C_KPART + int(L));
             }
             leave();
             return;
@@ -1612,7 +1614,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
                 }
                 raise(W::C_VREQ);
                 __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-                raise(W::C_SLOT + 4);
+                raise(W::C_SLOT + int(L));
             }
             leave();
             return;
@@ -2415,7 +2417,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
                         for (int i = 0; i < 8; i++) q_reg[i] = q_lds[i * 64 + lane];
                         qz_reg[0] = *reinterpret_cast<const half8 *>(qz_lds + lane * 8);
                         qz_reg[1] = *reinterpret_cast<const half8 *>(qz_lds + (64 + lane) * 8);
-                        await(W::C_KPART + 0, round + 1);  // the round's keys and scales are in LDS (one loader per round)
+                        await(W::C_KPART + int(round & 1), round / 2 + 1);  // the round's keys and scales are in LDS (its loader's counter)
                         const unsigned char *kb = lds_raw + W::K_OFF + blk * W::K_BLOCK_BYTES;
                         KeyRegs<BITS> kreg[4];
 #pragma unroll
@@ -2556,7 +2558,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
                 raise(W::C_BUILT);  // this wave is through with the round's keys, scores, scales and biases
 
                 // ---- phase C: O += P V of the wave's k-steps ----
-                await(W::C_SLOT + 4, round + 1);  // the round's values are in LDS (one loader per round)
+                await(W::C_SLOT + int(round & 1), round / 2 + 1);  // the round's values are in LDS (its loader's counter)
                 {
                     ValRegs<BITS> vreg[WAVE_STEPS];
 #pragma unroll
