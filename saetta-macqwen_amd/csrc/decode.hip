@@ -261,6 +261,48 @@ __device__ __forceinline__ float half_bits_to_float(uint32_t bits16) {
     return (float)__builtin_bit_cast(_Float16, uint16_t(bits16));
 }
 
+// The largest of four lane groups' values.  (By the instruction: fmaxf of a value that comes out of an exchange takes two more, which
+// quiet what might be a signalling NaN.)
+struct RawMaxOp {
+    __device__ __forceinline__ float operator()(float a, float b) const {
+        float r;
+        asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+        return r;
+    }
+};
+
+// The f16 of one group of a pair in the scales' planes, of two tokens: sel, of group_sel, names the group.
+typedef _Float16 half2_ __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t group_sel(int group) { return group & 1 ? 0x07060302u : 0x05040100u; }
+__device__ __forceinline__ half2_ group_halves(uint32_t w0, uint32_t w1, uint32_t sel) { return __builtin_bit_cast(half2_, perm(w1, w0, sel)); }
+
+// One query row's probability operand of a k-step, times the value scales of a group (sv, zv: the tokens' dwords of scales and biases,
+// sel: the group's).  The two lanes of a head (n and n + 8) make four of the lane group's eight tokens each (p4), both parts, and hand
+// over what the other one feeds: the hi lane (n < 8) feeds hi parts and wants the other lane's of tokens 4-7, the lo lane lo parts
+// and the other lane's of tokens 0-3.  A product with a scale and its lo part are fused operations that take the f16 as it is, two
+// tokens' from one permute, and the exchange writes half of a row's lanes (bank masks): 40 vector instructions where shifts, conversions
+// and selects made 54.
+__device__ __forceinline__ half8 one_row_operand(const floatx4 &p4, float f, const u32x4 &sv, const u32x4 &zv, uint32_t sel, float &zacc) {
+    const half2_ s[2] = {group_halves(sv.x, sv.y, sel), group_halves(sv.z, sv.w, sel)}, z[2] = {group_halves(zv.x, zv.y, sel), group_halves(zv.z, zv.w, sel)};
+    float x[4], lo[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float p = p4[e] * f;
+        zacc = fmaf(p, float(z[e >> 1][e & 1]), zacc);
+        x[e] = fmaf(p, float(s[e >> 1][e & 1]), 0.0f);
+        lo[e] = fmaf(p, float(s[e >> 1][e & 1]), -__builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x[e]) & 0xffffe000u));
+    }
+    // round toward zero: exact truncation to the hi part
+    int hi0 = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pkrtz(x[0], x[1])), hi1 = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pkrtz(x[2], x[3]));
+    int lo0 = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pkrtz(lo[0], lo[1])), lo1 = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pkrtz(lo[2], lo[3]));
+    constexpr int ROR_8 = 0x128, UPPER = 0xc, LOWER = 0x3;  // lanes 8-15 | 0-7 of a row of 16
+    uint32_t o[4] = {uint32_t(__builtin_amdgcn_update_dpp(hi0, lo0, ROR_8, 0xf, UPPER, false)), uint32_t(__builtin_amdgcn_update_dpp(hi1, lo1, ROR_8, 0xf, UPPER, false)),
+                     uint32_t(__builtin_amdgcn_update_dpp(lo0, hi0, ROR_8, 0xf, LOWER, false)), uint32_t(__builtin_amdgcn_update_dpp(lo1, hi1, ROR_8, 0xf, LOWER, false))};
+    // (pinned: left alone, the compiler moves an operand's arithmetic down to its use, behind the wait for the values)
+    asm volatile("" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
+    return as_half8(o[0], o[1], o[2], o[3]);
+}
+
 // ---- the step before the scores, taken in -------------------------------------------------------
 //
 // A token step of a plan records attention_prep_store, the partial and the reduce stage of a layer one after the other.
@@ -2391,10 +2433,24 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
         if constexpr (W::ALTERNATE) if (alt) {
             // ---- a share of more than one round: rounds of up to ALT_BLOCKS blocks in alternate halves of LDS ----
             // Round r lies in the blocks ALT_BLOCKS (r % 2) .. of the keys' and the values' places, of the scales and of
-            // the block table: every computing wave takes the scores of one block (4-bit codes: two) and two k-steps (four)
+            // the block table: every computing wave takes the scores of one block and two k-steps
             // of O += P V per round, and the loaders fill the other half meanwhile.  A half is free for round r + 2 when
             // every wave has built its operands (keys, scales, scores) and is through with the values of round r.
             constexpr int AB = W::ALT_BLOCKS, WAVE_BLOCKS = AB / W::WAVES, WAVE_STEPS = AB / 4;
+            // The query operands are held over the rounds: read anew in each they were 80 KB of the round's way through LDS, in front of its
+            // first product.  With the operands of one_row_operand, 4-bit codes at 150000 tokens 31.65 -> 30.25 us a layer, 60000 19.1 -> 17.9, 216000
+            // 40.8 -> 38.9; 8-bit codes, whose rounds wait for memory, 1 % and less.  What the loaders alone take there, with no arithmetic
+            // at all, is 25.4.  Tried here: scores a round ahead of the operands, so that no wave waits for another's (32.7); four
+            // places of 8 blocks for 4-bit codes, two rounds of every loader on their way (34.4: what has landed is told of later); the
+            // values and the next keys read as soon as they are there, under the operands (31.9).
+            half8 q_reg[8], qz_reg[2];
+#pragma unroll
+            for (int i = 0; i < 8; i++) q_reg[i] = q_lds[i * 64 + lane];
+            qz_reg[0] = *reinterpret_cast<const half8 *>(qz_lds + lane * 8);
+            qz_reg[1] = *reinterpret_cast<const half8 *>(qz_lds + (64 + lane) * 8);
+#pragma unroll
+            for (int i = 0; i < 8; i++) asm volatile("" : "+v"(q_reg[i]));
+            asm volatile("" : "+v"(qz_reg[0]), "+v"(qz_reg[1]));
 #pragma unroll 1
             for (uint32_t round = 0; round < n_rounds; round++) {
                 const uint32_t base = (blk_begin + place(round) * per_round) * BLOCK, nb = blocks_of(place(round));
@@ -2412,11 +2468,6 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
                         if (round > 1) await(W::C_BUILT, W::WAVES * (round - 1));
                         if (j == 0 && n < 8) bmax_lds[n * W::BSTRIDE + blk] = NO_SCORE, bsum_lds[n * W::BSTRIDE + blk] = 0.0f;
                     } else {
-                        half8 q_reg[8], qz_reg[2];
-#pragma unroll
-                        for (int i = 0; i < 8; i++) q_reg[i] = q_lds[i * 64 + lane];
-                        qz_reg[0] = *reinterpret_cast<const half8 *>(qz_lds + lane * 8);
-                        qz_reg[1] = *reinterpret_cast<const half8 *>(qz_lds + (64 + lane) * 8);
                         await(W::C_KPART + int(round & 1), round / 2 + 1);  // the round's keys and scales are in LDS (its loader's counter)
                         const unsigned char *kb = lds_raw + W::K_OFF + blk * W::K_BLOCK_BYTES;
                         KeyRegs<BITS> kreg[4];
@@ -2459,12 +2510,15 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
                             float d = 0.0f;
 #pragma unroll
                             for (int gg = 0; gg < 4; gg++) d += half_bits_to_float(sw[2 * tk + (gg >> 1)] >> (16 * (gg & 1))) * r[gg][tk];
-                            float v = sc[tk] + d * C1;
-                            v += dpp<0x128>(v);  // row_ror 8: the other part (hi | lo) of the same head
-                            sc[tk] = base + tok0 + tk < round_limit ? v : NO_SCORE;  // (also whatever a block past the round left in LDS)
+                            const float v = sc[tk] + d * C1;
+                            sc[tk] = v + dpp<0x128>(v);  // row_ror 8: the other part (hi | lo) of the same head
+                        }
+                        if (base + BLOCK * (rblk + 1) > round_limit) {
+#pragma unroll
+                            for (int tk = 0; tk < 4; tk++) sc[tk] = base + tok0 + tk < round_limit ? sc[tk] : NO_SCORE;  // (also whatever a block past the round left in LDS)
                         }
                         float cm = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
-                        cm = across_rows<16, 64>(cm, MaxOp());
+                        cm = across_rows<16, 64>(cm, RawMaxOp());
                         float sum = 0.0f;
 #pragma unroll
                         for (int tk = 0; tk < 4; tk++) {
@@ -2518,7 +2572,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
                 half8 p_alt[WAVE_STEPS];
                 {
                     const int hh = n >> 3;  // this lane makes tokens 8j + 4 hh .. + 3 of a k-step
-                    const int sh = 16 * (g & 1);
+                    const uint32_t sel = group_sel(g);
 #pragma unroll
                     for (int i = 0; i < WAVE_STEPS; i++) {
                         if (uint32_t(2 * (2 * i + b2)) >= nb) {  // the k-step has no tokens
@@ -2533,26 +2587,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
                         const u32x4 zv = *reinterpret_cast<const u32x4 *>(vsp + W::SB_ARRAY / 4);
                         // 2^(block maximum - maximum so far) * P_UP (2^8, so that the lo part stays a normal f16)
                         const float f = __builtin_amdgcn_exp2f(bmax_lds[(n & 7) * W::BSTRIDE + blk] - nm + 8.0f);
-                        const uint32_t sw[4] = {sv.x, sv.y, sv.z, sv.w}, zw[4] = {zv.x, zv.y, zv.z, zv.w};
-                        float x[4], lo[4];
-#pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            const float p = pt[e] * f;
-                            zacc += p * half_bits_to_float(zw[e] >> sh);
-                            x[e] = p * half_bits_to_float(sw[e] >> sh);
-                            lo[e] = x[e] - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x[e]) & 0xffffe000u);
-                        }
-                        // round toward zero: exact truncation to the hi part
-                        const uint32_t hi0 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x[0], x[1]));
-                        const uint32_t hi1 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x[2], x[3]));
-                        const uint32_t lo0 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo[0], lo[1]));
-                        const uint32_t lo1 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo[2], lo[3]));
-                        const uint32_t send0 = hh ? hi0 : lo0, send1 = hh ? hi1 : lo1;
-                        const uint32_t recv0 = uint32_t(__builtin_amdgcn_update_dpp(0, int(send0), 0x128, 0xf, 0xf, false));  // row_ror 8
-                        const uint32_t recv1 = uint32_t(__builtin_amdgcn_update_dpp(0, int(send1), 0x128, 0xf, 0xf, false));
-                        uint32_t o[4] = {hh ? recv0 : hi0, hh ? recv1 : hi1, hh ? lo0 : recv0, hh ? lo1 : recv1};
-                        asm volatile("" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
-                        p_alt[i] = as_half8(o[0], o[1], o[2], o[3]);
+                        p_alt[i] = one_row_operand(pt, f, sv, zv, sel, zacc);
                     }
                 }
                 raise(W::C_BUILT);  // this wave is through with the round's keys, scores, scales and biases
@@ -2659,13 +2694,16 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
                         float d = 0.0f;
 #pragma unroll
                         for (int gg = 0; gg < 4; gg++) d += half_bits_to_float(sw[2 * tk + (gg >> 1)] >> (16 * (gg & 1))) * r[gg][tk];
-                        float v = s[tk] + d * C1;
-                        v += dpp<0x128>(v);  // row_ror 8: the other part (hi | lo) of the same head
-                        s[tk] = base + tok0 + tk < round_limit ? v : NO_SCORE;  // (also whatever a block past the round left in LDS)
+                        const float v = s[tk] + d * C1;
+                        s[tk] = v + dpp<0x128>(v);  // row_ror 8: the other part (hi | lo) of the same head
+                    }
+                    if (base + BLOCK * (blk + 1) > round_limit) {
+#pragma unroll
+                        for (int tk = 0; tk < 4; tk++) s[tk] = base + tok0 + tk < round_limit ? s[tk] : NO_SCORE;  // (also whatever a block past the round left in LDS)
                     }
                     // the block's softmax relative to its own maximum, per head
                     float cm = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-                    cm = across_rows<16, 64>(cm, MaxOp());
+                    cm = across_rows<16, 64>(cm, RawMaxOp());
                     float sum = 0.0f;
 #pragma unroll
                     for (int tk = 0; tk < 4; tk++) {
@@ -2727,7 +2765,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
             half8 p_op[W::SLOTS];
             {
                 const int hh = n >> 3;  // this lane makes tokens 8j + 4 hh .. + 3 of a k-step
-                const int sh = 16 * (g & 1);
+                const uint32_t sel = group_sel(g);
                 const bool fifth = extra && b2 == 0;  // k-step 8: block 16 (lane groups 0 and 1; the others repeat them with factor 0)
 #pragma unroll
                 for (int sl = 0; sl < W::SLOTS; sl++) {
@@ -2748,29 +2786,7 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
                     const u32x4 zv = *reinterpret_cast<const u32x4 *>(vsp + W::SB_ARRAY / 4);
                     // 2^(block maximum - round maximum) * P_UP (2^8, so that the lo part stays a normal f16)
                     const float f = __builtin_amdgcn_exp2f(bmax_lds[(n & 7) * W::BSTRIDE + 2 * ks + (j >> 1)] - nm + 8.0f);
-                    const uint32_t sw[4] = {sv.x, sv.y, sv.z, sv.w}, zw[4] = {zv.x, zv.y, zv.z, zv.w};
-                    float x[4], lo[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const float p = pt[e] * f;
-                        zacc += p * half_bits_to_float(zw[e] >> sh);
-                        x[e] = p * half_bits_to_float(sw[e] >> sh);
-                        lo[e] = x[e] - __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x[e]) & 0xffffe000u);
-                    }
-                    // round toward zero: exact truncation to the hi part
-                    const uint32_t hi0 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x[0], x[1]));
-                    const uint32_t hi1 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x[2], x[3]));
-                    const uint32_t lo0 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo[0], lo[1]));
-                    const uint32_t lo1 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo[2], lo[3]));
-                    // the hi lane (n < 8) feeds hi parts and wants the other lane's hi parts of tokens 4-7; the lo
-                    // lane feeds lo parts and wants the other lane's lo parts of tokens 0-3
-                    const uint32_t send0 = hh ? hi0 : lo0, send1 = hh ? hi1 : lo1;
-                    const uint32_t recv0 = uint32_t(__builtin_amdgcn_update_dpp(0, int(send0), 0x128, 0xf, 0xf, false));  // row_ror 8
-                    const uint32_t recv1 = uint32_t(__builtin_amdgcn_update_dpp(0, int(send1), 0x128, 0xf, 0xf, false));
-                    uint32_t o[4] = {hh ? recv0 : hi0, hh ? recv1 : hi1, hh ? lo0 : recv0, hh ? lo1 : recv1};
-                    // (pinned: left alone, the compiler moves an operand's arithmetic down to its use, behind the wait for the values)
-                    asm volatile("" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
-                    p_op[sl] = as_half8(o[0], o[1], o[2], o[3]);
+                    p_op[sl] = one_row_operand(pt, f, sv, zv, sel, zacc);
                 }
             }
             if (more) raise(W::C_BUILT);  // this wave is through with the round's scores, scales and biases
