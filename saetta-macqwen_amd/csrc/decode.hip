@@ -2925,22 +2925,27 @@ static __device__ __align__(256) float scratch[STATIC_PART_O_FLOATS + STATIC_PAR
 constexpr int STATIC_MAX_DEVICES = 64;
 float *g_static_scratch[STATIC_MAX_DEVICES] = {};
 
-// One workgroup per (q head, row, 16 dims of the head): wave w takes a quarter of the splits, lane
-// (slot = lane / 4, quad = lane % 4) PER_LANE of them and four dims.  Latency is all there is to it: every load is
+// One workgroup per (q head, row, DIMS dims of the head): wave w takes a quarter of the splits, lane
+// (slot = lane / QUADS, quad = lane % QUADS) PER_LANE of them and four dims.  Latency is all there is to it: every load is
 // requested before anything is waited for (buffer loads, whose slots past the last split read zero: with a branch around each
 // the compiler waited for one before it asked for the next, and for the position before the first), a wave sums its splits
 // relative to its own maximum, so that the four waves meet once, through LDS.
 // A layer's token step, us, ten layers in a graph: 8-bit 300 tokens of 8192 9.1 -> 8.6, halves 4096 of 8192 10.9 -> 10.3, 8-bit 32768
 // 16.8 -> 16.0; eight rows at 1000 tokens 18.3 -> 17.3.
+// DIMS: a split's maximum and sum are a line of their own, read by every workgroup of a head, and 16 dims are half a line of its O,
+// so one row, which is latency, has many workgroups, and more rows, which are bytes, have wide ones.  Us a layer's step, 16, 32, 64, 128
+// dims: one row 8-bit 32768 tokens 15.67, 15.75, 15.91; two 16.98, 16.61, 16.86; three 22.24, 22.10, 21.90, 22.85; six of halves 57123 35.08,
+// 34.42, 34.40; eight 20000 28.2, 26.9, 26.8, 8-bit 30.2, 29.1, 28.9, 29.5.  (The maxima and sums of a head in a row, as [row][head][split]: three
+// rows 22.2 -> 21.8, but four of 4 bits at 3000 13.4 -> 13.8, one row 15.3 -> 15.4: eight scattered stores a split.)
 // WAIT: slots past the splits at work are left out of the requests, which have to wait for the position then.  One and two
 // rows read them all the same: the wait costs more than up to 2 MB of old partials a row.
-constexpr int REDUCE_DIMS = 16;
-template <int PER_LANE, bool WAIT>
+template <int DIMS, int PER_LANE, bool WAIT>
 __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
+    constexpr uint32_t QUADS = DIMS / 4, SLOTS = 64 / QUADS;
     __shared__ float wave_m[4], wave_l[4];
-    __shared__ floatx4 wave_o[4][4];
+    __shared__ floatx4 wave_o[4][QUADS];
     const uint32_t h = blockIdx.x, row = blockIdx.y, slice = blockIdx.z;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, slot = lane >> 2, quad = lane & 3;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, slot = lane / QUADS, quad = lane % QUADS;
     const size_t qh = size_t(row) * a.heads + h;
     const uint32_t position = a.tp->position, kv_len = a.tp->kv_len;
     uint32_t parts = 0, fresh = 0;
@@ -2954,7 +2959,7 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
     const __amdgpu_buffer_rsrc_t o_rsrc = make_rsrc(a.part_o + size_t(row) * records * DIM, records * DIM * 4);
     const __amdgpu_buffer_rsrc_t ml_rsrc = make_rsrc(a.part_ml + size_t(row) * records * 2, records * 8);
     const __amdgpu_buffer_rsrc_t g_rsrc = make_rsrc(a.q_and_gate + (qh * 2 + 1) * DIM, DIM * 4);
-    auto split_of = [&](int i) { return 16 * PER_LANE * wave + slot + 16 * i; };
+    auto split_of = [&](int i) { return SLOTS * PER_LANE * wave + slot + SLOTS * i; };
     floatx2 mlv[PER_LANE];
     floatx4 pv[PER_LANE];
 #pragma unroll
@@ -2962,9 +2967,9 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
         const uint32_t c = split_of(i), record = c * a.heads + h;
         const bool need = c < (WAIT ? parts : a.nsplits) || (WAIT && c == fresh);
         mlv[i] = __builtin_bit_cast(floatx2, __builtin_amdgcn_raw_buffer_load_b64(ml_rsrc, need ? int(record * 8) : OOB, 0, 0));
-        pv[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(o_rsrc, need ? int(record * (DIM * 4) + (REDUCE_DIMS * slice + 4 * quad) * 4) : OOB, 0, 0));
+        pv[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(o_rsrc, need ? int(record * (DIM * 4) + (DIMS * slice + 4 * quad) * 4) : OOB, 0, 0));
     }
-    const float g = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(g_rsrc, tid < REDUCE_DIMS ? int(REDUCE_DIMS * slice + tid) * 4 : OOB, 0, 0));
+    const float g = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(g_rsrc, tid < DIMS ? int(DIMS * slice + tid) * 4 : OOB, 0, 0));
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (!WAIT) splits_at_work();
     float m[PER_LANE], mx = NO_SCORE;
@@ -2979,8 +2984,14 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
     }
     // the wave's maximum; like the sums, over the 16 slots (lanes 4 apart: two steps inside a row of 16 lanes, two across
     // rows), the four quads of a slot having the same m and l
-    mx = fmaxf(mx, dpp<0x124>(mx)), mx = fmaxf(mx, dpp<0x128>(mx));  // row_ror 4, row_ror 8
+    if constexpr (QUADS <= 4) mx = fmaxf(mx, dpp<0x124>(mx));  // row_ror 4
+    if constexpr (QUADS <= 8) mx = fmaxf(mx, dpp<0x128>(mx));  // row_ror 8
     mx = across_rows<16, 64>(mx, MaxOp());
+    auto over_slots = [](float x) {
+        if constexpr (QUADS <= 4) x += dpp<0x124>(x);
+        if constexpr (QUADS <= 8) x += dpp<0x128>(x);
+        return across_rows<16, 64>(x, SumOp());
+    };
     float l = 0.0f;
     floatx4 o = {0, 0, 0, 0};
 #pragma unroll
@@ -2989,19 +3000,14 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
         l += w * mlv[i][1];
         o += pv[i] * w;
     }
-    l += dpp<0x124>(l), l += dpp<0x128>(l);
-    l = across_rows<16, 64>(l, SumOp());
+    l = over_slots(l);
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        float x = o[e];
-        x += dpp<0x124>(x), x += dpp<0x128>(x);
-        o[e] = across_rows<16, 64>(x, SumOp());
-    }
+    for (int e = 0; e < 4; e++) o[e] = over_slots(o[e]);
     if (lane == 0) wave_m[wave] = mx, wave_l[wave] = l;
-    if (lane < 4) wave_o[wave][lane] = o;  // (lane = quad)
+    if (lane < QUADS) wave_o[wave][lane] = o;  // (lane = quad)
     const float open = __builtin_amdgcn_rcpf(1.0f + __expf(-g));
     __syncthreads();
-    if (tid < REDUCE_DIMS) {
+    if (tid < DIMS) {
         const float M = fmaxf(fmaxf(wave_m[0], wave_m[1]), fmaxf(wave_m[2], wave_m[3]));
         float total = 0.0f, sum = 0.0f;
 #pragma unroll
@@ -3010,10 +3016,22 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
             total += f * wave_l[w];
             sum += f * wave_o[w][tid >> 2][tid & 3];
         }
-        a.out[qh * DIM + REDUCE_DIMS * slice + tid] = sum * __builtin_amdgcn_rcpf(total) * open;
+        a.out[qh * DIM + DIMS * slice + tid] = sum * __builtin_amdgcn_rcpf(total) * open;
     }
 }
-static_assert(MAX_SPLITS <= 4 * 64, "four splits a lane at most");
+static_assert(MAX_SPLITS <= 4 * 64, "launch_reduce's variants");
+
+// (more rows than one have a workgroup per CU, and half as many splits at most)
+template <int DIMS, bool WAIT>
+void launch_reduce(hipStream_t stream, const ReduceArgs &a) {
+    constexpr int ONE = DIMS / 16;  // splits a lane takes, of 64
+    const dim3 grid(a.heads, a.rows, DIM / DIMS);
+    if (a.nsplits <= MAX_SPLITS / 4) return launch(attention_reduce_kernel<DIMS, ONE, WAIT>, grid, 256, 0, stream, a);
+    if constexpr (DIMS == 16) {
+        if (a.nsplits > MAX_SPLITS / 2) return launch(attention_reduce_kernel<DIMS, 4 * ONE, WAIT>, grid, 256, 0, stream, a);
+    }
+    launch(attention_reduce_kernel<DIMS, 2 * ONE, WAIT>, grid, 256, 0, stream, a);
+}
 
 uint32_t splits_for(uint32_t capacity, uint32_t wanted) {
     // Never more than the 128-token chunks of the capacity, so that scratch sized as
@@ -3270,10 +3288,9 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
             }
         }
         ReduceArgs r{part_o, part_ml, q_and_gate, out, heads, capacity, nsplits, rows, d_tp, decode_len ? 1u : 0u, last_is_new};
-        void (*const reduce[][2])(ReduceArgs) = {{attention_reduce_kernel<1, false>, attention_reduce_kernel<1, true>},
-                                                 {attention_reduce_kernel<2, false>, attention_reduce_kernel<2, true>},
-                                                 {attention_reduce_kernel<4, false>, attention_reduce_kernel<4, true>}};
-        launch(reduce[nsplits <= 64 ? 0 : nsplits <= 128 ? 1 : 2][rows > 2], dim3(heads, rows, DIM / REDUCE_DIMS), 256, 0, stream, r);
+        if (rows == 1) launch_reduce<16, false>(stream, r);
+        else if (rows == 2) launch_reduce<32, false>(stream, r);
+        else launch_reduce<64, true>(stream, r);
     }
     return launch_status(what);
 }
@@ -3330,7 +3347,7 @@ int raise_lds_of_bits() {
 }  // namespace
 
 int setup_decode() {
-    if (int rc = load_kernel(reinterpret_cast<const void *>(attention_reduce_kernel<1, false>))) return rc;
+    if (int rc = load_kernel(reinterpret_cast<const void *>(attention_reduce_kernel<16, 1, false>))) return rc;
     {
         // (runs once per device, with that device current)
         int dev = 0;

@@ -522,6 +522,32 @@ def test_rounds_of_as_many_blocks_as_there_is_room_for(m, kind, splits):
         assert worst < MAX_ABS_F64, (tokens, worst)
 
 
+@pytest.mark.parametrize("splits", [1, 3, 63, 64, 65, 128])
+@pytest.mark.parametrize("m", [1, 2, 3, 8])
+def test_merge_of_any_number_of_splits(m, splits):
+    # The merge's workgroups have 16, 32 or 64 dims by the number of rows and a lane one or two times as many splits from 65 on.
+    # Half of the splits without a block: what lies in their places (NaN) has no weight.
+    rng = np.random.default_rng(4500 + splits)
+    capacity = 16384
+    k, v = (rng.standard_normal((2048, VALUES)).astype(np.float32) for _ in range(2))
+    q = rng.standard_normal((m, H, D)).astype(np.float32)
+    qg = rng.standard_normal((m, H, 2 * D)).astype(np.float32)
+    rows = saetta.AttentionRows(H, KV, capacity, m)
+    rows.splits = splits
+    for tokens in [2048, max(splits // 2, 1) * 16 + m]:
+        pos = tokens - m
+        kc, vc, kf, vf = cache_pair(k[:tokens], v[:tokens], saetta.KvBits.Half, capacity, poison=True)
+        rows.part_o.fill_(float("nan")), rows.part_ml.fill_(float("nan"))
+        out = torch.full((m, H, D), float("nan"), device="cuda")
+        plan = saetta.Plan()
+        rows.record(plan, m, dev(q), kc, vc, dev(qg), out, [saetta.TokenParams(0, pos + r).as_tensor("cuda") for r in range(m)])
+        plan.build().run()
+        got = host(out)
+        assert np.isfinite(got).all(), tokens
+        worst = np.abs(got - oracle.rows(q, kf, vf, pos, m, q_and_gate=qg, threads=8, f64=True)).max()
+        assert worst < MAX_ABS_F64, (tokens, worst)
+
+
 @pytest.mark.parametrize("splits", [100, 64, 7])
 def test_several_rows_with_fewer_splits(splits):
     # RowsAttentionParams.splits is an upper bound the caller may lower (src/rows.rs:344-367).  In a
