@@ -357,17 +357,20 @@ __device__ __forceinline__ void cached_row(const void *data, const uint16_t *sca
     }
 }
 
-// A workgroup of the new rows: q heads head0 .. head0 + heads - 1 of rows row0 .. row0 + nrows - 1 (of up to R).  A wave takes whole
-// heads: lane l holds dims l, 64 + l, 128 + l, 192 + l.
+// What a workgroup makes of the new rows: the keys and values of all rows up to its last, q heads head0 .. head0 + heads - 1 of rows
+// row0 .. row0 + nrows - 1 (of up to R), in LDS and, those that are its own, in memory.  A wave takes whole heads: lane l holds dims l,
+// 64 + l, 128 + l, 192 + l.
+struct NewRows {
+    float *keys, *values, *queries;  // [row][256] as the cache gives them; [row][head][256]
+};
 template <int BITS, int R>
-__device__ __forceinline__ void new_rows(const PartialArgs &a, const PrepArgs &p, unsigned char *lds, uint32_t waves, uint32_t row0, uint32_t nrows,
-                                         uint32_t head0, uint32_t heads) {
+__device__ __forceinline__ NewRows make_rows(const PartialArgs &a, const PrepArgs &p, unsigned char *lds, uint32_t waves, uint32_t row0, uint32_t nrows,
+                                             uint32_t head0, uint32_t heads, uint32_t position) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, kv = blockIdx.y, kvh = a.kv_heads, rows = row0 + nrows;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     float2 *rope = reinterpret_cast<float2 *>(lds);                                          // [row][32] sine, cosine
-    float *keys = reinterpret_cast<float *>(lds + R * 32 * 8), *values = keys + rows * DIM;  // [row][256]: as the cache gives them
-    float *queries = values + rows * DIM;                                                    // [row][head][256]
-    const uint32_t position = a.tp->position, kv_len = a.tp->kv_len;
+    float *keys = reinterpret_cast<float *>(lds + R * 32 * 8), *values = keys + rows * DIM;
+    float *queries = values + rows * DIM;
     // items: the rows' keys, their values, then the q heads
     const uint32_t items = 2 * rows + nrows * heads;
     float next[4];
@@ -454,6 +457,17 @@ __device__ __forceinline__ void new_rows(const PartialArgs &a, const PrepArgs &p
         }
     }
     __syncthreads();
+    return {keys, values, queries};
+}
+
+// A workgroup of the new rows (see make_rows).
+template <int BITS, int R>
+__device__ __forceinline__ void new_rows(const PartialArgs &a, const PrepArgs &p, unsigned char *lds, uint32_t waves, uint32_t row0, uint32_t nrows,
+                                         uint32_t head0, uint32_t heads) {
+    const uint32_t lane = threadIdx.x & 63, kv = blockIdx.y, kvh = a.kv_heads;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t position = a.tp->position, kv_len = a.tp->kv_len;
+    const auto [keys, values, queries] = make_rows<BITS, R>(a, p, lds, waves, row0, nrows, head0, heads, position);
     // the new tokens' partial result of every (row, head): scores in units of log2(e), as the other splits'
     for (uint32_t pair = wave; pair < nrows * heads; pair += waves) {
         const uint32_t row = row0 + pair / heads, seen = tokens_new(a, position, kv_len, row);
@@ -3033,6 +3047,150 @@ void launch_reduce(hipStream_t stream, const ReduceArgs &a) {
     launch(attention_reduce_kernel<DIMS, 2 * ONE, WAIT>, grid, 256, 0, stream, a);
 }
 
+// ---- a token step of a cache of one split: one launch -----------------------------------------------
+//
+// In a cache of up to 128 tokens (SAETTA_CHUNK) there is one split, so the step is neither work for the matrix cores nor anything to merge:
+// three launches and their trips through memory.  Here a workgroup of 512 threads takes a q head of a row: it makes the head's query and,
+// for itself, the new keys and values (make_rows; the first head's workgroup of a row stores them), and has the whole context beside them.
+// Sixteen lanes hold a token, 16 dims each, keys and values alike; what is in the cache is asked for before anything is known, as
+// far as the cache goes, and dropped by select where no token is.  Products and sums in f32, of the values that the cache gives.
+// A layer's step, us, ten layers in a graph, three launches -> one: 119 tokens of halves, one row 11.2 -> 6.9, two 12.2 -> 7.1, four 15.0 -> 7.6, eight
+// 17.4 -> 8.1; 8-bit 11.1 -> 7.8, 11.7 -> 7.9, 14.7 -> 8.5, 19.5 -> 9.2; 4-bit 11.1 -> 8.2, 11.7 -> 8.3, 14.7 -> 8.9, 20.3 -> 9.7; 20 tokens, one row, 8.7 -> 6.9,
+// 9.4 -> 7.8, 9.5 -> 8.2.  What is left is the launch, the trips to the position and to the rows, and the chain of the new rows (norm, rotation,
+// quantizer).  Threads: 256 take 7.3 (halves, one row) and 9.4 (eight), 8.3 and 11.1 (8-bit); 1024 7.5 and 8.2, 8.2 and 9.0.
+// The line is where there is a second split.
+constexpr int ALONE_TOKENS = SAETTA_CHUNK, ALONE_THREADS = 512, ALONE_PASS = ALONE_THREADS / 16, ALONE_PASSES = ALONE_TOKENS / ALONE_PASS;
+struct AloneArgs {
+    PartialArgs a;
+    PrepArgs prep;
+    float *out;
+};
+
+template <int BITS>
+__global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(AloneArgs t) {
+    constexpr int R = SAETTA_MAX_ROWS, WORDS = BITS / 2;  // dwords of 16 values
+    constexpr int ROWS_BYTES = R * 32 * 8 + (2 * R + 1) * DIM * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char rows_lds[ROWS_BYTES];
+    __shared__ float score_lds[ALONE_TOKENS + R], prob_lds[ALONE_TOKENS + R];
+    __shared__ __attribute__((aligned(16))) float o_lds[ALONE_THREADS / 64][DIM];
+    const PartialArgs &a = t.a;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, part = tid & 15, sub = tid >> 4;  // part: dims 16 part .. + 15; sub: token of a pass
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t row = blockIdx.x / SAETTA_GQA_GROUP, head0 = blockIdx.x % SAETTA_GQA_GROUP, kv = blockIdx.y, kvh = a.kv_heads;
+    const uint32_t position = a.tp->position, kv_len = a.tp->kv_len;
+    const size_t of_head = size_t(row) * a.heads + kv * SAETTA_GQA_GROUP + head0;
+
+    // ---- the cache ----
+    struct Sixteen {
+        uint32_t w[WORDS];
+        uint32_t scale, bias;
+    };
+    Sixteen key[ALONE_PASSES], value[ALONE_PASSES];
+    auto ask = [&](Sixteen &x, const void *data, const uint16_t *scales, const uint16_t *biases, uint32_t token) {
+        const size_t at = size_t(token) * kvh + kv;
+        const uint32_t *src = static_cast<const uint32_t *>(data) + at * (DIM * BITS / 32) + part * WORDS;
+        if constexpr (BITS == 4) {
+            const u32x2 v = *reinterpret_cast<const u32x2 *>(src);
+            x.w[0] = v.x, x.w[1] = v.y;
+        } else {
+#pragma unroll
+            for (int i = 0; i < WORDS / 4; i++) {
+                const u32x4 v = reinterpret_cast<const u32x4 *>(src)[i];
+                x.w[4 * i] = v.x, x.w[4 * i + 1] = v.y, x.w[4 * i + 2] = v.z, x.w[4 * i + 3] = v.w;
+            }
+        }
+        if constexpr (BITS != 16) x.scale = scales[at * 4 + part / 4], x.bias = biases[at * 4 + part / 4];
+    };
+#pragma unroll
+    for (int i = 0; i < ALONE_PASSES; i++) ask(key[i], a.kdata, a.kscales, a.kbiases, min(uint32_t(i * ALONE_PASS) + sub, a.capacity - 1));  // (no branch: each would wait)
+#pragma unroll
+    for (int i = 0; i < ALONE_PASSES; i++) ask(value[i], a.vdata, a.vscales, a.vbiases, min(uint32_t(i * ALONE_PASS) + sub, a.capacity - 1));
+    const float gate = t.prep.q_and_gate[(of_head * 2 + 1) * DIM + (tid & (DIM - 1))];
+    auto sixteen = [](const Sixteen &x, float (&v)[16]) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            if constexpr (BITS == 16) {
+                v[e] = half_bits_to_float(x.w[e / 2] >> (16 * (e & 1)));
+            } else {
+                constexpr int PER = 32 / BITS;
+                v[e] = fmaf(half_bits_to_float(x.scale), float((x.w[e / PER] >> (e % PER * BITS)) & ((1u << BITS) - 1)), half_bits_to_float(x.bias));
+            }
+        }
+    };
+
+    // ---- the new rows ----
+    const auto [keys, values, queries] = make_rows<BITS, R>(a, t.prep, rows_lds, ALONE_THREADS / 64, row, 1, head0, 1, position);
+
+    // ---- the scores, in units of log2(e): tokens of the cache that the row sees, then the new ones ----
+    const uint32_t before = tokens_before(a, position, kv_len), fresh = tokens_new(a, position, kv_len, row);
+    // (a decode sees min(kv_len, capacity) tokens: where the record says more than position + 1, rows past the new one too)
+    const uint32_t past = a.decode_len ? min(kv_len, a.capacity) : 0;
+    const float c = a.scale * 1.4426950408889634f;
+    float q[16];
+#pragma unroll
+    for (int e = 0; e < 16; e++) q[e] = queries[part * 16 + e] * c;
+#pragma unroll
+    for (int i = 0; i < ALONE_PASSES; i++) {
+        const uint32_t token = i * ALONE_PASS + sub;
+        float k[16], s = 0.0f;
+        sixteen(key[i], k);
+#pragma unroll
+        for (int e = 0; e < 16; e++) s += q[e] * k[e];
+        s = group_reduce<16>(s, SumOp());
+        const bool live = token < before || (token > position && token < past);
+        if (part == 0) score_lds[token] = live ? s : NO_SCORE;
+    }
+    for (uint32_t n = wave; n < uint32_t(R); n += ALONE_THREADS / 64) {
+        float s = NO_SCORE;
+        if (n < fresh) {
+            s = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; i++) s += queries[64 * i + lane] * c * keys[n * DIM + 64 * i + lane];
+            s = group_reduce<64>(s, SumOp());
+        }
+        if (lane == 0) score_lds[ALONE_TOKENS + n] = s;
+    }
+    __syncthreads();
+
+    // ---- the softmax: every wave for itself, the first hands the probabilities out ----
+    float s[3] = {score_lds[lane], score_lds[64 + lane], lane < uint32_t(R) ? score_lds[ALONE_TOKENS + lane] : NO_SCORE};
+    const float m = group_reduce<64>(fmaxf(fmaxf(s[0], s[1]), s[2]), MaxOp());
+#pragma unroll
+    for (int i = 0; i < 3; i++) s[i] = s[i] > 0.5f * NO_SCORE ? __builtin_amdgcn_exp2f(s[i] - m) : 0.0f;
+    const float l = group_reduce<64>(s[0] + s[1] + s[2], SumOp());
+    if (wave == 0) {
+        prob_lds[lane] = s[0], prob_lds[64 + lane] = s[1];
+        if (lane < uint32_t(R)) prob_lds[ALONE_TOKENS + lane] = s[2];
+    }
+    __syncthreads();
+
+    // ---- the values ----
+    float o[16];
+#pragma unroll
+    for (int e = 0; e < 16; e++) o[e] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < ALONE_PASSES; i++) {
+        const float p = prob_lds[i * ALONE_PASS + sub];
+        float v[16];
+        sixteen(value[i], v);
+#pragma unroll
+        for (int e = 0; e < 16; e++) o[e] += p > 0.0f ? p * v[e] : 0.0f;  // (never a product with what lies where no token is)
+    }
+#pragma unroll
+    for (int e = 0; e < 16; e++) o[e] = across_rows<16, 64>(o[e], SumOp());
+    if (lane < 16) {
+#pragma unroll
+        for (int e = 0; e < 16; e += 4) *reinterpret_cast<floatx4 *>(&o_lds[wave][16 * part + e]) = floatx4{o[e], o[e + 1], o[e + 2], o[e + 3]};
+    }
+    __syncthreads();
+    if (tid >= uint32_t(DIM)) return;
+    float sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < ALONE_THREADS / 64; w++) sum += o_lds[w][tid];
+    for (uint32_t n = 0; n < fresh; n++) sum += prob_lds[ALONE_TOKENS + n] * values[n * DIM + tid];
+    t.out[of_head * DIM + tid] = sum * __builtin_amdgcn_rcpf(l) * __builtin_amdgcn_rcpf(1.0f + __expf(-gate));
+}
+
 uint32_t splits_for(uint32_t capacity, uint32_t wanted) {
     // Never more than the 128-token chunks of the capacity, so that scratch sized as
     // rows * ceil(capacity / 128) * heads partials is always enough.
@@ -3166,9 +3324,10 @@ void launch_partial_rows(hipStream_t stream, const PartialArgs &a, bool one_per_
 // inverse_root take, and the new tokens take a split of their own: with fewer than 4 the context would be left with too few
 // workgroups.  (The branch to the library's sine and cosine inside them was 1 to 1.6 % of a step at 32768 tokens of 8 bits,
 // taken or not.)
-bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const float *q_and_gate, bool keys_first, TokenArgs &token) {
+// out: where the step is to be one launch, which then writes it (a cache of up to ALONE_TOKENS), else nullptr.
+bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const float *q_and_gate, const float *out, bool keys_first, TokenArgs &token) {
     const size_t n = list.launches.size();
-    if (n < 2 || a.nsplits < 4) return false;
+    if (n < 2 || (!out && a.nsplits < 4)) return false;
     const LaunchRecord &before = list.launches[n - 2], &partial = list.launches[n - 1];
     if (before.kind != LAUNCH_PREP || partial.kind != LAUNCH_PARTIAL || int(before.bits) != bits || int(partial.bits) != bits || before.rows != a.rows) return false;
     const PartialArgs &b = list.arg<PartialArgs>(partial, 0);
@@ -3192,7 +3351,7 @@ bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const fl
                            {prep.k_norm, DIM * sizeof(float)}, {a.tp, sizeof(saetta_token_params)}},
                outputs[] = {{prep.k_back, prep.k_back ? row_kv : 0}, {prep.q_out, row_q}, {a.part_o, partials * DIM * sizeof(float)},
                             {a.part_ml, partials * 2 * sizeof(float)}, {a.kdata, data}, {a.vdata, data}, {a.kscales, scales},
-                            {a.kbiases, scales}, {a.vscales, scales}, {a.vbiases, scales}};
+                            {a.kbiases, scales}, {a.vscales, scales}, {a.vbiases, scales}, {out, out ? row_q : 0}};
     for (const Span &o : outputs) {
         for (const Span &i : inputs) {
             if (!apart(o, i)) return false;
@@ -3202,6 +3361,7 @@ bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const fl
         }
     }
     token = TokenArgs{a, prep, SAETTA_GQA_GROUP};
+    if (out) return true;
     const uint32_t room = MAX_SPLITS / 2;  // workgroups of a kv head, one to a CU
     if (keys_first && (bits == 16 || code_rows(bits, a.rows, a.capacity, true))) {
         // a workgroup per new row, for which a full context gives up CUs (two rows to one: 6 rows at 57123 tokens 36.2 against
@@ -3280,7 +3440,14 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
         uint32_t last_is_new = 0;
         if (LaunchList *list = recording()) {
             TokenArgs token;
-            if (one_per_cu && token_step(*list, a, bits, q_and_gate, keys_first, token)) {
+            if (capacity <= uint32_t(ALONE_TOKENS) && token_step(*list, a, bits, q_and_gate, out, keys_first, token)) {
+                list->launches.pop_back(), list->launches.pop_back();
+                const AloneArgs alone{token.a, token.prep, out};
+                launch(bits == 16 ? attention_token_alone_kernel<16> : bits == 8 ? attention_token_alone_kernel<8> : attention_token_alone_kernel<4>,
+                       dim3(rows * SAETTA_GQA_GROUP, kv_heads), ALONE_THREADS, 0, stream, alone);
+                return launch_status(what);
+            }
+            if (one_per_cu && token_step(*list, a, bits, q_and_gate, nullptr, keys_first, token)) {
                 list->launches.pop_back(), list->launches.pop_back();
                 partial(&token);
                 last_is_new = 1;

@@ -124,6 +124,49 @@ def test_a_length_of_the_callers_own(kind, capacity):
                 assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), (position, kv_len)
 
 
+@pytest.mark.parametrize("rows", [1, 2, 5, 8])
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_cache_of_one_split_takes_one_launch(kind, rows):
+    # Up to 128 tokens: a workgroup per (row, q head) does the whole step.  No context, around a pass of 16 tokens, the last rows that
+    # fit and rows that do not; a decode also without the new token and with rows past it.
+    step = Step(kind, 128, rows, seed=500 + 10 * rows + kind.value)
+    assert launches(step) == 1
+    built = step.plan.build()
+    for position in (0, 1, 15, 16, 17, 100, 128 - rows, 127, 130):
+        for kv_len in (None,) if rows > 1 else (None, 1, position, position + 2, position + 40, 200):
+            if kv_len == 0:
+                continue  # (no token at all: no number)
+            want = step.run(step.plan.run_serial, position, kv_len)
+            before = [host(b).copy() for b in step.cache.buffers()]
+            got = step.run(built.run, position, kv_len)
+            assert np.isfinite(want[0]).all() and np.isfinite(got[0]).all(), (position, kv_len)
+            assert np.abs(got[0] - want[0]).max() < 2e-5, (position, kv_len)
+            for x, y in zip(got[1:], want[1:3] + before):
+                assert np.array_equal(x.view(np.uint8), y.view(np.uint8)), (position, kv_len)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_one_launch_where_its_buffers_lie_apart(kind):
+    def result_over_the_key(step):
+        step.k = step.out[:, :VALUES].view(step.rows, VALUES)
+    for lay in (key_in_place, result_over_the_key):
+        check_laid_over(Step(kind, 128, 1, seed=70 + kind.value, lay=lay), (0, 50, 127))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_one_launch_drops_what_is_not_in_use(kind):
+    # NaN in the rows past the context: halves, or scales and biases
+    step = Step(kind, 128, 3, seed=90 + kind.value)
+    built = step.plan.build()
+    for buffer in step.cache.buffers():
+        if buffer.dtype == torch.float16:
+            rows = buffer.view(128, -1)
+            rows[37:] = float("nan")
+    want = step.run(step.plan.run_serial, 37)
+    got = step.run(built.run, 37)
+    assert np.isfinite(got[0]).all() and np.abs(got[0] - want[0]).max() < 2e-5
+
+
 def check_laid_over(step, positions):
     """A step with buffers over each other keeps its launches; outputs as the ops one by one, what is stored bit for bit."""
     assert launches(step) == 3
