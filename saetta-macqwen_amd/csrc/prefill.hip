@@ -1622,6 +1622,12 @@ FlashPlan tiles_plan(uint32_t pos, uint32_t tokens, uint32_t kv_heads, float &ti
 // The whole call, halves, what it was -> parts: 7 tokens at 3000 31.3 -> 19.5 us, at 20000 49.8 -> 29.9, at 100000 186 -> 54.6; 30 at 3000 34.1 ->
 // 22.2, at 40000 79.0 -> 54.4; 64 at 1500 32.7 -> 20.9, at 20000 64.6 -> 52.8; 128 at 1000 25.0 -> 22.8, at 3000 35.6 -> 31.6; 250 at 1500
 // 36.2 -> 31.9.  Left alone: 128 at 10000 54.1 and 53.5, 250 at 4000 46.8 and 52.1 (with codes 49.3 and 53.8).
+// Against its keys in parts a workgroup that goes through all of them is counted a quarter dearer, over codes a third: the figure above
+// is the lowest that sends a chunk away from the tiles, and 300 to 600 keys take longer (12 tokens over 8-bit codes at 400 take 18.4 us, by
+// the figure 12.7).  Whole calls, unsplit -> in two or three parts, halves | 8-bit | 4-bit: 12 tokens at 330 12.8 (left whole) | 16.6 -> 14.9 | 15.4 ->
+// 14.4; 12 at 540 17.6 -> 13.2 | 19.6 -> 15.2 | 20.1 -> 14.7; 60 at 470 17.0 -> 14.2 | 19.8 -> 16.3 | 20.7 -> 16.1; 100 at 400 15.2 -> 14.3 | 20.2 -> 16.6 |
+// 18.1 -> 16.5; 150 at 470 19.9 -> 17.2 | 20.3 -> 19.1 | 21.0 -> 19.1.  That holds up to row groups for 0.3 of the CUs (so that two parts fill
+// 0.6 of them): 200 tokens of 2 kv heads at 400 would go from 20.4 to 24.6 over 8-bit codes and 250 from 22.6 to 25.4.
 void choose_small(FlashPlan &f, uint32_t pos, uint32_t tokens, uint32_t kv_heads, int bits, float tiles_us) {
     const bool codes = bits != 16;
     const float SMALL_US = 5.0f, BLOCK_US = codes ? 0.59f : 0.5f;
@@ -1633,7 +1639,8 @@ void choose_small(FlashPlan &f, uint32_t pos, uint32_t tokens, uint32_t kv_heads
     const float small_us = rounds_us(f.cus, groups, float(longest), float(shortest), SMALL_US, BLOCK_US, 0.0f);
     f.small = small_us < tiles_us;
     if (2 * uint64_t(groups) > f.cus) return;
-    float best = 0.95f * (f.small ? small_us : tiles_us);
+    const bool few = 10 * uint64_t(groups) <= 3 * uint64_t(f.cus);
+    float best = !f.small ? 0.95f * tiles_us : !few ? 0.95f * small_us : codes ? 1.35f * small_us : 1.25f * small_us;
     const uint32_t least = (longest + SMALL_MAX_PARTS - 1) / SMALL_MAX_PARTS;
     for (uint32_t pb = (least + SMALL_WAVES - 1) / SMALL_WAVES * SMALL_WAVES; pb < longest; pb += SMALL_WAVES) {
         const uint32_t nparts = (longest + pb - 1) / pb, items = groups * nparts;

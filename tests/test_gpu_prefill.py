@@ -375,6 +375,32 @@ def test_no_workspace_is_as_good_as_one(kind, pos, tokens, kv):
         assert call(ws.data_ptr(), nbytes) == -6  # SAETTA_E_SCRATCH
 
 
+@pytest.mark.parametrize("kind,pos,tokens,kv,split", [(saetta.KvBits.Half, 379, 5, 2, False), (saetta.KvBits.Half, 380, 5, 2, True), (saetta.KvBits.Eight, 314, 6, 2, False),
+                                                      (saetta.KvBits.Four, 315, 6, 2, True), (saetta.KvBits.Half, 480, 152, 2, True), (saetta.KvBits.Half, 480, 153, 2, False),
+                                                      (saetta.KvBits.Eight, 400, 152, 2, True), (saetta.KvBits.Four, 400, 153, 2, False), (saetta.KvBits.Eight, 511, 1, 1, True)])
+def test_few_row_groups_over_some_hundred_keys(kind, pos, tokens, kv, split):
+    # at the lines of the rule: the blocks from which keys go to parts, 76 row groups and 78 (256 CUs); recorded without a workspace
+    # the same chunk takes all of its keys in one workgroup a row group
+    call, out, p, want = chunk(kind, pos, tokens, kv)
+    size = saetta.attention_prefill.workspace_bytes(p)
+    ws = torch.full((size,), 0xff, dtype=torch.uint8, device="cuda")
+    lib, results = saetta.ffi.lib(), []
+    assert lib.saetta_plan_begin() == 0
+    results.append(call(None, 0))
+    plan = ctypes.c_void_p(lib.saetta_plan_end())
+    assert results == [0], lib.saetta_last_error()
+    try:
+        for run_it in (lambda: call(ws.data_ptr(), size), lambda: lib.saetta_plan_run(saetta.host._stream(), plan)):
+            out.fill_(float("nan"))
+            assert run_it() == 0, lib.saetta_last_error()
+            assert float((out.double() - want).norm() / want.norm()) < REL_RMS
+            assert float((out - want).abs().max()) < MAX_ABS
+        assert bool((ws != 0xff).any()) == split
+    finally:
+        torch.cuda.synchronize()
+        lib.saetta_plan_free(plan)
+
+
 @pytest.mark.parametrize("pos,tokens", [(2045, 3), (2300, 4), (4200, 3), (8186, 5), (8200, 4), (16300, 2)])
 def test_many_parts_are_merged_by_teams(pos, tokens):
     # 8 parts of 8 blocks and one team, 9 and more and four: teams without a part, one batch each and two, a last batch of one
