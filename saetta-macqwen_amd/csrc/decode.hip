@@ -58,6 +58,7 @@
 //   attention_partial_kernel_c   the same over codes: two rows and more in the caches that code_rows names
 //                                (decode_code_rows.hpp)
 //   attention_reduce_kernel      the merge of the splits and the gate
+//   attention_token_alone_kernel a recorded token step over a cache of one split: store, attention and gate
 // Which one runs is decided in run_attention from the launch arguments alone, so that the partial
 // and the reduce stage of a step agree on the number of splits.
 #include "common.hpp"
