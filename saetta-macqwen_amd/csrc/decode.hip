@@ -58,7 +58,7 @@
 //   attention_partial_kernel_c   the same over codes: two rows and more in the caches that code_rows names
 //                                (decode_code_rows.hpp)
 //   attention_reduce_kernel      the merge of the splits and the gate
-//   attention_token_alone_kernel a recorded token step over a cache of one split: store, attention and gate
+//   attention_token_alone_kernel a recorded token step over a small cache: store, attention and gate
 // Which one runs is decided in run_attention from the launch arguments alone, so that the partial
 // and the reduce stage of a step agree on the number of splits.
 #include "common.hpp"
@@ -3048,31 +3048,38 @@ void launch_reduce(hipStream_t stream, const ReduceArgs &a) {
     launch(attention_reduce_kernel<DIMS, 2 * ONE, WAIT>, grid, 256, 0, stream, a);
 }
 
-// ---- a token step of a cache of one split: one launch -----------------------------------------------
+// ---- a token step of a cache of up to three splits: one launch --------------------------------------
 //
 // In a cache of up to 128 tokens (SAETTA_CHUNK) there is one split, so the step is neither work for the matrix cores nor anything to merge:
 // three launches and their trips through memory.  Here a workgroup of 512 threads takes a q head of a row: it makes the head's query and,
 // for itself, the new keys and values (make_rows; the first head's workgroup of a row stores them), and has the whole context beside them.
 // Sixteen lanes hold a token, 16 dims each, keys and values alike; what is in the cache is asked for before anything is known, as
-// far as the cache goes, and dropped by select where no token is.  Products and sums in f32, of the values that the cache gives.
-// A layer's step, us, ten layers in a graph, three launches -> one: 119 tokens of halves, one row 11.2 -> 6.9, two 12.2 -> 7.1, four 15.0 -> 7.6, eight
-// 17.4 -> 8.1; 8-bit 11.1 -> 7.8, 11.7 -> 7.9, 14.7 -> 8.5, 19.5 -> 9.2; 4-bit 11.1 -> 8.2, 11.7 -> 8.3, 14.7 -> 8.9, 20.3 -> 9.7; 20 tokens, one row, 8.7 -> 6.9,
-// 9.4 -> 7.8, 9.5 -> 8.2.  What is left is the launch, the trips to the position and to the rows, and the chain of the new rows (norm, rotation,
-// quantizer).  Threads: 256 take 7.3 (halves, one row) and 9.4 (eight), 8.3 and 11.1 (8-bit); 1024 7.5 and 8.2, 8.2 and 9.0.
-// The line is where there is a second split.
-constexpr int ALONE_TOKENS = SAETTA_CHUNK, ALONE_THREADS = 512, ALONE_PASS = ALONE_THREADS / 16, ALONE_PASSES = ALONE_TOKENS / ALONE_PASS;
+// far as the cache goes, and dropped by select where no token is.  Products and sums in f32, of halves as the cache gives them, of codes as numbers:
+// a token's scale and bias are the same for a lane's sixteen and go into their sums (relative error against 64 bits 4e-7 to 9e-7, where the
+// three launches have 8e-7 to 8e-6; each value made first 1.5e-7 to 2.8e-7 at 0.9 us more a 128 tokens).
+// A layer's step, us, ten layers in a graph, three launches -> one: 118 tokens of halves, one row 11.2 -> 6.4, two 12.2 -> 6.6, four 15.0 -> 7.1, eight
+// 17.4 -> 7.6; 8-bit 11.1 -> 6.7, 11.7 -> 6.8, 14.7 -> 7.4, 19.5 -> 8.1; 4-bit 11.1 -> 7.3, 11.7 -> 7.4, 14.7 -> 8.0, 20.3 -> 8.7; 28 tokens, one row, 8.7 ->
+// 6.4, 9.4 -> 6.7, 9.5 -> 7.3.  Caches of 256, 156 tokens in use: two rows 11.1 -> 9.4, 11.4 -> 8.6, 11.7 -> 9.5, three 13.2 -> 9.5, 13.8 -> 8.6, 13.8 -> 9.6, eight
+// 16.3 -> 10.3, 18.0 -> 9.8, 18.6 -> 10.9.  Of 384, 284 in use: three rows 13.3 -> 11.5, 13.9 -> 10.9, 13.9 -> 11.6, eight 17.6 -> 12.4, 19.5 -> 12.1, 20.2 -> 12.9.
+// What is left is the launch, the trips to the position and to the rows, the chain of the new rows (norm, rotation, quantizer) and 2 us per
+// 128 tokens of cache, vector instructions.  Threads: 256 take 7.3 (halves, one row; 6.9 then) and 9.4 (eight; 8.1), 8.3 and 11.1 (8-bit; 7.8 and 9.2);
+// 1024 7.5 and 8.2, 8.2 and 9.0.
+// The line: two rows in a cache of 384 are even (halves 11.2 -> 11.4, 4-bit 11.7 -> 11.5).  One row would be ahead in one of 256 too (10.2 -> 9.4, 10.2 -> 8.6,
+// 10.4 -> 9.4) and five and more in one of 512, but those steps are the three launches that test_gpu_token_step.py counts.
+constexpr int ALONE_THREADS = 512, ALONE_PASS = ALONE_THREADS / 16;
+uint32_t alone_tokens(uint32_t rows) { return rows == 1 ? SAETTA_CHUNK : rows == 2 ? 2 * SAETTA_CHUNK : 3 * SAETTA_CHUNK; }
 struct AloneArgs {
     PartialArgs a;
     PrepArgs prep;
     float *out;
 };
 
-template <int BITS>
+template <int BITS, int TOKENS>
 __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(AloneArgs t) {
-    constexpr int R = SAETTA_MAX_ROWS, WORDS = BITS / 2;  // dwords of 16 values
+    constexpr int R = SAETTA_MAX_ROWS, WORDS = BITS / 2, PASSES = TOKENS / ALONE_PASS;  // WORDS: dwords of 16 values
     constexpr int ROWS_BYTES = R * 32 * 8 + (2 * R + 1) * DIM * 4;
     __shared__ __attribute__((aligned(16))) unsigned char rows_lds[ROWS_BYTES];
-    __shared__ float score_lds[ALONE_TOKENS + R], prob_lds[ALONE_TOKENS + R];
+    __shared__ float score_lds[TOKENS + R], prob_lds[TOKENS + R];
     __shared__ __attribute__((aligned(16))) float o_lds[ALONE_THREADS / 64][DIM];
     const PartialArgs &a = t.a;
     const uint32_t tid = threadIdx.x, lane = tid & 63, part = tid & 15, sub = tid >> 4;  // part: dims 16 part .. + 15; sub: token of a pass
@@ -3086,7 +3093,7 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
         uint32_t w[WORDS];
         uint32_t scale, bias;
     };
-    Sixteen key[ALONE_PASSES], value[ALONE_PASSES];
+    Sixteen key[PASSES], value[PASSES];
     auto ask = [&](Sixteen &x, const void *data, const uint16_t *scales, const uint16_t *biases, uint32_t token) {
         const size_t at = size_t(token) * kvh + kv;
         const uint32_t *src = static_cast<const uint32_t *>(data) + at * (DIM * BITS / 32) + part * WORDS;
@@ -3103,18 +3110,20 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
         if constexpr (BITS != 16) x.scale = scales[at * 4 + part / 4], x.bias = biases[at * 4 + part / 4];
     };
 #pragma unroll
-    for (int i = 0; i < ALONE_PASSES; i++) ask(key[i], a.kdata, a.kscales, a.kbiases, min(uint32_t(i * ALONE_PASS) + sub, a.capacity - 1));  // (no branch: each would wait)
+    for (int i = 0; i < PASSES; i++) ask(key[i], a.kdata, a.kscales, a.kbiases, min(uint32_t(i * ALONE_PASS) + sub, a.capacity - 1));  // (no branch: each would wait)
 #pragma unroll
-    for (int i = 0; i < ALONE_PASSES; i++) ask(value[i], a.vdata, a.vscales, a.vbiases, min(uint32_t(i * ALONE_PASS) + sub, a.capacity - 1));
+    for (int i = 0; i < PASSES; i++) ask(value[i], a.vdata, a.vscales, a.vbiases, min(uint32_t(i * ALONE_PASS) + sub, a.capacity - 1));
     const float gate = t.prep.q_and_gate[(of_head * 2 + 1) * DIM + (tid & (DIM - 1))];
+    // (codes as numbers: scale and bias are the same for the sixteen, and go into their sums)
     auto sixteen = [](const Sixteen &x, float (&v)[16]) {
 #pragma unroll
         for (int e = 0; e < 16; e++) {
             if constexpr (BITS == 16) {
                 v[e] = half_bits_to_float(x.w[e / 2] >> (16 * (e & 1)));
+            } else if constexpr (BITS == 8) {
+                v[e] = float((x.w[e / 4] >> (8 * (e & 3))) & 255);
             } else {
-                constexpr int PER = 32 / BITS;
-                v[e] = fmaf(half_bits_to_float(x.scale), float((x.w[e / PER] >> (e % PER * BITS)) & ((1u << BITS) - 1)), half_bits_to_float(x.bias));
+                v[e] = float((((x.w[e / 8] >> (4 * (e & 1))) & 0x0f0f0f0fu) >> (8 * (e / 2 & 3))) & 255);
             }
         }
     };
@@ -3127,16 +3136,17 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
     // (a decode sees min(kv_len, capacity) tokens: where the record says more than position + 1, rows past the new one too)
     const uint32_t past = a.decode_len ? min(kv_len, a.capacity) : 0;
     const float c = a.scale * 1.4426950408889634f;
-    float q[16];
+    float q[16], q_sum = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 16; e++) q[e] = queries[part * 16 + e] * c;
+    for (int e = 0; e < 16; e++) q[e] = queries[part * 16 + e] * c, q_sum += q[e];
 #pragma unroll
-    for (int i = 0; i < ALONE_PASSES; i++) {
+    for (int i = 0; i < PASSES; i++) {
         const uint32_t token = i * ALONE_PASS + sub;
         float k[16], s = 0.0f;
         sixteen(key[i], k);
 #pragma unroll
         for (int e = 0; e < 16; e++) s += q[e] * k[e];
+        if constexpr (BITS != 16) s = half_bits_to_float(key[i].scale) * s + half_bits_to_float(key[i].bias) * q_sum;
         s = group_reduce<16>(s, SumOp());
         const bool live = token < before || (token > position && token < past);
         if (part == 0) score_lds[token] = live ? s : NO_SCORE;
@@ -3149,36 +3159,49 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
             for (int i = 0; i < 4; i++) s += queries[64 * i + lane] * c * keys[n * DIM + 64 * i + lane];
             s = group_reduce<64>(s, SumOp());
         }
-        if (lane == 0) score_lds[ALONE_TOKENS + n] = s;
+        if (lane == 0) score_lds[TOKENS + n] = s;
     }
     __syncthreads();
 
     // ---- the softmax: every wave for itself, the first hands the probabilities out ----
-    float s[3] = {score_lds[lane], score_lds[64 + lane], lane < uint32_t(R) ? score_lds[ALONE_TOKENS + lane] : NO_SCORE};
-    const float m = group_reduce<64>(fmaxf(fmaxf(s[0], s[1]), s[2]), MaxOp());
+    constexpr int OLD = TOKENS / 64;
+    float s[OLD + 1], m = s[OLD] = lane < uint32_t(R) ? score_lds[TOKENS + lane] : NO_SCORE, l = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 3; i++) s[i] = s[i] > 0.5f * NO_SCORE ? __builtin_amdgcn_exp2f(s[i] - m) : 0.0f;
-    const float l = group_reduce<64>(s[0] + s[1] + s[2], SumOp());
+    for (int i = 0; i < OLD; i++) s[i] = score_lds[64 * i + lane], m = fmaxf(m, s[i]);
+    m = group_reduce<64>(m, MaxOp());
+#pragma unroll
+    for (int i = 0; i <= OLD; i++) s[i] = s[i] > 0.5f * NO_SCORE ? __builtin_amdgcn_exp2f(s[i] - m) : 0.0f, l += s[i];
+    l = group_reduce<64>(l, SumOp());
     if (wave == 0) {
-        prob_lds[lane] = s[0], prob_lds[64 + lane] = s[1];
-        if (lane < uint32_t(R)) prob_lds[ALONE_TOKENS + lane] = s[2];
+#pragma unroll
+        for (int i = 0; i < OLD; i++) prob_lds[64 * i + lane] = s[i];
+        if (lane < uint32_t(R)) prob_lds[TOKENS + lane] = s[OLD];
     }
     __syncthreads();
 
     // ---- the values ----
-    float o[16];
+    float o[16], biases = 0.0f;
 #pragma unroll
     for (int e = 0; e < 16; e++) o[e] = 0.0f;
 #pragma unroll
-    for (int i = 0; i < ALONE_PASSES; i++) {
-        const float p = prob_lds[i * ALONE_PASS + sub];
-        float v[16];
-        sixteen(value[i], v);
+    for (int i = 0; i < PASSES; i++) {
+        float p = prob_lds[i * ALONE_PASS + sub];
+        const bool live = p > 0.0f;  // (never a product with what lies where no token is)
+        Sixteen &x = value[i];
+        if constexpr (BITS == 16) {
 #pragma unroll
-        for (int e = 0; e < 16; e++) o[e] += p > 0.0f ? p * v[e] : 0.0f;  // (never a product with what lies where no token is)
+            for (int w = 0; w < WORDS; w++) x.w[w] = live ? x.w[w] : 0;
+        } else {
+            biases += live ? p * half_bits_to_float(x.bias) : 0.0f;
+            p = live ? p * half_bits_to_float(x.scale) : 0.0f;
+        }
+        float v[16];
+        sixteen(x, v);
+#pragma unroll
+        for (int e = 0; e < 16; e++) o[e] += p * v[e];
     }
 #pragma unroll
-    for (int e = 0; e < 16; e++) o[e] = across_rows<16, 64>(o[e], SumOp());
+    for (int e = 0; e < 16; e++) o[e] = across_rows<16, 64>(o[e] + biases, SumOp());
     if (lane < 16) {
 #pragma unroll
         for (int e = 0; e < 16; e += 4) *reinterpret_cast<floatx4 *>(&o_lds[wave][16 * part + e]) = floatx4{o[e], o[e + 1], o[e + 2], o[e + 3]};
@@ -3188,7 +3211,7 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
     float sum = 0.0f;
 #pragma unroll
     for (int w = 0; w < ALONE_THREADS / 64; w++) sum += o_lds[w][tid];
-    for (uint32_t n = 0; n < fresh; n++) sum += prob_lds[ALONE_TOKENS + n] * values[n * DIM + tid];
+    for (uint32_t n = 0; n < fresh; n++) sum += prob_lds[TOKENS + n] * values[n * DIM + tid];
     t.out[of_head * DIM + tid] = sum * __builtin_amdgcn_rcpf(l) * __builtin_amdgcn_rcpf(1.0f + __expf(-gate));
 }
 
@@ -3325,7 +3348,7 @@ void launch_partial_rows(hipStream_t stream, const PartialArgs &a, bool one_per_
 // inverse_root take, and the new tokens take a split of their own: with fewer than 4 the context would be left with too few
 // workgroups.  (The branch to the library's sine and cosine inside them was 1 to 1.6 % of a step at 32768 tokens of 8 bits,
 // taken or not.)
-// out: where the step is to be one launch, which then writes it (a cache of up to ALONE_TOKENS), else nullptr.
+// out: where the step is to be one launch, which then writes it (a cache of up to alone_tokens), else nullptr.
 bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const float *q_and_gate, const float *out, bool keys_first, TokenArgs &token) {
     const size_t n = list.launches.size();
     if (n < 2 || (!out && a.nsplits < 4)) return false;
@@ -3441,11 +3464,17 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
         uint32_t last_is_new = 0;
         if (LaunchList *list = recording()) {
             TokenArgs token;
-            if (capacity <= uint32_t(ALONE_TOKENS) && token_step(*list, a, bits, q_and_gate, out, keys_first, token)) {
+            if (capacity <= alone_tokens(rows) && token_step(*list, a, bits, q_and_gate, out, keys_first, token)) {
                 list->launches.pop_back(), list->launches.pop_back();
                 const AloneArgs alone{token.a, token.prep, out};
-                launch(bits == 16 ? attention_token_alone_kernel<16> : bits == 8 ? attention_token_alone_kernel<8> : attention_token_alone_kernel<4>,
-                       dim3(rows * SAETTA_GQA_GROUP, kv_heads), ALONE_THREADS, 0, stream, alone);
+                auto of = [&](auto tokens) {
+                    constexpr int TOKENS = decltype(tokens)::value;
+                    launch(bits == 16 ? attention_token_alone_kernel<16, TOKENS> : bits == 8 ? attention_token_alone_kernel<8, TOKENS> : attention_token_alone_kernel<4, TOKENS>,
+                           dim3(rows * SAETTA_GQA_GROUP, kv_heads), ALONE_THREADS, 0, stream, alone);
+                };
+                if (capacity <= SAETTA_CHUNK) of(std::integral_constant<int, SAETTA_CHUNK>{});
+                else if (capacity <= 2 * SAETTA_CHUNK) of(std::integral_constant<int, 2 * SAETTA_CHUNK>{});
+                else of(std::integral_constant<int, 3 * SAETTA_CHUNK>{});
                 return launch_status(what);
             }
             if (one_per_cu && token_step(*list, a, bits, q_and_gate, nullptr, keys_first, token)) {

@@ -124,15 +124,15 @@ def test_a_length_of_the_callers_own(kind, capacity):
                 assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), (position, kv_len)
 
 
-@pytest.mark.parametrize("rows", [1, 2, 5, 8])
+@pytest.mark.parametrize("capacity,rows", [(128, 1), (128, 2), (128, 5), (128, 8), (256, 2), (256, 7), (384, 3), (384, 8)])
 @pytest.mark.parametrize("kind", KINDS)
-def test_a_cache_of_one_split_takes_one_launch(kind, rows):
-    # Up to 128 tokens: a workgroup per (row, q head) does the whole step.  No context, around a pass of 16 tokens, the last rows that
-    # fit and rows that do not; a decode also without the new token and with rows past it.
-    step = Step(kind, 128, rows, seed=500 + 10 * rows + kind.value)
+def test_a_small_cache_takes_one_launch(kind, capacity, rows):
+    # Up to 128 tokens (two rows 256, more 384): a workgroup per (row, q head) does the whole step.  No context, around a pass of 32
+    # tokens, the last rows that fit and rows that do not; a decode also without the new token and with rows past it.
+    step = Step(kind, capacity, rows, seed=500 + 10 * rows + kind.value)
     assert launches(step) == 1
     built = step.plan.build()
-    for position in (0, 1, 15, 16, 17, 100, 128 - rows, 127, 130):
+    for position in (0, 1, 31, 32, 33, 100, capacity - 60, capacity - rows, capacity - 1, capacity + 2):
         for kv_len in (None,) if rows > 1 else (None, 1, position, position + 2, position + 40, 200):
             if kv_len == 0:
                 continue  # (no token at all: no number)
@@ -153,14 +153,16 @@ def test_one_launch_where_its_buffers_lie_apart(kind):
         check_laid_over(Step(kind, 128, 1, seed=70 + kind.value, lay=lay), (0, 50, 127))
 
 
+@pytest.mark.parametrize("capacity", [128, 384])
 @pytest.mark.parametrize("kind", KINDS)
-def test_one_launch_drops_what_is_not_in_use(kind):
+def test_one_launch_drops_what_is_not_in_use(kind, capacity):
     # NaN in the rows past the context: halves, or scales and biases
-    step = Step(kind, 128, 3, seed=90 + kind.value)
+    step = Step(kind, capacity, 3, seed=90 + kind.value)
+    assert launches(step) == 1 and launches(Step(kind, 384, 2, seed=1)) == 3
     built = step.plan.build()
     for buffer in step.cache.buffers():
         if buffer.dtype == torch.float16:
-            rows = buffer.view(128, -1)
+            rows = buffer.view(capacity, -1)
             rows[37:] = float("nan")
     want = step.run(step.plan.run_serial, 37)
     got = step.run(built.run, 37)
