@@ -3135,6 +3135,8 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
     const uint32_t before = tokens_before(a, position, kv_len), fresh = tokens_new(a, position, kv_len, row);
     // (a decode sees min(kv_len, capacity) tokens: where the record says more than position + 1, rows past the new one too)
     const uint32_t past = a.decode_len ? min(kv_len, a.capacity) : 0;
+    // (what is in use is told by the token's number all through, never by its score: a NaN in the cache is a NaN in the outputs)
+    auto live = [&](uint32_t token) { return token < before || (token > position && token < past); };
     const float c = a.scale * 1.4426950408889634f;
     float q[16], q_sum = 0.0f;
 #pragma unroll
@@ -3148,8 +3150,7 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
         for (int e = 0; e < 16; e++) s += q[e] * k[e];
         if constexpr (BITS != 16) s = half_bits_to_float(key[i].scale) * s + half_bits_to_float(key[i].bias) * q_sum;
         s = group_reduce<16>(s, SumOp());
-        const bool live = token < before || (token > position && token < past);
-        if (part == 0) score_lds[token] = live ? s : NO_SCORE;
+        if (part == 0) score_lds[token] = live(token) ? s : NO_SCORE;
     }
     for (uint32_t n = wave; n < uint32_t(R); n += ALONE_THREADS / 64) {
         float s = NO_SCORE;
@@ -3165,12 +3166,17 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
 
     // ---- the softmax: every wave for itself, the first hands the probabilities out ----
     constexpr int OLD = TOKENS / 64;
+    constexpr float UNUSED = -1.0f;  // in a probability's place
     float s[OLD + 1], m = s[OLD] = lane < uint32_t(R) ? score_lds[TOKENS + lane] : NO_SCORE, l = 0.0f;
 #pragma unroll
     for (int i = 0; i < OLD; i++) s[i] = score_lds[64 * i + lane], m = fmaxf(m, s[i]);
     m = group_reduce<64>(m, MaxOp());
 #pragma unroll
-    for (int i = 0; i <= OLD; i++) s[i] = s[i] > 0.5f * NO_SCORE ? __builtin_amdgcn_exp2f(s[i] - m) : 0.0f, l += s[i];
+    for (int i = 0; i <= OLD; i++) {
+        const bool used = i < OLD ? live(64 * i + lane) : lane < fresh;
+        s[i] = __builtin_amdgcn_exp2f(s[i] - m);
+        l += used ? s[i] : 0.0f, s[i] = used ? s[i] : UNUSED;
+    }
     l = group_reduce<64>(l, SumOp());
     if (wave == 0) {
 #pragma unroll
@@ -3186,14 +3192,14 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
 #pragma unroll
     for (int i = 0; i < PASSES; i++) {
         float p = prob_lds[i * ALONE_PASS + sub];
-        const bool live = p > 0.0f;  // (never a product with what lies where no token is)
+        const bool used = !(p < 0.0f);  // (never a product with what lies where no token is)
         Sixteen &x = value[i];
         if constexpr (BITS == 16) {
 #pragma unroll
-            for (int w = 0; w < WORDS; w++) x.w[w] = live ? x.w[w] : 0;
+            for (int w = 0; w < WORDS; w++) x.w[w] = used ? x.w[w] : 0;
         } else {
-            biases += live ? p * half_bits_to_float(x.bias) : 0.0f;
-            p = live ? p * half_bits_to_float(x.scale) : 0.0f;
+            biases += used ? p * half_bits_to_float(x.bias) : 0.0f;
+            p = used ? p * half_bits_to_float(x.scale) : 0.0f;
         }
         float v[16];
         sixteen(x, v);

@@ -169,6 +169,28 @@ def test_one_launch_drops_what_is_not_in_use(kind, capacity):
     assert np.isfinite(got[0]).all() and np.abs(got[0] - want[0]).max() < 2e-5
 
 
+@pytest.mark.parametrize("capacity,rows", [(128, 1), (128, 3), (256, 2), (384, 8)])
+@pytest.mark.parametrize("kind", KINDS)
+def test_one_launch_hides_no_nan(kind, capacity, rows):
+    # NaN in one token that is in use, for one kv head: in its key (every output of its heads), in its value (dims of them), in
+    # the new key, in the new value; the same outputs are numbers as by three launches.
+    step = Step(kind, capacity, rows, seed=110 + rows + kind.value)
+    assert launches(step) == 1
+    built, position, clean = step.plan.build(), capacity - 30, [b.clone() for b in step.cache.buffers()]
+    spots = [(i, token) for i, b in enumerate(clean) if b.dtype == torch.float16 for token in (0, 33, position - 1)]  # halves, or scales and biases
+    for spot, token in spots + [(x, position) for x in (step.k0, step.v0) if kind is saetta.KvBits.Half]:
+        for b, c in zip(step.cache.buffers(), clean):
+            b.copy_(c)
+        row = step.cache.buffers()[spot].view(capacity, KV, -1)[token, 1] if isinstance(spot, int) else spot[0, D:]
+        at, was = row.numel() // 4 + 1, row.clone()
+        row[at] = float("nan")
+        want, got = step.run(step.plan.run_serial, position), step.run(built.run, position)
+        row.copy_(was)
+        ok = np.isfinite(want[0]).reshape(rows, KV, -1)
+        assert ok[:, 0].all() and not ok[:, 1].all(), (token, at)
+        assert np.array_equal(ok, np.isfinite(got[0]).reshape(ok.shape)), (token, at)
+
+
 def check_laid_over(step, positions):
     """A step with buffers over each other keeps its launches; outputs as the ops one by one, what is stored bit for bit."""
     assert launches(step) == 3
