@@ -3057,15 +3057,30 @@ void launch_reduce(hipStream_t stream, const ReduceArgs &a) {
 // far as the cache goes, and dropped by select where no token is.  Products and sums in f32, of halves as the cache gives them, of codes as numbers:
 // a token's scale and bias are the same for a lane's sixteen and go into their sums (relative error against 64 bits 4e-7 to 9e-7, where the
 // three launches have 8e-7 to 8e-6; each value made first 1.5e-7 to 2.8e-7 at 0.9 us more a 128 tokens).
-// A layer's step, us, ten layers in a graph, three launches -> one: 118 tokens of halves, one row 11.2 -> 6.4, two 12.2 -> 6.6, four 15.0 -> 7.1, eight
-// 17.4 -> 7.6; 8-bit 11.1 -> 6.7, 11.7 -> 6.8, 14.7 -> 7.4, 19.5 -> 8.1; 4-bit 11.1 -> 7.3, 11.7 -> 7.4, 14.7 -> 8.0, 20.3 -> 8.7; 28 tokens, one row, 8.7 ->
-// 6.4, 9.4 -> 6.7, 9.5 -> 7.3.  Caches of 256, 156 tokens in use: two rows 11.1 -> 9.4, 11.4 -> 8.6, 11.7 -> 9.5, three 13.2 -> 9.5, 13.8 -> 8.6, 13.8 -> 9.6, eight
-// 16.3 -> 10.3, 18.0 -> 9.8, 18.6 -> 10.9.  Of 384, 284 in use: three rows 13.3 -> 11.5, 13.9 -> 10.9, 13.9 -> 11.6, eight 17.6 -> 12.4, 19.5 -> 12.1, 20.2 -> 12.9.
+// A layer's step, us, ten layers in a graph, three launches -> one:
+//   cache  rows  in use   halves          8-bit           4-bit
+//    128     1       4     8.7 ->  6.5     9.3 ->  6.7     9.4 ->  7.3
+//                  119    11.3 ->  6.4    11.2 ->  6.8    11.1 ->  7.3
+//            2     119    12.2 ->  6.6    11.6 ->  6.8    11.8 ->  7.3
+//            8     119    17.4 ->  7.6    19.5 ->  8.1    20.2 ->  8.8
+//    256     2       4     9.6 ->  8.3    10.2 ->  8.7    10.3 ->  9.6
+//                  240    12.4 ->  9.3    11.8 ->  8.7    11.9 ->  9.6
+//            3       4    10.4 ->  8.3    12.4 ->  8.7    12.7 ->  9.6
+//                  240    14.6 ->  9.3    14.5 ->  8.7    14.5 ->  9.7
+//    384     3       4    10.5 ->  9.9    12.5 -> 11.1    12.7 -> 11.7
+//                  370    14.6 -> 11.5    14.5 -> 11.0    14.6 -> 11.7
+//            4       4    11.0 -> 10.3    12.8 -> 11.6    13.1 -> 12.3
+//            8       4    13.2 -> 10.7    14.2 -> 12.3    14.6 -> 13.0
+//                  370    17.7 -> 12.3    19.5 -> 12.2    20.3 -> 13.0
+// Ahead at every length, which matters: it is not known where a step is recorded.  Halves in more than 128 leave out the passes that have no
+// token in use; without that, three rows of 384 take 11.6 at any length, behind the three launches up to some 100 tokens.  Codes, ahead as
+// they are, don't: the branches would cost a full cache 3 to 5 % (8-bit, three rows of 384 at 370, 11.0 -> 11.3, 4-bit 11.7 -> 12.2; at 4 tokens 9.0 and
+// 8.5); nor do halves in 128 (6.1 at 4 tokens, 6.5 at 119).
 // What is left is the launch, the trips to the position and to the rows, the chain of the new rows (norm, rotation, quantizer) and 2 us per
 // 128 tokens of cache, vector instructions.  Threads: 256 take 7.3 (halves, one row; 6.9 then) and 9.4 (eight; 8.1), 8.3 and 11.1 (8-bit; 7.8 and 9.2);
 // 1024 7.5 and 8.2, 8.2 and 9.0.
-// The line: two rows in a cache of 384 are even (halves 11.2 -> 11.4, 4-bit 11.7 -> 11.5).  One row would be ahead in one of 256 too (10.2 -> 9.4, 10.2 -> 8.6,
-// 10.4 -> 9.4) and five and more in one of 512, but those steps are the three launches that test_gpu_token_step.py counts.
+// The line: two rows in a cache of 384 are even (halves 11.2 -> 11.4, 4-bit 11.7 -> 11.5).  One row would be ahead in one of 256 too (156 in use 10.2 -> 9.4 | 10.2 -> 8.6 |
+// 10.4 -> 9.4) and five and more in one of 512: slower than it could be, for those steps are the three launches that test_gpu_token_step.py counts.
 constexpr int ALONE_THREADS = 512, ALONE_PASS = ALONE_THREADS / 16;
 uint32_t alone_tokens(uint32_t rows) { return rows == 1 ? SAETTA_CHUNK : rows == 2 ? 2 * SAETTA_CHUNK : 3 * SAETTA_CHUNK; }
 struct AloneArgs {
@@ -3137,6 +3152,10 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
     const uint32_t past = a.decode_len ? min(kv_len, a.capacity) : 0;
     // (what is in use is told by the token's number all through, never by its score: a NaN in the cache is a NaN in the outputs)
     auto live = [&](uint32_t token) { return token < before || (token > position && token < past); };
+    // (SKIP: a pass of tokens none of which is in use is left out)
+    constexpr bool SKIP = BITS == 16 && TOKENS > SAETTA_CHUNK;
+    const uint32_t end = max(before, past);
+    auto in_use = [&](int pass) { return !SKIP || uint32_t(pass * ALONE_PASS) < end; };
     const float c = a.scale * 1.4426950408889634f;
     float q[16], q_sum = 0.0f;
 #pragma unroll
@@ -3144,12 +3163,16 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
 #pragma unroll
     for (int i = 0; i < PASSES; i++) {
         const uint32_t token = i * ALONE_PASS + sub;
-        float k[16], s = 0.0f;
-        sixteen(key[i], k);
+        float s = NO_SCORE;
+        if (in_use(i)) {
+            float k[16];
+            sixteen(key[i], k);
+            s = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 16; e++) s += q[e] * k[e];
-        if constexpr (BITS != 16) s = half_bits_to_float(key[i].scale) * s + half_bits_to_float(key[i].bias) * q_sum;
-        s = group_reduce<16>(s, SumOp());
+            for (int e = 0; e < 16; e++) s += q[e] * k[e];
+            if constexpr (BITS != 16) s = half_bits_to_float(key[i].scale) * s + half_bits_to_float(key[i].bias) * q_sum;
+            s = group_reduce<16>(s, SumOp());
+        }
         if (part == 0) score_lds[token] = live(token) ? s : NO_SCORE;
     }
     for (uint32_t n = wave; n < uint32_t(R); n += ALONE_THREADS / 64) {
@@ -3191,6 +3214,7 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
     for (int e = 0; e < 16; e++) o[e] = 0.0f;
 #pragma unroll
     for (int i = 0; i < PASSES; i++) {
+        if (!in_use(i)) continue;
         float p = prob_lds[i * ALONE_PASS + sub];
         const bool used = !(p < 0.0f);  // (never a product with what lies where no token is)
         Sixteen &x = value[i];
