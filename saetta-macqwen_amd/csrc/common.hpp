@@ -65,7 +65,7 @@ struct LaunchRecord {
     // What a launch is, for a call that may take launches recorded before it into one of its own.
     uint32_t kind = 0, bits = 0, rows = 0;
 };
-enum : uint32_t { LAUNCH_PREP = 1, LAUNCH_PARTIAL = 2, LAUNCH_CONV = 3 };
+enum : uint32_t { LAUNCH_PREP = 1, LAUNCH_PARTIAL = 2, LAUNCH_CONV = 3, LAUNCH_ALONE = 4 };
 // Launches in order; the arguments lie in `bytes`, each at its offset, 16-byte aligned.
 struct LaunchList {
     std::vector<LaunchRecord> launches;
@@ -74,6 +74,8 @@ struct LaunchList {
     int device = 0;
     template <class T>
     const T &arg(const LaunchRecord &r, uint32_t i) const { return *reinterpret_cast<const T *>(bytes.data() + offsets[r.first_arg + i]); }
+    template <class T>
+    T &arg(const LaunchRecord &r, uint32_t i) { return *reinterpret_cast<T *>(bytes.data() + offsets[r.first_arg + i]); }
 };
 // The list this thread records into, or nullptr: launches are made.
 LaunchList *&recording();

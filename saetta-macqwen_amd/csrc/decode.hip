@@ -3087,6 +3087,7 @@ struct AloneArgs {
     PartialArgs a;
     PrepArgs prep;
     float *out;
+    uint32_t keep;  // 1: the step's partials go to its scratch too, everything in the first split (0.1 to 0.2 us)
 };
 
 template <int BITS, int TOKENS>
@@ -3243,6 +3244,11 @@ __global__ __launch_bounds__(ALONE_THREADS) void attention_token_alone_kernel(Al
     for (int w = 0; w < ALONE_THREADS / 64; w++) sum += o_lds[w][tid];
     for (uint32_t n = 0; n < fresh; n++) sum += prob_lds[TOKENS + n] * values[n * DIM + tid];
     t.out[of_head * DIM + tid] = sum * __builtin_amdgcn_rcpf(l) * __builtin_amdgcn_rcpf(1.0f + __expf(-gate));
+    if (!t.keep) return;
+    const size_t first = size_t(row) * a.nsplits * a.heads + kv * SAETTA_GQA_GROUP + head0;
+    a.part_o[first * DIM + tid] = sum;
+    for (uint32_t split = 1; split < a.nsplits; split++) a.part_o[(first + split * a.heads) * DIM + tid] = 0.0f;
+    if (tid < a.nsplits) *reinterpret_cast<floatx2 *>(a.part_ml + 2 * (first + tid * a.heads)) = tid == 0 ? floatx2{m, l} : floatx2{NO_SCORE, 0.0f};
 }
 
 uint32_t splits_for(uint32_t capacity, uint32_t wanted) {
@@ -3434,6 +3440,17 @@ bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const fl
     return true;
 }
 
+// A reduce stage is recorded over the scratch of `a`: a step of one launch that was the last to use it leaves its partials there.
+void read_again(LaunchList &list, const PartialArgs &a) {
+    for (size_t n = list.launches.size(); n-- > 0;) {
+        const LaunchRecord &r = list.launches[n];
+        if (r.kind == LAUNCH_PARTIAL && list.arg<PartialArgs>(r, 0).part_o == a.part_o) return;
+        if (r.kind != LAUNCH_ALONE || list.arg<AloneArgs>(r, 0).a.part_o != a.part_o) continue;
+        list.arg<AloneArgs>(r, 0).keep = 1;
+        return;
+    }
+}
+
 int run_attention(hipStream_t stream, int bits, const float *q, const void *kdata, const void *vdata,
                   const uint16_t *ks, const uint16_t *kz, const uint16_t *vs, const uint16_t *vz,
                   float *part_o, float *part_ml, const float *q_and_gate, float *out, uint32_t heads,
@@ -3496,7 +3513,7 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
             TokenArgs token;
             if (capacity <= alone_tokens(rows) && token_step(*list, a, bits, q_and_gate, out, keys_first, token)) {
                 list->launches.pop_back(), list->launches.pop_back();
-                const AloneArgs alone{token.a, token.prep, out};
+                const AloneArgs alone{token.a, token.prep, out, 0};
                 auto of = [&](auto tokens) {
                     constexpr int TOKENS = decltype(tokens)::value;
                     launch(bits == 16 ? attention_token_alone_kernel<16, TOKENS> : bits == 8 ? attention_token_alone_kernel<8, TOKENS> : attention_token_alone_kernel<4, TOKENS>,
@@ -3505,6 +3522,7 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
                 if (capacity <= SAETTA_CHUNK) of(std::integral_constant<int, SAETTA_CHUNK>{});
                 else if (capacity <= 2 * SAETTA_CHUNK) of(std::integral_constant<int, 2 * SAETTA_CHUNK>{});
                 else of(std::integral_constant<int, 3 * SAETTA_CHUNK>{});
+                tag_launch(LAUNCH_ALONE, uint32_t(bits), rows);
                 return launch_status(what);
             }
             if (one_per_cu && token_step(*list, a, bits, q_and_gate, nullptr, keys_first, token)) {
@@ -3512,6 +3530,8 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
                 partial(&token);
                 last_is_new = 1;
                 nsplits = token.a.nsplits;
+            } else {
+                read_again(*list, a);
             }
         }
         ReduceArgs r{part_o, part_ml, q_and_gate, out, heads, capacity, nsplits, rows, d_tp, decode_len ? 1u : 0u, last_is_new};

@@ -193,6 +193,31 @@ def test_one_launch_hides_no_nan(kind, capacity, rows):
         assert np.array_equal(ok, np.isfinite(got[0]).reshape(ok.shape)), (token, at)
 
 
+@pytest.mark.parametrize("capacity,rows", [(128, 1), (128, 8), (256, 2), (384, 3)])
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_second_merge_of_one_launch(kind, capacity, rows):
+    # another reduce stage over the step's scratch, with a gate of its own, recorded behind it
+    step = Step(kind, capacity, rows, seed=130 + rows + kind.value)
+    att = step.att or step.cache.decode
+    gates, out = dev(np.random.default_rng(rows).standard_normal((rows, H, 2 * D)).astype(np.float32)), torch.zeros(rows, H * D, device="cuda")
+    keys, values = step.cache.quant or (step.cache.keys, step.cache.values)
+    record = att.record if kind is saetta.KvBits.Half else att.record_quant
+    if rows == 1:
+        record(step.plan, step.q, keys, values, gates, out)
+    else:
+        record(step.plan, rows, step.q, keys, values, gates, out, [step.plan.params] * rows)
+    step.plan.ops.pop(-2)  # (its partial stage)
+    assert launches(step) == 2
+    built = step.plan.build()
+    for position in (0, 50, capacity - rows):
+        step.run(step.plan.run_serial, position)
+        want = host(out).copy()
+        for t in (out, att.part_o, att.part_ml):
+            t.fill_(float("nan"))
+        step.run(built.run, position)
+        assert np.abs(host(out) - want).max() < 2e-5, position
+
+
 def check_laid_over(step, positions):
     """A step with buffers over each other keeps its launches; outputs as the ops one by one, what is stored bit for bit."""
     assert launches(step) == 3
