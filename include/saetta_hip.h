@@ -197,8 +197,7 @@ int saetta_token_params_set(saetta_stream_t stream, saetta_token_params *d_tp, s
  * any thread, also on several at once; under stream capture it becomes part of the graph.  Launches
  * recorded one after the other over the same buffers may become one: a token's store, partial and
  * reduce stage, a DeltaNet conv and the chunk it feeds; what they write is the same, the partials in
- * scratch aside (a step over a cache of up to 384 tokens leaves them there only for further reduce
- * stages of the same plan).  Where their
+ * scratch aside, which are there for the reduce stages of the same plan only.  Where their
  * buffers overlap (k_back in the place of k, scratch over inputs that are done with) they stay
  * launches of their own.  begin fails while the
  * thread is recording, end returns NULL when it is not. */

@@ -65,7 +65,7 @@ struct LaunchRecord {
     // What a launch is, for a call that may take launches recorded before it into one of its own.
     uint32_t kind = 0, bits = 0, rows = 0;
 };
-enum : uint32_t { LAUNCH_PREP = 1, LAUNCH_PARTIAL = 2, LAUNCH_CONV = 3, LAUNCH_ALONE = 4 };
+enum : uint32_t { LAUNCH_PREP = 1, LAUNCH_PARTIAL = 2, LAUNCH_CONV = 3, LAUNCH_ALONE = 4, LAUNCH_REDUCE = 5 };
 // Launches in order; the arguments lie in `bytes`, each at its offset, 16-byte aligned.
 struct LaunchList {
     std::vector<LaunchRecord> launches;

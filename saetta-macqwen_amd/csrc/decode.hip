@@ -3440,14 +3440,21 @@ bool token_step(const LaunchList &list, const PartialArgs &a, int bits, const fl
     return true;
 }
 
-// A reduce stage is recorded over the scratch of `a`: a step of one launch that was the last to use it leaves its partials there.
-void read_again(LaunchList &list, const PartialArgs &a) {
+// A further reduce stage is recorded over the scratch of `a`: of the partials as the step that was the last to use it divides them, where
+// that is a step in fewer launches.  One in a single launch leaves them there only for this.
+void read_again(LaunchList &list, const PartialArgs &a, uint32_t &nsplits, uint32_t &last_is_new) {
     for (size_t n = list.launches.size(); n-- > 0;) {
         const LaunchRecord &r = list.launches[n];
         if (r.kind == LAUNCH_PARTIAL && list.arg<PartialArgs>(r, 0).part_o == a.part_o) return;
-        if (r.kind != LAUNCH_ALONE || list.arg<AloneArgs>(r, 0).a.part_o != a.part_o) continue;
-        list.arg<AloneArgs>(r, 0).keep = 1;
-        return;
+        if (r.kind == LAUNCH_REDUCE && list.arg<ReduceArgs>(r, 0).part_o == a.part_o) {
+            const ReduceArgs &b = list.arg<ReduceArgs>(r, 0);
+            if (b.last_is_new && b.rows == a.rows && b.heads == a.heads && b.capacity == a.capacity) nsplits = b.nsplits, last_is_new = 1;
+            return;
+        }
+        if (r.kind == LAUNCH_ALONE && list.arg<AloneArgs>(r, 0).a.part_o == a.part_o) {
+            list.arg<AloneArgs>(r, 0).keep = 1;
+            return;
+        }
     }
 }
 
@@ -3531,13 +3538,14 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
                 last_is_new = 1;
                 nsplits = token.a.nsplits;
             } else {
-                read_again(*list, a);
+                read_again(*list, a, nsplits, last_is_new);
             }
         }
         ReduceArgs r{part_o, part_ml, q_and_gate, out, heads, capacity, nsplits, rows, d_tp, decode_len ? 1u : 0u, last_is_new};
         if (rows == 1) launch_reduce<16, false>(stream, r);
         else if (rows == 2) launch_reduce<32, false>(stream, r);
         else launch_reduce<64, true>(stream, r);
+        tag_launch(LAUNCH_REDUCE, uint32_t(bits), rows);
     }
     return launch_status(what);
 }

@@ -193,10 +193,10 @@ def test_one_launch_hides_no_nan(kind, capacity, rows):
         assert np.array_equal(ok, np.isfinite(got[0]).reshape(ok.shape)), (token, at)
 
 
-@pytest.mark.parametrize("capacity,rows", [(128, 1), (128, 8), (256, 2), (384, 3)])
+@pytest.mark.parametrize("capacity,rows,count", [(128, 1, 1), (128, 8, 1), (256, 2, 1), (384, 3, 1), (512, 1, 2), (8192, 4, 2), (40960, 1, 2), (40960, 3, 2), (49152, 6, 2)])
 @pytest.mark.parametrize("kind", KINDS)
-def test_a_second_merge_of_one_launch(kind, capacity, rows):
-    # another reduce stage over the step's scratch, with a gate of its own, recorded behind it
+def test_a_second_merge(kind, capacity, rows, count):
+    # another reduce stage over the step's scratch, with a gate of its own, recorded behind it; and one more
     step = Step(kind, capacity, rows, seed=130 + rows + kind.value)
     att = step.att or step.cache.decode
     gates, out = dev(np.random.default_rng(rows).standard_normal((rows, H, 2 * D)).astype(np.float32)), torch.zeros(rows, H * D, device="cuda")
@@ -207,7 +207,8 @@ def test_a_second_merge_of_one_launch(kind, capacity, rows):
     else:
         record(step.plan, rows, step.q, keys, values, gates, out, [step.plan.params] * rows)
     step.plan.ops.pop(-2)  # (its partial stage)
-    assert launches(step) == 2
+    step.plan.ops.append(step.plan.ops[-1])
+    assert launches(step) == count + 2
     built = step.plan.build()
     for position in (0, 50, capacity - rows):
         step.run(step.plan.run_serial, position)
