@@ -2997,8 +2997,8 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
         if (!live) mlv[i][1] = 0.0f, pv[i] = floatx4{0, 0, 0, 0};
         mx = fmaxf(mx, m[i]);
     }
-    // the wave's maximum; like the sums, over the 16 slots (lanes 4 apart: two steps inside a row of 16 lanes, two across
-    // rows), the four quads of a slot having the same m and l
+    // the wave's maximum; like the sums, over the SLOTS slots, whose lanes are QUADS apart: with 4 quads two steps inside a row of 16
+    // lanes, with 8 one, with 16 none, then two across rows.  The quads of a slot have the same m and l.
     if constexpr (QUADS <= 4) mx = fmaxf(mx, dpp<0x124>(mx));  // row_ror 4
     if constexpr (QUADS <= 8) mx = fmaxf(mx, dpp<0x128>(mx));  // row_ror 8
     mx = across_rows<16, 64>(mx, MaxOp());
@@ -3034,18 +3034,22 @@ __global__ __launch_bounds__(256) void attention_reduce_kernel(ReduceArgs a) {
         a.out[qh * DIM + DIMS * slice + tid] = sum * __builtin_amdgcn_rcpf(total) * open;
     }
 }
-static_assert(MAX_SPLITS <= 4 * 64, "launch_reduce's variants");
 
-// (more rows than one have a workgroup per CU, and half as many splits at most)
+// (more rows than one have a workgroup per CU, and half as many splits at most: run_attention)
 template <int DIMS, bool WAIT>
-void launch_reduce(hipStream_t stream, const ReduceArgs &a) {
-    constexpr int ONE = DIMS / 16;  // splits a lane takes, of 64
+int launch_reduce(hipStream_t stream, const ReduceArgs &a) {
+    constexpr uint32_t ONE = DIMS / 16, HALF = MAX_SPLITS / 2;  // splits a lane takes, of 64
+    static_assert(4 * (64 / (DIMS / 4)) * ONE == 64 && HALF <= 2 * 64 && MAX_SPLITS <= 4 * 64, "a split has a place");
     const dim3 grid(a.heads, a.rows, DIM / DIMS);
-    if (a.nsplits <= MAX_SPLITS / 4) return launch(attention_reduce_kernel<DIMS, ONE, WAIT>, grid, 256, 0, stream, a);
-    if constexpr (DIMS == 16) {
-        if (a.nsplits > MAX_SPLITS / 2) return launch(attention_reduce_kernel<DIMS, 4 * ONE, WAIT>, grid, 256, 0, stream, a);
+    if (a.nsplits <= 64) {
+        launch(attention_reduce_kernel<DIMS, ONE, WAIT>, grid, 256, 0, stream, a);
+    } else if (a.nsplits <= HALF) {
+        launch(attention_reduce_kernel<DIMS, 2 * ONE, WAIT>, grid, 256, 0, stream, a);
+    } else {
+        SAETTA_REQUIRE(DIMS == 16, SAETTA_E_SHAPE, "merge of %u rows: %u splits, %u at most", a.rows, a.nsplits, HALF);
+        if constexpr (DIMS == 16) launch(attention_reduce_kernel<DIMS, 4 * ONE, WAIT>, grid, 256, 0, stream, a);
     }
-    launch(attention_reduce_kernel<DIMS, 2 * ONE, WAIT>, grid, 256, 0, stream, a);
+    return SAETTA_OK;
 }
 
 // ---- a token step of a cache of up to three splits: one launch --------------------------------------
@@ -3542,9 +3546,7 @@ int run_attention(hipStream_t stream, int bits, const float *q, const void *kdat
             }
         }
         ReduceArgs r{part_o, part_ml, q_and_gate, out, heads, capacity, nsplits, rows, d_tp, decode_len ? 1u : 0u, last_is_new};
-        if (rows == 1) launch_reduce<16, false>(stream, r);
-        else if (rows == 2) launch_reduce<32, false>(stream, r);
-        else launch_reduce<64, true>(stream, r);
+        if (int rc = rows == 1 ? launch_reduce<16, false>(stream, r) : rows == 2 ? launch_reduce<32, false>(stream, r) : launch_reduce<64, true>(stream, r)) return rc;
         tag_launch(LAUNCH_REDUCE, uint32_t(bits), rows);
     }
     return launch_status(what);
