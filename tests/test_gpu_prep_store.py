@@ -198,18 +198,20 @@ def test_verify_rows_and_decode_after_store(kind):
     dqg = dev(qg)
     saetta.record_store(plan, dqg, dev(k), dev(v), dev(qn), dev(kn), q, keys, values, p, capacity, rows=m, k_back=k_back)
     att = saetta.AttentionRows(H, KV, capacity, m)
-    params = [plan.params] * m
-    if kind is saetta.KvBits.Half:
-        att.record(plan, m, q, keys, values, dqg, out, params)
-    else:
-        att.record_quant(plan, m, q, keys, values, dqg, out, params)
+    record = att.record if kind is saetta.KvBits.Half else att.record_quant
+    record(plan, m, q, keys, values, dqg, out, [plan.params] * m)
     plan.set_params(saetta.TokenParams(0, ctx))
     plan.build().run()
+    # (the step may take the new rows from where it made them: the attention by itself has what it stored)
+    read_back, alone = torch.full_like(out, float("nan")), saetta.Plan()
+    record(alone, m, q, keys, values, dqg, read_back, [plan.params] * m)
+    alone.build().run()
     kb = host(k_back)
     for r in range(m):
         kf[ctx + r], vf[ctx + r] = stored(kb[r]), stored(v[r])
     want = oracle.rows(host(q), kf, vf, ctx, m, q_and_gate=qg, threads=8, f64=True)
     assert np.abs(host(out) - want).max() < 2e-5
+    assert np.abs(host(read_back) - want).max() < 2e-5
 
 
 def test_rejected_arguments():

@@ -13,6 +13,10 @@ KINDS = [saetta.KvBits.Half, saetta.KvBits.Eight, saetta.KvBits.Four]
 PREP = saetta.PrepParams(H, KV, D, 64, 1e7, 1e-6)
 
 
+def poison(rows):
+    rows.fill_(float("nan") if rows.dtype == torch.float16 else -1)
+
+
 class Step:
     def __init__(self, kind, capacity, rows, seed, rope_dims=64, lay=lambda step: None, theta=1e7, eps=1e-6):
         rng = np.random.default_rng(seed)
@@ -30,6 +34,7 @@ class Step:
         keys, values = self.cache.quant or (self.cache.keys, self.cache.values)
         self.q, self.out, self.back = (torch.zeros(rows, n, device="cuda") for n in (H * D, H * D, VALUES))
         self.k0, self.v0 = self.k.clone(), self.v.clone()
+        self.clean = [b.clone() for b in self.cache.buffers()]
         self.att = saetta.AttentionRows(H, KV, self.cache.capacity, rows) if rows > 1 else None
         lay(self)  # (buffers over others)
         self.k.copy_(self.k0), self.v.copy_(self.v0)
@@ -44,6 +49,10 @@ class Step:
                 self.plan, rows, self.q, keys, values, self.qg, self.out, [self.plan.params] * rows)
 
     def run(self, how, position, kv_len=None):
+        # every run finds the cache as it was, with NaN (codes: all ones) where the step stores: what is there behind it is its own
+        for buffer, was in zip(self.cache.buffers(), self.clean):
+            buffer.copy_(was)
+            poison(buffer.view(self.cache.capacity, -1)[position:position + self.rows])
         params = saetta.TokenParams(0, position)
         params.kv_len = position + 1 if kv_len is None else kv_len
         self.plan.set_params(params)
@@ -71,7 +80,6 @@ def test_fused_step_equals_the_ops_one_by_one(kind, capacity, rows):
     # no context; one block and less; around a block's end; several rounds; the last rows; rows that do not fit
     for position in (0, 1, 15, 16, 100, cap // 2 + 3, cap - rows, cap - 1, cap + 2):
         want = step.run(step.plan.run_serial, position)
-        before = [host(b).copy() for b in step.cache.buffers()]
         got = step.run(built.run, position)
         if position == 0 or position <= cap - rows:
             assert np.isfinite(got[0]).all(), position
@@ -80,7 +88,7 @@ def test_fused_step_equals_the_ops_one_by_one(kind, capacity, rows):
         assert np.abs(got[0] - want[0])[ok].max(initial=0.0) < 2e-5, position
         assert np.array_equal(got[1], want[1]), position
         assert np.array_equal(got[2], want[2]), position
-        for a, b in zip(got[3:], before):
+        for a, b in zip(got[3:], want[3:]):
             assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), position
 
 
@@ -139,11 +147,10 @@ def test_a_small_cache_takes_one_launch(kind, capacity, rows):
             if kv_len == 0:
                 continue  # (no token at all: no number)
             want = step.run(step.plan.run_serial, position, kv_len)
-            before = [host(b).copy() for b in step.cache.buffers()]
             got = step.run(built.run, position, kv_len)
             assert np.isfinite(want[0]).all() and np.isfinite(got[0]).all(), (position, kv_len)
             assert np.abs(got[0] - want[0]).max() < 2e-5, (position, kv_len)
-            for x, y in zip(got[1:], want[1:3] + before):
+            for x, y in zip(got[1:], want[1:]):
                 assert np.array_equal(x.view(np.uint8), y.view(np.uint8)), (position, kv_len)
 
 
@@ -155,20 +162,43 @@ def test_one_launch_where_its_buffers_lie_apart(kind):
         check_laid_over(Step(kind, 128, 1, seed=70 + kind.value, lay=lay), (0, 50, 127))
 
 
-@pytest.mark.parametrize("capacity", [128, 384])
+@pytest.mark.parametrize("capacity,rows", [(128, 1), (128, 3), (256, 2), (384, 3), (384, 8)])
 @pytest.mark.parametrize("kind", KINDS)
-def test_one_launch_drops_what_is_not_in_use(kind, capacity):
-    # NaN in the rows past the context: halves, or scales and biases
-    step = Step(kind, capacity, 3, seed=90 + kind.value)
-    assert launches(step) == 1 and launches(Step(kind, 384, 2, seed=1)) == 3
-    built = step.plan.build()
-    for buffer in step.cache.buffers():
-        if buffer.dtype == torch.float16:
-            rows = buffer.view(capacity, -1)
-            rows[37:] = float("nan")
-    want = step.run(step.plan.run_serial, 37)
-    got = step.run(built.run, 37)
-    assert np.isfinite(got[0]).all() and np.abs(got[0] - want[0]).max() < 2e-5
+def test_one_launch_drops_what_is_not_in_use(kind, capacity, rows):
+    # NaN and codes of all ones in the rows past the context; a decode also without its last tokens and with rows past the new one
+    step = Step(kind, capacity, rows, seed=90 + kind.value)
+    assert launches(step) == 1
+    built, clean = step.plan.build(), step.clean
+    for kv_len in (None,) if rows > 1 else (None, 20, 38, 39, 75):
+        step.clean = [b.clone() for b in clean]
+        for buffer in step.clean:
+            poison(buffer.view(capacity, -1)[kv_len or 37:])
+        want, got = step.run(step.plan.run_serial, 37, kv_len), step.run(built.run, 37, kv_len)
+        assert np.isfinite(got[0]).all() and np.abs(got[0] - want[0]).max() < 2e-5, kv_len
+        for x, y in zip(got[1:], want[1:]):
+            assert np.array_equal(x.view(np.uint8), y.view(np.uint8)), kv_len
+
+
+@pytest.mark.parametrize("capacity,rows", [(128, 1), (256, 2), (384, 8)])
+@pytest.mark.parametrize("kind", KINDS)
+def test_one_launch_against_64_bits(kind, capacity, rows):
+    # A few channels 8 times as large as the rest.  A score's terms (codes with the bias not yet taken off) add up to some 70 in units of
+    # log2(e), half an ulp of which is 4e-6: a weight of the softmax, and so an output, is off by less than that of itself.
+    step = Step(kind, capacity, rows, seed=150 + kind.value)
+    assert launches(step) == 1
+    rng = np.random.default_rng(rows)
+    fill = rng.standard_normal((2, capacity, VALUES)).astype(np.float32)
+    fill[:, :, [7, 101, 230, 333, 460]] *= 8
+    for x, half, quant in zip(fill, (step.cache.keys, step.cache.values), step.cache.quant or (None, None)):
+        half.copy_(dev(x).flatten().half()) if quant is None else quant.encode(dev(x), 0, capacity)
+    step.clean, built = [b.clone() for b in step.cache.buffers()], step.plan.build()
+    for position in (5, capacity // 2 + 3, capacity - rows):
+        got = step.run(built.run, position)
+        held = step.cache.quant and [host(saetta.dequantize(*c.tensors(), kind)) for c in step.cache.quant]
+        keys, values = (x.reshape(capacity, VALUES) for x in held or [host(c.float()) for c in (step.cache.keys, step.cache.values)])
+        want = oracle.rows(got[1], keys, values, position, rows, q_and_gate=host(step.qg), threads=8, f64=True).reshape(got[0].shape)
+        error = np.linalg.norm(got[0] - want) / np.linalg.norm(want)
+        assert error < 4e-6, (position, error)
 
 
 @pytest.mark.parametrize("capacity,rows", [(128, 1), (128, 3), (256, 2), (384, 8)])
@@ -178,12 +208,10 @@ def test_one_launch_hides_no_nan(kind, capacity, rows):
     # the new key, in the new value; the same outputs are numbers as by three launches.
     step = Step(kind, capacity, rows, seed=110 + rows + kind.value)
     assert launches(step) == 1
-    built, position, clean = step.plan.build(), capacity - 30, [b.clone() for b in step.cache.buffers()]
-    spots = [(i, token) for i, b in enumerate(clean) if b.dtype == torch.float16 for token in (0, 33, position - 1)]  # halves, or scales and biases
+    built, position = step.plan.build(), capacity - 30
+    spots = [(i, token) for i, b in enumerate(step.clean) if b.dtype == torch.float16 for token in (0, 33, position - 1)]  # halves, or scales and biases
     for spot, token in spots + [(x, position) for x in (step.k0, step.v0) if kind is saetta.KvBits.Half]:
-        for b, c in zip(step.cache.buffers(), clean):
-            b.copy_(c)
-        row = step.cache.buffers()[spot].view(capacity, KV, -1)[token, 1] if isinstance(spot, int) else spot[0, D:]
+        row = step.clean[spot].view(capacity, KV, -1)[token, 1] if isinstance(spot, int) else spot[0, D:]
         at, was = row.numel() // 4 + 1, row.clone()
         row[at] = float("nan")
         want, got = step.run(step.plan.run_serial, position), step.run(built.run, position)
