@@ -2453,8 +2453,10 @@ __device__ __forceinline__ void attention_partial_s_body(const PartialArgs &a, c
             // every wave has built its operands (keys, scales, scores) and is through with the values of round r.
             constexpr int AB = W::ALT_BLOCKS, WAVE_BLOCKS = AB / W::WAVES, WAVE_STEPS = AB / 4;
             // The query operands are held over the rounds: read anew in each they were 80 KB of the round's way through LDS, in front of its
-            // first product.  With the operands of one_row_operand, 4-bit codes at 150000 tokens 31.65 -> 30.25 us a layer, 60000 19.1 -> 17.9, 216000
-            // 40.8 -> 38.9; 8-bit codes, whose rounds wait for memory, 1 % and less.  What the loaders alone take there, with no arithmetic
+            // first product.  What makes a round of 4-bit codes shorter, us a layer at 60000 | 150000 | 216000 tokens, without -> with it: the operands held
+            // 18.2 -> 17.8 | 31.0 -> 30.05 | 39.8 -> 38.4; one_row_operand 18.1 | 30.6 | 39.2 (a single round of 32768 tokens 13.3 -> 13.05); the mask in the last
+            // block only 17.95 | 30.4 | 39.0; RawMaxOp 17.85 | 30.25 | 38.7.  8-bit codes, whose rounds wait for memory: the mask 20.9 -> 20.6 at 60000,
+            // 15.4 -> 15.3 at 32768, the others nothing.  What the loaders alone take at 150000 tokens of 4 bits, with no arithmetic
             // at all, is 25.4.  Tried here: scores a round ahead of the operands, so that no wave waits for another's (32.7); four
             // places of 8 blocks for 4-bit codes, two rounds of every loader on their way (34.4: what has landed is told of later); the
             // values and the next keys read as soon as they are there, under the operands (31.9).
